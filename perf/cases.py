@@ -38,31 +38,31 @@ HEADS = [(16, 4, 128), (32, 8, 128), (32, 8, 64), (16, 16, 64), (16, 16, 128), (
 def listed():
     return [
         # one projection of a serving batch's decode step outside a captured graph: 45 MB of weights
-        dict(name="int8 linear, 16 tokens", kind="linear_int8", tokens=16, k=4096, n=11008, bias=False),
+        dict(name="int8 linear 16 tokens", kind="linear_int8", tokens=16, k=4096, n=11008, bias=False),
         # a prompt whose length is no multiple of anything, through a feed-forward projection with a bias
-        dict(name="fp8 linear, 3001 tokens", kind="linear_fp8", tokens=3001, k=2048, n=11264, bias=True, dynamic=True),
+        dict(name="fp8 linear 3001 tokens", kind="linear_fp8", tokens=3001, k=2048, n=11264, bias=True, dynamic=True),
         # one training step's linear layer, forward and backward
-        dict(name="fp8 training, 4096", kind="train_fp8", tokens=4096, k=4096, n=4096, bias=True, dynamic=False),
+        dict(name="fp8 training 4096", kind="train_fp8", tokens=4096, k=4096, n=4096, bias=True, dynamic=False),
         # the block-scaled product of a large prompt
-        dict(name="block fp8, 8192 tokens", kind="linear_block", tokens=8192, k=7168, n=2048),
+        dict(name="block fp8 8192 tokens", kind="linear_block", tokens=8192, k=7168, n=2048),
         # causal attention of fresh prompts, tensors as the model's projections give them
-        dict(name="prompt attention, dense", kind="prompt_attn", paged=False, batch=4, new=2048, cached=0, heads=16,
+        dict(name="prompt attention dense", kind="prompt_attn", paged=False, batch=4, new=2048, cached=0, heads=16,
              kv_heads=4, dim=128),
         # a ragged batch of a paged server, some of each prompt's prefix cached already, heads of 64
-        dict(name="prompt attention, paged", kind="prompt_attn", paged=True, batch=16, new=700, cached=500, heads=32,
+        dict(name="prompt attention paged", kind="prompt_attn", paged=True, batch=16, new=700, cached=500, heads=32,
              kv_heads=8, dim=64),
         # a paged server's decode step, ragged contexts
-        dict(name="decode attention, paged", kind="decode_attn", batch=32, context=3000, heads=16, kv_heads=4, dim=128),
+        dict(name="decode attention paged", kind="decode_attn", batch=32, context=3000, heads=16, kv_heads=4, dim=128),
         # a batch of prompts through the dense decoder, int8 weights and activations
-        dict(name="dense int8 prompt, 32 x 512", kind="prompt", model="dense", batch=32, seq=512),
+        dict(name="dense int8 prompt 32 x 512", kind="prompt", model="dense", batch=32, seq=512),
         # ... and the decode step that follows
-        dict(name="dense int8 step, 32 x 512", kind="step", model="dense", batch=32, seq=512),
+        dict(name="dense int8 step 32 x 512", kind="step", model="dense", batch=32, seq=512),
         # a batch of prompts through latent and lightning attention
-        dict(name="lugitar prompt, 32 x 512", kind="prompt", model="lugitar", batch=32, seq=512),
+        dict(name="lugitar prompt 32 x 512", kind="prompt", model="lugitar", batch=32, seq=512),
         # one long prompt through recurrences, delta rule and attention with a sink
-        dict(name="sarulix prompt, 1 x 4096", kind="prompt", model="sarulix", batch=1, seq=4096),
+        dict(name="sarulix prompt 1 x 4096", kind="prompt", model="sarulix", batch=1, seq=4096),
         # ... and a batch's decode step
-        dict(name="sarulix step, 32 x 512", kind="step", model="sarulix", batch=32, seq=512),
+        dict(name="sarulix step 32 x 512", kind="step", model="sarulix", batch=32, seq=512),
     ]
 
 
