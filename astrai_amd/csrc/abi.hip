@@ -505,9 +505,45 @@ int astrai_w8a8_attn_prefill_bf16(const void* q, const void* k_cache, const void
     if (batch == 0 || seq == 0) return ASTRAI_W8A8_OK;
     w8a8::AttnPrefillArgs a{q, k_cache, v_cache, positions, out, (int)batch, (int)seq, (int)n_heads,
                             (int)n_kv_heads, (int)head_dim, max_len, scale};
+    a.q_stride = {n_heads * seq * head_dim, seq * head_dim, head_dim};
+    a.k_stride = a.v_stride = {n_kv_heads * max_len * head_dim, max_len * head_dim, head_dim};
     if (!w8a8::launch_attn_prefill(a, static_cast<hipStream_t>(stream)))
         return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_prefill_bf16: shape not supported");
     return check_launch("attn_prefill_bf16");
+}
+
+int astrai_w8a8_attn_prefill_strided_bf16(const void* q, const void* k, const void* v, const int64_t* strides,
+                                          const int64_t* positions, void* out, int64_t batch, int64_t q_len,
+                                          int64_t kv_len, int64_t n_heads, int64_t n_kv_heads, int64_t head_dim,
+                                          int64_t causal_offset, float scale, void* stream) {
+    if (!q || !k || !v || !strides || !out)
+        return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: null pointer");
+    if (batch < 0 || q_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || kv_len <= 0 || n_heads % n_kv_heads ||
+        q_len > (1 << 24) || batch > (1 << 20) || kv_len > INT32_MAX || causal_offset > INT32_MAX / 2)
+        return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: bad dims");
+    if (!w8a8::attn_prefill_supported((int)n_heads, (int)n_kv_heads, (int)head_dim) &&
+        !w8a8::attn_prefill_split_supported((int)n_heads, (int)n_kv_heads, (int)head_dim))
+        return fail(ASTRAI_W8A8_UNSUPPORTED,
+                    "attn_prefill_strided_bf16: needs head_dim 64 or 128 and n_heads / n_kv_heads in {1, 2, 4, 8}");
+    for (int i = 0; i < 9; ++i)
+        if (strides[i] < 0 || strides[i] % 8)
+            return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: strides must be multiples of 8 elements");
+    if (kv_len * strides[5] >= ((int64_t)1 << 31) || kv_len * strides[8] >= ((int64_t)1 << 31))
+        return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_prefill_strided_bf16: one head's rows must span less than 4 GiB");
+    if (!(scale > 0.0f)) return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: scale must be positive");
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out))
+        return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: pointers must be 16-byte aligned");
+    if (batch == 0 || q_len == 0) return ASTRAI_W8A8_OK;
+    w8a8::AttnPrefillArgs a{q, k, v, positions, out, (int)batch, (int)q_len, (int)n_heads,
+                            (int)n_kv_heads, (int)head_dim, kv_len, scale};
+    a.q_stride = {strides[0], strides[1], strides[2]};
+    a.k_stride = {strides[3], strides[4], strides[5]};
+    a.v_stride = {strides[6], strides[7], strides[8]};
+    a.causal = causal_offset >= 0;
+    a.causal_offset = (int)(causal_offset < 0 ? 0 : causal_offset);
+    if (!w8a8::launch_attn_prefill(a, static_cast<hipStream_t>(stream)))
+        return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_prefill_strided_bf16: shape not supported");
+    return check_launch("attn_prefill_strided_bf16");
 }
 
 int astrai_w8a8_attn_paged_prefill_bf16(const void* q, const void* k_pool, const void* v_pool,
@@ -567,6 +603,14 @@ int astrai_w8a8_attn_paged_prefill_masked_bf16(
     return check_launch("attn_paged_prefill_bf16");
 }
 
+// The prompt shapes that both kernels take (attn_prefill_split_supported) run the block kernel from this many
+// (64-row tile, query head) pairs, and attn_rows.hip with its context split below: the block kernel does not
+// split a context, so a few tiles over a long one leave the chip idle. Measured, split rows kernel -> block
+// kernel: 256 pairs 47 -> 18 us (32 / 8 heads x 64, 4 x 200 tokens behind 500), 31 -> 22 us (16 / 16 x 64, same),
+// 41 -> 38 us (16 / 2 x 64, 2 x 256 behind 1000); 128 pairs 31 -> 35 us (16 / 16 x 64, 2 x 256 behind 1000),
+// 75 -> 81 us (32 / 8 x 64, 256 behind 4000).
+constexpr int64_t kPrefillMinRowBlocks = 256;
+
 int64_t astrai_w8a8_attn_paged_rows_workspace_floats(int64_t batch_or_tiles, int64_t n_heads,
                                                      int64_t n_kv_heads, int64_t head_dim,
                                                      int64_t nsplit, int prefill) {
@@ -610,6 +654,21 @@ int astrai_w8a8_attn_paged_rows_bf16(
     if (need > 0 && workspace_floats < need)
         return fail(ASTRAI_W8A8_BAD_ARG, "attn_paged_rows_bf16: workspace too small (%lld floats needed)",
                     (long long)need);
+    if (prefill && !mask && w8a8::attn_prefill_split_supported((int)n_heads, (int)n_kv_heads, (int)head_dim) &&
+        num_slots * n_kv_heads * head_dim * 2 < ((int64_t)1 << 32) &&
+        (nsplit == 1 || batch_or_tiles * n_heads >= kPrefillMinRowBlocks)) {
+        w8a8::AttnPrefillArgs p{};
+        p.q = q; p.k_cache = k_pool; p.v_cache = v_pool; p.out = out;
+        p.n_heads = (int)n_heads; p.n_kv_heads = (int)n_kv_heads; p.head_dim = (int)head_dim; p.scale = scale;
+        p.req_to_token = req_to_token; p.req_pool_indices = req_pool_indices;
+        p.kv_indptr = kv_indptr; p.qo_indptr = qo_indptr;
+        p.q_tile_to_batch = q_tile_to_batch; p.q_tile_to_index = q_tile_to_index;
+        p.num_q_tiles = (int)batch_or_tiles; p.causal = causal ? 1 : 0;
+        p.rtt_stride = max_context_len; p.num_slots = num_slots; p.num_requests = num_requests;
+        if (!w8a8::launch_attn_prefill(p, static_cast<hipStream_t>(stream)))
+            return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_paged_rows_bf16: shape not supported");
+        return check_launch("attn_paged_rows_bf16");
+    }
     w8a8::AttnRowsArgs a{};
     a.q = q; a.k_cache = k_pool; a.v_cache = v_pool; a.req_to_token = req_to_token;
     a.req_pool_indices = req_pool_indices; a.kv_indptr = kv_indptr; a.qo_indptr = qo_indptr;

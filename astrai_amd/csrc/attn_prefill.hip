@@ -1,5 +1,6 @@
-// Causal grouped-query attention of a block of new tokens against the dense bf16
-// KV cache (prefill, chunked or whole), head_dim 128, bf16 MFMAs, fp32 softmax.
+// Causal grouped-query attention of a block of new tokens (prefill, chunked or whole), head_dim
+// 128 or 64, bf16 MFMAs, fp32 softmax: against the dense bf16 KV cache, against key / value tensors
+// of any row, head and batch stride, or against a pool behind a slot table.
 //
 // The reference expands the KV heads and calls SDPA on [batch, heads, seq, head_dim]
 // tensors with a mask tensor (astrai/extension/backend/attention.py:244-253,443-498,
@@ -9,8 +10,8 @@
 // and the output is written token-major [batch, seq, heads*head_dim], the layout the
 // output projection reads.
 //
-// One workgroup per (batch, KV head, 32 query tokens); wave r takes query head
-// hk*n_rep + r. Keys are handled in 32-key tiles:
+// One workgroup per (batch, KV head, 32 * QSUB query tokens); wave r takes query head
+// hk*n_rep + r % n_rep and the 32 tokens r / n_rep of the block. Keys are handled in 32-key tiles:
 //   S^T = K.Q^T on v_mfma_f32_32x32x16_bf16 with keys as rows and queries as columns,
 //     so a lane owns ONE query (column lane%32) and 16 of a tile's 32 scores: row maxima
 //     and sums are per-lane reductions plus one exchange with lane^32;
@@ -18,13 +19,15 @@
 //     rounded to bf16 in place (its register order fixes which 8 keys a lane half
 //     contributes per 16-key step), and the V^T operand is read out of the row-major
 //     value tile with ds_read_b64_tr_b16, the LDS read that hands each lane of a
-//     16-lane group four values down a column (four keys of one dim);
-//   keys and values sit in LDS as 256-byte rows of 16-byte chunks XOR-swizzled by row
-//     (keys by row%16 for the 32-row operand reads, values by 4*(row%4) for the
-//     transposing reads, which touch four consecutive rows at a time).
+//     16-lane group four values down a column (four keys of one dim). SPLIT instances (the
+//     shapes that attn_rows.hip would take otherwise, whose probabilities have 16 bits of
+//     mantissa) enter P as a bf16 head and a bf16 remainder, two MFMAs;
+//   keys and values sit in LDS as rows of 16-byte chunks XOR-swizzled by row so that the 16 rows
+//     a key operand read touches, and the 4 rows a transposing read touches, fall into
+//     different banks.
 // A wave's instruction stream is a software pipeline over tiles, written out and
-// pinned with sched_barrier: the eight score MFMAs of tile T+1 are interleaved with
-// the exponentials of tile T, and the eight P.V MFMAs of tile T with the masking and
+// pinned with sched_barrier: the score MFMAs of tile T+1 are interleaved with
+// the exponentials of tile T, and the P.V MFMAs of tile T with the masking and
 // row maximum of tile T+1, so the matrix pipe and the vector ALU work at the same
 // time inside one wave (a wave issues in order: a softmax phase between two MFMA
 // phases leaves each unit idle while the other runs). Keys and values arrive by
@@ -32,6 +35,20 @@
 // both one 64-key block ahead; one workgroup barrier per block; no staging registers. Tiles that every
 // query of the wave sees whole skip the masking code; the accumulators are rescaled
 // only when a row maximum has outgrown the reference maximum by 2^8.
+//
+// The direct-to-LDS loads are written in assembly (they have no output register): behind the
+// builtin the compiler orders every transposing read after all loads in flight (s_waitcnt vmcnt(0)),
+// which puts a whole memory round trip into each 64-key block. The blocks without and with masking
+// are two loops, not two branches of one: at a join of the two the compiler moved all accumulators
+// from one register set to another on every block.
+// What bounds it: the vector ALU and the matrix pipe about equally (16 exponentials and ~65 other
+// vector instructions per lane beside 16 MFMAs of 32 cycles a tile, two waves per SIMD). Measured (graph
+// replays, before -> after the two points above, the backward walk and reading strided tensors in place):
+// 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 148 -> 80 us (860 TFLOP/s; before it
+// went through the paged form), ragged 16 x 175..700 tokens of 32/8 heads x 64 in a pool 173 -> 77 us
+// (450 TFLOP/s, P in two terms; before on the general kernel). 192 / 135 registers where the joined
+// loops took 256 with spills: two / three workgroups per CU.
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -45,74 +62,102 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kD = 128;    // head_dim
-constexpr int kQB = 32;    // query tokens per workgroup
-constexpr int kKB = 64;    // keys per block
-constexpr int kKRow = 256;                 // bytes per key row in LDS
-constexpr int kKTileBytes = 32 * kKRow;    // 8 KiB: one 32-key tile
-constexpr int kKRingBytes = 4 * kKTileBytes;
-constexpr int kVBytes = kKB * kKRow;        // 16 KiB: 64 value rows
-constexpr float kNegBig = -1e30f;          // finite stand-in for -inf: no inf - inf
+constexpr int kKB = 64;            // keys per block
+constexpr float kNegBig = -1e30f;  // finite stand-in for -inf: no inf - inf
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* lds_wave_base,
-                                          uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, voff, soff, 0, 0);
+// A raw buffer descriptor in scalar registers, as lds_dma16's assembly takes it (see make_rsrc).
+__device__ __forceinline__ u32x4 make_desc(const void* p, uint32_t bytes) {
+    const uint64_t addr = (uint64_t)p;
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(addr >> 32) & 0xffffu)),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
 }
 
-// PAGED: the queries are packed [total_q, heads, 128] with per-request row ranges
-// (qo_indptr), the caches are token-granular pools [slots, kv_heads, 128] reached through
+// 16 bytes per lane from the buffer into LDS at lds_addr + 16 * lane (lds_addr the same for the whole
+// wave). Out-of-range lanes write zeros. The caller waits (vmcnt) before the bytes are read.
+// (m0 is a reserved register that nothing else in this file's kernels uses.)
+__device__ __forceinline__ void lds_dma16(u32x4 desc, uint32_t lds_addr, uint32_t voff) {
+    __asm__ volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, 0 offen lds"
+        :
+        : "s"(lds_addr), "v"(voff), "s"(desc)
+        : "memory");
+}
+
+// PAGED: the queries are packed [total_q, heads, D] with per-request row ranges
+// (qo_indptr), the caches are token-granular pools [slots, kv_heads, D] reached through
 // req_to_token, and a 64-row query tile t of the caller's schedule belongs to request
 // q_tile_to_batch[t], rows 64 * q_tile_to_index[t] .. of it (csrc/kernels/attention/
 // paged_prefill.cu:4-34, layout_policies.cuh:67-93,174-232; the schedule is built in
-// astrai/inference/cache/pool.py:219-234). Two workgroups share a tile. Query row i of a
+// astrai/inference/cache/pool.py:219-234). Query row i of a
 // request of q_len rows and kv_len keys sees keys 0 .. kv_len - q_len + i (all of them
-// without the causal flag), so nothing has to be fetched to know the key range.
+// without the causal flag), so nothing has to be fetched to know the key range. Workgroups walk
+// the schedule backwards: a sequence's last tiles see the most keys and start first.
 // MASK (paged only): a bool tensor says, per sequence, (head,) (query row,) and position,
 // what may be attended on top of the causal range (csrc/kernels/attention/mma_utils.cuh:190-199);
 // every tile then takes the masking path.
-template <int NREP, bool PAGED, bool MASK = false>
-__global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_kernel(AttnPrefillArgs a) {
-    constexpr int K_DMA = kKB / 4 / NREP;              // 1 KiB key loads per wave and block
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kKRingBytes + 2 * kVBytes];
+template <int D, int NREP, int QSUB, bool PAGED, bool MASK, bool SPLIT>
+__global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void attn_prefill_kernel(AttnPrefillArgs a) {
+    constexpr int WAVES = NREP * QSUB;
+    constexpr int QB = 32 * QSUB;                 // query tokens per workgroup
+    constexpr int ROW = 2 * D;                    // bytes per key or value row in LDS
+    constexpr int TILE = 32 * ROW;                // one 32-key tile
+    constexpr int RING = 4 * TILE;                // keys
+    constexpr int VBUF = kKB * ROW;               // 64 value rows
+    constexpr int LPR = ROW / 16;                 // 16-byte chunks (lanes of a load) per row
+    constexpr int RPI = 64 / LPR;                 // rows per 1 KiB load
+    constexpr int DMA = kKB / RPI / WAVES;        // loads per wave, tensor and block
+    constexpr int KS = D / 16;                    // score MFMAs per tile
+    constexpr int DT = D / 32;                    // 32-dim output tiles
+    static_assert(DMA >= 1 && (!PAGED || QB <= 64), "shape");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[RING + 2 * VBUF];
+    const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qi = lane & 31, h = lane >> 5;
+    const int rep = wave % NREP, qsub = wave / NREP;
+    // XOR swizzles (in chunks) of key and value rows: see the file comment
+    auto swz_k = [](int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); };
+    auto swz_v = [](int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); };
 
     int hk, rows_total, row0;   // KV head; query rows of the sequence; first row of this block
     int64_t tok0;               // index of row 0 of the sequence in the token-major output
     const uint16_t* qbase;      // row 0 of the sequence, this wave's head
     int64_t q_row_stride;       // elements between consecutive query rows
-    int pq, kmax, pmin;         // this lane's newest visible key; the block's extremes
+    int pq, kmax;               // this lane's newest visible key; the block's newest
     [[maybe_unused]] const int* table = nullptr;
-    [[maybe_unused]] int kv_len = 0, b_dense = 0, seq_index = 0;
+    [[maybe_unused]] int b_dense = 0, seq_index = 0;
+    [[maybe_unused]] int block_pos = -1;  // dense, with positions: that of the block's row `lane`
     if constexpr (PAGED) {
-        const int idx = (int)blockIdx.x;
+        constexpr int SUBS = 64 / QB;  // workgroups that share a tile
+        const int idx = (int)(gridDim.x - 1 - blockIdx.x);
         hk = idx % a.n_kv_heads;
-        const int sub = (idx / a.n_kv_heads) & 1, tile = idx / (2 * a.n_kv_heads);
+        const int sub = (idx / a.n_kv_heads) % SUBS, tile = idx / (SUBS * a.n_kv_heads);
         const int req_i = a.q_tile_to_batch[tile];
         seq_index = req_i;
         const int q_start = a.qo_indptr[req_i];
         rows_total = a.qo_indptr[req_i + 1] - q_start;
-        row0 = a.q_tile_to_index[tile] * 64 + sub * kQB;
-        if (row0 >= rows_total) return;  // the tile's second half lies past the request
+        row0 = a.q_tile_to_index[tile] * 64 + sub * QB;
+        if (row0 >= rows_total) return;  // this part of the tile lies past the request
         const int64_t req = a.req_pool_indices[req_i];
         const bool req_ok = req >= 0 && req < a.num_requests;  // a bad row reads as an empty sequence
-        kv_len = req_ok ? (int)min((int64_t)(a.kv_indptr[req_i + 1] - a.kv_indptr[req_i]), a.rtt_stride) : 0;
+        const int kv_len = req_ok ? (int)min((int64_t)(a.kv_indptr[req_i + 1] - a.kv_indptr[req_i]), a.rtt_stride) : 0;
         table = a.req_to_token + (req_ok ? req : 0) * a.rtt_stride;
         tok0 = q_start;
-        q_row_stride = (int64_t)a.n_heads * kD;
-        qbase = static_cast<const uint16_t*>(a.q) + ((int64_t)q_start * a.n_heads + hk * NREP + wave) * kD;
-        const int last = min(row0 + kQB, rows_total) - 1;
+        q_row_stride = (int64_t)a.n_heads * D;
+        qbase = static_cast<const uint16_t*>(a.q) + ((int64_t)q_start * a.n_heads + hk * NREP + rep) * D;
+        const int last = min(row0 + QB, rows_total) - 1;
         const int shift = a.causal ? kv_len - rows_total : INT_MIN;
-        pq = a.causal ? min(shift + row0 + qi, kv_len - 1) : kv_len - 1;
+        pq = a.causal ? min(shift + row0 + qsub * 32 + qi, kv_len - 1) : kv_len - 1;
         kmax = a.causal ? min(shift + last, kv_len - 1) : kv_len - 1;
-        pmin = a.causal ? min(shift + row0, kv_len - 1) : kv_len - 1;
     } else {
-        const int nqb = (a.seq + kQB - 1) / kQB;
+        const int nqb = (a.seq + QB - 1) / QB;
         const int groups = a.batch * a.n_kv_heads;
         const int qb = nqb - 1 - (int)(blockIdx.x / groups);  // longest key ranges first
         const int bk = (int)(blockIdx.x % groups);
@@ -120,17 +165,25 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
         b_dense = b;
         hk = bk % a.n_kv_heads;
         rows_total = a.seq;
-        row0 = qb * kQB;
+        row0 = qb * QB;
         tok0 = (int64_t)b * a.seq;
-        q_row_stride = kD;
-        qbase = static_cast<const uint16_t*>(a.q) + ((int64_t)b * a.n_heads + hk * NREP + wave) * a.seq * kD;
-        // The position is requested first and looked at last: the query rows and the first
-        // key tiles do not depend on it.
-        pq = row0 + qi < a.seq ? (int)a.positions[row0 + qi] : -1;
-        kmax = pmin = 0;
+        q_row_stride = a.q_stride.row;
+        qbase = static_cast<const uint16_t*>(a.q) + b * a.q_stride.batch + (hk * NREP + rep) * a.q_stride.head;
+        kmax = 0;
+        if (a.positions) {
+            // The positions are requested first and looked at last: the query rows and the first
+            // key tiles do not depend on them. (Blocks of up to 64 rows: launch_attn_prefill.)
+            block_pos = lane < QB && row0 + lane < a.seq ? (int)a.positions[row0 + lane] : -1;
+            pq = -1;
+        } else {
+            const int last = min(row0 + QB, rows_total) - 1;
+            const int newest = (int)a.max_len - 1;
+            pq = a.causal ? min(a.causal_offset + row0 + qsub * 32 + qi, newest) : newest;
+            kmax = a.causal ? min(a.causal_offset + last, newest) : newest;
+        }
     }
-    const int head = hk * NREP + wave;
-    const int s_row = row0 + qi;
+    const int head = hk * NREP + rep;
+    const int s_row = row0 + qsub * 32 + qi;
     const bool row_live = s_row < rows_total;
     // this lane's row of the mask and how many of its positions the mask covers (none for a
     // query row the mask has no row for: nothing is read there and nothing attended)
@@ -144,28 +197,29 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
     }
 
     const uint16_t* qrow = qbase + (int64_t)min(s_row, rows_total - 1) * q_row_stride;
-    u32x4 qf[8];
+    u32x4 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qrow + ks * 16 + h * 8);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qrow + ks * 16 + h * 8);
 
-    // keys: straight from the cache into LDS, 1 KiB (four rows) per instruction; lane l
-    // lands at row l/16, chunk position l%16 and therefore asks for chunk (l%16) ^ (row%16).
-    // Dense cache: the descriptor covers the whole row range of this (batch, KV head):
+    // keys: straight from memory into LDS, 1 KiB (RPI rows) per instruction; lane l
+    // lands at row l / LPR, chunk position l % LPR and therefore asks for that chunk ^ swizzle(row).
+    // Dense: the descriptor covers the whole row range of this (batch, KV head):
     // whatever a row past the newest position holds, its scores are replaced (not scaled)
     // by the mask. Paged: the descriptor covers the pool and each lane looks up the slot of
     // its row; rows past the sequence ask for an offset outside it and arrive as zeros.
-    const int64_t pool_row = (int64_t)a.n_kv_heads * kKRow;  // bytes from one slot to the next
-    const size_t cache_off = PAGED ? (size_t)hk * kD
-                                   : ((size_t)b_dense * a.n_kv_heads + hk) * (size_t)a.max_len * kD;
-    const uint16_t* kc = static_cast<const uint16_t*>(a.k_cache) + cache_off;
-    const uint16_t* vc = static_cast<const uint16_t*>(a.v_cache) + cache_off;
-    const uint32_t pool_bytes = PAGED ? (uint32_t)(a.num_slots * pool_row - hk * kKRow) : 0u;
-    const __amdgpu_buffer_rsrc_t rk = make_rsrc(kc, PAGED ? pool_bytes : (uint32_t)a.max_len * (uint32_t)kKRow);
+    const uint32_t k_row = PAGED ? (uint32_t)a.n_kv_heads * ROW : (uint32_t)(a.k_stride.row * 2);  // bytes from row to row
+    const uint32_t v_row = PAGED ? k_row : (uint32_t)(a.v_stride.row * 2);
+    const uint16_t* kc = static_cast<const uint16_t*>(a.k_cache) +
+                         (PAGED ? (int64_t)hk * D : b_dense * a.k_stride.batch + hk * a.k_stride.head);
+    const uint16_t* vc = static_cast<const uint16_t*>(a.v_cache) +
+                         (PAGED ? (int64_t)hk * D : b_dense * a.v_stride.batch + hk * a.v_stride.head);
+    const uint32_t pool_bytes = PAGED ? (uint32_t)(a.num_slots * k_row - hk * ROW) : 0u;
+    const u32x4 rk = make_desc(kc, PAGED ? pool_bytes : (uint32_t)(a.max_len - 1) * k_row + ROW);
     // Paged: one load per wave fetches the slots of all rows its next loads cover (lane l <
     // RPW: this wave's l-th key row; the next RPW lanes: its value rows); the loads take each
     // row's slot from the lane that holds it. Looked up one block ahead, so that the table
     // access is not a second memory round trip in front of every load.
-    constexpr int RPW = 4 * K_DMA;  // rows of a 64-row block that this wave loads
+    constexpr int RPW = RPI * DMA;  // rows of a 64-row block that this wave loads
     auto lookup = [&](int t0, int kbv) -> int {
         const int l = lane & (2 * RPW - 1);  // (lanes past 2 RPW repeat the pattern, unused)
         const int key = l < RPW ? t0 * 32 + wave * RPW + l : kbv * kKB + wave * RPW + (l - RPW);
@@ -174,25 +228,25 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
     };
     auto paged_off = [&](int slots, int src_lane, int swz) -> uint32_t {
         const int slot = __builtin_amdgcn_ds_bpermute(src_lane << 2, slots);
-        return slot >= 0 ? (uint32_t)(slot * pool_row) + (uint32_t)(((lane & 15) ^ swz) << 4) : kOutOfRange;
+        return slot >= 0 ? (uint32_t)slot * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz) << 4) : kOutOfRange;
     };
-    [[maybe_unused]] uint32_t k_voff[K_DMA];
+    [[maybe_unused]] uint32_t k_voff[DMA];
     if constexpr (!PAGED) {
 #pragma unroll
-        for (int j = 0; j < K_DMA; ++j) {
-            const int row = (wave * K_DMA + j) * 4 + (lane >> 4);
-            k_voff[j] = (uint32_t)row * kKRow + (uint32_t)(((lane & 15) ^ (row & 15)) << 4);
+        for (int j = 0; j < DMA; ++j) {
+            const int row = (wave * DMA + j) * RPI + lane / LPR;
+            k_voff[j] = (uint32_t)row * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz_k(row)) << 4);
         }
     }
     // tiles t0 and t0+1 (64 keys) into their ring slots
     auto dma_k = [&](int t0, [[maybe_unused]] int slots) {
 #pragma unroll
-        for (int j = 0; j < K_DMA; ++j) {
-            const int inst = wave * K_DMA + j;  // 16 instructions of 4 rows; 8 per tile
-            const int row = inst * 4 + (lane >> 4);
-            const uint32_t off = PAGED ? paged_off(slots, j * 4 + (lane >> 4), row & 15)
-                                       : k_voff[j] + (uint32_t)t0 * kKTileBytes;
-            lds_dma16(rk, lds + ((t0 + (inst >> 3)) & 3) * kKTileBytes + (inst & 7) * 4 * kKRow, off, 0);
+        for (int j = 0; j < DMA; ++j) {
+            const int inst = wave * DMA + j;  // 64 / RPI instructions; half of them per tile
+            const uint32_t off = PAGED ? paged_off(slots, j * RPI + lane / LPR, swz_k(inst * RPI + lane / LPR))
+                                       : k_voff[j] + (uint32_t)(t0 * 32) * k_row;
+            const int tile_inst = 32 / RPI;
+            lds_dma16(rk, lds0 + ((t0 + inst / tile_inst) & 3) * TILE + (inst % tile_inst) * 1024, off);
         }
     };
     [[maybe_unused]] int slots = 0;
@@ -205,84 +259,100 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
     dma_k(1, slots);
 
     if constexpr (!PAGED) {
-        // what the block's queries may see
-        kmax = pq;
-        pmin = row_live ? pq : INT_MAX;
+        if (a.positions) {
+            block_pos = min(block_pos, (int)a.max_len - 1);  // (a token past the cache sees what it holds)
+            pq = __shfl(block_pos, qsub * 32 + qi, kWave);
+            // what the block's queries may see: every lane ends up with the same value
+            kmax = block_pos;
 #pragma unroll
-        for (int off = 16; off; off >>= 1) {
-            kmax = max(kmax, __shfl_xor(kmax, off, kWave));
-            pmin = min(pmin, __shfl_xor(pmin, off, kWave));
+            for (int off = 32; off; off >>= 1) kmax = max(kmax, __shfl_xor(kmax, off, kWave));
         }
-        // every lane holds the same extremes by now: keep them in scalar registers (loop
-        // bounds, the value descriptor's size)
-        kmax = min(__builtin_amdgcn_readfirstlane(kmax), (int)a.max_len - 1);
-        pmin = __builtin_amdgcn_readfirstlane(pmin);
+        kmax = __builtin_amdgcn_readfirstlane(kmax);
     }
+    // what this wave's queries see: all of them up to pmin, none past kmax_w (equal to kmax with one
+    // group of 32 tokens per workgroup)
+    int pmin = row_live ? pq : 1 << 30, kmax_w = row_live ? pq : -1;
+#pragma unroll
+    for (int off = 16; off; off >>= 1) {
+        pmin = min(pmin, __shfl_xor(pmin, off, kWave));
+        kmax_w = max(kmax_w, __shfl_xor(kmax_w, off, kWave));
+    }
+    pmin = __builtin_amdgcn_readfirstlane(pmin);
+    kmax_w = __builtin_amdgcn_readfirstlane(min(kmax_w, kmax));
     const bool sees_a_key = pq >= 0;
-    if (!row_live) pq = kmax;  // rows past the end see everything and are never stored
-    const int nkb = kmax / kKB + 1;  // (kmax = -1, an empty sequence: one block of masked keys)
+    if (!row_live) pq = kmax_w;  // rows past the end see everything and are never stored
+    const int nkb = kmax / kKB + 1;     // (kmax = -1, an empty sequence: one block of masked keys)
+    const int tiles_w = kmax_w / 32 + 1;  // tiles this wave computes
 
-    // values: the same way into a 64-row buffer; chunk position (l%16) holds chunk
-    // (l%16) ^ 4*(row%4). Rows past kmax arrive as zeros, so a stale cache row can never
-    // meet a zero probability as 0 * NaN.
-    const __amdgpu_buffer_rsrc_t rv = make_rsrc(vc, PAGED ? pool_bytes : (uint32_t)(kmax + 1) * (uint32_t)kKRow);
-    [[maybe_unused]] uint32_t v_voff[K_DMA];
+    // values: the same way into a 64-row buffer. Rows past kmax arrive as zeros, so a stale cache
+    // row can never meet a zero probability as 0 * NaN.
+    const u32x4 rv = make_desc(vc, PAGED ? pool_bytes : kmax >= 0 ? (uint32_t)kmax * v_row + ROW : 0u);
+    [[maybe_unused]] uint32_t v_voff[DMA];
     if constexpr (!PAGED) {
 #pragma unroll
-        for (int j = 0; j < K_DMA; ++j) {
-            const int row = (wave * K_DMA + j) * 4 + (lane >> 4);
-            v_voff[j] = (uint32_t)row * kKRow + (uint32_t)(((lane & 15) ^ (4 * (row & 3))) << 4);
+        for (int j = 0; j < DMA; ++j) {
+            const int row = (wave * DMA + j) * RPI + lane / LPR;
+            v_voff[j] = (uint32_t)row * v_row + (uint32_t)(((lane & (LPR - 1)) ^ swz_v(row)) << 4);
         }
     }
     auto dma_v = [&](int kb, [[maybe_unused]] int slots) {
 #pragma unroll
-        for (int j = 0; j < K_DMA; ++j) {
-            const int row = (wave * K_DMA + j) * 4 + (lane >> 4);
-            const uint32_t off = PAGED ? paged_off(slots, RPW + j * 4 + (lane >> 4), 4 * (row & 3))
-                                       : v_voff[j] + (uint32_t)kb * kVBytes;
-            lds_dma16(rv, lds + kKRingBytes + (kb & 1) * kVBytes + (wave * K_DMA + j) * 4 * kKRow, off, 0);
+        for (int j = 0; j < DMA; ++j) {
+            const int inst = wave * DMA + j;
+            const uint32_t off = PAGED ? paged_off(slots, RPW + j * RPI + lane / LPR, swz_v(inst * RPI + lane / LPR))
+                                       : v_voff[j] + (uint32_t)(kb * kKB) * v_row;
+            lds_dma16(rv, lds0 + RING + (kb & 1) * VBUF + inst * 1024, off);
         }
     };
 
-    f32x16 o[4];
+    f32x16 o[DT];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
     // m_run is the reference maximum the probabilities are taken against, in log2 units.
     // It follows the true running maximum lazily: only when some query of the wave has
-    // outgrown it by more than kSlack does the wave pay for rescaling its 64 accumulators;
+    // outgrown it by more than kSlack does the wave pay for rescaling its accumulators;
     // until then probabilities may reach 2^kSlack, which fp32 sums and bf16 operands hold.
     constexpr float kSlack = 8.0f;
     float m_run = kNegBig, l_run = 0.0f;
     const float c = a.scale * 1.44269504088896340736f;  // scores to log2 units
     const f32x16 zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    // byte offset of this lane's k-step 0 key chunk inside a tile, and of its V^T row
-    const int k_lane = qi * kKRow;
     // V^T operand of 32 dims x 16 keys: two transposing reads. In each 16-lane group, lane
     // 4j+q points at row j, dims 4q..4q+3 of a 4-row x 16-dim patch and receives dim (its
     // index in the group) of rows 0..3. Lane half h takes rows 4h..4h+3 and 8+4h..8+4h+3 of
     // the 16-key step: the keys its P^T registers hold (register 4g+j = key 8g + 4h + j).
-    // (bits 6-7 of the offset are dt ^ j: the dim tile is XORed into the offset as well)
+    // (the swizzle leaves the chunk bits of the dim tile free: it is XORed into the offset as well)
     const int v_lane0 = [&] {
         const int sl = lane & 15, j = sl >> 2, q = sl & 3, g1 = (lane >> 4) & 1;
-        return (4 * h + j) * kKRow + ((((2 * g1 + (q >> 1)) ^ (4 * j)) << 4) | ((q & 1) << 3));
+        return (4 * h + j) * ROW + ((((2 * g1 + (q >> 1)) ^ swz_v(j)) << 4) | ((q & 1) << 3));
     }();
-    // key operand of k-step ks: chunk (2ks + h) ^ (row % 16) of this lane's row. The tile
-    // offset and the row offset are multiples of 256, so the k-step can be XORed into the
-    // whole byte offset: one address register per tile instead of eight.
-    const int k_lane0 = k_lane + ((h ^ (qi & 15)) << 4);
+    // key operand of k-step ks: chunk (2ks + h) ^ swizzle(row) of this lane's row. The tile
+    // offset and the row offset are multiples of the row size, so the k-step can be XORed into the
+    // whole byte offset: one address register per tile instead of one per k-step.
+    const int k_lane0 = qi * ROW + ((h ^ swz_k(qi)) << 4);
     auto k_frag = [&](int tile_off, int ks) -> u32x4 {
         return *reinterpret_cast<const u32x4*>(lds + ((tile_off + k_lane0) ^ (ks << 5)));
     };
-    auto v_frag = [&](int vt_off, int t, int dt) -> u32x4 {
+    // T0: first key of the tile; PARTIAL with several token groups per workgroup: rows past this
+    // wave's newest key are other queries' keys and are replaced by zeros (their probabilities here
+    // are zero, and 0 * NaN would not be)
+    auto v_frag = [&](auto mask_tag, int T0, int vt_off, int t, int dt) -> u32x4 {
         typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-        const uint8_t* src = lds + ((vt_off + v_lane0) ^ (dt << 6)) + t * 16 * kKRow;
+        const uint8_t* src = lds + ((vt_off + v_lane0) ^ (dt << 6)) + t * 16 * ROW;
         const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
-        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * kKRow));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * ROW));
         const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-        return u32x4{l2.x, l2.y, h2.x, h2.y};
+        u32x4 v = {l2.x, l2.y, h2.x, h2.y};
+        if constexpr (QSUB > 1 && decltype(mask_tag)::value) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int key = T0 + t * 16 + (w >> 1) * 8 + 4 * h + 2 * (w & 1);
+                v[w] &= (key <= kmax_w ? 0xffffu : 0u) | (key < kmax_w ? 0xffff0000u : 0u);
+            }
+        }
+        return v;
     };
     // masking and this lane's share of the row maximum of tile T (raw scores; c > 0 keeps order)
     auto mask_max4 = [&](auto mask_tag, int T, f32x16& s, int g, float m) -> float {
@@ -317,61 +387,74 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
             m_run = m_new;
             l_run *= alpha;
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
         }
-        const int kt = ((T + 1) & 3) * kKTileBytes;
+        const int kt = ((T + 1) & 3) * TILE;
+        constexpr int NV = 2 * DT;                 // value operands of a tile
+        constexpr int NM = NV * (SPLIT ? 2 : 1);   // P.V MFMAs
+        constexpr int EPK = 8 / KS;                // score pairs per score MFMA
         uint32_t pk[8];
+        [[maybe_unused]] uint32_t pr[8];
         float l_add = 0.0f;
-        u32x4 kf[8], vf[8];
+        u32x4 kf[KS], vf[NV];
         kf[0] = k_frag(kt, 0);
         kf[1] = k_frag(kt, 1);
         __builtin_amdgcn_sched_barrier(0);
-        // ---- eight score MFMAs of tile T+1, each followed by two exponentials of tile T
+        // ---- the score MFMAs of tile T+1, each followed by exponentials of tile T
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            if (ks + 2 < 8) kf[ks + 2] = k_frag(kt, ks + 2);
-            if (ks >= 6) vf[ks - 6] = v_frag(vt, 0, ks - 6);
+        for (int ks = 0; ks < KS; ++ks) {
+            if (ks + 2 < KS) kf[ks + 2] = k_frag(kt, ks + 2);
+            if (ks >= KS - 2) vf[ks - (KS - 2)] = v_frag(mask_tag, T * 32, vt, 0, ks - (KS - 2));
             s_out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8, kf[ks]), __builtin_bit_cast(bf16x8, qf[ks]),
                 ks == 0 ? zero16 : s_out, 0, 0, 0);
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * ks], c, -m_run));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * ks + 1], c, -m_run));
-            l_add += p0 + p1;
-            pk[ks] = pack_bf16x2(p0, p1);
+#pragma unroll
+            for (int u = 0; u < EPK; ++u) {
+                const int i = ks * EPK + u;
+                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * i], c, -m_run));
+                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * i + 1], c, -m_run));
+                l_add += p0 + p1;
+                pk[i] = pack_bf16x2(p0, p1);
+                if constexpr (SPLIT)
+                    pr[i] = pack_bf16x2(p0 - __uint_as_float(pk[i] << 16), p1 - __uint_as_float(pk[i] & 0xffff0000u));
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         l_run += l_add;
-        // ---- eight P.V MFMAs of tile T, the later ones followed by the maximum of tile T+1
+        // ---- the P.V MFMAs of tile T, the last ones followed by the maximum of tile T+1
         float m = kNegBig;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int t = i >> 2, dt = i & 3;
-            if (i + 2 < 8) vf[i + 2] = v_frag(vt, (i + 2) >> 2, (i + 2) & 3);
-            const u32x4 pf = {pk[4 * t], pk[4 * t + 1], pk[4 * t + 2], pk[4 * t + 3]};
+        for (int n = 0; n < NM; ++n) {
+            const int i = SPLIT ? n >> 1 : n, t = i / DT, dt = i % DT;
+            if ((!SPLIT || (n & 1) == 0) && i + 2 < NV)
+                vf[i + 2] = v_frag(mask_tag, T * 32, vt, (i + 2) / DT, (i + 2) % DT);
+            u32x4 pf = {pk[4 * t], pk[4 * t + 1], pk[4 * t + 2], pk[4 * t + 3]};
+            if constexpr (SPLIT)
+                if (n & 1) pf = u32x4{pr[4 * t], pr[4 * t + 1], pr[4 * t + 2], pr[4 * t + 3]};
             o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8, vf[i]), __builtin_bit_cast(bf16x8, pf), o[dt], 0, 0, 0);
-            if (i >= 4) m = mask_max4(mask_tag, T + 1, s_out, i - 4, m);
+            if (n >= NM - 4) m = mask_max4(mask_tag, T + 1, s_out, n - (NM - 4), m);
             __builtin_amdgcn_sched_barrier(0);
         }
         m_out = fmaxf(m, __shfl_xor(m, 32, kWave));
     };
 
     // ---- prologue: tiles 0..2 and the first value block; scores of tile 0
-    const int tfull = (__builtin_amdgcn_readfirstlane(pmin) + 1) / 32;  // tiles every query sees whole
-    const int nfast = MASK ? 0 : max(tfull - 1, 0) / 2;  // blocks whose steps only produce unmasked tiles
+    const int tfull = (pmin + 1) / 32;  // tiles every query of the wave sees whole
+    const int nfast = MASK ? 0 : min(max(tfull - 1, 0), tiles_w) / 2;  // blocks whose steps only produce unmasked tiles
     dma_v(0, slots);
     if constexpr (PAGED) slots = lookup(3, 1);  // what the first block's loads will ask for
     // tile 0 needs the queries and the key tiles, not the values: wait for everything but
-    // this wave's K_DMA value loads (the newest), which get the scores of tile 0 to land
-    __builtin_amdgcn_s_waitcnt(0x0f70 | K_DMA);  // vmcnt(K_DMA)
+    // this wave's DMA value loads (the newest), which get the scores of tile 0 to land
+    __builtin_amdgcn_s_waitcnt(0x0f70 | DMA);  // vmcnt(DMA)
     __syncthreads();
     f32x16 sa, sb;
     float ma, mb;
     {
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
             sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8, k_frag(0, ks)), __builtin_bit_cast(bf16x8, qf[ks]),
                 ks == 0 ? zero16 : sa, 0, 0, 0);
@@ -382,97 +465,147 @@ __global__ __launch_bounds__(64 * NREP, NREP >= 4 ? 2 : 1) void attn_prefill_ker
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __syncthreads();  // values landed; tile 0's ring slot is overwritten by the first block's loads
-    for (int kb = 0; kb < nkb; ++kb) {
-        const int cur = kb & 1;
+    auto begin_block = [&](int kb) {
         dma_k(2 * kb + 3, slots);  // tiles 2kb+3, 2kb+4: their ring slots held tiles 2kb-1 and 2kb
         if (kb + 1 < nkb) dma_v(kb + 1, slots);
         if constexpr (PAGED) slots = lookup(2 * kb + 5, kb + 2);  // for the next block's loads
-        const int vt = kKRingBytes + cur * kVBytes;
-        if (kb < nfast) {
-            step(std::false_type{}, 2 * kb, sa, ma, sb, mb, vt);
-            step(std::false_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + 32 * kKRow);
-        } else {
-            step(std::true_type{}, 2 * kb, sa, ma, sb, mb, vt);
-            step(std::true_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + 32 * kKRow);
-        }
+    };
+    auto end_block = [&] {
         __builtin_amdgcn_s_waitcnt(0x0070);
         __syncthreads();
+    };
+    int kb = 0;
+    for (; kb < nfast; ++kb) {
+        begin_block(kb);
+        const int vt = RING + (kb & 1) * VBUF;
+        step(std::false_type{}, 2 * kb, sa, ma, sb, mb, vt);
+        step(std::false_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + TILE);
+        end_block();
     }
-    // ---- normalise and write [batch, seq, heads*128]: through this wave's quarter of the
-    // (now idle) key ring, so that the 32 x 128 tile leaves as whole 256-byte rows
+    for (; kb < tiles_w / 2; ++kb) {
+        begin_block(kb);
+        const int vt = RING + (kb & 1) * VBUF;
+        step(std::true_type{}, 2 * kb, sa, ma, sb, mb, vt);
+        step(std::true_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + TILE);
+        end_block();
+    }
+    if (tiles_w & 1) {  // a last block of one tile
+        begin_block(kb);
+        step(std::true_type{}, 2 * kb, sa, ma, sb, mb, RING + (kb & 1) * VBUF);
+        end_block();
+        ++kb;
+    }
+    for (; kb < nkb; ++kb) {  // keys that only later tokens of the workgroup see
+        begin_block(kb);
+        end_block();
+    }
+    // ---- normalise and write [batch, seq, heads*D]: through this wave's part of the
+    // (now idle) LDS, so that the 32 x D tile leaves as whole rows
     l_run += __shfl_xor(l_run, 32, kWave);
     // a row that sees no key at all (empty sequence, or more queries than keys) yields zeros
     // (with a mask tensor a row may have met nothing but masked scores: its reference maximum
     // then still is the stand-in for -inf, times c once it has been through a rescale)
     const bool met_a_key = !MASK || m_run > 0.5f * kNegBig * fminf(c, 1.0f);
-    const float inv = (l_run > 0.0f && sees_a_key && met_a_key) ? 1.0f / l_run : 0.0f;
-    {
-        uint8_t* const mine = lds + wave * kKTileBytes;
+    const bool has_value = l_run > 0.0f && sees_a_key && met_a_key;
+    const float inv = has_value ? 1.0f / l_run : 0.0f;
+    // (its accumulators hold whatever masked scores made of them: the difference of two roundings of
+    // c * kNegBig may be large enough for an infinite probability)
+    if (!has_value) {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
+    }
+    {
+        uint8_t* const mine = lds + wave * TILE;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 u32x2 w;
                 w.x = pack_bf16x2(o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv);
                 w.y = pack_bf16x2(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
                 // row qi, dims 32dt + 8g + 4h ..+3: chunk 4dt+g (XOR-swizzled by row), half h
-                *reinterpret_cast<u32x2*>(mine + qi * kKRow + (((4 * dt + g) ^ (qi & 15)) << 4) + h * 8) = w;
+                *reinterpret_cast<u32x2*>(mine + qi * ROW + (((4 * dt + g) ^ (qi & (LPR - 1))) << 4) + h * 8) = w;
             }
-        uint16_t* const obase = static_cast<uint16_t*>(a.out) + ((tok0 + row0) * a.n_heads + head) * kD;
-        const int r4 = lane >> 4, c16 = lane & 15;
+        const int first = row0 + qsub * 32;
+        uint16_t* const obase = static_cast<uint16_t*>(a.out) + ((tok0 + first) * a.n_heads + head) * D;
+        const int r = lane / LPR, ch = lane & (LPR - 1);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int row = i * 4 + r4;
-            const u32x4 v = *reinterpret_cast<const u32x4*>(mine + row * kKRow + ((c16 ^ (row & 15)) << 4));
-            if (row0 + row < rows_total)
-                *reinterpret_cast<u32x4*>(obase + (size_t)row * a.n_heads * kD + c16 * 8) = v;
+        for (int i = 0; i < 32 / RPI; ++i) {
+            const int row = i * RPI + r;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(mine + row * ROW + ((ch ^ (row & (LPR - 1))) << 4));
+            if (first + row < rows_total)
+                *reinterpret_cast<u32x4*>(obase + (size_t)row * a.n_heads * D + ch * 8) = v;
         }
     }
+}
+
+template <int D, int NREP, int QSUB, bool SPLIT>
+bool launch_shape(const AttnPrefillArgs& a, hipStream_t stream) {
+    // tokens per workgroup: a schedule tile has 64 rows, and the kernel reads the positions of 64
+    constexpr int QP = 32 * QSUB <= 64 ? QSUB : 2;
+    const bool paged = a.req_to_token != nullptr, narrow = paged || a.positions;
+    const int rows = 32 * (narrow ? QP : QSUB);
+    const int64_t wgs = paged ? (int64_t)a.num_q_tiles * (64 / rows) * a.n_kv_heads
+                              : (int64_t)((a.seq + rows - 1) / rows) * a.batch * a.n_kv_heads;
+    if (wgs > INT_MAX) return false;
+    const dim3 grid((unsigned)wgs), block(64 * NREP * (narrow ? QP : QSUB));
+    if (paged && a.mask) {
+        if constexpr (!SPLIT)
+            attn_prefill_kernel<D, NREP, QP, true, true, SPLIT><<<grid, block, 0, stream>>>(a);
+        else
+            return false;
+    } else if (paged) {
+        attn_prefill_kernel<D, NREP, QP, true, false, SPLIT><<<grid, block, 0, stream>>>(a);
+    } else if (narrow) {
+        attn_prefill_kernel<D, NREP, QP, false, false, SPLIT><<<grid, block, 0, stream>>>(a);
+    } else {
+        attn_prefill_kernel<D, NREP, QSUB, false, false, SPLIT><<<grid, block, 0, stream>>>(a);
+    }
+    return true;
 }
 
 }  // namespace
 
 bool attn_prefill_supported(int n_heads, int n_kv_heads, int head_dim) {
-    if (head_dim != kD || n_kv_heads <= 0 || n_heads % n_kv_heads) return false;
+    if (head_dim != 128 || n_kv_heads <= 0 || n_heads % n_kv_heads) return false;
     const int n_rep = n_heads / n_kv_heads;
     return n_rep == 2 || n_rep == 4 || n_rep == 8;
 }
 
+bool attn_prefill_split_supported(int n_heads, int n_kv_heads, int head_dim) {
+    if (n_kv_heads <= 0 || n_heads % n_kv_heads) return false;
+    const int n_rep = n_heads / n_kv_heads;
+    return head_dim == 64 ? n_rep == 1 || n_rep == 2 || n_rep == 4 || n_rep == 8 : head_dim == 128 && n_rep == 1;
+}
+
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream) {
-    if (!attn_prefill_supported(a.n_heads, a.n_kv_heads, a.head_dim)) return false;
+    const bool split = attn_prefill_split_supported(a.n_heads, a.n_kv_heads, a.head_dim);
+    if (!split && !attn_prefill_supported(a.n_heads, a.n_kv_heads, a.head_dim)) return false;
     const bool paged = a.req_to_token != nullptr;
     if (a.mask && (!paged || a.mask_width <= 0 || a.mask_rows <= 0)) return false;
     const int n_rep = a.n_heads / a.n_kv_heads;
-    int64_t wgs;
+    const int64_t row = 2 * (int64_t)a.head_dim;
     if (paged) {
         if (!a.req_pool_indices || !a.kv_indptr || !a.qo_indptr || !a.q_tile_to_batch || !a.q_tile_to_index ||
             a.num_q_tiles <= 0 || a.rtt_stride <= 0 || a.num_slots <= 0 || a.num_requests <= 0)
             return false;
-        if (a.num_slots * (int64_t)a.n_kv_heads * kKRow >= ((int64_t)1 << 32)) return false;  // 32-bit pool offsets
-        wgs = (int64_t)a.num_q_tiles * 2 * a.n_kv_heads;
+        if (a.num_slots * a.n_kv_heads * row >= ((int64_t)1 << 32)) return false;  // 32-bit pool offsets
     } else {
         if (a.batch <= 0 || a.seq <= 0 || a.max_len <= 0) return false;
-        wgs = (int64_t)((a.seq + kQB - 1) / kQB) * a.batch * a.n_kv_heads;
+        if (a.max_len * std::max(a.k_stride.row, a.v_stride.row) * 2 >= ((int64_t)1 << 32)) return false;  // 32-bit offsets
     }
-    if (wgs > INT_MAX) return false;
-    const dim3 grid((unsigned)wgs);
-#define W8A8_LAUNCH_PREFILL(R)                                                          \
-    do {                                                                                \
-        if (paged && a.mask)                                                            \
-            attn_prefill_kernel<R, true, true><<<grid, dim3(64 * R), 0, stream>>>(a);   \
-        else if (paged)                                                                 \
-            attn_prefill_kernel<R, true><<<grid, dim3(64 * R), 0, stream>>>(a);         \
-        else                                                                            \
-            attn_prefill_kernel<R, false><<<grid, dim3(64 * R), 0, stream>>>(a);        \
-    } while (0)
-    if (n_rep == 2)
-        W8A8_LAUNCH_PREFILL(2);
-    else if (n_rep == 4)
-        W8A8_LAUNCH_PREFILL(4);
-    else
-        W8A8_LAUNCH_PREFILL(8);
-#undef W8A8_LAUNCH_PREFILL
-    return true;
+    if (a.head_dim == 64) {
+        if (n_rep == 1) return launch_shape<64, 1, 4, true>(a, stream);
+        if (n_rep == 2) return launch_shape<64, 2, 2, true>(a, stream);
+        if (n_rep == 4) return launch_shape<64, 4, 1, true>(a, stream);
+        return launch_shape<64, 8, 1, true>(a, stream);
+    }
+    if (n_rep == 1) return launch_shape<128, 1, 4, true>(a, stream);
+    if (n_rep == 2) return launch_shape<128, 2, 2, false>(a, stream);
+    if (n_rep == 4) return launch_shape<128, 4, 1, false>(a, stream);
+    return launch_shape<128, 8, 1, false>(a, stream);
 }
 
 }  // namespace w8a8

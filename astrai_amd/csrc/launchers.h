@@ -144,17 +144,23 @@ bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream);
 
 // attn_prefill.hip: causal grouped-query attention of a block of new tokens against
 // the dense bf16 KV cache; head_dim 128, n_heads / n_kv_heads in {2, 4, 8}
+struct AttnStride {
+    int64_t batch, head, row;  // elements; rows of head_dim consecutive elements, 16-byte aligned
+};
 struct AttnPrefillArgs {
-    const void* q;             // bf16 [batch, n_heads, seq, 128]
-    const void* k_cache;       // bf16 [batch, n_kv_heads, max_len, 128]
-    const void* v_cache;       // same
-    const int64_t* positions;  // int64 [seq]: position of each new token (keys <= it are attended)
-    void* out;                 // bf16 [batch, seq, n_heads * 128]
+    const void* q;             // bf16 [batch, n_heads, seq, head_dim] at q_stride
+    const void* k_cache;       // bf16 [batch, n_kv_heads, max_len, head_dim] at k_stride
+    const void* v_cache;       // same, at v_stride
+    const int64_t* positions;  // int64 [seq]: position of each new token (keys <= it are attended), or null:
+                               // row i sees keys 0 .. causal_offset + i if causal is set, else all max_len
+    void* out;                 // bf16 [batch, seq, n_heads * head_dim]
     int batch, seq, n_heads, n_kv_heads, head_dim;
     int64_t max_len;
     float scale;
-    // paged mode (req_to_token != null): q and out are packed [total_q, n_heads, 128], the
-    // caches are pools [slots, n_kv_heads, 128]; positions, batch, seq and max_len are unused
+    AttnStride q_stride, k_stride, v_stride;
+    int causal_offset;
+    // paged mode (req_to_token != null): q and out are packed [total_q, n_heads, head_dim], the
+    // caches are pools [slots, n_kv_heads, head_dim]; positions, strides, batch, seq and max_len are unused
     const int* req_to_token;      // int32 [requests, rtt_stride]: slot of (request, position)
     const int* req_pool_indices;  // int32 [batch]: row of req_to_token of each sequence
     const int* kv_indptr;         // int32 [batch + 1]: prefix sums of the key counts
@@ -174,6 +180,8 @@ struct AttnPrefillArgs {
     int mask_rows, mask_width;
 };
 bool attn_prefill_supported(int n_heads, int n_kv_heads, int head_dim);
+// the shapes it takes in place of attn_rows.hip (probabilities as two bf16 terms, no mask tensor)
+bool attn_prefill_split_supported(int n_heads, int n_kv_heads, int head_dim);
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream);
 
 // attn_rows.hip: paged attention for every head_dim in {32, 64, 128, 256} and every

@@ -75,6 +75,8 @@ PROTOTYPES = {
          _I64, _I64, _I64, _INT, ctypes.c_float, _P], _INT),
     "astrai_w8a8_attn_prefill_bf16": (
         [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_float, _P], _INT),
+    "astrai_w8a8_attn_prefill_strided_bf16": (
+        [_P, _P, _P, ctypes.POINTER(_I64), _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_float, _P], _INT),
     "astrai_w8a8_attn_decode_bf16": (
         [_P, _P, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_float, _P],
         _INT),
@@ -1575,6 +1577,52 @@ def _token_major(t, layout):
     return (t.transpose(1, 2) if layout == BHLD else t).contiguous()
 
 
+def _strided_view(t, layout):
+    """``(t, (batch, head, row) strides)`` of a 4-D tensor as the strided prompt kernel reads it: in
+    place if rows are consecutive values at 16-byte boundaries, else a contiguous copy."""
+    if t.stride(3) != 1 or t.stride(0) % 8 or t.stride(1) % 8 or t.stride(2) % 8 or t.data_ptr() % 16:
+        t = t.contiguous()
+    s = t.stride()
+    return t, (s[0], s[1], s[2]) if layout == BHLD else (s[0], s[2], s[1])
+
+
+# (tile of 64 query rows, query head) pairs from which the block kernel serves the shapes that the general
+# kernel with its context split serves otherwise (kPrefillMinRowBlocks in csrc/abi.hip, with the figures)
+PREFILL_MIN_ROW_BLOCKS = 256
+
+
+def attn_prefill_strided_takes(batch: int, q_len: int, kv_len: int, n_heads: int, n_kv_heads: int,
+                               head_dim: int) -> bool:
+    """Whether a block without a mask tensor runs :func:`attn_prefill_strided`: always where the block kernel is
+    the only tuned one (:func:`attn_prefill_supported`); for head_dim 64 and for one query head per KV head
+    where the keys are mostly the block's own, or enough blocks fill the chip."""
+    if attn_prefill_supported(n_heads, n_kv_heads, head_dim):
+        return True
+    if n_heads % n_kv_heads or (head_dim, n_heads // n_kv_heads) not in ((64, 1), (64, 2), (64, 4), (64, 8), (128, 1)):
+        return False
+    return kv_len <= 2 * q_len or batch * n_heads * -(-q_len // 64) >= PREFILL_MIN_ROW_BLOCKS
+
+
+def attn_prefill_strided(q, k, v, layout: int, causal_offset: int = -1, positions: Optional[torch.Tensor] = None,
+                         scale: float = 0.0) -> Optional[torch.Tensor]:
+    """Attention of ``q`` against ``k`` / ``v`` (bf16, 4-D in ``layout``) read where they lie; row ``i`` sees keys
+    ``0 .. i + causal_offset`` (all of them below 0), or ``0 .. positions[i]``. Returns ``[batch, q_len, heads,
+    head_dim]``, or None if one head's rows span more than the kernel's 32-bit offsets reach."""
+    lib = _require()
+    l_ax, h_ax = (2, 1) if layout == BHLD else (1, 2)
+    b, q_len, h, d = q.size(0), q.size(l_ax), q.size(h_ax), q.size(3)
+    kv_len, hkv = k.size(l_ax), k.size(h_ax)
+    (q, qs), (k, ks), (v, vs) = _strided_view(q, layout), _strided_view(k, layout), _strided_view(v, layout)
+    if kv_len * max(ks[2], vs[2]) >= 2 ** 31:
+        return None
+    out = torch.empty((b, q_len, h, d), device=q.device, dtype=torch.bfloat16)
+    _check(lib.astrai_w8a8_attn_prefill_strided_bf16(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), (_I64 * 9)(*qs, *ks, *vs), _ptr(positions), out.data_ptr(), b,
+        q_len, kv_len, h, hkv, d, min(causal_offset, kv_len), float(scale if scale and scale > 0.0 else d ** -0.5),
+        _stream(q)), lib)
+    return out
+
+
 def attn_cache_rows_supported(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
     """Head shapes :func:`attn_cache_rows` takes (those of the general paged kernel)."""
     return head_dim in (32, 64, 128, 256) and n_heads % n_kv_heads == 0 and n_heads // n_kv_heads <= 16
@@ -1608,6 +1656,10 @@ def attn_cache_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         raise RuntimeError("attn_cache_rows: the caches must be contiguous [batch, n_kv_heads, max_len, head_dim]")
     n_rep, pairs = h // hkv, b * hkv
     with _on_device(q.device):
+        if s > 1 and attn_prefill_strided_takes(b, s, max_len, h, hkv, d):
+            out = attn_prefill_strided(q, k_cache, v_cache, BHLD, positions=positions.contiguous())
+            if out is not None:
+                return out.view(b, s, h * d)
         table, rows = _identity_paging(pairs, max_len, q.device)
         key = ("ramp", pairs, str(q.device))
         if key not in _index_cache:
@@ -1679,10 +1731,10 @@ def attn_prefill_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Op
     query rows per sequence against ``k`` / ``v`` tensors in either layout; the result has
     ``q``'s layout. ``causal_offset >= 0``: row ``i`` sees keys ``0 .. i + causal_offset``
     (prefill_split_q_mma.cuh:121-124); ``mask`` (bool, True = attend) is ``[batch, kv_len]``,
-    ``[batch, 1 | q_len, kv_len]`` or ``[batch, 1 | heads, 1 | q_len, kv_len]``. Layout 0 without
-    a mask runs the dense-cache kernel in place; the other cases run the ragged paged kernel
-    over the token-major tensors (layout 0 is copied for it); an offset other than
-    ``kv_len - q_len`` is expressed through the mask."""
+    ``[batch, 1 | q_len, kv_len]`` or ``[batch, 1 | heads, 1 | q_len, kv_len]``. Without a
+    mask the block kernel reads the tensors in place (:func:`attn_prefill_strided`); the other cases run the
+    ragged paged kernel over the token-major tensors (layout 0 is copied for it), an offset other than
+    ``kv_len - q_len`` expressed through the mask."""
     b, q_len, kv_len, h, hkv, d = _dense_args(q, k, v, layout, "attn_prefill")
     m4 = _dense_mask(mask, b, q_len, kv_len, h)
     if d not in (32, 64, 128, 256) or h // hkv > 16:
@@ -1690,11 +1742,11 @@ def attn_prefill_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Op
     with _on_device(q.device):
         if kv_len == 0 or b == 0 or q_len == 0:
             return torch.zeros_like(q)
+        if m4 is None and attn_prefill_strided_takes(b, q_len, kv_len, h, hkv, d):
+            out = attn_prefill_strided(q, k, v, layout, causal_offset, scale=scale)
+            if out is not None:
+                return out if layout == BLHD else out.transpose(1, 2)
         rows_i = torch.arange(q_len, dtype=torch.int64, device=q.device)
-        if layout == BHLD and m4 is None and k.is_contiguous() and v.is_contiguous() and attn_prefill_supported(h, hkv, d):
-            pos = torch.full_like(rows_i, kv_len - 1) if causal_offset < 0 else (rows_i + causal_offset).clamp_max(kv_len - 1)
-            out = attn_prefill(q.contiguous(), k, v, pos, scale=scale if scale > 0 else None)
-            return out.view(b, q_len, h, d).transpose(1, 2)
         causal = causal_offset >= 0 and causal_offset == kv_len - q_len
         if causal_offset >= 0 and not causal:
             band = torch.arange(kv_len, device=q.device)[None, :] <= (rows_i + causal_offset)[:, None]

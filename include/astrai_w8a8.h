@@ -384,6 +384,24 @@ int astrai_w8a8_attn_prefill_bf16(const void* q_bf16, const void* k_cache_bf16,
                                   float scale, void* stream);
 
 /*
+ * Attention of a block of q_len query rows per sequence against key / value tensors in any
+ * memory order (the tensors of csrc/kernels/attention/prefill.cu in either of its layouts, views
+ * of a fused projection, a dense cache), without copying or re-addressing them.
+ *   strides    host array of nine element strides, multiples of 8: batch, head and row of q, of k
+ *              and of v; a row's head_dim values are consecutive. kv_len * row stride < 2^31.
+ *   positions  NULL, or int64 [q_len] on the device: row i sees keys 0 .. positions[i] (at most kv_len)
+ *   causal_offset  without positions: row i sees keys 0 .. i + causal_offset (< 0: all kv_len keys)
+ *   out        bf16 [batch, q_len, n_heads, head_dim]
+ * head_dim 64 or 128, n_heads / n_kv_heads in {1, 2, 4, 8}. Arithmetic of attn_prefill_bf16;
+ * head_dim 64 and n_heads == n_kv_heads: of attn_paged_rows_bf16.
+ */
+int astrai_w8a8_attn_prefill_strided_bf16(const void* q_bf16, const void* k_bf16, const void* v_bf16,
+                                          const int64_t* strides, const int64_t* positions, void* out_bf16,
+                                          int64_t batch, int64_t q_len, int64_t kv_len, int64_t n_heads,
+                                          int64_t n_kv_heads, int64_t head_dim, int64_t causal_offset,
+                                          float scale, void* stream);
+
+/*
  * The same causal block attention over ragged sequences in a token-granular paged cache.
  * Replaces attn_paged_prefill (csrc/kernels/attention/paged_prefill.cu:4-52, addressing
  * policies PackedQSchedule / PagedKV in csrc/kernels/attention/layout_policies.cuh:67-93,
@@ -446,8 +464,9 @@ int astrai_w8a8_attn_paged_prefill_masked_bf16(
  *              [total_q, n_heads, head_dim], the 64-row tile schedule, batch_or_tiles = tiles
  * One wave per (block of up to 16 / (n_heads / n_kv_heads) query rows, KV head, context
  * split): bf16 MFMAs for the scores and for P.V (P as a bf16 head plus a bf16 remainder), fp32
- * softmax statistics and accumulation, one rounding of the output. Correct for every shape,
- * not tuned like the head_dim-128 kernels (prefill re-reads the keys once per row block).
+ * softmax statistics and accumulation, one rounding of the output. Correct for every shape;
+ * prefill without a mask at head_dim 64, or 128 with n_heads == n_kv_heads, runs the block kernel
+ * of attn_prefill_bf16 with P in two terms where there are enough tiles for it.
  *   nsplit     in [1, 64]: 1 = every wave owns a whole context and writes the output itself,
  *              no workspace (NULL allowed); > 1 = partial results in the workspace and a
  *              merge kernel
