@@ -44,6 +44,20 @@ void launch_sum_norm(const SumNormArgs& a, int dtype, bool y_float, hipStream_t 
 constexpr int kActSilu = 0, kActGelu = 1;   // gelu in its tanh form
 void launch_act_mul(const void* gu, void* h, int64_t rows, int ff, int act, int dtype, hipStream_t stream);
 
+// ---- mix_linear.hip -------------------------------------------------------------------------
+constexpr int kFewRowsMax = 64;
+struct FewRowsArgs {
+    const void* x;     // bf16 [m, k], rows ldx apart
+    int64_t ldx;
+    const void* w;     // bf16 [n, k]; with an activation [2 n, k], gate rows first
+    const void* bias;  // bf16 [n] or null
+    void* out;         // [m, n]
+    int m, n, k;
+};
+bool few_rows_linear_supported(int64_t m, int64_t n, int64_t k, bool act);
+// act: kActSilu / kActGelu (out = act(gate) * up), or -1
+bool launch_few_rows_linear(const FewRowsArgs& a, int act, bool out_float, hipStream_t stream);
+
 struct HeadNormArgs {
     const void* o;    // [rows, heads * vp]
     const void* g;    // [rows, ldg]

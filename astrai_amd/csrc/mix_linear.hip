@@ -1,0 +1,193 @@
+// y = x W^T for the few tokens of a decode step (up to 64 rows), bf16 operands, fp32 sums: bound by the
+// stream of the weights, which are read exactly once with the streaming cache hint. Three epilogues: bf16 with
+// a bias, fp32 (what leaves the accumulators), and act(gate) * up of a weight that holds the rows of gate, then
+// those of up, so that the pair of products never reaches memory.
+//
+// The weight rows are dealt out in equal contiguous ranges over about one workgroup per compute unit; the
+// waves of a workgroup split K into contiguous slices of 256-byte items (128 values) and keep all tokens and
+// row groups of their slice, so a workgroup reads x once. Every load moves 4 rows x 256 contiguous bytes; an
+// item of 16 rows is turned into MFMA operand order (lane = row, 16 bytes of K) through a wave-private LDS
+// patch whose XOR chunk swizzle keeps the row-major writes and the operand reads free of conflicts. Weights
+// and x take the same route, so any order of K inside an item is the same for both. Each unit's registers are
+// refilled for the next item as soon as it has been consumed: the bytes in flight stay the same from the first
+// instruction to the last. The waves' partial sums are added through LDS in wave order.
+#include "mix_common.cuh"
+#include "mix_launchers.h"
+
+namespace astrai_mix {
+
+namespace {
+
+constexpr int kItem = 256;  // bytes of K per item
+constexpr int kMaxGroups = 3;
+
+template <int ACT>
+__device__ __forceinline__ float act_of(float z) {
+    return ACT == kActGelu ? gelu_as<uint16_t>(z) : silu_fast(z);
+}
+
+__device__ __forceinline__ void to_operand_order(uint8_t* patch, int lane, const u32x4 (&in)[4], u32x4 (&out)[4]) {
+    const int c16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = i * 4 + g;
+        *reinterpret_cast<u32x4*>(patch + row * 256 + ((c16 ^ row) << 4)) = in[i];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = *reinterpret_cast<const u32x4*>(patch + c16 * 256 + (((4 * j + g) ^ c16) << 4));
+}
+
+// RG: groups of 16 weight rows per workgroup (ACT >= 0: of gate and of up each); MB: groups of 16 tokens;
+// NW: waves. ACT: -1 none.
+template <int RG, int MB, int NW, int ACT, bool F32>
+__global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a, int rows_per_wg) {
+    constexpr int HALVES = ACT >= 0 ? 2 : 1;
+    constexpr int WG = RG * HALVES;              // weight units per item
+    constexpr int P = MB + WG;
+    constexpr int PATCH = 8192, RED = WG * MB * 1024;
+    constexpr int WAVE_LDS = PATCH > RED ? PATCH : RED;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    const int lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int items = a.k / (kItem / 2);
+    const int i0 = wave * items / NW, i1 = (wave + 1) * items / NW;
+    const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, a.n);
+    const uint32_t w_row = (uint32_t)a.k * 2, x_row = (uint32_t)a.ldx * 2;
+    const __amdgpu_buffer_rsrc_t rw = w8a8::make_rsrc(a.w, (uint32_t)(HALVES * a.n) * w_row);
+    const __amdgpu_buffer_rsrc_t rx = w8a8::make_rsrc(a.x, (uint32_t)(a.m - 1) * x_row + w_row);
+
+    f32x4 acc[WG][MB];
+#pragma unroll
+    for (int r = 0; r < WG; ++r)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[r][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    uint8_t* const wpatch = smem + wave * WAVE_LDS;
+    uint8_t* const xpatch = wpatch + 4096;
+    u32x4 ring[P][4];
+    auto issue = [&](u32x4 (&dst)[4], int item, int s) {
+        const bool live = item < i1;
+        const uint32_t k0 = (uint32_t)item * kItem;
+        if (s < MB) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // tokens past m lie past the descriptor: zeros
+                dst[i] = w8a8::buf_load16(
+                    rx, live ? (uint32_t)(s * 16 + i * 4 + g) * x_row + (uint32_t)c16 * 16 : w8a8::kOutOfRange, k0);
+        } else {
+            const int u = s - MB, half = u / RG;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = r0 + (u - half * RG) * 16 + i * 4 + g;
+                dst[i] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rw, live && row < r1 ? (uint32_t)(half * a.n + row) * w_row + (uint32_t)c16 * 16 : w8a8::kOutOfRange,
+                    k0, 2);  // 2: not kept once delivered
+            }
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < P; ++s) issue(ring[s], i0, s);
+    for (int item = i0; item < i1; ++item) {
+        u32x4 xf[MB][4];
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+            if (s < MB) {
+                to_operand_order(xpatch, lane, ring[s], xf[s < MB ? s : 0]);
+            } else {
+                u32x4 wf[4];
+                to_operand_order(wpatch, lane, ring[s], wf);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int b = 0; b < MB; ++b) acc[s < MB ? 0 : s - MB][b] = mfma16(wf[j], xf[b][j], acc[s < MB ? 0 : s - MB][b]);
+            }
+            issue(ring[s], item + 1, s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    __syncthreads();  // the patches are free
+    f32x4* const red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int r = 0; r < WG; ++r)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) red[wave * (WAVE_LDS / 16) + (r * MB + b) * 64 + lane] = acc[r][b];
+    __syncthreads();
+    auto total = [&](int unit) {
+        f32x4 s = red[unit * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) s += red[w * (WAVE_LDS / 16) + unit * 64 + lane];
+        return s;
+    };
+#pragma unroll
+    for (int t = wave; t < RG * MB; t += NW) {
+        const int m = (t % MB) * 16 + c16, row = r0 + (t / MB) * 16 + g * 4;
+        if (m >= a.m || row >= r1) continue;
+        f32x4 v = total(t);
+        const int64_t at = (int64_t)m * a.n + row;
+        if constexpr (ACT >= 0) {
+            const f32x4 up = total(t + RG * MB);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {  // both factors as the products' own bf16 output would hold them
+                const float gate = w8a8::bf16_to_f32(f32_to_bf16(v[e]));
+                v[e] = act_of<ACT>(gate) * w8a8::bf16_to_f32(f32_to_bf16(up[e]));
+            }
+        } else if (a.bias) {
+            v += Elem<uint16_t>::get4(static_cast<const uint16_t*>(a.bias) + row);
+        }
+        if constexpr (F32) Elem<float>::put4(static_cast<float*>(a.out) + at, v);
+        else Elem<uint16_t>::put4(static_cast<uint16_t*>(a.out) + at, v);
+    }
+}
+
+template <int RG, int MB, int NW, int ACT, bool F32>
+void launch_inst(const FewRowsArgs& a, int rows, hipStream_t stream) {
+    constexpr int units = RG * (ACT >= 0 ? 2 : 1) * MB * 1024;
+    constexpr int lds = NW * (units > 8192 ? units : 8192);
+    static_assert(lds <= 64 * 1024, "within the limit that needs no attribute");
+    few_rows_linear_kernel<RG, MB, NW, ACT, F32><<<dim3((unsigned)((a.n + rows - 1) / rows)), dim3(NW * 64), lds, stream>>>(a, rows);
+}
+
+template <int RG, int NW, int ACT, bool F32>
+void launch_mb(const FewRowsArgs& a, int rows, hipStream_t stream) {
+    if (a.m <= 16) launch_inst<RG, 1, NW, ACT, F32>(a, rows, stream);
+    else if (a.m <= 32) launch_inst<RG, 2, NW, ACT, F32>(a, rows, stream);
+    else launch_inst<RG, 4, NW, ACT, F32>(a, rows, stream);
+}
+
+template <int ACT, bool F32>
+void launch_rg(const FewRowsArgs& a, hipStream_t stream) {
+    // rows dealt out over 256 workgroups (a multiple of them where a range would be over GROUPS * 16 rows),
+    // in fours: one load instruction
+    constexpr int GROUPS = ACT >= 0 ? 2 : kMaxGroups;
+    const int wgs = 256 * ((a.n + 256 * GROUPS * 16 - 1) / (256 * GROUPS * 16));
+    const int rows = ((a.n + wgs - 1) / wgs + 3) & ~3;
+    if (rows > 32) {
+        if constexpr (GROUPS == 3) launch_mb<3, 4, ACT, F32>(a, rows, stream);
+    } else if (rows > 16) {
+        launch_mb<2, 4, ACT, F32>(a, rows, stream);
+    } else if (a.k >= 1024) {
+        launch_mb<1, 8, ACT, F32>(a, rows, stream);
+    } else {
+        launch_mb<1, 4, ACT, F32>(a, rows, stream);
+    }
+}
+
+}  // namespace
+
+bool few_rows_linear_supported(int64_t m, int64_t n, int64_t k, bool act) {
+    return m > 0 && m <= kFewRowsMax && n > 0 && n % 4 == 0 && k > 0 && k % (kItem / 2) == 0 &&
+           n * k * (act ? 4 : 2) < ((int64_t)1 << 31);
+}
+
+bool launch_few_rows_linear(const FewRowsArgs& a, int act, bool out_float, hipStream_t stream) {
+    if (!few_rows_linear_supported(a.m, a.n, a.k, act >= 0) || a.ldx < a.k || a.ldx % 8 ||
+        (int64_t)kFewRowsMax * a.ldx * 2 >= ((int64_t)1 << 31))
+        return false;
+    if (act == kActGelu) launch_rg<kActGelu, false>(a, stream);
+    else if (act == kActSilu) launch_rg<kActSilu, false>(a, stream);
+    else if (out_float) launch_rg<-1, true>(a, stream);
+    else launch_rg<-1, false>(a, stream);
+    return true;
+}
+
+}  // namespace astrai_mix

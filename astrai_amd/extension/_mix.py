@@ -40,6 +40,7 @@ PROTOTYPES = {
     "astrai_mix_sum_norm": (
         [_P, _I64, _P, _I64, _F32, _P, _P, _I64] + [_P] * 4 + [_I64, _I64, _F32, _INT, _INT, _P], _INT),
     "astrai_mix_act_mul": ([_P, _P, _I64, _I64, _INT, _INT, _P], _INT),
+    "astrai_mix_few_rows_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _INT, _P], _INT),
     "astrai_mix_head_gated_rms_norm": ([_P, _P, _I64, _P, _P] + [_I64] * 4 + [_F32, _INT, _P], _INT),
     "astrai_mix_gated_rms_norm": ([_P, _P, _I64, _P, _P, _I64, _I64, _I64, _F32, _INT, _P], _INT),
     "astrai_mix_latent_append": (
@@ -243,6 +244,44 @@ def act_mul(gu: torch.Tensor, act: str) -> torch.Tensor:
 
 def silu_mul(gu: torch.Tensor) -> torch.Tensor:
     return act_mul(gu, "silu")
+
+
+FEW_ROWS = 64   # most rows of few_rows_linear
+
+
+def few_rows_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                              act: Optional[str] = None) -> bool:
+    """The calls :func:`few_rows_linear` takes: bf16 on one GPU, up to 64 rows of ``x [.., k]`` at 16-byte
+    boundaries, ``k`` a multiple of 128, the outputs of 4, weights under 2 GiB."""
+    n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
+    rows = x.numel() // k if k else 0
+    if x.size(-1) != k or not 0 < rows <= FEW_ROWS or k % 128 or n % 4 or weight.numel() * 2 >= 2 ** 31:
+        return False
+    if not (x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and weight.device == x.device):
+        return False
+    if not weight.is_contiguous() or weight.data_ptr() % 16 or x.data_ptr() % 16:
+        return False
+    if bias is not None and not (act is None and bias.dtype == torch.bfloat16 and bias.device == x.device
+                                 and bias.is_contiguous() and bias.data_ptr() % 8 == 0):
+        return False
+    return x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and k <= x.stride(0) < 2 ** 23)
+
+
+def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                    act: Optional[str] = None, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """``F.linear`` of a few rows (a decode step), or ``act(gate) * up`` of a weight that holds the rows of
+    gate before those of up: what :func:`act_mul` makes of the product, in one launch."""
+    lib = _require()
+    if not few_rows_linear_supported(x, weight, bias, act) or out_dtype not in _DTYPES:
+        raise RuntimeError("few_rows_linear: operands are not covered")
+    n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
+    m = x.numel() // k
+    with _on_device(x.device):
+        out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=out_dtype)
+        _check(lib.astrai_mix_few_rows_linear(
+            x.data_ptr(), k if x.is_contiguous() else x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
+            out.data_ptr(), m, n, k, -1 if act is None else ACTIVATIONS[act], int(out_dtype == torch.float32), _stream(x)), lib)
+    return out
 
 
 def head_gated_rms_norm(o: torch.Tensor, g: torch.Tensor, weight: torch.Tensor, count: int, eps: float) -> torch.Tensor:

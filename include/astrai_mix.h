@@ -63,6 +63,17 @@ int astrai_mix_sum_norm(const void* y, int64_t ldy, const int64_t* tokens, int64
 /* h = act(gate) * up; gu [rows, 2 ff] (gate columns, then up), ff % 8 == 0. */
 int astrai_mix_act_mul(const void* gu, void* h, int64_t rows, int64_t ff, int act, int dtype, void* stream);
 
+/*
+ * out = x W^T of a few rows (m <= 64), the weights streamed once; bf16 operands, fp32 sums.
+ *   x    bf16 [m, k], rows ldx apart (ldx >= k, a multiple of 8); k % 128 == 0
+ *   w    bf16 [n, k]; with an activation [2 n, k], the rows of gate before those of up; n % 4 == 0
+ *   act  -1: out = x W^T + bias (bf16 [n] or NULL), fp32 if out_float, else bf16
+ *        ASTRAI_MIX_SILU / _GELU: out = act(gate) * up in bf16, both rounded to bf16 first (as act_mul on
+ *        the product's output); no bias, no fp32
+ */
+int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m,
+                               int64_t n, int64_t k, int act, int out_float, void* stream);
+
 /* out = o / sqrt(mean(o^2) + eps) * w * sigmoid(g); the mean over `count` of the n columns (the
  * others are padding). g rows have stride ldg. n % 4 == 0, ldg % 4 == 0. */
 int astrai_mix_gated_rms_norm(const void* o, const void* g, int64_t ldg, const float* w, void* out,
