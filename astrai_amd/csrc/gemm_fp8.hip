@@ -25,12 +25,18 @@ void launch_big(const GemmArgs& g, hipStream_t stream) {
 template <int Fmt, int ScaleKind>
 void launch_for(const GemmArgs& g, hipStream_t stream) {
 #ifndef W8A8_NO_WAVE128
-    if (wave128_shape_ok(g)) {
+    if (wave128_takes(g)) {
+        GemmArgs head, tail;
         if (const int r = ragged_tail_rows(g)) {
-            GemmArgs head, tail;
             split_rows(g, r, ScaleKind == SCALE_ROWCOL, head, tail);
             if (wave128_shape_ok(head) && launch_gemv_fp8(tail, Fmt, ScaleKind, stream))   // (disjoint rows: either order)
                 return launch_big<Fmt, ScaleKind>(head, stream);
+        }
+        if (const int r = tile_tail_rows(g)) {
+            split_rows(g, r, ScaleKind == SCALE_ROWCOL, head, tail);
+            if (mid128_shape_ok(tail)) launch_mid128<Op32F8<Fmt>, ScaleKind>(tail, stream);
+            else launch_small64<Op32F8<Fmt>, ScaleKind>(tail, stream);
+            return launch_big<Fmt, ScaleKind>(head, stream);
         }
         return launch_big<Fmt, ScaleKind>(g, stream);
     }

@@ -13,14 +13,21 @@ namespace w8a8 {
 bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_decode_kernel) {
     if (!tiled_shape_ok(g)) return false;
 #ifndef W8A8_NO_WAVE128
-    if (wave128_shape_ok(g)) {
+    if (wave128_takes(g)) {
+        GemmArgs head, tail;
         if (const int r = tail_on_decode_kernel ? ragged_tail_rows(g) : 0) {
-            GemmArgs head, tail;
             split_rows(g, r, true, head, tail);
             if (wave128_shape_ok(head) && launch_gemv_int8(tail, stream)) {   // (disjoint rows: either order)
                 launch_wave128<Op32I8, SCALE_ROWCOL>(head, stream);
                 return true;
             }
+        }
+        if (const int r = tile_tail_rows(g)) {
+            split_rows(g, r, true, head, tail);
+            if (mid128_shape_ok(tail)) launch_mid128<Op32I8, SCALE_ROWCOL>(tail, stream);
+            else launch_small64<Op32I8, SCALE_ROWCOL>(tail, stream);
+            launch_wave128<Op32I8, SCALE_ROWCOL>(head, stream);
+            return true;
         }
         launch_wave128<Op32I8, SCALE_ROWCOL>(g, stream);
     } else

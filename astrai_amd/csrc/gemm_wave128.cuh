@@ -595,6 +595,8 @@ inline bool wave128_shape_ok(const GemmArgs& g) {
     return pingpong_shape_ok(g) && g.out_kind == OUT_BF16 && (g.n & 7) == 0 && g.n <= (1 << 22);
 }
 
+constexpr int64_t kTailTiles = 384;
+
 // A token count a little above a multiple of 256 (M = 256 q + r, 0 < r <= 128) can cost the
 // large-tile kernel a whole extra round of workgroups for r rows (4100 x 4096 x 4096: 272 tiles on
 // 256 compute units, 96 us against 69 us at 4096 rows). When it does, and the weight-streaming
@@ -620,6 +622,33 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
     if (rowcol) tail.sa = g.sa + row0;
     tail.out = static_cast<uint8_t*>(g.out) + row0 * (size_t)g.n * 2;
     if (g.resid) tail.resid = static_cast<const uint8_t*>(g.resid) + row0 * (size_t)g.n * 2;
+}
+
+// Plain bf16 products that the large tiles take: where they fill most of the chip, or where 128 x 128 tiles
+// would need a second round of two workgroups per compute unit (from 513 of them). One round of large tiles is
+// cheaper than that however empty: K = 2048 27 us against 33 (3072 x 3072), K = 4096 46 against 58 (2816 x 4096),
+// K = 5632 61 against 71 (5000 x 2048), K = 11008 105 against 136 (2816 x 4096); one round of 128 x 128 tiles
+// (512) is cheaper the other way: 22, 40, 49, 91 us.
+inline bool wave128_takes(const GemmArgs& g) {
+    if (wave128_shape_ok(g)) return true;
+    if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 256 || g.out_kind != OUT_BF16 || (g.n & 7) != 0 || g.n > (1 << 22))
+        return false;
+    return (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 512;
+}
+
+// Rows of a product that are better served by smaller tiles in a launch of their own: those past the last
+// row of tiles that fits whole rounds of 256 large tiles, where they make up at most kTailTiles tiles of
+// 128 x 128. Returns their number, else 0. The last round of large tiles costs nearly as much with few tiles as
+// with many. Measured (fp8, one launch -> two; tiles of the tail): 4300 x 4096 x 4096 84 -> 63 us (64), 4300 x 4096 x
+// 11008 199 -> 142 (64), 3001 x 11264 x 2048 77 -> 73 (176), 3001 x 11008 x 4096 133 -> 123 (172), 5000 x 4096 x 4096
+// 86 -> 77 (256), 5500 x 4096 x 4096 87 -> 84 (352); beyond that nothing is left: 6000 x 4096 x 4096 89 -> 89
+// (480), 6500 x 11264 x 2048 134 -> 141 (440).
+inline int tile_tail_rows(const GemmArgs& g) {
+    const int64_t tm = (g.m + 255) / 256, tn = (g.n + 255) / 256, rounds = (tm * tn + 255) / 256;
+    const int64_t head = (rounds - 1) * 256 / tn;  // row tiles that stay
+    if (rounds < 2 || head < 1 || head >= tm) return 0;
+    const int64_t rows = g.m - head * 256;
+    return (rows + 127) / 128 * ((g.n + 127) / 128) <= kTailTiles ? (int)rows : 0;
 }
 
 template <class Op, int ScaleKind, int Epi = EPI_PLAIN>
