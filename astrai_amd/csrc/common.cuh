@@ -89,6 +89,11 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
     return (uint16_t)(pack_bf16x2(f, 0.0f) & 0xffffu);
 }
 
+// y + b, y rounded to bf16 first if asked for (a bias added to a product that has left its kernel)
+__device__ __forceinline__ float add_bias(float y, float b, bool round_first) {
+    return (round_first ? bf16_to_f32(f32_to_bf16(y)) : y) + b;
+}
+
 // Saturating fp32 -> fp8 pair (low 16 bits of the result). The hardware
 // converter rounds to nearest even; magnitudes are clamped to the finite max
 // first (NaN passes through the clamp untouched and converts to NaN).

@@ -19,8 +19,19 @@ namespace {
 // even -- its loop walks two slabs a turn --, else on the 32x32x64 MFMA.
 template <int Fmt, int ScaleKind>
 void launch_big(const GemmArgs& g, hipStream_t stream) {
-    if ((g.k & 255) == 0) launch_wave128_q16<Fmt, ScaleKind>(g, stream);
-    else launch_wave128<Op32F8<Fmt>, ScaleKind>(g, stream);
+    const bool round_first = g.bias && g.round_first;
+    if ((g.k & 255) == 0) {
+        if constexpr (Fmt == 0 && ScaleKind == SCALE_TENSOR)
+            if (round_first) return launch_wave128_q16<0, SCALE_TENSOR, true>(g, stream);
+        if (!round_first) return launch_wave128_q16<Fmt, ScaleKind>(g, stream);
+    }
+    if (!round_first) return launch_wave128<Op32F8<Fmt>, ScaleKind>(g, stream);
+    // (an odd number of slabs: that kernel's epilogue has no registers to spare)
+    GemmArgs plain = g;
+    plain.bias = nullptr;
+    if ((g.k & 255) == 0) launch_wave128_q16<Fmt, ScaleKind>(plain, stream);
+    else launch_wave128<Op32F8<Fmt>, ScaleKind>(plain, stream);
+    launch_add_bias_bf16(g.out, g.bias, g.m, g.n, stream);
 }
 template <int Fmt, int ScaleKind>
 void launch_for(const GemmArgs& g, hipStream_t stream) {

@@ -222,7 +222,7 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
                     if constexpr (ScaleKind == SCALE_BLOCK128) {
                         v[j] = f + ((bias && n + j < g.n) ? bf16_to_f32(bias[n + j]) : 0.0f);
                     } else if constexpr (ScaleKind == SCALE_TENSOR) {
-                        v[j] = f * s_tensor + b4[ni][q][j];
+                        v[j] = g.round_first ? add_bias(f * s_tensor, b4[ni][q][j], true) : f * s_tensor + b4[ni][q][j];
                     } else {
 #pragma clang fp contract(off)
                         const float scaled = f * sx[mi] * sw4[ni][q][j];

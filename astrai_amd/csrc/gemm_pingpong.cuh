@@ -535,7 +535,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
                         if constexpr (ScaleKind == SCALE_TENSOR) f = f * (es.sa * es.sb);
                         else if constexpr (ScaleKind == SCALE_ROWCOL) f = f * sx * sw4[j];
                         else f = f * blk_s[mi];
-                        v[j] = f + b4[j];
+                        v[j] = add_bias(f, b4[j], g.round_first);
                     }
                     u32x2 pk;
                     pk.x = pack_bf16x2(v[0], v[1]);

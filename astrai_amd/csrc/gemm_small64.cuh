@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
             if constexpr (ScaleKind == SCALE_BLOCK128) {
                 v[j] = f + ((bias && n + j < g.n) ? bf16_to_f32(bias[n + j]) : 0.0f);
             } else if constexpr (ScaleKind == SCALE_TENSOR) {
-                v[j] = f * s_tensor + b4[q][j];
+                v[j] = g.round_first ? add_bias(f * s_tensor, b4[q][j], true) : f * s_tensor + b4[q][j];
             } else {
 #pragma clang fp contract(off)
                 const float scaled = f * sx * sw4[q][j];

@@ -37,7 +37,8 @@
 
 namespace w8a8 {
 
-template <int Fmt, int ScaleKind, int KO = 0>
+// RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it
+template <int Fmt, int ScaleKind, int KO = 0, bool RoundFirst = false>
 __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(GemmArgs g) {
     static_assert(ScaleKind == SCALE_TENSOR || ScaleKind == SCALE_ROWCOL, "per-tensor or row x column scales");
     PP_STAMP_INIT();
@@ -289,7 +290,9 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(G
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const float f = acc[ni][mi][j];
-                        if constexpr (ScaleKind == SCALE_TENSOR) {
+                        if constexpr (ScaleKind == SCALE_TENSOR && RoundFirst) {
+                            v[j] = add_bias(f * s_tensor, b4[j], true);
+                        } else if constexpr (ScaleKind == SCALE_TENSOR) {
                             v[j] = f * s_tensor + b4[j];
                         } else {
 #pragma clang fp contract(off)
@@ -315,11 +318,11 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(G
     PP_STAMP();
 }
 
-template <int Fmt, int ScaleKind>
+template <int Fmt, int ScaleKind, bool RoundFirst = false>
 inline void launch_wave128_q16(const GemmArgs& g, hipStream_t stream) {
     using Cfg = Wave128Cfg;
     const int tiles = ((g.m + Cfg::BM - 1) / Cfg::BM) * ((g.n + Cfg::BN - 1) / Cfg::BN);
-    auto kern = gemm_wave128_q16_kernel<Fmt, ScaleKind>;
+    auto kern = gemm_wave128_q16_kernel<Fmt, ScaleKind, 0, RoundFirst>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
     note_kernel("wave128_q16");

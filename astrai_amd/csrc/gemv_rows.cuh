@@ -291,7 +291,7 @@ __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCach
             // (per-tensor fp8: e_sx is the product of the two steps, e_sw is 1)
 #pragma clang fp contract(off)
             const float f = (float)sum[j] * e_sx[ti] * e_sw[ti][j];
-            v[j] = f + e_b[ti][j];
+            v[j] = add_bias(f, e_b[ti][j], !Op::kIsInt && g.round_first);
         }
         if constexpr (ROPE) {
             // what the plain epilogue would have stored, as the rotary kernel would read it

@@ -44,6 +44,7 @@ struct GemmArgs {
     int out_kind;
     float* row_max = nullptr;  // SwiGLU epilogue only: fp32 [M, N/128] partial row maxima of |h|
     const void* resid = nullptr;  // residual epilogue only: bf16 [M,N]; out = bf16(bf16(y) + resid)
+    bool round_first = false;  // with a bias: out = bf16(bf16(y) + bias) instead of bf16(y + bias)
 };
 
 // quantize.hip
@@ -233,6 +234,8 @@ bool launch_gemm_int8_swiglu(const GemmArgs& g, hipStream_t stream);
 // shapes it takes; false otherwise (the caller runs the plain GEMM and an addition pass).
 bool launch_gemm_int8_resid(const GemmArgs& g, hipStream_t stream);
 // out = bf16(y + resid) over `total` bf16 elements; out may be y
+// out[m, n] = bf16(out[m, n] + bias[n]), n % 8 == 0
+void launch_add_bias_bf16(void* out, const void* bias, int64_t rows, int64_t n, hipStream_t stream);
 void launch_add_bf16(const void* y, const void* resid, void* out, int64_t total, hipStream_t stream);
 bool launch_gemm_fp8_tiled(const GemmArgs& g, int fmt, hipStream_t stream);
 // sa per activation row [M], sb per weight row [N], bf16 output

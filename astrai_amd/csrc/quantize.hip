@@ -448,6 +448,22 @@ __global__ __launch_bounds__(kThreads) void add_bf16_kernel(
     if (t < total) out[t] = f32_to_bf16(bf16_to_f32(y[t]) + bf16_to_f32(resid[t]));
 }
 
+// out = bf16(out + bias) in place, bias[n] of each row (n % 8 == 0)
+__global__ __launch_bounds__(kThreads) void add_bias_bf16_kernel(uint16_t* out, const uint16_t* __restrict__ bias,
+                                                                 int64_t total, int n) {
+    const int64_t stride = (int64_t)gridDim.x * kThreads * 8;
+    for (int64_t i = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 8; i < total; i += stride) {
+        float a[8], b[8];
+        unpack8(*reinterpret_cast<const u32x4*>(out + i), a);
+        const uint16_t* const bp = bias + (int)(i % n);   // (a bias is aligned to its elements only)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) b[j] = bf16_to_f32(bp[j]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] += b[j];
+        *reinterpret_cast<u32x4*>(out + i) = pack8(a);
+    }
+}
+
 // s = bf16(x + res) (when res is given; written to sum_out), y = bf16(w * (rstd * s))
 // with rstd = rsqrt(mean(s^2) + eps) in fp32 -- one rounding, the arithmetic of
 // F.rms_norm on a bf16 tensor (model/components/norm.py:7-15) -- then the per-row
@@ -915,6 +931,12 @@ void launch_add_bf16(const void* y, const void* resid, void* out, int64_t total,
     const int64_t blocks = want < 1 ? 1 : (want > 4096 ? 4096 : want);
     add_bf16_kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(
         static_cast<const uint16_t*>(y), static_cast<const uint16_t*>(resid), static_cast<uint16_t*>(out), total);
+}
+
+void launch_add_bias_bf16(void* out, const void* bias, int64_t rows, int64_t n, hipStream_t stream) {
+    const int64_t blocks = (rows * n / 8 + kThreads - 1) / kThreads;
+    add_bias_bf16_kernel<<<dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kThreads), 0, stream>>>(
+        static_cast<uint16_t*>(out), static_cast<const uint16_t*>(bias), rows * n, (int)n);
 }
 
 void launch_add_rmsnorm_quantize_int8_rows(const void* x, const void* res, const void* w, float eps,

@@ -85,6 +85,7 @@ PROTOTYPES = {
     "astrai_w8a8_quantize_bf16_fp8_block128_act": ([_P, _P, _P, _I64, _I64, _P], _INT),
     "astrai_w8a8_quantize_bf16_fp8_block128_weight": ([_P, _P, _P, _I64, _I64, _P], _INT),
     "astrai_w8a8_gemm_fp8_pt": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _INT, _P], _INT),
+    "astrai_w8a8_gemm_fp8_pt_rounded_bias": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_fp8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_fp8_block128": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
@@ -267,13 +268,14 @@ def quantize_bf16(x: torch.Tensor, scale: torch.Tensor, fmt: int):
 
 def mm_fp8(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
            out_dtype: int = 0, out_scale: Optional[torch.Tensor] = None,
-           bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+           bias: Optional[torch.Tensor] = None, round_first: bool = False) -> torch.Tensor:
     """Pre-quantized fp8 GEMM ``a @ b^T * sa * sb``. mm.cu:128-184. ``bias`` (bf16
     ``[N]``, bf16 output only) is an extension used by the fused linear forward.
     Scales are fp32 scalars, as the reference's binding demands (mm.cu:49-54) -- or,
     for bf16 output, the shapes its CPU kernel's broadcast accepts besides
     (ops/fp8.py:118): ``sa`` one step per activation row (``[M]`` / ``[M, 1]``) and / or
-    ``sb`` one per weight row (``[N]`` / ``[1, N]``)."""
+    ``sb`` one per weight row (``[N]`` / ``[1, N]``). ``round_first`` (scalar scales, bf16
+    output): the bias joins the product already rounded to bf16."""
     lib = _require()
     _gpu(a, "mm_fp8")
     _gpu(b, "mm_fp8")
@@ -323,6 +325,10 @@ def mm_fp8(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
                 _check(lib.astrai_w8a8_gemm_fp8_ptpc(
                     a_c.data_ptr(), b_c.data_ptr(), sa_v.data_ptr(), sb_v.data_ptr(), _ptr(bias),
                     out.data_ptr(), m, n, k, 1 if a.dtype == torch.float8_e5m2 else 0, _stream(a)), lib)
+            elif round_first and bias is not None and out_dtype == 0:
+                _check(lib.astrai_w8a8_gemm_fp8_pt_rounded_bias(
+                    a_c.data_ptr(), b_c.data_ptr(), sa.data_ptr(), sb.data_ptr(), bias.data_ptr(), out.data_ptr(),
+                    m, n, k, 1 if a.dtype == torch.float8_e5m2 else 0, _stream(a)), lib)
             else:
                 _check(lib.astrai_w8a8_gemm_fp8_pt(
                     a_c.data_ptr(), b_c.data_ptr(), sa.data_ptr(), sb.data_ptr(),

@@ -36,6 +36,7 @@ from astrai_amd.extension.ops.fp8 import (
     linear_forward_fp8,
     mm_fp8,
     mm_fp8_bias,
+    mm_fp8_rounded_bias,
     new_amax_partials,
     quantize_bf16,
     quantize_bf16_partials,
@@ -357,7 +358,11 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None):
         else:
             sw = _dynamic_scale(w, st.recipe, fmt)
             w8, _ = quantize_bf16(w, sw, fmt)
-        out = mm_fp8(x8, w8, sx, sw).reshape(*x.shape[:-1], w.size(0))
+        shape = (*x.shape[:-1], w.size(0))
+        if bias is not None and bias.is_cuda and bias.dtype == torch.bfloat16 and bias.shape == (w.size(0),) \
+                and bias.device == x.device and bias.numel() and x2.size(1):
+            return mm_fp8_rounded_bias(x8, w8, sx, sw, bias).reshape(shape)
+        out = mm_fp8(x8, w8, sx, sw).reshape(shape)
         if bias is not None and bias.numel():
             out = out + bias
         return out

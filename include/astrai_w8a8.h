@@ -520,6 +520,15 @@ int astrai_w8a8_gemm_fp8_pt(const void* a8, const void* b8, const float* sa,
                             int out_dtype, void* stream);
 
 /*
+ * gemm_fp8_pt to bf16 with the bias added to the rounded product, out = bf16(bf16(acc * *sa * *sb) +
+ * bias[n]): what the product followed by an addition of its own gives (dynamic scaling adds the bias that
+ * way, astrai/extension/fp8.py:289-302), without the pass over the output in between.
+ */
+int astrai_w8a8_gemm_fp8_pt_rounded_bias(const void* a8, const void* b8, const float* sa, const float* sb,
+                                         const void* bias_bf16, void* out_bf16, int64_t m, int64_t n, int64_t k,
+                                         int fmt, void* stream);
+
+/*
  * The per-tensor GEMM above with one scale per activation row and one per weight row:
  *   out[m,n] = bf16( (sum_k a8[m,k] * b8[n,k]) * sa[m] * sb[n] + bias[n] )
  * sa fp32 [M], sb fp32 [N]. The reference's CUDA binding takes scalars only
