@@ -21,13 +21,20 @@
 // LDS rows of 16-byte chunks are XOR-swizzled so that the 16 rows an operand read touches (keys) or
 // the four rows a transposing read touches (values) fall into different banks. The loads' buffer
 // descriptor is rebuilt per block to end at the newest visible key: rows past it and padding
-// columns arrive as zeros without predicates.
+// columns arrive as zeros without predicates. They are issued from assembly: behind the builtin the compiler
+// orders every transposing read after all loads in flight, a memory round trip per block. Tiles that every query
+// of the wave sees whole skip the masks, in a loop of their own (at a join of two kinds of steps all accumulators
+// would change registers). Bound by the matrix pipe with latent heads (28 MFMAs a tile), by the vector ALU with
+// soft-capped scores (two more quarter-rate operations a score). Measured inside the models, before -> after
+// these points: latent 32 x 512 tokens, 16 heads 113 -> 105 us; grouped 1 x 4096, 16/4 heads 176 -> 158 us.
 // A wave's stream is a software pipeline over tiles: the score MFMAs of tile T + 1 are issued among the
 // exponentials of tile T, the value MFMAs of tile T among the masking of tile T + 1. One copy of the
 // step masks every tile: a second copy without masking costs more in registers and code than the
 // compares (157 us against 107 us for 32 x 512 tokens, 16 heads of 128 + 64).
 #include "mix_common.cuh"
 #include "mix_launchers.h"
+
+#include <type_traits>
 
 namespace astrai_mix {
 
@@ -36,8 +43,25 @@ namespace {
 constexpr int kQB = 128;   // query tokens per workgroup
 constexpr int kKB = 64;    // keys per block (two tiles)
 
-__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* lds_wave_base, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, voff, 0, 0, 0);
+// A raw buffer descriptor in scalar registers (see w8a8::make_rsrc), as lds_dma16's assembly takes it.
+__device__ __forceinline__ u32x4 make_desc(const void* p, uint32_t bytes) {
+    const uint64_t addr = (uint64_t)p;
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(addr >> 32) & 0xffffu)),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+// 16 bytes per lane from the buffer into LDS at lds_addr + 16 * lane (lds_addr the same for the whole wave).
+// Out-of-range lanes write zeros. The caller waits (vmcnt) before the bytes are read. (m0 is a reserved
+// register that nothing else in this file's kernels uses.)
+__device__ __forceinline__ void lds_dma16(u32x4 desc, uint32_t lds_addr, uint32_t voff) {
+    __asm__ volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, 0 offen lds"
+        :
+        : "s"(lds_addr), "v"(voff), "s"(desc)
+        : "memory");
 }
 
 // which of a row's C chunks sits at position 0: 16 consecutive rows cover all banks
@@ -57,13 +81,19 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     constexpr int JN = CN / 4, JR = CR / 4, JV = CV / 4;          // loads per wave and 64-key block
     constexpr int IN = CN / 2, IR = CR / 2;                       // loads per 32-key tile, all waves
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qi = lane & 31, h2 = lane >> 5;
     const int groups = a.batch * d.heads;
     const int nqb = (a.seq + kQB - 1) / kQB;
-    const int qb = nqb - 1 - (int)(blockIdx.x / groups), bh = (int)(blockIdx.x % groups);   // longest key ranges first
+    // Longest key ranges first; where all workgroups are resident at once, two to a compute unit, the second 256
+    // run the other way, so that the longest share a unit with the shortest (1 x 4096 tokens, 16 heads:
+    // 158 -> 129 us)
+    const int order = gridDim.x <= 512 && blockIdx.x >= 256 ? (int)(gridDim.x + 255 - blockIdx.x) : (int)blockIdx.x;
+    const int qb = nqb - 1 - order / groups, bh = order % groups;
     const int b = bh / d.heads, head = bh % d.heads;
     const int kv_head = GQA ? head / a.group : head, kv_heads = GQA ? d.heads / a.group : d.heads;
     const int dk = d.dn + d.dr;
@@ -79,6 +109,9 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     const int w_first = a.start + q0 + wave * 32, w_last = min(w_first + 31, kmax);
     const int ta = w_live ? (max(w_first - d.window + 1, 0) - kmin) / 32 : 1 << 28;
     const int tb = w_live ? (w_last - kmin) / 32 : -1;
+    // of them, those that every query of the wave sees whole: [fa, fb)
+    const int fa = w_live ? (max(w_last - d.window + 1, 0) - kmin + 31) / 32 : 0;
+    const int fb = w_live ? (w_first + 1 - kmin) / 32 : 0;
     const int nblocks = (kmax - kmin) / kKB + 1;
 
     u32x4 qf[NK];
@@ -119,31 +152,31 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     }
     auto rows_rsrc = [](const uint8_t* p, int rows, int64_t ld, int bytes) {
         const int64_t n = rows > 0 ? (int64_t)(rows - 1) * ld + bytes : 0;
-        return w8a8::make_rsrc(p, (uint32_t)n);
+        return make_desc(p, (uint32_t)n);
     };
     // tiles t0 and t0 + 1 into their ring slots
     auto dma_k = [&](int t0) {
         const int key = kmin + t0 * 32, rows = min(kmax - key + 1, kKB);
-        const __amdgpu_buffer_rsrc_t rn = rows_rsrc(kv + (int64_t)key * ldkv, rows, ldkv, d.dn * 2);
+        const u32x4 rn = rows_rsrc(kv + (int64_t)key * ldkv, rows, ldkv, d.dn * 2);
 #pragma unroll
         for (int j = 0; j < JN; ++j) {
             const int inst = wave * JN + j;
-            lds_dma16(rn, lds + ((t0 + inst / IN) & 3) * kTile + (inst % IN) * 1024, on[j]);
+            lds_dma16(rn, lds0 + ((t0 + inst / IN) & 3) * kTile + (inst % IN) * 1024, on[j]);
         }
         if constexpr (DR > 0) {
-            const __amdgpu_buffer_rsrc_t rr = rows_rsrc(kr + (int64_t)key * ldc, rows, ldc, d.dr * 2);
+            const u32x4 rr = rows_rsrc(kr + (int64_t)key * ldc, rows, ldc, d.dr * 2);
 #pragma unroll
             for (int j = 0; j < JR; ++j) {
                 const int inst = wave * JR + j;
-                lds_dma16(rr, lds + ((t0 + inst / IR) & 3) * kTile + 32 * kNRow + (inst % IR) * 1024, orr[j]);
+                lds_dma16(rr, lds0 + ((t0 + inst / IR) & 3) * kTile + 32 * kNRow + (inst % IR) * 1024, orr[j]);
             }
         }
     };
     auto dma_v = [&](int kb) {
         const int key = kmin + kb * kKB, rows = min(kmax - key + 1, kKB);
-        const __amdgpu_buffer_rsrc_t rv = rows_rsrc(kv + (int64_t)key * ldkv + d.dn * 2, rows, ldkv, d.vp * 2);
+        const u32x4 rv = rows_rsrc(kv + (int64_t)key * ldkv + d.dn * 2, rows, ldkv, d.vp * 2);
 #pragma unroll
-        for (int j = 0; j < JV; ++j) lds_dma16(rv, lds + kRing + (kb & 1) * kVBuf + (wave * JV + j) * 1024, ov[j]);
+        for (int j = 0; j < JV; ++j) lds_dma16(rv, lds0 + kRing + (kb & 1) * kVBuf + (wave * JV + j) * 1024, ov[j]);
     };
 
     f32x16 o[NV];
@@ -160,7 +193,8 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     // capped scores leave mask_max4 in log2 units
     const bool capped = GQA && a.softcap > 0.0f;
     const float c = capped ? 1.0f : d.scale * kLog2e;
-    const float cap_in = capped ? d.scale / a.softcap : 0.0f, cap_out = a.softcap * kLog2e;
+    // softcap tanh(s scale / softcap) = softcap - 2 softcap / (1 + e^(2 s scale / softcap)), e^ as 2^
+    const float cap_in = capped ? 2.0f * kLog2e * d.scale / a.softcap : 0.0f, cap_out = a.softcap * kLog2e;
     const f32x16 zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     // key operand of step ks: chunk (2 ks + h2) ^ swizzle of this lane's row. Rows are powers of two and
@@ -180,19 +214,24 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
         const uint8_t* src = lds + ((vt + v_lane) ^ (i << 6)) + t * 16 * kVRow;
         return join(lds_read_tr(src), lds_read_tr(src + 8 * kVRow));
     };
-    auto mask_max4 = [&](int T, f32x16& s, int g, float m) -> float {
+    auto mask_max4 = [&](auto mask_tag, int T, f32x16& s, int g, float m) __attribute__((always_inline)) -> float {
+        constexpr bool PARTIAL = decltype(mask_tag)::value;  // some score of the tile may be hidden
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int e = 4 * g + j, key = kmin + T * 32 + g * 8 + h2 * 4 + j;
-            if (capped) s[e] = cap_out * tanh_fast(s[e] * cap_in);
-            s[e] = (key <= pq && key >= plo) ? s[e] : kNegBig;
+            if (capped) {
+                const float u = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[e] * cap_in));
+                s[e] = __builtin_fmaf(u, -2.0f * cap_out, cap_out);
+            }
+            if (PARTIAL) s[e] = (key <= pq && key >= plo) ? s[e] : kNegBig;
             m = fmaxf(m, s[e]);
         }
         return m;
     };
     // In: s_in = masked scores of tile T, m_in their maximum. Out: the values of tile T added to o;
-    // s_out = scores of tile T + 1, m_out their maximum. vt: LDS offset of tile T's value rows.
-    auto step = [&](int T, f32x16& s_in, float m_in, f32x16& s_out, float& m_out, int vt) {
+    // s_out = scores of tile T + 1, m_out their maximum. vt: LDS offset of tile T's value rows. The tag says
+    // whether tile T + 1 needs its mask.
+    auto step = [&](auto mask_tag, int T, f32x16& s_in, float m_in, f32x16& s_out, float& m_out, int vt) __attribute__((always_inline)) {
         const float m_sc = m_in * c;
         if (__any(m_sc > m_run + kSlack)) {
             const float m_new = fmaxf(m_run, m_sc);
@@ -234,8 +273,8 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
             o[dt] = mfma32(vf[i], ph, o[dt]);
             o[dt] = mfma32(vf[i], pl, o[dt]);
 #pragma unroll
-            for (int g = i * 4 / (2 * NV); g < (i + 1) * 4 / (2 * NV); ++g) m = mask_max4(T + 1, s_out, g, m);
-            }
+            for (int g = i * 4 / (2 * NV); g < (i + 1) * 4 / (2 * NV); ++g) m = mask_max4(mask_tag, T + 1, s_out, g, m);
+        }
         m_out = fmaxf(m, __shfl_xor(m, 32, kWave));
     };
     dma_k(0);
@@ -252,19 +291,60 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
         for (int ks = 0; ks < NK; ++ks) sa = mfma32(k_frag(0, ks), qf[ks], ks == 0 ? zero16 : sa);
         float m = kNegBig;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) m = mask_max4(0, sa, g, m);
+        for (int g = 0; g < 4; ++g) m = mask_max4(std::true_type{}, 0, sa, g, m);
         ma = fmaxf(m, __shfl_xor(m, 32, kWave));
     }
     __syncthreads();  // tile 0's ring slot is overwritten by the first block's loads
-    for (int kb = 0; kb < nblocks; ++kb) {
+    auto begin_block = [&](int kb) {
         dma_k(2 * kb + 3);  // tiles 2kb+3, 2kb+4: their ring slots held tiles 2kb-1 and 2kb
         if (kb + 1 < nblocks) dma_v(kb + 1);
-        const int vt = kRing + (kb & 1) * kVBuf;
-        // (the step before the wave's first tile runs on hidden scores and brings in that tile's)
-        if (2 * kb >= ta - 1 && 2 * kb <= tb) step(2 * kb, sa, ma, sb, mb, vt);
-        if (2 * kb + 1 >= ta - 1 && 2 * kb + 1 <= tb) step(2 * kb + 1, sb, mb, sa, ma, vt + 32 * kVRow);
+    };
+    auto end_block = [&] {
         __builtin_amdgcn_s_waitcnt(0x0070);
         __syncthreads();
+    };
+    // The wave's steps are first .. tb (the step before its first tile runs on hidden scores and brings in
+    // that tile's), two to a block; blocks before and after only load for the other waves. Runs of blocks
+    // are loops of their own, so that every step finds the accumulators where the last one left them.
+    int kb = 0;
+    const int first = max(ta - 1, 0), pairs = (tb + 1) / 2;
+    for (; kb < min(first / 2, nblocks); ++kb) {
+        begin_block(kb);
+        end_block();
+    }
+    if (w_live && (first & 1)) {
+        begin_block(kb);
+        step(std::true_type{}, 2 * kb + 1, sb, mb, sa, ma, kRing + (kb & 1) * kVBuf + 32 * kVRow);
+        end_block();
+        ++kb;
+    }
+    auto masked_pairs = [&](int end) __attribute__((always_inline)) {
+        for (; kb < end; ++kb) {
+            begin_block(kb);
+            const int vt = kRing + (kb & 1) * kVBuf;
+            step(std::true_type{}, 2 * kb, sa, ma, sb, mb, vt);
+            step(std::true_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + 32 * kVRow);
+            end_block();
+        }
+    };
+    masked_pairs(min(fa / 2, pairs));   // (block kb brings in tiles 2kb+1 and 2kb+2)
+    for (const int end = (fb - 1) / 2; kb < end; ++kb) {
+        begin_block(kb);
+        const int vt = kRing + (kb & 1) * kVBuf;
+        step(std::false_type{}, 2 * kb, sa, ma, sb, mb, vt);
+        step(std::false_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + 32 * kVRow);
+        end_block();
+    }
+    masked_pairs(pairs);
+    if (tb >= 0 && (tb & 1) == 0 && kb == tb / 2) {   // a last block of one step
+        begin_block(kb);
+        step(std::true_type{}, 2 * kb, sa, ma, sb, mb, kRing + (kb & 1) * kVBuf);
+        end_block();
+        ++kb;
+    }
+    for (; kb < nblocks; ++kb) {
+        begin_block(kb);
+        end_block();
     }
     if (!w_live) return;
     // normalise, gate, and write through LDS (idle by now), so that rows leave in whole pieces
