@@ -159,10 +159,12 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     } else {
         const int nqb = (a.seq + QB - 1) / QB;
         const int groups = a.batch * a.n_kv_heads;
-        // Longest key ranges first; where all workgroups are resident at once, two to a compute unit, the second
-        // 256 run the other way, so that the longest share a unit with the shortest (what that gives was measured
-        // on the like walk of mix_prefill.hip: 158 -> 129 us for one sequence of 4096)
-        const int order = gridDim.x <= 512 && blockIdx.x >= 256 ? (int)(gridDim.x + 255 - blockIdx.x) : (int)blockIdx.x;
+        // Longest key ranges first; where all workgroups are resident at once, two to a compute unit (four waves
+        // each), the second 256 run the other way, so that the longest share a unit with the shortest: 1 x 4096
+        // tokens, 16/4 heads x 128, 97 -> 93 us. With eight waves a unit holds one, and the second 256 start as
+        // units become free: longest first is the better order (32/4 heads: 140 us, reversed 161)
+        const bool turned = WAVES <= 4 && gridDim.x <= 512 && blockIdx.x >= 256;
+        const int order = turned ? (int)(gridDim.x + 255 - blockIdx.x) : (int)blockIdx.x;
         const int qb = nqb - 1 - order / groups;
         const int bk = order % groups;
         const int b = bk / a.n_kv_heads;

@@ -26,7 +26,7 @@
 // of the wave sees whole skip the masks, in a loop of their own (at a join of two kinds of steps all accumulators
 // would change registers). Bound by the matrix pipe with latent heads (28 MFMAs a tile), by the vector ALU with
 // soft-capped scores (two more quarter-rate operations a score). Measured inside the models, before -> after
-// these points: latent 32 x 512 tokens, 16 heads 113 -> 105 us; grouped 1 x 4096, 16/4 heads 176 -> 158 us.
+// these points: latent 32 x 512 tokens, 16 heads 113 -> 105 us; grouped 1 x 4096, 16/4 heads 176 -> 160 us.
 // A wave's stream is a software pipeline over tiles: the score MFMAs of tile T + 1 are issued among the
 // exponentials of tile T, the value MFMAs of tile T among the masking of tile T + 1. One copy of the
 // step masks every tile: a second copy without masking costs more in registers and code than the
@@ -90,8 +90,8 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     const int groups = a.batch * d.heads;
     const int nqb = (a.seq + kQB - 1) / kQB;
     // Longest key ranges first; where all workgroups are resident at once, two to a compute unit, the second 256
-    // run the other way, so that the longest share a unit with the shortest (1 x 4096 tokens, 16 heads:
-    // 158 -> 129 us)
+    // run the other way, so that the longest share a unit with the shortest (1 x 4096 tokens, 16 heads,
+    // inside the model: 160 -> 148 us)
     const int order = gridDim.x <= 512 && blockIdx.x >= 256 ? (int)(gridDim.x + 255 - blockIdx.x) : (int)blockIdx.x;
     const int qb = nqb - 1 - order / groups, bh = order % groups;
     const int b = bh / d.heads, head = bh % d.heads;
