@@ -12,7 +12,8 @@
 //          second would overflow under strong decays), so pairs are grouped by the highest bit in which t
 //          and j differ: with m the middle of their common block of 2, 4, 8 or 16 tokens, L_tj is
 //          (decays m .. t)(decays j + 1 .. m - 1), both <= 1. One wave per such level and product.
-//   walk   chunk after chunk per head; a wave owns 16 or 32 value columns and all key channels, S in fp32
+//   walk   chunk after chunk per head; a wave owns 16 or 32 value columns and all key channels (with few heads: 32
+//          key channels, delta_walk_split_kernel), S in fp32
 //          accumulators. With value columns as MFMA columns throughout, every accumulator (S, V - Y, U) is
 //          the next product's operand already; images stream into LDS by direct loads, one chunk ahead.
 // 32-bit factors enter the matrix cores as two bf16 terms; a 16-deep contraction uses the two halves of a
@@ -480,6 +481,175 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* lds
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, voff, 0, 0, 0);
 }
 
+// The walk of few heads: one workgroup per 16 value columns, its waves share the key channels, 32 each. A chunk's
+// serial chain is then short (two state tiles to split, three products for a part of Y, the parts summed through LDS,
+// U, four products), each image word goes straight into the registers of the one wave that multiplies it (the few
+// all need excepted), and three chunks are under way: the general walk waits for its next image at each chunk. Y's
+// parts change hands behind the chunk's barrier, O's a barrier later, off the chain. Column blocks of a head run on
+// one XCD and find its images in that L2. Bound by the chain: some 170 instructions at four cycles and the latencies
+// of 5 products and two trips through LDS. 16 heads, 128 x 128, 4096 tokens: 373 us as the general walk, 153 here.
+template <int DP>
+__global__ __launch_bounds__(64 * (DP / 32), DP <= 128 ? 2 : 1) void delta_walk_split_kernel(DeltaArgs a, int chunks) {
+    constexpr int W = DP / 32, NS = W, kBuf = Image<DP>::kDma * 1024, kAhead = 3;
+    __shared__ f32x4 part_y[2][W][64], part_o[2][W][64];
+    const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = a.vp / 16, turn = (int)blockIdx.x / 8;
+    const int bh = turn / tiles * 8 + (int)blockIdx.x % 8;
+    if (bh >= a.batch * a.heads) return;
+    const int b = bh / a.heads, h = bh % a.heads, v = turn % tiles * 16 + c16;
+    const uint8_t* image = static_cast<const uint8_t*>(a.image) + (int64_t)bh * chunks * kBuf;
+    const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv) + (int64_t)b * a.seq * a.ldq;
+    const int ldo = a.heads * a.vp;
+    uint16_t* out = static_cast<uint16_t*>(a.out) + (int64_t)b * a.seq * ldo;
+    float* state = a.state + ((int64_t)b * a.heads + h) * a.dp * a.vp + v;
+
+    f32x4 st[2];    // rows 32 wave + 16 i + 4 g + e, column v
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int d = 32 * wave + 16 * i + 4 * g + e;
+            st[i][e] = d < a.dp ? state[(int64_t)d * a.vp] : 0.0f;
+        }
+    uint32_t v_off[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v_off[e] = (uint32_t)((4 * g + e) * a.ldq + 2 * a.kv_heads * a.dp + h * a.vp + v) * 2;
+    const uint32_t o_off = (uint32_t)(4 * g * ldo + h * a.vp + v) * 2;
+    const uint32_t p_off = wave ? 1u << 31 : lane * 16;   // one wave adds P U, the others zeros
+    struct Chunk {
+        u32x4 kh, kl, qh, ql, lk[2], t, p;
+        f32x4 decay[2];
+        uint16_t v[4];
+    };
+    // the chunk to load: addresses run along (past the end: the last one once more, for nothing)
+    int left = a.seq;
+    const uint8_t* im_next = image;
+    const uint16_t* v_next = qkv;
+    auto load = [&](Chunk& x) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t im = w8a8::make_rsrc(im_next, kBuf);
+        const __amdgpu_buffer_rsrc_t rv = w8a8::make_rsrc(v_next, min(kC, left) * a.ldq * 2);
+        auto frag = [&](int i) { return w8a8::buf_load16(im, lane * 16, i * 1024); };
+        x.kh = frag(wave);
+        x.kl = frag(NS + wave);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[e] = __builtin_amdgcn_raw_buffer_load_b16(rv, v_off[e], 0, 0);
+        x.qh = frag(2 * NS + wave);
+        x.ql = frag(3 * NS + wave);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            x.decay[i] = __builtin_bit_cast(f32x4, w8a8::buf_load16(im, g * 16, Image<DP>::kFrags * 1024 + 128 * wave + 64 * i));
+        x.t = frag(6 * NS);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) x.lk[i] = frag(4 * NS + 2 * wave + i);
+        x.p = w8a8::buf_load16(im, p_off, (6 * NS + 1) * 1024);
+        const bool more = left > kC;
+        left -= more ? kC : 0;
+        im_next += more ? kBuf : 0;
+        v_next += more ? (int64_t)kC * a.ldq : 0;
+    };
+    // O of the chunk before: this wave's rows of the four of each lane (of eight waves the upper four do the lower
+    // ones' rows once more, with the same words)
+    constexpr int kRows = W < 4 ? 4 / W : 1;
+    uint16_t* o_next = out - (int64_t)kC * ldo;
+    int o_left = a.seq + kC;
+    auto fetch_o = [&](int c, float (&part)[kRows][W]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i)
+#pragma unroll
+            for (int w = 0; w < W; ++w) part[i][w] = reinterpret_cast<const float*>(&part_o[c & 1][w][lane])[(wave + W * i) % 4];
+    };
+    auto put_o = [&](const float (&part)[kRows][W]) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t r = w8a8::make_rsrc(o_next, o_left > a.seq ? 0 : min(kC, o_left) * ldo * 2);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            float o = part[i][0];
+#pragma unroll
+            for (int w = 1; w < W; ++w) o += part[i][w];
+            __builtin_amdgcn_raw_buffer_store_b16(w8a8::f32_to_bf16(o), r, o_off + (uint32_t)((wave + W * i) % 4 * ldo) * 2, 0, 0);
+        }
+        o_next += (int64_t)kC * ldo;
+        o_left -= kC;
+    };
+    auto step = [&](Chunk& x, Chunk& next, int c) __attribute__((always_inline)) {
+        u32x4 sh, sl;
+        {
+            const u32x4 p0 = split4(st[0]), p1 = split4(st[1]);
+            sh = u32x4{p0[0], p0[1], p1[0], p1[1]};
+            sl = u32x4{p0[2], p0[3], p1[2], p1[3]};
+        }
+        f32x4 y = {0, 0, 0, 0}, o = {0, 0, 0, 0};
+        y = mfma16(x.kh, sh, y);
+        y = mfma16(x.kl, sh, y);
+        y = mfma16(x.kh, sl, y);
+        part_y[c & 1][wave][lane] = y;
+        o = mfma16(x.qh, sh, o);
+        __syncthreads();
+        f32x4 py[W];
+        float po[kRows][W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) py[w] = part_y[c & 1][w][lane];
+        fetch_o(c - 1, po);
+        __builtin_amdgcn_sched_barrier(0);   // these first, the rest while they are under way
+        load(next);
+        o = mfma16(x.ql, sh, o);
+        o = mfma16(x.qh, sl, o);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st[i][e] *= x.decay[i][e];
+        __builtin_amdgcn_sched_barrier(0);
+        y = py[0];
+#pragma unroll
+        for (int w = 1; w < W; ++w) y += py[w];
+        f32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = w8a8::bf16_to_f32(x.v[e]) - y[e];
+        const u32x4 rs = split4(r);
+        f32x4 u = {0, 0, 0, 0};
+        u = mfma16(x.t, u32x4{rs[0], rs[1], rs[0], rs[1]}, u);
+        u = mfma16(x.t, u32x4{rs[2], rs[3], rs[2], rs[3]}, u);
+        put_o(po);
+        __builtin_amdgcn_sched_barrier(0);
+        const u32x4 us = split4(u), uh = {us[0], us[1], us[0], us[1]}, ul = {us[2], us[3], us[2], us[3]};
+        st[0] = mfma16(x.lk[0], uh, st[0]);
+        st[1] = mfma16(x.lk[1], uh, st[1]);
+        st[0] = mfma16(x.lk[0], ul, st[0]);
+        st[1] = mfma16(x.lk[1], ul, st[1]);
+        o = mfma16(x.p, uh, o);
+        o = mfma16(x.p, ul, o);
+        part_o[c & 1][wave][lane] = o;
+    };
+    Chunk x[kAhead + 1];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+        load(x[i]);
+        __builtin_amdgcn_sched_barrier(0);   // (in this order, so that the loop's waits can count)
+    }
+    static_assert(kAhead == 3, "the walk's turns");
+    int c = 0;
+    for (; c + 4 <= chunks; c += 4) {   // (no way out in between: where paths meet, every load would be waited for)
+        step(x[0], x[3], c);
+        step(x[1], x[0], c + 1);
+        step(x[2], x[1], c + 2);
+        step(x[3], x[2], c + 3);
+    }
+    if (c < chunks) step(x[0], x[3], c);
+    if (c + 1 < chunks) step(x[1], x[0], c + 1);
+    if (c + 2 < chunks) step(x[2], x[1], c + 2);
+    __syncthreads();
+    float po[kRows][W];
+    fetch_o(chunks - 1, po);
+    put_o(po);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int d = 32 * wave + 16 * i + 4 * g + e;
+            if (d < a.dp) state[(int64_t)d * a.vp] = st[i][e];
+        }
+}
+
 // VT: 16-column value tiles per wave
 template <int DP, int VT>
 __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void delta_walk_kernel(DeltaArgs a, int chunks) {
@@ -620,6 +790,15 @@ void chunk_t(const DeltaArgs& a, hipStream_t stream) {
     (void)once;
     const int chunks = (a.seq + kC - 1) / kC;
     delta_prep_kernel<DP><<<dim3((unsigned)chunks, (unsigned)a.heads, (unsigned)a.batch), kPrepThreads, shared, stream>>>(a, chunks);
+    // Up to 512 blocks of 16 columns (two workgroups to a compute unit, all resident) a chunk's latency decides, past
+    // that the work. 128 x 128, both products, split / general: 64 blocks x 4096 tokens 210 / 416 us, 512 x 1024
+    // 117 / 148, 1024 x 1024 265 / 206; 256 x 256: 512 x 1024 202 / 238, 1024 x 1024 453 / 320. (Small heads still
+    // gain a little at 1024 blocks: 64 x 64, 512 tokens 115 / 121.)
+    const int tiles = a.vp / 16, groups = (a.batch * a.heads + 7) / 8;
+    if ((int64_t)a.batch * a.heads * tiles <= 512) {
+        delta_walk_split_kernel<DP><<<(unsigned)(groups * 8 * tiles), 2 * DP, 0, stream>>>(a, chunks);
+        return;
+    }
     // wide slices read every image once; narrow ones make more workgroups
     if (DP <= 128 && a.vp > 64 && (int64_t)a.batch * a.heads >= 256) walk_t<DP, 2>(a, chunks, stream);
     else walk_t<DP, 1>(a, chunks, stream);
