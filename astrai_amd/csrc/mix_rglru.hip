@@ -85,7 +85,18 @@ __global__ __launch_bounds__(256, 3) void rglru_chunk_kernel(RglruArgs a, int cs
                     s = state[ch];
                 } else {
                     s = slot(a.nseg - 1, 1)[ch];
-                    for (int j = 0; j < seg; ++j) s = fmaf(slot(j, 0)[ch], s, slot(j, 1)[ch]);
+                    for (int j = 0; j < seg; j += 8) {   // (eight at a time: the loads are under way together)
+                        float da[8], db[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const int from = min(j + i, seg - 1);
+                            da[i] = slot(from, 0)[ch];
+                            db[i] = slot(from, 1)[ch];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            if (j + i < seg) s = fmaf(da[i], s, db[i]);
+                    }
                 }
             } else if (last) {
                 slot(seg, 1)[ch] = state[ch];
@@ -349,10 +360,11 @@ void chunk_t(const RglruArgs& a, hipStream_t stream) {
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     }();
     (void)once;
-    // parts of a block's outputs: until there are about two workgroups per CU, each wave keeping a tile
+    // parts of a block's outputs: until there are about two workgroups per CU, each wave keeping as many tiles as the
+    // others (16 channel tiles over 12 waves, 4096 tokens: 98 us, over 8 waves 65)
     const int most = (a.bp + 63) / 64;
     int csplit = 1;
-    while (csplit < most && (int64_t)a.nseg * a.blocks * a.batch * csplit < 512) ++csplit;
+    while (csplit < most && ((int64_t)a.nseg * a.blocks * a.batch * csplit < 512 || most % csplit)) ++csplit;
     const dim3 grid((unsigned)a.nseg, (unsigned)(a.blocks * csplit), (unsigned)a.batch);
     if (a.nseg > 1) rglru_chunk_kernel<NT, false><<<grid, 256, shared, stream>>>(a, csplit);
     rglru_chunk_kernel<NT, true><<<grid, 256, shared, stream>>>(a, csplit);
