@@ -176,23 +176,53 @@ int astrai_w8a8_amax_ring_push(float* hist, int n, int idx, const float* amax, f
     return check_launch("amax_ring_push");
 }
 
+namespace {
+int check_quantize_transpose(const char* what, const void* x, const void* x8, const void* x8t, const float* scale,
+                             int64_t rows, int64_t cols, int fmt) {
+    if (!x || !x8t || !scale) return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
+    if (rows < 0 || cols < 0 || rows > (int64_t)65535 * 128 || cols > ((int64_t)1 << 31) - 64)
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: bad dims", what);
+    if (fmt != ASTRAI_W8A8_E4M3 && fmt != ASTRAI_W8A8_E5M2)
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmt must be 0 (e4m3) or 1 (e5m2)", what);
+    if (!aligned16(x) || !aligned16(x8t) || (x8 && !aligned16(x8)))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
+    return ASTRAI_W8A8_OK;
+}
+}  // namespace
+
 int astrai_w8a8_quantize_transpose_bf16_fp8(const void* x, void* x8, void* x8t, const float* scale,
                                             float* amax, int64_t rows, int64_t cols, int fmt,
                                             void* stream) {
-    if (!x || !x8t || !scale)
-        return fail(ASTRAI_W8A8_BAD_ARG, "quantize_transpose_bf16_fp8: null pointer");
-    if (rows < 0 || cols < 0 || rows > (int64_t)65535 * 128 || cols > ((int64_t)1 << 31) - 64)
-        return fail(ASTRAI_W8A8_BAD_ARG, "quantize_transpose_bf16_fp8: bad dims");
-    if (fmt != ASTRAI_W8A8_E4M3 && fmt != ASTRAI_W8A8_E5M2)
-        return fail(ASTRAI_W8A8_BAD_ARG,
-                    "quantize_transpose_bf16_fp8: fmt must be 0 (e4m3) or 1 (e5m2)");
-    if (!aligned16(x) || !aligned16(x8t) || (x8 && !aligned16(x8)))
-        return fail(ASTRAI_W8A8_BAD_ARG,
-                    "quantize_transpose_bf16_fp8: pointers must be 16-byte aligned");
-    if (rows == 0 || cols == 0) return ASTRAI_W8A8_OK;
-    w8a8::launch_quantize_transpose_fp8(x, x8, x8t, scale, amax, rows, cols, fmt,
+    const int rc = check_quantize_transpose("quantize_transpose_bf16_fp8", x, x8, x8t, scale, rows, cols, fmt);
+    if (rc != ASTRAI_W8A8_OK || rows == 0 || cols == 0) return rc;
+    w8a8::launch_quantize_transpose_fp8(x, x8, x8t, scale, amax, nullptr, nullptr, rows, cols, rows, fmt,
                                         static_cast<hipStream_t>(stream));
     return check_launch("quantize_transpose_bf16_fp8");
+}
+
+int astrai_w8a8_quantize_transpose_padded_bf16_fp8(const void* x, void* x8, void* x8t, const float* scale,
+                                                   float* maxima, float* colsums, int64_t rows, int64_t cols,
+                                                   int64_t ldt, int fmt, void* stream) {
+    const char* what = "quantize_transpose_padded_bf16_fp8";
+    const int rc = check_quantize_transpose(what, x, x8, x8t, scale, rows, cols, fmt);
+    if (rc != ASTRAI_W8A8_OK) return rc;
+    if (ldt < rows || ldt > (rows + 127) / 128 * 128 || (ldt != rows && ldt % 16 != 0))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: row length %lld for %lld rows", what, (long long)ldt, (long long)rows);
+    if (colsums && !maxima) return fail(ASTRAI_W8A8_BAD_ARG, "%s: column sums come with maxima", what);
+    if (rows == 0 || cols == 0) return ASTRAI_W8A8_OK;
+    w8a8::launch_quantize_transpose_fp8(x, x8, x8t, scale, nullptr, maxima, colsums, rows, cols, ldt, fmt,
+                                        static_cast<hipStream_t>(stream));
+    return check_launch(what);
+}
+
+int astrai_w8a8_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows,
+                               int64_t cols, void* stream) {
+    if ((amax && !maxima) || (bias && !colsums)) return fail(ASTRAI_W8A8_BAD_ARG, "gradient_stats: null pointer");
+    if (rows <= 0 || cols <= 0 || rows > (int64_t)65535 * 128 || cols > ((int64_t)1 << 31) - 64)
+        return fail(ASTRAI_W8A8_BAD_ARG, "gradient_stats: bad dims");
+    if (!amax && !bias) return ASTRAI_W8A8_OK;
+    w8a8::launch_gradient_stats(maxima, amax, colsums, bias, rows, cols, static_cast<hipStream_t>(stream));
+    return check_launch("gradient_stats");
 }
 
 int astrai_w8a8_quantize_bf16_int8_rows(const void* x, void* xq, float* s, int64_t rows,

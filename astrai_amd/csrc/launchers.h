@@ -62,8 +62,14 @@ void launch_amax_ring_push(float* hist, int n, int idx, const float* amax, const
 void launch_amax_bf16(const void* x, float* amax, float* partials, int64_t total, hipStream_t stream);
 // codes of a [rows, cols] matrix row-major (x8, may be null) and transposed (x8t, [cols, rows])
 void launch_quantize_transpose_fp8(const void* x, void* x8, void* x8t, const float* scale,
-                                   float* amax, int64_t rows, int64_t cols, int fmt,
-                                   hipStream_t stream);
+                                   float* amax, float* maxima, float* colsums, int64_t rows, int64_t cols,
+                                   int64_t ldt, int fmt, hipStream_t stream);
+// workgroups of that launch, each of which writes one of `maxima`
+constexpr int kGradientMaxima = 2048;
+int quantize_transpose_blocks(int64_t rows, int64_t cols);
+// amax (or null) from the maxima, the bias gradient (or null) from the column sums of that launch
+void launch_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows, int64_t cols,
+                           hipStream_t stream);
 void launch_quantize_int8_rows(const void* x, void* xq, float* s, int64_t rows, int64_t k,
                                hipStream_t stream);
 // fused producers: (residual add +) RMSNorm + per-row int8; SwiGLU product + per-row

@@ -247,19 +247,26 @@ __global__ __launch_bounds__(kWave) void amax_ring_push_kernel(
 // 256-byte runs in, 128-byte runs out in both layouts. A thread converts 4 rows
 // x 8 columns per pass, packs the four rows of each column into a dword and
 // writes it to a column-major LDS tile (pitch 132 bytes); the tile then leaves
-// as 16-byte pieces of the transposed rows.
+// as 16-byte pieces of the transposed rows. A transposed row may be longer than `rows` (up to whole tiles):
+// zero codes fill it, so that the contraction over it has the length that the large products take.
+// STATS (the gradient): the workgroup's maximum goes to maxima[blockIdx.x], the tile's column sums in fp32 to
+// colsums[row tile][column]; gradient_stats_kernel finishes both. The values are in registers anyway: a reduction
+// of the whole matrix for the bias gradient was another read of it, the maximum through one cleared slot a fill
+// launch (backward of 4096 x 4096 weights, 4096 tokens: 169 us, here 153).
 constexpr int kTrRows = 128, kTrCols = 128, kTrPitch = kTrRows + 4;
 
-template <int Fmt>
+template <int Fmt, bool STATS>
 __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
     const uint16_t* __restrict__ x, uint8_t* __restrict__ x8, uint8_t* __restrict__ x8t,
-    const float* __restrict__ scale, float* __restrict__ amax, int64_t rows, int64_t cols) {
+    const float* __restrict__ scale, float* __restrict__ amax, float* __restrict__ colsums, int64_t rows,
+    int64_t cols, int64_t ldt) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[kTrCols * kTrPitch];
     __shared__ float slots[kThreads / kWave];
+    [[maybe_unused]] __shared__ float sums[STATS ? kThreads / kWave : 1][STATS ? kTrCols : 1];
     const int cc = threadIdx.x & 15, r4 = threadIdx.x >> 4;
     const float step = *scale;
     const bool vec = (cols & 7) == 0;
-    const bool runs = (rows & 15) == 0;  // 16-byte pieces stay aligned and inside the matrix
+    const bool runs = (ldt & 15) == 0;  // 16-byte pieces stay aligned and inside the matrix
     const int64_t tiles_x = (cols + kTrCols - 1) / kTrCols;
     const int64_t ntiles = tiles_x * ((rows + kTrRows - 1) / kTrRows);
     float local = 0.0f;
@@ -268,6 +275,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
         const int64_t c = c0 + cc * 8;
         // all eight 16-byte pieces of the thread requested before the first is converted
         u32x4 raw[2][4];
+        [[maybe_unused]] float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         const bool col_in = vec && c < cols;
 #pragma unroll
         for (int pass = 0; pass < 2; ++pass)
@@ -293,6 +301,10 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
                         if (c + j < cols) f[j] = bf16_to_f32(x[r * cols + c + j]);
                 }
                 local = fmaxf(local, amax8(f));
+                if constexpr (STATS) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) sum[j] += f[j];
+                }
                 q[i] = quant8_fp8<Fmt>(f, step);
                 if (x8) {
                     if (whole) {
@@ -321,12 +333,29 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
                     *reinterpret_cast<uint32_t*>(tile + (cc * 8 + half * 4 + j) * kTrPitch + pass * 64 + r4 * 4) = d[j];
             }
         }
+        if constexpr (STATS) {   // over the wave's four row groups (lanes 16 apart)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                sum[j] += __shfl_xor(sum[j], 16, kWave);
+                sum[j] += __shfl_xor(sum[j], 32, kWave);
+            }
+            if ((threadIdx.x & 63) < 16) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) sums[threadIdx.x >> 6][cc * 8 + j] = sum[j];
+            }
+        }
         __syncthreads();
+        if constexpr (STATS) {
+            const int64_t cs = c0 + threadIdx.x;
+            if (colsums && threadIdx.x < kTrCols && cs < cols)
+                colsums[(t / tiles_x) * cols + cs] =
+                    (sums[0][threadIdx.x] + sums[1][threadIdx.x]) + (sums[2][threadIdx.x] + sums[3][threadIdx.x]);
+        }
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
             const int cl = (threadIdx.x >> 3) + 32 * h;
             const int64_t ct = c0 + cl, rt = r0 + (threadIdx.x & 7) * 16;
-            if (ct >= cols || rt >= rows) continue;
+            if (ct >= cols || rt >= ldt) continue;
             const uint8_t* src = tile + cl * kTrPitch + (threadIdx.x & 7) * 16;
             u32x4 v;
             v.x = *reinterpret_cast<const uint32_t*>(src);
@@ -334,18 +363,18 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
             v.z = *reinterpret_cast<const uint32_t*>(src + 8);
             v.w = *reinterpret_cast<const uint32_t*>(src + 12);
             if (runs) {
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(x8t + ct * rows + rt));
+                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(x8t + ct * ldt + rt));
             } else {
                 const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                 for (int b = 0; b < 16; ++b)
-                    if (rt + b < rows)
-                        x8t[ct * rows + rt + b] = (uint8_t)((w[b >> 2] >> ((b & 3) * 8)) & 0xffu);
+                    if (rt + b < ldt)
+                        x8t[ct * ldt + rt + b] = (uint8_t)((w[b >> 2] >> ((b & 3) * 8)) & 0xffu);
             }
         }
         // the first tile's maximum goes out early when more tiles follow (block_max also
         // separates this tile's LDS reads from the next tile's writes)
-        if (amax && t == blockIdx.x && t + gridDim.x < ntiles && gridDim.x >= 64 &&
+        if (!STATS && amax && t == blockIdx.x && t + gridDim.x < ntiles && gridDim.x >= 64 &&
             blockIdx.x % kEarlyEvery == 0)
             publish_early(amax, local, slots);
         else
@@ -353,8 +382,37 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
     }
     if (amax) {
         const float m = block_max(local, slots);
-        if (threadIdx.x == 0) atomic_max_nonneg(amax, m);
+        if constexpr (STATS) {
+            if (threadIdx.x == 0) amax[blockIdx.x] = m;
+        } else {
+            if (threadIdx.x == 0) atomic_max_nonneg(amax, m);
+        }
     }
+}
+
+// What the gradient's quantizer left: bias gradients from the column sums of `tiles` row tiles (64 columns to a
+// workgroup, four tiles at a time), the last workgroup takes the maximum over `nmax` workgroups' maxima.
+__global__ __launch_bounds__(kThreads) void gradient_stats_kernel(const float* __restrict__ maxima, int nmax,
+                                                                  float* __restrict__ amax,
+                                                                  const float* __restrict__ colsums, int64_t tiles,
+                                                                  uint16_t* __restrict__ bias, int64_t cols) {
+    __shared__ float part[kThreads / kWave][kWave];
+    __shared__ float slots[kThreads / kWave];
+    if (amax && blockIdx.x == gridDim.x - 1) {
+        float m = 0.0f;
+        for (int i = threadIdx.x; i < nmax; i += kThreads) m = fmaxf(m, maxima[i]);
+        m = block_max(m, slots);
+        if (threadIdx.x == 0) *amax = m;
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t c = (int64_t)blockIdx.x * kWave + lane;
+    float s = 0.0f;
+    if (c < cols)
+        for (int64_t t = wave; t < tiles; t += kThreads / kWave) s += colsums[t * cols + c];
+    part[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && c < cols) bias[c] = f32_to_bf16((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]));
 }
 
 // ---- per-row int8 ---------------------------------------------------------
@@ -898,19 +956,31 @@ void launch_amax_bf16(const void* x, float* amax, float* partials, int64_t total
 }
 
 void launch_quantize_transpose_fp8(const void* x, void* x8, void* x8t, const float* scale,
-                                   float* amax, int64_t rows, int64_t cols, int fmt,
-                                   hipStream_t stream) {
+                                   float* amax, float* maxima, float* colsums, int64_t rows, int64_t cols,
+                                   int64_t ldt, int fmt, hipStream_t stream) {
     if (rows <= 0 || cols <= 0) return;
-    // a workgroup per tile while they are all resident at once (eight per compute unit)
-    const int64_t ntiles = ((cols + kTrCols - 1) / kTrCols) * ((rows + kTrRows - 1) / kTrRows);
-    const dim3 grid((unsigned)(ntiles <= 2048 ? ntiles : 2048));
+    const dim3 grid((unsigned)quantize_transpose_blocks(rows, cols));
     auto* xi = static_cast<const uint16_t*>(x);
     auto* o = static_cast<uint8_t*>(x8);
     auto* ot = static_cast<uint8_t*>(x8t);
-    if (fmt == 0)
-        quantize_transpose_fp8_kernel<0><<<grid, dim3(kThreads), 0, stream>>>(xi, o, ot, scale, amax, rows, cols);
-    else
-        quantize_transpose_fp8_kernel<1><<<grid, dim3(kThreads), 0, stream>>>(xi, o, ot, scale, amax, rows, cols);
+    auto run = [&](auto kern, float* a) { kern<<<grid, dim3(kThreads), 0, stream>>>(xi, o, ot, scale, a, colsums, rows, cols, ldt); };
+    if (maxima) run(fmt ? quantize_transpose_fp8_kernel<1, true> : quantize_transpose_fp8_kernel<0, true>, maxima);
+    else run(fmt ? quantize_transpose_fp8_kernel<1, false> : quantize_transpose_fp8_kernel<0, false>, amax);
+}
+
+// a workgroup per tile while they are all resident at once (eight per compute unit)
+int quantize_transpose_blocks(int64_t rows, int64_t cols) {
+    const int64_t ntiles = ((cols + kTrCols - 1) / kTrCols) * ((rows + kTrRows - 1) / kTrRows);
+    return (int)(ntiles <= kGradientMaxima ? ntiles : kGradientMaxima);
+}
+
+void launch_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows, int64_t cols,
+                           hipStream_t stream) {
+    const int64_t blocks = (bias ? (cols + kWave - 1) / kWave : 0) + (amax ? 1 : 0);
+    if (rows <= 0 || cols <= 0 || blocks <= 0) return;
+    gradient_stats_kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(
+        maxima, quantize_transpose_blocks(rows, cols), amax, colsums, (rows + kTrRows - 1) / kTrRows,
+        static_cast<uint16_t*>(bias), cols);
 }
 
 void launch_quantize_int8_rows(const void* x, void* xq, float* s, int64_t rows, int64_t k,

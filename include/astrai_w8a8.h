@@ -117,6 +117,22 @@ int astrai_w8a8_quantize_transpose_bf16_fp8(const void* x_bf16, void* x8, void* 
                                             int64_t cols, int fmt, void* stream);
 
 /*
+ * The same with transposed rows of ldt codes, rows <= ldt <= rows rounded up to whole 128 (a multiple
+ * of 16 where it is more than rows): zeros follow the rows' codes, which changes nothing in a
+ * contraction over them. maxima (may be NULL): 2048 floats, of which the launch writes one maximum
+ * per workgroup; colsums (may be NULL, needs maxima): ceil(rows / 128) x cols floats, the column sums
+ * of each 128 rows. astrai_w8a8_gradient_stats turns them into amax[1] and / or the column sums of
+ * the whole matrix in bf16 (either may be NULL): the bias gradient of a Linear.
+ */
+#define ASTRAI_W8A8_GRADIENT_MAXIMA 2048
+int astrai_w8a8_quantize_transpose_padded_bf16_fp8(const void* x_bf16, void* x8, void* x8t,
+                                                   const float* scale, float* maxima, float* colsums,
+                                                   int64_t rows, int64_t cols, int64_t ldt, int fmt,
+                                                   void* stream);
+int astrai_w8a8_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias_bf16,
+                               int64_t rows, int64_t cols, void* stream);
+
+/*
  * bf16 -> int8, symmetric, one scale per row (per token for activations, per
  * output channel for weights). No counterpart in the reference (it has no int8
  * path); same conventions as the fp8 quantizer.
