@@ -21,8 +21,8 @@
 //     probabilities it needs from the lanes that hold them (same 16-lane group).
 //   The waves' and lane groups' partial (max, sum, acc) are merged through LDS and
 //   written to a workspace.
-// Kernel 2 merges the splits of a token and writes bf16.
-#include "common.cuh"
+// Kernel 2 merges the splits of a token and writes bf16 (without a split kernel 1 writes it).
+#include "attn_merge.cuh"
 #include "launchers.h"
 
 namespace w8a8 {
@@ -240,6 +240,29 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
         }
     }
     __syncthreads();
+    if (a.nsplit == 1 && !a.out_q) {
+        // the whole context was this workgroup's: nothing to merge (128 sequences x 200 keys, 16 / 4 heads: 16.0 us with
+        // the second launch, 12.6 without); thread -> (query, two dims)
+        for (int e = threadIdx.x * 2; e < nq * kD; e += 512) {
+            const int q = e / kD, d = e - q * kD;
+            float mm = kNegBig;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sh_ml[w][q][0]);
+            float v0 = 0.0f, v1 = 0.0f, ll = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const float f = __expf(sh_ml[w][q][0] - mm);
+                v0 += sh_acc[w][q][d] * f;
+                v1 += sh_acc[w][q][d + 1] * f;
+                ll += sh_ml[w][q][1] * f;
+            }
+            const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;  // a token with no visible key yields zeros
+            const int64_t token = (int64_t)b * a.seq + q % a.seq;
+            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(a.out) + (token * a.n_heads + hk * n_rep + q / a.seq) * kD + d) =
+                pack_bf16x2(v0 * inv, v1 * inv);
+        }
+        return;
+    }
     // merge the four waves; thread -> (query, dim)
     float* ws = a.ws + (int64_t)blockIdx.x * NQ * kWsRow;
     for (int e = threadIdx.x; e < NQ * kD; e += 256) {
@@ -263,7 +286,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
 }
 
 // One workgroup per (batch, token): all heads, 8 output values per thread and
-// pass. Besides (or instead of) the bf16 row it can emit the per-token int8
+// pass. Besides (or instead of) the bf16 row it emits the per-token int8
 // quantization of that row -- the input of the int8 output projection -- computed
 // on the bf16-rounded values, i.e. what the separate quantizer would produce.
 constexpr int kMergeCache = 4;  // rows up to 4 * 256 * 8 = 8192 wide stay in registers
@@ -314,7 +337,6 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(AttnDecodeArgs a
 #pragma unroll
         for (int d = 0; d < 8; ++d) local = fmaxf(local, fabsf(keep[c][d]));
     }
-    if (!a.out_q) return;
     // per-token int8: step = max(amax, 1e-12) / 127, round half to even, clamp
     const float step = fmaxf(merge_block_max(local, slots), 1e-12f) / 127.0f;
     if (threadIdx.x == 0) a.out_scale[blockIdx.x] = step;
@@ -336,6 +358,30 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(AttnDecodeArgs a
     }
 }
 
+// bf16 output alone: a workgroup takes a few heads of a token
+template <int NQ>
+__global__ __launch_bounds__(256) void attn_decode_merge_heads_kernel(AttnDecodeArgs a) {
+    const MergeShape<kD> shape(a.nsplit, a.n_heads);
+    const int n_rep = a.n_heads / a.n_kv_heads, per_token = a.n_heads / shape.heads;
+    const int h0 = (int)blockIdx.x % per_token * shape.heads, token = (int)blockIdx.x / per_token;
+    const int b = token / a.seq, s = token % a.seq;
+    merge_splits<kD>(shape, [&](int i) {
+        const int hk = (h0 + i) / n_rep, q = (h0 + i - hk * n_rep) * a.seq + s;
+        return a.ws + ((int64_t)(b * a.n_kv_heads + hk) * a.nsplit) * NQ * kWsRow + q * kWsRow;
+    }, NQ * kWsRow, a.nsplit, static_cast<uint16_t*>(a.out) + ((int64_t)token * a.n_heads + h0) * kD);
+}
+
+template <int NQ>
+void launch_merge(const AttnDecodeArgs& a, hipStream_t stream) {
+    const unsigned tokens = (unsigned)(a.batch * a.seq);
+    if (a.out_q) {
+        attn_decode_merge_kernel<NQ><<<dim3(tokens), dim3(256), 0, stream>>>(a);
+    } else if (a.nsplit > 1) {
+        const MergeShape<kD> shape(a.nsplit, a.n_heads);
+        attn_decode_merge_heads_kernel<NQ><<<dim3(tokens * (unsigned)(a.n_heads / shape.heads)), dim3(256), 0, stream>>>(a);
+    }
+}
+
 }  // namespace
 
 int64_t attn_decode_workspace_floats(int batch, int n_kv_heads, int nsplit, int nq) {
@@ -349,7 +395,6 @@ bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream) {
     if (a.head_dim != kD || nq > 8 || nq <= 0 || a.nsplit <= 0) return false;
     if (a.n_heads * kD > kMergeCache * 256 * 8) return false;  // the merge kernel keeps a token's row in registers
     const unsigned grid1 = (unsigned)(a.batch * a.n_kv_heads * a.nsplit);
-    const unsigned grid2 = (unsigned)(a.batch * a.seq);
     const bool paged = a.req_to_token != nullptr;
     if (paged && (a.seq != 1 || !a.req_pool_indices || !a.kv_indptr || a.rtt_stride <= 0)) return false;
     if (a.mask && (!paged || a.mask_width <= 0)) return false;
@@ -360,7 +405,7 @@ bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream) {
             attn_decode_partial_kernel<4, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
         else
             attn_decode_partial_kernel<4, false><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        attn_decode_merge_kernel<4><<<dim3(grid2), dim3(256), 0, stream>>>(a);
+        launch_merge<4>(a, stream);
     } else {
         if (paged && a.mask)
             attn_decode_partial_kernel<8, true, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
@@ -368,7 +413,7 @@ bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream) {
             attn_decode_partial_kernel<8, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
         else
             attn_decode_partial_kernel<8, false><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        attn_decode_merge_kernel<8><<<dim3(grid2), dim3(256), 0, stream>>>(a);
+        launch_merge<8>(a, stream);
     }
     return true;
 }

@@ -24,7 +24,7 @@
 // value tile through LDS. Correct for every shape, not tuned like the head_dim-128 kernels.
 #include <climits>
 
-#include "common.cuh"
+#include "attn_merge.cuh"
 #include "launchers.h"
 
 namespace w8a8 {
@@ -464,42 +464,24 @@ __global__ __launch_bounds__(256) void attn_rows_shared_kernel(AttnRowsArgs a) {
             u32x2{pack_bf16x2(o[c][0] * inv, o[c][1] * inv), pack_bf16x2(o[c][2] * inv, o[c][3] * inv)};
 }
 
-// With a context split: one workgroup per query row slot of the schedule (decode: per
-// sequence) merges the splits of every head of the row and writes out[row, head, :] in bf16.
+// With a context split: the splits of a query row slot of the schedule (decode: of a sequence), a few heads to a
+// workgroup, to out[row, head, :] in bf16.
 template <int D>
 __global__ __launch_bounds__(256) void attn_rows_merge_kernel(AttnRowsArgs a) {
     constexpr int WS_ROW = D + 2;
-    const int n_rep = a.n_heads / a.n_kv_heads;
+    const MergeShape<D> shape(a.nsplit, a.n_heads);
+    const int n_rep = a.n_heads / a.n_kv_heads, per_row = a.n_heads / shape.heads;
     const int rows = a.rows_per_block;
     const int slots_per_block = a.qo_indptr ? rows : 1;
-    const int block = blockIdx.x / slots_per_block, q_s = blockIdx.x - block * slots_per_block;
+    const int h0 = (int)(blockIdx.x % per_row) * shape.heads, item = (int)(blockIdx.x / per_row);
+    const int block = item / slots_per_block, q_s = item - block * slots_per_block;
     const RowBlock rb = row_block(a, block);
     const int row = rb.r0 + q_s;
     if (row >= rb.q_len) return;
-    const int width = a.n_heads * D;
-    uint16_t* out = static_cast<uint16_t*>(a.out) + (int64_t)(rb.q_start + row) * width;
-    for (int e = threadIdx.x * 8; e < width; e += 256 * 8) {
-        const int h = e / D, d0 = e - h * D;
-        const int hk = h / n_rep, q = (h - hk * n_rep) * rows + q_s;
-        const float* base = a.ws + (((int64_t)block * a.n_kv_heads + hk) * a.nsplit) * kNQ * WS_ROW + q * WS_ROW;
-        float mm = kNegBig;
-        for (int j = 0; j < a.nsplit; ++j) mm = fmaxf(mm, base[(int64_t)j * kNQ * WS_ROW + D]);
-        float v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, ll = 0.0f;
-        for (int j = 0; j < a.nsplit; ++j) {
-            const float* r = base + (int64_t)j * kNQ * WS_ROW;
-            const float f = __expf(r[D] - mm);
-            ll += r[D + 1] * f;
-#pragma unroll
-            for (int d = 0; d < 8; ++d) v[d] += r[d0 + d] * f;
-        }
-        const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;  // a row with no visible key yields zeros
-        u32x4 ov;
-        ov.x = pack_bf16x2(v[0] * inv, v[1] * inv);
-        ov.y = pack_bf16x2(v[2] * inv, v[3] * inv);
-        ov.z = pack_bf16x2(v[4] * inv, v[5] * inv);
-        ov.w = pack_bf16x2(v[6] * inv, v[7] * inv);
-        *reinterpret_cast<u32x4*>(out + e) = ov;
-    }
+    merge_splits<D>(shape, [&](int i) {
+        const int hk = (h0 + i) / n_rep, q = (h0 + i - hk * n_rep) * rows + q_s;
+        return a.ws + (((int64_t)block * a.n_kv_heads + hk) * a.nsplit) * kNQ * WS_ROW + q * WS_ROW;
+    }, kNQ * WS_ROW, a.nsplit, static_cast<uint16_t*>(a.out) + ((int64_t)(rb.q_start + row) * a.n_heads + h0) * D);
 }
 
 template <int D>
@@ -517,7 +499,10 @@ void launch_for_dim(const AttnRowsArgs& a, unsigned grid1, unsigned grid2, hipSt
         attn_rows_partial_kernel<D, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
     else
         attn_rows_partial_kernel<D, false><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-    if (a.nsplit > 1) attn_rows_merge_kernel<D><<<dim3(grid2), dim3(256), 0, stream>>>(a);
+    if (a.nsplit > 1) {
+        const MergeShape<D> shape(a.nsplit, a.n_heads);
+        attn_rows_merge_kernel<D><<<dim3(grid2 * (unsigned)(a.n_heads / shape.heads)), dim3(256), 0, stream>>>(a);
+    }
 }
 
 }  // namespace
@@ -563,7 +548,7 @@ bool launch_attn_rows(AttnRowsArgs a, hipStream_t stream) {
     a.num_items = blocks * a.n_kv_heads * a.nsplit;  // one wave each, four to a workgroup
     const int64_t grid1 = (a.num_items + 3) / 4;
     const int64_t grid2 = prefill ? blocks * a.rows_per_block : blocks;
-    if (grid1 > INT_MAX || grid2 > INT_MAX) return false;
+    if (grid1 > INT_MAX || (a.nsplit > 1 ? grid2 * a.n_heads : grid2) > INT_MAX) return false;
     switch (a.head_dim) {
         case 32: launch_for_dim<32>(a, (unsigned)grid1, (unsigned)grid2, stream); break;
         case 64: launch_for_dim<64>(a, (unsigned)grid1, (unsigned)grid2, stream); break;

@@ -878,6 +878,16 @@ def decode_nsplit(pairs: int, max_keys: int) -> int:
     return max(1, min(8, 512 // max(1, pairs), max_keys // 160))
 
 
+def paged_nsplit(pairs: int, max_keys: int) -> int:
+    """:func:`decode_nsplit` of a paged step, whose bf16 output a merge of any number of splits side by side writes: below
+    64 pairs as many splits as make 512 workgroups, none that could not hold 64 keys of the slot table's width (one
+    sequence of 8192 keys, 16 / 4 heads: 8 splits 36 us, 64 13; four of 3000: 8 splits 20, 32 13; from 64 pairs on
+    more than eight splits gain nothing: eight sequences of 8192, 32 / 8 heads 40 us with 8, 38 with 16)."""
+    if pairs >= 64:
+        return decode_nsplit(pairs, max_keys)
+    return max(1, min(64, 512 // max(1, pairs), max_keys // 64))
+
+
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
                 scale: Optional[float] = None, nsplit: int = 0, quantized: bool = False):
     """``q [batch, n_heads, seq, 128]`` (bf16) against the dense caches
@@ -1013,7 +1023,7 @@ def attn_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         scale = d ** -0.5
     user_nsplit = nsplit > 0
     if nsplit <= 0:
-        nsplit = decode_nsplit(b * hkv, req_to_token.size(1))
+        nsplit = paged_nsplit(b * hkv, req_to_token.size(1))
     with _on_device(q.device):
         if new_k is not None:
             if new_k.shape != (b, hkv, d) or new_v.shape != (b, hkv, d):
