@@ -838,6 +838,12 @@ int astrai_w8a8_gemm_int8_ptpc(const void* a, const void* b, const float* sa, co
     return check_launch("gemm_int8_ptpc");
 }
 
+int astrai_w8a8_linear_int8_bf16(const void* x, const void* wq, const float* sw, const void* bias, void* xq, float* sx,
+                                 void* out, int64_t m, int64_t n, int64_t k, void* stream) {
+    if (int rc = astrai_w8a8_quantize_bf16_int8_rows(x, xq, sx, m, k, stream)) return rc;
+    return astrai_w8a8_gemm_int8_ptpc(xq, wq, sx, sw, bias, out, m, n, k, ASTRAI_W8A8_OUT_BF16, stream);
+}
+
 int astrai_w8a8_gemm_int8_ptpc_resid(const void* a, const void* b, const float* sa, const float* sb,
                                      const void* bias, const void* resid, void* out, int64_t m,
                                      int64_t n, int64_t k, void* stream) {

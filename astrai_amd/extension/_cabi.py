@@ -91,6 +91,7 @@ PROTOTYPES = {
     "astrai_w8a8_gemm_fp8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_fp8_block128": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
+    "astrai_w8a8_linear_int8_bf16": ([_P] * 7 + [_I64] * 3 + [_P], _INT),
     "astrai_w8a8_gemv_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_tiled": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_rope_cache": (
@@ -1283,6 +1284,26 @@ def mm_int8(a: torch.Tensor, b: torch.Tensor, sa: Optional[torch.Tensor],
             else:
                 _check(fn(a_c.data_ptr(), b_c.data_ptr(), _ptr(sa), _ptr(sb), _ptr(bias),
                           out.data_ptr(), m, n, k, out_dtype, _stream(a)), lib)
+    return out
+
+
+def linear_int8(x: torch.Tensor, wq: torch.Tensor, sw: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``mm_int8`` of ``quantize_int8_rows(x)``, ``[..., N]``: one library call where the operands are as the kernels take
+    them."""
+    k, n, dev = x.size(-1), wq.size(0), x.device
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and k % 16 == 0 and x.numel() and n
+            and wq.dtype == torch.int8 and wq.dim() == 2 and wq.size(1) == k and wq.is_contiguous() and wq.device == dev
+            and sw.dtype == torch.float32 and sw.numel() == n and sw.is_contiguous() and sw.device == dev
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.numel() == n and bias.is_contiguous() and bias.device == dev))):
+        xq, sx = quantize_int8_rows(x)
+        return mm_int8(xq, wq, sx, sw, bias).reshape(*x.shape[:-1], n)
+    lib, m = _require(), x.numel() // k
+    with _on_device(dev):
+        codes = torch.empty(m * (k + 4), device=dev, dtype=torch.uint8)   # codes, then a step per row
+        out = torch.empty((*x.shape[:-1], n), device=dev, dtype=torch.bfloat16)
+        at = codes.data_ptr()
+        _check(lib.astrai_w8a8_linear_int8_bf16(x.data_ptr(), wq.data_ptr(), sw.data_ptr(), _ptr(bias), at, at + m * k,
+                                                out.data_ptr(), m, n, k, _stream(x)), lib)
     return out
 
 

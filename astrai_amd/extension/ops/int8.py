@@ -145,6 +145,14 @@ def linear_forward_int8(x, wq, sw, bias: Optional[torch.Tensor] = None) -> torch
     return out.reshape(*x.shape[:-1], wq.size(0))
 
 
+def linear_forward_int8_kernels(x, wq, sw, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`linear_forward_int8` for callers that are themselves a device kernel of a dispatcher op: autograd, tracing,
+    fake tensors, batching and dispatch modes are above them, so the two steps need no ops of their own (a call of each
+    costs the host 5 us) and share one library call (16 tokens through 4096 x 11008 weights, eager: 27.0 us with ops of
+    their own, 22.4 with two library calls, 14.8 with one; the kernels take 13)."""
+    return _mod().linear_int8(x, wq, sw, bias)
+
+
 @custom_op("custom::int8_add_rmsnorm_quantize", mutates_args=())
 def int8_add_rmsnorm_quantize(
     x: torch.Tensor, weight: torch.Tensor, eps: float, res: Optional[torch.Tensor] = None

@@ -21,6 +21,7 @@ import torch
 from astrai_amd.extension import dispatch
 from astrai_amd.extension.ops.int8 import (
     linear_forward_int8,
+    linear_forward_int8_kernels,
     quantize_int8_per_channel,
 )
 
@@ -114,10 +115,10 @@ def prepare_int8_weights(module: torch.nn.Module) -> int:
     return n
 
 
-def int8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
+def int8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, linear=linear_forward_int8) -> torch.Tensor:
     wq, sw = _state.get_weight(w)
     b = bias if (bias is not None and bias.numel()) else None
-    return linear_forward_int8(x, wq, sw, b)
+    return linear(x, wq, sw, b)
 
 
 def _int8_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -132,7 +133,7 @@ def _int8_handler(x, w, bias):
         and (bias is None or bias.dtype == torch.bfloat16)
         and _int8_supported(x, w)
     ):
-        return int8_linear_forward(x, w, bias)
+        return int8_linear_forward(x, w, bias, linear_forward_int8_kernels)
     return None
 
 

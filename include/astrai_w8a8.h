@@ -582,6 +582,14 @@ int astrai_w8a8_gemm_int8_ptpc(const void* a, const void* b, const float* sa,
                                void* stream);
 
 /*
+ * A Linear over bf16 rows in one call: quantize_bf16_int8_rows of x [m, k] into xq [m, k] and sx [m], then
+ * gemm_int8_ptpc of them with wq [n, k], sw [n] and the optional bias into out [m, n] bf16.
+ */
+int astrai_w8a8_linear_int8_bf16(const void* x_bf16, const void* wq, const float* sw, const void* bias_bf16,
+                                 void* xq, float* sx, void* out_bf16, int64_t m, int64_t n, int64_t k,
+                                 void* stream);
+
+/*
  * The decode int8 kernels on their own: same contract as
  * astrai_w8a8_gemm_int8_ptpc but requires M <= 128 and K % 256 == 0, and
  * returns ASTRAI_W8A8_UNSUPPORTED otherwise.
