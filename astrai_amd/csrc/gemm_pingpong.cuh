@@ -535,7 +535,10 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
                         if constexpr (ScaleKind == SCALE_TENSOR) f = f * (es.sa * es.sb);
                         else if constexpr (ScaleKind == SCALE_ROWCOL) f = f * sx * sw4[j];
                         else f = f * blk_s[mi];
-                        v[j] = add_bias(f, b4[j], g.round_first);
+                        // (a product rounded before its bias has per-tensor steps; a choice made here costs the
+                        // block-scaled products 0.7 us of 36)
+                        if constexpr (ScaleKind == SCALE_TENSOR) v[j] = g.round_first ? add_bias(f, b4[j], true) : f + b4[j];
+                        else v[j] = f + b4[j];
                     }
                     u32x2 pk;
                     pk.x = pack_bf16x2(v[0], v[1]);

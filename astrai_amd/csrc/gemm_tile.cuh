@@ -87,7 +87,10 @@ __device__ __forceinline__ void store_subtile(const GemmArgs& g, const EpilogueS
             const float sw = (n + j < g.n) ? g.sb[n + j] : 0.0f;
             f = f * sx * sw;
         }
-        if (bias && n + j < g.n) f = add_bias(f, bf16_to_f32(bias[n + j]), g.round_first);
+        if (bias && n + j < g.n) {
+            if constexpr (ScaleKind == SCALE_TENSOR) f = add_bias(f, bf16_to_f32(bias[n + j]), g.round_first);
+            else f += bf16_to_f32(bias[n + j]);
+        }
         v[j] = f;
     }
     const bool n_vec = (g.n & 3) == 0;
