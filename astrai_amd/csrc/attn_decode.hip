@@ -51,7 +51,9 @@ __device__ __forceinline__ int lane_read_i(int v, int src_lane) {
 // length kv_indptr[b+1] - kv_indptr[b] and one query token, the newest.
 // MASK (paged only): a bool tensor [batch, mask_width] picks the positions a sequence may
 // attend on top of its length (csrc/kernels/attention/mma_utils.cuh:196-199)
-template <int NQ, bool PAGED, bool MASK = false>
+// WHOLE: one split, bf16 output: the kernel writes the row itself (128 sequences x 200 keys, 16 / 4 heads: 16.0 us with a
+// merge launch behind it, 12.8 without)
+template <int NQ, bool PAGED, bool MASK, bool WHOLE>
 __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs a) {
     __shared__ float sh_acc[4][NQ][kD];
     __shared__ float sh_ml[4][NQ][2];
@@ -240,9 +242,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
         }
     }
     __syncthreads();
-    if (a.nsplit == 1 && !a.out_q) {
-        // the whole context was this workgroup's: nothing to merge (128 sequences x 200 keys, 16 / 4 heads: 16.0 us with
-        // the second launch, 12.6 without); thread -> (query, two dims)
+    if constexpr (WHOLE) {   // thread -> (query, two dims)
         for (int e = threadIdx.x * 2; e < nq * kD; e += 512) {
             const int q = e / kD, d = e - q * kD;
             float mm = kNegBig;
@@ -376,9 +376,27 @@ void launch_merge(const AttnDecodeArgs& a, hipStream_t stream) {
     const unsigned tokens = (unsigned)(a.batch * a.seq);
     if (a.out_q) {
         attn_decode_merge_kernel<NQ><<<dim3(tokens), dim3(256), 0, stream>>>(a);
-    } else if (a.nsplit > 1) {
+    } else {
         const MergeShape<kD> shape(a.nsplit, a.n_heads);
         attn_decode_merge_heads_kernel<NQ><<<dim3(tokens * (unsigned)(a.n_heads / shape.heads)), dim3(256), 0, stream>>>(a);
+    }
+}
+
+template <int NQ, bool WHOLE>
+void launch_partial(const AttnDecodeArgs& a, unsigned grid, hipStream_t stream) {
+    auto kern = !a.req_to_token ? attn_decode_partial_kernel<NQ, false, false, WHOLE>
+                : a.mask        ? attn_decode_partial_kernel<NQ, true, true, WHOLE>
+                                : attn_decode_partial_kernel<NQ, true, false, WHOLE>;
+    kern<<<dim3(grid), dim3(256), 0, stream>>>(a);
+}
+
+template <int NQ>
+void launch_rows(const AttnDecodeArgs& a, unsigned grid, hipStream_t stream) {
+    if (a.nsplit == 1 && !a.out_q) {
+        launch_partial<NQ, true>(a, grid, stream);
+    } else {
+        launch_partial<NQ, false>(a, grid, stream);
+        launch_merge<NQ>(a, stream);
     }
 }
 
@@ -398,23 +416,8 @@ bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream) {
     const bool paged = a.req_to_token != nullptr;
     if (paged && (a.seq != 1 || !a.req_pool_indices || !a.kv_indptr || a.rtt_stride <= 0)) return false;
     if (a.mask && (!paged || a.mask_width <= 0)) return false;
-    if (nq <= 4) {
-        if (paged && a.mask)
-            attn_decode_partial_kernel<4, true, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        else if (paged)
-            attn_decode_partial_kernel<4, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        else
-            attn_decode_partial_kernel<4, false><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        launch_merge<4>(a, stream);
-    } else {
-        if (paged && a.mask)
-            attn_decode_partial_kernel<8, true, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        else if (paged)
-            attn_decode_partial_kernel<8, true><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        else
-            attn_decode_partial_kernel<8, false><<<dim3(grid1), dim3(256), 0, stream>>>(a);
-        launch_merge<8>(a, stream);
-    }
+    if (nq <= 4) launch_rows<4>(a, grid1, stream);
+    else launch_rows<8>(a, grid1, stream);
     return true;
 }
 
