@@ -880,13 +880,16 @@ def decode_nsplit(pairs: int, max_keys: int) -> int:
 
 
 def paged_nsplit(pairs: int, max_keys: int) -> int:
-    """:func:`decode_nsplit` of a paged step, whose bf16 output a merge of any number of splits side by side writes: below
+    """:func:`decode_nsplit` of a paged step, whose bf16 output a merge of any number of splits side by side writes. Below
     64 pairs as many splits as make 512 workgroups, none that could not hold 64 keys of the slot table's width (one
-    sequence of 8192 keys, 16 / 4 heads: 8 splits 36 us, 64 13; four of 3000: 8 splits 20, 32 13; from 64 pairs on
-    more than eight splits gain nothing: eight sequences of 8192, 32 / 8 heads 40 us with 8, 38 with 16)."""
+    sequence of 8192 keys, 16 / 4 heads: 8 splits 36 us, 64 12; four of 3000: 8 splits 20, 32 12). From 64 pairs on
+    three workgroups for each CU, none that could not hold 160 keys (two for each CU, three: 32 x 3000 keys, 16 / 4 heads
+    33.2 us, 31.1, 32 / 4 heads 40.8, 36.2; 64 x 1500 41.2, 34.1; sequences of 100 keys behind a table of 16384 9.5,
+    10.7)."""
+    pairs = max(1, pairs)
     if pairs >= 64:
-        return decode_nsplit(pairs, max_keys)
-    return max(1, min(64, 512 // max(1, pairs), max_keys // 64))
+        return max(1, min(768 // pairs, max_keys // 160))
+    return max(1, min(64, 512 // pairs, max_keys // 64))
 
 
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
