@@ -1050,8 +1050,10 @@ def attn_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
             return out  # (an empty tensor has no address to hand over)
         m_ptr, m_stride, m_width = (mask.data_ptr(), mask.stride(0), mask.size(1)) if mask is not None else (0, 0, 0)
         if d != 128 or h > 64 or h // hkv > 8:  # the shapes only the general kernel takes
-            if not user_nsplit:  # one wave per (sequence, kv head, split): enough of them to fill the chip
-                nsplit = max(1, min(64, 2048 // max(1, b * hkv), rtt.size(1) // 64))
+            if not user_nsplit:
+                # one wave per (sequence, kv head, split): three to a SIMD (two, three, 32 / 8 heads x 64: 32 x 3000 keys
+                # 35.0 us, 31.2; 128 x 1000 43.5, 38.0; 16 / 16 heads x 64, 64 x 1500: 62, 54.7; fewer pairs the same)
+                nsplit = max(1, min(64, 3072 // max(1, b * hkv), rtt.size(1) // 64))
             _paged_rows(lib, q_c, k_cache, v_cache, rtt, rpi, ind, None, (m_ptr, m_stride, 0, 0, 1, m_width),
                         out, b, nsplit, False, scale, o_part_buf)
             return out
