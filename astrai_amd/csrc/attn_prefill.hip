@@ -510,9 +510,10 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     l_run += __shfl_xor(l_run, 32, kWave);
     // a row that sees no key at all (empty sequence, or more queries than keys) yields zeros
     // (with a mask tensor a row may have met nothing but masked scores: its reference maximum
-    // then still is the stand-in for -inf, times c once it has been through a rescale)
-    const bool met_a_key = !MASK || m_run > 0.5f * kNegBig * fminf(c, 1.0f);
-    const bool has_value = l_run > 0.0f && sees_a_key && met_a_key;
+    // then still is the stand-in for -inf, times c once it has been through a rescale, and its
+    // sum is no NaN). A NaN in l_run comes from a score the row sees, and goes out.
+    const bool met_a_key = !MASK || m_run > 0.5f * kNegBig * fminf(c, 1.0f) || l_run != l_run;
+    const bool has_value = l_run != 0.0f && sees_a_key && met_a_key;
     const float inv = has_value ? 1.0f / l_run : 0.0f;
     // (its accumulators hold whatever masked scores made of them: the difference of two roundings of
     // c * kNegBig may be large enough for an infinite probability)
