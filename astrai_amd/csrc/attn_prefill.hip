@@ -275,6 +275,9 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         }
         kmax = __builtin_amdgcn_readfirstlane(kmax);
     }
+    // (rows that lie before the first key count from below it: -1 for all of them, so that every wave of the
+    // workgroup walks the same blocks, one of masked keys)
+    kmax = max(kmax, -1);
     // what this wave's queries see: all of them up to pmin, none past kmax_w (equal to kmax with one
     // group of 32 tokens per workgroup)
     int pmin = row_live ? pq : 1 << 30, kmax_w = row_live ? pq : -1;
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         kmax_w = max(kmax_w, __shfl_xor(kmax_w, off, kWave));
     }
     pmin = __builtin_amdgcn_readfirstlane(pmin);
-    kmax_w = __builtin_amdgcn_readfirstlane(min(kmax_w, kmax));
+    kmax_w = max(__builtin_amdgcn_readfirstlane(min(kmax_w, kmax)), -1);
     const bool sees_a_key = pq >= 0;
     if (!row_live) pq = kmax_w;  // rows past the end see everything and are never stored
     const int nkb = kmax / kKB + 1;     // (kmax = -1, an empty sequence: one block of masked keys)
