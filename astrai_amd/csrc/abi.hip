@@ -611,7 +611,7 @@ int astrai_w8a8_attn_paged_prefill_masked_bf16(
     if (!w8a8::attn_prefill_supported((int)n_heads, (int)n_kv_heads, (int)head_dim))
         return fail(ASTRAI_W8A8_UNSUPPORTED,
                     "attn_paged_prefill_bf16: needs head_dim 128 and n_heads / n_kv_heads in {2, 4, 8}");
-    if (num_slots * n_kv_heads * 256 >= ((int64_t)1 << 32))
+    if (!w8a8::attn_prefill_pool_ok(num_slots, (int)n_kv_heads, (int)head_dim))
         return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_paged_prefill_bf16: a pool must stay under 4 GiB");
     if (!(scale > 0.0f)) return fail(ASTRAI_W8A8_BAD_ARG, "attn_paged_prefill_bf16: scale must be positive");
     if (!aligned16(q) || !aligned16(k_pool) || !aligned16(v_pool) || !aligned16(out))
@@ -685,7 +685,7 @@ int astrai_w8a8_attn_paged_rows_bf16(
         return fail(ASTRAI_W8A8_BAD_ARG, "attn_paged_rows_bf16: workspace too small (%lld floats needed)",
                     (long long)need);
     if (prefill && !mask && w8a8::attn_prefill_split_supported((int)n_heads, (int)n_kv_heads, (int)head_dim) &&
-        num_slots * n_kv_heads * head_dim * 2 < ((int64_t)1 << 32) &&
+        w8a8::attn_prefill_pool_ok(num_slots, (int)n_kv_heads, (int)head_dim) &&
         (nsplit == 1 || batch_or_tiles * n_heads >= kPrefillMinRowBlocks)) {
         w8a8::AttnPrefillArgs p{};
         p.q = q; p.k_cache = k_pool; p.v_cache = v_pool; p.out = out;

@@ -65,6 +65,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kKB = 64;            // keys per block
 constexpr float kNegBig = -1e30f;  // finite stand-in for -inf: no inf - inf
 
+// The offset of a row that is to read as zeros, and the most bytes a descriptor of this file spans: pools and heads
+// go up to 4 GiB, past the 2 GiB of kOutOfRange.
+constexpr uint32_t kMissing = 0xffffff00u;
+
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 // A raw buffer descriptor in scalar registers, as lds_dma16's assembly takes it (see make_rsrc).
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     };
     auto paged_off = [&](int slots, int src_lane, int swz) -> uint32_t {
         const int slot = __builtin_amdgcn_ds_bpermute(src_lane << 2, slots);
-        return slot >= 0 ? (uint32_t)slot * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz) << 4) : kOutOfRange;
+        return slot >= 0 ? (uint32_t)slot * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz) << 4) : kMissing;
     };
     [[maybe_unused]] uint32_t k_voff[DMA];
     if constexpr (!PAGED) {
@@ -590,18 +594,21 @@ bool attn_prefill_split_supported(int n_heads, int n_kv_heads, int head_dim) {
     return head_dim == 64 ? n_rep == 1 || n_rep == 2 || n_rep == 4 || n_rep == 8 : head_dim == 128 && n_rep == 1;
 }
 
+bool attn_prefill_pool_ok(int64_t num_slots, int n_kv_heads, int head_dim) {
+    return num_slots <= (int64_t)kMissing / (2 * (int64_t)n_kv_heads * head_dim);
+}
+
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream) {
     const bool split = attn_prefill_split_supported(a.n_heads, a.n_kv_heads, a.head_dim);
     if (!split && !attn_prefill_supported(a.n_heads, a.n_kv_heads, a.head_dim)) return false;
     const bool paged = a.req_to_token != nullptr;
     if (a.mask && (!paged || a.mask_width <= 0 || a.mask_rows <= 0)) return false;
     const int n_rep = a.n_heads / a.n_kv_heads;
-    const int64_t row = 2 * (int64_t)a.head_dim;
     if (paged) {
         if (!a.req_pool_indices || !a.kv_indptr || !a.qo_indptr || !a.q_tile_to_batch || !a.q_tile_to_index ||
             a.num_q_tiles <= 0 || a.rtt_stride <= 0 || a.num_slots <= 0 || a.num_requests <= 0)
             return false;
-        if (a.num_slots * a.n_kv_heads * row >= ((int64_t)1 << 32)) return false;  // 32-bit pool offsets
+        if (!attn_prefill_pool_ok(a.num_slots, a.n_kv_heads, a.head_dim)) return false;
     } else {
         if (a.batch <= 0 || a.seq <= 0 || a.max_len <= 0) return false;
         if (a.max_len * std::max(a.k_stride.row, a.v_stride.row) * 2 >= ((int64_t)1 << 32)) return false;  // 32-bit offsets

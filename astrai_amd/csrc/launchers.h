@@ -189,6 +189,8 @@ struct AttnPrefillArgs {
 bool attn_prefill_supported(int n_heads, int n_kv_heads, int head_dim);
 // the shapes it takes in place of attn_rows.hip (probabilities as two bf16 terms, no mask tensor)
 bool attn_prefill_split_supported(int n_heads, int n_kv_heads, int head_dim);
+// pools whose rows its 32-bit offsets reach (under 4 GiB)
+bool attn_prefill_pool_ok(int64_t num_slots, int n_kv_heads, int head_dim);
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream);
 
 // attn_rows.hip: paged attention for every head_dim in {32, 64, 128, 256} and every
