@@ -558,7 +558,7 @@ int astrai_w8a8_attn_prefill_strided_bf16(const void* q, const void* k, const vo
     for (int i = 0; i < 9; ++i)
         if (strides[i] < 0 || strides[i] % 8)
             return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: strides must be multiples of 8 elements");
-    if (kv_len * strides[5] >= ((int64_t)1 << 31) || kv_len * strides[8] >= ((int64_t)1 << 31))
+    if (kv_len * strides[5] > ((int64_t)1 << 31) - 128 || kv_len * strides[8] > ((int64_t)1 << 31) - 128)
         return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_prefill_strided_bf16: one head's rows must span less than 4 GiB");
     if (!(scale > 0.0f)) return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: scale must be positive");
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out))

@@ -298,14 +298,15 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     const int tiles_w = kmax_w / 32 + 1;  // tiles this wave computes
 
     // values: the same way into a 64-row buffer. Rows past kmax arrive as zeros, so a stale cache
-    // row can never meet a zero probability as 0 * NaN.
+    // row can never meet a zero probability as 0 * NaN. (With far strides those rows' offsets pass 32 bits: they
+    // must not come round to a place inside. Keys may: their scores are replaced.)
     const u32x4 rv = make_desc(vc, PAGED ? pool_bytes : kmax >= 0 ? (uint32_t)kmax * v_row + ROW : 0u);
     [[maybe_unused]] uint32_t v_voff[DMA];
     if constexpr (!PAGED) {
 #pragma unroll
         for (int j = 0; j < DMA; ++j) {
             const int row = (wave * DMA + j) * RPI + lane / LPR;
-            v_voff[j] = (uint32_t)row * v_row + (uint32_t)(((lane & (LPR - 1)) ^ swz_v(row)) << 4);
+            v_voff[j] = (uint32_t)min((uint64_t)row * v_row + (((lane & (LPR - 1)) ^ swz_v(row)) << 4), (uint64_t)kMissing);
         }
     }
     auto dma_v = [&](int kb, [[maybe_unused]] int slots) {
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         for (int j = 0; j < DMA; ++j) {
             const int inst = wave * DMA + j;
             const uint32_t off = PAGED ? paged_off(slots, RPW + j * RPI + lane / LPR, swz_v(inst * RPI + lane / LPR))
-                                       : v_voff[j] + (uint32_t)(kb * kKB) * v_row;
+                                       : min(__builtin_elementwise_add_sat(v_voff[j], (uint32_t)(kb * kKB) * v_row), kMissing);
             lds_dma16(rv, lds0 + RING + (kb & 1) * VBUF + inst * 1024, off);
         }
     };
@@ -611,7 +612,7 @@ bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream) {
         if (!attn_prefill_pool_ok(a.num_slots, a.n_kv_heads, a.head_dim)) return false;
     } else {
         if (a.batch <= 0 || a.seq <= 0 || a.max_len <= 0) return false;
-        if (a.max_len * std::max(a.k_stride.row, a.v_stride.row) * 2 >= ((int64_t)1 << 32)) return false;  // 32-bit offsets
+        if (a.max_len * std::max(a.k_stride.row, a.v_stride.row) * 2 > (int64_t)kMissing) return false;  // 32-bit offsets
     }
     if (a.head_dim == 64) {
         if (n_rep == 1) return launch_shape<64, 1, 4, true>(a, stream);

@@ -1691,7 +1691,7 @@ def attn_prefill_strided(q, k, v, layout: int, causal_offset: int = -1, position
     b, q_len, h, d = q.size(0), q.size(l_ax), q.size(h_ax), q.size(3)
     kv_len, hkv = k.size(l_ax), k.size(h_ax)
     (q, qs), (k, ks), (v, vs) = _strided_view(q, layout), _strided_view(k, layout), _strided_view(v, layout)
-    if kv_len * max(ks[2], vs[2]) >= 2 ** 31:
+    if kv_len * max(ks[2], vs[2]) > 2 ** 31 - 128:
         return None
     out = torch.empty((b, q_len, h, d), device=q.device, dtype=torch.bfloat16)
     _check(lib.astrai_w8a8_attn_prefill_strided_bf16(

@@ -404,7 +404,7 @@ int astrai_w8a8_attn_prefill_bf16(const void* q_bf16, const void* k_cache_bf16,
  * memory order (the tensors of csrc/kernels/attention/prefill.cu in either of its layouts, views
  * of a fused projection, a dense cache), without copying or re-addressing them.
  *   strides    host array of nine element strides, multiples of 8: batch, head and row of q, of k
- *              and of v; a row's head_dim values are consecutive. kv_len * row stride < 2^31.
+ *              and of v; a row's head_dim values are consecutive. kv_len * row stride <= 2^31 - 128.
  *   positions  NULL, or int64 [q_len] on the device: row i sees keys 0 .. positions[i] (at most kv_len)
  *   causal_offset  without positions: row i sees keys 0 .. i + causal_offset (< 0: all kv_len keys)
  *   out        bf16 [batch, q_len, n_heads, head_dim]

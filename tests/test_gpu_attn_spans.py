@@ -29,3 +29,18 @@ def test_missing_slots_of_a_large_pool(h, g, d, nbytes):
     # (the same kernel but for the largest pool, whose shapes with P in two terms differ by an ulp: 2^-7)
     err = (got.float() - want.float()).abs()
     assert torch.isfinite(got).all() and (err <= 2.0 ** -7 * want.float().abs() + 2 * 5 * 2.0 ** -16).all()
+
+
+def test_rows_past_the_newest_key_of_a_far_strided_tensor():
+    from astrai_amd.extension import _cabi
+    base = torch.full((1 << 31,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    q = torch.randn(1, 8, 40, 64, device=DEV).bfloat16()
+    # whole blocks of 64 keys are fetched: of the rows behind the last, the second lies past 2^32 bytes
+    for m in (65, 33, 2):
+        stride = ((1 << 31) - 128) // m // 8 * 8
+        k = torch.as_strided(base, (1, 2, m, 64), (8, 64, stride, 1))
+        k.copy_(torch.randn(1, 2, m, 64, device=DEV))
+        want = _cabi.attn_prefill_strided(q, k.contiguous(), k.contiguous(), _cabi.BHLD)
+        got = _cabi.attn_prefill_strided(q, k, k, _cabi.BHLD)
+        assert torch.isfinite(got).all() and torch.equal(got, want), m
+        k.fill_(float("nan"))
