@@ -1690,6 +1690,11 @@ def attn_prefill_strided(q, k, v, layout: int, causal_offset: int = -1, position
     l_ax, h_ax = (2, 1) if layout == BHLD else (1, 2)
     b, q_len, h, d = q.size(0), q.size(l_ax), q.size(h_ax), q.size(3)
     kv_len, hkv = k.size(l_ax), k.size(h_ax)
+    if not (q.is_cuda and q.dtype == k.dtype == v.dtype == torch.bfloat16 and k.device == v.device == q.device):
+        raise RuntimeError("attn_prefill_strided: q, k and v must be bf16 on one GPU")
+    if positions is not None and not (positions.dtype == torch.int64 and positions.shape == (q_len,)
+                                      and positions.is_contiguous() and positions.device == q.device):
+        raise RuntimeError("attn_prefill_strided: positions must be contiguous int64 [q_len] on q's device")
     (q, qs), (k, ks), (v, vs) = _strided_view(q, layout), _strided_view(k, layout), _strided_view(v, layout)
     if kv_len * max(ks[2], vs[2]) > 2 ** 31 - 128:
         return None
@@ -1717,13 +1722,13 @@ def cache_context_len(positions: torch.Tensor, max_len: int) -> torch.Tensor:
 def attn_cache_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                     positions: torch.Tensor) -> torch.Tensor:
     """Attention of new tokens ``q [batch, n_heads, seq, head_dim]`` at ``positions [seq]``
-    (int64, on the device) against the dense head-major caches ``[batch, n_kv_heads, max_len,
-    head_dim]`` through the general paged kernel, for the head shapes the tuned dense kernels
-    do not take (head_dim 32 / 64 / 256, any grouping up to 16). Every (sequence, KV head) pair
-    is addressed as one sequence of a one-head pool -- the cache rows of a KV head are
-    contiguous -- with the pair's query heads as its heads; nothing of the cache is copied
-    and no length is read on the host. A row attends keys at positions <= its own. Returns
-    token-major ``[batch, seq, n_heads * head_dim]``."""
+    (whole numbers on the device; one of them stands for all tokens) against the dense head-major caches
+    ``[batch, n_kv_heads, max_len, head_dim]``, bf16, for the head shapes the tuned dense kernels do not take
+    (any grouping up to 16). Several tokens of a shape that the block kernel has (:func:`attn_prefill_strided_takes`)
+    read the caches through strides. Else every (sequence, KV head) pair is addressed as one sequence of a one-head
+    pool of the general paged kernel -- the cache rows of a KV head are contiguous -- with the pair's query heads as
+    its heads. Nothing of the cache is copied and no length is read on the host. A row attends keys at positions <=
+    its own. Returns token-major ``[batch, seq, n_heads * head_dim]``."""
     _gpu(q, "attn_cache_rows")
     b, h, s, d = q.shape
     hkv, max_len = k_cache.size(1), k_cache.size(2)
@@ -1732,10 +1737,14 @@ def attn_cache_rows(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if k_cache.shape != (b, hkv, max_len, d) or v_cache.shape != k_cache.shape \
             or not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise RuntimeError("attn_cache_rows: the caches must be contiguous [batch, n_kv_heads, max_len, head_dim]")
+    if not (q.dtype == k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.device == v_cache.device == q.device):
+        raise RuntimeError("attn_cache_rows: q and the caches must be bf16 on one device")
+    if s > 1 and not (positions.device == q.device and positions.shape in ((s,), (1,))):
+        raise RuntimeError("attn_cache_rows: positions must be [seq] or [1] on q's device")
     n_rep, pairs = h // hkv, b * hkv
     with _on_device(q.device):
-        if s > 1 and attn_prefill_strided_takes(b, s, max_len, h, hkv, d):
-            out = attn_prefill_strided(q, k_cache, v_cache, BHLD, positions=positions.contiguous())
+        if s > 1 and b and positions.dtype in (torch.int64, torch.int32) and attn_prefill_strided_takes(b, s, max_len, h, hkv, d):
+            out = attn_prefill_strided(q, k_cache, v_cache, BHLD, positions=positions.to(torch.int64).expand(s).contiguous())
             if out is not None:
                 return out.view(b, s, h * d)
         table, rows = _identity_paging(pairs, max_len, q.device)

@@ -105,3 +105,43 @@ def test_head_dim_64_decoder_runs_the_general_kernel(monkeypatch):
     assert cos > 0.999, cos
     assert (got - want).abs().max().item() <= 0.05 * want.abs().max().item()
     assert torch.equal(eager, graph)
+
+
+SHARED = [(4, 2, 64), (4, 4, 128), (8, 2, 128), (4, 2, 32)]   # the block kernel's shapes, and one it does not have
+
+
+def _operands(h, hkv, d, s=20, max_len=48, b=2):
+    g = torch.Generator().manual_seed(d)
+    q = torch.randn(b, h, s, d, generator=g).bfloat16().to(DEV)
+    k, v = (torch.randn(b, hkv, max_len, d, generator=g).bfloat16().to(DEV) for _ in range(2))
+    return q, k, v, torch.arange(9, 9 + s, device=DEV)
+
+
+@pytest.mark.parametrize("h,hkv,d", SHARED)
+def test_attn_cache_rows_positions_it_takes(h, hkv, d):
+    from astrai_amd.extension import _cabi
+    q, k, v, pos = _operands(h, hkv, d)
+    want = _cabi.attn_cache_rows(q, k, v, pos)
+    assert torch.equal(_cabi.attn_cache_rows(q, k, v, pos.int()), want)
+    assert torch.equal(_cabi.attn_cache_rows(q, k, v, pos.repeat_interleave(2)[::2]), want)
+    every = _cabi.attn_cache_rows(q, k, v, torch.full_like(pos, 30))
+    assert torch.equal(_cabi.attn_cache_rows(q, k, v, torch.tensor([30], device=DEV)), every)
+    none = _cabi.attn_cache_rows(q[:0], k[:0], v[:0], pos)
+    assert none.shape == (0, 20, h * d)
+
+
+@pytest.mark.parametrize("h,hkv,d", SHARED)
+def test_attn_cache_rows_refuses_operands_it_cannot_read(h, hkv, d):
+    from astrai_amd.extension import _cabi
+    q, k, v, pos = _operands(h, hkv, d)
+    bad = [(q.half(), k.half(), v.half(), pos), (q, k.half(), v.half(), pos), (q, k, v.cpu(), pos), (q, k.cpu(), v.cpu(), pos),
+           (q, k, v, pos.cpu()), (q, k, v, pos[:19]), (q, k, v, torch.cat((pos, pos))), (q, k, v, pos[:, None])]
+    for args in bad:
+        with pytest.raises(RuntimeError):
+            _cabi.attn_cache_rows(*args)
+    if _cabi.attn_prefill_strided_takes(2, 20, 48, h, hkv, d):
+        for p in (pos.int(), pos[:1], pos.cpu(), pos.repeat_interleave(2)[::2]):
+            with pytest.raises(RuntimeError, match="positions"):
+                _cabi.attn_prefill_strided(q, k, v, _cabi.BHLD, positions=p)
+        with pytest.raises(RuntimeError, match="bf16"):
+            _cabi.attn_prefill_strided(q.half(), k.half(), v.half(), _cabi.BHLD, 0)
