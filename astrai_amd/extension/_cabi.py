@@ -1659,7 +1659,8 @@ def _strided_view(t, layout):
     """``(t, (batch, head, row) strides)`` of a 4-D tensor as the strided prompt kernel reads it: in
     place if rows are consecutive values at 16-byte boundaries, else a contiguous copy."""
     if t.stride(3) != 1 or t.stride(0) % 8 or t.stride(1) % 8 or t.stride(2) % 8 or t.data_ptr() % 16:
-        t = t.contiguous()
+        # (not contiguous(): a tensor may count as contiguous at an odd address, or with any stride of a size 1)
+        t = t.clone(memory_format=torch.contiguous_format)
     s = t.stride()
     return t, (s[0], s[1], s[2]) if layout == BHLD else (s[0], s[2], s[1])
 

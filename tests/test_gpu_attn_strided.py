@@ -118,3 +118,17 @@ def test_nan_in_a_later_value_stays_within_its_block():
         v[0, 160] = float("nan")
         out = _cabi.attn_prefill_strided(q, k, v, _cabi.BLHD, 0)
         assert torch.isfinite(out[0, :160]).all() and out[0, 160:].isnan().all(), (h, g, d)
+
+
+@pytest.mark.parametrize("h,g,d", SHAPES[:2] + SHAPES[4:6])
+def test_tensors_off_the_16_byte_grid_that_count_as_contiguous(h, g, d):
+    from astrai_amd.extension import _cabi
+    q, k, v = _tensors(1, 70, 70, h, g, d, seed=d)
+    want = _cabi.attn_prefill_strided(q, k, v, _cabi.BLHD, 0)
+    shifted = [torch.cat((t.new_zeros(1), t.flatten()))[1:].view_as(t) for t in (q, k, v)]
+    assert all(t.is_contiguous() and t.data_ptr() % 16 for t in shifted)
+    assert torch.equal(_cabi.attn_prefill_strided(*shifted, _cabi.BLHD, 0), want)
+    odd = [torch.as_strided(t, t.shape, (t.stride(0) + 1, *t.stride()[1:])) for t in (q, k, v)]   # of a batch of one
+    assert all(t.is_contiguous() for t in odd)
+    assert torch.equal(_cabi.attn_prefill_strided(*odd, _cabi.BLHD, 0), want)
+    assert torch.equal(_cabi.attn_prefill_qkv(*shifted, causal_offset=0, layout=_cabi.BLHD), want)
