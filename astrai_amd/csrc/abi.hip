@@ -549,7 +549,7 @@ int astrai_w8a8_attn_prefill_strided_bf16(const void* q, const void* k, const vo
     if (!q || !k || !v || !strides || !out)
         return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: null pointer");
     if (batch < 0 || q_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || kv_len <= 0 || n_heads % n_kv_heads ||
-        q_len > (1 << 24) || batch > (1 << 20) || kv_len > INT32_MAX || causal_offset > INT32_MAX / 2)
+        q_len > (1 << 30) || batch > (1 << 24) || kv_len > INT32_MAX || causal_offset > INT32_MAX / 2)
         return fail(ASTRAI_W8A8_BAD_ARG, "attn_prefill_strided_bf16: bad dims");
     if (!w8a8::attn_prefill_supported((int)n_heads, (int)n_kv_heads, (int)head_dim) &&
         !w8a8::attn_prefill_split_supported((int)n_heads, (int)n_kv_heads, (int)head_dim))

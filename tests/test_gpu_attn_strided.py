@@ -132,3 +132,13 @@ def test_tensors_off_the_16_byte_grid_that_count_as_contiguous(h, g, d):
     assert all(t.is_contiguous() for t in odd)
     assert torch.equal(_cabi.attn_prefill_strided(*odd, _cabi.BLHD, 0), want)
     assert torch.equal(_cabi.attn_prefill_qkv(*shifted, causal_offset=0, layout=_cabi.BLHD), want)
+
+
+def test_more_than_a_million_short_sequences():
+    from astrai_amd.extension import _cabi
+    b = (1 << 20) + 3
+    q, k, v = (torch.randn(b, 2, n, 64, device=DEV).bfloat16() for n in (2, 1, 1))
+    got = _cabi.attn_prefill_qkv(q, k, v, causal_offset=0, layout=_cabi.BLHD)
+    for at in (0, 1 << 19, b - 5):
+        part = slice(at, at + 5)
+        assert torch.equal(got[part], _cabi.attn_prefill_qkv(q[part], k[part], v[part], causal_offset=0, layout=_cabi.BLHD))
