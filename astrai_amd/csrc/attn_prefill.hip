@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     int pq, kmax;               // this lane's newest visible key; the block's newest
     [[maybe_unused]] const int* table = nullptr;
     [[maybe_unused]] int b_dense = 0, seq_index = 0;
-    [[maybe_unused]] int block_pos = -1;  // dense, with positions: that of the block's row `lane`
+    [[maybe_unused]] int64_t block_pos = -1;  // dense, with positions: that of the block's row `lane`
     if constexpr (PAGED) {
         constexpr int SUBS = 64 / QB;  // workgroups that share a tile
         const int idx = (int)(gridDim.x - 1 - blockIdx.x);
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         if (a.positions) {
             // The positions are requested first and looked at last: the query rows and the first
             // key tiles do not depend on them. (Blocks of up to 64 rows: launch_attn_prefill.)
-            block_pos = lane < QB && row0 + lane < a.seq ? (int)a.positions[row0 + lane] : -1;
+            block_pos = lane < QB && row0 + lane < a.seq ? a.positions[row0 + lane] : -1;
             pq = -1;
         } else {
             const int last = min(row0 + QB, rows_total) - 1;
@@ -270,10 +270,11 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
 
     if constexpr (!PAGED) {
         if (a.positions) {
-            block_pos = min(block_pos, (int)a.max_len - 1);  // (a token past the cache sees what it holds)
-            pq = __shfl(block_pos, qsub * 32 + qi, kWave);
+            // (a token past the cache sees what it holds; positions are whole 64-bit numbers)
+            const int newest = (int)max(min(block_pos, a.max_len - 1), (int64_t)-1);
+            pq = __shfl(newest, qsub * 32 + qi, kWave);
             // what the block's queries may see: every lane ends up with the same value
-            kmax = block_pos;
+            kmax = newest;
 #pragma unroll
             for (int off = 32; off; off >>= 1) kmax = max(kmax, __shfl_xor(kmax, off, kWave));
         }

@@ -110,7 +110,7 @@ def test_head_dim_64_decoder_runs_the_general_kernel(monkeypatch):
 SHARED = [(4, 2, 64), (4, 4, 128), (8, 2, 128), (4, 2, 32)]   # the block kernel's shapes, and one it does not have
 
 
-def _operands(h, hkv, d, s=20, max_len=48, b=2):
+def _operands(h, hkv, d, s=20, max_len=40, b=2):
     g = torch.Generator().manual_seed(d)
     q = torch.randn(b, h, s, d, generator=g).bfloat16().to(DEV)
     k, v = (torch.randn(b, hkv, max_len, d, generator=g).bfloat16().to(DEV) for _ in range(2))
@@ -139,9 +139,24 @@ def test_attn_cache_rows_refuses_operands_it_cannot_read(h, hkv, d):
     for args in bad:
         with pytest.raises(RuntimeError):
             _cabi.attn_cache_rows(*args)
-    if _cabi.attn_prefill_strided_takes(2, 20, 48, h, hkv, d):
+    if _cabi.attn_prefill_strided_takes(2, 20, 40, h, hkv, d):
         for p in (pos.int(), pos[:1], pos.cpu(), pos.repeat_interleave(2)[::2]):
             with pytest.raises(RuntimeError, match="positions"):
                 _cabi.attn_prefill_strided(q, k, v, _cabi.BHLD, positions=p)
         with pytest.raises(RuntimeError, match="bf16"):
             _cabi.attn_prefill_strided(q.half(), k.half(), v.half(), _cabi.BHLD, 0)
+
+
+@pytest.mark.parametrize("h,hkv,d", SHARED)
+def test_attn_cache_rows_positions_beyond_32_bits(h, hkv, d):
+    """A token far past the cache sees what it holds, one far before it nothing."""
+    from astrai_amd.extension import _cabi
+    q, k, v, pos = _operands(h, hkv, d)
+    far, near = pos.clone(), pos.clone()
+    far[-3:], near[-3:] = torch.tensor([2 ** 31 + 3, 2 ** 32 + 5, 2 ** 62]), 39
+    far[:2], near[:2] = torch.tensor([-2 ** 32, -2 ** 33 + 9]), -1
+    want = _cabi.attn_cache_rows(q, k, v, near)
+    assert want[:, :2].eq(0).all() and want[:, 2:].ne(0).any(-1).all()
+    assert torch.equal(_cabi.attn_cache_rows(q, k, v, far), want)
+    if _cabi.attn_prefill_supported(h, hkv, d):
+        assert torch.equal(_cabi.attn_prefill(q, k, v, far), _cabi.attn_prefill(q, k, v, near))
