@@ -52,7 +52,7 @@
 #include <climits>
 #include <type_traits>
 
-#include "common.cuh"
+#include "lds_dma.cuh"
 #include "launchers.h"
 
 namespace w8a8 {
@@ -70,27 +70,6 @@ constexpr float kNegBig = -1e30f;  // finite stand-in for -inf: no inf - inf
 constexpr uint32_t kMissing = 0xffffff00u;
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-
-// A raw buffer descriptor in scalar registers, as lds_dma16's assembly takes it (see make_rsrc).
-__device__ __forceinline__ u32x4 make_desc(const void* p, uint32_t bytes) {
-    const uint64_t addr = (uint64_t)p;
-    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(addr >> 32) & 0xffffu)),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
-// 16 bytes per lane from the buffer into LDS at lds_addr + 16 * lane (lds_addr the same for the whole
-// wave). Out-of-range lanes write zeros. The caller waits (vmcnt) before the bytes are read.
-// (m0 is a reserved register that nothing else in this file's kernels uses.)
-__device__ __forceinline__ void lds_dma16(u32x4 desc, uint32_t lds_addr, uint32_t voff) {
-    __asm__ volatile(
-        "s_mov_b32 m0, %0\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, 0 offen lds"
-        :
-        : "s"(lds_addr), "v"(voff), "s"(desc)
-        : "memory");
-}
 
 // PAGED: the queries are packed [total_q, heads, D] with per-request row ranges
 // (qo_indptr), the caches are token-granular pools [slots, kv_heads, D] reached through
@@ -256,7 +235,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             const uint32_t off = PAGED ? paged_off(slots, j * RPI + lane / LPR, swz_k(inst * RPI + lane / LPR))
                                        : k_voff[j] + (uint32_t)(t0 * 32) * k_row;
             const int tile_inst = 32 / RPI;
-            lds_dma16(rk, lds0 + ((t0 + inst / tile_inst) & 3) * TILE + (inst % tile_inst) * 1024, off);
+            lds_dma16<false>(rk, lds0 + ((t0 + inst / tile_inst) & 3) * TILE + (inst % tile_inst) * 1024, off);
         }
     };
     [[maybe_unused]] int slots = 0;
@@ -316,7 +295,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             const int inst = wave * DMA + j;
             const uint32_t off = PAGED ? paged_off(slots, RPW + j * RPI + lane / LPR, swz_v(inst * RPI + lane / LPR))
                                        : min(__builtin_elementwise_add_sat(v_voff[j], (uint32_t)(kb * kKB) * v_row), kMissing);
-            lds_dma16(rv, lds0 + RING + (kb & 1) * VBUF + inst * 1024, off);
+            lds_dma16<false>(rv, lds0 + RING + (kb & 1) * VBUF + inst * 1024, off);
         }
     };
 

@@ -31,6 +31,7 @@
 // exponentials of tile T, the value MFMAs of tile T among the masking of tile T + 1. One copy of the
 // step masks every tile: a second copy without masking costs more in registers and code than the
 // compares (157 us against 107 us for 32 x 512 tokens, 16 heads of 128 + 64).
+#include "lds_dma.cuh"
 #include "mix_common.cuh"
 #include "mix_launchers.h"
 
@@ -42,27 +43,6 @@ namespace {
 
 constexpr int kQB = 128;   // query tokens per workgroup
 constexpr int kKB = 64;    // keys per block (two tiles)
-
-// A raw buffer descriptor in scalar registers (see w8a8::make_rsrc), as lds_dma16's assembly takes it.
-__device__ __forceinline__ u32x4 make_desc(const void* p, uint32_t bytes) {
-    const uint64_t addr = (uint64_t)p;
-    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(addr >> 32) & 0xffffu)),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-
-// 16 bytes per lane from the buffer into LDS at lds_addr + 16 * lane (lds_addr the same for the whole wave).
-// Out-of-range lanes write zeros. The caller waits (vmcnt) before the bytes are read. (m0 is a reserved
-// register that nothing else in this file's kernels uses.)
-__device__ __forceinline__ void lds_dma16(u32x4 desc, uint32_t lds_addr, uint32_t voff) {
-    __asm__ volatile(
-        "s_mov_b32 m0, %0\n\t"
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, 0 offen lds"
-        :
-        : "s"(lds_addr), "v"(voff), "s"(desc)
-        : "memory");
-}
 
 // which of a row's C chunks sits at position 0: 16 consecutive rows cover all banks
 template <int C>
@@ -152,7 +132,7 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
     }
     auto rows_rsrc = [](const uint8_t* p, int rows, int64_t ld, int bytes) {
         const int64_t n = rows > 0 ? (int64_t)(rows - 1) * ld + bytes : 0;
-        return make_desc(p, (uint32_t)n);
+        return w8a8::make_desc(p, (uint32_t)n);
     };
     // tiles t0 and t0 + 1 into their ring slots
     auto dma_k = [&](int t0) {
@@ -161,14 +141,14 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
 #pragma unroll
         for (int j = 0; j < JN; ++j) {
             const int inst = wave * JN + j;
-            lds_dma16(rn, lds0 + ((t0 + inst / IN) & 3) * kTile + (inst % IN) * 1024, on[j]);
+            w8a8::lds_dma16<true>(rn, lds0 + ((t0 + inst / IN) & 3) * kTile + (inst % IN) * 1024, on[j]);
         }
         if constexpr (DR > 0) {
             const u32x4 rr = rows_rsrc(kr + (int64_t)key * ldc, rows, ldc, d.dr * 2);
 #pragma unroll
             for (int j = 0; j < JR; ++j) {
                 const int inst = wave * JR + j;
-                lds_dma16(rr, lds0 + ((t0 + inst / IR) & 3) * kTile + 32 * kNRow + (inst % IR) * 1024, orr[j]);
+                w8a8::lds_dma16<true>(rr, lds0 + ((t0 + inst / IR) & 3) * kTile + 32 * kNRow + (inst % IR) * 1024, orr[j]);
             }
         }
     };
@@ -176,7 +156,7 @@ __global__ __launch_bounds__(256, 2) void mix_prefill_kernel(LatentPrefillArgs a
         const int key = kmin + kb * kKB, rows = min(kmax - key + 1, kKB);
         const u32x4 rv = rows_rsrc(kv + (int64_t)key * ldkv + d.dn * 2, rows, ldkv, d.vp * 2);
 #pragma unroll
-        for (int j = 0; j < JV; ++j) lds_dma16(rv, lds0 + kRing + (kb & 1) * kVBuf + (wave * JV + j) * 1024, ov[j]);
+        for (int j = 0; j < JV; ++j) w8a8::lds_dma16<true>(rv, lds0 + kRing + (kb & 1) * kVBuf + (wave * JV + j) * 1024, ov[j]);
     };
 
     f32x16 o[NV];
