@@ -100,7 +100,8 @@ def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Opti
     if weight.size(0) > 16384 and x.numel() > 32 * x.size(-1):
         return False
     return (_mix.few_rows_linear_supported(x, weight, bias, act) and not torch.is_autocast_enabled("cuda")
-            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)) and not _linear_policy_on())
+            and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, weight, bias)))
+            and not _linear_policy_on())
 
 
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
