@@ -108,6 +108,22 @@ def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
     return _mix.few_rows_linear(x, weight, bias) if few_rows(x, weight, bias) else F.linear(x, weight, bias)
 
 
+class HeadLinear(Linear):
+    """The output head: a plain ``Linear``, of few rows as :func:`linear` runs them."""
+
+    def forward(self, x: Tensor) -> Tensor:
+        return linear(x, self.weight, self.bias)
+
+
+def observed(module: nn.Module) -> bool:
+    """A call of ``module`` runs more than its class's ``forward``: hooks, its own or those of every module, or a
+    ``forward`` set on the instance."""
+    every = nn.modules.module
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
+                or every._global_backward_pre_hooks or "forward" in vars(module))
+
+
 def heads_of(name: str, heads: int, *dims: int) -> Rows:
     return Rows(name, heads, tuple((d, pad_to(d)) for d in dims))
 
@@ -581,9 +597,9 @@ class GatedMLP(nn.Module):
                 lin.assign(name, t)
 
     def forward(self, h: Tensor) -> Tensor:
-        w = self.gate_up.weight
-        if few_rows(h, w, act=self.act):
-            return self.down(_mix.few_rows_linear(h, w, act=self.act))
+        up = self.gate_up
+        if type(up) is PackedLinear and up.bias is None and not observed(up) and few_rows(h, up.weight, act=self.act):
+            return self.down(_mix.few_rows_linear(h, up.weight, act=self.act))
         return self.down(_mix.act_mul(self.gate_up(h), self.act))
 
 
@@ -597,7 +613,7 @@ class MixerLM(nn.Module):
         self.embed = Embedding(config.vocab, config.width)
         self.layers = nn.ModuleList(layers)
         self.final_norm = Fp32Vector(config.width)
-        self.head = Linear(config.width, config.vocab)
+        self.head = HeadLinear(config.width, config.vocab)
         self._ready = False
 
     def reset(self) -> None:
@@ -671,4 +687,4 @@ class MixerLM(nn.Module):
         hidden = h.reshape(ctx.batch, ctx.seq, -1)
         if logits_at is not None:
             hidden = hidden.index_select(1, logits_at)
-        return {"logits": linear(hidden, self.head.weight, self.head.bias), "hidden_states": hidden, "residual": x.reshape(ctx.batch, ctx.seq, -1)}
+        return {"logits": self.head(hidden), "hidden_states": hidden, "residual": x.reshape(ctx.batch, ctx.seq, -1)}

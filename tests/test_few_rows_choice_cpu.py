@@ -27,3 +27,61 @@ def test_gradients_of_every_operand(which):
     out = mixers.linear(*ops)
     out.sum().backward()
     assert ops[which].grad is not None
+
+
+def _ways(mlp):
+    """Which way ``mlp`` goes: the kernel with the activation in its epilogue, or the two modules."""
+    x = torch.randn(4, 16)
+    calls = []
+    with pytest.MonkeyPatch.context() as m, torch.no_grad():
+        m.setattr(_mix, "few_rows_linear", lambda h, w, b=None, act=None: (calls.append(act), torch.zeros(4, w.size(0) // (1 if act is None else 2)))[1])
+        m.setattr(_mix, "act_mul", lambda gu, act: (calls.append("act_mul"), gu[:, :gu.size(1) // 2])[1])
+        mlp(x)
+    return calls
+
+
+def test_the_gate_product_is_a_module_call_where_something_watches():
+    mlp = mixers.GatedMLP(16, 24)
+    assert _ways(mlp) == ["silu", None]
+    seen = []
+    for register in ("register_forward_hook", "register_forward_pre_hook"):
+        hook = getattr(mlp.gate_up, register)(lambda *a: seen.append(1))
+        assert _ways(mlp) == [None, "act_mul", None] and seen.pop()
+        hook.remove()
+    hook = torch.nn.modules.module.register_module_forward_hook(lambda *a: seen.append(1))
+    try:
+        assert "act_mul" in _ways(mlp) and len(seen) >= 2
+    finally:
+        hook.remove()
+    forward, mlp.gate_up.forward = mlp.gate_up.forward, lambda x: torch.ones(4, 48)
+    assert _ways(mlp) == ["act_mul", None]
+    del mlp.gate_up.forward
+    assert _ways(mlp) == ["silu", None]
+    torch.nn.utils.parametrize.register_parametrization(mlp.gate_up, "weight", torch.nn.Identity())
+    assert _ways(mlp) == [None, "act_mul", None]
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner, self.weight = inner, inner.weight
+
+        def forward(self, x):
+            return self.inner(x) + 1
+
+    mlp = mixers.GatedMLP(16, 24)
+    mlp.gate_up = Wrapped(mlp.gate_up)
+    assert _ways(mlp) == [None, "act_mul", None]
+
+
+def test_the_head_is_a_module_call():
+    from types import SimpleNamespace
+    model = mixers.MixerLM(SimpleNamespace(vocab=8, width=16), [])
+    ctx, h, seen = SimpleNamespace(batch=2, seq=3), torch.randn(6, 16), []
+    hook = model.head.register_forward_hook(lambda module, args, out: seen.append(args[0].shape))
+    with pytest.MonkeyPatch.context() as m, torch.no_grad():
+        m.setattr(_mix, "few_rows_linear", lambda x, w, b=None, act=None: x @ w.t())
+        out = model.finish(h, h, ctx, torch.tensor([2]))
+        assert out["logits"].shape == (2, 1, 8) and seen == [(2, 1, 16)]
+        hook.remove()
+        model.head = torch.nn.Sequential(torch.nn.Linear(16, 4), torch.nn.Linear(4, 5))
+        assert model.finish(h, h, ctx, None)["logits"].shape == (2, 3, 5)
