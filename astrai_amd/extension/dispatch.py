@@ -66,6 +66,12 @@ def install() -> None:
         _lib.impl("linear_backward", _linear_backward_cuda_impl)
 
 
+def linear_is_stock() -> bool:
+    """No handler takes ``F.linear`` calls at present. A handler with an ``enabled()`` of its own (both policies here)
+    takes none while that is false; any other may."""
+    return all(hasattr(h, "enabled") and not h.enabled() for h in _handlers)
+
+
 def register_handler(h: Handler, backward: Optional[Callable] = None) -> None:
     if h not in _handlers:
         _handlers.append(h)

@@ -480,5 +480,6 @@ def _fp8_backward_handler(input_tensor, grad_output, weight, output_mask):
     return None
 
 
+_fp8_handler.enabled = fp8_linear_enabled
 # importing this module installs the aten::linear override (fp8.py:404-406)
 dispatch.register_handler(_fp8_handler, _fp8_backward_handler)

@@ -137,4 +137,5 @@ def _int8_handler(x, w, bias):
     return None
 
 
+_int8_handler.enabled = int8_linear_enabled
 dispatch.register_handler(_int8_handler)

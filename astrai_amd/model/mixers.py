@@ -20,7 +20,6 @@ Padded rows and columns of weights are zero, so padded activations are zero ever
 from __future__ import annotations
 
 import math
-import sys
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -29,7 +28,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
-from astrai_amd.extension import _mix
+from astrai_amd.extension import _mix, dispatch
 from astrai_amd.extension._mix import RING_STEPS, DeltaShape, GqaShape, LatentShape, pad_to
 from astrai_amd.model.cache import MixerCache
 from astrai_amd.model.decoder import Embedding, Linear, rotary_table, yarn_frequencies
@@ -82,18 +81,9 @@ class Rows:
         return out.reshape(self.padded, *t.shape[2:])
 
 
-def _linear_policy_on() -> bool:
-    """A quantizing policy takes ``F.linear`` calls at present (a module that is not loaded has none)."""
-    for module, enabled in (("w8a8", "int8_linear_enabled"), ("fp8", "fp8_linear_enabled")):
-        m = sys.modules.get("astrai_amd.extension." + module)
-        if m is not None and getattr(m, enabled)():
-            return True
-    return False
-
-
 def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
     """Whether this product runs on the kernel for a decode step's few rows: everything ``F.linear`` may have
-    to do besides (gradients, autocasting, a quantizing policy) is left to it, and so are more than 32 rows with
+    to do besides (gradients, autocasting, a policy's handler) is left to it, and so are more than 32 rows with
     more than 16384 outputs, where reading x out of L2 in every workgroup is the larger stream (32000 x 2048 at
     64 rows: 34.2 us against the vendor library's 33.2; at 32 rows 26.8 against 33.2; 11264 x 2048 at 64 rows
     12.9 against 17.2)."""
@@ -101,7 +91,7 @@ def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Opti
         return False
     return (_mix.few_rows_linear_supported(x, weight, bias, act) and not torch.is_autocast_enabled("cuda")
             and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, weight, bias)))
-            and not _linear_policy_on())
+            and dispatch.linear_is_stock())
 
 
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:

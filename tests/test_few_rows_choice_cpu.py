@@ -85,3 +85,17 @@ def test_the_head_is_a_module_call():
         hook.remove()
         model.head = torch.nn.Sequential(torch.nn.Linear(16, 4), torch.nn.Linear(4, 5))
         assert model.finish(h, h, ctx, None)["logits"].shape == (2, 3, 5)
+
+
+def test_other_handlers_of_linear_get_the_call(monkeypatch):
+    from astrai_amd.extension import dispatch, fp8, w8a8
+    x, w, b = _operands()
+    with torch.no_grad():
+        assert mixers.few_rows(x, w, b)
+        with w8a8.int8_autocast(True):
+            assert not mixers.few_rows(x, w, b)
+        with fp8.fp8_autocast(True):
+            assert not mixers.few_rows(x, w, b)
+        assert mixers.few_rows(x, w, b)
+        monkeypatch.setattr(dispatch, "_handlers", [*dispatch._handlers, lambda x, w, b: None])
+        assert not mixers.few_rows(x, w, b)
