@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from astrai_amd.extension import _mix, dispatch
 from astrai_amd.extension._mix import RING_STEPS, DeltaShape, GqaShape, LatentShape, pad_to
@@ -81,17 +82,27 @@ class Rows:
         return out.reshape(self.padded, *t.shape[2:])
 
 
+def plain(*tensors: Optional[Tensor]) -> bool:
+    """Eager tensors and nothing between them and a kernel that reads their memory: no subclass or ``torch.func``
+    wrapper, no tangents, no dispatch or function mode, no trace."""
+    return (all(t is None or (type(t) in (Tensor, nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+                for t in tensors)
+            and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0 and torch._C._get_tracing_state() is None)
+
+
 def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
     """Whether this product runs on the kernel for a decode step's few rows: everything ``F.linear`` may have
-    to do besides (gradients, autocasting, a policy's handler) is left to it, and so are more than 32 rows with
+    to do besides (gradients, autocasting, a policy's handler, transforms) is left to it, and so are more than 32 rows with
     more than 16384 outputs, where reading x out of L2 in every workgroup is the larger stream (32000 x 2048 at
     64 rows: 34.2 us against the vendor library's 33.2; at 32 rows 26.8 against 33.2; 11264 x 2048 at 64 rows
     12.9 against 17.2)."""
-    if weight.size(0) > 16384 and x.numel() > 32 * x.size(-1):
+    rows = x.numel() // x.size(-1) if x.size(-1) else 0
+    if torch.compiler.is_compiling() or rows > (_mix.FEW_ROWS if weight.size(0) <= 16384 else 32):
         return False
-    return (_mix.few_rows_linear_supported(x, weight, bias, act) and not torch.is_autocast_enabled("cuda")
-            and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, weight, bias)))
-            and dispatch.linear_is_stock())
+    return (plain(x, weight, bias) and _mix.few_rows_linear_supported(x, weight, bias, act) and dispatch.linear_is_stock()
+            and not torch.is_autocast_enabled("cuda")
+            and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, weight, bias))))
 
 
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:

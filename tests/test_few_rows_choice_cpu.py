@@ -9,7 +9,8 @@ from astrai_amd.model import mixers
 
 @pytest.fixture(autouse=True)
 def any_shape(monkeypatch):
-    monkeypatch.setattr(_mix, "few_rows_linear_supported", lambda *a, **k: True)
+    # (it looks at addresses, which wrapped and fake tensors do not have)
+    monkeypatch.setattr(_mix, "few_rows_linear_supported", lambda x, w, *a, **k: bool(x.data_ptr() and w.data_ptr()))
 
 
 def _operands():
@@ -99,3 +100,49 @@ def test_other_handlers_of_linear_get_the_call(monkeypatch):
         assert mixers.few_rows(x, w, b)
         monkeypatch.setattr(dispatch, "_handlers", [*dispatch._handlers, lambda x, w, b: None])
         assert not mixers.few_rows(x, w, b)
+
+
+def test_transforms_tangents_modes_and_traces():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w, b = _operands()
+    want = torch.nn.functional.linear(x, w, b)
+
+    def taken(*a, **k):
+        raise AssertionError("the kernel was called")
+
+    with pytest.MonkeyPatch.context() as m, torch.no_grad():
+        m.setattr(_mix, "few_rows_linear", taken)
+        with pytest.raises(AssertionError):
+            mixers.linear(x, w, b)
+        assert torch.allclose(torch.func.vmap(lambda r: mixers.linear(r[None], w, b)[0])(x), want, atol=1e-5)
+        assert torch.allclose(torch.func.vmap(lambda r: mixers.linear(x, r[None])[:, 0])(w).t(), want - b, atol=1e-5)
+        assert torch.func.jvp(lambda t: mixers.linear(t, w, b), (x,), (x,))[1].shape == want.shape
+        assert torch.func.grad(lambda t: mixers.linear(t, w, b).sum())(x).shape == x.shape
+        with forward_ad.dual_level():
+            assert forward_ad.unpack_dual(mixers.linear(forward_ad.make_dual(x, x), w, b)).tangent is not None
+        with FlopCounterMode(display=False) as flops:
+            mixers.linear(x, w, b)
+        assert flops.get_total_flops() == 2 * 4 * 16 * 8
+        with FakeTensorMode() as fake:
+            mixers.linear(*(fake.from_tensor(t) for t in (x, w, b)))
+
+        class Counting(TorchFunctionMode):
+            calls = 0
+
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                self.calls += func is torch.nn.functional.linear
+                return func(*args, **(kwargs or {}))
+
+        with Counting() as mode:
+            mixers.linear(x, w, b)
+        assert mode.calls == 1
+
+        class Sub(torch.Tensor):
+            pass
+
+        assert type(mixers.linear(x.as_subclass(Sub), w, b)) is Sub
+        assert torch.allclose(torch.jit.trace(lambda t: mixers.linear(t, w, b), (x,), check_trace=False)(2 * x), 2 * want - b, atol=1e-5)
+        assert torch.allclose(torch.compile(lambda t: mixers.linear(t, w, b), backend="eager")(x), want)
