@@ -337,11 +337,12 @@ def _dynamic_scale(t: torch.Tensor, recipe: FP8Recipe, fmt: str) -> torch.Tensor
     return recipe.scale_from_history(amax, fmt)
 
 
-def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None):
+def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_product: bool = False):
     """Scaled fp8 linear forward (fp8.py:275-305).
 
     Dynamic scaling: measure both operands, quantize, pre-quantized GEMM to bf16,
-    then add the bias in bf16 (two roundings, as the reference does). Delayed
+    then add the bias in bf16 (two roundings, as the reference does); ``bias_in_product``, for callers
+    below autograd: in the GEMM's epilogue, same bits. Delayed
     scaling: quantize with the rings' current steps inside the fused forward,
     then push the returned amax values."""
     st = fp8_state()
@@ -359,7 +360,7 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None):
             sw = _dynamic_scale(w, st.recipe, fmt)
             w8, _ = quantize_bf16(w, sw, fmt)
         shape = (*x.shape[:-1], w.size(0))
-        if bias is not None and bias.is_cuda and bias.dtype == torch.bfloat16 and bias.shape == (w.size(0),) \
+        if bias_in_product and bias is not None and bias.is_cuda and bias.dtype == torch.bfloat16 and bias.shape == (w.size(0),) \
                 and bias.device == x.device and bias.numel() and x2.size(1):
             return mm_fp8_rounded_bias(x8, w8, sx, sw, bias).reshape(shape)
         out = mm_fp8(x8, w8, sx, sw).reshape(shape)
@@ -466,7 +467,7 @@ def _fp8_handler(x, w, bias):
         and w.dtype == torch.bfloat16
         and _fp8_supported(x, w)
     ):
-        return fp8_linear_forward(x, w, bias)
+        return fp8_linear_forward(x, w, bias, True)
     return None
 
 

@@ -49,3 +49,17 @@ def test_dynamic_forward_with_a_bias():
         wide = fp8.fp8_linear_forward(x, w, b)
         assert wide.dtype == torch.float32 and torch.equal(wide, plain + b)
     fp8.fp8_state().reset()
+
+
+def test_a_direct_forward_keeps_the_bias_gradient():
+    """The function itself stands above autograd: under dynamic scaling the bias is added to the finished product."""
+    from astrai_amd.extension import fp8
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x, w, b = (torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16) for s in ((33, 256), (40, 256), (40,)))
+    with fp8.fp8_autocast(True, recipe=fp8.DynamicScaling()):
+        out = fp8.fp8_linear_forward(x, w, b.requires_grad_(True))
+        out.backward(torch.ones_like(out))
+        assert torch.equal(b.grad, torch.full_like(b, 33))
+        with torch.no_grad():
+            assert torch.equal(torch.nn.functional.linear(x, w, b), out)
+    fp8.fp8_state().reset()
