@@ -91,14 +91,30 @@ def plain(*tensors: Optional[Tensor]) -> bool:
             and torch._C._len_torch_function_stack() == 0 and torch._C._get_tracing_state() is None)
 
 
+def few_rows_most(n: int, k: int, act: bool) -> int:
+    """Most rows of ``x`` with which a product of ``n`` weight rows of ``k`` values (``act``: of gate and up together) is
+    faster on :func:`_mix.few_rows_linear` than on the vendor library (us, ours / the library's). Up to 32 rows nearly all
+    are (2048 x 2048 6 / 11, 28672 x 4096 45 / 55). Of 33 and more each workgroup holds x twice as wide, and it pays
+    where one round of 256 workgroups holds the weight (12288 rows: 64 rows of 4096 values 22.5 / 25.1; 13312: 30.0 /
+    26.0; up to 2048 values also the start of a second, 16384 17.9 / 18.3) and the weight is the larger stream against
+    one x to a workgroup (64 rows of 5632: 2048 15.0 / 18.1, 1024 13.9 / 10.7). With an activation the library's side is
+    two launches (64 rows, 16384 x 5632 38 / 42). Rows a power of two of 16 KiB or more apart share memory channels: 32 rows
+    of 8192 values 4096 18.5 / 18.7, 8192 33.2 / 31.7, with an activation 12288 43 / 46, 16384 64 / 59."""
+    if k >= 8192 and k & (k - 1) == 0 and n * k > (12288 << 13 if act else 1 << 25):
+        return 0
+    if act:
+        wide = n <= 16384
+    else:
+        wide = n <= (16384 if k <= 2048 else 12288) and (k <= 4096 or n >= 2048)
+    return _mix.FEW_ROWS if wide else 32
+
+
 def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
     """Whether this product runs on the kernel for a decode step's few rows: everything ``F.linear`` may have
-    to do besides (gradients, autocasting, a policy's handler, transforms) is left to it, and so are more than 32 rows with
-    more than 16384 outputs, where reading x out of L2 in every workgroup is the larger stream (32000 x 2048 at
-    64 rows: 34.2 us against the vendor library's 33.2; at 32 rows 26.8 against 33.2; 11264 x 2048 at 64 rows
-    12.9 against 17.2)."""
-    rows = x.numel() // x.size(-1) if x.size(-1) else 0
-    if torch.compiler.is_compiling() or rows > (_mix.FEW_ROWS if weight.size(0) <= 16384 else 32):
+    to do besides (gradients, autocasting, a policy's handler, transforms) is left to it, and so are the sizes at which
+    the library is the faster one."""
+    k = x.size(-1)
+    if torch.compiler.is_compiling() or not k or x.numel() // k > few_rows_most(weight.size(0), k, act is not None):
         return False
     return (plain(x, weight, bias) and _mix.few_rows_linear_supported(x, weight, bias, act) and dispatch.linear_is_stock()
             and not torch.is_autocast_enabled("cuda")

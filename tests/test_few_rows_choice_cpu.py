@@ -146,3 +146,14 @@ def test_transforms_tangents_modes_and_traces():
         assert type(mixers.linear(x.as_subclass(Sub), w, b)) is Sub
         assert torch.allclose(torch.jit.trace(lambda t: mixers.linear(t, w, b), (x,), check_trace=False)(2 * x), 2 * want - b, atol=1e-5)
         assert torch.allclose(torch.compile(lambda t: mixers.linear(t, w, b), backend="eager")(x), want)
+
+
+@pytest.mark.parametrize("n,k,act,most", [
+    (2048, 2048, None, 64), (16384, 2048, None, 64), (16388, 2048, None, 32), (12288, 4096, None, 64), (13312, 4096, None, 32),
+    (1024, 4096, None, 64), (1024, 5632, None, 32), (2048, 5632, None, 64), (32000, 2048, None, 32), (4096, 8192, None, 64),
+    (8192, 8192, None, 0), (16384, 4096, "silu", 64), (16392, 4096, "silu", 32), (12288, 8192, "silu", 64), (16384, 8192, "silu", 0)])
+def test_sizes_at_which_the_kernel_is_the_faster_one(n, k, act, most):
+    w = torch.zeros(1).expand(n, k)
+    with torch.no_grad():
+        for rows in (1, 32, 33, 64, 65):
+            assert mixers.few_rows(torch.zeros(1).expand(rows, k), w, act=act) == (rows <= most)
