@@ -122,7 +122,10 @@ def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Opti
 
 
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
-    return _mix.few_rows_linear(x, weight, bias) if few_rows(x, weight, bias) else F.linear(x, weight, bias)
+    # (the rows first: a prompt's eager products are to pay nothing for the question)
+    if x.numel() > _mix.FEW_ROWS * x.size(-1) or not few_rows(x, weight, bias):
+        return F.linear(x, weight, bias)
+    return _mix.few_rows_linear(x, weight, bias)
 
 
 class HeadLinear(Linear):
@@ -226,7 +229,7 @@ def linear_f32(x: Tensor, weight: Tensor) -> Tensor:
     """``x W^T`` in fp32: bf16 operands keep their fp32 accumulators' digits."""
     if x.dtype == torch.float32:
         return F.linear(x, weight)
-    if few_rows(x, weight):
+    if x.numel() <= _mix.FEW_ROWS * x.size(-1) and few_rows(x, weight):
         return _mix.few_rows_linear(x, weight, out_dtype=torch.float32)
     return torch.mm(x, weight.t(), out_dtype=torch.float32)
 
@@ -615,7 +618,8 @@ class GatedMLP(nn.Module):
 
     def forward(self, h: Tensor) -> Tensor:
         up = self.gate_up
-        if type(up) is PackedLinear and up.bias is None and not observed(up) and few_rows(h, up.weight, act=self.act):
+        if (h.numel() <= _mix.FEW_ROWS * h.size(-1) and type(up) is PackedLinear and up.bias is None and not observed(up)
+                and few_rows(h, up.weight, act=self.act)):
             return self.down(_mix.few_rows_linear(h, up.weight, act=self.act))
         return self.down(_mix.act_mul(self.gate_up(h), self.act))
 
