@@ -31,7 +31,9 @@ struct Small64Cfg {
     static_assert(S >= 3 && 4 * (S - 2) < 64, "ring depth");
 };
 
-template <class Op, int ScaleKind, int S>
+// RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it (see gemm_mid128.cuh; 200 x 2048
+// x 2048 6.2 us, with the choice in the epilogue 6.3)
+template <class Op, int ScaleKind, int S, bool RoundFirst>
 __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
     using Cfg = Small64Cfg<S>;
     using Acc = typename Op::Acc;
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
             if constexpr (ScaleKind == SCALE_BLOCK128) {
                 v[j] = f + ((bias && n + j < g.n) ? bf16_to_f32(bias[n + j]) : 0.0f);
             } else if constexpr (ScaleKind == SCALE_TENSOR) {
-                v[j] = g.round_first ? add_bias(f * s_tensor, b4[q][j], true) : f * s_tensor + b4[q][j];
+                v[j] = RoundFirst ? add_bias(f * s_tensor, b4[q][j], true) : f * s_tensor + b4[q][j];
             } else {
 #pragma clang fp contract(off)
                 const float scaled = f * sx * sw4[q][j];
@@ -232,11 +234,13 @@ inline bool small64_shape_ok(const GemmArgs& g) {
 // kernel is the 16 KiB a 64 x 64 tile pulls out of L2 per slab, not latency.
 constexpr int kSmall64Stages = 4;
 
-template <class Op, int ScaleKind>
+template <class Op, int ScaleKind, bool RoundFirst = false>
 inline void launch_small64(const GemmArgs& g, hipStream_t stream) {
     using Cfg = Small64Cfg<kSmall64Stages>;
+    if constexpr (!RoundFirst && ScaleKind == SCALE_TENSOR)
+        if (g.round_first) return launch_small64<Op, ScaleKind, true>(g, stream);
     const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64);
-    auto kern = gemm_small64_kernel<Op, ScaleKind, kSmall64Stages>;
+    auto kern = gemm_small64_kernel<Op, ScaleKind, kSmall64Stages, RoundFirst>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
     note_kernel("small64");
