@@ -175,10 +175,12 @@ void launch_rows(const GemmArgs& g, const RopeCacheArgs& rc, hipStream_t stream)
 }
 
 // fp8: the same plan and the same token-group instances; bf16 or fp32-accumulator output
-template <int Fmt, int RG, int MB, int NW>
+template <int Fmt, int RG, int MB, int NW, bool RoundFirst = false>
 void launch_rows_fp8_inst(const GemmArgs& g, const RowsPlan& p, bool rowcol, hipStream_t stream) {
+    if constexpr (!RoundFirst)
+        if (g.round_first) return launch_rows_fp8_inst<Fmt, RG, MB, NW, true>(g, p, rowcol, stream);
     constexpr int lds_bytes = gemv_rows_lds_bytes<RG, MB, NW>();
-    auto kern = gemv_fp8_rows_kernel<Fmt, RG, MB, NW>;
+    auto kern = gemv_fp8_rows_kernel<Fmt, RG, MB, NW, RoundFirst>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_allowed);
     note_kernel("gemv_rows_fp8");
