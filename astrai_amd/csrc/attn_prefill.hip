@@ -41,9 +41,10 @@
 // which puts a whole memory round trip into each 64-key block. The blocks without and with masking
 // are two loops, not two branches of one: at a join of the two the compiler moved all accumulators
 // from one register set to another on every block.
-// What bounds it: the vector ALU and the matrix pipe about equally (16 exponentials and ~65 other
-// vector instructions per lane beside 16 MFMAs of 32 cycles a tile, two waves per SIMD). Measured (graph
-// replays, before -> after the two points above, the backward walk and reading strided tensors in place):
+// What bounds it: vector ALU and matrix pipe of a SIMD share its issue slots (16 exponentials and ~65 other vector
+// instructions per lane beside 16 MFMAs of 32 cycles a tile, two waves per SIMD). Counters: 4 x 2048 tokens, 16/4 heads x
+// 128: matrix pipe busy 48% of the SIMD cycles, vector ALU 53%; ragged, 32/8 heads x 64 with P in two terms: 37% and 72%.
+// Measured (graph replays, before -> after the two points above, the backward walk and reading strided tensors in place):
 // 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 148 -> 80 us (860 TFLOP/s; before it
 // went through the paged form), ragged 16 x 175..700 tokens of 32/8 heads x 64 in a pool 173 -> 77 us
 // (450 TFLOP/s, P in two terms; before on the general kernel). 192 / 135 registers where the joined

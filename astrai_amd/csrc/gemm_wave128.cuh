@@ -595,8 +595,6 @@ inline bool wave128_shape_ok(const GemmArgs& g) {
     return pingpong_shape_ok(g) && g.out_kind == OUT_BF16 && (g.n & 7) == 0 && g.n <= (1 << 22);
 }
 
-constexpr int64_t kTailTiles = 384;
-
 // A token count a little above a multiple of 256 (M = 256 q + r, 0 < r <= 128) can cost the
 // large-tile kernel a whole extra round of workgroups for r rows (4100 x 4096 x 4096: 272 tiles on
 // 256 compute units, 96 us against 69 us at 4096 rows). When it does, and the weight-streaming
@@ -643,6 +641,7 @@ inline bool wave128_takes(const GemmArgs& g) {
 // 11008 199 -> 142 (64), 3001 x 11264 x 2048 77 -> 73 (176), 3001 x 11008 x 4096 133 -> 123 (172), 5000 x 4096 x 4096
 // 86 -> 77 (256), 5500 x 4096 x 4096 87 -> 84 (352); beyond that nothing is left: 6000 x 4096 x 4096 89 -> 89
 // (480), 6500 x 11264 x 2048 134 -> 141 (440).
+constexpr int64_t kTailTiles = 384;
 inline int tile_tail_rows(const GemmArgs& g) {
     const int64_t tm = (g.m + 255) / 256, tn = (g.n + 255) / 256, rounds = (tm * tn + 255) / 256;
     const int64_t head = (rounds - 1) * 256 / tn;  // row tiles that stay

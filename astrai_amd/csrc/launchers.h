@@ -149,8 +149,8 @@ struct AttnDecodeArgs {
 int64_t attn_decode_workspace_floats(int batch, int n_kv_heads, int nsplit, int nq);
 bool launch_attn_decode(const AttnDecodeArgs& a, hipStream_t stream);
 
-// attn_prefill.hip: causal grouped-query attention of a block of new tokens against
-// the dense bf16 KV cache; head_dim 128, n_heads / n_kv_heads in {2, 4, 8}
+// attn_prefill.hip: causal grouped-query attention of a block of new tokens against a dense bf16 KV cache, strided
+// tensors or a paged pool; head_dim 128 or 64, n_heads / n_kv_heads in {1, 2, 4, 8}
 struct AttnStride {
     int64_t batch, head, row;  // elements; rows of head_dim consecutive elements, 16-byte aligned
 };
@@ -241,9 +241,9 @@ bool launch_gemm_int8_swiglu(const GemmArgs& g, hipStream_t stream);
 // Row-range kernel for up to 128 tokens (K % 256 == 0), four-wave 256x256 kernel for the large
 // shapes it takes; false otherwise (the caller runs the plain GEMM and an addition pass).
 bool launch_gemm_int8_resid(const GemmArgs& g, hipStream_t stream);
-// out = bf16(y + resid) over `total` bf16 elements; out may be y
 // out[m, n] = bf16(out[m, n] + bias[n]), n % 8 == 0
 void launch_add_bias_bf16(void* out, const void* bias, int64_t rows, int64_t n, hipStream_t stream);
+// out = bf16(y + resid) over `total` bf16 elements; out may be y
 void launch_add_bf16(const void* y, const void* resid, void* out, int64_t total, hipStream_t stream);
 bool launch_gemm_fp8_tiled(const GemmArgs& g, int fmt, hipStream_t stream);
 // sa per activation row [M], sb per weight row [N], bf16 output

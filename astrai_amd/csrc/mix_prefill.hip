@@ -28,9 +28,8 @@
 // soft-capped scores (two more quarter-rate operations a score). Measured inside the models, before -> after
 // these points: latent 32 x 512 tokens, 16 heads 113 -> 105 us; grouped 1 x 4096, 16/4 heads 176 -> 160 us.
 // A wave's stream is a software pipeline over tiles: the score MFMAs of tile T + 1 are issued among the
-// exponentials of tile T, the value MFMAs of tile T among the masking of tile T + 1. One copy of the
-// step masks every tile: a second copy without masking costs more in registers and code than the
-// compares (157 us against 107 us for 32 x 512 tokens, 16 heads of 128 + 64).
+// exponentials of tile T, the value MFMAs of tile T among the masking of tile T + 1. (An unmasked copy of the step behind
+// a branch instead of in a loop of its own: 157 us against 107 us for 32 x 512 tokens, 16 heads of 128 + 64.)
 #include "lds_dma.cuh"
 #include "mix_common.cuh"
 #include "mix_launchers.h"

@@ -882,10 +882,12 @@ def decode_nsplit(pairs: int, max_keys: int) -> int:
 def paged_nsplit(pairs: int, max_keys: int) -> int:
     """:func:`decode_nsplit` of a paged step, whose bf16 output a merge of any number of splits side by side writes. Below
     64 pairs as many splits as make 512 workgroups, none that could not hold 64 keys of the slot table's width (one
-    sequence of 8192 keys, 16 / 4 heads: 8 splits 36 us, 64 12; four of 3000: 8 splits 20, 32 12). From 64 pairs on
-    three workgroups for each CU, none that could not hold 160 keys (two for each CU, three: 32 x 3000 keys, 16 / 4 heads
-    33.2 us, 31.1, 32 / 4 heads 40.8, 36.2; 64 x 1500 41.2, 34.1; sequences of 100 keys behind a table of 16384 9.5,
-    10.7)."""
+    sequence of 8192 keys, 16 / 4 heads: 8 splits 36 us, 64 12; four of 3000: 8 splits 20, 32 12; short ones behind a
+    wide table do not lose: one of 100 keys 10.3, 9.0, 15 of 100 11.8, 8.8). From 64 pairs on three workgroups for each
+    CU, none that could not hold 160 keys, against two (16 / 4 heads, 32 x 3000 keys 33.2 us, 31.1; 32 / 4 heads 40.8,
+    36.2; 64 x 1500 32.4, 28.7). The context's length decides and only the table's width is known here: up to some 500
+    keys behind a wide table two are as good or better (64 x 100 9.5, 10.5; 64 x 300 13.5, 13.3; 32 x 530 12.3, 13.0), past
+    1000 three."""
     pairs = max(1, pairs)
     if pairs >= 64:
         return max(1, min(768 // pairs, max_keys // 160))

@@ -699,8 +699,9 @@ def rglru_nseg(batch: int, blocks: int, bp: int, seq: int) -> int:
     """Segments of a sequence that run side by side. A segment is walked tile by tile, 5.8 us per 64 tokens, so few
     sequences are cut until there are about four workgroups for each CU, into segments of as many tiles each, down to
     one (1 x 4096 tokens, 8 blocks of 256: 8 segments 97 us, 16 69, 32 65; 1 x 512: 4 segments 28, 8 18). Cut,
-    everything is computed twice: from about 176 workgroups on one walk is the shorter (128: 98 us whole, 66 cut;
-    256: 58 whole, 64 cut), and so it is for two tiles, whose halves would be walked twice."""
+    everything is computed twice: from about 176 workgroups on one walk is the shorter (1024 tokens, blocks of 256: 128
+    workgroups 100 us whole, 65 cut, 160 101, 76, 192 102, 106, 256 112, 116; blocks of 128: 176 80, 60, 192 80, 81, 256
+    81, 82), and so it is for two tiles, whose halves would be walked twice."""
     groups, tiles = batch * blocks * -(-bp // 64), -(-seq // 64)
     return 1 if groups > 176 or tiles <= 2 else -(-tiles // max(1, tiles * groups // 1024))
 
