@@ -47,7 +47,7 @@
 // Measured (graph replays, before -> after the two points above, the backward walk and reading strided tensors in place):
 // 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 148 -> 80 us (860 TFLOP/s; before it
 // went through the paged form), ragged 16 x 175..700 tokens of 32/8 heads x 64 in a pool 173 -> 77 us
-// (450 TFLOP/s, P in two terms; before on the general kernel). 192 / 135 registers where the joined
+// (450 TFLOP/s, P in two terms; before on the general kernel). 186 / 133 registers where the joined
 // loops took 256 with spills: two / three workgroups per CU.
 #include <algorithm>
 #include <climits>
