@@ -273,7 +273,6 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     }
     pmin = __builtin_amdgcn_readfirstlane(pmin);
     kmax_w = max(__builtin_amdgcn_readfirstlane(min(kmax_w, kmax)), -1);
-    const bool sees_a_key = pq >= 0;
     if (!row_live) pq = kmax_w;  // rows past the end see everything and are never stored
     const int nkb = kmax / kKB + 1;     // (kmax = -1, an empty sequence: one block of masked keys)
     const int tiles_w = kmax_w / 32 + 1;  // tiles this wave computes
@@ -310,8 +309,11 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     // outgrown it by more than kSlack does the wave pay for rescaling its accumulators;
     // until then probabilities may reach 2^kSlack, which fp32 sums and bf16 operands hold.
     constexpr float kSlack = 8.0f;
-    float m_run = kNegBig, l_run = 0.0f;
+    // It starts half way between any score and a hidden key's, whose probability is then an exact zero: started at
+    // the stand-in itself, a row whose first tiles are hidden took it for a maximum, and the rounding of c times it
+    // for a probability, infinite at every other scale.
     const float c = a.scale * 1.44269504088896340736f;  // scores to log2 units
+    float m_run = 0.5f * kNegBig * fminf(c, 1.0f), l_run = 0.0f;
     const f32x16 zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     // V^T operand of 32 dims x 16 keys: two transposing reads. In each 16-lane group, lane
@@ -497,15 +499,11 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     // ---- normalise and write [batch, seq, heads*D]: through this wave's part of the
     // (now idle) LDS, so that the 32 x D tile leaves as whole rows
     l_run += __shfl_xor(l_run, 32, kWave);
-    // a row that sees no key at all (empty sequence, or more queries than keys) yields zeros
-    // (with a mask tensor a row may have met nothing but masked scores: its reference maximum
-    // then still is the stand-in for -inf, times c once it has been through a rescale, and its
-    // sum is no NaN). A NaN in l_run comes from a score the row sees, and goes out.
-    const bool met_a_key = !MASK || m_run > 0.5f * kNegBig * fminf(c, 1.0f) || l_run != l_run;
-    const bool has_value = l_run != 0.0f && sees_a_key && met_a_key;
+    // a row that meets no key (empty sequence, more queries than keys, all of them masked) has a sum of zero and
+    // yields zeros. A NaN in l_run comes from a score the row sees, and goes out.
+    const bool has_value = l_run != 0.0f;
     const float inv = has_value ? 1.0f / l_run : 0.0f;
-    // (its accumulators hold whatever masked scores made of them: the difference of two roundings of
-    // c * kNegBig may be large enough for an infinite probability)
+    // (its accumulators hold zeros times what the value rows held)
     if (!has_value) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
