@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
         float p[4], ps = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            p[i] = (sc[i] > 0.5f * kNegBig) ? __expf(sc[i] - m_new) : 0.0f;
+            p[i] = sc[i] <= 0.5f * kNegBig ? 0.0f : __expf(sc[i] - m_new);  // (so that a NaN is not taken for hidden)
             ps += p[i];
         }
         ps += __shfl_xor(ps, 16, kWave);

@@ -137,7 +137,7 @@ __device__ __forceinline__ void tile_step(const u32x4 (&kf)[D / 32], const u32x4
     float p[4], ps = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        p[i] = (sc[i] > 0.5f * kNegBig) ? __expf(sc[i] - m_new) : 0.0f;
+        p[i] = sc[i] <= 0.5f * kNegBig ? 0.0f : __expf(sc[i] - m_new);  // (so that a NaN is not taken for hidden)
         ps += p[i];
     }
     l = l * alpha + ps;  // this lane's four keys only: the four lanes of a query are added up at the end

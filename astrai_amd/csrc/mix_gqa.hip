@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void gqa_partial_kernel(GqaRowsArgs a, GqaDims
         for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                s[u][e] = s[u][e] > 0.5f * kNegBig ? __builtin_amdgcn_exp2f(s[u][e] - m_new) : 0.0f;
+                s[u][e] = s[u][e] <= 0.5f * kNegBig ? 0.0f : __builtin_amdgcn_exp2f(s[u][e] - m_new);  // (so that a NaN is not taken for hidden)
                 l += s[u][e];
             }
         u32x4 hi, lo;

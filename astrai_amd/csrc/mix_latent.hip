@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, RH <= 8 ? 2 : 1) void latent_partial_kernel(La
         l *= alpha;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            p[e] = p[e] > 0.5f * kNegBig ? __builtin_amdgcn_exp2f(p[e] - m_new) : 0.0f;
+            p[e] = p[e] <= 0.5f * kNegBig ? 0.0f : __builtin_amdgcn_exp2f(p[e] - m_new);  // (so that a NaN is not taken for hidden)
             l += p[e];
         }
         u32x4 hi, lo;
