@@ -286,6 +286,23 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
     return check_launch("few_rows_linear");
 }
 
+int astrai_mix_prompt_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m, int64_t n,
+                             int64_t k, int act, void* stream) {
+    MIX_TRY(check_ptrs("prompt_linear", x, w, (const void*)out));
+    if (bias) MIX_TRY(check_ptrs("prompt_linear", bias));
+    if (act != -1 && act != ASTRAI_MIX_SILU && act != ASTRAI_MIX_GELU)
+        return fail(ASTRAI_MIX_BAD_ARG, "prompt_linear: unknown activation %d", act);
+    if (act != -1 && bias) return fail(ASTRAI_MIX_BAD_ARG, "prompt_linear: an activation takes no bias");
+    if (m < 0 || m > kMaxInt || n <= 0 || n > kMaxInt || k <= 0 || k > kMaxInt || ldx < k || ldx > kMaxInt)
+        return fail(ASTRAI_MIX_BAD_ARG, "prompt_linear: bad size %lld x %lld x %lld", (long long)m, (long long)n, (long long)k);
+    if (m == 0) return ASTRAI_MIX_OK;
+    const PromptLinearArgs a = {x, ldx, w, bias, out, (int)m, (int)n, (int)k};
+    if (!launch_prompt_linear(a, act, static_cast<hipStream_t>(stream)))
+        return fail(ASTRAI_MIX_UNSUPPORTED, "prompt_linear: %lld x %lld x %lld is not covered", (long long)m, (long long)n,
+                    (long long)k);
+    return check_launch("prompt_linear");
+}
+
 int astrai_mix_head_gated_rms_norm(const void* o, const void* g, int64_t ldg, const float* w, void* out, int64_t rows,
                                    int64_t heads, int64_t vp, int64_t count, float eps, int dtype, void* stream) {
     MIX_TRY(check_dtype("head_gated_rms_norm", dtype));

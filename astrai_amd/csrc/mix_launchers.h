@@ -58,6 +58,19 @@ bool few_rows_linear_supported(int64_t m, int64_t n, int64_t k, bool act);
 // act: kActSilu / kActGelu (out = act(gate) * up), or -1
 bool launch_few_rows_linear(const FewRowsArgs& a, int act, bool out_float, hipStream_t stream);
 
+// ---- mix_gemm.hip ---------------------------------------------------------------------------
+struct PromptLinearArgs {
+    const void* x;     // bf16 [m, k], rows ldx apart
+    int64_t ldx;
+    const void* w;     // bf16 [n, k]; with an activation [2 n, k], gate rows first
+    const void* bias;  // bf16 [n] or null; null with an activation
+    void* out;         // bf16 [m, n]
+    int m, n, k;
+};
+bool prompt_linear_supported(int64_t m, int64_t n, int64_t k, int64_t ldx, bool act);
+// act: kActSilu / kActGelu (out = act(gate) * up), or -1
+bool launch_prompt_linear(const PromptLinearArgs& a, int act, hipStream_t stream);
+
 struct HeadNormArgs {
     const void* o;    // [rows, heads * vp]
     const void* g;    // [rows, ldg]

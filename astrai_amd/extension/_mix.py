@@ -41,6 +41,7 @@ PROTOTYPES = {
         [_P, _I64, _P, _I64, _F32, _P, _P, _I64] + [_P] * 4 + [_I64, _I64, _F32, _INT, _INT, _P], _INT),
     "astrai_mix_act_mul": ([_P, _P, _I64, _I64, _INT, _INT, _P], _INT),
     "astrai_mix_few_rows_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _INT, _P], _INT),
+    "astrai_mix_prompt_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _P], _INT),
     "astrai_mix_head_gated_rms_norm": ([_P, _P, _I64, _P, _P] + [_I64] * 4 + [_F32, _INT, _P], _INT),
     "astrai_mix_gated_rms_norm": ([_P, _P, _I64, _P, _P, _I64, _I64, _I64, _F32, _INT, _P], _INT),
     "astrai_mix_latent_append": (
@@ -281,6 +282,41 @@ def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
         _check(lib.astrai_mix_few_rows_linear(
             x.data_ptr(), k if x.is_contiguous() else x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
             out.data_ptr(), m, n, k, -1 if act is None else ACTIVATIONS[act], int(out_dtype == torch.float32), _stream(x)), lib)
+    return out
+
+
+def prompt_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                            act: Optional[str] = None) -> bool:
+    """The calls :func:`prompt_linear` takes: bf16 on one GPU, any number of rows of ``x [.., k]`` at 16-byte boundaries,
+    ``k`` a multiple of 128, the outputs of 8, operands under 2 GiB each."""
+    n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
+    rows = x.numel() // k if k else 0
+    if x.size(-1) != k or rows <= 0 or k % 128 or n % 8 or (weight.size(0) + 256) * k * 2 >= 2 ** 31 or n >= 2 ** 22:
+        return False
+    if not (x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and weight.device == x.device):
+        return False
+    if not weight.is_contiguous() or weight.data_ptr() % 16 or x.data_ptr() % 16:
+        return False
+    if bias is not None and not (act is None and bias.dtype == torch.bfloat16 and bias.device == x.device
+                                 and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
+        return False
+    if not (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k)):
+        return False
+    return (rows + 256) * (k if x.is_contiguous() else x.stride(0)) * 2 < 2 ** 31
+
+
+def prompt_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                  act: Optional[str] = None) -> torch.Tensor:
+    """``F.linear`` of a prompt's rows, or ``act(gate) * up`` as :func:`few_rows_linear`."""
+    lib = _require()
+    if not prompt_linear_supported(x, weight, bias, act):
+        raise RuntimeError("prompt_linear: operands are not covered")
+    n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
+    with _on_device(x.device):
+        out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=x.dtype)
+        _check(lib.astrai_mix_prompt_linear(
+            x.data_ptr(), k if x.is_contiguous() else x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
+            out.data_ptr(), x.numel() // k, n, k, -1 if act is None else ACTIVATIONS[act], _stream(x)), lib)
     return out
 
 

@@ -40,6 +40,8 @@ LATENT_ROWS_MAX = 16
 GQA_ROWS_MAX = 16
 # a block of at most this many tokens runs the recurrence token by token
 LIGHTNING_STEP_MAX = 8
+# from this many rows on a product may run on `prompt_linear`
+PROMPT_ROWS = 512
 
 
 @dataclass
@@ -109,23 +111,54 @@ def few_rows_most(n: int, k: int, act: bool) -> int:
     return _mix.FEW_ROWS if wide else 32
 
 
-def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
-    """Whether this product runs on the kernel for a decode step's few rows: everything ``F.linear`` may have
-    to do besides (gradients, autocasting, a policy's handler, transforms) is left to it, and so are the sizes at which
-    the library is the faster one."""
-    k = x.size(-1)
-    if torch.compiler.is_compiling() or not k or x.numel() // k > few_rows_most(weight.size(0), k, act is not None):
-        return False
-    return (plain(x, weight, bias) and _mix.few_rows_linear_supported(x, weight, bias, act) and dispatch.linear_is_stock()
-            and not torch.is_autocast_enabled("cuda")
+def only_product(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> bool:
+    """Whether ``F.linear`` would have nothing to do besides the product: no gradients, autocasting, policy's handler of
+    ``aten::linear``, transforms. Otherwise the call is left to it."""
+    return (plain(x, weight, bias) and dispatch.linear_is_stock() and not torch.is_autocast_enabled("cuda")
             and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, weight, bias))))
 
 
+def few_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
+    """Whether this product runs on the kernel for a decode step's few rows: what :func:`only_product` refuses is left to
+    ``F.linear``, and so are the sizes at which the library is the faster one."""
+    k = x.size(-1)
+    if torch.compiler.is_compiling() or not k or x.numel() // k > few_rows_most(weight.size(0), k, act is not None):
+        return False
+    return only_product(x, weight, bias) and _mix.few_rows_linear_supported(x, weight, bias, act)
+
+
+def tile_fill(m: int, n: int) -> float:
+    """The share of the compute units' tiles that holds outputs where ``m x n`` of them go out on 256 x 256 tiles, 256 at
+    a time."""
+    tiles = -(-m // 256) * -(-n // 256)
+    return m * n / (65536 * 256 * max(-(-tiles // 256), 1))
+
+
+def prompt_rows(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, act: Optional[str] = None) -> bool:
+    """Whether this product of a prompt's rows runs on :func:`_mix.prompt_linear`, whose rate is 1.45 PFLOP/s times
+    :func:`tile_fill`. With an activation the library's side is its product and ``act_mul``, together 0.9 to 1.2
+    (us, ours / theirs, gate and up of 5632 from 2048 values: 1024 rows (fill 0.69) 42 / 56, 2048 (0.69) 86 / 91, 4096
+    (0.92) 139 / 180, 16384 (1) 533 / 627; 1500 (0.50) 86 / 79). Without one the library reaches 1.4 to 1.6 where the
+    outputs are whole tiles, which no fill makes up for, and 0.9 to 1.1 where they are not (2048 values to 3664: 3000 rows
+    (0.65) 42 / 50, 16384 (0.89) 187 / 225, 5000 (0.55) 86 / 80; to 6416: 2048 (0.78) 45 / 55, 8192 (0.78) 182 / 188, 5000
+    (0.64) 132 / 129)."""
+    k = x.size(-1)
+    if torch.compiler.is_compiling() or not k:
+        return False
+    m, n = x.numel() // k, weight.size(0)
+    if tile_fill(m, n) < 0.65 or (act is None and n % 256 == 0):
+        return False
+    return only_product(x, weight, bias) and _mix.prompt_linear_supported(x, weight, bias, act)
+
+
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
-    # (the rows first: a prompt's eager products are to pay nothing for the question)
-    if x.numel() > _mix.FEW_ROWS * x.size(-1) or not few_rows(x, weight, bias):
-        return F.linear(x, weight, bias)
-    return _mix.few_rows_linear(x, weight, bias)
+    # (the sizes first: eager products of middling prompts are to pay nothing for the question)
+    if x.numel() > _mix.FEW_ROWS * x.size(-1):
+        if x.numel() >= PROMPT_ROWS * x.size(-1) and weight.size(0) % 256 and prompt_rows(x, weight, bias):
+            return _mix.prompt_linear(x, weight, bias)
+    elif few_rows(x, weight, bias):
+        return _mix.few_rows_linear(x, weight, bias)
+    return F.linear(x, weight, bias)
 
 
 class HeadLinear(Linear):
@@ -617,10 +650,11 @@ class GatedMLP(nn.Module):
                 lin.assign(name, t)
 
     def forward(self, h: Tensor) -> Tensor:
-        up = self.gate_up
-        if (h.numel() <= _mix.FEW_ROWS * h.size(-1) and type(up) is PackedLinear and up.bias is None and not observed(up)
-                and few_rows(h, up.weight, act=self.act)):
-            return self.down(_mix.few_rows_linear(h, up.weight, act=self.act))
+        up, rows = self.gate_up, h.numel() // max(h.size(-1), 1)
+        if (rows <= _mix.FEW_ROWS or rows >= PROMPT_ROWS) and type(up) is PackedLinear and up.bias is None and not observed(up):
+            fused, pays = ((_mix.few_rows_linear, few_rows) if rows <= _mix.FEW_ROWS else (_mix.prompt_linear, prompt_rows))
+            if pays(h, up.weight, act=self.act):
+                return self.down(fused(h, up.weight, act=self.act))
         return self.down(_mix.act_mul(self.gate_up(h), self.act))
 
 

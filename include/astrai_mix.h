@@ -74,6 +74,13 @@ int astrai_mix_act_mul(const void* gu, void* h, int64_t rows, int64_t ff, int ac
 int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m,
                                int64_t n, int64_t k, int act, int out_float, void* stream);
 
+/*
+ * The same of a prompt's rows, on 256 x 256 tiles, bf16 out; k % 128 == 0, n % 8 == 0, x, w and 256 rows of out each under
+ * 2 GiB. The sums run in one order whatever m is.
+ */
+int astrai_mix_prompt_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m, int64_t n,
+                             int64_t k, int act, void* stream);
+
 /* out = o / sqrt(mean(o^2) + eps) * w * sigmoid(g); the mean over `count` of the n columns (the
  * others are padding). g rows have stride ldg. n % 4 == 0, ldg % 4 == 0. */
 int astrai_mix_gated_rms_norm(const void* o, const void* g, int64_t ldg, const float* w, void* out,

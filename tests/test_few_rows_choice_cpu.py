@@ -157,3 +157,15 @@ def test_sizes_at_which_the_kernel_is_the_faster_one(n, k, act, most):
     with torch.no_grad():
         for rows in (1, 32, 33, 64, 65):
             assert mixers.few_rows(torch.zeros(1).expand(rows, k), w, act=act) == (rows <= most)
+
+
+@pytest.mark.parametrize("m,n,act,taken", [
+    (1024, 2 * 5632, "silu", True), (16384, 2 * 5632, "gelu_tanh", True), (1500, 2 * 5632, "silu", False),
+    (4096, 3664, None, True), (5000, 3664, None, False), (4096, 4096, None, False), (2048, 6416, None, True)])
+def test_prompt_sizes_at_which_the_tiles_are_the_faster_ones(monkeypatch, m, n, act, taken):
+    monkeypatch.setattr(_mix, "prompt_linear_supported", lambda *a: True)
+    x, w = torch.zeros(1).expand(m, 2048), torch.zeros(1).expand(n, 2048)
+    with torch.no_grad():
+        assert mixers.prompt_rows(x, w, act=act) == taken
+    w = torch.zeros(1).expand(n, 2048).requires_grad_(True)
+    assert not mixers.prompt_rows(x, w, act=act)
