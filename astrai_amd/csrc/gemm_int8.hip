@@ -1,9 +1,9 @@
 // int8 x int8 -> int32 MFMA GEMMs, per-token x per-channel dequant epilogue.
-// Large shapes run v_mfma_i32_32x32x32_i8 on 256x256 tiles: the four-wave
-// 128x128-register-tile kernel for bf16 output, the eight-wave ping-pong kernel
+// Large shapes run on 256x256 tiles: the four-wave
+// 128x128-register-tile kernel (v_mfma_i32_16x16x64_i8) for bf16 output, the eight-wave ping-pong kernel (32x32x32)
 // for int32 output; shapes with too few of those tiles for the chip run 128x128
-// tiles of the same instruction; the generic tiled kernel takes everything else.
-#include "gemm_wave128.cuh"
+// tiles of the latter instruction; the generic tiled kernel takes everything else.
+#include "gemm_wave128_i8.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
 #include "gemm_tile.cuh"
@@ -18,7 +18,7 @@ bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_
         if (const int r = tail_on_decode_kernel ? ragged_tail_rows(g) : 0) {
             split_rows(g, r, true, head, tail);
             if (wave128_shape_ok(head) && launch_gemv_int8(tail, stream)) {   // (disjoint rows: either order)
-                launch_wave128<Op32I8, SCALE_ROWCOL>(head, stream);
+                launch_wave128_i8<>(head, stream);
                 return true;
             }
         }
@@ -26,10 +26,10 @@ bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_
             split_rows(g, r, true, head, tail);
             if (mid128_shape_ok(tail)) launch_mid128<Op32I8, SCALE_ROWCOL>(tail, stream);
             else launch_small64<Op32I8, SCALE_ROWCOL>(tail, stream);
-            launch_wave128<Op32I8, SCALE_ROWCOL>(head, stream);
+            launch_wave128_i8<>(head, stream);
             return true;
         }
-        launch_wave128<Op32I8, SCALE_ROWCOL>(g, stream);
+        launch_wave128_i8<>(g, stream);
     } else
 #endif
     if (pingpong_shape_ok(g))
@@ -46,7 +46,7 @@ bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_
 bool launch_gemm_int8_swiglu(const GemmArgs& g, hipStream_t stream) {
     if (!tiled_shape_ok(g) || !wave128_shape_ok(g) || (g.n & 127) != 0 || g.bias != nullptr || !g.row_max)
         return false;
-    launch_wave128<Op32I8, SCALE_ROWCOL, EPI_SWIGLU>(g, stream);
+    launch_wave128_i8<EPI_SWIGLU>(g, stream);
     return true;
 }
 
@@ -58,11 +58,11 @@ bool launch_gemm_int8_resid(const GemmArgs& g, hipStream_t stream) {
         GemmArgs head, tail;
         split_rows(g, r, true, head, tail);
         if (wave128_shape_ok(head) && launch_gemv_int8(tail, stream)) {
-            launch_wave128<Op32I8, SCALE_ROWCOL, EPI_RESID>(head, stream);
+            launch_wave128_i8<EPI_RESID>(head, stream);
             return true;
         }
     }
-    launch_wave128<Op32I8, SCALE_ROWCOL, EPI_RESID>(g, stream);
+    launch_wave128_i8<EPI_RESID>(g, stream);
     return true;
 }
 
@@ -73,7 +73,7 @@ bool launch_gemm_int8_rope_cache_large(const GemmArgs& g, const RopeCacheArgs& r
     const int64_t lim = (int64_t)1 << 31;
     if ((int64_t)g.m * rc.n_heads * 256 >= lim || (int64_t)rc.batch * rc.n_kv_heads * rc.max_len * 256 >= lim)
         return false;
-    launch_wave128<Op32I8, SCALE_ROWCOL, EPI_ROPE>(g, stream, rc);
+    launch_wave128_i8<EPI_ROPE>(g, stream, rc);
     return true;
 }
 

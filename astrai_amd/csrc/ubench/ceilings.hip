@@ -45,7 +45,15 @@ __device__ unsigned random_fp8x4(unsigned seed, int random) {
     return r;
 }
 
-// WHICH: 0 fp8 16x16x128, 1 fp8 32x32x64, 2 i8 32x32x32, 3 i8 16x16x64
+// (of bf16 the same bytes are sign, exponents about 1 and mantissas at random)
+__device__ int random_bf16x2(unsigned seed, int random) {
+    return random ? (int)((hash32(seed) & 0x80ff80ffu) | 0x3f003f00u) : 0;
+}
+
+// The small MFMAs in assembly, sums in place: behind the builtins the compiler rotates sums through other registers.
+#define MFMA_IN_PLACE(op, c, a, b) __asm__ volatile(op " %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b))
+
+// WHICH: 0 fp8 16x16x128, 1 fp8 32x32x64, 2 i8 32x32x32, 3 i8 16x16x64, 4 bf16 16x16x32, 5 bf16 32x32x16
 template <int WHICH>
 __global__ __launch_bounds__(256) void mfma_loop(int iters, float* out, unsigned long long* t,
                                                  int random) {
@@ -60,6 +68,10 @@ __global__ __launch_bounds__(256) void mfma_loop(int iters, float* out, unsigned
         for (int j = 0; j < 4; ++j) {
             a4[i][j] = random ? (int)hash32(threadIdx.x * 131 + i * 17 + j) : 0;
             b4[i][j] = random ? (int)hash32(threadIdx.x * 257 + i * 29 + j + 99) : 0;
+            if (WHICH >= 4) {
+                a4[i][j] = random_bf16x2(threadIdx.x * 131 + i * 17 + j, random);
+                b4[i][j] = random_bf16x2(threadIdx.x * 257 + i * 29 + j + 99, random);
+            }
         }
     const unsigned long long w0 = wall_clock64(), c0 = clock64();
     float s = 0;
@@ -69,7 +81,8 @@ __global__ __launch_bounds__(256) void mfma_loop(int iters, float* out, unsigned
         for (int it = 0; it < iters; ++it)
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                c[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i & 3], b[(i >> 1) & 3], c[i], 0, 0, 0, 0, 0, 0);
+                MFMA_IN_PLACE("v_mfma_f32_16x16x128_f8f6f4", c[i], a[i & 3], b[(i >> 1) & 3]);
+        __asm__ volatile("s_nop 15");
         for (int i = 0; i < 8; ++i) s += c[i][0];
     } else if constexpr (WHICH == 1) {
         f32x16 c[4];
@@ -89,13 +102,33 @@ __global__ __launch_bounds__(256) void mfma_loop(int iters, float* out, unsigned
             for (int i = 0; i < 4; ++i)
                 c[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a4[i], b4[(i + 1) & 3], c[i], 0, 0, 0);
         for (int i = 0; i < 4; ++i) s += c[i][0];
+    } else if constexpr (WHICH == 4) {
+        f32x4 c[8];
+        for (int i = 0; i < 8; ++i) c[i] = f32x4{0, 0, 0, 0};
+        for (int it = 0; it < iters; ++it)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) MFMA_IN_PLACE("v_mfma_f32_16x16x32_bf16", c[i], a4[i & 3], b4[(i >> 1) & 3]);
+        __asm__ volatile("s_nop 15");
+        for (int i = 0; i < 8; ++i) s += c[i][0];
+    } else if constexpr (WHICH == 5) {
+        typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+        f32x16 c[4];
+        for (int i = 0; i < 4; ++i)
+            for (int j = 0; j < 16; ++j) c[i][j] = 0;
+        for (int it = 0; it < iters; ++it)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                c[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a4[i]),
+                                                               __builtin_bit_cast(bf16x8, b4[(i + 1) & 3]), c[i], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) s += c[i][0];
     } else {
         i32x4 c[8];
         for (int i = 0; i < 8; ++i) c[i] = i32x4{0, 0, 0, 0};
         for (int it = 0; it < iters; ++it)
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                c[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a4[i & 3], b4[(i >> 1) & 3], c[i], 0, 0, 0);
+                MFMA_IN_PLACE("v_mfma_i32_16x16x64_i8", c[i], a4[i & 3], b4[(i >> 1) & 3]);
+        __asm__ volatile("s_nop 15");
         for (int i = 0; i < 8; ++i) s += c[i][0];
     }
     const unsigned long long w1 = wall_clock64(), c1 = clock64();
@@ -213,6 +246,8 @@ int main() {
     run_mfma<0>("fp8 16x16x128", 8 * 2.0 * 16 * 16 * 128, out, t);
     run_mfma<2>("i8 32x32x32", 4 * 2.0 * 32 * 32 * 32, out, t);
     run_mfma<3>("i8 16x16x64", 8 * 2.0 * 16 * 16 * 64, out, t);
+    run_mfma<5>("bf16 32x32x16", 4 * 2.0 * 32 * 32 * 16, out, t);
+    run_mfma<4>("bf16 16x16x32", 8 * 2.0 * 16 * 16 * 32, out, t);
 
     const size_t big = (size_t)1 << 30;
     void* buf;

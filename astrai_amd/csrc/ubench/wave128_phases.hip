@@ -30,18 +30,18 @@ using namespace w8a8;
 
 template <class Op, int SK, int KO>
 static float time_us(const GemmArgs& g) {
-    auto kern = gemm_wave128_kernel<Op, SK, EPI_PLAIN, KO>;
+    auto kern = gemm_wave128_kernel<Op, SK, KO>;
     CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Wave128Cfg::LDS_BYTES));
     const int tiles = ((g.m + 255) / 256) * ((g.n + 255) / 256);
     hipEvent_t e0, e1;
     CK(hipEventCreate(&e0));
     CK(hipEventCreate(&e1));
-    for (int i = 0; i < 300; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g, RopeCacheArgs{});
+    for (int i = 0; i < 300; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g);
     CK(hipDeviceSynchronize());
     std::vector<float> ts;
     for (int rep = 0; rep < 7; ++rep) {
         CK(hipEventRecord(e0));
-        for (int i = 0; i < 100; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g, RopeCacheArgs{});
+        for (int i = 0; i < 100; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g);
         CK(hipEventRecord(e1));
         CK(hipEventSynchronize(e1));
         float ms;
@@ -214,10 +214,9 @@ int main(int argc, char** argv) {
 
     CK(hipMemset(a, 0, (size_t)M * K));
     CK(hipMemset(b, 0, (size_t)N * K));
-    for (int which = 0; which < 2; ++which) {
-        const float us = which ? time_us<Op32I8, SCALE_ROWCOL, 0>(g) : time_us<Op32F8<0>, SCALE_TENSOR, 0>(g);
-        printf("%s zeros %dx%dx%d: %.2f us; stamps of workgroup 0 in shader clock cycles\n",
-               which ? "int8" : "fp8", M, N, K, us);
+    {
+        const float us = time_us<Op32F8<0>, SCALE_TENSOR, 0>(g);
+        printf("fp8 zeros %dx%dx%d: %.2f us; stamps of workgroup 0 in shader clock cycles\n", M, N, K, us);
         print_stamps(dbg, K, {0, 3});
     }
     {
@@ -227,7 +226,6 @@ int main(int argc, char** argv) {
     }
     knockouts<Op32F8<0>, SCALE_TENSOR>("fp8 zeros", g);
     knockouts_q16<SCALE_TENSOR>("fp8 zeros", g);
-    knockouts<Op32I8, SCALE_ROWCOL>("int8 zeros", g);
 
     {
         std::vector<unsigned char> ra((size_t)M * K), rb((size_t)N * K);
@@ -243,15 +241,6 @@ int main(int argc, char** argv) {
     for (int rep = 0; rep < 3; ++rep)
         printf("alternating, normal operands: 32x32x64 %.2f us, 16x16x128 %.2f us\n",
                time_us<Op32F8<0>, SCALE_TENSOR, 0>(g), time_q16_us<SCALE_TENSOR, 0>(g));
-    {
-        std::vector<signed char> ra((size_t)M * K), rb((size_t)N * K);
-        auto gauss = [] { float u = 0; for (int i = 0; i < 12; ++i) u += (float)rand() / RAND_MAX; return u - 6.0f; };
-        for (auto& x : ra) x = (signed char)std::max(-127.0f, std::min(127.0f, rintf(gauss() * 127.0f / 4.5f)));
-        for (auto& x : rb) x = (signed char)std::max(-127.0f, std::min(127.0f, rintf(gauss() * 127.0f / 4.5f)));
-        CK(hipMemcpy(a, ra.data(), ra.size(), hipMemcpyHostToDevice));
-        CK(hipMemcpy(b, rb.data(), rb.size(), hipMemcpyHostToDevice));
-    }
-    knockouts<Op32I8, SCALE_ROWCOL>("int8 normal operands (amax at 4.5 sigma)", g);
     pingpong_section(dbg);
     return 0;
 }

@@ -288,10 +288,10 @@ def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
 def prompt_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                             act: Optional[str] = None) -> bool:
     """The calls :func:`prompt_linear` takes: bf16 on one GPU, any number of rows of ``x [.., k]`` at 16-byte boundaries,
-    ``k`` a multiple of 128, the outputs of 8, operands under 2 GiB each."""
+    ``k`` a multiple of 64, the outputs of 8, operands under 2 GiB each."""
     n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
     rows = x.numel() // k if k else 0
-    if x.size(-1) != k or rows <= 0 or k % 128 or n % 8 or (weight.size(0) + 256) * k * 2 >= 2 ** 31 or n >= 2 ** 22:
+    if x.size(-1) != k or rows <= 0 or k % 64 or n % 8 or (weight.size(0) + 256) * k * 2 >= 2 ** 31 or n >= 2 ** 22:
         return False
     if not (x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and weight.device == x.device):
         return False

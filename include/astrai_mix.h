@@ -75,7 +75,7 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
                                int64_t n, int64_t k, int act, int out_float, void* stream);
 
 /*
- * The same of a prompt's rows, on 256 x 256 tiles, bf16 out; k % 128 == 0, n % 8 == 0, x, w and 256 rows of out each under
+ * The same of a prompt's rows, on 256 x 256 tiles, bf16 out; k % 64 == 0, n % 8 == 0, x, w and 256 rows of out each under
  * 2 GiB. The sums run in one order whatever m is.
  */
 int astrai_mix_prompt_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m, int64_t n,
