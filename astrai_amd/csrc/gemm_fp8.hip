@@ -1,11 +1,9 @@
 // fp8 (OCP e4m3fn / e5m2) MFMA GEMMs, per-tensor scales (optional bias, bf16 /
 // e4m3 / fp32 output) or one scale per activation row and per weight row (bf16 output).
 // Large shapes run 256x256 tiles: the four-wave 128x128-register-tile kernel for bf16
-// output (v_mfma_f32_16x16x128_f8f6f4, or v_mfma_f32_32x32x64_f8f6f4 for an odd number of
-// K slabs), the eight-wave ping-pong kernel (32x32x64) for the other outputs; bf16 shapes with too few of
-// those tiles for the chip run 128x128 tiles of the same instruction; the generic
+// output (v_mfma_f32_16x16x128_f8f6f4), the eight-wave ping-pong kernel (32x32x64) for the other outputs; bf16 shapes with too few of
+// those tiles for the chip run 128x128 tiles of that instruction; the generic
 // tiled kernel takes everything else.
-#include "gemm_wave128.cuh"
 #include "gemm_wave128_q16.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
@@ -14,23 +12,14 @@
 namespace w8a8 {
 
 namespace {
-// The four-wave kernel has two instances: on the 16x16x128 MFMA (faster under the board's power
-// cap: 49.6 against 52.3 us at 4096^3 on normally distributed operands) when the slab count is
-// even -- its loop walks two slabs a turn --, else on the 32x32x64 MFMA.
 template <int Fmt, int ScaleKind>
 void launch_big(const GemmArgs& g, hipStream_t stream) {
-    const bool round_first = g.bias && g.round_first;
-    if ((g.k & 255) == 0) {
-        if constexpr (Fmt == 0 && ScaleKind == SCALE_TENSOR)
-            if (round_first) return launch_wave128_q16<0, SCALE_TENSOR, true>(g, stream);
-        if (!round_first) return launch_wave128_q16<Fmt, ScaleKind>(g, stream);
-    }
-    if (!round_first) return launch_wave128<Op32F8<Fmt>, ScaleKind>(g, stream);
-    // (an odd number of slabs: that kernel's epilogue has no registers to spare)
+    if (!g.bias || !g.round_first) return launch_wave128_q16<Fmt, ScaleKind>(g, stream);
+    if constexpr (Fmt == 0 && ScaleKind == SCALE_TENSOR) return launch_wave128_q16<0, SCALE_TENSOR, true>(g, stream);
+    // (no instance: nothing asks for the others often)
     GemmArgs plain = g;
     plain.bias = nullptr;
-    if ((g.k & 255) == 0) launch_wave128_q16<Fmt, ScaleKind>(plain, stream);
-    else launch_wave128<Op32F8<Fmt>, ScaleKind>(plain, stream);
+    launch_wave128_q16<Fmt, ScaleKind>(plain, stream);
     launch_add_bias_bf16(g.out, g.bias, g.m, g.n, stream);
 }
 template <int Fmt, int ScaleKind>

@@ -1,13 +1,36 @@
-// The main loop of the 256 x 256 NT products on 16x16 MFMAs of 16 cycles (int8, bf16): four waves of 128 x 128, one to a
-// SIMD, software-pipelined inside each wave. The walk is that of gemm_wave128_q16.cuh (a slab is 128 bytes of K, its
-// quadrants of 64 x 64 in an order in which consecutive ones share an operand half, the half the next one is missing read
-// from LDS meanwhile, direct-to-LDS loads two slabs ahead into three activation and two weight stages, one barrier a
-// slab); a slab is two MFMAs of a pair of 16-row sub-tiles, on the two 16-byte pieces of a lane, where fp8 has one of 32
-// cycles. All MFMAs of the first pieces of a quadrant come before those of the second, sixteen accumulators apart.
+// The main loop of the 256 x 256 NT products on 16x16 MFMAs: four waves of 128 x 128, one to a SIMD, software-pipelined
+// inside each wave. Operand bytes only: 8-bit or bf16 values differ in the instruction.
 //
-// Why the small MFMAs: under the power cap loops of nothing else sustain on random operands 1.82 PFLOP/s of bf16
-// 32x32x16 and 1.92 of 16x16x32, 3.36 POP/s of int8 32x32x32 and 3.77 of 16x16x64. (On zeros 2.48 and 2.33, 4.96 and 4.71;
-// other instructions fit less well beside them: 32 cycles of a large one hide 24 of others, 16 of a small one about 4.)
+// A slab is 128 bytes of K: one fp8 16x16x128 MFMA of 32 cycles for a pair of 16-row sub-tiles, or two of 16 cycles
+// (int8 16x16x64, bf16 16x16x32) on the two 16-byte pieces of a lane; all MFMAs of the first pieces of a quadrant come
+// before those of the second, sixteen accumulators apart. A slab is cut into quadrants: the 128(m) x 128(n) wave tile =
+// 2 x 2 quadrants of 64 x 64 = 4 x 4 pairs of sub-tiles, 512 MFMA cycles. A quadrant needs one half of the wave's
+// activation rows (4 sub-tiles of 16 rows: 32 registers) and one half of its weight rows (32 registers). The
+// quadrants are walked so that consecutive ones share one of the two halves, and
+// during a quadrant the one half the next quadrant is missing is read from LDS into
+// the buffer that is idle: four 32-register buffers XA, XB (activation halves 0, 1)
+// and WA, WB (weight halves 0, 1).
+// The walk has period two slabs (Q<x half><w half>, what is read meanwhile):
+//   even slab k:   Q00 | W1(k) -> WB     Q01 | X1(k) -> XB      -- barrier --
+//                  Q11 | X0(k+1) -> XA   Q10 | W1(k+1) -> WB
+//   odd slab k+1:  Q01 | W0(k+1) -> WA   Q00 | X1(k+1) -> XB    -- barrier --
+//                  Q10 | X0(k+2) -> XA   Q11 | W0(k+2) -> WA
+// Every quadrant has 8 LDS reads of 1 KiB and 4 direct-to-LDS loads between its MFMAs. The order is written out and pinned,
+// so that the MFMA pipe always has the next instruction waiting; the loads are spread evenly, because the CU's one load
+// path takes a 1 KiB instruction every 16 cycles: four waves must not issue them faster than one per 128 cycles each.
+// Three activation and two weight stages (all 160 KiB): all of a slab's operands have been read when its second quadrant
+// ends, at the slab's one barrier; the activation rows of slab k+2 are fetched before it (into the stage of slab k-1), the
+// weight rows behind it.
+//
+// Operand roles and layouts: weight rows are the first MFMA operand; lane l supplies
+// row (l & 15) of a sub-tile and the 32 bytes of K-group (l >> 4) (chunks 2g, 2g+1
+// of the row's eight 16-byte chunks; any assignment of K bytes to lanes is a valid
+// contraction as long as both operands share it); the accumulator lane holds, for
+// token m = l & 15, the four outputs n = 4 (l >> 4) .. + 3 of the sub-tile.
+//
+// Why not 32x32 MFMAs: under the power cap loops of nothing else sustain on random operands 1.82 PFLOP/s of bf16
+// 32x32x16 and 1.92 of 16x16x32, 3.36 POP/s of int8 32x32x32 and 3.77 of 16x16x64, 3.77 PFLOP/s of fp8 32x32x64 and 4.16
+// of 16x16x128. (On zeros 2.48 and 2.33, 4.96 and 4.71, 4.99 and 4.98; other instructions fit less well beside them: 32 cycles of a large one hide 24 of others, 16 of a small one about 4.)
 // The sums stay in one register each, by assembly: behind the builtins the compiler gives results other registers than
 // it takes sums from and moves them back, which halves the rate.
 #pragma once
@@ -15,17 +38,46 @@
 
 namespace w8a8 {
 
-struct Walk16I8 {
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+
+// A lane's 32 bytes of a row, as the MFMAs of a slab take them: one for each 16-byte piece,
+struct Walk16Pieces {
+    static constexpr int kMfmas = 2;
+    struct Frag {
+        u32x4 piece[2];
+        __device__ __forceinline__ void set(int j, u32x4 v) { piece[j] = v; }
+    };
+};
+
+struct Walk16I8 : Walk16Pieces {
     using Acc = i32x4;
-    static __device__ __forceinline__ void mma(u32x4 w, u32x4 x, Acc& acc) {
-        __asm__ volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
+    static __device__ __forceinline__ void mma(int c, const Frag& w, const Frag& x, Acc& acc) {
+        __asm__ volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(w.piece[c]), "v"(x.piece[c]));
     }
 };
 
-struct Walk16Bf16 {
+struct Walk16Bf16 : Walk16Pieces {
     using Acc = f32x4;
-    static __device__ __forceinline__ void mma(u32x4 w, u32x4 x, Acc& acc) {
-        __asm__ volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
+    static __device__ __forceinline__ void mma(int c, const Frag& w, const Frag& x, Acc& acc) {
+        __asm__ volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w.piece[c]), "v"(x.piece[c]));
+    }
+};
+
+// or one of twice the cycles for both (Fmt 0 e4m3, 1 e5m2)
+template <int Fmt>
+struct Walk16F8 {
+    static constexpr int kMfmas = 1;
+    using Acc = f32x4;
+    struct Frag {
+        u32x8 both;
+        __device__ __forceinline__ void set(int j, u32x4 v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) both[4 * j + e] = v[e];
+        }
+    };
+    static __device__ __forceinline__ void mma(int, const Frag& w, const Frag& x, Acc& acc) {
+        __asm__ volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0 cbsz:%3 blgp:%3"
+                         : "+a"(acc) : "v"(w.both), "v"(x.both), "n"(Fmt));
     }
 };
 
@@ -41,11 +93,13 @@ __device__ __forceinline__ void walk16_offsets(int lane, int first, int live, ui
 
 // acc[weight sub-tile][token sub-tile] of a wave's 128 x 128: lane (lgrp, lrow) = (lane >> 4, lane & 15) holds, for token
 // 16 mi + lrow, weight rows 16 ni + 4 lgrp .. + 3. The stages are free for other use when it returns.
-template <class Op>
+// (KO: knock-outs, see gemm_wave128.cuh)
+template <class Op, int KO = 0>
 __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_bytes, const uint32_t (&x_off)[8],
                                        const void* w, uint32_t w_bytes, const uint32_t (&w_off)[8], int slabs,
                                        typename Op::Acc (&acc)[8][8]) {
     using Cfg = Wave128Cfg;
+    using Frag = typename Op::Frag;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lrow = lane & 15, lgrp = lane >> 4;
@@ -58,29 +112,34 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
         lds_dma16(rw, dma_base + Cfg::W_BASE + stage * Cfg::OPERAND_BYTES + r * 1024, w_off[r], k0);
     };
 
-    // the lane's two 16-byte pieces of its row of a 16-row sub-tile
-    int frag_off[2];
+    // the lane's two 16-byte pieces of its row of a 16-row sub-tile. (Whole addresses that the compiler does not take apart
+    // again: every weight stage and sub-tile is then a constant offset away, every sub-tile of an activation stage too.)
+    int x_rd[2], w_rd[2];
     {
         const int sw = (lrow & 7) ^ ((lrow >> 3) & 1);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) frag_off[j] = lrow * 128 + (((2 * lgrp + j) ^ sw) << 4);
+        for (int j = 0; j < 2; ++j) {
+            const int off = lrow * 128 + (((2 * lgrp + j) ^ sw) << 4);
+            x_rd[j] = off + (wave & 1) * 128 * 128;
+            w_rd[j] = off + (wave >> 1) * 128 * 128 + Cfg::W_BASE;
+            __asm__("" : "+v"(x_rd[j]), "+v"(w_rd[j]));
+        }
     }
-    const int x_rd = (wave & 1) * 128 * 128, w_rd = Cfg::W_BASE + (wave >> 1) * 128 * 128;
     // read r of 8 of half h of an operand: piece r / 4 of sub-tile 4h + r % 4
-    auto read_x = [&](int r, int stage, int h, u32x4 (&f)[4][2]) __attribute__((always_inline)) {
-        f[r & 3][r >> 2] = *reinterpret_cast<const u32x4*>(
-            lds + x_rd + stage * Cfg::OPERAND_BYTES + (4 * h + (r & 3)) * 2048 + frag_off[r >> 2]);
+    auto read_x = [&](int r, int stage, int h, Frag (&f)[4]) __attribute__((always_inline)) {
+        f[r & 3].set(r >> 2, *reinterpret_cast<const u32x4*>(
+            lds + x_rd[r >> 2] + stage * Cfg::OPERAND_BYTES + (4 * h + (r & 3)) * 2048));
     };
-    auto read_w = [&](int r, int stage, int h, u32x4 (&f)[4][2]) __attribute__((always_inline)) {
-        f[r & 3][r >> 2] = *reinterpret_cast<const u32x4*>(
-            lds + w_rd + stage * Cfg::OPERAND_BYTES + (4 * h + (r & 3)) * 2048 + frag_off[r >> 2]);
+    auto read_w = [&](int r, int stage, int h, Frag (&f)[4]) __attribute__((always_inline)) {
+        f[r & 3].set(r >> 2, *reinterpret_cast<const u32x4*>(
+            lds + w_rd[r >> 2] + stage * Cfg::OPERAND_BYTES + (4 * h + (r & 3)) * 2048));
     };
 
 #pragma unroll
     for (int ni = 0; ni < 8; ++ni)
 #pragma unroll
         for (int mi = 0; mi < 8; ++mi) acc[ni][mi] = typename Op::Acc{0, 0, 0, 0};
-    u32x4 xa[4][2], xb[4][2], wa[4][2], wb[4][2];
+    Frag xa[4], xb[4], wa[4], wb[4];
 
     // slabs 0 and 1 in flight; slab 0 visible; halves 0 of slab 0 in xa, wa
     {
@@ -95,37 +154,49 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
         for (int r = 0; r < 8; ++r) dma_x(r, rx1, 1, 128u);
 #pragma unroll
         for (int r = 0; r < 8; ++r) dma_w(r, rw1, 1, 128u);
-        wait_vmcnt<16>();  // slab 0
+        if constexpr (KO & KO_LOADS) {  // every stage holds operand bytes once and for all
+#pragma unroll
+            for (int r = 0; r < 8; ++r) dma_x(r, rx1, 2, 256u);
+            wait_vmcnt<0>();
+        } else {
+            wait_vmcnt<16>();  // slab 0
+        }
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 8; ++r) read_x(r, 0, 0, xa);
 #pragma unroll
         for (int r = 0; r < 8; ++r) read_w(r, 0, 0, wa);
+        if constexpr (KO & KO_LDS_READS) {  // all four buffers hold operand bytes once and for all
+#pragma unroll
+            for (int r = 0; r < 8; ++r) read_x(r, 0, 1, xb);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) read_w(r, 0, 1, wb);
+        }
     }
 
     int xs = 0;  // k % 3
     // One quadrant: 32 MFMAs on (xf, wf); between them the 8 reads of the half the next quadrant is missing (in the first
     // half: the last has returned when they are needed) and 4 loads
-    auto phase = [&](const u32x4 (&xf)[4][2], const u32x4 (&wf)[4][2], int xh, int wh, auto&& rd, auto&& ld) __attribute__((always_inline)) {
+    auto phase = [&](const Frag (&xf)[4], const Frag (&wf)[4], int xh, int wh, auto&& rd, auto&& ld) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
+        for (int i = 0; i < 16 * Op::kMfmas; ++i) {
             const int c = i >> 4, mi = (i >> 2) & 3, ni = i & 3;
-            Op::mma(wf[ni][c], xf[mi][c], acc[4 * wh + ni][4 * xh + mi]);
+            if constexpr (!(KO & KO_MFMA)) Op::mma(c, wf[ni], xf[mi], acc[4 * wh + ni][4 * xh + mi]);
 #pragma unroll
             for (int r = 0; r < 8; ++r)
-                if (r * 2 == i) rd(r);
+                if (r * Op::kMfmas == i && !(KO & KO_LDS_READS)) rd(r);
 #pragma unroll
             for (int d = 0; d < 4; ++d)
-                if (d * 8 + 4 == i) ld(d);
+                if ((d * 4 + 2) * Op::kMfmas == i && !(KO & KO_LOADS)) ld(d);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     // one slab; ODD: its place in the two-slab walk. Past the end of K the loads run on an empty descriptor
     auto slab = [&](auto odd_c, int k) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd_c)::value;
-        const int ws = k & 1;
+        constexpr int ws = ODD ? 1 : 0;           // k % 2
         const int xs1 = (xs == 2) ? 0 : xs + 1;   // (k + 1) % 3
         const int xs2 = (xs == 0) ? 2 : xs - 1;   // (k + 2) % 3
         const uint32_t k2 = (uint32_t)(k + 2) << 7;
@@ -143,7 +214,7 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
         }
         // Slab k+1 has landed for this wave (all but this half's eight loads are older) and this wave has read slab k;
         // after the barrier both hold for every wave
-        wait_vmcnt<8>();
+        wait_vmcnt<(KO & KO_LOADS) ? 0 : 8>();
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         phase_barrier();
         // (after the last slab the reads fetch stale bytes that are never used)

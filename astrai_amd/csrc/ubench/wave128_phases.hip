@@ -1,6 +1,6 @@
 // Where the four-wave 256x256x128 GEMM kernel's time goes, measured on the kernel itself:
 //   1. phase stamps (the shader clock counter read by every wave at kernel start, main-loop
-//      start, main-loop end and kernel end; workgroup 0) on all-zero operands, where the clock
+//      end (its prologue included) and kernel end; workgroup 0) on all-zero operands, where the clock
 //      stays at its maximum;
 //   2. knock-outs: the same kernel with one class of instructions removed (LDS operand reads,
 //      global->LDS loads, MFMAs, output stores), timed on zeros and on normally distributed fp8
@@ -8,7 +8,6 @@
 //      power cap, so a knocked-out class gives back its issue slots AND its energy (clock).
 // Build: make -C astrai_amd/csrc ubench     Run: astrai_amd/csrc/ubench/wave128_phases [M N K]
 #define W8A8_PP_TIMING 1
-#include "../gemm_wave128.cuh"
 #include "../gemm_wave128_q16.cuh"
 
 #include <algorithm>
@@ -28,33 +27,8 @@ using namespace w8a8;
         }                                                                              \
     } while (0)
 
-template <class Op, int SK, int KO>
-static float time_us(const GemmArgs& g) {
-    auto kern = gemm_wave128_kernel<Op, SK, KO>;
-    CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Wave128Cfg::LDS_BYTES));
-    const int tiles = ((g.m + 255) / 256) * ((g.n + 255) / 256);
-    hipEvent_t e0, e1;
-    CK(hipEventCreate(&e0));
-    CK(hipEventCreate(&e1));
-    for (int i = 0; i < 300; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g);
-    CK(hipDeviceSynchronize());
-    std::vector<float> ts;
-    for (int rep = 0; rep < 7; ++rep) {
-        CK(hipEventRecord(e0));
-        for (int i = 0; i < 100; ++i) kern<<<tiles, 256, Wave128Cfg::LDS_BYTES, 0>>>(g);
-        CK(hipEventRecord(e1));
-        CK(hipEventSynchronize(e1));
-        float ms;
-        CK(hipEventElapsedTime(&ms, e0, e1));
-        ts.push_back(ms * 10.0f);
-    }
-    std::sort(ts.begin(), ts.end());
-    return ts[3];
-}
-
-// the 16x16x128 instance of the four-wave kernel (fp8 only)
 template <int SK, int KO>
-static float time_q16_us(const GemmArgs& g) {
+static float time_us(const GemmArgs& g) {
     auto kern = gemm_wave128_q16_kernel<0, SK, KO>;
     CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Wave128Cfg::LDS_BYTES));
     const int tiles = ((g.m + 255) / 256) * ((g.n + 255) / 256);
@@ -160,40 +134,23 @@ static void pingpong_section(unsigned long long* dbg) {
         printf("ping-pong kernel, per-tensor scales, %s: %.2f us (%.0f Tops/s)\n",
                random ? "normal operands" : "zeros", us, ops / us / 1e6);
         if (!random) print_stamps(dbg, K, {0, 4});
-        us = time_us<Op32F8<0>, SCALE_TENSOR, 0>(g);
+        us = time_us<SCALE_TENSOR, 0>(g);
         printf("four-wave kernel, per-tensor scales, %s: %.2f us (%.0f Tops/s)\n",
                random ? "normal operands" : "zeros", us, ops / us / 1e6);
     }
     CK(hipFree(a)); CK(hipFree(b)); CK(hipFree(out)); CK(hipFree(s));
 }
 
-template <class Op, int SK>
+template <int SK>
 static void knockouts(const char* what, const GemmArgs& g) {
     const double ops = 2.0 * g.m * g.n * (double)g.k;
-    const float base = time_us<Op, SK, 0>(g);
+    const float base = time_us<SK, 0>(g);
     printf("%s: whole kernel %.2f us (%.0f Tops/s)\n", what, base, ops / base / 1e6);
-    printf("  without LDS operand reads      %.2f us\n", time_us<Op, SK, KO_LDS_READS>(g));
-    printf("  without global->LDS loads      %.2f us\n", time_us<Op, SK, KO_LOADS>(g));
-    printf("  without either                 %.2f us\n", time_us<Op, SK, KO_LDS_READS | KO_LOADS>(g));
-    printf("  without output stores          %.2f us\n", time_us<Op, SK, KO_STORES>(g));
-    printf("  without MFMAs                  %.2f us\n", time_us<Op, SK, KO_MFMA>(g));
-}
-
-template <int SK>
-static void knockouts_q16(const char* what, const GemmArgs& g) {
-    const double ops = 2.0 * g.m * g.n * (double)g.k;
-    const float base = time_q16_us<SK, 0>(g);
-    printf("%s, 16x16x128 instance: whole kernel %.2f us (%.0f Tops/s)\n", what, base, ops / base / 1e6);
-    printf("  without LDS operand reads      %.2f us\n", time_q16_us<SK, KO_LDS_READS>(g));
-    printf("  without global->LDS loads      %.2f us\n", time_q16_us<SK, KO_LOADS>(g));
-    printf("  without either                 %.2f us\n", time_q16_us<SK, KO_LDS_READS | KO_LOADS>(g));
-    printf("  without output stores          %.2f us\n", time_q16_us<SK, KO_STORES>(g));
-    printf("  without MFMAs                  %.2f us\n", time_q16_us<SK, KO_MFMA>(g));
-    printf("  without the per-slab barrier   %.2f us\n", time_q16_us<SK, KO_BARRIER>(g));
-    printf("  without the per-slab waits     %.2f us\n", time_q16_us<SK, KO_WAITS>(g));
-    printf("  without barrier and waits      %.2f us\n", time_q16_us<SK, KO_BARRIER | KO_WAITS>(g));
-    printf("  without barrier, waits, loads and LDS reads %.2f us\n",
-           time_q16_us<SK, KO_BARRIER | KO_WAITS | KO_LOADS | KO_LDS_READS>(g));
+    printf("  without LDS operand reads      %.2f us\n", time_us<SK, KO_LDS_READS>(g));
+    printf("  without global->LDS loads      %.2f us\n", time_us<SK, KO_LOADS>(g));
+    printf("  without either                 %.2f us\n", time_us<SK, KO_LDS_READS | KO_LOADS>(g));
+    printf("  without output stores          %.2f us\n", time_us<SK, KO_STORES>(g));
+    printf("  without MFMAs                  %.2f us\n", time_us<SK, KO_MFMA>(g));
 }
 
 int main(int argc, char** argv) {
@@ -215,17 +172,11 @@ int main(int argc, char** argv) {
     CK(hipMemset(a, 0, (size_t)M * K));
     CK(hipMemset(b, 0, (size_t)N * K));
     {
-        const float us = time_us<Op32F8<0>, SCALE_TENSOR, 0>(g);
+        const float us = time_us<SCALE_TENSOR, 0>(g);
         printf("fp8 zeros %dx%dx%d: %.2f us; stamps of workgroup 0 in shader clock cycles\n", M, N, K, us);
         print_stamps(dbg, K, {0, 3});
     }
-    {
-        const float us = time_q16_us<SCALE_TENSOR, 0>(g);
-        printf("fp8 16x16x128 instance zeros %dx%dx%d: %.2f us; stamps of workgroup 0 in shader clock cycles\n", M, N, K, us);
-        print_stamps(dbg, K, {0, 3});
-    }
-    knockouts<Op32F8<0>, SCALE_TENSOR>("fp8 zeros", g);
-    knockouts_q16<SCALE_TENSOR>("fp8 zeros", g);
+    knockouts<SCALE_TENSOR>("fp8 zeros", g);
 
     {
         std::vector<unsigned char> ra((size_t)M * K), rb((size_t)N * K);
@@ -235,12 +186,7 @@ int main(int argc, char** argv) {
         CK(hipMemcpy(a, ra.data(), ra.size(), hipMemcpyHostToDevice));
         CK(hipMemcpy(b, rb.data(), rb.size(), hipMemcpyHostToDevice));
     }
-    knockouts<Op32F8<0>, SCALE_TENSOR>("fp8 normal operands (amax at 4.5 sigma)", g);
-    knockouts_q16<SCALE_TENSOR>("fp8 normal operands (amax at 4.5 sigma)", g);
-    // the two instances in alternation on the same operands
-    for (int rep = 0; rep < 3; ++rep)
-        printf("alternating, normal operands: 32x32x64 %.2f us, 16x16x128 %.2f us\n",
-               time_us<Op32F8<0>, SCALE_TENSOR, 0>(g), time_q16_us<SCALE_TENSOR, 0>(g));
+    knockouts<SCALE_TENSOR>("fp8 normal operands (amax at 4.5 sigma)", g);
     pingpong_section(dbg);
     return 0;
 }

@@ -1,0 +1,46 @@
+"""8-bit products on the 256 x 256 tiles: even and odd numbers of K slabs, ragged edges, tile counts of every kind."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _codes(seed, rows, k):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randint(-127, 128, (rows, k), generator=g, device=DEV, dtype=torch.int8)
+
+
+@pytest.mark.parametrize("m,n,k", [(3585, 3720, 256), (3500, 3592, 384), (4096, 4096, 640), (8200, 1800, 896)])
+def test_int8_bits(m, n, k):
+    """bf16 of the exact sum times both steps, rounded product by product (and once more for bias and residual)."""
+    from astrai_amd.extension import _cabi
+    a, b = _codes(m, m, k), _codes(n, n, k)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    sa, sb = (torch.rand(r, generator=g, device=DEV) * 0.01 + 0.001 for r in (m, n))
+    bias, resid = (torch.randn(*s, generator=g, device=DEV).bfloat16() for s in ((n,), (m, n)))
+    acc = (a.float() @ b.float().t())   # (sums under 2^24: exact)
+    y = acc * sa[:, None] * sb
+    assert torch.equal(_cabi.mm_int8(a, b, sa, sb), y.bfloat16())
+    assert "wave128" in _cabi.last_kernel()
+    assert torch.equal(_cabi.mm_int8(a, b, sa, sb, bias), (y + bias.float()).bfloat16())
+    assert torch.equal(_cabi.mm_int8_resid(a, b, sa, sb, resid), (y.bfloat16().float() + resid.float()).bfloat16())
+
+
+@pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("m,n,k", [(3585, 3720, 256), (3500, 3592, 384), (4096, 4096, 640)])
+def test_fp8_against_float64(fmt, m, n, k):
+    """One rounding to bf16 (2^-8 of |y|), fp32 sums; bias before or behind a rounding."""
+    from astrai_amd.extension import _cabi
+    g = torch.Generator(device=DEV).manual_seed(k)
+    a, b = (torch.randn(r, k, generator=g, device=DEV).to(fmt) for r in (m, n))
+    sa, sb = (torch.rand(1, generator=g, device=DEV) + 0.5 for _ in range(2))
+    bias = torch.randn(n, generator=g, device=DEV).bfloat16()
+    step = (sa.double() * sb.double()).item()
+    y, weight = a.double() @ b.double().t() * step, a.double().abs() @ b.double().abs().t() * step
+    slack = 2.0 ** -8 * y.abs() + k * 2.0 ** -23 * weight
+    for extra, kw in ((0.0, {}), (bias.double(), dict(bias=bias)), (bias.double(), dict(bias=bias, round_first=True))):
+        got = _cabi.mm_fp8(a, b, sa, sb, **kw).double()
+        want = y + extra
+        assert ((got - want).abs() <= slack + 2.0 ** -8 * want.abs()).all(), kw
