@@ -4,16 +4,42 @@
 // 128x128 tiles of the same instruction for mid-size shapes (a slab's product scaled before it
 // joins the accumulator), the generic tiled kernel otherwise (one 16x16x128 MFMA per scale
 // block, partial product promoted with sa[m,kb] * sb[n/128,kb]).
-#include "gemm_pingpong.cuh"
+#include "gemm_wave128.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
 #include "gemm_tile.cuh"
 
 namespace w8a8 {
 
+namespace {
+
+// Tiles of 256 x 256 where they fill most of the chip, or where 128 x 128 tiles would put a second workgroup on compute
+// units (from 257 of them), which takes nearly twice as long as one (7168 -> 2048: 1900 tokens, 240 tiles, 69 us with the
+// quantizer, 2300, 288, 105), where a round of large tiles costs little more than the first: 86 us at 2300 tokens, 92 at
+// 4096 (113), 4096 -> 4096 54 at 1100 (63) and 56 at 2500 (93), 2048 -> 7168 36 at 1500 (53).
+bool large_tiles_take(const GemmArgs& g) {
+    if ((g.n & 7) != 0 || g.out_kind != OUT_BF16) return false;
+    return pingpong_shape_ok(g) || (g.k >= 256 && (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 256);
+}
+
+// Tails on smaller tiles as in tile_tail_rows, up to the same number: 4300 x 7168 x 2048 158 -> 94 us (32 tiles), 4300 x 4096 x
+// 4096 117 -> 89 (64), 5000 x 4096 x 4096 120 -> 113 (256); 3001 x 2048 x 7168 68 -> 74 (336), not taken.
+constexpr int64_t kBlockTailTiles = 256;
+
+}  // namespace
+
 bool launch_gemm_fp8_block128_tiled(const GemmArgs& g, hipStream_t stream) {
     if (!tiled_shape_ok(g) || (g.k & 127) != 0) return false;
-    if (pingpong_shape_ok(g) && (g.n & 7) == 0 && g.out_kind == OUT_BF16) {
+    if (large_tiles_take(g)) {
+        if (const int r = tile_tail_rows(g, kBlockTailTiles)) {
+            GemmArgs head, tail;
+            split_rows(g, r, false, head, tail);
+            tail.sa = g.sa + (size_t)head.m * (g.k >> 7);   // a step per row and K block
+            if (mid128_shape_ok(tail)) launch_mid128<Op32F8<0>, SCALE_BLOCK128>(tail, stream);
+            else launch_small64<Op32F8<0>, SCALE_BLOCK128>(tail, stream);
+            launch_pingpong<Op32F8<0>, SCALE_BLOCK128, PingPongCfgBlock>(head, stream);
+            return true;
+        }
         launch_pingpong<Op32F8<0>, SCALE_BLOCK128, PingPongCfgBlock>(g, stream);
         return true;
     }

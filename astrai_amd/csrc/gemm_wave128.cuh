@@ -69,16 +69,15 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
     if (g.resid) tail.resid = static_cast<const uint8_t*>(g.resid) + row0 * (size_t)g.n * 2;
 }
 
-// Plain bf16 products that the large tiles take: where they fill most of the chip, or where 128 x 128 tiles
-// would need a second round of two workgroups per compute unit (from 513 of them). One round of large tiles is
-// cheaper than that however empty: K = 2048 27 us against 33 (3072 x 3072), K = 4096 46 against 58 (2816 x 4096),
-// K = 5632 61 against 71 (5000 x 2048), K = 11008 105 against 136 (2816 x 4096); one round of 128 x 128 tiles
-// (512) is cheaper the other way: 22, 40, 49, 91 us.
+// Plain bf16 products that the large tiles take: where they fill most of the chip, or from 449 tiles of 128 x 128 on. Two
+// workgroups of those share a compute unit and take longer the more units have two, where a round of large tiles costs
+// the same however empty (int8, us, 128 x 128 / large: 2048 -> 2048 34 / 34 at 448 tiles, 36 / 34 at 512; 5632 -> 2048
+// 65 / 65 and 71 / 67; 4096 -> 4096 49 / 50 and 53 / 50; 11008 -> 4096 105 / 106 and 117 / 108, 97 / 104 at 384).
 inline bool wave128_takes(const GemmArgs& g) {
     if (wave128_shape_ok(g)) return true;
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 256 || g.out_kind != OUT_BF16 || (g.n & 7) != 0 || g.n > (1 << 22))
         return false;
-    return (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 512;
+    return (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 448;
 }
 
 // Rows of a product that are better served by smaller tiles in a launch of their own: those past the last
@@ -89,12 +88,12 @@ inline bool wave128_takes(const GemmArgs& g) {
 // 86 -> 77 (256), 5500 x 4096 x 4096 87 -> 84 (352); beyond that nothing is left: 6000 x 4096 x 4096 89 -> 89
 // (480), 6500 x 11264 x 2048 134 -> 141 (440).
 constexpr int64_t kTailTiles = 384;
-inline int tile_tail_rows(const GemmArgs& g) {
+inline int tile_tail_rows(const GemmArgs& g, int64_t most = kTailTiles) {
     const int64_t tm = (g.m + 255) / 256, tn = (g.n + 255) / 256, rounds = (tm * tn + 255) / 256;
     const int64_t head = (rounds - 1) * 256 / tn;  // row tiles that stay
     if (rounds < 2 || head < 1 || head >= tm) return 0;
     const int64_t rows = g.m - head * 256;
-    return (rows + 127) / 128 * ((g.n + 127) / 128) <= kTailTiles ? (int)rows : 0;
+    return (rows + 127) / 128 * ((g.n + 127) / 128) <= most ? (int)rows : 0;
 }
 
 }  // namespace w8a8

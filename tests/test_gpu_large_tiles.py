@@ -44,3 +44,20 @@ def test_fp8_against_float64(fmt, m, n, k):
         got = _cabi.mm_fp8(a, b, sa, sb, **kw).double()
         want = y + extra
         assert ((got - want).abs() <= slack + 2.0 ** -8 * want.abs()).all(), kw
+
+
+@pytest.mark.parametrize("m,n,k", [(1100, 4096, 512), (4300, 4096, 256), (2570, 2056, 384), (6000, 1536, 256), (1500, 7168, 256)])
+def test_block_scales_against_float64(m, n, k):
+    """The 128-block product where it moves to large tiles, and where its last rows go out on smaller ones."""
+    from astrai_amd.extension.ops import fp8_block
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x = (torch.randn(m, k, generator=g, device=DEV) * torch.rand(m, 1, generator=g, device=DEV)).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.1).bfloat16()
+    (x8, sx), (w8, sw) = fp8_block.quantize_act_block128(x), fp8_block.quantize_weight_block128(w)
+    xd = x8.double().reshape(m, k // 128, 128) * sx.double().reshape(m, k // 128, 1)
+    rows = torch.arange(n, device=DEV) // 128
+    wd = w8.double().reshape(n, k // 128, 128) * sw.double().reshape(-1, k // 128)[rows][:, :, None]
+    want = xd.reshape(m, k) @ wd.reshape(n, k).t()
+    weight = xd.abs().reshape(m, k) @ wd.abs().reshape(n, k).t()
+    got = fp8_block.mm_fp8_blockscaled(x8, w8, sx, sw).double()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + k * 2.0 ** -23 * weight).all()
