@@ -781,6 +781,142 @@ int astrai_w8a8_gemm_fp8_pt_rounded_bias(const void* a8, const void* b8, const f
     return check_launch("gemm_fp8_pt_rounded_bias");
 }
 
+namespace {
+
+// what both fp8 Linear entries check of one operand's ring and step
+int check_fp8_operand(const char* what, const void* t, const void* codes, const float* step, const float* maxima,
+                      const float* hist, int len, int idx, bool measure) {
+    if (!t || !codes || !step || !maxima) return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
+    if (!aligned16(t) || !aligned16(codes) || !aligned16(maxima))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
+    if (!measure && (!hist || len <= 0 || idx < 0 || idx >= len))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: a ring with idx in [0, n) is needed", what);
+    return ASTRAI_W8A8_OK;
+}
+
+int64_t whole256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// rows of dW's contraction: whole 128 of them, as the large products take it (dW of 4096 x 4096 weights, 1001 rows: 2502 us on
+// the general product, 41 padded). Below 128 rows the product of small tiles takes multiples of 16 as they are (64 rows:
+// 29 us, padded 34; 100 rows: 237, padded 34).
+int64_t contracted_rows(int64_t m) { return m < 128 && m % 16 == 0 ? m : (m + 127) / 128 * 128; }
+
+struct BackwardScratch {
+    int64_t g8, g8t, w8t, x8t, stats, maxima, steps, bytes;
+};
+BackwardScratch backward_scratch(int64_t m, int64_t n, int64_t k) {
+    const int64_t ldt = contracted_rows(m);
+    BackwardScratch s;
+    s.g8 = 0;
+    s.g8t = s.g8 + whole256(m * n);
+    s.w8t = s.g8t + whole256(n * ldt);
+    s.x8t = s.w8t + whole256(n * k);
+    s.stats = s.x8t + whole256(k * ldt);
+    s.maxima = s.stats + whole256(4 * (w8a8::kGradientMaxima + (m + 127) / 128 * n));
+    s.steps = s.maxima + 3 * 4 * w8a8::kAmaxPartials;
+    s.bytes = s.steps + 256;
+    return s;
+}
+
+}  // namespace
+
+int astrai_w8a8_linear_fp8_bf16(const void* x, void* x8, float* x_step, float* x_maxima, float* x_hist, int x_len, int x_idx,
+                                const void* w, void* w8, float* w_step, float* w_maxima, float* w_hist, int w_len, int w_idx,
+                                const void* bias, int round_first, void* out, int64_t m, int64_t n, int64_t k, int fmt,
+                                int measure, float fmax, float pow2_margin, void* stream) {
+    const char* what = "linear_fp8_bf16";
+    if (int rc = check_fp8_operand(what, x, x8, x_step, x_maxima, x_hist, x_len, x_idx, measure != 0)) return rc;
+    if (w) {
+        if (int rc = check_fp8_operand(what, w, w8, w_step, w_maxima, w_hist, w_len, w_idx, measure != 0)) return rc;
+    } else if (!w8 || !w_step) {
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
+    }
+    if (fmt != ASTRAI_W8A8_E4M3 && fmt != ASTRAI_W8A8_E5M2)
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmt must be 0 (e4m3) or 1 (e5m2)", what);
+    if (m <= 0 || n <= 0 || k <= 0) return fail(ASTRAI_W8A8_BAD_ARG, "%s: sizes must be positive", what);
+    if (!(fmax > 0.0f) || !(pow2_margin > 0.0f))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmax and pow2_margin must be positive", what);
+    if (int rc = check_gemm(what, x8, w8, out, m, n, k)) return rc;
+    auto s = static_cast<hipStream_t>(stream);
+    if (measure) {
+        w8a8::launch_amax_bf16(x, nullptr, x_maxima, m * k, s);
+        if (w) w8a8::launch_amax_bf16(w, nullptr, w_maxima, n * k, s);
+        w8a8::launch_quantize_fp8_measured(x, x8, {x_maxima, fmax, pow2_margin}, x_step, m * k, fmt, s);
+        if (w) w8a8::launch_quantize_fp8_measured(w, w8, {w_maxima, fmax, pow2_margin}, w_step, n * k, fmt, s);
+    } else {
+        w8a8::launch_quantize_fp8(x, x8, x_step, nullptr, x_maxima, m * k, fmt, s);
+        if (w) w8a8::launch_quantize_fp8(w, w8, w_step, nullptr, w_maxima, n * k, fmt, s);
+    }
+    const int rc = round_first && bias
+        ? astrai_w8a8_gemm_fp8_pt_rounded_bias(x8, w8, x_step, w_step, bias, out, m, n, k, fmt, stream)
+        : astrai_w8a8_gemm_fp8_pt(x8, w8, x_step, w_step, nullptr, bias, out, m, n, k, fmt, ASTRAI_W8A8_OUT_BF16, stream);
+    if (rc) return rc;
+    if (!measure && w)
+        w8a8::launch_amax_ring_push_pair({x_hist, x_len, x_idx, x_step, fmax, pow2_margin}, x_maxima,
+                                         {w_hist, w_len, w_idx, w_step, fmax, pow2_margin}, w_maxima, s);
+    else if (!measure)
+        w8a8::launch_amax_ring_push(x_hist, x_len, x_idx, nullptr, x_maxima, nullptr, x_step, fmax, pow2_margin, s);
+    return check_launch(what);
+}
+
+int64_t astrai_w8a8_linear_fp8_backward_scratch_bytes(int64_t m, int64_t n, int64_t k) {
+    return m > 0 && n > 0 && k > 0 ? backward_scratch(m, n, k).bytes : 0;
+}
+
+int astrai_w8a8_linear_fp8_backward_bf16(const void* g, const void* x, const void* w, const float* g_step, const float* x_step,
+                                         const float* w_step, void* scratch, void* grad_x, void* grad_w, void* grad_bias,
+                                         int64_t m, int64_t n, int64_t k, int fmt, float* g_hist, int g_len, int g_idx,
+                                         float fmax, float pow2_margin, void* stream) {
+    const char* what = "linear_fp8_backward_bf16";
+    if (!g || !x || !w || !scratch || !grad_x || !grad_w) return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
+    if (!aligned16(g) || !aligned16(x) || !aligned16(w) || !aligned16(scratch) || !aligned16(grad_x) || !aligned16(grad_w) ||
+        !aligned16(grad_bias))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
+    const bool measure = !g_hist;
+    if (!measure && (!g_step || !x_step || !w_step || g_len <= 0 || g_idx < 0 || g_idx >= g_len))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: steps and a ring with idx in [0, n) are needed", what);
+    if (fmt != ASTRAI_W8A8_E4M3 && fmt != ASTRAI_W8A8_E5M2)
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmt must be 0 (e4m3) or 1 (e5m2)", what);
+    if (m <= 0 || n <= 0 || k <= 0 || m > (int64_t)65535 * 128 || n > ((int64_t)1 << 31) - 64 || k > ((int64_t)1 << 31) - 64)
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: bad dims", what);
+    if (!(fmax > 0.0f) || !(pow2_margin > 0.0f))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmax and pow2_margin must be positive", what);
+    const BackwardScratch at = backward_scratch(m, n, k);
+    const int64_t ldt = contracted_rows(m);
+    auto* base = static_cast<uint8_t*>(scratch);
+    auto* stats = reinterpret_cast<float*>(base + at.stats);
+    auto* maxima = reinterpret_cast<float*>(base + at.maxima);
+    auto* steps = reinterpret_cast<float*>(base + at.steps);
+    float* colsums = grad_bias ? stats + w8a8::kGradientMaxima : nullptr;
+    auto s = static_cast<hipStream_t>(stream);
+    w8a8::MeasuredStep from[3];
+    const float *sg = g_step, *sx = x_step, *sw = w_step;
+    if (measure) {
+        const void* const t[3] = {g, x, w};
+        const int64_t size[3] = {m * n, m * k, n * k};
+        for (int i = 0; i < 3; ++i) {
+            from[i] = {maxima + i * w8a8::kAmaxPartials, fmax, pow2_margin};
+            w8a8::launch_amax_bf16(t[i], nullptr, maxima + i * w8a8::kAmaxPartials, size[i], s);
+        }
+        sg = steps, sx = steps + 1, sw = steps + 2;
+    }
+    // the gradient's maxima and column sums leave with its codes
+    w8a8::launch_quantize_transpose_fp8(g, base + at.g8, base + at.g8t, sg, nullptr, !measure || grad_bias ? stats : nullptr,
+                                        colsums, m, n, ldt, fmt, s, from[0]);
+    w8a8::launch_quantize_transpose_fp8(w, nullptr, base + at.w8t, sw, nullptr, nullptr, nullptr, n, k, n, fmt, s, from[2]);
+    if (int rc = astrai_w8a8_gemm_fp8_pt(base + at.g8, base + at.w8t, sg, sw, nullptr, nullptr, grad_x, m, k, n, fmt,
+                                         ASTRAI_W8A8_OUT_BF16, stream))
+        return rc;
+    w8a8::launch_quantize_transpose_fp8(x, nullptr, base + at.x8t, sx, nullptr, nullptr, nullptr, m, k, ldt, fmt, s, from[1]);
+    if (int rc = astrai_w8a8_gemm_fp8_pt(base + at.g8t, base + at.x8t, sg, sx, nullptr, nullptr, grad_w, n, k, ldt, fmt,
+                                         ASTRAI_W8A8_OUT_BF16, stream))
+        return rc;
+    w8a8::RingArgs ring;   // (last: the products read the step that it refreshes)
+    if (!measure) ring = {g_hist, g_len, g_idx, const_cast<float*>(g_step), fmax, pow2_margin};
+    w8a8::launch_gradient_stats(stats, nullptr, colsums, grad_bias, m, n, s, ring);
+    return check_launch(what);
+}
+
 int astrai_w8a8_gemm_fp8_ptpc(const void* a8, const void* b8, const float* sa, const float* sb,
                               const void* bias, void* out, int64_t m, int64_t n, int64_t k,
                               int fmt, void* stream) {

@@ -53,6 +53,14 @@ struct GemmArgs {
 constexpr int kAmaxPartials = 1024;
 void launch_quantize_fp8(const void* x, void* x8, const float* scale, float* amax, float* partials,
                          int64_t total, int fmt, hipStream_t stream);
+// The step max((max / fmax) / pow2_margin, 1e-12) of the maximum over kAmaxPartials maxima that another launch left, formed
+// by the quantizer itself and stored to *scale.
+struct MeasuredStep {
+    const float* maxima = nullptr;
+    float fmax = 1.0f, pow2_margin = 1.0f;
+};
+void launch_quantize_fp8_measured(const void* x, void* x8, const MeasuredStep& measured, float* scale, int64_t total, int fmt,
+                                  hipStream_t stream);
 // hist[idx] = fresh; *scale = max((max(hist) / fmax) / pow2_margin, 1e-12), with fresh = *amax or
 // the maximum of the kAmaxPartials partials (then also stored to *amax_out when that is given)
 void launch_amax_ring_push(float* hist, int n, int idx, const float* amax, const float* partials,
@@ -63,13 +71,21 @@ void launch_amax_bf16(const void* x, float* amax, float* partials, int64_t total
 // codes of a [rows, cols] matrix row-major (x8, may be null) and transposed (x8t, [cols, rows])
 void launch_quantize_transpose_fp8(const void* x, void* x8, void* x8t, const float* scale,
                                    float* amax, float* maxima, float* colsums, int64_t rows, int64_t cols,
-                                   int64_t ldt, int fmt, hipStream_t stream);
+                                   int64_t ldt, int fmt, hipStream_t stream, const MeasuredStep& measured = {});
 // workgroups of that launch, each of which writes one of `maxima`
 constexpr int kGradientMaxima = 2048;
 int quantize_transpose_blocks(int64_t rows, int64_t cols);
 // amax (or null) from the maxima, the bias gradient (or null) from the column sums of that launch
+// and a push of that maximum through a ring, if there is one
+struct RingArgs {
+    float* hist = nullptr;
+    int n = 0, idx = 0;
+    float* scale = nullptr;
+    float fmax = 1.0f, pow2_margin = 1.0f;
+};
+void launch_amax_ring_push_pair(const RingArgs& a, const float* pa, const RingArgs& b, const float* pb, hipStream_t stream);
 void launch_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows, int64_t cols,
-                           hipStream_t stream);
+                           hipStream_t stream, const RingArgs& ring = {});
 void launch_quantize_int8_rows(const void* x, void* xq, float* s, int64_t rows, int64_t k,
                                hipStream_t stream);
 // fused producers: (residual add +) RMSNorm + per-row int8; SwiGLU product + per-row

@@ -4,6 +4,8 @@
 // lane), the correctly rounded fp32 quotient by the step (the CPU kernel's arithmetic,
 // astrai/extension/ops/fp8.py:80; formed without a division sequence per element where the
 // step is shared, see quant8_fp8), hardware RNE conversion, 8-byte stores.
+#include <type_traits>
+
 #include "common.cuh"
 #include "launchers.h"
 #include "row_ops.cuh"
@@ -106,18 +108,41 @@ __device__ __forceinline__ void store_partial(float* partials, float local, floa
         for (int i = gridDim.x + threadIdx.x; i < kAmaxBlocks; i += kThreads) partials[i] = 0.0f;
 }
 
+// Where a quantizer's step comes from: *scale, or (MEASURED: dynamic scaling) it is that of the maximum over another
+// kernel's per-workgroup maxima, which every workgroup forms for itself (4 KB out of L2; a launch of its own in between
+// took 2.2 us and a gap) and the first one stores to *measured_scale.
+struct StepArgs {
+    float* measured_scale;
+    const float* maxima;   // kAmaxBlocks of them
+    float fmax, pow2_margin;
+};
+
+template <bool MEASURED>
+__device__ __forceinline__ float step_of(const float* __restrict__ scale, const StepArgs& a, float* slots) {
+    if constexpr (!MEASURED) {
+        return *scale;
+    } else {
+        static_assert(kAmaxBlocks == 4 * kThreads, "one load a thread");
+        const f32x4 v = *reinterpret_cast<const f32x4*>(a.maxima + threadIdx.x * 4);
+        const float peak = block_max(fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), 0.0f), slots);
+        const float step = fmaxf((peak / a.fmax) / a.pow2_margin, 1e-12f);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.measured_scale = step;
+        return step;
+    }
+}
+
 __device__ __forceinline__ void publish_early(float* amax, float local, float* slots) {
     const float m = block_max(local, slots);
     if (threadIdx.x == 0 && m > 0.0f)
         atomicMax(reinterpret_cast<unsigned int*>(amax), __float_as_uint(m));
 }
 
-template <int Fmt>
+template <int Fmt, bool MEASURED>
 __global__ __launch_bounds__(kThreads) void quantize_fp8_kernel(
-    const uint16_t* __restrict__ x, uint8_t* __restrict__ x8, const float* __restrict__ scale,
+    const uint16_t* __restrict__ x, uint8_t* __restrict__ x8, const float* __restrict__ scale, StepArgs from,
     float* __restrict__ amax, float* __restrict__ partials, int64_t total) {
     __shared__ float slots[kThreads / kWave];
-    const float step = *scale;
+    const float step = step_of<MEASURED>(scale, from, slots);
     float local = 0.0f;
     const int64_t nvec = total >> 3;
     const int64_t stride = (int64_t)gridDim.x * kThreads;
@@ -216,6 +241,19 @@ __global__ __launch_bounds__(kThreads) void amax_bf16_kernel(
 // (amax may be the ring's own slot: dynamic scaling is a ring of length one)
 // (partials: the fresh value is the maximum of a quantizer's kAmaxBlocks per-workgroup maxima
 // instead of *amax; amax_out, when given, receives it)
+__device__ __forceinline__ void ring_push_wave(float* hist, int n, int idx, float fresh, float* scale, float fmax,
+                                               float pow2_margin) {
+    const int lane = threadIdx.x & (kWave - 1);
+    float peak = 0.0f;
+    for (int i = lane; i < n; i += kWave) {
+        float h = hist[i];
+        if (i == idx) hist[i] = h = fresh;
+        peak = fmaxf(peak, h);
+    }
+    peak = wave_max(peak);
+    if (lane == 0) *scale = fmaxf((peak / fmax) / pow2_margin, 1e-12f);
+}
+
 __global__ __launch_bounds__(kWave) void amax_ring_push_kernel(
     float* hist, int n, int idx, const float* amax, const float* partials, float* amax_out,
     float* scale, float fmax, float pow2_margin) {
@@ -229,14 +267,7 @@ __global__ __launch_bounds__(kWave) void amax_ring_push_kernel(
     } else {
         fresh = *amax;
     }
-    float peak = 0.0f;
-    for (int i = threadIdx.x; i < n; i += kWave) {
-        float h = hist[i];
-        if (i == idx) hist[i] = h = fresh;
-        peak = fmaxf(peak, h);
-    }
-    peak = wave_max(peak);
-    if (threadIdx.x == 0) *scale = fmaxf((peak / fmax) / pow2_margin, 1e-12f);
+    ring_push_wave(hist, n, idx, fresh, scale, fmax, pow2_margin);
 }
 
 // ---- per-tensor fp8, row-major and transposed codes in one pass -----------
@@ -255,16 +286,16 @@ __global__ __launch_bounds__(kWave) void amax_ring_push_kernel(
 // launch (backward of 4096 x 4096 weights, 4096 tokens: 169 us, here 153).
 constexpr int kTrRows = 128, kTrCols = 128, kTrPitch = kTrRows + 4;
 
-template <int Fmt, bool STATS>
+template <int Fmt, bool STATS, bool MEASURED>
 __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
     const uint16_t* __restrict__ x, uint8_t* __restrict__ x8, uint8_t* __restrict__ x8t,
-    const float* __restrict__ scale, float* __restrict__ amax, float* __restrict__ colsums, int64_t rows,
+    const float* __restrict__ scale, StepArgs from, float* __restrict__ amax, float* __restrict__ colsums, int64_t rows,
     int64_t cols, int64_t ldt) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[kTrCols * kTrPitch];
     __shared__ float slots[kThreads / kWave];
     [[maybe_unused]] __shared__ float sums[STATS ? kThreads / kWave : 1][STATS ? kTrCols : 1];
     const int cc = threadIdx.x & 15, r4 = threadIdx.x >> 4;
-    const float step = *scale;
+    const float step = step_of<MEASURED>(scale, from, slots);
     const bool vec = (cols & 7) == 0;
     const bool runs = (ldt & 15) == 0;  // 16-byte pieces stay aligned and inside the matrix
     const int64_t tiles_x = (cols + kTrCols - 1) / kTrCols;
@@ -391,18 +422,20 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
 }
 
 // What the gradient's quantizer left: bias gradients from the column sums of `tiles` row tiles (64 columns to a
-// workgroup, four tiles at a time), the last workgroup takes the maximum over `nmax` workgroups' maxima.
+// workgroup, four tiles at a time), the last workgroup takes the maximum over `nmax` workgroups' maxima and pushes it
+// through the gradient's ring, if there is one.
 __global__ __launch_bounds__(kThreads) void gradient_stats_kernel(const float* __restrict__ maxima, int nmax,
                                                                   float* __restrict__ amax,
                                                                   const float* __restrict__ colsums, int64_t tiles,
-                                                                  uint16_t* __restrict__ bias, int64_t cols) {
+                                                                  uint16_t* __restrict__ bias, int64_t cols, RingArgs ring) {
     __shared__ float part[kThreads / kWave][kWave];
     __shared__ float slots[kThreads / kWave];
-    if (amax && blockIdx.x == gridDim.x - 1) {
+    if ((amax || ring.hist) && blockIdx.x == gridDim.x - 1) {
         float m = 0.0f;
         for (int i = threadIdx.x; i < nmax; i += kThreads) m = fmaxf(m, maxima[i]);
         m = block_max(m, slots);
-        if (threadIdx.x == 0) *amax = m;
+        if (amax && threadIdx.x == 0) *amax = m;
+        if (ring.hist && threadIdx.x < kWave) ring_push_wave(ring.hist, ring.n, ring.idx, m, ring.scale, ring.fmax, ring.pow2_margin);
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -923,8 +956,9 @@ __global__ __launch_bounds__(kThreads) void quantize_fp8_weight128_kernel(
 
 }  // namespace
 
-void launch_quantize_fp8(const void* x, void* x8, const float* scale, float* amax, float* partials,
-                         int64_t total, int fmt, hipStream_t stream) {
+template <bool MEASURED>
+static void launch_quantize_fp8_step(const void* x, void* x8, const float* scale, const StepArgs& from, float* amax,
+                                     float* partials, int64_t total, int fmt, hipStream_t stream) {
     if (total <= 0) return;
     const int64_t nvec = (total + 7) / 8;
     // two groups of kUnroll vectors per thread where the tensor is large enough
@@ -932,12 +966,33 @@ void launch_quantize_fp8(const void* x, void* x8, const float* scale, float* ama
     if (blocks > kAmaxBlocks) blocks = kAmaxBlocks;
     auto xs = static_cast<const uint16_t*>(x);
     auto xo = static_cast<uint8_t*>(x8);
-    if (fmt)
-        quantize_fp8_kernel<1><<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(
-            xs, xo, scale, amax, partials, total);
-    else
-        quantize_fp8_kernel<0><<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(
-            xs, xo, scale, amax, partials, total);
+    auto* const kern = fmt ? quantize_fp8_kernel<1, MEASURED> : quantize_fp8_kernel<0, MEASURED>;
+    kern<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(xs, xo, scale, from, amax, partials, total);
+}
+
+void launch_quantize_fp8(const void* x, void* x8, const float* scale, float* amax, float* partials,
+                         int64_t total, int fmt, hipStream_t stream) {
+    launch_quantize_fp8_step<false>(x, x8, scale, StepArgs{}, amax, partials, total, fmt, stream);
+}
+
+void launch_quantize_fp8_measured(const void* x, void* x8, const MeasuredStep& measured, float* scale, int64_t total, int fmt,
+                                  hipStream_t stream) {
+    launch_quantize_fp8_step<true>(x, x8, nullptr, StepArgs{scale, measured.maxima, measured.fmax, measured.pow2_margin},
+                                   nullptr, nullptr, total, fmt, stream);
+}
+
+// Two tensors' pushes side by side, a workgroup each.
+__global__ __launch_bounds__(kWave) void amax_ring_push_pair_kernel(RingArgs a, const float* pa, RingArgs b, const float* pb) {
+    const RingArgs r = blockIdx.x ? b : a;
+    const float* const partials = blockIdx.x ? pb : pa;
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kAmaxBlocks / kWave; ++i) m = fmaxf(m, partials[i * kWave + threadIdx.x]);
+    ring_push_wave(r.hist, r.n, r.idx, wave_max(m), r.scale, r.fmax, r.pow2_margin);
+}
+
+void launch_amax_ring_push_pair(const RingArgs& a, const float* pa, const RingArgs& b, const float* pb, hipStream_t stream) {
+    amax_ring_push_pair_kernel<<<dim3(2), dim3(kWave), 0, stream>>>(a, pa, b, pb);
 }
 
 void launch_amax_ring_push(float* hist, int n, int idx, const float* amax, const float* partials,
@@ -957,15 +1012,22 @@ void launch_amax_bf16(const void* x, float* amax, float* partials, int64_t total
 
 void launch_quantize_transpose_fp8(const void* x, void* x8, void* x8t, const float* scale,
                                    float* amax, float* maxima, float* colsums, int64_t rows, int64_t cols,
-                                   int64_t ldt, int fmt, hipStream_t stream) {
+                                   int64_t ldt, int fmt, hipStream_t stream, const MeasuredStep& measured) {
     if (rows <= 0 || cols <= 0) return;
+    const StepArgs from = {const_cast<float*>(scale), measured.maxima, measured.fmax, measured.pow2_margin};
     const dim3 grid((unsigned)quantize_transpose_blocks(rows, cols));
     auto* xi = static_cast<const uint16_t*>(x);
     auto* o = static_cast<uint8_t*>(x8);
     auto* ot = static_cast<uint8_t*>(x8t);
-    auto run = [&](auto kern, float* a) { kern<<<grid, dim3(kThreads), 0, stream>>>(xi, o, ot, scale, a, colsums, rows, cols, ldt); };
-    if (maxima) run(fmt ? quantize_transpose_fp8_kernel<1, true> : quantize_transpose_fp8_kernel<0, true>, maxima);
-    else run(fmt ? quantize_transpose_fp8_kernel<1, false> : quantize_transpose_fp8_kernel<0, false>, amax);
+    auto run = [&](auto stats, auto m) {
+        constexpr bool S = decltype(stats)::value, M = decltype(m)::value;
+        auto* const kern = fmt ? quantize_transpose_fp8_kernel<1, S, M> : quantize_transpose_fp8_kernel<0, S, M>;
+        kern<<<grid, dim3(kThreads), 0, stream>>>(xi, o, ot, scale, from, S ? maxima : amax, colsums, rows, cols, ldt);
+    };
+    if (maxima && measured.maxima) run(std::true_type{}, std::true_type{});
+    else if (maxima) run(std::true_type{}, std::false_type{});
+    else if (measured.maxima) run(std::false_type{}, std::true_type{});
+    else run(std::false_type{}, std::false_type{});
 }
 
 // a workgroup per tile while they are all resident at once (eight per compute unit)
@@ -975,12 +1037,12 @@ int quantize_transpose_blocks(int64_t rows, int64_t cols) {
 }
 
 void launch_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows, int64_t cols,
-                           hipStream_t stream) {
-    const int64_t blocks = (bias ? (cols + kWave - 1) / kWave : 0) + (amax ? 1 : 0);
+                           hipStream_t stream, const RingArgs& ring) {
+    const int64_t blocks = (bias ? (cols + kWave - 1) / kWave : 0) + (amax || ring.hist ? 1 : 0);
     if (rows <= 0 || cols <= 0 || blocks <= 0) return;
     gradient_stats_kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(
         maxima, quantize_transpose_blocks(rows, cols), amax, colsums, (rows + kTrRows - 1) / kTrRows,
-        static_cast<uint16_t*>(bias), cols);
+        static_cast<uint16_t*>(bias), cols, ring);
 }
 
 void launch_quantize_int8_rows(const void* x, void* xq, float* s, int64_t rows, int64_t k,

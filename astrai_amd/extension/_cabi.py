@@ -92,6 +92,11 @@ PROTOTYPES = {
     "astrai_w8a8_gemm_fp8_block128": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_linear_int8_bf16": ([_P] * 7 + [_I64] * 3 + [_P], _INT),
+    "astrai_w8a8_linear_fp8_bf16": (
+        ([_P] * 5 + [_INT] * 2) * 2 + [_P, _INT, _P] + [_I64] * 3 + [_INT] * 2 + [_F32] * 2 + [_P], _INT),
+    "astrai_w8a8_linear_fp8_backward_scratch_bytes": ([_I64] * 3, _I64),
+    "astrai_w8a8_linear_fp8_backward_bf16": (
+        [_P] * 10 + [_I64] * 3 + [_INT, _P, _INT, _INT, _F32, _F32, _P], _INT),
     "astrai_w8a8_gemv_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_tiled": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_rope_cache": (
@@ -381,6 +386,79 @@ def linear_forward_fp8(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
     w8, amax_w = quantize_bf16(w, sw, 0)
     out = mm_fp8(x8, w8, sx, sw, 0, None, bias if has_bias else None)
     return out.reshape(*x.shape[:-1], n), amax_x, amax_w
+
+
+def _plain_bf16(t: torch.Tensor, dev: torch.device) -> bool:
+    return t.dtype == torch.bfloat16 and t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def linear_fp8_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
+    """Whether :func:`linear_fp8` takes these: bf16 on one GPU as the kernels read them, ``K % 16 == 0``, nothing empty."""
+    k, dev = x.size(-1), x.device
+    return (x.is_cuda and k % 16 == 0 and x.numel() > 0 and w.numel() > 0 and _plain_bf16(x, dev) and _plain_bf16(w, dev)
+            and (bias is None or (bias.shape == (w.size(0),) and _plain_bf16(bias, dev))))
+
+
+def _ring(ring, ref: torch.Tensor):
+    """A ring's ``(address, length, index)``."""
+    if ring is None:
+        return None, 0, 0
+    hist, idx = ring
+    if not (hist.device == ref.device and hist.dtype == torch.float32 and hist.is_contiguous()):
+        raise RuntimeError("hist must be a contiguous float32 tensor on the input device")
+    return hist.data_ptr(), hist.numel(), idx
+
+
+def linear_fp8(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], codes: Optional[torch.Tensor],
+               steps, rings, fmt: int, fmax: float, pow2_margin: float) -> torch.Tensor:
+    """An fp8 Linear in one library call (:func:`linear_fp8_operands` said yes): ``x`` and, unless its ``codes`` are given,
+    ``w`` quantized, the product, the pushes. ``rings`` of x and w, ``(history, index)``: ``steps`` are used and then
+    refreshed (no ring of w with given codes). No ring of x: each step is measured, ``steps[1]`` that of given codes, and
+    the bias joins the product rounded to bf16."""
+    lib, dev = _require(), x.device
+    n, k = w.shape
+    m = x.numel() // k
+    measure = rings[0] is None
+    for step, name in zip(steps, ("sx", "sw")):
+        if step is not None:
+            _check_scale(step, x, name)
+    with _on_device(dev):
+        # maxima of x, of w; steps; codes of x; codes of w
+        steps_at, x_at = 2 * 4 * AMAX_PARTIALS, 2 * 4 * AMAX_PARTIALS + 256
+        w_at = x_at + -(-m * k // 256) * 256
+        scratch = torch.empty(w_at + (n * k if codes is None else 0), device=dev, dtype=torch.uint8)
+        out = torch.empty((*x.shape[:-1], n), device=dev, dtype=torch.bfloat16)
+        at = scratch.data_ptr()
+        _check(lib.astrai_w8a8_linear_fp8_bf16(
+            x.data_ptr(), at + x_at, at + steps_at if steps[0] is None else steps[0].data_ptr(), at, *_ring(rings[0], x),
+            w.data_ptr() if codes is None else None, at + w_at if codes is None else codes.data_ptr(),
+            at + steps_at + 4 if steps[1] is None else steps[1].data_ptr(), at + 4 * AMAX_PARTIALS, *_ring(rings[1], x),
+            _ptr(bias), measure, out.data_ptr(), m, n, k, fmt, measure, fmax, pow2_margin, _stream(x)), lib)
+    return out
+
+
+def linear_fp8_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, want_bias: bool, steps, ring, fmt: int,
+                        fmax: float, pow2_margin: float):
+    """Its input, weight and (or an empty tensor) bias gradient in one library call, the operands as
+    :func:`linear_fp8_operands` has them. ``ring`` ``(history, index)`` of the gradient, whose step is refreshed behind the
+    products; without one each step is measured."""
+    lib, dev = _require(), g.device
+    n, k = w.shape
+    m = x.numel() // k
+    if steps is None:
+        steps = (None, None, None)
+    for step, name in zip(steps, ("sg", "sx", "sw")):
+        if step is not None:
+            _check_scale(step, g, name)
+    with _on_device(dev):
+        scratch = torch.empty(lib.astrai_w8a8_linear_fp8_backward_scratch_bytes(m, n, k), device=dev, dtype=torch.uint8)
+        gx, gw = torch.empty_like(x), torch.empty_like(w)
+        gb = torch.empty(n if want_bias else 0, device=dev, dtype=g.dtype)
+        _check(lib.astrai_w8a8_linear_fp8_backward_bf16(
+            g.data_ptr(), x.data_ptr(), w.data_ptr(), *(_ptr(t) for t in steps), scratch.data_ptr(), gx.data_ptr(),
+            gw.data_ptr(), gb.data_ptr() if want_bias else None, m, n, k, fmt, *_ring(ring, g), fmax, pow2_margin, _stream(g)),
+            lib)
+    return gx, gw, gb
 
 
 def fp8_mm(a: torch.Tensor, b: torch.Tensor, sx: torch.Tensor, sw: torch.Tensor) -> torch.Tensor:

@@ -33,7 +33,10 @@ from astrai_amd.extension.ops.fp8 import (
     amax_ring_push,
     amax_ring_push_partials,
     linear_backward_fp8,
+    linear_backward_fp8_kernels,
     linear_forward_fp8,
+    linear_fp8_kernels,
+    linear_fp8_takes,
     mm_fp8,
     mm_fp8_bias,
     mm_fp8_rounded_bias,
@@ -128,6 +131,10 @@ class _AmaxRing:
                                 float(2 ** recipe.margin))
         self.idx = (self.idx + 1) % self.hist.numel()
 
+    def advance(self) -> None:
+        """A kernel has pushed into slot ``idx``."""
+        self.idx = (self.idx + 1) % self.hist.numel()
+
     def push(self, amax: torch.Tensor, recipe: FP8Recipe, fmt: str) -> None:
         # record first, then refresh: the step used next reflects amax seen so far
         if self.hist.is_cuda and type(recipe) in (DelayedScaling, DynamicScaling) \
@@ -203,6 +210,14 @@ class FP8TensorMeta:
         """True when every slot of the weight ring holds the amax of ``w`` as it is
         now, so that one more push would change neither the ring nor the step."""
         return self._same_weight(w) and self.w_repeats >= self.recipe.history_len
+
+    def settled_codes(self, w: torch.Tensor) -> torch.Tensor:
+        """The codes of a settled weight, made once."""
+        hit = self.w_cached
+        if hit is None or hit[0]() is not w or hit[1] != w._version:
+            w8, amax_w = quantize_bf16(w, self.w_scale, "e4m3")
+            hit = self.w_cached = (weakref.ref(w), w._version, w8, amax_w)
+        return hit[2]
 
     def note_w_push(self, w: torch.Tensor) -> None:
         self.w_cached = None  # the step may have moved with this push
@@ -337,6 +352,32 @@ def _dynamic_scale(t: torch.Tensor, recipe: FP8Recipe, fmt: str) -> torch.Tensor
     return recipe.scale_from_history(amax, fmt)
 
 
+def _forward_in_one_call(st: FP8State, meta: FP8TensorMeta, x, w, bias, fmt: str) -> Optional[torch.Tensor]:
+    """:func:`fp8_linear_forward` as one library call, with the same arithmetic and bookkeeping. ``None`` where the general
+    path is asked for: other recipes, operands that are not as the kernels read them."""
+    if not linear_fp8_takes(x, w, bias):
+        return None
+    if isinstance(st.recipe, DynamicScaling):
+        if type(st.recipe) is not DynamicScaling:
+            return None
+        sw, codes = st.dynamic_weight(w, fmt) if st.caches_weight(w) else (None, None)
+        return linear_fp8_kernels(x, w, bias, codes, (None, sw), (None, None), fmt, FP8_MAX[fmt], st.recipe.margin)
+    if not (meta._x.takes_partials(meta.recipe) and meta._w.takes_partials(meta.recipe)):
+        return None
+    if not meta.x_init:
+        meta.init_x(x, fmt)
+    codes, ring_w = None, (meta.w_hist, meta.w_idx)
+    if st.caches_weight(w) and meta.w_settled(w):
+        codes, ring_w = meta.settled_codes(w), None
+    out = linear_fp8_kernels(x, w, bias, codes, (meta.x_scale, meta.w_scale), ((meta.x_hist, meta.x_idx), ring_w), "e4m3",
+                             FP8_MAX[fmt], meta.recipe.margin)
+    meta._x.advance()
+    if codes is None:
+        meta._w.advance()
+        meta.note_w_push(w)
+    return out
+
+
 def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_product: bool = False):
     """Scaled fp8 linear forward (fp8.py:275-305).
 
@@ -350,6 +391,10 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_prod
     meta = st.get_weight_meta(w)
     if not meta.w_init:
         meta.init_w(w, fmt)
+    if bias_in_product:
+        out = _forward_in_one_call(st, meta, x, w, bias if bias is not None and bias.numel() else None, fmt)
+        if out is not None:
+            return out
     if isinstance(st.recipe, DynamicScaling):
         x2 = x.reshape(-1, w.size(1))
         sx = _dynamic_scale(x2, st.recipe, fmt)
@@ -373,20 +418,17 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_prod
         # The weight ring already holds this weight's amax in every slot: pushing it
         # again would leave ring and step as they are, so codes made with that step
         # stay valid until the weight is written to.
-        hit = meta.w_cached
-        if hit is None or hit[0]() is not w or hit[1] != w._version:
-            w8, amax_w = quantize_bf16(w, meta.w_scale, "e4m3")
-            meta.w_cached = (weakref.ref(w), w._version, w8, amax_w)
+        w8 = meta.settled_codes(w)
         x2 = x.reshape(-1, w.size(1))
         has_bias = bias is not None and bias.numel() > 0
         if meta._x.takes_partials(meta.recipe) and x2.numel():
             x8 = quantize_bf16_partials(x2, meta.x_scale, "e4m3", meta._x.partials)
-            out = mm_fp8_bias(x8, meta.w_cached[2], meta.x_scale, meta.w_scale,
+            out = mm_fp8_bias(x8, w8, meta.x_scale, meta.w_scale,
                               bias if has_bias else None).reshape(*x.shape[:-1], w.size(0))
             meta._x.push_partials(meta.recipe, fmt)
             return out
         x8, amax_x = quantize_bf16(x2, meta.x_scale, "e4m3")
-        out = mm_fp8_bias(x8, meta.w_cached[2], meta.x_scale, meta.w_scale,
+        out = mm_fp8_bias(x8, w8, meta.x_scale, meta.w_scale,
                           bias if has_bias else None).reshape(*x.shape[:-1], w.size(0))
         meta.update_x(amax_x, fmt)
         return out
@@ -411,6 +453,26 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_prod
     return out
 
 
+def _backward_in_one_call(st: FP8State, meta: FP8TensorMeta, g, x, w, masks, fmt: str, dynamic: bool):
+    """:func:`fp8_linear_backward` as one library call; ``None`` as for the forward."""
+    if not (masks[0] and masks[1] and linear_fp8_takes(x, w, None) and linear_fp8_takes(g, w, None)
+            and g.size(-1) == w.size(0) and x.size(-1) == w.size(1)
+            and x.numel() // w.size(1) == g.numel() // w.size(0) <= 65535 * 128):
+        return None
+    if dynamic:
+        if type(st.recipe) is not DynamicScaling:
+            return None
+        return linear_backward_fp8_kernels(g, x, w, masks[2], None, None, fmt, FP8_MAX[fmt], st.recipe.margin)
+    if not meta._g.takes_partials(meta.recipe):
+        return None
+    if not meta.g_init:
+        meta.init_g(g, fmt)
+    grads = linear_backward_fp8_kernels(g, x, w, masks[2], (meta.g_scale, meta.x_scale, meta.w_scale),
+                                        (meta.g_hist, meta.g_idx), fmt, FP8_MAX[fmt], meta.recipe.margin)
+    meta._g.advance()
+    return grads
+
+
 def fp8_linear_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, masks):
     """Scaled fp8 linear backward (fp8.py:308-330): gradient quantized once in the
     backward format, dX and dW GEMMs share it."""
@@ -418,6 +480,9 @@ def fp8_linear_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, masks
     fmt = st.fp8_format.bwd()
     meta = st.get_weight_meta(w)
     dynamic = isinstance(st.recipe, DynamicScaling)
+    grads = _backward_in_one_call(st, meta, g, x, w, masks, fmt, dynamic)
+    if grads is not None:
+        return grads
     if dynamic:
         sg = _dynamic_scale(g, st.recipe, fmt)
         sw = _dynamic_scale(w, st.recipe, fmt)

@@ -27,6 +27,9 @@ def _fp8_mm_module() -> SimpleNamespace:
         quantize_bf16=_cabi.quantize_bf16,
         mm_fp8=_cabi.mm_fp8,
         linear_forward_fp8=_cabi.linear_forward_fp8,
+        linear_fp8=_cabi.linear_fp8,
+        linear_fp8_operands=_cabi.linear_fp8_operands,
+        linear_fp8_backward=_cabi.linear_fp8_backward,
         linear_backward_fp8=_cabi.linear_backward_fp8,
         mm_fp8_acc=_cabi.mm_fp8_acc,
         quantize_transpose_bf16=_cabi.quantize_transpose_bf16,

@@ -590,6 +590,33 @@ int astrai_w8a8_linear_int8_bf16(const void* x_bf16, const void* wq, const float
                                  void* stream);
 
 /*
+ * An fp8 Linear over bf16 rows in one call: x [m, k] is quantized into x8 (and w [n, k] into w8 unless w is NULL and w8,
+ * w_step are given), then out [m, n] bf16 = x8 w8^T * x_step * w_step with the optional bias, which joins the product
+ * rounded to bf16 if round_first.
+ *   measure != 0  a step is max((max |t| / fmax) / pow2_margin, 1e-12) of this tensor, stored to *x_step (*w_step);
+ *                 the rings are unused
+ *   measure == 0  the steps are used as they are; then the maxima are pushed through the rings (amax_ring_push), which
+ *                 refreshes them
+ *   x_maxima, w_maxima: scratch of ASTRAI_W8A8_AMAX_PARTIALS floats each
+ */
+int astrai_w8a8_linear_fp8_bf16(const void* x_bf16, void* x8, float* x_step, float* x_maxima, float* x_hist, int x_len,
+                                int x_idx, const void* w_bf16, void* w8, float* w_step, float* w_maxima, float* w_hist,
+                                int w_len, int w_idx, const void* bias_bf16, int round_first, void* out_bf16, int64_t m,
+                                int64_t n, int64_t k, int fmt, int measure, float fmax, float pow2_margin, void* stream);
+
+/*
+ * Its backward: grad_x [m, k] = g w, grad_w [n, k] = g^T x from codes of all three, grad_bias [n] (or NULL) the column sums
+ * of g. With g_hist the steps are used as they are and max |g| is pushed through that ring afterwards, which refreshes
+ * *g_step; without, each step is measured (as above). scratch: astrai_w8a8_linear_fp8_backward_scratch_bytes(m, n, k),
+ * 16-byte aligned.
+ */
+int64_t astrai_w8a8_linear_fp8_backward_scratch_bytes(int64_t m, int64_t n, int64_t k);
+int astrai_w8a8_linear_fp8_backward_bf16(const void* g_bf16, const void* x_bf16, const void* w_bf16, const float* g_step,
+                                         const float* x_step, const float* w_step, void* scratch, void* grad_x_bf16,
+                                         void* grad_w_bf16, void* grad_bias_bf16, int64_t m, int64_t n, int64_t k, int fmt,
+                                         float* g_hist, int g_len, int g_idx, float fmax, float pow2_margin, void* stream);
+
+/*
  * The decode int8 kernels on their own: same contract as
  * astrai_w8a8_gemm_int8_ptpc but requires M <= 128 and K % 256 == 0, and
  * returns ASTRAI_W8A8_UNSUPPORTED otherwise.

@@ -1,0 +1,102 @@
+"""The fp8 policy's forward and backward as one library call each against its general path: the same outputs, gradients,
+histories and steps, bit for bit."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from astrai_amd.extension import fp8
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(autouse=True)
+def fresh():
+    fp8.fp8_state().reset()
+    yield
+    fp8.fp8_state().reset()
+
+
+def _mk(seed, *size, std=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*size, generator=g, device=DEV) * std).bfloat16()
+
+
+def _steps(monkeypatch, general, recipe, shape, n, bias, grads, fmt, cache):
+    calls = []
+    take = fp8.linear_fp8_takes
+    monkeypatch.setattr(fp8, "linear_fp8_takes", lambda *a: not general and (calls.append(take(*a)) or calls[-1]))
+    fp8.fp8_state().reset()
+    k = shape[-1]
+    w, b = _mk(1, n, k, std=0.02), _mk(2, n) if bias else None
+    if grads:
+        w.requires_grad_(True)
+    out = []
+    with fp8.fp8_autocast(True, recipe=recipe(), fp8_format=fmt):
+        fp8.fp8_cache_weights(cache)
+        for t in range(4):
+            x = _mk(10 + t, *shape, std=1.0 + t).requires_grad_(grads)
+            with torch.set_grad_enabled(grads):
+                y = F.linear(x, w, b)
+            out.append(y.detach())
+            if grads:
+                out += torch.autograd.grad(y, [x, w], _mk(20 + t, *y.shape, std=0.01))
+        meta = fp8.fp8_state().peek_weight_meta(w)
+        out += [r for ring in (meta._x, meta._w, meta._g) for r in (ring.hist, ring.scale, torch.tensor(ring.idx))]
+    monkeypatch.setattr(fp8, "linear_fp8_takes", take)
+    return out, calls
+
+
+@pytest.mark.parametrize("recipe", [lambda: fp8.DelayedScaling(history_len=3, margin=1), fp8.DynamicScaling])
+@pytest.mark.parametrize("shape,n,bias", [((1, 256), 256, False), ((3, 5, 512), 512, True), ((100, 272), 272, True),
+                                          ((1037, 1024), 1024, False), ((64, 64, 256), 264, True)])
+@pytest.mark.parametrize("grads,fmt,cache", [(False, "hybrid", None), (False, "e5m2", False), (True, "hybrid", None),
+                                             (True, "e4m3", True)])
+def test_same_as_the_general_path(monkeypatch, recipe, shape, n, bias, grads, fmt, cache):
+    got, calls = _steps(monkeypatch, False, recipe, shape, n, bias, grads, fmt, cache)
+    want, none = _steps(monkeypatch, True, recipe, shape, n, bias, grads, fmt, cache)
+    assert all(calls) and calls and not none
+    for a, b in zip(got, want, strict=True):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_operands_that_are_left_to_the_general_path():
+    from astrai_amd.extension.ops.fp8 import linear_fp8_takes
+    x, w = _mk(1, 8, 256), _mk(2, 64, 256)
+    assert linear_fp8_takes(x, w, None) and linear_fp8_takes(x, w, _mk(3, 64))
+    for bad in (_mk(1, 8, 512)[:, ::2], _mk(1, 256, 8).t(), x.float(), x.cpu(), _mk(1, 0, 256), _mk(1, 9 * 256)[1:2049].reshape(8, 256)):
+        assert not linear_fp8_takes(bad, w, None)
+    assert not linear_fp8_takes(_mk(1, 8, 250), _mk(2, 64, 250), None)
+    for bad in (_mk(3, 64).float(), _mk(3, 1, 64), _mk(3, 128)[::2]):
+        assert not linear_fp8_takes(x, w, bad)
+
+
+def test_infinities_and_nan_reach_the_step_alike(monkeypatch):
+    """A maximum passes NaN by and keeps an infinity, on both paths."""
+    for value in (float("inf"), float("nan")):
+        outs = []
+        for general in (False, True):
+            fp8.fp8_state().reset()
+            take = fp8.linear_fp8_takes
+            monkeypatch.setattr(fp8, "linear_fp8_takes", lambda *a: not general and take(*a))
+            x, w = _mk(1, 40, 256), _mk(2, 64, 256)
+            x[3, 7] = value
+            with torch.no_grad(), fp8.fp8_autocast(True, recipe=fp8.DynamicScaling()):
+                outs.append(F.linear(x, w))
+            monkeypatch.setattr(fp8, "linear_fp8_takes", take)
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+def test_replayed_in_a_graph():
+    x, w = _mk(1, 40, 256), _mk(2, 64, 256)
+    with torch.no_grad(), fp8.fp8_autocast(True, recipe=fp8.DynamicScaling()):
+        F.linear(x, w)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = F.linear(x, w)
+        for t in range(4):
+            x.copy_(_mk(30 + t, 40, 256, std=1.0 + t))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, F.linear(x, w))
