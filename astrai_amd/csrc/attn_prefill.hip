@@ -25,30 +25,31 @@
 //   keys and values sit in LDS as rows of 16-byte chunks XOR-swizzled by row so that the 16 rows
 //     a key operand read touches, and the 4 rows a transposing read touches, fall into
 //     different banks.
-// A wave's instruction stream is a software pipeline over tiles, written out and
-// pinned with sched_barrier: the score MFMAs of tile T+1 are interleaved with
-// the exponentials of tile T, and the P.V MFMAs of tile T with the masking and
-// row maximum of tile T+1, so the matrix pipe and the vector ALU work at the same
-// time inside one wave (a wave issues in order: a softmax phase between two MFMA
-// phases leaves each unit idle while the other runs). Keys and values arrive by
-// direct-to-LDS loads, keys into a ring of four tiles, values into two 64-key buffers,
-// both one 64-key block ahead; one workgroup barrier per block; no staging registers. Tiles that every
-// query of the wave sees whole skip the masking code; the accumulators are rescaled
-// only when a row maximum has outgrown the reference maximum by 2^8.
+// A wave's instruction stream is a software pipeline over tiles, written out and pinned with sched_barrier: a step issues
+// the score MFMAs of tile T+1 and the P.V MFMAs of tile T-1 with the exponentials of tile T spread evenly behind all
+// of them, an element behind each. A 32x32x16 MFMA leaves the vector ALU 24 of its 32 cycles (4 for most instructions, 8
+// for an exponential); what exceeds that in one slot delays the next MFMA and what is left unused in another is lost: 16
+// slots of 20 cycles take 536, eight of 44 and eight empty ones 640. Row maxima of tile T+1 go behind the last MFMAs,
+// the question whether one has outgrown its reference into the next step. Keys and values arrive by direct-to-LDS
+// loads into two rings of four tiles, values two tiles behind the keys, one 64-key block ahead, one load to every second
+// MFMA of a block's first step (all at once they stall the waves that issue them); one workgroup barrier per block; no
+// staging registers. Dense loads keep their lane's offset, the descriptors move along instead; the loop over unmasked
+// blocks goes once round the rings, so that its LDS offsets are constants. Tiles that every query of the wave sees whole
+// skip the masking code; the accumulators are rescaled only when a row maximum has outgrown the reference maximum by 2^8.
 //
 // The direct-to-LDS loads are written in assembly (they have no output register): behind the
 // builtin the compiler orders every transposing read after all loads in flight (s_waitcnt vmcnt(0)),
 // which puts a whole memory round trip into each 64-key block. The blocks without and with masking
 // are two loops, not two branches of one: at a join of the two the compiler moved all accumulators
 // from one register set to another on every block.
-// What bounds it: vector ALU and matrix pipe of a SIMD share its issue slots (16 exponentials and ~65 other vector
-// instructions per lane beside 16 MFMAs of 32 cycles a tile, two waves per SIMD). Counters: 4 x 2048 tokens, 16/4 heads x
-// 128: matrix pipe busy 48% of the SIMD cycles, vector ALU 53%; ragged, 32/8 heads x 64 with P in two terms: 37% and 72%.
-// Measured (graph replays, before -> after the two points above, the backward walk and reading strided tensors in place):
-// 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 148 -> 80 us (860 TFLOP/s; before it
-// went through the paged form), ragged 16 x 175..700 tokens of 32/8 heads x 64 in a pool 173 -> 77 us
-// (450 TFLOP/s, P in two terms; before on the general kernel). 186 / 133 registers where the joined
-// loops took 256 with spills: two / three workgroups per CU.
+// What bounds it: 53 vector instructions, 16 exponentials, 16 MFMAs and 24 LDS reads a tile and wave; a tile takes 890
+// cycles alone on a SIMD, 790 with two waves (512 are the MFMAs'; operand reads 190, the branch and the barrier 100),
+// under a clock that the power limit holds at 1.7 GHz for long sequences (2.1 for short ones).
+// Measured (graph replays): 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 75 us (915 TFLOP/s), ragged
+// 16 x 175..700 tokens of 32/8 heads x 64 in a pool 75.7 us (P in two terms); with the exponentials behind the score
+// MFMAs alone, the loads in a burst and offsets formed for each (120 vector instructions a tile) 80.3 and 78.2. Up to 236 /
+// 170 registers: two / three workgroups per CU. 64 query tokens a workgroup halve the loads, but couple eight waves:
+// 4 x 2048 72.3 us (75.5 here, same run), 1 x 4096 92.8 (76.4), 32 x 512 64.5 (57.9); not kept.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -90,15 +91,14 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     constexpr int QB = 32 * QSUB;                 // query tokens per workgroup
     constexpr int ROW = 2 * D;                    // bytes per key or value row in LDS
     constexpr int TILE = 32 * ROW;                // one 32-key tile
-    constexpr int RING = 4 * TILE;                // keys
-    constexpr int VBUF = kKB * ROW;               // 64 value rows
+    constexpr int RING = 4 * TILE;                // keys; as much again for values
     constexpr int LPR = ROW / 16;                 // 16-byte chunks (lanes of a load) per row
     constexpr int RPI = 64 / LPR;                 // rows per 1 KiB load
     constexpr int DMA = kKB / RPI / WAVES;        // loads per wave, tensor and block
     constexpr int KS = D / 16;                    // score MFMAs per tile
     constexpr int DT = D / 32;                    // 32-dim output tiles
     static_assert(DMA >= 1 && (!PAGED || QB <= 64), "shape");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[RING + 2 * VBUF];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * RING];
     const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane(
         (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
 
@@ -204,21 +204,31 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     const uint16_t* vc = static_cast<const uint16_t*>(a.v_cache) +
                          (PAGED ? (int64_t)hk * D : b_dense * a.v_stride.batch + hk * a.v_stride.head);
     const uint32_t pool_bytes = PAGED ? (uint32_t)(a.num_slots * k_row - hk * ROW) : 0u;
-    const u32x4 rk = make_desc(kc, PAGED ? pool_bytes : (uint32_t)(a.max_len - 1) * k_row + ROW);
+    u32x4 rk = make_desc(kc, PAGED ? pool_bytes : (uint32_t)(a.max_len - 1) * k_row + ROW);
     // Paged: one load per wave fetches the slots of all rows its next loads cover (lane l <
     // RPW: this wave's l-th key row; the next RPW lanes: its value rows); the loads take each
     // row's slot from the lane that holds it. Looked up one block ahead, so that the table
     // access is not a second memory round trip in front of every load.
     constexpr int RPW = RPI * DMA;  // rows of a 64-row block that this wave loads
-    auto lookup = [&](int t0, int kbv) -> int {
+    auto lookup = [&](int t0, int v0) -> int {  // first key tile, first value tile (-1: before the first key)
         const int l = lane & (2 * RPW - 1);  // (lanes past 2 RPW repeat the pattern, unused)
-        const int key = l < RPW ? t0 * 32 + wave * RPW + l : kbv * kKB + wave * RPW + (l - RPW);
-        int slot = (key <= kmax) ? table[key] : -1;
-        return slot < a.num_slots ? slot : -1;
+        const int key = l < RPW ? t0 * 32 + wave * RPW + l : v0 * 32 + wave * RPW + (l - RPW);
+        const int slot = (key >= 0 && key <= kmax) ? table[key] : -1;
+        return slot;
     };
-    auto paged_off = [&](int slots, int src_lane, int swz) -> uint32_t {
-        const int slot = __builtin_amdgcn_ds_bpermute(src_lane << 2, slots);
-        return slot >= 0 ? (uint32_t)slot * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz) << 4) : kMissing;
+    // the rows' offsets in the lanes that looked them up (kMissing: chunk offsets added to it stay past the pool)
+    auto rows_of = [&](int slot) -> uint32_t {
+        return slot >= 0 && slot < a.num_slots ? (uint32_t)slot * k_row : kMissing;
+    };
+    auto paged_off = [&](uint32_t rows, int src_lane, int swz) -> uint32_t {
+        return (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane << 2, (int)rows) + (uint32_t)(((lane & (LPR - 1)) ^ swz) << 4);
+    };
+    // Dense: the descriptors move along with the keys, so that a load's offset is a constant of its lane
+    auto advance = [](u32x4& desc, uint64_t bytes) {
+        const uint64_t addr = (((uint64_t)desc.y << 32) | desc.x) + bytes;
+        desc.x = (uint32_t)addr;
+        desc.y = (uint32_t)(addr >> 32);
+        desc.z = desc.z > bytes ? desc.z - (uint32_t)bytes : 0u;
     };
     [[maybe_unused]] uint32_t k_voff[DMA];
     if constexpr (!PAGED) {
@@ -228,25 +238,32 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             k_voff[j] = (uint32_t)row * k_row + (uint32_t)(((lane & (LPR - 1)) ^ swz_k(row)) << 4);
         }
     }
-    // tiles t0 and t0+1 (64 keys) into their ring slots
-    auto dma_k = [&](int t0, [[maybe_unused]] int slots) {
+    // tiles t0 and t0+1 (64 keys) into their ring slots: where in memory, and one load of them
+    constexpr int TI = 32 / RPI;  // loads per tile
+    auto k_off = [&](int j, [[maybe_unused]] uint32_t rows) -> uint32_t {
+        const int inst = wave * DMA + j;  // 64 / RPI loads; half of them per tile
+        return PAGED ? paged_off(rows, j * RPI + lane / LPR, swz_k(inst * RPI + lane / LPR)) : k_voff[j];
+    };
+    auto dma_k = [&](int j, int t0, uint32_t off) {
+        const int inst = wave * DMA + j;
+        lds_dma16<false>(rk, lds0 + ((t0 + inst / TI) & 3) * TILE + (inst % TI) * 1024, off);
+    };
+    auto dma_k_all = [&](int t0, uint32_t rows) {
 #pragma unroll
-        for (int j = 0; j < DMA; ++j) {
-            const int inst = wave * DMA + j;  // 64 / RPI instructions; half of them per tile
-            const uint32_t off = PAGED ? paged_off(slots, j * RPI + lane / LPR, swz_k(inst * RPI + lane / LPR))
-                                       : k_voff[j] + (uint32_t)(t0 * 32) * k_row;
-            const int tile_inst = 32 / RPI;
-            lds_dma16<false>(rk, lds0 + ((t0 + inst / tile_inst) & 3) * TILE + (inst % tile_inst) * 1024, off);
-        }
+        for (int j = 0; j < DMA; ++j) dma_k(j, t0, k_off(j, rows));
     };
     [[maybe_unused]] int slots = 0;
     if constexpr (PAGED) {
-        dma_k(0, lookup(0, 0));
-        slots = lookup(1, 0);  // tiles 1, 2 and value block 0
+        const int first = lookup(0, 0);
+        slots = lookup(1, -1);  // key tiles 1, 2 and value tiles -1, 0
+        dma_k_all(0, rows_of(first));
+        dma_k_all(1, rows_of(slots));
     } else {
-        dma_k(0, 0);
+        dma_k_all(0, 0);
+        advance(rk, (uint64_t)k_row * 32);
+        dma_k_all(1, 0);
+        advance(rk, (uint64_t)k_row * 64);  // the first block's: tiles 3, 4
     }
-    dma_k(1, slots);
 
     if constexpr (!PAGED) {
         if (a.positions) {
@@ -277,10 +294,10 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     const int nkb = kmax / kKB + 1;     // (kmax = -1, an empty sequence: one block of masked keys)
     const int tiles_w = kmax_w / 32 + 1;  // tiles this wave computes
 
-    // values: the same way into a 64-row buffer. Rows past kmax arrive as zeros, so a stale cache
-    // row can never meet a zero probability as 0 * NaN. (With far strides those rows' offsets pass 32 bits: they
-    // must not come round to a place inside. Keys may: their scores are replaced.)
-    const u32x4 rv = make_desc(vc, PAGED ? pool_bytes : kmax >= 0 ? (uint32_t)kmax * v_row + ROW : 0u);
+    // values: the same way into a ring of their own, two tiles behind the keys. Rows past kmax arrive as zeros, so a
+    // stale cache row can never meet a zero probability as 0 * NaN. (With far strides those rows' offsets pass 32
+    // bits: they must not come round to a place inside. Keys may: their scores are replaced.)
+    u32x4 rv = make_desc(vc, PAGED ? pool_bytes : kmax >= 0 ? (uint32_t)kmax * v_row + ROW : 0u);
     [[maybe_unused]] uint32_t v_voff[DMA];
     if constexpr (!PAGED) {
 #pragma unroll
@@ -289,14 +306,13 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             v_voff[j] = (uint32_t)min((uint64_t)row * v_row + (((lane & (LPR - 1)) ^ swz_v(row)) << 4), (uint64_t)kMissing);
         }
     }
-    auto dma_v = [&](int kb, [[maybe_unused]] int slots) {
-#pragma unroll
-        for (int j = 0; j < DMA; ++j) {
-            const int inst = wave * DMA + j;
-            const uint32_t off = PAGED ? paged_off(slots, RPW + j * RPI + lane / LPR, swz_v(inst * RPI + lane / LPR))
-                                       : min(__builtin_elementwise_add_sat(v_voff[j], (uint32_t)(kb * kKB) * v_row), kMissing);
-            lds_dma16<false>(rv, lds0 + RING + (kb & 1) * VBUF + inst * 1024, off);
-        }
+    auto v_off = [&](int j, [[maybe_unused]] uint32_t rows) -> uint32_t {
+        const int inst = wave * DMA + j;
+        return PAGED ? paged_off(rows, RPW + j * RPI + lane / LPR, swz_v(inst * RPI + lane / LPR)) : v_voff[j];
+    };
+    auto dma_v = [&](int j, int t0, uint32_t off) {
+        const int inst = wave * DMA + j;
+        lds_dma16<false>(rv, lds0 + RING + ((t0 + inst / TI) & 3) * TILE + (inst % TI) * 1024, off);
     };
 
     f32x16 o[DT];
@@ -313,7 +329,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     // the stand-in itself, a row whose first tiles are hidden took it for a maximum, and the rounding of c times it
     // for a probability, infinite at every other scale.
     const float c = a.scale * 1.44269504088896340736f;  // scores to log2 units
-    float m_run = 0.5f * kNegBig * fminf(c, 1.0f), l_run = 0.0f;
+    float m_run = 0.5f * kNegBig * fminf(c, 1.0f), l_run = 0.0f, m_lim = m_run + kSlack;
     const f32x16 zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f,
                            0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     // V^T operand of 32 dims x 16 keys: two transposing reads. In each 16-lane group, lane
@@ -330,14 +346,14 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     // whole byte offset: one address register per tile instead of one per k-step.
     const int k_lane0 = qi * ROW + ((h ^ swz_k(qi)) << 4);
     auto k_frag = [&](int tile_off, int ks) -> u32x4 {
-        return *reinterpret_cast<const u32x4*>(lds + ((tile_off + k_lane0) ^ (ks << 5)));
+        return *reinterpret_cast<const u32x4*>(lds + tile_off + (k_lane0 ^ (ks << 5)));
     };
     // T0: first key of the tile; PARTIAL with several token groups per workgroup: rows past this
     // wave's newest key are other queries' keys and are replaced by zeros (their probabilities here
     // are zero, and 0 * NaN would not be)
     auto v_frag = [&](auto mask_tag, int T0, int vt_off, int t, int dt) -> u32x4 {
         typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-        const uint8_t* src = lds + ((vt_off + v_lane0) ^ (dt << 6)) + t * 16 * ROW;
+        const uint8_t* src = lds + vt_off + (v_lane0 ^ (dt << 6)) + t * 16 * ROW;
         const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
         const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 8 * ROW));
         const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
@@ -350,6 +366,13 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             }
         }
         return v;
+    };
+    // the larger of this lane's and lane^32's value, without a round trip through LDS
+    auto max_halves = [](float m) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+        float both;
+        __asm__("v_max_f32 %0, %1, %2" : "=v"(both) : "v"(r[0]), "v"(r[1]));  // (fmaxf would make each quiet first)
+        return both;
     };
     // masking and this lane's share of the row maximum of tile T (raw scores; c > 0 keeps order)
     auto mask_max4 = [&](auto mask_tag, int T, f32x16& s, int g, float m) __attribute__((always_inline)) -> float {
@@ -373,75 +396,133 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         return m;
     };
 
-    // One tile step. In: s_in = raw (masked) scores of tile T, m_in = its row maximum (both lane
-    // halves). Out: P.V of tile T added to o; s_out = scores of tile T+1, m_out = their maximum.
-    auto step = [&](auto mask_tag, int T, f32x16& s_in, float m_in, f32x16& s_out, float& m_out,
-                    int vt /* LDS offset of the 32 value rows of tile T */) __attribute__((always_inline)) {
-        const float m_sc = m_in * c;
-        if (__any(m_sc > m_run + kSlack)) {
-            const float m_new = fmaxf(m_run, m_sc);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    constexpr int NV = 2 * DT;                 // value operands of a tile
+    constexpr int NM = NV * (SPLIT ? 2 : 1);   // P.V MFMAs
+    constexpr int NS = KS + NM;                // slots (MFMAs) of a step
+    constexpr int KD = KS / 2, V0 = SPLIT ? 2 : 4;  // key / value operands are requested that many ahead
+    static_assert(V0 <= KS && V0 <= NV && KD <= NM, "lead");
+    // P of a tile: bf16 pairs, and their remainders
+    struct Probs {
+        uint32_t hi[8];
+        uint32_t lo[SPLIT ? 8 : 1];
+    };
+    auto pv = [&](const Probs& p, int n, u32x4 (&vf)[NV]) __attribute__((always_inline)) {
+        const int i = SPLIT ? n >> 1 : n, t = i / DT, dt = i % DT;
+        u32x4 pf = {p.hi[4 * t], p.hi[4 * t + 1], p.hi[4 * t + 2], p.hi[4 * t + 3]};
+        if constexpr (SPLIT)
+            if (n & 1) pf = u32x4{p.lo[4 * t], p.lo[4 * t + 1], p.lo[4 * t + 2], p.lo[4 * t + 3]};
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(bf16x8, vf[i]), __builtin_bit_cast(bf16x8, pf), o[dt], 0, 0, 0);
+    };
+    auto k_first = [&](int T, u32x4 (&kf)[KS]) __attribute__((always_inline)) {  // a step's first key operands
+#pragma unroll
+        for (int ks = 0; ks < KD; ++ks) kf[ks] = k_frag((T & 3) * TILE, ks);
+    };
+    [[maybe_unused]] uint32_t k_at[DMA], v_at[DMA];  // where the block's loads go to (paged: looked up at its start)
+
+    // One step: the scores of tile T+1, P of tile T, and P.V of tile T-1, the exponentials spread evenly over all of
+    // its MFMAs. In: s_in = raw (masked) scores of tile T; grow_in: some row's maximum m_in (both lane halves) has
+    // outgrown the reference. Out: p_out = P of tile T; s_out, m_out, grow_out the same for tile T+1.
+    // first_tag: a block's first step, which issues its loads (K tiles T+3, T+4, V tiles T+1, T+2), and reads the
+    // second step's first key operands.
+    auto step = [&](auto mask_tag, auto ring_tag, auto first_tag, int T, f32x16& s_in, float m_in, bool grow_in, f32x16& s_out,
+                    float& m_out, bool& grow_out, const Probs& p_in, Probs& p_out, u32x4 (&kf)[KS])
+                    __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first_tag)::value;
+        constexpr int RING0 = decltype(ring_tag)::value;  // ring slot of the block's first tile; -1: from T
+        constexpr int AT = RING0 + (FIRST ? 0 : 1);
+        auto slot_of = [&](int d) { return RING0 >= 0 ? (AT + d + 4) & 3 : (T + d) & 3; };
+        float alpha = 1.0f;
+        if (__builtin_expect(grow_in, 0)) {
+            __asm__ volatile("" ::: "memory");  // (a branch, not four selects)
+            const float m_new = fmaxf(m_run, m_in * c);
+            alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             m_run = m_new;
+            m_lim = m_new + kSlack;
             l_run *= alpha;
+        }
+        const int kt = slot_of(1) * TILE, vt = RING + slot_of(-1) * TILE;
+        float l_add = 0.0f, e0 = 0.0f, e1 = 0.0f, m = kNegBig;
+        u32x4 vf[NV];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            // operands of later MFMAs
+            if (n + KD < KS) kf[n + KD] = k_frag(kt, n + KD);
+            if (n >= KS - V0 && n < KS)
+                vf[n - (KS - V0)] = v_frag(mask_tag, (T - 1) * 32, vt, (n - (KS - V0)) / DT, (n - (KS - V0)) % DT);
+            if (n >= KS && (!SPLIT || ((n - KS) & 1) == 0)) {
+                const int i = (SPLIT ? (n - KS) >> 1 : n - KS) + V0;
+                if (i < NV) vf[i] = v_frag(mask_tag, (T - 1) * 32, vt, i / DT, i % DT);
+            }
+            if constexpr (FIRST)
+                if (n >= NS - KD) kf[n - (NS - KD)] = k_frag(slot_of(2) * TILE, n - (NS - KD));
+            if (n < KS) {
+                s_out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, kf[n]), __builtin_bit_cast(bf16x8, qf[n]), n == 0 ? zero16 : s_out, 0, 0, 0);
+            } else {
+                pv(p_in, n - KS, vf);
+            }
+            if constexpr (FIRST) {
+                // the block's loads, one at a time: together they stall the waves that issue them
+#pragma unroll
+                for (int l = 0; l < 2 * DMA; ++l)
+                    if (n == 1 + l * (NS - 2) / (2 * DMA)) {
+                        if (l < DMA) dma_k(l, slot_of(3), PAGED ? k_at[l] : k_off(l, 0));
+                        else dma_v(l - DMA, slot_of(1), PAGED ? v_at[l - DMA] : v_off(l - DMA, 0));
+                    }
+            }
+            // exponentials: element e behind MFMA e * NS / 16
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (n == e * NS / 16) {
+                    float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[e], c, -m_run));
+                    __asm__ volatile("" : "+v"(p));  // here: its uses are a step away, and the compiler would move it there
+                    if ((e & 1) == 0) {
+                        e0 = p;
+                    } else {
+                        e1 = p;
+                        l_add += e0 + e1;
+                        uint32_t hi = pack_bf16x2(e0, e1);
+                        __asm__ volatile("" : "+v"(hi), "+v"(l_add));
+                        p_out.hi[e >> 1] = hi;
+                        if constexpr (SPLIT) {
+                            uint32_t lo = pack_bf16x2(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xffff0000u));
+                            __asm__ volatile("" : "+v"(lo));
+                            p_out.lo[e >> 1] = lo;
+                        }
+                    }
+                }
+            if (n >= NS - 6 && n < NS - 2) m = mask_max4(mask_tag, T + 1, s_out, n - (NS - 6), m);
+            if (n == NS - 2) m_out = max_halves(m);
+            if (n == NS - 1) grow_out = __any(m_out * c > m_lim);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        l_run += l_add;
+        if (__builtin_expect(grow_in, 0)) {  // P.V of tile T-1 was still against the old reference
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
         }
-        const int kt = ((T + 1) & 3) * TILE;
-        constexpr int NV = 2 * DT;                 // value operands of a tile
-        constexpr int NM = NV * (SPLIT ? 2 : 1);   // P.V MFMAs
-        constexpr int EPK = 8 / KS;                // score pairs per score MFMA
-        uint32_t pk[8];
-        [[maybe_unused]] uint32_t pr[8];
-        float l_add = 0.0f;
-        u32x4 kf[KS], vf[NV];
-        kf[0] = k_frag(kt, 0);
-        kf[1] = k_frag(kt, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        // ---- the score MFMAs of tile T+1, each followed by exponentials of tile T
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (ks + 2 < KS) kf[ks + 2] = k_frag(kt, ks + 2);
-            if (ks >= KS - 2) vf[ks - (KS - 2)] = v_frag(mask_tag, T * 32, vt, 0, ks - (KS - 2));
-            s_out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                __builtin_bit_cast(bf16x8, kf[ks]), __builtin_bit_cast(bf16x8, qf[ks]),
-                ks == 0 ? zero16 : s_out, 0, 0, 0);
-#pragma unroll
-            for (int u = 0; u < EPK; ++u) {
-                const int i = ks * EPK + u;
-                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * i], c, -m_run));
-                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[2 * i + 1], c, -m_run));
-                l_add += p0 + p1;
-                pk[i] = pack_bf16x2(p0, p1);
-                if constexpr (SPLIT)
-                    pr[i] = pack_bf16x2(p0 - __uint_as_float(pk[i] << 16), p1 - __uint_as_float(pk[i] & 0xffff0000u));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        l_run += l_add;
-        // ---- the P.V MFMAs of tile T, the last ones followed by the maximum of tile T+1
-        float m = kNegBig;
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-            const int i = SPLIT ? n >> 1 : n, t = i / DT, dt = i % DT;
-            if ((!SPLIT || (n & 1) == 0) && i + 2 < NV)
-                vf[i + 2] = v_frag(mask_tag, T * 32, vt, (i + 2) / DT, (i + 2) % DT);
-            u32x4 pf = {pk[4 * t], pk[4 * t + 1], pk[4 * t + 2], pk[4 * t + 3]};
-            if constexpr (SPLIT)
-                if (n & 1) pf = u32x4{pr[4 * t], pr[4 * t + 1], pr[4 * t + 2], pr[4 * t + 3]};
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                __builtin_bit_cast(bf16x8, vf[i]), __builtin_bit_cast(bf16x8, pf), o[dt], 0, 0, 0);
-            if (n >= NM - 4) m = mask_max4(mask_tag, T + 1, s_out, n - (NM - 4), m);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        m_out = fmaxf(m, __shfl_xor(m, 32, kWave));
     };
 
-    // ---- prologue: tiles 0..2 and the first value block; scores of tile 0
+    // ---- prologue: key tiles 0..2, value tiles -1 (zeros) and 0; scores of tile 0
     const int tfull = (pmin + 1) / 32;  // tiles every query of the wave sees whole
     const int nfast = MASK ? 0 : min(max(tfull - 1, 0), tiles_w) / 2;  // blocks whose steps only produce unmasked tiles
-    dma_v(0, slots);
+#pragma unroll
+    for (int j = 0; j < DMA; ++j) {
+        uint32_t off;
+        if constexpr (PAGED) {
+            off = v_off(j, rows_of(slots));
+        } else {
+            const int row = (wave * DMA + j) * RPI + lane / LPR;
+            off = row < 32 ? kMissing
+                           : (uint32_t)min((uint64_t)(row - 32) * v_row + (((lane & (LPR - 1)) ^ swz_v(row)) << 4), (uint64_t)kMissing);
+        }
+        dma_v(j, -1, off);
+    }
+    if constexpr (!PAGED) advance(rv, (uint64_t)v_row * 32);  // the first block's: tiles 1, 2
     if constexpr (PAGED) slots = lookup(3, 1);  // what the first block's loads will ask for
     // tile 0 needs the queries and the key tiles, not the values: wait for everything but
     // this wave's DMA value loads (the newest), which get the scores of tile 0 to land
@@ -449,6 +530,8 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     __syncthreads();
     f32x16 sa, sb;
     float ma, mb;
+    bool ga, gb;
+    Probs pa, pb;
     {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
@@ -458,44 +541,73 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         float m = kNegBig;
 #pragma unroll
         for (int g = 0; g < 4; ++g) m = mask_max4(std::true_type{}, 0, sa, g, m);
-        ma = fmaxf(m, __shfl_xor(m, 32, kWave));
+        ma = max_halves(m);
+        ga = __any(ma * c > m_lim);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pb.hi[i] = 0;
+#pragma unroll
+        for (int i = 0; i < (SPLIT ? 8 : 1); ++i) pb.lo[i] = 0;
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __syncthreads();  // values landed; tile 0's ring slot is overwritten by the first block's loads
-    auto begin_block = [&](int kb) {
-        dma_k(2 * kb + 3, slots);  // tiles 2kb+3, 2kb+4: their ring slots held tiles 2kb-1 and 2kb
-        if (kb + 1 < nkb) dma_v(kb + 1, slots);
-        if constexpr (PAGED) slots = lookup(2 * kb + 5, kb + 2);  // for the next block's loads
+    u32x4 kf[KS];
+    k_first(1, kf);
+    auto begin_block = [&]([[maybe_unused]] int kb) {
+        if constexpr (PAGED) {
+#pragma unroll
+            for (int j = 0; j < DMA; ++j) k_at[j] = k_off(j, rows_of(slots)), v_at[j] = v_off(j, rows_of(slots));
+            slots = lookup(2 * kb + 5, 2 * kb + 3);  // for the next block's loads
+        }
     };
-    auto end_block = [&] {
+    auto end_block = [&](int next_tile) {  // (or its ring slot)
+        if constexpr (!PAGED) {
+            advance(rk, (uint64_t)k_row * 64);
+            advance(rv, (uint64_t)v_row * 64);
+        }
         __builtin_amdgcn_s_waitcnt(0x0070);
         __syncthreads();
+        k_first(next_tile, kf);
+    };
+    auto block = [&](auto mask_tag, auto ring_tag, int kb) __attribute__((always_inline)) {
+        constexpr int R = decltype(ring_tag)::value;
+        begin_block(kb);
+        step(mask_tag, ring_tag, std::true_type{}, 2 * kb, sa, ma, ga, sb, mb, gb, pb, pa, kf);
+        step(mask_tag, ring_tag, std::false_type{}, 2 * kb + 1, sb, mb, gb, sa, ma, ga, pa, pb, kf);
+        end_block(R >= 0 ? R + 3 : 2 * kb + 3);
     };
     int kb = 0;
-    for (; kb < nfast; ++kb) {
-        begin_block(kb);
-        const int vt = RING + (kb & 1) * VBUF;
-        step(std::false_type{}, 2 * kb, sa, ma, sb, mb, vt);
-        step(std::false_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + TILE);
-        end_block();
+    for (; kb + 1 < nfast; kb += 2) {  // two blocks: once round the rings, so that every LDS offset is a constant
+        block(std::false_type{}, std::integral_constant<int, 0>{}, kb);
+        block(std::false_type{}, std::integral_constant<int, 2>{}, kb + 1);
     }
-    for (; kb < tiles_w / 2; ++kb) {
+    for (; kb < tiles_w / 2; ++kb) block(std::true_type{}, std::integral_constant<int, -1>{}, kb);
+    auto last_pv = [&](const Probs& p) __attribute__((always_inline)) {
+        const int vt = RING + ((tiles_w - 1) & 3) * TILE;
+        u32x4 vf[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) vf[i] = v_frag(std::true_type{}, (tiles_w - 1) * 32, vt, i / DT, i % DT);
+#pragma unroll
+        for (int n = 0; n < NM; ++n) pv(p, n, vf);
+    };
+    if (tiles_w & 1) {  // a last block of one tile, whose values are there already (the next block's loads replace them)
         begin_block(kb);
-        const int vt = RING + (kb & 1) * VBUF;
-        step(std::true_type{}, 2 * kb, sa, ma, sb, mb, vt);
-        step(std::true_type{}, 2 * kb + 1, sb, mb, sa, ma, vt + TILE);
-        end_block();
-    }
-    if (tiles_w & 1) {  // a last block of one tile
-        begin_block(kb);
-        step(std::true_type{}, 2 * kb, sa, ma, sb, mb, RING + (kb & 1) * VBUF);
-        end_block();
+        step(std::true_type{}, std::integral_constant<int, -1>{}, std::true_type{}, 2 * kb, sa, ma, ga, sb, mb, gb, pb, pa, kf);
+        last_pv(pa);
+        end_block(2 * kb + 3);
         ++kb;
+    } else {
+        last_pv(pb);
     }
     for (; kb < nkb; ++kb) {  // keys that only later tokens of the workgroup see
         begin_block(kb);
-        end_block();
+#pragma unroll
+        for (int j = 0; j < DMA; ++j) {
+            dma_k(j, 2 * kb + 3, PAGED ? k_at[j] : k_off(j, 0));
+            dma_v(j, 2 * kb + 1, PAGED ? v_at[j] : v_off(j, 0));
+        }
+        end_block(2 * kb + 3);
     }
+    if constexpr (WAVES * TILE > RING) __syncthreads();  // some staging areas lie over the values
     // ---- normalise and write [batch, seq, heads*D]: through this wave's part of the
     // (now idle) LDS, so that the 32 x D tile leaves as whole rows
     l_run += __shfl_xor(l_run, 32, kWave);

@@ -53,6 +53,18 @@ def test_every_shape_and_edge(h, g, d, n, m):
     _check(got, *_reference(q, k, v, pos.clamp_max(m - 1)), f"{h}/{g}x{d} {n} of {m} positions")
 
 
+@pytest.mark.parametrize("h,g,d", [(2, 2, 64), (4, 2, 64), (4, 1, 64), (2, 2, 128), (4, 2, 128), (4, 1, 128), (8, 1, 128)])
+@pytest.mark.parametrize("cached", [0, 31, 129])
+def test_odd_and_even_tiles_blocks_and_rounds_of_the_rings(h, g, d, cached):
+    """Every remainder of the walk: the last block of one tile or two, an odd block behind the pairs, none and several."""
+    from astrai_amd.extension import _cabi
+    for n in (32, 64, 96, 129, 161, 192, 224, 257, 289, 352, 417):
+        q, k, v = _tensors(1, n, n + cached, h, g, d, seed=n)
+        newest = torch.arange(n) + cached
+        got = _cabi.attn_prefill_strided(q, k, v, _cabi.BLHD, cached)
+        _check(got, *_reference(q, k, v, newest), f"{h}/{g}x{d} {n} behind {cached}")
+
+
 @pytest.mark.parametrize("h,g,d", SHAPES)
 def test_memory_orders_give_the_same_bits(h, g, d):
     from astrai_amd.extension import _cabi
