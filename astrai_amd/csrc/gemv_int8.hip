@@ -137,11 +137,17 @@ RowsPlan plan_rows(const GemmArgs& g) {
     return p;
 }
 
-template <int RG, int MB, int NW, bool ROPE>
+template <int RG, int MB, int NW, bool ROPE, bool WH = false, bool XH = false>
 void launch_rows_inst(const GemmArgs& g, const RopeCacheArgs& rc, const RowsPlan& p, hipStream_t stream) {
+    if constexpr (RG == 1 && !WH && !XH) {   // half groups: 2048 outputs of a decode step are 8 rows to a workgroup
+        if (p.rows_per_wg <= 8) return launch_rows_inst<RG, MB, NW, ROPE, true, XH>(g, rc, p, stream);
+    }
+    if constexpr (MB == 1 && !XH) {
+        if (g.m <= 8) return launch_rows_inst<RG, MB, NW, ROPE, WH, true>(g, rc, p, stream);
+    }
     constexpr int lds_bytes = gemv_rows_lds_bytes<RG, MB, NW>();
     static_assert(lds_bytes <= 160 * 1024, "patches and partials of all waves must fit in LDS");
-    auto kern = gemv_int8_rows_kernel<RG, MB, NW, 1, ROPE>;
+    auto kern = gemv_int8_rows_kernel<RG, MB, NW, ROPE, WH, XH>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_allowed);
     note_kernel(ROPE ? "gemv_rows_rope" : "gemv_rows");
@@ -175,12 +181,15 @@ void launch_rows(const GemmArgs& g, const RopeCacheArgs& rc, hipStream_t stream)
 }
 
 // fp8: the same plan and the same token-group instances; bf16 or fp32-accumulator output
-template <int Fmt, int RG, int MB, int NW, bool RoundFirst = false>
+template <int Fmt, int RG, int MB, int NW, bool RoundFirst = false, bool WH = false>
 void launch_rows_fp8_inst(const GemmArgs& g, const RowsPlan& p, bool rowcol, hipStream_t stream) {
+    if constexpr (RG == 1 && !WH) {
+        if (p.rows_per_wg <= 8) return launch_rows_fp8_inst<Fmt, RG, MB, NW, RoundFirst, true>(g, p, rowcol, stream);
+    }
     if constexpr (!RoundFirst)
-        if (g.round_first) return launch_rows_fp8_inst<Fmt, RG, MB, NW, true>(g, p, rowcol, stream);
+        if (g.round_first) return launch_rows_fp8_inst<Fmt, RG, MB, NW, true, WH>(g, p, rowcol, stream);
     constexpr int lds_bytes = gemv_rows_lds_bytes<RG, MB, NW>();
-    auto kern = gemv_fp8_rows_kernel<Fmt, RG, MB, NW, RoundFirst>;
+    auto kern = gemv_fp8_rows_kernel<Fmt, RG, MB, NW, RoundFirst, WH>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_allowed);
     note_kernel("gemv_rows_fp8");
@@ -211,10 +220,13 @@ void launch_rows_fp8(const GemmArgs& g, bool rowcol, hipStream_t stream) {
     else launch_rows_fp8_mb<Fmt, 1, 4>(g, p, rowcol, stream);
 }
 
-template <int RG, int MB, int NW>
+template <int RG, int MB, int NW, bool WH = false>
 void launch_rows_fp8_block_inst(const GemmArgs& g, const RowsPlan& p, hipStream_t stream) {
+    if constexpr (RG == 1 && !WH) {
+        if (p.rows_per_wg <= 8) return launch_rows_fp8_block_inst<RG, MB, NW, true>(g, p, stream);
+    }
     constexpr int lds_bytes = gemv_rows_lds_bytes<RG, MB, NW>();
-    auto kern = gemv_fp8_block128_rows_kernel<RG, MB, NW>;
+    auto kern = gemv_fp8_block128_rows_kernel<RG, MB, NW, WH>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_allowed);
     note_kernel("gemv_rows_fp8_block128");

@@ -18,6 +18,10 @@
 //    XOR chunk swizzle that keeps both the row-major writes and the operand reads
 //    conflict-free. Weights and activations take the same route, so any K order inside
 //    an item is the same for both operands.
+//  * Loads of rows and tokens that are not there are left out, and those past a wave's last item: each costs the
+//    load path of the compute unit 16 cycles. int8 2048 -> 2048 4.62 -> 4.28 us (32 tokens), 6.1 -> 5.2 (64), 5632 -> 2048
+//    10.0 -> 8.9, 4096 -> 4096 9.6 -> 8.3 (64), 11008 -> 4096 13.7 -> 13.3 (32); fp8 7168 -> 2048 15.1 -> 12.7 (96); block
+//    steps 4096 -> 11008 11.5 -> 10.9 (16). One with 2 to 16 tokens -2 to -4%, int8 K = 5632 with 16 tokens 5.62 -> 5.70.
 //  * int32 partials of the waves are summed through LDS (integer addition: the split
 //    keeps the accumulator bit-exact), then the dequant epilogue, optionally continued
 //    by rotary embedding and the KV-cache write for a fused q|k|v projection.
@@ -25,6 +29,8 @@
 //    registers (any K order inside an item is a valid contraction); the waves' fp32 partials
 //    are added in wave order, so a result does not change from launch to launch.
 #pragma once
+
+#include <type_traits>
 
 #include "common.cuh"
 #include "launchers.h"
@@ -78,7 +84,9 @@ template <class Op, class = void> struct rows_op_block { static constexpr bool v
 template <class Op> struct rows_op_block<Op, decltype((void)Op::kBlock)> { static constexpr bool value = Op::kBlock; };
 
 // `rowcol`: one step per token and per weight row (always so for int8); else one per tensor
-template <class Op, int RG, int MB, int NW, int IB, bool ROPE, bool RoundFirst = false>
+// WH, XH: of the last group of weight rows / of tokens at most 8 are there: the other half is not asked for (a load past
+// every row costs the unit's one load path its 16 cycles as any other)
+template <class Op, int RG, int MB, int NW, bool WH, bool XH, bool ROPE, bool RoundFirst = false>
 __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCacheArgs& rc, int rows_per_wg,
                                                bool rowcol) {
     using Acc = typename Op::Acc;
@@ -157,103 +165,104 @@ __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCach
     const uint32_t lane_off = (uint32_t)lgrp * (uint32_t)K + (uint32_t)lrow * 16;
 
     // A unit is four load instructions = 16 rows x 256 bytes of one operand; an item is MB
-    // activation units (token groups) followed by RG weight units (row groups). The wave
-    // keeps a ring of IB items in flight: as soon as a unit has been consumed, the same unit
-    // of the item IB further on is requested into its registers, so the number of bytes
-    // in flight per wave stays constant from the first instruction to the last (a burst of
+    // activation units (token groups) followed by RG weight units (row groups). As soon as a
+    // unit has been consumed, the same unit of the next item is requested into its registers, so
+    // the number of bytes in flight per wave stays constant until the last item (a burst of
     // every load followed by one wait measured slower by more than a microsecond, and so did
     // fewer, deeper bursts: the memory system is fed best by many waves with a steady, modest
     // window each).
     constexpr int P = MB + RG;
-    u32x4 ring[IB][P][4];
+    u32x4 ring[P][4] = {};
+    auto loads_of = [](int s) { return s < MB ? (XH && s == MB - 1 ? 2 : 4) : (WH && s == P - 1 ? 2 : 4); };
     // block steps of an item's two K-blocks, per unit: activations' for token s * 16 + lrow, weights'
     // for the 128-row block of rows r0 + (s - MB) * 16 + 4 * lgrp .. + 3 (requested with the unit)
-    [[maybe_unused]] f32x2 steps[IB][P];
+    [[maybe_unused]] f32x2 steps[P];
     [[maybe_unused]] const int kblocks = K >> 7;
     auto issue_steps = [&](f32x2& dst, int item, int s) {
         if constexpr (rows_op_block<Op>::value) {
             dst = f32x2{0.0f, 0.0f};
-            if (item < i1) {
-                if (s < MB) {
-                    const int m = s * 16 + lrow;
-                    if (m < g.m) dst = *reinterpret_cast<const f32x2*>(g.sa + (size_t)m * kblocks + 2 * item);
-                } else {
-                    const int row = r0 + (s - MB) * 16 + 4 * lgrp;
-                    if (row < r1) dst = *reinterpret_cast<const f32x2*>(g.sb + (size_t)(row >> 7) * kblocks + 2 * item);
-                }
+            if (s < MB) {
+                const int m = s * 16 + lrow;
+                if (m < g.m) dst = *reinterpret_cast<const f32x2*>(g.sa + (size_t)m * kblocks + 2 * item);
+            } else {
+                const int row = r0 + (s - MB) * 16 + 4 * lgrp;
+                if (row < r1) dst = *reinterpret_cast<const f32x2*>(g.sb + (size_t)(row >> 7) * kblocks + 2 * item);
             }
         }
     };
+    // The last item requests nothing, in a copy of the body of its own; with all registers taken and more (fp8, 128 tokens of
+    // three row groups) the copy spilled 63 instead of 25, 21.2 -> 23.0 us: there it asks for rows past every end.
+    constexpr bool ONE_BODY = !Op::kIsInt && RG * MB >= 24;
     auto issue = [&](u32x4 (&dst)[4], int item, int s) {
-        const bool live = item < i1;
+        const bool live = !ONE_BODY || item < i1;
         const uint32_t k0 = (uint32_t)item << 8;
         if (s < MB) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)   // tokens past M start past num_records: zeros
+            for (int i = 0; i < loads_of(s); ++i)   // tokens past M start past num_records: zeros
                 dst[i] = buf_load16(rx, live ? lane_off + (uint32_t)(s * 16 + i * 4) * (uint32_t)K : kOutOfRange, k0);
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < loads_of(s); ++i) {
                 const int row = r0 + (s - MB) * 16 + i * 4;   // + lgrp, inside lane_off
                 dst[i] = buf_load16_aux<kAuxStream>(
-                    rw, (live && row + lgrp < r1) ? lane_off + (uint32_t)row * (uint32_t)K : kOutOfRange, k0);
+                    rw, live && row + lgrp < r1 ? lane_off + (uint32_t)row * (uint32_t)K : kOutOfRange, k0);
             }
         }
     };
-#pragma unroll
-    for (int t = 0; t < IB; ++t)
+    auto consume = [&](auto last_tag, int item) {
+        u32x4 xf[MB][4];
+        [[maybe_unused]] f32x2 xs[MB];
 #pragma unroll
         for (int s = 0; s < P; ++s) {
-            issue(ring[t][s], i0 + t, s);
-            issue_steps(steps[t][s], i0 + t, s);
-        }
-
-    for (int ib = i0; ib < i1; ib += IB) {
+            if (s < MB) {
+                to_operand_order(xpatch, lane, ring[s], xf[s < MB ? s : 0]);
+                if constexpr (rows_op_block<Op>::value) xs[s < MB ? s : 0] = steps[s];
+            } else {
+                u32x4 wf[4];
+                to_operand_order(wpatch, lane, ring[s], wf);
+                if constexpr (Op::kIsInt) {
 #pragma unroll
-        for (int t = 0; t < IB; ++t) {
-            u32x4 xf[MB][4];
-            [[maybe_unused]] f32x2 xs[MB];
+                    for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int s = 0; s < P; ++s) {
-                if (s < MB) {
-                    to_operand_order(xpatch, lane, ring[t][s], xf[s < MB ? s : 0]);
-                    if constexpr (rows_op_block<Op>::value) xs[s < MB ? s : 0] = steps[t][s];
+                        for (int b = 0; b < MB; ++b)
+                            acc[s < MB ? 0 : s - MB][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                                (i32x4)wf[j], (i32x4)xf[b][j], acc[s < MB ? 0 : s - MB][b], 0, 0, 0);
+                } else if constexpr (rows_op_block<Op>::value) {
+                    const f32x2 ws = steps[s];
+#pragma unroll
+                    for (int j = 0; j < 4; j += 2)
+#pragma unroll
+                        for (int b = 0; b < MB; ++b) {
+                            const f32x4 part = OpF8<0>::mma(wf[j], wf[j + 1], xf[b][j], xf[b][j + 1],
+                                                            f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                            const float sc = xs[b][j >> 1] * ws[j >> 1];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[s < MB ? 0 : s - MB][b][e] += part[e] * sc;
+                        }
                 } else {
-                    u32x4 wf[4];
-                    to_operand_order(wpatch, lane, ring[t][s], wf);
-                    if constexpr (Op::kIsInt) {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
+                    for (int j = 0; j < 4; j += 2)
 #pragma unroll
-                            for (int b = 0; b < MB; ++b)
-                                acc[s < MB ? 0 : s - MB][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                                    (i32x4)wf[j], (i32x4)xf[b][j], acc[s < MB ? 0 : s - MB][b], 0, 0, 0);
-                    } else if constexpr (rows_op_block<Op>::value) {
-                        const f32x2 ws = steps[t][s];
-#pragma unroll
-                        for (int j = 0; j < 4; j += 2)
-#pragma unroll
-                            for (int b = 0; b < MB; ++b) {
-                                const f32x4 part = OpF8<0>::mma(wf[j], wf[j + 1], xf[b][j], xf[b][j + 1],
-                                                                f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                                const float sc = xs[b][j >> 1] * ws[j >> 1];
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) acc[s < MB ? 0 : s - MB][b][e] += part[e] * sc;
-                            }
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; j += 2)
-#pragma unroll
-                            for (int b = 0; b < MB; ++b)
-                                acc[s < MB ? 0 : s - MB][b] = OpF8<Op::kFmt>::mma(
-                                    wf[j], wf[j + 1], xf[b][j], xf[b][j + 1], acc[s < MB ? 0 : s - MB][b]);
-                    }
+                        for (int b = 0; b < MB; ++b)
+                            acc[s < MB ? 0 : s - MB][b] = OpF8<Op::kFmt>::mma(
+                                wf[j], wf[j + 1], xf[b][j], xf[b][j + 1], acc[s < MB ? 0 : s - MB][b]);
                 }
-                issue(ring[t][s], ib + t + IB, s);
-                issue_steps(steps[t][s], ib + t + IB, s);
-                __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (!decltype(last_tag)::value) {
+                issue(ring[s], item + 1, s);
+                issue_steps(steps[s], item + 1, s);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    if (i0 < i1) {
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+            issue(ring[s], i0, s);
+            issue_steps(steps[s], i0, s);
+        }
+        for (int item = i0; item + (ONE_BODY ? 0 : 1) < i1; ++item) consume(std::false_type{}, item);
+        if constexpr (!ONE_BODY) consume(std::true_type{}, i1 - 1);
     }
 
     // sum the waves' partials through LDS (the patches are free now)
@@ -350,21 +359,21 @@ __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCach
     }
 }
 
-template <int RG, int MB, int NW, int IB, bool ROPE>
+template <int RG, int MB, int NW, bool ROPE, bool WH, bool XH>
 __global__ __launch_bounds__(NW * 64) void gemv_int8_rows_kernel(GemmArgs g, RopeCacheArgs rc, int rows_per_wg) {
-    gemv_rows_body<RowsOpI8, RG, MB, NW, IB, ROPE>(g, rc, rows_per_wg, true);
+    gemv_rows_body<RowsOpI8, RG, MB, NW, WH, XH, ROPE>(g, rc, rows_per_wg, true);
 }
 
 // RoundFirst: the product is rounded to bf16 before the bias joins it (chosen in the epilogue: 100 x 4096 x 4096 12.5 ->
 // 12.75 us for every product)
-template <int Fmt, int RG, int MB, int NW, bool RoundFirst>
+template <int Fmt, int RG, int MB, int NW, bool RoundFirst, bool WH>
 __global__ __launch_bounds__(NW * 64) void gemv_fp8_rows_kernel(GemmArgs g, int rows_per_wg, int rowcol) {
-    gemv_rows_body<RowsOpF8<Fmt>, RG, MB, NW, 1, false, RoundFirst>(g, RopeCacheArgs{}, rows_per_wg, rowcol != 0);
+    gemv_rows_body<RowsOpF8<Fmt>, RG, MB, NW, WH, false, false, RoundFirst>(g, RopeCacheArgs{}, rows_per_wg, rowcol != 0);
 }
 
-template <int RG, int MB, int NW>
+template <int RG, int MB, int NW, bool WH>
 __global__ __launch_bounds__(NW * 64) void gemv_fp8_block128_rows_kernel(GemmArgs g, int rows_per_wg) {
-    gemv_rows_body<RowsOpF8Block, RG, MB, NW, 1, false>(g, RopeCacheArgs{}, rows_per_wg, false);
+    gemv_rows_body<RowsOpF8Block, RG, MB, NW, WH, false, false>(g, RopeCacheArgs{}, rows_per_wg, false);
 }
 
 template <int RG, int MB, int NW>

@@ -10,7 +10,14 @@
 // patch whose XOR chunk swizzle keeps the row-major writes and the operand reads free of conflicts. Weights
 // and x take the same route, so any order of K inside an item is the same for both. Each unit's registers are
 // refilled for the next item as soon as it has been consumed: the bytes in flight stay the same from the first
-// instruction to the last. The waves' partial sums are added through LDS in wave order.
+// instruction to the last, when nothing is left to request. The waves' partial sums are added through LDS in wave order.
+//
+// What bounds it (graph replays over weights that no cache holds): the stream from 20 MB on (2048 -> 32000, 131 MB, 22.5 us at 1
+// token, 5.8 TB/s), below it launch and the load path's 16 cycles for every 1 KiB instruction, of x as much as of the
+// weights: leaving out those for rows and tokens that are not there and those past the last item took 2048 -> 2048 from 4.3
+// to 3.8 us (1 token) and 5.6 to 5.3 (32), 2048 -> 6656 from 7.6 to 6.8 and 8.4 to 8.2, gate|up of 5632 9.85 -> 9.6 and 11.3 -> 11.0.
+#include <type_traits>
+
 #include "mix_common.cuh"
 #include "mix_launchers.h"
 
@@ -38,8 +45,8 @@ __device__ __forceinline__ void to_operand_order(uint8_t* patch, int lane, const
 }
 
 // RG: groups of 16 weight rows per workgroup (ACT >= 0: of gate and of up each); MB: groups of 16 tokens;
-// NW: waves. ACT: -1 none.
-template <int RG, int MB, int NW, int ACT, bool F32>
+// NW: waves. ACT: -1 none. IB: items under way (two where a wave's eight rows leave too few bytes in flight). WH, XH: of the last group of weight rows / of tokens at most 8 are there.
+template <int RG, int MB, int NW, int ACT, bool F32, bool WH, bool XH, int IB>
 __global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a, int rows_per_wg) {
     constexpr int HALVES = ACT >= 0 ? 2 : 1;
     constexpr int WG = RG * HALVES;              // weight units per item
@@ -64,44 +71,74 @@ __global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a,
 
     uint8_t* const wpatch = smem + wave * WAVE_LDS;
     uint8_t* const xpatch = wpatch + 4096;
-    u32x4 ring[P][4];
+    u32x4 ring[IB][P][4] = {};
+    // (a load past every row costs the unit's one load path its 16 cycles as any other: left out)
+    auto loads_of = [](int s) { return s < MB ? (XH && s == MB - 1 ? 2 : 4) : (WH && (s - MB) % RG == RG - 1 ? 2 : 4); };
     auto issue = [&](u32x4 (&dst)[4], int item, int s) {
-        const bool live = item < i1;
         const uint32_t k0 = (uint32_t)item * kItem;
         if (s < MB) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)  // tokens past m lie past the descriptor: zeros
-                dst[i] = w8a8::buf_load16(
-                    rx, live ? (uint32_t)(s * 16 + i * 4 + g) * x_row + (uint32_t)c16 * 16 : w8a8::kOutOfRange, k0);
+            for (int i = 0; i < loads_of(s); ++i)  // tokens past m lie past the descriptor: zeros
+                dst[i] = w8a8::buf_load16(rx, (uint32_t)(s * 16 + i * 4 + g) * x_row + (uint32_t)c16 * 16, k0);
         } else {
             const int u = s - MB, half = u / RG;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < loads_of(s); ++i) {
                 const int row = r0 + (u - half * RG) * 16 + i * 4 + g;
                 dst[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rw, live && row < r1 ? (uint32_t)(half * a.n + row) * w_row + (uint32_t)c16 * 16 : w8a8::kOutOfRange,
+                    rw, row < r1 ? (uint32_t)(half * a.n + row) * w_row + (uint32_t)c16 * 16 : w8a8::kOutOfRange,
                     k0, 2);  // 2: not kept once delivered
             }
         }
     };
-#pragma unroll
-    for (int s = 0; s < P; ++s) issue(ring[s], i0, s);
-    for (int item = i0; item < i1; ++item) {
+    // an item; NEXT: the item that many further on is requested into its registers, a unit at a time
+    auto consume = [&](u32x4 (&units)[P][4], auto next_tag, int item) {
+        constexpr int NEXT = decltype(next_tag)::value;
         u32x4 xf[MB][4];
 #pragma unroll
         for (int s = 0; s < P; ++s) {
             if (s < MB) {
-                to_operand_order(xpatch, lane, ring[s], xf[s < MB ? s : 0]);
+                to_operand_order(xpatch, lane, units[s], xf[s < MB ? s : 0]);
             } else {
                 u32x4 wf[4];
-                to_operand_order(wpatch, lane, ring[s], wf);
+                to_operand_order(wpatch, lane, units[s], wf);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int b = 0; b < MB; ++b) acc[s < MB ? 0 : s - MB][b] = mfma16(wf[j], xf[b][j], acc[s < MB ? 0 : s - MB][b]);
             }
-            issue(ring[s], item + 1, s);
+            if constexpr (NEXT > 0) issue(units[s], item + NEXT, s);
             __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto request = [&](u32x4 (&units)[P][4], int item) {
+#pragma unroll
+        for (int s = 0; s < P; ++s) issue(units[s], item, s);
+    };
+    constexpr std::integral_constant<int, 0> none{};
+    constexpr std::integral_constant<int, IB> next{};
+    if (i0 < i1) {
+        int item = i0;
+        request(ring[0], item);
+        if constexpr (IB == 1) {
+            for (; item + 1 < i1; ++item) consume(ring[0], next, item);
+            consume(ring[0], none, item);
+        } else if (i1 - i0 == 1) {
+            consume(ring[0], none, item);
+        } else {
+            request(ring[1], item + 1);
+            for (; item + 3 < i1; item += 2) {
+                consume(ring[0], next, item);
+                consume(ring[1], next, item + 1);
+            }
+            if (item + 2 < i1) {
+                consume(ring[0], next, item);
+                consume(ring[1], none, item + 1);
+                consume(ring[0], none, item + 2);
+            } else {
+                consume(ring[0], none, item);
+                consume(ring[1], none, item + 1);
+            }
         }
     }
 
@@ -139,19 +176,32 @@ __global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a,
     }
 }
 
-template <int RG, int MB, int NW, int ACT, bool F32>
+template <int RG, int MB, int NW, int ACT, bool F32, bool WH, bool XH, int IB = 1>
 void launch_inst(const FewRowsArgs& a, int rows, hipStream_t stream) {
     constexpr int units = RG * (ACT >= 0 ? 2 : 1) * MB * 1024;
     constexpr int lds = NW * (units > 8192 ? units : 8192);
     static_assert(lds <= 64 * 1024, "within the limit that needs no attribute");
-    few_rows_linear_kernel<RG, MB, NW, ACT, F32><<<dim3((unsigned)((a.n + rows - 1) / rows)), dim3(NW * 64), lds, stream>>>(a, rows);
+    few_rows_linear_kernel<RG, MB, NW, ACT, F32, WH, XH, IB>
+        <<<dim3((unsigned)((a.n + rows - 1) / rows)), dim3(NW * 64), lds, stream>>>(a, rows);
+}
+
+template <int RG, int NW, int ACT, bool F32, bool WH>
+void launch_mb(const FewRowsArgs& a, int rows, hipStream_t stream) {
+    if constexpr (RG == 1 && NW == 8 && ACT < 0) {
+        // Up to 8 tokens x costs little, and two items under way feed the stream (5632 -> 2048, 1 token 8.0 -> 6.6 us, 8 tokens
+        // 8.0 -> 7.2), if a wave has more than two in all (2048 -> 2048 3.8 -> 3.9). 16 tokens and more are bound by x.
+        if (a.m <= 8 && a.k >= 4096) return launch_inst<RG, 1, NW, ACT, F32, WH, true, 2>(a, rows, stream);
+    }
+    if (a.m <= 8) launch_inst<RG, 1, NW, ACT, F32, WH, true>(a, rows, stream);
+    else if (a.m <= 16) launch_inst<RG, 1, NW, ACT, F32, WH, false>(a, rows, stream);
+    else if (a.m <= 32) launch_inst<RG, 2, NW, ACT, F32, WH, false>(a, rows, stream);
+    else launch_inst<RG, 4, NW, ACT, F32, WH, false>(a, rows, stream);
 }
 
 template <int RG, int NW, int ACT, bool F32>
-void launch_mb(const FewRowsArgs& a, int rows, hipStream_t stream) {
-    if (a.m <= 16) launch_inst<RG, 1, NW, ACT, F32>(a, rows, stream);
-    else if (a.m <= 32) launch_inst<RG, 2, NW, ACT, F32>(a, rows, stream);
-    else launch_inst<RG, 4, NW, ACT, F32>(a, rows, stream);
+void launch_wh(const FewRowsArgs& a, int rows, hipStream_t stream) {
+    if (rows <= RG * 16 - 8) launch_mb<RG, NW, ACT, F32, true>(a, rows, stream);
+    else launch_mb<RG, NW, ACT, F32, false>(a, rows, stream);
 }
 
 template <int ACT, bool F32>
@@ -162,13 +212,13 @@ void launch_rg(const FewRowsArgs& a, hipStream_t stream) {
     const int wgs = 256 * ((a.n + 256 * GROUPS * 16 - 1) / (256 * GROUPS * 16));
     const int rows = ((a.n + wgs - 1) / wgs + 3) & ~3;
     if (rows > 32) {
-        if constexpr (GROUPS == 3) launch_mb<3, 4, ACT, F32>(a, rows, stream);
+        if constexpr (GROUPS == 3) launch_wh<3, 4, ACT, F32>(a, rows, stream);
     } else if (rows > 16) {
-        launch_mb<2, 4, ACT, F32>(a, rows, stream);
+        launch_wh<2, 4, ACT, F32>(a, rows, stream);
     } else if (a.k >= 1024) {
-        launch_mb<1, 8, ACT, F32>(a, rows, stream);
+        launch_wh<1, 8, ACT, F32>(a, rows, stream);
     } else {
-        launch_mb<1, 4, ACT, F32>(a, rows, stream);
+        launch_wh<1, 4, ACT, F32>(a, rows, stream);
     }
 }
 

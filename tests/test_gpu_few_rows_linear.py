@@ -37,6 +37,16 @@ def test_against_float64(m, n, k):
     assert torch.equal(_mix.few_rows_linear(wide[:, 8:8 + k], w), _mix.few_rows_linear(x, w))
 
 
+@pytest.mark.parametrize("m", [1, 8, 9])
+@pytest.mark.parametrize("n,k", [(1024, 3968), (1024, 4096), (2048, 4224), (2044, 4736), (2052, 4096), (2048, 5632), (5636, 1024),
+                                 (6148, 256)])
+def test_half_groups_and_one_or_two_items_under_way(m, n, k):
+    """8 rows or tokens and fewer of a group of sixteen, one more; every remainder of the walk over a wave's items."""
+    from astrai_amd.extension import _mix
+    x, w = _mk(m, m, k), _mk(n, n, k, std=k ** -0.5)
+    _check(_mix.few_rows_linear(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t(), 1)
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("m,ff,k", [(1, 8, 128), (3, 5632, 256), (17, 104, 384), (32, 4104, 1152), (64, 8200, 128)])
 def test_activation_epilogue(act, m, ff, k):
