@@ -22,13 +22,17 @@ struct Mid128Cfg {
     static constexpr int MI = 2, NI = 1;                 // 32-row sub-tiles per wave: 64 m x 32 n
     static constexpr int OPERAND_BYTES = 128 * BK;       // one operand's slab: 16 KiB
     static constexpr int STAGE_BYTES = 2 * OPERAND_BYTES;
-    static constexpr int LDS_BYTES = 2 * STAGE_BYTES;    // 64 KiB
 };
 
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it. An instance of its own: chosen
 // in the epilogue, it cost every per-tensor product 0.2 us (354 x 11008 x 4096: 34.3 -> 34.6).
-template <class Op, int ScaleKind, bool RoundFirst>
-__global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(GemmArgs g) {
+// S: LDS stages. 2: as above. 4: for launches of one workgroup per compute unit at most, where nobody covers its waits (1500
+// cycles a slab, against 300 of MFMAs): a ring filled four slabs ahead, one barrier per slab, the fragments of slab k + 1
+// read into a second register set beside the MFMAs of slab k; 1050 cycles a slab, bound by LDS (96 KiB of fragments, 32 KiB of
+// loads). int8 / fp8, us: 256 x 11264 x 2048 14.7 / 14.2 -> 13.1 / 12.6, 640 x 4096 x 4096 22.8 / 22.5 -> 20.5 / 18.7, 130 x 11008
+// x 4096 22.4 / 23.7 -> 18.7 / 18.4, 600 x 4096 x 11008 49.2 / 49.4 -> 43.9 / 39.9; 2048^3 (256 tiles) 16.0 / 15.1 either way.
+template <class Op, int ScaleKind, bool RoundFirst, int S>
+__global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid128_kernel(GemmArgs g) {
     using Cfg = Mid128Cfg;
     using Acc = typename Op::Acc;
     constexpr int MI = Cfg::MI, NI = Cfg::NI;
@@ -82,8 +86,8 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
     // instruction. Lane l lands at row l>>3, position l&7 of its 1 KiB block and fetches logical
     // chunk (l&7) ^ f(row): c0 for even instructions, c0 ^ 1 for odd ones. Rows past M / N are
     // past the buffer's num_records and read as zero.
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(g.a, (uint32_t)g.m * (uint32_t)K);
-    const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.b, (uint32_t)g.n * (uint32_t)K);
+    const uint32_t x_bytes = (uint32_t)g.m * (uint32_t)K, w_bytes = (uint32_t)g.n * (uint32_t)K;
+    const __amdgpu_buffer_rsrc_t rx0 = make_rsrc(g.a, x_bytes), rw0 = make_rsrc(g.b, w_bytes);
     uint32_t x_off[2], w_off[2];
     {
         const int c0 = (lane & 7) ^ (lane >> 3);
@@ -96,7 +100,13 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
     }
     const uint32_t row8 = 8u * (uint32_t)K;
     uint8_t* const dma_base = lds + wave * (16 * 128);
-    auto issue = [&](int stage, uint32_t k0) {
+    auto issue = [&](int stage, int slab) __attribute__((always_inline)) {   // past the last slab: zeros, no memory traffic
+        __amdgpu_buffer_rsrc_t rx = rx0, rw = rw0;
+        if constexpr (S > 2) {
+            rx = make_rsrc(g.a, slab < ksteps ? x_bytes : 0u);
+            rw = make_rsrc(g.b, slab < ksteps ? w_bytes : 0u);
+        }
+        const uint32_t k0 = (uint32_t)slab << 7;
         uint8_t* const dst = dma_base + stage * Cfg::STAGE_BYTES;
 #pragma unroll
         for (int r = 0; r < 2; ++r) lds_dma16(rx, dst + r * 1024, x_off[r & 1] + (uint32_t)r * row8, k0);
@@ -141,9 +151,8 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
         }
     };
 
-    auto compute = [&](int stage) {
+    auto read = [&](int stage, u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4]) __attribute__((always_inline)) {
         const uint8_t* const base = lds + stage * Cfg::STAGE_BYTES;
-        u32x4 xf[MI][4], wf[NI][4];
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
@@ -154,6 +163,8 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 xf[mi][j] = *reinterpret_cast<const u32x4*>(base + x_rd + mi * 4096 + frag_off[j]);
+    };
+    auto multiply = [&](u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4]) __attribute__((always_inline)) {
         if constexpr (ScaleKind == SCALE_BLOCK128) {
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
@@ -180,27 +191,57 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
 
     // ---- main loop: slab k+1 in flight while slab k is read; a barrier before a stage is
     // read (every wave's part has landed) and one before it is filled again
-    request_steps(0);
-    issue(0, 0u);
-    for (int k = 0; k < ksteps; ++k) {
-        if constexpr (ScaleKind == SCALE_BLOCK128) {
+    if constexpr (S == 2) {
+        request_steps(0);
+        issue(0, 0);
+        for (int k = 0; k < ksteps; ++k) {
+            if constexpr (ScaleKind == SCALE_BLOCK128) {
+    #pragma unroll
+                for (int mi = 0; mi < MI; ++mi) blk_sa[mi] = blk_sa_next[mi];
+                blk_sb = blk_sb_next;
+            }
+            if (k + 1 < ksteps) {
+                issue((k + 1) & 1, k + 1);
+                wait_vmcnt<4>();   // the four loads of slab k are older than those just issued
+            } else {
+                wait_vmcnt<0>();
+            }
+            phase_barrier();
+            // (after the wait: the next slab's steps are then older than the slab loads of the following
+            // iteration, whose wait they pass without holding it up -- a compute phase has gone by)
+            request_steps(k + 1);
+            u32x4 xf[MI][4], wf[NI][4];
+            read(k & 1, xf, wf);
+            multiply(xf, wf);
+            wait_lgkmcnt0();
+            phase_barrier();
+        }
+    } else {
+        static_assert(ScaleKind != SCALE_BLOCK128, "the wait counts leave no room for the steps' loads");
+        u32x4 xa[MI][4], wa[NI][4], xb[MI][4], wb[NI][4];
 #pragma unroll
-            for (int mi = 0; mi < MI; ++mi) blk_sa[mi] = blk_sa_next[mi];
-            blk_sb = blk_sb_next;
-        }
-        if (k + 1 < ksteps) {
-            issue((k + 1) & 1, (uint32_t)(k + 1) << 7);
-            wait_vmcnt<4>();   // the four loads of slab k are older than those just issued
-        } else {
-            wait_vmcnt<0>();
-        }
+        for (int t = 0; t < S; ++t) issue(t, t);
+        wait_vmcnt<4 * (S - 1)>();
         phase_barrier();
-        // (after the wait: the next slab's steps are then older than the slab loads of the following
-        // iteration, whose wait they pass without holding it up -- a compute phase has gone by)
-        request_steps(k + 1);
-        compute(k & 1);
-        wait_lgkmcnt0();
-        phase_barrier();
+        read(0, xa, wa);
+        // in: this slab's fragments, its reads under way
+        auto slab = [&](int k, u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4], u32x4 (&xn)[MI][4], u32x4 (&wn)[NI][4])
+                        __attribute__((always_inline)) {
+            wait_lgkmcnt0();
+            wait_vmcnt<4 * (S - 2)>();   // slab k + 1 has landed
+            phase_barrier();             // for every wave, and every wave has read slab k: its stage is free
+            issue(k & (S - 1), k + S);
+            read((k + 1) & (S - 1), xn, wn);   // (past the last slab: zeros)
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(xf, wf);
+        };
+        int k = 0;
+        for (; k + 1 < ksteps; k += 2) {
+            slab(k, xa, wa, xb, wb);
+            slab(k + 1, xb, wb, xa, wa);
+        }
+        if (k < ksteps) slab(k, xa, wa, xb, wb);
+        wait_vmcnt<0>();
     }
 
     // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad): 8-byte stores
@@ -251,24 +292,28 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, 4) void gemm_mid128_kernel(Gemm
 // 3072 x 2048 13.2 against 15.1 us, 1024 x 2048 x 2048 13.3 against 14.9 us, 512 x 4096 x 4096 (128
 // tiles) 22.5 against 22.3 us; from there on this kernel wins: 768 x 3072 x 2048 (144 tiles) 14.2
 // against 16.4 us, 256 x 11008 x 4096 (172) 23.7 against 28.6 us, 1024 x 3072 x 2048 16.0 against
-// 23.6 us, 2048 x 3072 x 2048 22.9 against 30.7 us)
+// 23.6 us, 2048 x 3072 x 2048 22.9 against 30.7 us). With four stages the line stays: 512 x 4096 x 4096 19.9 / 19.0 (int8 / fp8)
+// against 20.4 / 17.7 on 64 x 64 tiles, 1024 x 2048 x 2048 12.3 against 10.1, 700 x 2048 x 5632 (96) 22.5 against 19.8
 inline bool mid128_shape_ok(const GemmArgs& g) {
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 128 || g.out_kind != OUT_BF16) return false;
     const int64_t tiles = (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128);
     return tiles >= 140;
 }
 
-template <class Op, int ScaleKind, bool RoundFirst = false>
+template <class Op, int ScaleKind, bool RoundFirst = false, int S = 2>
 inline void launch_mid128(const GemmArgs& g, hipStream_t stream) {
     using Cfg = Mid128Cfg;
     if constexpr (!RoundFirst && ScaleKind == SCALE_TENSOR)
         if (g.round_first) return launch_mid128<Op, ScaleKind, true>(g, stream);
     const int tiles = ((g.m + Cfg::BM - 1) / Cfg::BM) * ((g.n + Cfg::BN - 1) / Cfg::BN);
-    auto kern = gemm_mid128_kernel<Op, ScaleKind, RoundFirst>;
+    if constexpr (S == 2 && ScaleKind != SCALE_BLOCK128)
+        if (tiles <= 256) return launch_mid128<Op, ScaleKind, RoundFirst, 4>(g, stream);
+    constexpr int lds_bytes = S * Cfg::STAGE_BYTES;
+    auto kern = gemm_mid128_kernel<Op, ScaleKind, RoundFirst, S>;
     static std::atomic<uint64_t> lds_allowed{0};
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_allowed);
     note_kernel(ScaleKind == SCALE_BLOCK128 ? "mid128_block128" : "mid128");
-    kern<<<dim3((unsigned)tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(g);
+    kern<<<dim3((unsigned)tiles), dim3(Cfg::THREADS), lds_bytes, stream>>>(g);
 }
 
 }  // namespace w8a8

@@ -1,4 +1,4 @@
-"""8-bit products on the 256 x 256 tiles: even and odd numbers of K slabs, ragged edges, tile counts of every kind."""
+"""8-bit products on the 256 x 256 and 128 x 128 tiles: even and odd numbers of K slabs, ragged edges, tile counts of every kind."""
 
 import pytest
 import torch
@@ -61,3 +61,23 @@ def test_block_scales_against_float64(m, n, k):
     weight = xd.abs().reshape(m, k) @ wd.abs().reshape(n, k).t()
     got = fp8_block.mm_fp8_blockscaled(x8, w8, sx, sw).double()
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + k * 2.0 ** -23 * weight).all()
+
+
+@pytest.mark.parametrize("m,n", [(185, 9000), (1500, 1536), (2048, 2040), (1300, 3072)])
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 896])
+def test_128_tiles_of_one_and_of_two_workgroups_a_unit(m, n, k):
+    """Fewer slabs than LDS stages, as many, odd and even numbers of them; one workgroup to a compute unit and more."""
+    from astrai_amd.extension import _cabi
+    a, b = _codes(m, m, k), _codes(n, n, k)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    sa, sb = (torch.rand(r, generator=g, device=DEV) * 0.01 + 0.001 for r in (m, n))
+    acc = (a.float() @ b.float().t())   # (sums under 2^24: exact)
+    assert torch.equal(_cabi.mm_int8(a, b, sa, sb), (acc * sa[:, None] * sb).bfloat16())
+    assert "mid128" in _cabi.last_kernel()
+    one, bias = torch.ones(1, device=DEV), torch.randn(n, generator=g, device=DEV).bfloat16()
+    a8, b8 = ((t.float() / 16).to(torch.float8_e4m3fn) for t in (a, b))
+    y, weight = a8.double() @ b8.double().t(), a8.double().abs() @ b8.double().abs().t()
+    for extra, kw in ((0.0, {}), (bias.double(), dict(bias=bias, round_first=True))):
+        want = y + extra
+        bound = 2.0 ** -8 * (y.abs() + want.abs()) + k * 2.0 ** -23 * weight
+        assert ((_cabi.mm_fp8(a8, b8, one, one, **kw).double() - want).abs() <= bound).all()
