@@ -49,7 +49,7 @@
 // 16 x 175..700 tokens of 32/8 heads x 64 in a pool 75.7 us (P in two terms); with the exponentials behind the score
 // MFMAs alone, the loads in a burst and offsets formed for each (120 vector instructions a tile) 80.3 and 78.2. Up to 236 /
 // 170 registers: two / three workgroups per CU. 64 query tokens a workgroup halve the loads, but couple eight waves:
-// 4 x 2048 72.3 us (75.5 here, same run), 1 x 4096 92.8 (76.4), 32 x 512 64.5 (57.9); not kept.
+// 2 x 4096 126 us (133 here, same run), 4 x 2048 74 (74), 16 x 1024 89 (85), 1 x 4096 93 (76), 32 x 512 64.5 (58); not kept.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
