@@ -392,10 +392,12 @@ def _plain_bf16(t: torch.Tensor, dev: torch.device) -> bool:
     return t.dtype == torch.bfloat16 and t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
-def linear_fp8_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
-    """Whether :func:`linear_fp8` takes these: bf16 on one GPU as the kernels read them, ``K % 16 == 0``, nothing empty."""
+def linear_fp8_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, inner: int = 1) -> bool:
+    """Whether :func:`linear_fp8` takes these: bf16 on one GPU as the kernels read them, ``K % 16 == 0``, nothing empty,
+    rows of ``x`` as wide as ``w.size(inner)`` (0: ``x`` is the output's gradient)."""
     k, dev = x.size(-1), x.device
-    return (x.is_cuda and k % 16 == 0 and x.numel() > 0 and w.numel() > 0 and _plain_bf16(x, dev) and _plain_bf16(w, dev)
+    return (x.is_cuda and w.dim() == 2 and k == w.size(inner) and k % 16 == 0 and x.numel() > 0 and w.numel() > 0
+            and _plain_bf16(x, dev) and _plain_bf16(w, dev)
             and (bias is None or (bias.shape == (w.size(0),) and _plain_bf16(bias, dev))))
 
 
@@ -417,6 +419,8 @@ def linear_fp8(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], c
     the bias joins the product rounded to bf16."""
     lib, dev = _require(), x.device
     n, k = w.shape
+    if x.size(-1) != k:   # (the kernels count rows by the element: they would write past `out`)
+        raise RuntimeError(f"linear_fp8: inner dim mismatch, x [.., {x.size(-1)}] and w [{n}, {k}]")
     m = x.numel() // k
     measure = rings[0] is None
     for step, name in zip(steps, ("sx", "sw")):
@@ -445,6 +449,8 @@ def linear_fp8_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, want_
     lib, dev = _require(), g.device
     n, k = w.shape
     m = x.numel() // k
+    if x.size(-1) != k or g.size(-1) != n or g.numel() != m * n:
+        raise RuntimeError(f"linear_fp8_backward: shape mismatch, g {tuple(g.shape)}, x {tuple(x.shape)}, w {tuple(w.shape)}")
     if steps is None:
         steps = (None, None, None)
     for step, name in zip(steps, ("sg", "sx", "sw")):

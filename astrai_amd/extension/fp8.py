@@ -455,8 +455,7 @@ def fp8_linear_forward(x: torch.Tensor, w: torch.Tensor, bias=None, bias_in_prod
 
 def _backward_in_one_call(st: FP8State, meta: FP8TensorMeta, g, x, w, masks, fmt: str, dynamic: bool):
     """:func:`fp8_linear_backward` as one library call; ``None`` as for the forward."""
-    if not (masks[0] and masks[1] and linear_fp8_takes(x, w, None) and linear_fp8_takes(g, w, None)
-            and g.size(-1) == w.size(0) and x.size(-1) == w.size(1)
+    if not (masks[0] and masks[1] and linear_fp8_takes(x, w, None) and linear_fp8_takes(g, w, None, 0)
             and x.numel() // w.size(1) == g.numel() // w.size(0) <= 65535 * 128):
         return None
     if dynamic:

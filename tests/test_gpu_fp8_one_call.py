@@ -70,6 +70,11 @@ def test_operands_that_are_left_to_the_general_path():
     assert not linear_fp8_takes(_mk(1, 8, 250), _mk(2, 64, 250), None)
     for bad in (_mk(3, 64).float(), _mk(3, 1, 64), _mk(3, 128)[::2]):
         assert not linear_fp8_takes(x, w, bad)
+    for recipe in (fp8.DynamicScaling(), fp8.DelayedScaling()):   # rows of another width: refused, as by the general path
+        for bad in (_mk(1, 8, 512), _mk(1, 8, 128)):
+            assert not linear_fp8_takes(bad, w, None)
+            with torch.no_grad(), fp8.fp8_autocast(True, recipe=recipe), pytest.raises(RuntimeError):
+                fp8.fp8_linear_forward(bad, w, None, True)
 
 
 def test_infinities_and_nan_reach_the_step_alike(monkeypatch):

@@ -290,3 +290,27 @@ def test_weight_side_padding_is_made_once_and_follows_writes():
     assert len(_cabi._padded_weights) <= n
     small, ws, ks = _cabi._pad_k(a[:2, :40], a[:3, :40])        # too small to repay a copy
     assert ks == 40 and small.shape == (2, 40)
+
+
+def test_one_call_fp8_linear_refuses_rows_of_another_width(monkeypatch):
+    """Rows are counted by the element, so rows as wide as another weight's would be written past the output, or leave
+    half of it unwritten."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from astrai_amd.extension import _cabi
+
+    monkeypatch.setattr(_cabi, "_plain_bf16", lambda t, dev: True)   # (addresses: fake tensors have none)
+    with FakeTensorMode():
+        mk = lambda *s: torch.empty(*s, device="cuda", dtype=torch.bfloat16)
+        w, g = mk(64, 256), mk(8, 64)
+        assert _cabi.linear_fp8_operands(mk(8, 256), w) and _cabi.linear_fp8_operands(g, w, None, 0)
+        for bad in (mk(8, 512), mk(8, 64), mk(8, 128)):
+            assert not _cabi.linear_fp8_operands(bad, w)
+        assert not _cabi.linear_fp8_operands(mk(8, 256), w, None, 0)
+        assert not _cabi.linear_fp8_operands(mk(8, 64), mk(64), None, 0) and not _cabi.linear_fp8_operands(mk(8, 1), mk(4, 16, 1))
+    x, w, g = (torch.zeros(*s, dtype=torch.bfloat16) for s in ((8, 512), (64, 256), (16, 64)))
+    with pytest.raises(RuntimeError, match="inner dim mismatch"):
+        _cabi.linear_fp8(x, w, None, None, (None, None), (None, None), 0, 448.0, 1.0)
+    for gb, xb in ((g, x), (g[:8, :32], x[:, :256]), (g, x[:, :256])):
+        with pytest.raises(RuntimeError, match="shape mismatch"):
+            _cabi.linear_fp8_backward(gb, xb, w, False, None, None, 0, 448.0, 1.0)
