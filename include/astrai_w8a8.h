@@ -560,6 +560,9 @@ int astrai_w8a8_gemm_fp8_ptpc(const void* a8, const void* b8, const float* sa,
  * Pre-quantized e4m3fn GEMM with 128-block scales. No counterpart in the
  * reference. K must be a multiple of 128.
  *   out[m,n] = bf16( sum_kb (sum_{k in kb} a8[m,k]*b8[n,k]) * sa[m,kb] * sb[n/128,kb] + bias[n] )
+ * Steps may be of either sign; a NaN one makes its outputs NaN. Steps between 1e-15 and 1e15 in magnitude are taken as they
+ * are; on large tiles smaller ones, zeros among them, count as 1e-15 of their sign (the quantizers above give none below
+ * 2.2e-15), and sums past 3e38 times the smallest product of two steps of their row overflow.
  * At most 64 rows of `a8` with K % 256 == 0 (decode steps) run on the weight-streaming row-range
  * kernel, as the per-tensor decode shapes do.
  */

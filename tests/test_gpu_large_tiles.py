@@ -63,6 +63,38 @@ def test_block_scales_against_float64(m, n, k):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + k * 2.0 ** -23 * weight).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(1100, 4096, 512), (2570, 2056, 384), (4300, 4096, 256), (4096, 4096, 640)])
+def test_block_steps_of_any_sign_and_size(m, n, k):
+    """Negative, zero and NaN steps, steps as small as the quantizers give, and all of them beside ordinary ones in a row."""
+    from astrai_amd.extension import _cabi
+    g = torch.Generator(device=DEV).manual_seed(m)
+    a, b = (torch.randn(r, k, generator=g, device=DEV).to(torch.float8_e4m3fn) for r in (m, n))
+    sa = (torch.rand(m, k // 128, generator=g, device=DEV) + 0.5) * 1e-2
+    sb = (torch.rand(-(-n // 128), k // 128, generator=g, device=DEV) + 0.5) * 1e-2
+    least = 1e-12 / 448
+    sa[::3] *= -1
+    sb[1] *= -1
+    sa[5::7, 0] = sa[6::7, -1] = least     # in front of and behind ordinary steps,
+    sa[8::16] = least                      # in whole rows,
+    sb[2] = sb[-1, 0] = least              # and with the weights'
+    sa[9::32, 1] = 0.0
+    nan_rows, nan_block = slice(10, None, 64), 3
+    sa[nan_rows, 1] = sb[nan_block, 0] = float("nan")
+    cols = torch.arange(n, device=DEV) // 128
+    xd = a.double().reshape(m, -1, 128) * sa.double()[:, :, None]
+    wd = b.double().reshape(n, -1, 128) * sb.double()[cols][:, :, None]
+    xd, wd = xd.reshape(m, k), wd.reshape(n, k)
+    want, weight = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    got = _cabi.mm_fp8_block128(a, b, sa, sb).double()
+    nan = torch.zeros(m, n, device=DEV, dtype=torch.bool)
+    nan[nan_rows], nan[:, cols == nan_block] = True, True
+    assert torch.equal(got.isnan(), nan)
+    # (a zero step counts as 1e-15, the others are at most 0.015, codes of 448)
+    slack = 2.0 ** -8 * want.abs() + k * 2.0 ** -23 * weight + (k // 128) * 1.5e-17 * 128 * 448.0 ** 2 * (sa == 0).any(1, keepdim=True)
+    assert (((got - want).abs() <= slack) | nan).all()
+    assert (got[8] != 0).any() and (got[8, cols == 2].abs().max() < 1e-20)
+
+
 @pytest.mark.parametrize("m,n", [(185, 9000), (1500, 1536), (2048, 2040), (1300, 3072)])
 @pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 896])
 def test_128_tiles_of_one_and_of_two_workgroups_a_unit(m, n, k):
