@@ -286,6 +286,10 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
     return check_launch("few_rows_linear");
 }
 
+int astrai_mix_prompt_linear_takes(int64_t m, int64_t n, int64_t k, int64_t ldx, int act) {
+    return prompt_linear_supported(m, n, k, ldx, act >= 0);
+}
+
 int astrai_mix_prompt_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m, int64_t n,
                              int64_t k, int act, void* stream) {
     MIX_TRY(check_ptrs("prompt_linear", x, w, (const void*)out));

@@ -118,8 +118,10 @@ void launch_inst(const PromptLinearArgs& a, hipStream_t stream) {
 
 bool prompt_linear_supported(int64_t m, int64_t n, int64_t k, int64_t ldx, bool act) {
     constexpr int64_t kMost = (int64_t)1 << 31;   // bytes that the descriptors' offsets reach
-    return m > 0 && n > 0 && n % 8 == 0 && k > 0 && k % kSlab == 0 && ldx >= k && ldx % 8 == 0 &&
-           (m + Cfg::BM) * ldx * 2 < kMost && (n + Cfg::BN) * k * (act ? 4 : 2) < kMost && n * 2 * Cfg::BM < kMost;
+    if (m <= 0 || n <= 0 || k <= 0 || m >= kMost || n >= kMost || k >= kMost || ldx >= kMost) return false;
+    const int64_t rows = (act ? 2 : 1) * n;       // of the weight
+    return n % 8 == 0 && k % kSlab == 0 && ldx >= k && ldx % 8 == 0 && (m + Cfg::BM) * ldx < kMost / 2 &&
+           (rows + Cfg::BN) * k < kMost / 2 && n * 2 * Cfg::BM < kMost;
 }
 
 bool launch_prompt_linear(const PromptLinearArgs& a, int act, hipStream_t stream) {

@@ -41,6 +41,7 @@ PROTOTYPES = {
         [_P, _I64, _P, _I64, _F32, _P, _P, _I64] + [_P] * 4 + [_I64, _I64, _F32, _INT, _INT, _P], _INT),
     "astrai_mix_act_mul": ([_P, _P, _I64, _I64, _INT, _INT, _P], _INT),
     "astrai_mix_few_rows_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _INT, _P], _INT),
+    "astrai_mix_prompt_linear_takes": ([_I64] * 4 + [_INT], _INT),
     "astrai_mix_prompt_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _P], _INT),
     "astrai_mix_head_gated_rms_norm": ([_P, _P, _I64, _P, _P] + [_I64] * 4 + [_F32, _INT, _P], _INT),
     "astrai_mix_gated_rms_norm": ([_P, _P, _I64, _P, _P, _I64, _I64, _I64, _F32, _INT, _P], _INT),
@@ -288,10 +289,10 @@ def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
 def prompt_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                             act: Optional[str] = None) -> bool:
     """The calls :func:`prompt_linear` takes: bf16 on one GPU, any number of rows of ``x [.., k]`` at 16-byte boundaries,
-    ``k`` a multiple of 64, the outputs of 8, operands under 2 GiB each."""
+    ``k`` a multiple of 64, the outputs of 8, operands under 2 GiB each (the library says which sizes)."""
     n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
     rows = x.numel() // k if k else 0
-    if x.size(-1) != k or rows <= 0 or k % 64 or n % 8 or (weight.size(0) + 256) * k * 2 >= 2 ** 31 or n >= 2 ** 22:
+    if x.size(-1) != k or rows <= 0 or k % 64 or n % 8:
         return False
     if not (x.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and weight.device == x.device):
         return False
@@ -302,7 +303,8 @@ def prompt_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optiona
         return False
     if not (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k)):
         return False
-    return (rows + 256) * (k if x.is_contiguous() else x.stride(0)) * 2 < 2 ** 31
+    return bool(_require().astrai_mix_prompt_linear_takes(rows, n, k, k if x.is_contiguous() else x.stride(0),
+                                                          -1 if act is None else ACTIVATIONS[act]))
 
 
 def prompt_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,

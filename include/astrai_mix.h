@@ -76,8 +76,9 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
 
 /*
  * The same of a prompt's rows, on 256 x 256 tiles, bf16 out; k % 64 == 0, n % 8 == 0, x, w and 256 rows of out each under
- * 2 GiB. The sums run in one order whatever m is.
+ * 2 GiB (x and w with 256 rows more). The sums run in one order whatever m is. _takes: whether it takes these sizes.
  */
+int astrai_mix_prompt_linear_takes(int64_t m, int64_t n, int64_t k, int64_t ldx, int act);
 int astrai_mix_prompt_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* out, int64_t m, int64_t n,
                              int64_t k, int act, void* stream);
 

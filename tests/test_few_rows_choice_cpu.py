@@ -169,3 +169,19 @@ def test_prompt_sizes_at_which_the_tiles_are_the_faster_ones(monkeypatch, m, n, 
         assert mixers.prompt_rows(x, w, act=act) == taken
     w = torch.zeros(1).expand(n, 2048).requires_grad_(True)
     assert not mixers.prompt_rows(x, w, act=act)
+
+
+def test_a_prompts_products_are_taken_up_to_the_descriptors_reach():
+    """Weights whose offsets stay below 2 GiB: gate and up of 32512 from 16384 values do, with 256 rows to spare."""
+    lib = _mix.load()
+    assert lib is not None, _mix.load_error()
+    takes = lambda n, k, act, m=4096, ldx=None: bool(lib.astrai_mix_prompt_linear_takes(m, n, k, ldx or k, act))
+    for n, k in ((32512, 16384), (65280, 8192), (32632, 16384)):
+        assert takes(n, k, 0) and takes(n, k, 1) and takes(2 * n, k, -1), (n, k)
+        assert (2 * n + 256) * k * 2 < 2 ** 31
+    assert not takes(32640, 16384, 0) and not takes(65280, 16384, -1)
+    assert not takes(2 ** 22, 64, -1) and takes(2 ** 22 - 8, 64, -1)
+    assert takes(64, 16384, -1, 2 ** 16 - 257) and not takes(64, 16384, -1, 2 ** 16 - 256)
+    assert not takes(64, 64, -1, 2 ** 40) and not takes(64, 2 ** 40, -1) and not takes(2 ** 40, 64, -1)
+    assert not takes(60, 64, -1) and not takes(64, 96, -1) and not takes(64, 128, -1, ldx=120) and not takes(64, 128, -1, ldx=132)
+    assert not takes(64, 64, -1, 0)
