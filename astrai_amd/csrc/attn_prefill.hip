@@ -31,9 +31,9 @@
 // for an exponential); what exceeds that in one slot delays the next MFMA and what is left unused in another is lost: 16
 // slots of 20 cycles take 536, eight of 44 and eight empty ones 640. Row maxima of tile T+1 go behind the last MFMAs,
 // the question whether one has outgrown its reference into the next step. Keys and values arrive by direct-to-LDS
-// loads into two rings of four tiles, values two tiles behind the keys, one 64-key block ahead, one load to every second
-// MFMA of a block's first step (all at once they stall the waves that issue them); one workgroup barrier per block; no
-// staging registers. Dense loads keep their lane's offset, the descriptors move along instead; the loop over unmasked
+// loads into two rings of four tiles, values two tiles behind the keys, one 64-key block ahead (the first three tiles of
+// both at once), one load to every second MFMA of a block's first step (all at once they stall the waves that issue
+// them); one workgroup barrier per block; no staging registers. Dense loads keep their lane's offset, the descriptors move along instead; the loop over unmasked
 // blocks goes once round the rings, so that its LDS offsets are constants. Tiles that every query of the wave sees whole
 // skip the masking code; the accumulators are rescaled only when a row maximum has outgrown the reference maximum by 2^8.
 //
@@ -48,8 +48,9 @@
 // Counters of 4 x 2048 tokens: matrix pipe and vector ALU busy 58% of the SIMD cycles each (48 and 53 before).
 // Measured (graph replays): 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 75 us (915 TFLOP/s), ragged
 // 16 x 175..700 tokens of 32/8 heads x 64 in a pool 75.7 us (P in two terms); with the exponentials behind the score
-// MFMAs alone, the loads in a burst and offsets formed for each (120 vector instructions a tile) 80.3 and 78.2. Up to 236 /
-// 170 registers: two / three workgroups per CU. 64 query tokens a workgroup halve the loads, but couple eight waves:
+// MFMAs alone, the loads in a burst and offsets formed for each (120 vector instructions a tile) 80.3 and 78.2. Prompts of up
+// to 100 tokens were 0.2 to 0.3 us faster that way (8 x 100, 32/8 heads x 64: 6.8 and 7.15). Up to 238 /
+// 168 registers: two / three workgroups per CU. 64 query tokens a workgroup halve the loads, but couple eight waves:
 // 2 x 4096 126 us (133 here, same run), 4 x 2048 74 (74), 16 x 1024 89 (85), 1 x 4096 93 (76), 32 x 512 64.5 (58); not kept.
 #include <algorithm>
 #include <climits>
@@ -87,7 +88,7 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 // what may be attended on top of the causal range (csrc/kernels/attention/mma_utils.cuh:190-199);
 // every tile then takes the masking path.
 template <int D, int NREP, int QSUB, bool PAGED, bool MASK, bool SPLIT>
-__global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void attn_prefill_kernel(AttnPrefillArgs a) {
+__global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && NREP * QSUB == 4 ? 3 : 2) void attn_prefill_kernel(AttnPrefillArgs a) {
     constexpr int WAVES = NREP * QSUB;
     constexpr int QB = 32 * QSUB;                 // query tokens per workgroup
     constexpr int ROW = 2 * D;                    // bytes per key or value row in LDS
@@ -249,22 +250,28 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         const int inst = wave * DMA + j;
         lds_dma16<false>(rk, lds0 + ((t0 + inst / TI) & 3) * TILE + (inst % TI) * 1024, off);
     };
-    auto dma_k_all = [&](int t0, uint32_t rows) {
-#pragma unroll
-        for (int j = 0; j < DMA; ++j) dma_k(j, t0, k_off(j, rows));
+    // The first three tiles, keys and values alike: load i of the workgroup's is rows i * RPI .. of them, and wave i % WAVES's
+    constexpr int I3 = 3 * TI, T3 = (I3 + WAVES - 1) / WAVES;
+    [[maybe_unused]] uint32_t start_rows = 0;
+    auto start_load = [&](const u32x4& desc, int ring, int t, uint32_t stride, auto swz) __attribute__((always_inline)) {
+        const int i = wave + t * WAVES, row = i * RPI + lane / LPR;
+        if (I3 % WAVES && i >= I3) return;
+        const uint32_t chunk = (uint32_t)(((lane & (LPR - 1)) ^ swz(row)) << 4);
+        uint32_t off;
+        if constexpr (PAGED) off = (uint32_t)__builtin_amdgcn_ds_bpermute((t * RPI + lane / LPR) << 2, (int)start_rows) + chunk;
+        else off = (uint32_t)min((uint64_t)row * stride + chunk, (uint64_t)kMissing);
+        lds_dma16<false>(desc, lds0 + ring + i * 1024, off);
     };
     [[maybe_unused]] int slots = 0;
     if constexpr (PAGED) {
-        const int first = lookup(0, 0);
-        slots = lookup(1, -1);  // key tiles 1, 2 and value tiles -1, 0
-        dma_k_all(0, rows_of(first));
-        dma_k_all(1, rows_of(slots));
-    } else {
-        dma_k_all(0, 0);
-        advance(rk, (uint64_t)k_row * 32);
-        dma_k_all(1, 0);
-        advance(rk, (uint64_t)k_row * 64);  // the first block's: tiles 3, 4
+        const int key = (wave + lane / RPI * WAVES) * RPI + lane % RPI;
+        const int first = (key < 96 && key <= kmax) ? table[key] : -1;
+        slots = lookup(3, 1);  // what the first block's loads will ask for
+        start_rows = rows_of(first);
     }
+#pragma unroll
+    for (int t = 0; t < T3; ++t) start_load(rk, 0, t, k_row, swz_k);
+    if constexpr (!PAGED) advance(rk, (uint64_t)k_row * 96);
 
     if constexpr (!PAGED) {
         if (a.positions) {
@@ -397,6 +404,20 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         return m;
     };
 
+    // the same of a whole tile, chosen at run time (65 vector instructions more if some score may be hidden)
+    const int tfull = (pmin + 1) / 32;  // tiles every query of the wave sees whole
+    auto tile_max = [&](int T, f32x16& s) __attribute__((always_inline)) -> float {
+        float m = kNegBig;
+        if (!MASK && T < tfull) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) m = mask_max4(std::false_type{}, T, s, g, m);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) m = mask_max4(std::true_type{}, T, s, g, m);
+        }
+        return max_halves(m);
+    };
+
     constexpr int NV = 2 * DT;                 // value operands of a tile
     constexpr int NM = NV * (SPLIT ? 2 : 1);   // P.V MFMAs
     constexpr int NS = KS + NM;                // slots (MFMAs) of a step
@@ -406,6 +427,24 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     struct Probs {
         uint32_t hi[8];
         uint32_t lo[SPLIT ? 8 : 1];
+    };
+    // element e of P; the even one of a pair waits in `even` for the odd one
+    auto prob = [&](int e, const f32x16& s, Probs& out, float& even, float& l_add) __attribute__((always_inline)) {
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], c, -m_run));
+        __asm__ volatile("" : "+v"(p));  // here: its uses are a step away, and the compiler would move it there
+        if ((e & 1) == 0) {
+            even = p;
+            return;
+        }
+        l_add += even + p;
+        uint32_t hi = pack_bf16x2(even, p);
+        __asm__ volatile("" : "+v"(hi), "+v"(l_add));
+        out.hi[e >> 1] = hi;
+        if constexpr (SPLIT) {
+            uint32_t lo = pack_bf16x2(even - __uint_as_float(hi << 16), p - __uint_as_float(hi & 0xffff0000u));
+            __asm__ volatile("" : "+v"(lo));
+            out.lo[e >> 1] = lo;
+        }
     };
     auto pv = [&](const Probs& p, int n, u32x4 (&vf)[NV]) __attribute__((always_inline)) {
         const int i = SPLIT ? n >> 1 : n, t = i / DT, dt = i % DT;
@@ -424,12 +463,12 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
     // One step: the scores of tile T+1, P of tile T, and P.V of tile T-1, the exponentials spread evenly over all of
     // its MFMAs. In: s_in = raw (masked) scores of tile T; grow_in: some row's maximum m_in (both lane halves) has
     // outgrown the reference. Out: p_out = P of tile T; s_out, m_out, grow_out the same for tile T+1.
-    // first_tag: a block's first step, which issues its loads (K tiles T+3, T+4, V tiles T+1, T+2), and reads the
-    // second step's first key operands.
+    // first_tag: 1: a block's first step, which issues its loads (K tiles T+3, T+4, V tiles T+1, T+2), and reads the
+    // second step's first key operands; 2: a second one that chooses at run time whether the scores are masked.
     auto step = [&](auto mask_tag, auto ring_tag, auto first_tag, int T, f32x16& s_in, float m_in, bool grow_in, f32x16& s_out,
                     float& m_out, bool& grow_out, const Probs& p_in, Probs& p_out, u32x4 (&kf)[KS])
                     __attribute__((always_inline)) {
-        constexpr bool FIRST = decltype(first_tag)::value;
+        constexpr bool FIRST = decltype(first_tag)::value == 1, CHOOSE = decltype(first_tag)::value == 2;
         constexpr int RING0 = decltype(ring_tag)::value;  // ring slot of the block's first tile; -1: from T
         constexpr int AT = RING0 + (FIRST ? 0 : 1);
         auto slot_of = [&](int d) { return RING0 >= 0 ? (AT + d + 4) & 3 : (T + d) & 3; };
@@ -443,7 +482,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             l_run *= alpha;
         }
         const int kt = slot_of(1) * TILE, vt = RING + slot_of(-1) * TILE;
-        float l_add = 0.0f, e0 = 0.0f, e1 = 0.0f, m = kNegBig;
+        float l_add = 0.0f, e0 = 0.0f, m = kNegBig;
         u32x4 vf[NV];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -476,28 +515,17 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             // exponentials: element e behind MFMA e * NS / 16
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                if (n == e * NS / 16) {
-                    float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[e], c, -m_run));
-                    __asm__ volatile("" : "+v"(p));  // here: its uses are a step away, and the compiler would move it there
-                    if ((e & 1) == 0) {
-                        e0 = p;
-                    } else {
-                        e1 = p;
-                        l_add += e0 + e1;
-                        uint32_t hi = pack_bf16x2(e0, e1);
-                        __asm__ volatile("" : "+v"(hi), "+v"(l_add));
-                        p_out.hi[e >> 1] = hi;
-                        if constexpr (SPLIT) {
-                            uint32_t lo = pack_bf16x2(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xffff0000u));
-                            __asm__ volatile("" : "+v"(lo));
-                            p_out.lo[e >> 1] = lo;
-                        }
-                    }
-                }
-            if (n >= NS - 6 && n < NS - 2) m = mask_max4(mask_tag, T + 1, s_out, n - (NS - 6), m);
-            if (n == NS - 2) m_out = max_halves(m);
-            if (n == NS - 1) grow_out = __any(m_out * c > m_lim);
+                if (n == e * NS / 16) prob(e, s_in, p_out, e0, l_add);
+            if constexpr (!CHOOSE) {
+                if (n >= NS - 6 && n < NS - 2) m = mask_max4(mask_tag, T + 1, s_out, n - (NS - 6), m);
+                if (n == NS - 2) m_out = max_halves(m);
+                if (n == NS - 1) grow_out = __any(m_out * c > m_lim);
+            }
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (CHOOSE) {
+            m_out = tile_max(T + 1, s_out);
+            grow_out = __any(m_out * c > m_lim);
         }
         l_run += l_add;
         if (__builtin_expect(grow_in, 0)) {  // P.V of tile T-1 was still against the old reference
@@ -508,26 +536,14 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         }
     };
 
-    // ---- prologue: key tiles 0..2, value tiles -1 (zeros) and 0; scores of tile 0
-    const int tfull = (pmin + 1) / 32;  // tiles every query of the wave sees whole
+    // ---- prologue: key tiles 0..2, value tiles 0..2; scores of tile 0
     const int nfast = MASK ? 0 : min(max(tfull - 1, 0), tiles_w) / 2;  // blocks whose steps only produce unmasked tiles
 #pragma unroll
-    for (int j = 0; j < DMA; ++j) {
-        uint32_t off;
-        if constexpr (PAGED) {
-            off = v_off(j, rows_of(slots));
-        } else {
-            const int row = (wave * DMA + j) * RPI + lane / LPR;
-            off = row < 32 ? kMissing
-                           : (uint32_t)min((uint64_t)(row - 32) * v_row + (((lane & (LPR - 1)) ^ swz_v(row)) << 4), (uint64_t)kMissing);
-        }
-        dma_v(j, -1, off);
-    }
-    if constexpr (!PAGED) advance(rv, (uint64_t)v_row * 32);  // the first block's: tiles 1, 2
-    if constexpr (PAGED) slots = lookup(3, 1);  // what the first block's loads will ask for
-    // tile 0 needs the queries and the key tiles, not the values: wait for everything but
-    // this wave's DMA value loads (the newest), which get the scores of tile 0 to land
-    __builtin_amdgcn_s_waitcnt(0x0f70 | DMA);  // vmcnt(DMA)
+    for (int t = 0; t < T3; ++t) start_load(rv, RING, t, v_row, swz_v);
+    if constexpr (!PAGED) advance(rv, (uint64_t)v_row * 32);  // (the first block moves it on to tile 3)
+    // the scores need the queries and the key tiles, not the values, the newest of this wave's loads
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (I3 / WAVES));  // vmcnt(I3 / WAVES)
+    static_assert(I3 / WAVES < 16, "vmcnt's low bits");
     __syncthreads();
     f32x16 sa, sb;
     float ma, mb;
@@ -539,21 +555,15 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
             sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8, k_frag(0, ks)), __builtin_bit_cast(bf16x8, qf[ks]),
                 ks == 0 ? zero16 : sa, 0, 0, 0);
-        float m = kNegBig;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) m = mask_max4(std::true_type{}, 0, sa, g, m);
-        ma = max_halves(m);
+        ma = tile_max(0, sa);
         ga = __any(ma * c > m_lim);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pb.hi[i] = 0;
-#pragma unroll
-        for (int i = 0; i < (SPLIT ? 8 : 1); ++i) pb.lo[i] = 0;
     }
-    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-    __syncthreads();  // values landed; tile 0's ring slot is overwritten by the first block's loads
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __syncthreads();  // tile 0's ring slot is overwritten by the first block's loads
     u32x4 kf[KS];
     k_first(1, kf);
-    auto begin_block = [&]([[maybe_unused]] int kb) {
+    auto begin_block = [&](int kb) {
+        if (kb + 1 >= nkb) rk.z = 0;  // nobody is left to read them (paged: no such slots)
         if constexpr (PAGED) {
 #pragma unroll
             for (int j = 0; j < DMA; ++j) k_at[j] = k_off(j, rows_of(slots)), v_at[j] = v_off(j, rows_of(slots));
@@ -576,12 +586,6 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
         step(mask_tag, ring_tag, std::false_type{}, 2 * kb + 1, sb, mb, gb, sa, ma, ga, pa, pb, kf);
         end_block(R >= 0 ? R + 3 : 2 * kb + 3);
     };
-    int kb = 0;
-    for (; kb + 1 < nfast; kb += 2) {  // two blocks: once round the rings, so that every LDS offset is a constant
-        block(std::false_type{}, std::integral_constant<int, 0>{}, kb);
-        block(std::false_type{}, std::integral_constant<int, 2>{}, kb + 1);
-    }
-    for (; kb < tiles_w / 2; ++kb) block(std::true_type{}, std::integral_constant<int, -1>{}, kb);
     auto last_pv = [&](const Probs& p) __attribute__((always_inline)) {
         const int vt = RING + ((tiles_w - 1) & 3) * TILE;
         u32x4 vf[NV];
@@ -590,14 +594,67 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB >= 4 ? 2 : 1) void at
 #pragma unroll
         for (int n = 0; n < NM; ++n) pv(p, n, vf);
     };
-    if (tiles_w & 1) {  // a last block of one tile, whose values are there already (the next block's loads replace them)
-        begin_block(kb);
-        step(std::true_type{}, std::integral_constant<int, -1>{}, std::true_type{}, 2 * kb, sa, ma, ga, sb, mb, gb, pb, pa, kf);
-        last_pv(pa);
-        end_block(2 * kb + 3);
-        ++kb;
+    // The first block by itself, which for a short prompt is most of the way: no P.V in its first step, beside which the
+    // first values land; scores of a second tile only if there is one; masked only where some query needs it (as any other
+    // block, behind zeros as value tile -1 and with tile 1's values waited for at the end: 1 x 33 tokens, 16/4 heads x 128,
+    // 6.5 us, here 6.2; 8 x 100, 32/8 x 64, 7.35 and 7.15; 16 x 700 + 500 in a pool, 16/16 x 64, 64 and 61)
+    begin_block(0);
+    if (__builtin_expect(ga, 0)) {
+        m_run = fmaxf(m_run, ma * c);
+        m_lim = m_run + kSlack;
+    }
+    float even = 0.0f;
+    if (tiles_w > 1) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < KS; ++n) {
+            if (n + KD < KS) kf[n + KD] = k_frag(TILE, n + KD);
+            sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(bf16x8, kf[n]), __builtin_bit_cast(bf16x8, qf[n]), n == 0 ? zero16 : sb, 0, 0, 0);
+#pragma unroll
+            for (int l = 0; l < DMA; ++l)
+                if (n == l * KS / DMA) dma_k(l, 3, PAGED ? k_at[l] : k_off(l, 0));
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                if (n == e * KS / 16) prob(e, sa, pa, even, l_run);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        k_first(2, kf);
+        mb = tile_max(1, sb);
+        gb = __any(mb * c > m_lim);
     } else {
-        last_pv(pb);
+#pragma unroll
+        for (int l = 0; l < DMA; ++l) dma_k(l, 3, PAGED ? k_at[l] : k_off(l, 0));
+#pragma unroll
+        for (int e = 0; e < 16; ++e) prob(e, sa, pa, even, l_run);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70 | DMA);  // vmcnt(DMA): the values (its key loads are newer)
+    __syncthreads();
+    if (tiles_w > 1)
+        step(std::true_type{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{}, 1, sb, mb, gb, sa, ma, ga, pa, pb, kf);
+    else
+        last_pv(pa);
+    end_block(3);
+    int kb = 1;
+    for (; kb + 1 < nfast; kb += 2) {  // two blocks: once round the rings, so that every LDS offset is a constant
+        block(std::false_type{}, std::integral_constant<int, 2>{}, kb);
+        block(std::false_type{}, std::integral_constant<int, 0>{}, kb + 1);
+    }
+    if (kb < nfast) {
+        block(std::false_type{}, std::integral_constant<int, -1>{}, kb);
+        ++kb;
+    }
+    for (; kb < tiles_w / 2; ++kb) block(std::true_type{}, std::integral_constant<int, -1>{}, kb);
+    if (tiles_w > 1) {
+        if (tiles_w & 1) {  // a last block of one tile, whose values are there already (the next block's loads replace them)
+            begin_block(kb);
+            step(std::true_type{}, std::integral_constant<int, -1>{}, std::true_type{}, 2 * kb, sa, ma, ga, sb, mb, gb, pb, pa, kf);
+            last_pv(pa);
+            end_block(2 * kb + 3);
+            ++kb;
+        } else {
+            last_pv(pb);
+        }
     }
     for (; kb < nkb; ++kb) {  // keys that only later tokens of the workgroup see
         begin_block(kb);
