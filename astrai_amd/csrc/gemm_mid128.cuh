@@ -27,10 +27,12 @@ struct Mid128Cfg {
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it. An instance of its own: chosen
 // in the epilogue, it cost every per-tensor product 0.2 us (354 x 11008 x 4096: 34.3 -> 34.6).
 // S: LDS stages. 2: as above. 4: for launches of one workgroup per compute unit at most, where nobody covers its waits (1500
-// cycles a slab, against 300 of MFMAs): a ring filled four slabs ahead, one barrier per slab, the fragments of slab k + 1
+// cycles a slab, against 512 of MFMAs): a ring filled four slabs ahead, one barrier per slab, the fragments of slab k + 1
 // read into a second register set beside the MFMAs of slab k; 1050 cycles a slab, bound by LDS (96 KiB of fragments, 32 KiB of
 // loads). int8 / fp8, us: 256 x 11264 x 2048 14.7 / 14.2 -> 13.1 / 12.6, 640 x 4096 x 4096 22.8 / 22.5 -> 20.5 / 18.7, 130 x 11008
 // x 4096 22.4 / 23.7 -> 18.7 / 18.4, 600 x 4096 x 11008 49.2 / 49.4 -> 43.9 / 39.9; 2048^3 (256 tiles) 16.0 / 15.1 either way.
+// Up to four slabs the ring is filled once, and its larger prologue is a loss (600 x 4096 x 256 6.9 / 6.4 -> 7.3 / 7.0, x 512
+// 7.9 / 7.5 -> 8.1 / 7.75; x 640 the first where it is none): two stages.
 template <class Op, int ScaleKind, bool RoundFirst, int S>
 __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid128_kernel(GemmArgs g) {
     using Cfg = Mid128Cfg;
@@ -307,7 +309,7 @@ inline void launch_mid128(const GemmArgs& g, hipStream_t stream) {
         if (g.round_first) return launch_mid128<Op, ScaleKind, true>(g, stream);
     const int tiles = ((g.m + Cfg::BM - 1) / Cfg::BM) * ((g.n + Cfg::BN - 1) / Cfg::BN);
     if constexpr (S == 2 && ScaleKind != SCALE_BLOCK128)
-        if (tiles <= 256) return launch_mid128<Op, ScaleKind, RoundFirst, 4>(g, stream);
+        if (tiles <= 256 && g.k > 512) return launch_mid128<Op, ScaleKind, RoundFirst, 4>(g, stream);
     constexpr int lds_bytes = S * Cfg::STAGE_BYTES;
     auto kern = gemm_mid128_kernel<Op, ScaleKind, RoundFirst, S>;
     static std::atomic<uint64_t> lds_allowed{0};

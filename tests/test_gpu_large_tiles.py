@@ -96,9 +96,9 @@ def test_block_steps_of_any_sign_and_size(m, n, k):
 
 
 @pytest.mark.parametrize("m,n", [(185, 9000), (1500, 1536), (2048, 2040), (1300, 3072)])
-@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 896])
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 768, 896, 1024])
 def test_128_tiles_of_one_and_of_two_workgroups_a_unit(m, n, k):
-    """Fewer slabs than LDS stages, as many, odd and even numbers of them; one workgroup to a compute unit and more."""
+    """One to eight slabs, on two LDS stages and on four; one workgroup to a compute unit and more."""
     from astrai_amd.extension import _cabi
     a, b = _codes(m, m, k), _codes(n, n, k)
     g = torch.Generator(device=DEV).manual_seed(1)
