@@ -14,17 +14,18 @@ namespace w8a8 {
 namespace {
 
 // Tiles of 256 x 256 where they fill most of the chip, or where 128 x 128 tiles would put a second workgroup on compute
-// units (from 257 of them), which takes nearly twice as long as one (7168 -> 2048: 1900 tokens, 240 tiles, 69 us with the
-// quantizer, 2300, 288, 105), where a round of large tiles costs little more than the first: 86 us at 2300 tokens, 92 at
-// 4096 (113), 4096 -> 4096 54 at 1100 (63) and 56 at 2500 (93), 2048 -> 7168 36 at 1500 (53).
+// units (from 257 of them), which takes nearly twice as long as one, where a round of large tiles costs little more than the
+// first (us, 128 x 128 / large: 1100 x 4096 x 4096, 288 tiles, 56 / 43, x 512 12.7 / 11.4; 2300 x 2048 x 7168 97 / 71; 900 x
+// 7168 x 2048, 448 tiles, 32 / 26. Only 264 tiles whose last rows are nearly empty end sooner: 257 x 11264 x 2048 22 / 25).
 bool large_tiles_take(const GemmArgs& g) {
     if ((g.n & 7) != 0 || g.out_kind != OUT_BF16) return false;
     return pingpong_shape_ok(g) || (g.k >= 256 && (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 256);
 }
 
-// Tails on smaller tiles as in tile_tail_rows, up to the same number: 4300 x 7168 x 2048 158 -> 94 us (32 tiles), 4300 x 4096 x
-// 4096 117 -> 89 (64), 5000 x 4096 x 4096 120 -> 113 (256); 3001 x 2048 x 7168 68 -> 74 (336), not taken.
-constexpr int64_t kBlockTailTiles = 256;
+// Tails on smaller tiles as in tile_tail_rows (one launch / two; tiles of the tail): 4300 x 4096 x 4096 102 / 79 us (64), x 256
+// 19.8 / 17.5; 4500 x 4096 x 4096 101 / 86 (128); 4700 101 / 98 (192), x 256 19.6 / 19.9; 5000 x 4096 x 256 (256) 19.9 / 21.8, x
+// 1024 36.3 / 37.1, x 7168 166 / 165: not taken.
+constexpr int64_t kBlockTailTiles = 192;
 
 }  // namespace
 
