@@ -21,7 +21,8 @@
 //  * Loads of rows and tokens that are not there are left out, and those past a wave's last item: each costs the
 //    load path of the compute unit 16 cycles. int8 2048 -> 2048 4.62 -> 4.28 us (32 tokens), 6.1 -> 5.2 (64), 5632 -> 2048
 //    10.0 -> 8.9, 4096 -> 4096 9.6 -> 8.3 (64), 11008 -> 4096 13.7 -> 13.3 (32); fp8 7168 -> 2048 15.1 -> 12.7 (96); block
-//    steps 4096 -> 11008 11.5 -> 10.9 (16). One with 2 to 16 tokens -2 to -4%, int8 K = 5632 with 16 tokens 5.62 -> 5.70.
+//    steps 4096 -> 11008 11.5 -> 10.9 (16). 2 to 16 tokens 0 to -4%. With one or two items to a wave nothing is saved: block
+//    steps 1024 -> 1024 3.28 -> 3.36, fp8 1024 -> 12288 6.6 -> 6.8 (48).
 //  * int32 partials of the waves are summed through LDS (integer addition: the split
 //    keeps the accumulator bit-exact), then the dequant epilogue, optionally continued
 //    by rotary embedding and the KV-cache write for a fused q|k|v projection.
@@ -190,9 +191,12 @@ __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCach
             }
         }
     };
-    // The last item requests nothing, in a copy of the body of its own; with all registers taken and more (fp8, 128 tokens of
-    // three row groups) the copy spilled 63 instead of 25, 21.2 -> 23.0 us: there it asks for rows past every end.
+    // The last item requests nothing, in a copy of the body of its own. Where all registers are taken and more (fp8, 97 to
+    // 128 tokens of three row groups) the copy spilled 63 of them, here 25: one body, which asks for rows past every end, behind
+    // no branch (with one: 30, 2048 -> 11264 15.1 -> 15.7 us, -> 32000 38.4 -> 40.1). 65 to 96 tokens: 66 11.7 -> 11.3 by the
+    // copy, 96 12.0 -> 12.3.
     constexpr bool ONE_BODY = !Op::kIsInt && RG * MB >= 24;
+    static_assert(!ONE_BODY || !rows_op_block<Op>::value, "the steps' loads are not told where the items end");
     auto issue = [&](u32x4 (&dst)[4], int item, int s) {
         const bool live = !ONE_BODY || item < i1;
         const uint32_t k0 = (uint32_t)item << 8;
@@ -255,7 +259,7 @@ __device__ __forceinline__ void gemv_rows_body(const GemmArgs& g, const RopeCach
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (i0 < i1) {
+    if (ONE_BODY || i0 < i1) {
 #pragma unroll
         for (int s = 0; s < P; ++s) {
             issue(ring[s], i0, s);
