@@ -91,8 +91,9 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_i8_kernel(Ge
         const __amdgpu_buffer_rsrc_t rout = make_rsrc(dst_base, live_head ? dst_bytes : 0u);
         const int r4 = lane >> 4, c16 = lane & 15;
         // One wave per SIMD: nothing hides a memory round trip inside the epilogue, so everything
-        // it reads is requested ahead of its use -- the destinations of all 32 rows this lane will
-        // store (cache slots: one lookup of the token's position each) now, the (cos, sin) pairs of
+        // it reads is requested ahead of its use -- the destinations of the 8 rows this lane will
+        // store (cache slots: one lookup of the token's position each) a pass ahead (those of all four passes at once
+        // spilled 22 registers: 32 x 512 x 512 74.9 us, here 71.7), the (cos, sin) pairs of
         // a group of 32 columns x 16 tokens four groups before the group that uses them.
         // token index -> (sequence, token in sequence) without an integer division per row: the
         // float quotient of m < 2^23 is off by at most one, which the remainder shows
@@ -103,26 +104,27 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_i8_kernel(Ge
             if (sq < 0) { --bt; sq += rc.seq; }
             else if (sq >= rc.seq) { ++bt; sq -= rc.seq; }
         };
-        uint32_t dst_off[4][8];
-#pragma unroll
-        for (int p = 0; p < 4; ++p)
+        uint32_t dst_off[2][8];
+        auto find_rows = [&](int p) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int m = mw + p * 32 + i * 4 + r4;
                 int bt, sq;
                 split_token(m, bt, sq);
-                dst_off[p][i] = kOutOfRange;
+                uint32_t at = kOutOfRange;
                 if (m < g.m) {
                     if (is_q) {
-                        dst_off[p][i] = (uint32_t)((bt * rc.n_heads + hh) * rc.seq + sq) * 256u + (uint32_t)c16 * 16u;
+                        at = (uint32_t)((bt * rc.n_heads + hh) * rc.seq + sq) * 256u + (uint32_t)c16 * 16u;
                     } else {
                         const int64_t pos = rc.positions[sq];
                         if (pos >= 0 && pos < rc.max_len)
-                            dst_off[p][i] = (uint32_t)((int64_t)(bt * rc.n_kv_heads + hk) * rc.max_len + pos) * 256u +
-                                            (uint32_t)c16 * 16u;
+                            at = (uint32_t)((int64_t)(bt * rc.n_kv_heads + hk) * rc.max_len + pos) * 256u + (uint32_t)c16 * 16u;
                     }
                 }
+                dst_off[p & 1][i] = at;
             }
+        };
+        find_rows(0);
         // group gi = mi * 4 + c: the lane's token of sub-tile mi, columns 32 c .. 32 c + 31
         constexpr int kAhead = 4;
         f32x4 cs[kAhead + 1][2];
@@ -144,6 +146,7 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_i8_kernel(Ge
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             uint8_t* const buf = mine + (p & 1) * PASS_BYTES;
+            if (p + 1 < 4) find_rows(p + 1);
 #pragma unroll
             for (int gg = 0; gg < 8; ++gg) {
                 const int gi = p * 8 + gg, mi = gi >> 2;
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_i8_kernel(Ge
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(buf + (i * 4 + r4) * ROWB + c16 * 16);
-                __builtin_amdgcn_raw_buffer_store_b128(v, rout, dst_off[p][i], 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rout, dst_off[p & 1][i], 0, 0);
             }
         }
     } else if constexpr (Epi == EPI_SWIGLU) {
