@@ -56,8 +56,37 @@ def _steps(monkeypatch, general, recipe, shape, n, bias, grads, fmt, cache):
 def test_same_as_the_general_path(monkeypatch, recipe, shape, n, bias, grads, fmt, cache):
     got, calls = _steps(monkeypatch, False, recipe, shape, n, bias, grads, fmt, cache)
     want, none = _steps(monkeypatch, True, recipe, shape, n, bias, grads, fmt, cache)
-    assert all(calls) and calls and not none
+    # four forwards, and behind each (square weights) the input and the gradient of a backward
+    assert all(calls) and len(calls) == (12 if grads and n == shape[-1] else 4) and not none
     for a, b in zip(got, want, strict=True):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("recipe", [lambda: fp8.DelayedScaling(history_len=3, margin=1), fp8.DynamicScaling])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 512), (48, 512, 256), (100, 272, 1024), (130, 1040, 272), (1037, 256, 512)])
+@pytest.mark.parametrize("bias,fmt", [(False, "hybrid"), (True, "hybrid"), (True, "e4m3")])
+def test_backward_of_weights_that_are_not_square(monkeypatch, recipe, m, n, k, bias, fmt):
+    """Called directly: the gradient's handler takes square weights only."""
+    one = {name: getattr(fp8, name) for name in ("_forward_in_one_call", "_backward_in_one_call")}
+    results = []
+    for general in (False, True):
+        fp8.fp8_state().reset()
+        took = []
+        for name, call in one.items():
+            monkeypatch.setattr(fp8, name, lambda *a, call=call: (took.append(None if general else call(*a)), took[-1])[1])
+        w, out = _mk(1, n, k, std=0.02), []
+        with torch.no_grad(), fp8.fp8_autocast(True, recipe=recipe(), fp8_format=fmt):
+            for t in range(4):
+                x, g = _mk(10 + t, m, k, std=1.0 + t), _mk(20 + t, m, n, std=0.01)
+                out.append(fp8.fp8_linear_forward(x, w, None, True))
+                grads = fp8.fp8_linear_backward(g, x, w, [True, True, bias])
+                assert [tuple(t.shape) for t in grads] == [(m, k), (n, k), (n if bias else 0,)]
+                out += grads
+            meta = fp8.fp8_state().peek_weight_meta(w)
+        out += [r for ring in (meta._x, meta._w, meta._g) for r in (ring.hist, ring.scale, torch.tensor(ring.idx))]
+        assert len(took) == 8 and all((r is None) == general for r in took)
+        results.append(out)
+    for a, b in zip(*results, strict=True):
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
 
 
