@@ -69,15 +69,15 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
     if (g.resid) tail.resid = static_cast<const uint8_t*>(g.resid) + row0 * (size_t)g.n * 2;
 }
 
-// Plain bf16 products that the large tiles take: where they fill most of the chip, or from 513 tiles of 128 x 128 on, where
-// those need a third workgroup on some compute units and large tiles (two thirds of the units) cost the same however
-// few they are. Below, two to a unit are the faster ones (us, 128 x 128 / large, int8 and fp8: 3650 x 2048 x 4096, 464 tiles,
-// 38.6 / 39.8 and 35.4 / 37.4; 1900 x 4096 x 4096, 480, 39.5 / 40.0 and 36.7 / 37.7; 512 x 16384 x 11008, 512, fp8 108 / 110).
+// Plain bf16 products that the large tiles take: where they fill most of the chip, or from 449 tiles of 128 x 128 on. Two
+// workgroups of those share a compute unit and take longer the more units have two, where a round of large tiles costs
+// the same however empty (int8, us, 128 x 128 / large: 2048 -> 2048 34 / 34 at 448 tiles, 36 / 34 at 512; 5632 -> 2048
+// 65 / 65 and 71 / 67; 4096 -> 4096 49 / 50 and 53 / 50; 11008 -> 4096 105 / 106 and 117 / 108, 97 / 104 at 384).
 inline bool wave128_takes(const GemmArgs& g) {
     if (wave128_shape_ok(g)) return true;
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 256 || g.out_kind != OUT_BF16 || (g.n & 7) != 0 || g.n > (1 << 22))
         return false;
-    return (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 512;
+    return (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 448;
 }
 
 // Rows of a product that are better served by smaller tiles in a launch of their own: those past the last
