@@ -24,15 +24,15 @@ bool large_tiles_take(const GemmArgs& g) {
 
 // Tails on smaller tiles as in tile_tail_rows (one launch / two; tiles of the tail): 4300 x 4096 x 4096 102 / 79 us (64), x 256
 // 19.8 / 17.5; 4500 x 4096 x 4096 101 / 86 (128); 4700 101 / 98 (192), x 256 19.6 / 19.9; 5000 x 4096 x 256 (256) 19.9 / 21.8, x
-// 1024 36.3 / 37.1, x 7168 166 / 165: not taken.
-constexpr int64_t kBlockTailTiles = 192;
+// 1024 36.3 / 37.1, x 1536 46.1 / 46.1, x 4096 101 / 100, x 11008 249 / 233: more than 192 only with K from 1536 on.
+int64_t block_tail_tiles(const GemmArgs& g) { return g.k >= 1536 ? 256 : 192; }
 
 }  // namespace
 
 bool launch_gemm_fp8_block128_tiled(const GemmArgs& g, hipStream_t stream) {
     if (!tiled_shape_ok(g) || (g.k & 127) != 0) return false;
     if (large_tiles_take(g)) {
-        if (const int r = tile_tail_rows(g, kBlockTailTiles)) {
+        if (const int r = tile_tail_rows(g, block_tail_tiles(g))) {
             GemmArgs head, tail;
             split_rows(g, r, false, head, tail);
             tail.sa = g.sa + (size_t)head.m * (g.k >> 7);   // a step per row and K block

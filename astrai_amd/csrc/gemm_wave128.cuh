@@ -71,8 +71,9 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
 
 // Plain bf16 products that the large tiles take: where they fill most of the chip, or from 449 tiles of 128 x 128 on. Two
 // workgroups of those share a compute unit and take longer the more units have two, where a round of large tiles costs
-// the same however empty (int8, us, 128 x 128 / large: 2048 -> 2048 34 / 34 at 448 tiles, 36 / 34 at 512; 5632 -> 2048
-// 65 / 65 and 71 / 67; 4096 -> 4096 49 / 50 and 53 / 50; 11008 -> 4096 105 / 106 and 117 / 108, 97 / 104 at 384).
+// the same however empty (us, 128 x 128 / large, fp8 and int8: 2048 x 4096 x 512 14.5 / 12.0 and 15.1 / 13.5, x 4096 37.8 / 37.5
+// and 41.2 / 40.1, x 11008 87 / 86 and 96 / 90; 640 x 11776 x 4096, 460 tiles, 43 / 37 and 44 / 40). What it costs: up to 480
+// tiles with K of 2048 to 5632 1 to 5% (1800 x 4096 x 4096 36.5 / 37.9 and 39.5 / 40.2).
 inline bool wave128_takes(const GemmArgs& g) {
     if (wave128_shape_ok(g)) return true;
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 256 || g.out_kind != OUT_BF16 || (g.n & 7) != 0 || g.n > (1 << 22))
