@@ -17,7 +17,8 @@
 //                  Q10 | X0(k+2) -> XA   Q11 | W0(k+2) -> WA
 // Every quadrant has 8 LDS reads of 1 KiB and 4 direct-to-LDS loads between its MFMAs. The order is written out and pinned,
 // so that the MFMA pipe always has the next instruction waiting; the loads are spread evenly, because the CU's one load
-// path takes a 1 KiB instruction every 16 cycles: four waves must not issue them faster than one per 128 cycles each.
+// path takes a 1 KiB instruction every 16 cycles: four waves must not issue them faster than one per 64 cycles each, and have
+// 128 for each of a slab's sixteen.
 // Three activation and two weight stages (all 160 KiB): all of a slab's operands have been read when its second quadrant
 // ends, at the slab's one barrier; the activation rows of slab k+2 are fetched before it (into the stage of slab k-1), the
 // weight rows behind it.
@@ -93,8 +94,7 @@ __device__ __forceinline__ void walk16_offsets(int lane, int first, int live, ui
 
 // acc[weight sub-tile][token sub-tile] of a wave's 128 x 128: lane (lgrp, lrow) = (lane >> 4, lane & 15) holds, for token
 // 16 mi + lrow, weight rows 16 ni + 4 lgrp .. + 3. The stages are free for other use when it returns.
-// (KO: knock-outs, see gemm_wave128.cuh)
-template <class Op, int KO = 0>
+template <class Op>
 __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_bytes, const uint32_t (&x_off)[8],
                                        const void* w, uint32_t w_bytes, const uint32_t (&w_off)[8], int slabs,
                                        typename Op::Acc (&acc)[8][8]) {
@@ -154,25 +154,13 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
         for (int r = 0; r < 8; ++r) dma_x(r, rx1, 1, 128u);
 #pragma unroll
         for (int r = 0; r < 8; ++r) dma_w(r, rw1, 1, 128u);
-        if constexpr (KO & KO_LOADS) {  // every stage holds operand bytes once and for all
-#pragma unroll
-            for (int r = 0; r < 8; ++r) dma_x(r, rx1, 2, 256u);
-            wait_vmcnt<0>();
-        } else {
-            wait_vmcnt<16>();  // slab 0
-        }
+        wait_vmcnt<16>();  // slab 0
         __builtin_amdgcn_s_waitcnt(0xc07f);
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < 8; ++r) read_x(r, 0, 0, xa);
 #pragma unroll
         for (int r = 0; r < 8; ++r) read_w(r, 0, 0, wa);
-        if constexpr (KO & KO_LDS_READS) {  // all four buffers hold operand bytes once and for all
-#pragma unroll
-            for (int r = 0; r < 8; ++r) read_x(r, 0, 1, xb);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) read_w(r, 0, 1, wb);
-        }
     }
 
     int xs = 0;  // k % 3
@@ -183,13 +171,13 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
 #pragma unroll
         for (int i = 0; i < 16 * Op::kMfmas; ++i) {
             const int c = i >> 4, mi = (i >> 2) & 3, ni = i & 3;
-            if constexpr (!(KO & KO_MFMA)) Op::mma(c, wf[ni], xf[mi], acc[4 * wh + ni][4 * xh + mi]);
+            Op::mma(c, wf[ni], xf[mi], acc[4 * wh + ni][4 * xh + mi]);
 #pragma unroll
             for (int r = 0; r < 8; ++r)
-                if (r * Op::kMfmas == i && !(KO & KO_LDS_READS)) rd(r);
+                if (r * Op::kMfmas == i) rd(r);
 #pragma unroll
             for (int d = 0; d < 4; ++d)
-                if ((d * 4 + 2) * Op::kMfmas == i && !(KO & KO_LOADS)) ld(d);
+                if ((d * 4 + 2) * Op::kMfmas == i) ld(d);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -214,7 +202,7 @@ __device__ __forceinline__ void walk16(uint8_t* lds, const void* x, uint32_t x_b
         }
         // Slab k+1 has landed for this wave (all but this half's eight loads are older) and this wave has read slab k;
         // after the barrier both hold for every wave
-        wait_vmcnt<(KO & KO_LOADS) ? 0 : 8>();
+        wait_vmcnt<8>();
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         phase_barrier();
         // (after the last slab the reads fetch stale bytes that are never used)

@@ -29,12 +29,6 @@ struct Wave128Cfg {
     static_assert(4 * 2 * EPI_PASS_BYTES <= LDS_BYTES, "epilogue staging must fit");
 };
 
-// Knock-outs for the phase microbenchmark (ubench/wave128_phases.hip): each bit removes one
-// class of instructions so that its share of the kernel's time -- issue slots and, under the
-// power cap, clock -- can be read off a timing. The library instantiates KO = 0 only; a
-// knocked-out kernel computes nothing meaningful.
-enum : int { KO_LDS_READS = 1, KO_LOADS = 2, KO_MFMA = 4, KO_STORES = 8 };
-
 // bf16 output with whole 16-byte output pieces only; other outputs keep the
 // ping-pong kernel, whose epilogue handles every case
 inline bool wave128_shape_ok(const GemmArgs& g) {

@@ -10,7 +10,7 @@
 namespace w8a8 {
 
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it
-template <int Fmt, int ScaleKind, int KO = 0, bool RoundFirst = false>
+template <int Fmt, int ScaleKind, bool RoundFirst = false>
 __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(GemmArgs g) {
     static_assert(ScaleKind == SCALE_TENSOR || ScaleKind == SCALE_ROWCOL, "per-tensor or row x column scales");
     PP_STAMP_INIT();
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(G
     f32x4 acc[8][8];  // [n sub-tile][m sub-tile]
     PP_STAMP();
     PP_STAMP();
-    walk16<Walk16F8<Fmt>, KO>(lds, g.a, (uint32_t)g.m * (uint32_t)K, x_off, g.b, (uint32_t)g.n * (uint32_t)K, w_off, ksteps, acc);
+    walk16<Walk16F8<Fmt>>(lds, g.a, (uint32_t)g.m * (uint32_t)K, x_off, g.b, (uint32_t)g.n * (uint32_t)K, w_off, ksteps, acc);
 
     PP_STAMP();
     // ---------------- epilogue ----------------
@@ -118,9 +118,7 @@ __global__ __launch_bounds__(Wave128Cfg::THREADS) void gemm_wave128_q16_kernel(G
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(buf + (i * 4 + r4) * ROWB + c16 * 16);
-                if constexpr (!(KO & KO_STORES))
-                    __builtin_amdgcn_raw_buffer_store_b128(
-                        v, rout, lane_off + (uint32_t)(p * 32 + i * 4) * row_bytes, 0, 2);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rout, lane_off + (uint32_t)(p * 32 + i * 4) * row_bytes, 0, 2);
             }
         }
     }
@@ -131,7 +129,7 @@ template <int Fmt, int ScaleKind, bool RoundFirst = false>
 inline void launch_wave128_q16(const GemmArgs& g, hipStream_t stream) {
     using Cfg = Wave128Cfg;
     const int tiles = ((g.m + Cfg::BM - 1) / Cfg::BM) * ((g.n + Cfg::BN - 1) / Cfg::BN);
-    auto kern = gemm_wave128_q16_kernel<Fmt, ScaleKind, 0, RoundFirst>;
+    auto kern = gemm_wave128_q16_kernel<Fmt, ScaleKind, RoundFirst>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
     note_kernel("wave128_q16");

@@ -1,11 +1,7 @@
-// Where the four-wave 256x256x128 GEMM kernel's time goes, measured on the kernel itself:
-//   1. phase stamps (the shader clock counter read by every wave at kernel start, main-loop
-//      end (its prologue included) and kernel end; workgroup 0) on all-zero operands, where the clock
-//      stays at its maximum;
-//   2. knock-outs: the same kernel with one class of instructions removed (LDS operand reads,
-//      global->LDS loads, MFMAs, output stores), timed on zeros and on normally distributed fp8
-//      operands (the config-1 distribution). On toggling operands the chip runs against its
-//      power cap, so a knocked-out class gives back its issue slots AND its energy (clock).
+// Where the time of the 256 x 256 x 128 fp8 GEMM kernels goes: phase stamps of the kernels themselves (the shader clock
+// counter read by every wave at kernel start, main-loop start and end and kernel end; workgroup 0) on all-zero operands,
+// where the clock stays at its maximum, and their times on zeros and on normally distributed operands (the config-1
+// distribution), whose toggling bits run the chip against its power cap.
 // Build: make -C astrai_amd/csrc ubench     Run: astrai_amd/csrc/ubench/wave128_phases [M N K]
 #define W8A8_PP_TIMING 1
 #include "../gemm_wave128_q16.cuh"
@@ -27,9 +23,9 @@ using namespace w8a8;
         }                                                                              \
     } while (0)
 
-template <int SK, int KO>
+template <int SK>
 static float time_us(const GemmArgs& g) {
-    auto kern = gemm_wave128_q16_kernel<0, SK, KO>;
+    auto kern = gemm_wave128_q16_kernel<0, SK>;
     CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Wave128Cfg::LDS_BYTES));
     const int tiles = ((g.m + 255) / 256) * ((g.n + 255) / 256);
     hipEvent_t e0, e1;
@@ -134,23 +130,11 @@ static void pingpong_section(unsigned long long* dbg) {
         printf("ping-pong kernel, per-tensor scales, %s: %.2f us (%.0f Tops/s)\n",
                random ? "normal operands" : "zeros", us, ops / us / 1e6);
         if (!random) print_stamps(dbg, K, {0, 4});
-        us = time_us<SCALE_TENSOR, 0>(g);
+        us = time_us<SCALE_TENSOR>(g);
         printf("four-wave kernel, per-tensor scales, %s: %.2f us (%.0f Tops/s)\n",
                random ? "normal operands" : "zeros", us, ops / us / 1e6);
     }
     CK(hipFree(a)); CK(hipFree(b)); CK(hipFree(out)); CK(hipFree(s));
-}
-
-template <int SK>
-static void knockouts(const char* what, const GemmArgs& g) {
-    const double ops = 2.0 * g.m * g.n * (double)g.k;
-    const float base = time_us<SK, 0>(g);
-    printf("%s: whole kernel %.2f us (%.0f Tops/s)\n", what, base, ops / base / 1e6);
-    printf("  without LDS operand reads      %.2f us\n", time_us<SK, KO_LDS_READS>(g));
-    printf("  without global->LDS loads      %.2f us\n", time_us<SK, KO_LOADS>(g));
-    printf("  without either                 %.2f us\n", time_us<SK, KO_LDS_READS | KO_LOADS>(g));
-    printf("  without output stores          %.2f us\n", time_us<SK, KO_STORES>(g));
-    printf("  without MFMAs                  %.2f us\n", time_us<SK, KO_MFMA>(g));
 }
 
 int main(int argc, char** argv) {
@@ -172,11 +156,10 @@ int main(int argc, char** argv) {
     CK(hipMemset(a, 0, (size_t)M * K));
     CK(hipMemset(b, 0, (size_t)N * K));
     {
-        const float us = time_us<SCALE_TENSOR, 0>(g);
+        const float us = time_us<SCALE_TENSOR>(g);
         printf("fp8 zeros %dx%dx%d: %.2f us; stamps of workgroup 0 in shader clock cycles\n", M, N, K, us);
         print_stamps(dbg, K, {0, 3});
     }
-    knockouts<SCALE_TENSOR>("fp8 zeros", g);
 
     {
         std::vector<unsigned char> ra((size_t)M * K), rb((size_t)N * K);
@@ -186,7 +169,8 @@ int main(int argc, char** argv) {
         CK(hipMemcpy(a, ra.data(), ra.size(), hipMemcpyHostToDevice));
         CK(hipMemcpy(b, rb.data(), rb.size(), hipMemcpyHostToDevice));
     }
-    knockouts<SCALE_TENSOR>("fp8 normal operands (amax at 4.5 sigma)", g);
+    const float us = time_us<SCALE_TENSOR>(g);
+    printf("fp8 normal operands (amax at 4.5 sigma): %.2f us (%.0f Tops/s)\n", us, 2.0 * M * N * (double)K / us / 1e6);
     pingpong_section(dbg);
     return 0;
 }

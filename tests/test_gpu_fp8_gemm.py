@@ -280,14 +280,13 @@ def test_mm_fp8_token_tail_past_a_round_of_large_tiles(ops, fmt, m, n, k):
     assert_bf16_close(out, O.fp8_gemm_bias(a8[rows], b8, sa_r[rows], sb_r, None), what="tail rows, row/column steps")
 
 
-@pytest.mark.parametrize("m,n,k,fmt", [(3900, 4104, 1024, 0),   # even slab count: 16x16x128 instance
-                                       (3900, 4104, 1152, 0),   # odd slab count: 32x32x64 instance
-                                       (4097, 3848, 512, 1),    # e5m2, 16x16x128 instance
-                                       (4097, 3848, 384, 1)])   # e5m2, 32x32x64 instance
-def test_four_wave_kernel_both_mfma_instances_whole_output(ops, m, n, k, fmt):
-    """The large-tile bf16 kernel runs on the 16x16x128 MFMA for an even number of 128-byte K
-    slabs and on the 32x32x64 MFMA otherwise: ragged M and N, per-tensor steps with bias and
-    row / column steps, every output against the oracle."""
+@pytest.mark.parametrize("m,n,k,fmt", [(3900, 4104, 1024, 0),   # even slab count: whole turns of the two-slab walk
+                                       (3900, 4104, 1152, 0),   # odd slab count: a last slab of its own
+                                       (4097, 3848, 512, 1),    # e5m2, even
+                                       (4097, 3848, 384, 1)])   # e5m2, odd
+def test_four_wave_kernel_even_and_odd_slabs_whole_output(ops, m, n, k, fmt):
+    """The large-tile bf16 kernel walks two 128-byte K slabs a turn and an odd last one behind them: ragged M and N,
+    per-tensor steps with bias and row / column steps, every output against the oracle."""
     from astrai_amd.extension import _cabi
     print(f"case m={m} n={n} k={k} fmt={fmt}", flush=True)
     g = torch.Generator().manual_seed(m + n + k + fmt)
