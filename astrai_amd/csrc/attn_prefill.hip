@@ -45,7 +45,7 @@
 // What bounds it: 53 vector instructions, 16 exponentials, 16 MFMAs and 24 LDS reads a tile and wave; a tile takes 890
 // cycles alone on a SIMD, 790 with two waves (512 are the MFMAs'; operand reads 190, the branch and the barrier 100),
 // under a clock that the power limit holds at 1.7 GHz for long sequences (2.1 for short ones).
-// Counters of 4 x 2048 tokens: matrix pipe and vector ALU busy 58% of the SIMD cycles each (48 and 53 before).
+// Counters of 4 x 2048 tokens: matrix pipe busy 57% of the SIMD cycles, vector ALU 56% (48 and 53 before the exponentials were spread).
 // Measured (graph replays): 4 x 2048 causal tokens, 16/4 heads x 128 in [batch, seq, head] order 75 us (915 TFLOP/s), ragged
 // 16 x 175..700 tokens of 32/8 heads x 64 in a pool 75.7 us (P in two terms); with the exponentials behind the score
 // MFMAs alone, the loads in a burst and offsets formed for each (120 vector instructions a tile) 80.3 and 78.2. Prompts of up
