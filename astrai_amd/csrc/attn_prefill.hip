@@ -33,9 +33,10 @@
 // the question whether one has outgrown its reference into the next step. Keys and values arrive by direct-to-LDS
 // loads into two rings of four tiles, values two tiles behind the keys, one 64-key block ahead (the first three tiles of
 // both at once), one load to every second MFMA of a block's first step (all at once they stall the waves that issue
-// them); one workgroup barrier per block; no staging registers. Dense loads keep their lane's offset, the descriptors move along instead; the loop over unmasked
-// blocks goes once round the rings, so that its LDS offsets are constants. Tiles that every query of the wave sees whole
-// skip the masking code; the accumulators are rescaled only when a row maximum has outgrown the reference maximum by 2^8.
+// them); one workgroup barrier per block; no staging registers. Dense loads keep their lane's offset, the descriptors move
+// along instead; the loop over unmasked blocks goes once round the rings, so that its LDS offsets are constants. Tiles that
+// every query of the wave sees whole skip the masking code; the accumulators are rescaled only when a row maximum has
+// outgrown the reference maximum by 2^8.
 //
 // The direct-to-LDS loads are written in assembly (they have no output register): behind the
 // builtin the compiler orders every transposing read after all loads in flight (s_waitcnt vmcnt(0)),
