@@ -41,12 +41,12 @@ __device__ __forceinline__ Decay decay_fast(float sr, float br, float si, float 
     const float e = coef2 * r;
     Decay d;
     d.a = __builtin_amdgcn_exp2f(e);
-    constexpr float c = 1.38629436111989061883f;   // 2 ln 2
-    float p = fmaf(e, c / 5.0f, 1.0f);
-    p = fmaf(e * (c / 4.0f), p, 1.0f);
-    p = fmaf(e * (c / 3.0f), p, 1.0f);
-    p = fmaf(e * (c / 2.0f), p, 1.0f);
-    const float m = e > -0.07f ? -c * e * p : fmaf(-d.a, d.a, 1.0f);
+    constexpr double c = 1.38629436111989061883;   // 2 ln 2
+    float p = fmaf(e, (float)(-c * c * c * c * c / 120), (float)(-c * c * c * c / 24));
+    p = fmaf(e, p, (float)(-c * c * c / 6));
+    p = fmaf(e, p, (float)(-c * c / 2));
+    p = fmaf(e, p, (float)-c);
+    const float m = e > -0.07f ? e * p : fmaf(-d.a, d.a, 1.0f);
     d.b = __builtin_amdgcn_sqrtf(m) * i * u;
     return d;
 }
@@ -245,6 +245,169 @@ __global__ __launch_bounds__(256, 3) void rglru_chunk_kernel(RglruArgs a, int cs
     }
 }
 
+// A value of each of the four 16-lane groups, the same in all lanes: the swaps of rows and halves leave the vector ALU's
+// pipe no more than moves do, where a trip through LDS is a hundred cycles.
+__device__ __forceinline__ void of_groups(float v, float (&out)[4]) {
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const auto even = __builtin_amdgcn_permlane32_swap(rows[0], rows[0], false, false);
+    const auto odd = __builtin_amdgcn_permlane32_swap(rows[1], rows[1], false, false);
+    out[0] = __uint_as_float(even[0]);
+    out[1] = __uint_as_float(odd[0]);
+    out[2] = __uint_as_float(even[1]);
+    out[3] = __uint_as_float(odd[1]);
+}
+
+// rglru_chunk_kernel for blocks of 32 KS channels whose weights a wave can hold: a wave keeps both gates' operands of its
+// 16 channels (8 KS registers) and the carries for the whole segment, the next tile of u is on its way while this one
+// is worked on, and the lane groups' decays meet in registers. Same products and sums, tokens in the same order. Bound by the
+// vector ALU: some 45 instructions a channel and token, eight of them transcendental. 8 blocks of 256, both passes: 1 x 4096
+// tokens 63 us (weights from L2 for every tile, exchanges through LDS, one tile under way) -> 46; one pass: 8 x 1024 110 ->
+// 52, 32 x 256 68 -> 46. With y and the outputs through LDS in whole lines it took 54 and 59.
+template <int KS, bool OUT>
+__global__ __launch_bounds__(256, 2) void rglru_held_kernel(RglruArgs a) {
+    constexpr int NT = 4, kTile = NT * 16, kBp = KS * 32, kRow = kBp * 2 + 16, kParts = kBp / 64;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // two tiles of u
+    const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the parts of a block and segment share their tiles of u: on one die (workgroups go round the eight in turn)
+    const int turn = (int)blockIdx.x / 8, part = turn % kParts, item = turn / kParts * 8 + (int)blockIdx.x % 8;
+    if (item >= a.nseg * a.blocks * a.batch) return;
+    const int seg = item % a.nseg, blk = item / a.nseg % a.blocks, b = item / a.nseg / a.blocks;
+    const int cols = a.blocks * kBp;
+    const int tiles = (a.seq + kTile - 1) / kTile, per_seg = (tiles + a.nseg - 1) / a.nseg;
+    const int tok0 = min(seg * per_seg * kTile, a.seq), tok1 = min((seg + 1) * per_seg * kTile, a.seq);
+    const bool last = seg == a.nseg - 1;
+    const int ch = (part * 4 + wave) * 16 + c16, col = blk * kBp + ch;
+    auto slot = [&](int s, int which) { return a.scratch + (((int64_t)b * a.nseg + s) * 2 + which) * cols + col; };
+    float* state = a.state + (int64_t)b * cols + col;
+
+    float s_in = 0.0f, a_in = 1.0f;
+    if constexpr (OUT) {
+        if (a.nseg == 1) {
+            s_in = *state;
+        } else {
+            s_in = *slot(a.nseg - 1, 1);
+            for (int j = 0; j < seg; j += 8) {   // (eight at a time: the loads are under way together)
+                float da[8], db[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int from = min(j + i, seg - 1);
+                    da[i] = *slot(from, 0);
+                    db[i] = *slot(from, 1);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (j + i < seg) s_in = fmaf(da[i], s_in, db[i]);
+            }
+        }
+    } else if (last && g == 0) {
+        *slot(seg, 1) = *state;
+    }
+    if (!OUT && last) return;
+
+    u32x4 wr[KS], wi[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int64_t at = (int64_t)col * kBp + 32 * k + 8 * g;
+        wr[k] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.w_r) + at);
+        wi[k] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.w_i) + at);
+    }
+    const float br = -kLog2e * a.b_r[col], bi = -kLog2e * a.b_i[col], coef2 = kLog2e * a.coef[col];
+
+    const uint16_t* u = static_cast<const uint16_t*>(a.u) + (int64_t)b * a.seq * cols + blk * kBp;
+    u32x4 next[KS];
+    auto fetch = [&](int t0) {   // (tokens past the segment read as 0)
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int c = tid + i * 256, t = t0 + c / (KS * 4), e = c % (KS * 4);
+            next[i] = t < tok1 ? *reinterpret_cast<const u32x4*>(u + (int64_t)t * cols + e * 8) : u32x4{0, 0, 0, 0};
+        }
+    };
+    if (tok0 < tok1) fetch(tok0);
+    uint8_t* tile = lds;
+    for (int t0 = tok0; t0 < tok1; t0 += kTile) {
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int c = tid + i * 256;
+            *reinterpret_cast<u32x4*>(tile + c / (KS * 4) * kRow + c % (KS * 4) * 16) = next[i];
+        }
+        __syncthreads();   // the tile is there; the one before, in the other buffer, is no longer read
+        fetch(t0 + kTile);
+        const uint8_t* const now = tile;
+        tile = tile == lds ? lds + kTile * kRow : lds;
+        const int left = min(tok1 - t0, kTile);
+        uint16_t yv[OUT ? NT : 1][4];
+        // (buffer descriptors end with the segment: later tokens read as 0 and are not written)
+        const __amdgpu_buffer_rsrc_t ry = w8a8::make_rsrc(
+            static_cast<const uint16_t*>(a.proj) + ((int64_t)b * a.seq + t0) * a.ld, (uint32_t)(left * a.ld) * 2);
+        const __amdgpu_buffer_rsrc_t ro = w8a8::make_rsrc(
+            static_cast<const uint16_t*>(a.out) + ((int64_t)b * a.seq + t0) * cols, (uint32_t)(left * cols) * 2);
+        const uint32_t y_lane = (uint32_t)(4 * g * a.ld + a.y_off + col) * 2, o_lane = (uint32_t)(4 * g * cols + col) * 2;
+        if constexpr (OUT) {
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    yv[tt][e] = __builtin_amdgcn_raw_buffer_load_b16(ry, y_lane + (uint32_t)((tt * 16 + e) * a.ld) * 2, 0, 0);
+        }
+        const uint8_t* const lu = now + c16 * kRow + 16 * g;
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) {
+            f32x4 zr = {0, 0, 0, 0}, zi = {0, 0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const u32x4 x = *reinterpret_cast<const u32x4*>(lu + tt * 16 * kRow + k * 64);
+                zr = mfma16(x, wr[k], zr);
+                zi = mfma16(x, wi[k], zi);
+            }
+            const int tl = tt * 16 + 4 * g;   // this lane's first token in the tile
+            Decay d[4];
+            float pa = 1.0f, pb = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = w8a8::bf16_to_f32(*reinterpret_cast<const uint16_t*>(now + (tl + e) * kRow + ch * 2));
+                d[e] = decay_fast(zr[e], br, zi[e], bi, coef2, x);
+            }
+            if (left < kTile) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (tl + e >= left) d[e] = Decay{1.0f, 0.0f};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                pa *= d[e].a;
+                pb = fmaf(d[e].a, pb, d[e].b);
+            }
+            float ga[4], gb[4], start[4];
+            of_groups(pa, ga);
+            of_groups(pb, gb);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                start[i] = s_in;
+                s_in = fmaf(ga[i], s_in, gb[i]);
+            }
+            if constexpr (!OUT) {
+                a_in *= (ga[0] * ga[1]) * (ga[2] * ga[3]);
+            } else {
+                float s = g & 2 ? (g & 1 ? start[3] : start[2]) : (g & 1 ? start[1] : start[0]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s = fmaf(d[e].a, s, d[e].b);
+                    const float o = s * gelu_fast(w8a8::bf16_to_f32(yv[tt][e]));
+                    __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(o), ro, o_lane + (uint32_t)((tt * 16 + e) * cols) * 2, 0, 0);
+                }
+            }
+        }
+    }
+    if (g) return;
+    if constexpr (!OUT) {
+        *slot(seg, 0) = a_in;
+        *slot(seg, 1) = s_in;
+    } else if (last) {
+        *state = s_in;
+    }
+}
+
 // rows: a workgroup's sequences b0 .. b0 + nb - 1, seq tokens each, nb * seq <= 16
 __global__ __launch_bounds__(256) void rglru_step_kernel(RglruArgs a, int nb) {
     __shared__ f32x4 red[3][2][64];
@@ -370,6 +533,21 @@ void chunk_t(const RglruArgs& a, hipStream_t stream) {
     rglru_chunk_kernel<NT, true><<<grid, 256, shared, stream>>>(a, csplit);
 }
 
+template <int KS>
+void held_t(const RglruArgs& a, hipStream_t stream) {
+    constexpr int shared = 2 * 64 * (KS * 64 + 16);
+    static const hipError_t once = [] {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rglru_held_kernel<KS, true>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, shared);
+        return e != hipSuccess ? e : hipFuncSetAttribute(reinterpret_cast<const void*>(&rglru_held_kernel<KS, false>),
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, shared);
+    }();
+    (void)once;
+    const unsigned grid = ((unsigned)(a.nseg * a.blocks * a.batch) + 7) / 8 * 8 * (KS / 2);
+    if (a.nseg > 1) rglru_held_kernel<KS, false><<<grid, 256, shared, stream>>>(a);
+    rglru_held_kernel<KS, true><<<grid, 256, shared, stream>>>(a);
+}
+
 template <typename T>
 void general_t(const RglruArgs& a, hipStream_t stream) {
     const int cols = a.blocks * a.bp;
@@ -383,7 +561,18 @@ void general_t(const RglruArgs& a, hipStream_t stream) {
 // a tile of 64 tokens of 1024 channels: 129 KiB of LDS, the carries 8 KiB
 bool rglru_chunk_supported(int bp) { return bp <= 1024; }
 
-void launch_rglru_chunk(const RglruArgs& a, hipStream_t stream) { chunk_t<4>(a, stream); }
+// Whole groups of four waves of 16 channels whose weights fit the registers of two waves a SIMD are held
+// (1 x 4096 tokens: blocks of 64 44 -> 33 us, of 128 50 -> 37, of 256 63 -> 46); other blocks stream them.
+void launch_rglru_chunk(const RglruArgs& a, hipStream_t stream) {
+    const bool counted = (int64_t)a.nseg * a.blocks * a.batch < 1 << 28;   // (the held kernel's grid is one number)
+    switch (counted ? a.bp : 0) {
+        case 64: return held_t<2>(a, stream);
+        case 128: return held_t<4>(a, stream);
+        case 192: return held_t<6>(a, stream);
+        case 256: return held_t<8>(a, stream);
+        default: return chunk_t<4>(a, stream);
+    }
+}
 
 bool rglru_step_supported(int bp, int seq) { return bp > 0 && seq <= kRingSteps; }
 

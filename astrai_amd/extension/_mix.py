@@ -734,14 +734,19 @@ def rglru_chunk_supported(bp: int) -> bool:
 
 
 def rglru_nseg(batch: int, blocks: int, bp: int, seq: int) -> int:
-    """Segments of a sequence that run side by side. A segment is walked tile by tile, 5.8 us per 64 tokens, so few
-    sequences are cut until there are about four workgroups for each CU, into segments of as many tiles each, down to
-    one (1 x 4096 tokens, 8 blocks of 256: 8 segments 97 us, 16 69, 32 65; 1 x 512: 4 segments 28, 8 18). Cut,
-    everything is computed twice: from about 176 workgroups on one walk is the shorter (1024 tokens, blocks of 256: 128
-    workgroups 100 us whole, 65 cut, 160 101, 76, 192 102, 106, 256 112, 116; blocks of 128: 176 80, 60, 192 80, 81, 256
-    81, 82), and so it is for two tiles, whose halves would be walked twice."""
+    """Segments of a sequence that run side by side; cut, everything is computed twice. Blocks of 64, 128, 192 and 256 (the
+    kernel that holds their weights, 3.3 us per 64 tokens of 256 channels): as many as fill the chip with the two
+    workgroups a CU takes (8 blocks of 256: 1 x 4096 tokens, 8 segments 54 us, 16 46, 32 51; 4 x 2048, 4 segments 76, 8
+    80, 16 88); past 128 workgroups a sequence walked whole is the shorter (5 x 1000: whole 50 us, 3 segments 59, 8 58;
+    8 x 1024: 52, 75, 87). Others, 5.8 us per 64 tokens: about four workgroups for each CU, of as many tiles each, and
+    whole from 176 workgroups on (1024 tokens, 160 workgroups 101 us whole, 76 cut; 192 102 and 106). Two tiles are
+    not worth a second walk."""
     groups, tiles = batch * blocks * -(-bp // 64), -(-seq // 64)
-    return 1 if groups > 176 or tiles <= 2 else -(-tiles // max(1, tiles * groups // 1024))
+    held = bp % 64 == 0 and bp <= 256
+    if groups > (128 if held else 176) or tiles <= 2:
+        return 1
+    each = -(-tiles // min(tiles, 512 // groups)) if held else max(1, tiles * groups // 1024)
+    return -(-tiles // each)
 
 
 def _rglru_checks(what: str, proj, y_off, w_r, w_i, b_r, b_i, coef, state, *rows):

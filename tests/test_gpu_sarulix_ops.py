@@ -366,6 +366,14 @@ def test_recurrence_in_segments(nseg):
         c.check(c.run([130, 870], "chunk", nseg), TOL[BF16])
 
 
+@pytest.mark.parametrize("size", [64, 120, 192, 250])   # held weights: two, four, six and eight steps of 32 channels
+@pytest.mark.parametrize("nseg", [1, 3])
+def test_recurrence_held_weights(size, nseg):
+    log("rglru held", nseg, size)
+    c = Recurrence(3, size, 4, BF16, 400, batch=3, seed=size)
+    c.check(c.run([63, 65, 193, 79] if nseg == 1 else [129, 271], "chunk", nseg), TOL[BF16])
+
+
 @pytest.mark.parametrize("batch,taps", [(1, 4), (5, 3), (19, 2), (33, 1), (2, 7)])
 def test_recurrence_step(batch, taps):
     for blocks, size in ((3, 30), (2, 256)):
