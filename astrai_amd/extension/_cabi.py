@@ -12,6 +12,7 @@ anywhere in this module: without the HIP library every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import weakref
 import os
 from typing import Optional
@@ -104,6 +105,7 @@ PROTOTYPES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
+_host = None   # the native form of the everyday calls (csrc/host.cpp), there whenever _lib is
 _load_error: Optional[str] = None
 
 
@@ -111,7 +113,7 @@ def load() -> Optional[ctypes.CDLL]:
     """Load the shared library once; ``None`` (with the reason kept) if it is absent
     or does not carry the expected ABI. Never raises: the registry reports an
     unavailable kernel the way the reference's loader does (loader.py:36-44)."""
-    global _lib, _load_error
+    global _lib, _host, _load_error
     if _lib is not None or _load_error is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -126,7 +128,8 @@ def load() -> Optional[ctypes.CDLL]:
         got = lib.astrai_w8a8_abi_version()
         if got != ABI_VERSION:
             raise OSError(f"ABI version {got}, expected {ABI_VERSION}")
-    except (OSError, AttributeError) as e:
+        _host = importlib.import_module("astrai_amd.extension._host")
+    except (OSError, AttributeError, ImportError) as e:
         _load_error = f"{type(e).__name__}: {e}"
         return None
     _lib = lib
@@ -395,6 +398,10 @@ def _plain_bf16(t: torch.Tensor, dev: torch.device) -> bool:
 def linear_fp8_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, inner: int = 1) -> bool:
     """Whether :func:`linear_fp8` takes these: bf16 on one GPU as the kernels read them, ``K % 16 == 0``, nothing empty,
     rows of ``x`` as wide as ``w.size(inner)`` (0: ``x`` is the output's gradient)."""
+    if _host is not None:
+        answer = _host.linear_fp8_operands(x, w, bias, inner)
+        if answer is not None:
+            return answer
     k, dev = x.size(-1), x.device
     return (x.is_cuda and w.dim() == 2 and k == w.size(inner) and k % 16 == 0 and x.numel() > 0 and w.numel() > 0
             and _plain_bf16(x, dev) and _plain_bf16(w, dev)
@@ -417,7 +424,12 @@ def linear_fp8(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], c
     ``w`` quantized, the product, the pushes. ``rings`` of x and w, ``(history, index)``: ``steps`` are used and then
     refreshed (no ring of w with given codes). No ring of x: each step is measured, ``steps[1]`` that of given codes, and
     the bias joins the product rounded to bf16."""
-    lib, dev = _require(), x.device
+    lib = _require()
+    (x_hist, x_idx), (w_hist, w_idx) = rings[0] or (None, 0), rings[1] or (None, 0)
+    out = _host.linear_fp8(x, w, bias, codes, steps[0], steps[1], x_hist, x_idx, w_hist, w_idx, fmt, fmax, pow2_margin)
+    if out is not None:
+        return out
+    dev = x.device
     n, k = w.shape
     if x.size(-1) != k:   # (the kernels count rows by the element: they would write past `out`)
         raise RuntimeError(f"linear_fp8: inner dim mismatch, x [.., {x.size(-1)}] and w [{n}, {k}]")
@@ -446,7 +458,12 @@ def linear_fp8_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, want_
     """Its input, weight and (or an empty tensor) bias gradient in one library call, the operands as
     :func:`linear_fp8_operands` has them. ``ring`` ``(history, index)`` of the gradient, whose step is refreshed behind the
     products; without one each step is measured."""
-    lib, dev = _require(), g.device
+    lib = _require()
+    hist, idx = ring or (None, 0)
+    grads = _host.linear_fp8_backward(g, x, w, want_bias, *(steps or (None, None, None)), hist, idx, fmt, fmax, pow2_margin)
+    if grads is not None:
+        return grads
+    dev = g.device
     n, k = w.shape
     m = x.numel() // k
     if x.size(-1) != k or g.size(-1) != n or g.numel() != m * n:
@@ -978,6 +995,18 @@ def paged_nsplit(pairs: int, max_keys: int) -> int:
     return max(1, min(64, 512 // pairs, max_keys // 64))
 
 
+def _decode_is_general(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
+    """The shapes of a paged step that only the general kernel takes."""
+    return head_dim != 128 or n_heads > 64 or n_heads // n_kv_heads > 8
+
+
+def _rows_decode_nsplit(pairs: int, max_keys: int) -> int:
+    """Context splits of the general kernel's step, one wave per (sequence, kv head, split): three to a SIMD (two, three, 32 /
+    8 heads x 64: 32 x 3000 keys 35.0 us, 31.2; 128 x 1000 43.5, 38.0; 16 / 16 heads x 64, 64 x 1500: 62, 54.7; fewer
+    pairs the same)."""
+    return max(1, min(64, 3072 // max(1, pairs), max_keys // 64))
+
+
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
                 scale: Optional[float] = None, nsplit: int = 0, quantized: bool = False):
     """``q [batch, n_heads, seq, 128]`` (bf16) against the dense caches
@@ -1077,6 +1106,14 @@ def attn_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     ``ml_part_buf`` is not needed. ``mask``: bool ``[batch, width]``, True = attend
     that position (entry_utils.cuh:226-237); positions past ``width`` are not attended."""
     lib = _require()
+    if mask is new_k is new_v is out_buf is o_part_buf is None and q.dim() == k_cache.dim() == 3 and req_to_token.dim() == 2:
+        (b, h, d), hkv = q.shape, k_cache.size(1)
+        general = hkv == 0 or _decode_is_general(h, hkv, d)
+        splits = nsplit if nsplit > 0 else (_rows_decode_nsplit if general else paged_nsplit)(b * hkv, req_to_token.size(1))
+        out = _host.attn_paged_decode(q, k_cache, v_cache, req_to_token, req_pool_indices, kv_indptr, general, splits,
+                                      d ** -0.5 if scale is None or scale <= 0.0 else scale)
+        if out is not None:
+            return out
     _gpu(q, "attn_paged_decode")
     if mask is not None:
         if not mask.is_cuda or mask.dtype != torch.bool:
@@ -1135,11 +1172,9 @@ def attn_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
         if b == 0:
             return out  # (an empty tensor has no address to hand over)
         m_ptr, m_stride, m_width = (mask.data_ptr(), mask.stride(0), mask.size(1)) if mask is not None else (0, 0, 0)
-        if d != 128 or h > 64 or h // hkv > 8:  # the shapes only the general kernel takes
+        if _decode_is_general(h, hkv, d):
             if not user_nsplit:
-                # one wave per (sequence, kv head, split): three to a SIMD (two, three, 32 / 8 heads x 64: 32 x 3000 keys
-                # 35.0 us, 31.2; 128 x 1000 43.5, 38.0; 16 / 16 heads x 64, 64 x 1500: 62, 54.7; fewer pairs the same)
-                nsplit = max(1, min(64, 3072 // max(1, b * hkv), rtt.size(1) // 64))
+                nsplit = _rows_decode_nsplit(b * hkv, rtt.size(1))
             _paged_rows(lib, q_c, k_cache, v_cache, rtt, rpi, ind, None, (m_ptr, m_stride, 0, 0, 1, m_width),
                         out, b, nsplit, False, scale, o_part_buf)
             return out
@@ -1181,6 +1216,11 @@ def _paged_rows(lib, q, k_pool, v_pool, rtt, rpi, kv_indptr, schedule, m_args, o
         rtt.size(1), 1 if causal else 0, nsplit, float(scale), _stream(q)), lib)
 
 
+def _rows_nsplit(tiles: int, n_kv_heads: int) -> int:
+    """Context splits of the general paged kernel over a schedule of ``tiles``."""
+    return max(1, min(16, 2048 // max(1, tiles * 4 * n_kv_heads)))   # at least: one wave per row block, 4+ blocks per tile
+
+
 Q_TILE_ROWS = 64  # rows per tile of the schedule the reference builds (astrai/inference/workspace.py:13)
 
 
@@ -1201,6 +1241,14 @@ def attn_paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
     2, 4 or 8 runs the MFMA block kernel; other shapes the general kernel, whose context split
     ``nsplit`` (0: chosen here) only matters for short schedules."""
     lib = _require()
+    if mask is None and q.dim() == k_cache.dim() == 3 and k_cache.size(1):
+        h, hkv, d = q.size(1), k_cache.size(1), q.size(2)
+        out = _host.attn_paged_prefill(q, k_cache, v_cache, req_to_token, req_pool_indices, kv_indptr, qo_indptr, q_tile_to_batch,
+                                       q_tile_to_index, not attn_prefill_supported(h, hkv, d),
+                                       nsplit if nsplit > 0 else _rows_nsplit(q_tile_to_batch.numel(), hkv), causal_offset >= 0,
+                                       d ** -0.5 if scale is None or scale <= 0.0 else scale)
+        if out is not None:
+            return out
     _gpu(q, "attn_paged_prefill")
     m_args = (0, 0, 0, 0, 0, 0)
     if mask is not None:
@@ -1256,10 +1304,8 @@ def attn_paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
             return out  # (an empty tensor has no address to hand over)
         if not attn_prefill_supported(h, hkv, d):  # the shapes only the general kernel takes
             tiles = q_tile_to_batch.numel()
-            waves = tiles * 4 * hkv                  # at least: one wave per row block, 4+ blocks per tile
             _paged_rows(lib, q_c, k_cache, v_cache, tensors[0], tensors[1], tensors[2], tensors[3:], m_args,
-                        out, tiles, nsplit if nsplit > 0 else max(1, min(16, 2048 // max(1, waves))),
-                        causal_offset >= 0, scale)
+                        out, tiles, nsplit if nsplit > 0 else _rows_nsplit(tiles, hkv), causal_offset >= 0, scale)
             return out
         _check(lib.astrai_w8a8_attn_paged_prefill_masked_bf16(
             q_c.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), *[t.data_ptr() for t in tensors],
@@ -1381,6 +1427,10 @@ def mm_int8(a: torch.Tensor, b: torch.Tensor, sa: Optional[torch.Tensor],
 def linear_int8(x: torch.Tensor, wq: torch.Tensor, sw: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``mm_int8`` of ``quantize_int8_rows(x)``, ``[..., N]``: one library call where the operands are as the kernels take
     them."""
+    lib = _require()
+    out = _host.linear_int8(x, wq, sw, bias)
+    if out is not None:
+        return out
     k, n, dev = x.size(-1), wq.size(0), x.device
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and k % 16 == 0 and x.numel() and n
             and wq.dtype == torch.int8 and wq.dim() == 2 and wq.size(1) == k and wq.is_contiguous() and wq.device == dev
@@ -1388,7 +1438,7 @@ def linear_int8(x: torch.Tensor, wq: torch.Tensor, sw: torch.Tensor, bias: Optio
             and (bias is None or (bias.dtype == torch.bfloat16 and bias.numel() == n and bias.is_contiguous() and bias.device == dev))):
         xq, sx = quantize_int8_rows(x)
         return mm_int8(xq, wq, sx, sw, bias).reshape(*x.shape[:-1], n)
-    lib, m = _require(), x.numel() // k
+    m = x.numel() // k
     with _on_device(dev):
         codes = torch.empty(m * (k + 4), device=dev, dtype=torch.uint8)   # codes, then a step per row
         out = torch.empty((*x.shape[:-1], n), device=dev, dtype=torch.bfloat16)
@@ -1596,6 +1646,9 @@ def mm_int8_rope_cache(a: torch.Tensor, wqkv: torch.Tensor, sa: torch.Tensor, sb
 def quantize_fp8_block128_act(x: torch.Tensor):
     """bf16 ``[M,K]`` -> ``(x8 e4m3fn [M,K], sa fp32 [M,K/128])``."""
     lib = _require()
+    out = _host.quantize_block128_act(x)
+    if out is not None:
+        return out
     _gpu(x, "quantize_fp8_block128_act")
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise RuntimeError("x must be 2D bf16")
@@ -1635,6 +1688,9 @@ def mm_fp8_block128(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torc
                     bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """e4m3fn NT GEMM with ``sa [M,K/128]`` and ``sb [ceil(N/128),K/128]`` block scales."""
     lib = _require()
+    out = _host.mm_block128(a, b, sa, sb, bias)
+    if out is not None:
+        return out
     _gpu(a, "mm_fp8_block128")
     _gpu(b, "mm_fp8_block128")
     if a.dtype != torch.float8_e4m3fn or b.dtype != torch.float8_e4m3fn:
@@ -1909,6 +1965,11 @@ def attn_prefill_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Op
     mask the block kernel reads the tensors in place (:func:`attn_prefill_strided`); the other cases run the
     ragged paged kernel over the token-major tensors (layout 0 is copied for it), an offset other than
     ``kv_len - q_len`` expressed through the mask."""
+    if mask is None and layout == BLHD and q.dim() == k.dim() == 4 and _host is not None and k.size(2) and attn_prefill_strided_takes(
+            q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q.size(3)):
+        out = _host.attn_prefill(q, k, v, causal_offset, scale if scale and scale > 0.0 else q.size(3) ** -0.5)
+        if out is not None:
+            return out
     b, q_len, kv_len, h, hkv, d = _dense_args(q, k, v, layout, "attn_prefill")
     m4 = _dense_mask(mask, b, q_len, kv_len, h)
     if d not in (32, 64, 128, 256) or h // hkv > 16:

@@ -8,6 +8,7 @@ and without the HIP library every call raises (no CPU or PyTorch fallback).
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 from dataclasses import dataclass
 from typing import Optional
@@ -70,12 +71,13 @@ PROTOTYPES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
+_host = None   # the native form of the commonest calls (csrc/host_mix.cpp), there whenever _lib is
 _load_error: Optional[str] = None
 
 
 def load() -> Optional[ctypes.CDLL]:
     """Load the library once; ``None`` (with the reason kept) if it is absent or of another ABI."""
-    global _lib, _load_error
+    global _lib, _host, _load_error
     if _lib is not None or _load_error is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -90,7 +92,8 @@ def load() -> Optional[ctypes.CDLL]:
         got = lib.astrai_mix_abi_version()
         if got != ABI_VERSION:
             raise OSError(f"ABI version {got}, expected {ABI_VERSION}")
-    except (OSError, AttributeError) as e:
+        _host = importlib.import_module("astrai_amd.extension._host_mix")
+    except (OSError, AttributeError, ImportError) as e:
         _load_error = f"{type(e).__name__}: {e}"
         return None
     _lib = lib
@@ -153,6 +156,9 @@ def residual_norm(y: torch.Tensor, x: torch.Tensor, w_post: torch.Tensor, w_pre:
                   eps: float) -> torch.Tensor:
     """``x += mult * LN(y) * w_post`` (in place, fp32) and ``LN(x) * w_pre`` in ``y``'s dtype, returned."""
     lib = _require()
+    h = _host.residual_norm(y, x, w_post, w_pre, mult, eps)
+    if h is not None:
+        return h
     n, width = y.shape
     code = _dtype(y, "residual_norm")
     _dense("residual_norm", y.dtype, y)
@@ -195,6 +201,10 @@ def sum_norm(y: torch.Tensor, w: Optional[torch.Tensor], dtype: torch.dtype, eps
     ``y [n, width]`` and ``u`` may be rows of a wider matrix and have one type, ``dtype`` or float32. The residual
     goes to ``out`` (which may be ``x``) or a new tensor. Returns (residual, normed)."""
     lib = _require()
+    if dtype in _DTYPES:
+        both = _host.sum_norm(y, w, dtype == torch.bfloat16, eps, x, u, vec, tokens, mult, out)
+        if both is not None:
+            return both
     width = y.size(1)
     n = y.size(0) if tokens is None else tokens.numel()
     code = _DTYPES[dtype]
@@ -255,6 +265,8 @@ def few_rows_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optio
                               act: Optional[str] = None) -> bool:
     """The calls :func:`few_rows_linear` takes: bf16 on one GPU, up to 64 rows of ``x [.., k]`` at 16-byte
     boundaries, ``k`` a multiple of 128, the outputs of 4, weights under 2 GiB."""
+    if _host is not None and _host.few_rows_linear_takes(x, weight, bias, -1 if act is None else 0, FEW_ROWS):
+        return True
     n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
     rows = x.numel() // k if k else 0
     if x.size(-1) != k or not 0 < rows <= FEW_ROWS or k % 128 or n % 4 or weight.numel() * 2 >= 2 ** 31:
@@ -274,6 +286,10 @@ def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
     """``F.linear`` of a few rows (a decode step), or ``act(gate) * up`` of a weight that holds the rows of
     gate before those of up: what :func:`act_mul` makes of the product, in one launch."""
     lib = _require()
+    if out_dtype in _DTYPES:
+        out = _host.few_rows_linear(x, weight, bias, -1 if act is None else ACTIVATIONS[act], FEW_ROWS, out_dtype == torch.float32)
+        if out is not None:
+            return out
     if not few_rows_linear_supported(x, weight, bias, act) or out_dtype not in _DTYPES:
         raise RuntimeError("few_rows_linear: operands are not covered")
     n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
