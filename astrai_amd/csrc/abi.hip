@@ -838,23 +838,30 @@ int astrai_w8a8_linear_fp8_bf16(const void* x, void* x8, float* x_step, float* x
         return fail(ASTRAI_W8A8_BAD_ARG, "%s: fmax and pow2_margin must be positive", what);
     if (int rc = check_gemm(what, x8, w8, out, m, n, k)) return rc;
     auto s = static_cast<hipStream_t>(stream);
+    const float* product_step = x_step;
+    bool pushed = false;
     if (measure) {
-        w8a8::launch_amax_bf16(x, nullptr, x_maxima, m * k, s);
+        if (!w8a8::launch_quantize_fp8_small(x, x8, {nullptr, fmax, pow2_margin}, x_step, m * k, fmt, s)) {
+            w8a8::launch_amax_bf16(x, nullptr, x_maxima, m * k, s);
+            w8a8::launch_quantize_fp8_measured(x, x8, {x_maxima, fmax, pow2_margin}, x_step, m * k, fmt, s);
+        }
         if (w) w8a8::launch_amax_bf16(w, nullptr, w_maxima, n * k, s);
-        w8a8::launch_quantize_fp8_measured(x, x8, {x_maxima, fmax, pow2_margin}, x_step, m * k, fmt, s);
         if (w) w8a8::launch_quantize_fp8_measured(w, w8, {w_maxima, fmax, pow2_margin}, w_step, n * k, fmt, s);
     } else {
-        w8a8::launch_quantize_fp8(x, x8, x_step, nullptr, x_maxima, m * k, fmt, s);
+        pushed = !w && w8a8::launch_quantize_fp8_pushed(x, x8, {x_hist, x_len, x_idx, x_step, fmax, pow2_margin}, x_maxima, m * k,
+                                                        fmt, s);
+        if (pushed) product_step = x_maxima;
+        else w8a8::launch_quantize_fp8(x, x8, x_step, nullptr, x_maxima, m * k, fmt, s);
         if (w) w8a8::launch_quantize_fp8(w, w8, w_step, nullptr, w_maxima, n * k, fmt, s);
     }
     const int rc = round_first && bias
-        ? astrai_w8a8_gemm_fp8_pt_rounded_bias(x8, w8, x_step, w_step, bias, out, m, n, k, fmt, stream)
-        : astrai_w8a8_gemm_fp8_pt(x8, w8, x_step, w_step, nullptr, bias, out, m, n, k, fmt, ASTRAI_W8A8_OUT_BF16, stream);
+        ? astrai_w8a8_gemm_fp8_pt_rounded_bias(x8, w8, product_step, w_step, bias, out, m, n, k, fmt, stream)
+        : astrai_w8a8_gemm_fp8_pt(x8, w8, product_step, w_step, nullptr, bias, out, m, n, k, fmt, ASTRAI_W8A8_OUT_BF16, stream);
     if (rc) return rc;
     if (!measure && w)
         w8a8::launch_amax_ring_push_pair({x_hist, x_len, x_idx, x_step, fmax, pow2_margin}, x_maxima,
                                          {w_hist, w_len, w_idx, w_step, fmax, pow2_margin}, w_maxima, s);
-    else if (!measure)
+    else if (!measure && !pushed)
         w8a8::launch_amax_ring_push(x_hist, x_len, x_idx, nullptr, x_maxima, nullptr, x_step, fmax, pow2_margin, s);
     return check_launch(what);
 }

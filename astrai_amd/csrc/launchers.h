@@ -83,6 +83,14 @@ struct RingArgs {
     float* scale = nullptr;
     float fmax = 1.0f, pow2_margin = 1.0f;
 };
+// Few elements in one launch each; false (nothing is launched) past the limits or for a remainder of eight. measured.maxima is
+// not read: the quantizer measures, and stores the step to *scale. pushed: with the ring's step, which goes to *used and
+// is then refreshed.
+constexpr int64_t kSmallMeasured = 131072, kSmallPushed = 32768;
+bool launch_quantize_fp8_small(const void* x, void* x8, const MeasuredStep& measured, float* scale, int64_t total, int fmt,
+                               hipStream_t stream);
+bool launch_quantize_fp8_pushed(const void* x, void* x8, const RingArgs& ring, float* used, int64_t total, int fmt,
+                                hipStream_t stream);
 void launch_amax_ring_push_pair(const RingArgs& a, const float* pa, const RingArgs& b, const float* pb, hipStream_t stream);
 void launch_gradient_stats(const float* maxima, float* amax, const float* colsums, void* bias, int64_t rows, int64_t cols,
                            hipStream_t stream, const RingArgs& ring = {});

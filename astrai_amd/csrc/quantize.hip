@@ -270,6 +270,72 @@ __global__ __launch_bounds__(kWave) void amax_ring_push_kernel(
     ring_push_wave(hist, n, idx, fresh, scale, fmax, pow2_margin);
 }
 
+// ---- a few tokens in one launch each -------------------------------------------
+// In place of two launches around the product's own: a launch is 1.6 us of a chain and 2.6 us of the host.
+constexpr int kSmallThreads = 1024;
+
+// Dynamic scaling: every workgroup reads the whole tensor for its maximum (out of L2, one instruction a value where the
+// quantization takes fourteen) and quantizes its own 8192 elements. kBatch: loads under way.
+template <int Fmt, int kBatch>
+__global__ __launch_bounds__(kSmallThreads) void quantize_fp8_small_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ x8,
+                                                                           StepArgs to, int nvec) {
+    __shared__ float slots[kSmallThreads / kWave];
+    const int own = blockIdx.x * kSmallThreads + threadIdx.x;
+    u32x4 mine = {0u, 0u, 0u, 0u};
+    if (own < nvec) mine = *reinterpret_cast<const u32x4*>(x + (int64_t)own * 8);
+    float local = 0.0f;
+    for (int v0 = threadIdx.x; v0 < nvec; v0 += kBatch * kSmallThreads) {
+        u32x4 raw[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const int v = v0 + i * kSmallThreads;
+            raw[i] = u32x4{0u, 0u, 0u, 0u};
+            if (v < nvec) raw[i] = *reinterpret_cast<const u32x4*>(x + (int64_t)v * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            float f[8];
+            unpack8(raw[i], f);
+            local = fmaxf(local, amax8(f));
+        }
+    }
+    const float peak = block_max_t<kSmallThreads>(local, slots);
+    const float step = fmaxf((peak / to.fmax) / to.pow2_margin, 1e-12f);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *to.measured_scale = step;
+    if (own >= nvec) return;
+    float f[8];
+    unpack8(mine, f);
+    *reinterpret_cast<u32x2*>(x8 + (int64_t)own * 8) = quant8_fp8<Fmt>(f, step);
+}
+
+// Delayed scaling: one workgroup quantizes with the ring's step, leaves that step in *used for the product and pushes the
+// maximum. V: vectors of a thread.
+template <int Fmt, int V>
+__global__ __launch_bounds__(kSmallThreads) void quantize_fp8_pushed_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ x8,
+                                                                            RingArgs ring, float* __restrict__ used, int nvec) {
+    __shared__ float slots[kSmallThreads / kWave];
+    u32x4 raw[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int v = threadIdx.x + i * kSmallThreads;
+        raw[i] = u32x4{0u, 0u, 0u, 0u};
+        if (v < nvec) raw[i] = *reinterpret_cast<const u32x4*>(x + (int64_t)v * 8);
+    }
+    const float step = *ring.scale;
+    float local = 0.0f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int v = threadIdx.x + i * kSmallThreads;
+        float f[8];
+        unpack8(raw[i], f);
+        local = fmaxf(local, amax8(f));
+        if (v < nvec) *reinterpret_cast<u32x2*>(x8 + (int64_t)v * 8) = quant8_fp8<Fmt>(f, step);
+    }
+    const float peak = block_max_t<kSmallThreads>(local, slots);   // (by now everyone has read the step)
+    if (threadIdx.x == 0) *used = step;
+    if (threadIdx.x < kWave) ring_push_wave(ring.hist, ring.n, ring.idx, peak, ring.scale, ring.fmax, ring.pow2_margin);
+}
+
 // ---- per-tensor fp8, row-major and transposed codes in one pass -----------
 // The backward of a Linear contracts the gradient over both of its axes
 // (dX = g.w over N, dW = g^T.x over M; csrc/kernels/fp8/mm.cu:298-312 makes
@@ -979,6 +1045,46 @@ void launch_quantize_fp8_measured(const void* x, void* x8, const MeasuredStep& m
                                   hipStream_t stream) {
     launch_quantize_fp8_step<true>(x, x8, nullptr, StepArgs{scale, measured.maxima, measured.fmax, measured.pow2_margin},
                                    nullptr, nullptr, total, fmt, stream);
+}
+
+// The whole Linear, graph replays, us, two launches -> one. Dynamic: 1 token through 2048 x 2048 weights 7.3 -> 5.4, 32 11.1 ->
+// 8.6, 64 (131072 values, the limit) 12.1 -> 11.4; 4096 x 4096, 8 tokens 12.4 -> 9.4, 32 12.9 -> 12.1; at 180000 values the
+// workgroups' reads cost more than the launch (13.6, 14.3). Delayed, weight codes kept: 1 token 7.6 -> 5.9, 8 x 4096
+// values 12.0 -> 11.5: one compute unit's fourteen instructions a value catch up with the launch. Eager calls 2.6 us each less.
+bool launch_quantize_fp8_small(const void* x, void* x8, const MeasuredStep& measured, float* scale, int64_t total, int fmt,
+                               hipStream_t stream) {
+    if (total % 8 || total > kSmallMeasured) return false;
+    const int nvec = (int)(total / 8), blocks = (nvec + kSmallThreads - 1) / kSmallThreads;
+    auto run = [&](auto batch) {
+        constexpr int B = decltype(batch)::value;
+        auto* const kern = fmt ? quantize_fp8_small_kernel<1, B> : quantize_fp8_small_kernel<0, B>;
+        kern<<<dim3((unsigned)blocks), dim3(kSmallThreads), 0, stream>>>(
+            static_cast<const uint16_t*>(x), static_cast<uint8_t*>(x8),
+            StepArgs{scale, nullptr, measured.fmax, measured.pow2_margin}, nvec);
+    };
+    if (blocks == 1) run(std::integral_constant<int, 1>{});
+    else if (blocks == 2) run(std::integral_constant<int, 2>{});
+    else if (blocks <= 4) run(std::integral_constant<int, 4>{});
+    else run(std::integral_constant<int, 8>{});
+    return true;
+}
+
+bool launch_quantize_fp8_pushed(const void* x, void* x8, const RingArgs& ring, float* used, int64_t total, int fmt,
+                                hipStream_t stream) {
+    if (total % 8 || total > kSmallPushed) return false;
+    auto run = [&](auto most) {
+        constexpr int V = decltype(most)::value;
+        auto* const kern = fmt ? quantize_fp8_pushed_kernel<1, V> : quantize_fp8_pushed_kernel<0, V>;
+        kern<<<dim3(1), dim3(kSmallThreads), 0, stream>>>(static_cast<const uint16_t*>(x), static_cast<uint8_t*>(x8), ring, used,
+                                                          (int)(total / 8));
+    };
+    switch ((total + 8 * kSmallThreads - 1) / (8 * kSmallThreads)) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        default: run(std::integral_constant<int, 4>{});
+    }
+    return true;
 }
 
 // Two tensors' pushes side by side, a workgroup each.

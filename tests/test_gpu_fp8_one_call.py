@@ -62,6 +62,17 @@ def test_same_as_the_general_path(monkeypatch, recipe, shape, n, bias, grads, fm
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
 
 
+# one workgroup and part of the next, the limits of the quantizers that measure or push by themselves, just past them
+@pytest.mark.parametrize("recipe", [lambda: fp8.DelayedScaling(history_len=3, margin=1), fp8.DynamicScaling])
+@pytest.mark.parametrize("rows", [1, 512, 513, 1025, 2048, 2049, 4097, 8192, 8193])
+def test_few_values(monkeypatch, recipe, rows):
+    got, calls = _steps(monkeypatch, False, recipe, (rows, 16), 64, True, False, "hybrid", True)
+    want, none = _steps(monkeypatch, True, recipe, (rows, 16), 64, True, False, "hybrid", True)
+    assert all(calls) and len(calls) == 4 and not none
+    for a, b in zip(got, want, strict=True):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("recipe", [lambda: fp8.DelayedScaling(history_len=3, margin=1), fp8.DynamicScaling])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 512), (48, 512, 256), (100, 272, 1024), (130, 1040, 272), (1037, 256, 512)])
 @pytest.mark.parametrize("bias,fmt", [(False, "hybrid"), (True, "hybrid"), (True, "e4m3")])
