@@ -181,8 +181,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
             sc[i] = ok ? sc[i] * a.scale : kNegBig;
             tm = fmaxf(tm, sc[i]);
         }
-        tm = fmaxf(tm, __shfl_xor(tm, 16, kWave));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
+        tm = column_max(tm);
         const float m_new = fmaxf(m, tm);
         const float alpha = __expf(m - m_new);
         float p[4], ps = 0.0f;
@@ -191,8 +190,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
             p[i] = sc[i] <= 0.5f * kNegBig ? 0.0f : __expf(sc[i] - m_new);  // (so that a NaN is not taken for hidden)
             ps += p[i];
         }
-        ps += __shfl_xor(ps, 16, kWave);
-        ps += __shfl_xor(ps, 32, kWave);
+        ps = column_sum(ps);
         l = l * alpha + ps;
         m = m_new;
 
@@ -225,12 +223,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(AttnDecodeArgs
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            float v = acc[q][d];
-            v += __shfl_xor(v, 16, kWave);
-            v += __shfl_xor(v, 32, kWave);
-            acc[q][d] = v;
-        }
+        for (int d = 0; d < 8; ++d) acc[q][d] = column_sum(acc[q][d]);
     if (g == 0) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q)

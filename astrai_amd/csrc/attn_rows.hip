@@ -130,8 +130,7 @@ __device__ __forceinline__ void tile_step(const u32x4 (&kf)[D / 32], const u32x4
         sc[i] = ok ? sc[i] * scale : kNegBig;
         tm = fmaxf(tm, sc[i]);
     }
-    tm = fmaxf(tm, __shfl_xor(tm, 16, kWave));
-    tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
+    tm = column_max(tm);
     const float m_new = fmaxf(m, tm);
     const float alpha = __expf(m - m_new);
     float p[4], ps = 0.0f;
@@ -160,8 +159,7 @@ __device__ __forceinline__ void tile_step(const u32x4 (&kf)[D / 32], const u32x4
 }
 
 __device__ __forceinline__ float query_sum(float l) {
-    l += __shfl_xor(l, 16, kWave);
-    return l + __shfl_xor(l, 32, kWave);
+    return column_sum(l);
 }
 
 // workspace per (row block, kv head, split): kNQ rows of [D values | max | sum]

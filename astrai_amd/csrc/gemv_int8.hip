@@ -87,9 +87,7 @@ __global__ __launch_bounds__(64) void gemv_int8_dot_kernel(GemmArgs g) {
     int mine = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        int v = acc[r];
-#pragma unroll
-        for (int off = 32; off; off >>= 1) v += __shfl_xor(v, off, kWave);
+        const int v = wave_sum_i32(acc[r]);
         if (lane == r) mine = v;
     }
     if (writer) {

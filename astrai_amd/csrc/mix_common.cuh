@@ -18,6 +18,7 @@ using w8a8::kWave;
 using w8a8::pack_bf16x2;
 using w8a8::u32x2;
 using w8a8::u32x4;
+using w8a8::wave_sum;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -135,11 +136,5 @@ __device__ __forceinline__ u32x2 lds_read_tr(const uint8_t* src) {
 }
 
 __device__ __forceinline__ u32x4 join(u32x2 a, u32x2 b) { return u32x4{a.x, a.y, b.x, b.y}; }
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off; off >>= 1) v += __shfl_xor(v, off, kWave);
-    return v;
-}
 
 }  // namespace astrai_mix

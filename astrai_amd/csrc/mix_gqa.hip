@@ -166,8 +166,7 @@ __global__ __launch_bounds__(256) void gqa_partial_kernel(GqaRowsArgs a, GqaDims
                 s[u][e] = (key <= q_pos && key >= q_lo) ? score_of<true>(s[u][e], d) * kLog2e : kNegBig;
                 tm = fmaxf(tm, s[u][e]);
             }
-        tm = fmaxf(tm, __shfl_xor(tm, 16, kWave));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
+        tm = w8a8::column_max(tm);
         const float m_new = fmaxf(m, tm), alpha = __builtin_amdgcn_exp2f(m - m_new);
         m = m_new;
         l *= alpha;
@@ -201,8 +200,7 @@ __global__ __launch_bounds__(256) void gqa_partial_kernel(GqaRowsArgs a, GqaDims
         }
         __builtin_amdgcn_wave_barrier();
     }
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
+    l = w8a8::column_sum(l);
     __syncthreads();
     // the four waves' parts of each query: [wave][query][DV]
     float* const part = reinterpret_cast<float*>(lds);

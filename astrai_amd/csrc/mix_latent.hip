@@ -204,8 +204,7 @@ __global__ __launch_bounds__(256, RH <= 8 ? 2 : 1) void latent_partial_kernel(La
                 tm = fmaxf(tm, p[e + j]);
             }
         }
-        tm = fmaxf(tm, __shfl_xor(tm, 16, kWave));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
+        tm = w8a8::column_max(tm);
         const float m_new = fmaxf(m, tm);
         const float alpha = __builtin_amdgcn_exp2f(m - m_new);
         m = m_new;
@@ -238,8 +237,7 @@ __global__ __launch_bounds__(256, RH <= 8 ? 2 : 1) void latent_partial_kernel(La
         tile(t, 0, ka);
         if (t + 1 < t1) tile(t + 1, 1, kb);
     }
-    l += __shfl_xor(l, 16, kWave);
-    l += __shfl_xor(l, 32, kWave);
+    l = w8a8::column_sum(l);
     if (!live) return;
     // workspace per (row, split): rp values, then maximum and sum
     float* w = a.ws + (((int64_t)b * rows + row) * a.nsplit + split) * (d.rp + 4);

@@ -40,8 +40,15 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     const float* xi = EMBED ? nullptr : a.x_in + row * w;
 
     if constexpr (NV > 0) {
-        f32x4 v[NV];
+        f32x4 v[NV], g_post[NV], g_pre[NV];
         float s = 0.0f;
+        // (the weights with the row: loads do not move ahead of the reductions' barriers by themselves)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int c = (i * kRowThreads + tid) * 4;
+            g_pre[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_pre + c) : f32x4{0, 0, 0, 0};
+            if constexpr (!EMBED) g_post[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_post + c) : f32x4{0, 0, 0, 0};
+        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
@@ -72,9 +79,8 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
             for (int i = 0; i < NV; ++i) {
                 const int c = (i * kRowThreads + tid) * 4;
                 if (c < w) {
-                    const f32x4 g = *reinterpret_cast<const f32x4*>(a.w_post + c);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[i][e] = x[i][e] + v[i][e] * r * g[e];
+                    for (int e = 0; e < 4; ++e) v[i][e] = x[i][e] + v[i][e] * r * g_post[i][e];
                     s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
                 }
             }
@@ -100,10 +106,9 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
             if (c < w) {
-                const f32x4 g = *reinterpret_cast<const f32x4*>(a.w_pre + c);
                 f32x4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[e];
+                for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g_pre[i][e];
                 Elem<T>::put4(h + c, o);
             }
         }
@@ -164,8 +169,14 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     float* xo = a.x_out + row * w;
     T* h = static_cast<T*>(a.h) + row * w;
     if constexpr (NV > 0) {
-        f32x4 v[NV];
+        f32x4 v[NV], g[NV];
         float s = 0.0f;
+        // (the weights with the row: a load does not move ahead of the reduction's barrier by itself)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int c = (i * kRowThreads + tid) * 4;
+            g[i] = a.w && c < w ? *reinterpret_cast<const f32x4*>(a.w + c) : f32x4{0, 0, 0, 0};
+        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
@@ -189,9 +200,8 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
             if (c < w) {
                 f32x4 o = v[i];
                 if (a.w) {
-                    const f32x4 g = *reinterpret_cast<const f32x4*>(a.w + c);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[e];
+                    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[i][e];
                 }
                 Elem<T>::put4(h + c, o);
             }

@@ -432,10 +432,7 @@ __global__ __launch_bounds__(kThreads) void quantize_transpose_fp8_kernel(
         }
         if constexpr (STATS) {   // over the wave's four row groups (lanes 16 apart)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                sum[j] += __shfl_xor(sum[j], 16, kWave);
-                sum[j] += __shfl_xor(sum[j], 32, kWave);
-            }
+            for (int j = 0; j < 8; ++j) sum[j] = column_sum(sum[j]);
             if ((threadIdx.x & 63) < 16) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) sums[threadIdx.x >> 6][cc * 8 + j] = sum[j];
@@ -739,9 +736,7 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
                 for (int j = 0; j < 8; ++j) ssw[c & 3] += v[c][j] * v[c][j];
             }
 #pragma unroll
-            for (int wv = 0; wv < 4; ++wv)
-#pragma unroll
-                for (int off = 32; off; off >>= 1) ssw[wv] += __shfl_xor(ssw[wv], off, kWave);
+            for (int wv = 0; wv < 4; ++wv) ssw[wv] = wave_sum(ssw[wv]);
             float ss = ssw[0];
 #pragma unroll
             for (int wv = 1; wv < 4; ++wv) ss += ssw[wv];

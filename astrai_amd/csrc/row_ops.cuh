@@ -90,8 +90,7 @@ __device__ __forceinline__ float block_max_t(float v, float* slots) {
 
 // block-wide sum of a per-thread value; result valid in every thread
 __device__ __forceinline__ float block_sum(float v, float* slots) {
-#pragma unroll
-    for (int off = 32; off; off >>= 1) v += __shfl_xor(v, off, kWave);
+    v = wave_sum(v);
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) slots[wave] = v;
     __syncthreads();
