@@ -20,13 +20,14 @@ bool dense(const Tensor* t, c10::Device dev, int64_t rows, int64_t cols) {   // 
 bool near16(const Tensor& t, uintptr_t q = 16) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % q == 0; }
 
 struct FewRows {
-    const Tensor *x, *w, *bias;
+    const Tensor *x, *w, *bias = nullptr;
     int64_t act, most, m, n, k, ldx;   // act -1: none
     // x, weight, bias, act, most rows
     bool read(PyObject* const* a) {
-        if (!(x = tensor_of(a[0])) || !(w = tensor_of(a[1])) || !optional(a[2], bias) || !whole(a[3], act) || !whole(a[4], most) ||
-            !x->is_cuda() || x->dim() < 1 || w->dim() != 2)
-            return false;
+        return (x = tensor_of(a[0])) && (w = tensor_of(a[1])) && optional(a[2], bias) && whole(a[3], act) && whole(a[4], most) && fits();
+    }
+    bool fits() {
+        if (!x->is_cuda() || x->dim() < 1 || w->dim() != 2) return false;
         const auto dev = x->device();
         n = w->size(0) / (act < 0 ? 1 : 2), k = w->size(1), m = k ? x->numel() / k : 0;
         if (x->size(-1) != k || m <= 0 || m > most || k % 128 || n % 4 || w->numel() * 2 >= (int64_t)1 << 31 ||
@@ -46,6 +47,25 @@ PyObject* few_rows_linear_takes(PyObject*, PyObject* const* a, Py_ssize_t n_args
     FewRows r;
     if (n_args == 5 && r.read(a)) Py_RETURN_TRUE;
     Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+// few_rows_parts(x, weight, most, parts)
+PyObject* few_rows_parts(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    FewRows r;
+    int64_t parts;
+    if (n_args != 4 || !whole(a[3], parts) || parts < 1) Py_RETURN_NONE;
+    r.act = -1;
+    if (!(r.x = tensor_of(a[0])) || !(r.w = tensor_of(a[1])) || !whole(a[2], r.most) || !r.fits()) Py_RETURN_NONE;
+    const auto dev = r.x->device();
+    const c10::DeviceGuard guard(dev);
+    Tensor out = at::empty({parts, r.m, r.n}, at::TensorOptions().device(dev).dtype(at::kFloat));
+    const int rc = unlocked([&] {
+        return astrai_mix_few_rows_parts(r.x->data_ptr(), r.ldx, r.w->data_ptr(), out.data_ptr<float>(), r.m, r.n, r.k, parts,
+                                         stream_of(dev));
+    });
+    return rc ? failed(rc) : THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
 
@@ -73,12 +93,14 @@ PyObject* sum_norm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     double eps, mult;
     if (n_args != 10 || !(y = tensor_of(a[0])) || !optional(a[1], w) || !PyBool_Check(a[2]) || !real(a[3], eps) || !optional(a[4], x) ||
         !optional(a[5], u) || !optional(a[6], vec) || !optional(a[7], tokens) || !real(a[8], mult) || !optional(a[9], given) ||
-        !y->is_cuda() || y->dim() != 2)
+        !y->is_cuda() || (y->dim() != 2 && y->dim() != 3))
         Py_RETURN_NONE;
     const auto dev = y->device();
     const auto type = a[2] == Py_True ? at::kBFloat16 : at::kFloat;
-    const int64_t width = y->size(1), n = tokens ? tokens->numel() : y->size(0);
-    for (const Tensor* t : {y, u})
+    const bool parts = y->dim() == 3;   // planes to add up
+    const int64_t width = y->size(-1), n = tokens ? tokens->numel() : y->size(-2);
+    if (parts && (y->scalar_type() != at::kFloat || tokens || y->stride(2) != 1 || y->stride(1) < width)) Py_RETURN_NONE;
+    for (const Tensor* t : {parts ? u : y, u})
         if (t && (t->dim() != 2 || t->size(1) != width || t->stride(1) != 1 || t->stride(0) < width || t->device() != dev ||
                   t->scalar_type() != y->scalar_type() || (t->scalar_type() != type && t->scalar_type() != at::kFloat)))
             Py_RETURN_NONE;
@@ -90,6 +112,10 @@ PyObject* sum_norm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     Tensor out = given ? *given : at::empty({n, width}, on.dtype(at::kFloat)), h = at::empty({n, width}, on.dtype(type));
     const int rc = unlocked([&] {
         auto vector = [](const Tensor* t) { return t ? t->data_ptr<float>() : nullptr; };
+        if (parts)
+            return astrai_mix_sum_norm_parts(y->data_ptr<float>(), y->stride(1), y->stride(0), y->size(0), (float)mult, vector(x), vector(u),
+                                             u ? u->stride(0) : 0, vector(vec), out.data_ptr<float>(), vector(w), h.data_ptr(), n, width,
+                                             (float)eps, type == at::kFloat, stream_of(dev));
         return astrai_mix_sum_norm(y->data_ptr(), y->stride(0), tokens ? tokens->data_ptr<int64_t>() : nullptr, y->size(0), (float)mult,
                                    vector(x), ptr(u), u ? u->stride(0) : 0, vector(vec), out.data_ptr<float>(), vector(w),
                                    h.data_ptr(), n, width, (float)eps, y->scalar_type() == at::kFloat, type == at::kFloat,
@@ -107,17 +133,23 @@ PyObject* residual_norm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor *y, *x, *post, *pre;
     double mult, eps;
     if (n_args != 6 || !(y = tensor_of(a[0])) || !(x = tensor_of(a[1])) || !(post = tensor_of(a[2])) || !(pre = tensor_of(a[3])) ||
-        !real(a[4], mult) || !real(a[5], eps) || !y->is_cuda() || y->dim() != 2)
+        !real(a[4], mult) || !real(a[5], eps) || !y->is_cuda() || (y->dim() != 2 && y->dim() != 3))
         Py_RETURN_NONE;
     const auto dev = y->device();
-    const auto type = y->scalar_type();
-    const int64_t n = y->size(0), width = y->size(1);
+    const bool parts = y->dim() == 3;   // fp32 planes to add up, h in bf16
+    if (parts && y->scalar_type() != at::kFloat) Py_RETURN_NONE;
+    const auto type = parts ? at::kBFloat16 : y->scalar_type();
+    const int64_t n = y->size(-2), width = y->size(-1);
     if ((type != at::kBFloat16 && type != at::kFloat) || !y->is_contiguous() || !dense(x, dev, n, width) ||
         !dense(post, dev, -1, width) || !dense(pre, dev, -1, width))
         Py_RETURN_NONE;
     const c10::DeviceGuard guard(dev);
     Tensor h = at::empty({n, width}, at::TensorOptions().device(dev).dtype(type));
     const int rc = unlocked([&] {
+        if (parts)
+            return astrai_mix_residual_norm_parts(y->data_ptr<float>(), n * width, y->size(0), x->data_ptr<float>(), x->data_ptr<float>(),
+                                                  post->data_ptr<float>(), pre->data_ptr<float>(), h.data_ptr(), n, width, (float)mult,
+                                                  (float)eps, stream_of(dev));
         return astrai_mix_residual_norm(y->data_ptr(), x->data_ptr<float>(), x->data_ptr<float>(), post->data_ptr<float>(),
                                         pre->data_ptr<float>(), h.data_ptr(), n, width, (float)mult, (float)eps, type == at::kFloat,
                                         stream_of(dev));
@@ -126,7 +158,7 @@ PyObject* residual_norm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {ENTRY(few_rows_linear_takes), ENTRY(few_rows_linear), ENTRY(sum_norm), ENTRY(residual_norm), {nullptr, nullptr, 0, nullptr}};
+PyMethodDef methods[] = {ENTRY(few_rows_linear_takes), ENTRY(few_rows_linear), ENTRY(few_rows_parts), ENTRY(sum_norm), ENTRY(residual_norm), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_mix", nullptr, -1, methods};
 
 }  // namespace

@@ -221,8 +221,21 @@ int astrai_mix_residual_norm(const void* y, const float* x_in, float* x_out, con
         return fail(ASTRAI_MIX_BAD_ARG, "residual_norm: bad size %lld x %lld", (long long)rows, (long long)width);
     if (rows == 0) return ASTRAI_MIX_OK;
     ResidualNormArgs a = {y, nullptr, x_in, x_out, w_post, w_pre, h, rows, 0, (int)width, mult, eps};
-    launch_residual_norm(a, dtype, static_cast<hipStream_t>(stream));
+    launch_residual_norm(a, dtype, false, static_cast<hipStream_t>(stream));
     return check_launch("residual_norm");
+}
+
+int astrai_mix_residual_norm_parts(const float* y, int64_t plane, int64_t parts, const float* x_in, float* x_out, const float* w_post,
+                                   const float* w_pre, void* h, int64_t rows, int64_t width, float mult, float eps, void* stream) {
+    MIX_TRY(check_ptrs("residual_norm_parts", (const void*)y, (const void*)x_in, (const void*)x_out, (const void*)w_post,
+                       (const void*)w_pre, (const void*)h));
+    if (rows < 0 || rows > kMaxInt || width <= 0 || width > (1 << 24) || parts < 1 || parts > kMaxParts || plane < rows * width)
+        return fail(ASTRAI_MIX_BAD_ARG, "residual_norm_parts: bad size %lld x %lld x %lld", (long long)parts, (long long)rows,
+                    (long long)width);
+    if (rows == 0) return ASTRAI_MIX_OK;
+    ResidualNormArgs a = {y, nullptr, x_in, x_out, w_post, w_pre, h, rows, 0, (int)width, mult, eps, (int)parts, plane};
+    launch_residual_norm(a, ASTRAI_MIX_BF16, true, static_cast<hipStream_t>(stream));
+    return check_launch("residual_norm_parts");
 }
 
 int astrai_mix_embed_norm(const void* table, const int64_t* tokens, float* x_out, const float* w_pre, void* h,
@@ -235,7 +248,7 @@ int astrai_mix_embed_norm(const void* table, const int64_t* tokens, float* x_out
                     (long long)vocab);
     if (rows == 0) return ASTRAI_MIX_OK;
     ResidualNormArgs a = {table, tokens, nullptr, x_out, nullptr, w_pre, h, rows, vocab, (int)width, 0.0f, eps};
-    launch_residual_norm(a, dtype, static_cast<hipStream_t>(stream));
+    launch_residual_norm(a, dtype, false, static_cast<hipStream_t>(stream));
     return check_launch("embed_norm");
 }
 
@@ -256,6 +269,23 @@ int astrai_mix_sum_norm(const void* y, int64_t ldy, const int64_t* tokens, int64
     const SumNormArgs a = {y, ldy, tokens, x_in, u, u ? ldu : 0, vec, x_out, w, h, rows, vocab, (int)width, mult, eps};
     launch_sum_norm(a, dtype, y_float != 0, static_cast<hipStream_t>(stream));
     return check_launch("sum_norm");
+}
+
+int astrai_mix_sum_norm_parts(const float* y, int64_t ldy, int64_t plane, int64_t parts, float mult, const float* x_in, const float* u,
+                              int64_t ldu, const float* vec, float* x_out, const float* w, void* h, int64_t rows, int64_t width,
+                              float eps, int dtype, void* stream) {
+    MIX_TRY(check_dtype("sum_norm_parts", dtype));
+    MIX_TRY(check_ptrs("sum_norm_parts", (const void*)y, (const void*)x_out, (const void*)h));
+    for (const void* p : {(const void*)x_in, (const void*)u, (const void*)vec, (const void*)w})
+        if (p) MIX_TRY(check_ptrs("sum_norm_parts", p));
+    if (rows < 0 || rows > kMaxInt || width <= 0 || width > (1 << 24) || ldy < width || ldy > kMaxInt || (u && ldu < width) ||
+        parts < 1 || parts > kMaxParts || plane < (rows - 1) * ldy + width)
+        return fail(ASTRAI_MIX_BAD_ARG, "sum_norm_parts: bad size %lld x %lld x %lld (strides %lld, %lld)", (long long)parts,
+                    (long long)rows, (long long)width, (long long)ldy, (long long)ldu);
+    if (rows == 0) return ASTRAI_MIX_OK;
+    const SumNormArgs a = {y, ldy, nullptr, x_in, u, u ? ldu : 0, vec, x_out, w, h, rows, 0, (int)width, mult, eps, (int)parts, plane};
+    launch_sum_norm(a, dtype, true, static_cast<hipStream_t>(stream));
+    return check_launch("sum_norm_parts");
 }
 
 int astrai_mix_act_mul(const void* gu, void* h, int64_t rows, int64_t ff, int act, int dtype, void* stream) {
@@ -284,6 +314,20 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
         return fail(ASTRAI_MIX_UNSUPPORTED, "few_rows_linear: %lld x %lld x %lld is not covered", (long long)m, (long long)n,
                     (long long)k);
     return check_launch("few_rows_linear");
+}
+
+int astrai_mix_few_rows_parts(const void* x, int64_t ldx, const void* w, float* out, int64_t m, int64_t n, int64_t k, int64_t parts,
+                              void* stream) {
+    MIX_TRY(check_ptrs("few_rows_parts", x, w, (const void*)out));
+    if (m < 0 || m > kMaxInt || n <= 0 || n > kMaxInt || k <= 0 || k > kMaxInt || ldx < k || parts < 1 || parts > kMaxParts)
+        return fail(ASTRAI_MIX_BAD_ARG, "few_rows_parts: bad size %lld x %lld x %lld, %lld parts", (long long)m, (long long)n,
+                    (long long)k, (long long)parts);
+    if (m == 0) return ASTRAI_MIX_OK;
+    const FewRowsArgs a = {x, ldx, w, nullptr, out, (int)m, (int)n, (int)k, (int)parts};
+    if (!few_rows_linear_supported(m, n, k, false) || !launch_few_rows_linear(a, -1, true, static_cast<hipStream_t>(stream)))
+        return fail(ASTRAI_MIX_UNSUPPORTED, "few_rows_parts: %lld x %lld x %lld is not covered", (long long)m, (long long)n,
+                    (long long)k);
+    return check_launch("few_rows_parts");
 }
 
 int astrai_mix_prompt_linear_takes(int64_t m, int64_t n, int64_t k, int64_t ldx, int act) {

@@ -20,8 +20,11 @@ struct ResidualNormArgs {
     int64_t rows, vocab;
     int width;
     float mult, eps;
+    int parts = 1;          // y is the sum of so many planes, fp32
+    int64_t plane = 0;
 };
-void launch_residual_norm(const ResidualNormArgs& a, int dtype, hipStream_t stream);
+// y_float: y is float with bf16 h
+void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool y_float, hipStream_t stream);
 
 struct SumNormArgs {
     const void* y;          // [rows, ldy], or the embedding table [vocab, ldy] with `tokens`
@@ -37,6 +40,8 @@ struct SumNormArgs {
     int64_t rows, vocab;
     int width;
     float mult, eps;        // mult multiplies y
+    int parts = 1;          // y is the sum of so many planes, fp32
+    int64_t plane = 0;
 };
 // y_float: y and u are float with bf16 h
 void launch_sum_norm(const SumNormArgs& a, int dtype, bool y_float, hipStream_t stream);
@@ -51,9 +56,11 @@ struct FewRowsArgs {
     int64_t ldx;
     const void* w;     // bf16 [n, k]; with an activation [2 n, k], gate rows first
     const void* bias;  // bf16 [n] or null
-    void* out;         // [m, n]
+    void* out;         // [m, n]; of several splits of K [splits, m, n] fp32
     int m, n, k;
+    int splits = 1;
 };
+constexpr int kMaxParts = 4;   // most planes of sums that a row norm adds up
 bool few_rows_linear_supported(int64_t m, int64_t n, int64_t k, bool act);
 // act: kActSilu / kActGelu (out = act(gate) * up), or -1
 bool launch_few_rows_linear(const FewRowsArgs& a, int act, bool out_float, hipStream_t stream);

@@ -12,6 +12,11 @@
 // refilled for the next item as soon as it has been consumed: the bytes in flight stay the same from the first
 // instruction to the last, when nothing is left to request. The waves' partial sums are added through LDS in wave order.
 //
+// Several ranges of K by workgroups of their own (splits) make the row ranges longer and the part of x that a workgroup reads
+// shorter: x is most of the bytes that a workgroup pulls out of L2 where the weights have few rows. The fp32 sums of the
+// ranges lie in planes that the row norm behind the product adds up. With that norm (us, one range / four): 32 rows of 5632 ->
+// 2048 14.2 / 10.8, 2048 -> 2048 9.1 / 8.2; 16 rows 12.6 / 9.9, 8.2 / 7.5; 1 row 9.7 / 9.1, 7.2 / 7.2.
+//
 // What bounds it (graph replays over weights that no cache holds): the stream from 20 MB on (2048 -> 32000, 131 MB, 22.5 us at 1
 // token, 5.8 TB/s), below it launch and the load path's 16 cycles for every 1 KiB instruction, of x as much as of the
 // weights: leaving out those for rows and tokens that are not there and those past the last item took 2048 -> 2048 from 4.3
@@ -57,7 +62,8 @@ __global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a,
     const int lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int items = a.k / (kItem / 2);
-    const int i0 = wave * items / NW, i1 = (wave + 1) * items / NW;
+    const int part = blockIdx.y * NW + wave, parts = gridDim.y * NW;   // (blockIdx.y: a range of K whose sums stand by themselves)
+    const int i0 = part * items / parts, i1 = (part + 1) * items / parts;
     const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, a.n);
     const uint32_t w_row = (uint32_t)a.k * 2, x_row = (uint32_t)a.ldx * 2;
     const __amdgpu_buffer_rsrc_t rw = w8a8::make_rsrc(a.w, (uint32_t)(HALVES * a.n) * w_row);
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(NW * 64) void few_rows_linear_kernel(FewRowsArgs a,
         const int m = (t % MB) * 16 + c16, row = r0 + (t / MB) * 16 + g * 4;
         if (m >= a.m || row >= r1) continue;
         f32x4 v = total(t);
-        const int64_t at = (int64_t)m * a.n + row;
+        const int64_t at = ((int64_t)blockIdx.y * a.m + m) * a.n + row;
         if constexpr (ACT >= 0) {
             const f32x4 up = total(t + RG * MB);
 #pragma unroll
@@ -182,7 +188,7 @@ void launch_inst(const FewRowsArgs& a, int rows, hipStream_t stream) {
     constexpr int lds = NW * (units > 8192 ? units : 8192);
     static_assert(lds <= 64 * 1024, "within the limit that needs no attribute");
     few_rows_linear_kernel<RG, MB, NW, ACT, F32, WH, XH, IB>
-        <<<dim3((unsigned)((a.n + rows - 1) / rows)), dim3(NW * 64), lds, stream>>>(a, rows);
+        <<<dim3((unsigned)((a.n + rows - 1) / rows), (unsigned)a.splits), dim3(NW * 64), lds, stream>>>(a, rows);
 }
 
 template <int RG, int NW, int ACT, bool F32, bool WH>
@@ -209,7 +215,7 @@ void launch_rg(const FewRowsArgs& a, hipStream_t stream) {
     // rows dealt out over 256 workgroups (a multiple of them where a range would be over GROUPS * 16 rows),
     // in fours: one load instruction
     constexpr int GROUPS = ACT >= 0 ? 2 : kMaxGroups;
-    const int wgs = 256 * ((a.n + 256 * GROUPS * 16 - 1) / (256 * GROUPS * 16));
+    const int round = 256 / a.splits, wgs = round * ((a.n + round * GROUPS * 16 - 1) / (round * GROUPS * 16));
     const int rows = ((a.n + wgs - 1) / wgs + 3) & ~3;
     if (rows > 32) {
         if constexpr (GROUPS == 3) launch_wh<3, 4, ACT, F32>(a, rows, stream);
@@ -233,6 +239,7 @@ bool launch_few_rows_linear(const FewRowsArgs& a, int act, bool out_float, hipSt
     if (!few_rows_linear_supported(a.m, a.n, a.k, act >= 0) || a.ldx < a.k || a.ldx % 8 ||
         (int64_t)kFewRowsMax * a.ldx * 2 >= ((int64_t)1 << 31))
         return false;
+    if (a.splits != 1 && (a.splits < 1 || a.splits > kMaxParts || act >= 0 || !out_float || a.bias)) return false;
     if (act == kActGelu) launch_rg<kActGelu, false>(a, stream);
     else if (act == kActSilu) launch_rg<kActSilu, false>(a, stream);
     else if (out_float) launch_rg<-1, true>(a, stream);

@@ -18,10 +18,33 @@ namespace astrai_mix {
 
 namespace {
 
+// four columns of y, or of the sum of its planes (requested together, added in order)
+template <typename TY, typename A>
+__device__ __forceinline__ f32x4 sum4(const TY* y, const A& a) {
+    f32x4 v = Elem<TY>::get4(y);
+    if constexpr (sizeof(TY) == 4) {
+        if (a.parts == 4) {
+            const f32x4 p = Elem<TY>::get4(y + a.plane), q = Elem<TY>::get4(y + 2 * a.plane), r = Elem<TY>::get4(y + 3 * a.plane);
+            v = ((v + p) + q) + r;
+        } else {
+            for (int i = 1; i < a.parts; ++i) v += Elem<TY>::get4(y + i * a.plane);
+        }
+    }
+    return v;
+}
+
+template <typename TY, typename A>
+__device__ __forceinline__ float sum1(const TY* y, const A& a) {
+    float v = Elem<TY>::get(y);
+    if constexpr (sizeof(TY) == 4)
+        for (int i = 1; i < a.parts; ++i) v += Elem<TY>::get(y + i * a.plane);
+    return v;
+}
+
 // NV > 0: the row sits in NV registers of four per thread (width % 4 == 0, width <= 1024 NV).
 // NV == 0: any width, scalar accesses, x_out is the storage between the passes (a thread reads
 // back only what it wrote).
-template <typename T, int NV, bool EMBED>
+template <typename T, typename TY, int NV, bool EMBED>
 __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNormArgs a) {
     __shared__ float slots[kRowThreads / kWave];
     const int64_t row = blockIdx.x;
@@ -29,13 +52,13 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     const float inv_w = 1.0f / (float)w;
     float* xo = a.x_out + row * w;
     T* h = static_cast<T*>(a.h) + row * w;
-    const T* y = nullptr;
+    const TY* y = nullptr;
     if constexpr (EMBED) {
         int64_t tok = a.tokens[row];
         tok = tok < 0 ? 0 : (tok >= a.vocab ? a.vocab - 1 : tok);
-        y = static_cast<const T*>(a.y) + tok * w;
+        y = static_cast<const TY*>(a.y) + tok * w;
     } else {
-        y = static_cast<const T*>(a.y) + row * w;
+        y = static_cast<const TY*>(a.y) + row * w;
     }
     const float* xi = EMBED ? nullptr : a.x_in + row * w;
 
@@ -52,7 +75,7 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
-            v[i] = c < w ? Elem<T>::get4(y + c) : f32x4{0, 0, 0, 0};
+            v[i] = c < w ? sum4(y + c, a) : f32x4{0, 0, 0, 0};
             s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
         }
         if constexpr (!EMBED) {
@@ -115,17 +138,17 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     } else {
         float mean = 0.0f, r = 0.0f, s = 0.0f, q = 0.0f;
         if constexpr (!EMBED) {
-            for (int c = tid; c < w; c += kRowThreads) s += Elem<T>::get(y + c);
+            for (int c = tid; c < w; c += kRowThreads) s += sum1(y + c, a);
             mean = block_sum(s, slots) * inv_w;
             for (int c = tid; c < w; c += kRowThreads) {
-                const float d = Elem<T>::get(y + c) - mean;
+                const float d = sum1(y + c, a) - mean;
                 q += d * d;
             }
             r = a.mult / sqrtf(block_sum(q, slots) * inv_w + a.eps);
         }
         s = q = 0.0f;
         for (int c = tid; c < w; c += kRowThreads) {
-            float v = Elem<T>::get(y + c);
+            float v = sum1(y + c, a);
             if constexpr (!EMBED) v = xi[c] + (v - mean) * r * a.w_post[c];
             xo[c] = v;
             s += v;
@@ -140,15 +163,15 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     }
 }
 
-template <typename T, bool EMBED>
+template <typename T, typename TY, bool EMBED>
 void residual_norm_t(const ResidualNormArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)a.rows), block(kRowThreads);
     const int w = a.width;
-    if (w % 4 != 0 || w > 8192) residual_norm_kernel<T, 0, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 1024) residual_norm_kernel<T, 1, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 2048) residual_norm_kernel<T, 2, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 4096) residual_norm_kernel<T, 4, EMBED><<<grid, block, 0, stream>>>(a);
-    else residual_norm_kernel<T, 8, EMBED><<<grid, block, 0, stream>>>(a);
+    if (w % 4 != 0 || a.plane % 4 != 0 || w > 8192) residual_norm_kernel<T, TY, 0, EMBED><<<grid, block, 0, stream>>>(a);
+    else if (w <= 1024) residual_norm_kernel<T, TY, 1, EMBED><<<grid, block, 0, stream>>>(a);
+    else if (w <= 2048) residual_norm_kernel<T, TY, 2, EMBED><<<grid, block, 0, stream>>>(a);
+    else if (w <= 4096) residual_norm_kernel<T, TY, 4, EMBED><<<grid, block, 0, stream>>>(a);
+    else residual_norm_kernel<T, TY, 8, EMBED><<<grid, block, 0, stream>>>(a);
 }
 
 // x <- mult * (table[token] or y) + x_in + u + vec, each but the first optional; h = x / sqrt(mean(x^2) + eps) * w,
@@ -182,7 +205,7 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
             const int c = (i * kRowThreads + tid) * 4;
             v[i] = f32x4{0, 0, 0, 0};
             if (c < w) {
-                v[i] = Elem<TY>::get4(y + c);
+                v[i] = sum4(y + c, a);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[i][e] *= a.mult;
                 if (xi) v[i] += *reinterpret_cast<const f32x4*>(xi + c);
@@ -209,7 +232,7 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     } else {
         float s = 0.0f, r = 1.0f;
         for (int c = tid; c < w; c += kRowThreads) {
-            float v = Elem<TY>::get(y + c) * a.mult;
+            float v = sum1(y + c, a) * a.mult;
             if (xi) v += xi[c];
             if (u) v += Elem<TY>::get(u + c);
             if (a.vec) v += a.vec[c];
@@ -225,7 +248,7 @@ template <typename T, typename TY>
 void sum_norm_t(const SumNormArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)a.rows), block(kRowThreads);
     const int w = a.width;
-    if (w % 4 != 0 || a.ldy % 4 != 0 || a.ldu % 4 != 0 || w > 8192) sum_norm_kernel<T, TY, 0><<<grid, block, 0, stream>>>(a);
+    if (w % 4 != 0 || a.ldy % 4 != 0 || a.plane % 4 != 0 || a.ldu % 4 != 0 || w > 8192) sum_norm_kernel<T, TY, 0><<<grid, block, 0, stream>>>(a);
     else if (w <= 1024) sum_norm_kernel<T, TY, 1><<<grid, block, 0, stream>>>(a);
     else if (w <= 2048) sum_norm_kernel<T, TY, 2><<<grid, block, 0, stream>>>(a);
     else if (w <= 4096) sum_norm_kernel<T, TY, 4><<<grid, block, 0, stream>>>(a);
@@ -317,13 +340,14 @@ __global__ __launch_bounds__(256) void head_gated_rms_norm_kernel(HeadNormArgs a
 
 }  // namespace
 
-void launch_residual_norm(const ResidualNormArgs& a, int dtype, hipStream_t stream) {
+void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool y_float, hipStream_t stream) {
     if (dtype) {
-        if (a.tokens) residual_norm_t<float, true>(a, stream);
-        else residual_norm_t<float, false>(a, stream);
+        if (a.tokens) residual_norm_t<float, float, true>(a, stream);
+        else residual_norm_t<float, float, false>(a, stream);
     } else {
-        if (a.tokens) residual_norm_t<uint16_t, true>(a, stream);
-        else residual_norm_t<uint16_t, false>(a, stream);
+        if (a.tokens) residual_norm_t<uint16_t, uint16_t, true>(a, stream);
+        else if (y_float) residual_norm_t<uint16_t, float, false>(a, stream);
+        else residual_norm_t<uint16_t, uint16_t, false>(a, stream);
     }
 }
 

@@ -42,6 +42,10 @@ PROTOTYPES = {
         [_P, _I64, _P, _I64, _F32, _P, _P, _I64] + [_P] * 4 + [_I64, _I64, _F32, _INT, _INT, _P], _INT),
     "astrai_mix_act_mul": ([_P, _P, _I64, _I64, _INT, _INT, _P], _INT),
     "astrai_mix_few_rows_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _INT, _P], _INT),
+    "astrai_mix_few_rows_parts": ([_P, _I64, _P, _P] + [_I64] * 4 + [_P], _INT),
+    "astrai_mix_sum_norm_parts": (
+        [_P] + [_I64] * 3 + [_F32, _P, _P, _I64] + [_P] * 4 + [_I64, _I64, _F32, _INT, _P], _INT),
+    "astrai_mix_residual_norm_parts": ([_P, _I64, _I64] + [_P] * 5 + [_I64, _I64, _F32, _F32, _P], _INT),
     "astrai_mix_prompt_linear_takes": ([_I64] * 4 + [_INT], _INT),
     "astrai_mix_prompt_linear": ([_P, _I64, _P, _P, _P] + [_I64] * 3 + [_INT, _P], _INT),
     "astrai_mix_head_gated_rms_norm": ([_P, _P, _I64, _P, _P] + [_I64] * 4 + [_F32, _INT, _P], _INT),
@@ -154,11 +158,14 @@ def pad_to(n: int, q: int = HEAD_PAD) -> int:
 
 def residual_norm(y: torch.Tensor, x: torch.Tensor, w_post: torch.Tensor, w_pre: torch.Tensor, mult: float,
                   eps: float) -> torch.Tensor:
-    """``x += mult * LN(y) * w_post`` (in place, fp32) and ``LN(x) * w_pre`` in ``y``'s dtype, returned."""
+    """``x += mult * LN(y) * w_post`` (in place, fp32) and ``LN(x) * w_pre`` in ``y``'s dtype, returned. Planes of
+    :func:`few_rows_parts` for ``y``: of their sum, bf16."""
     lib = _require()
     h = _host.residual_norm(y, x, w_post, w_pre, mult, eps)
     if h is not None:
         return h
+    if y.dim() == 3:
+        raise RuntimeError("residual_norm: planes, residual and weights do not fit")
     n, width = y.shape
     code = _dtype(y, "residual_norm")
     _dense("residual_norm", y.dtype, y)
@@ -199,12 +206,15 @@ def sum_norm(y: torch.Tensor, w: Optional[torch.Tensor], dtype: torch.dtype, eps
     """The residual ``mult * y + x + u + vec`` in fp32 (every term but the first optional; ``y`` the table whose rows
     ``tokens`` are taken, if given) and its RMS norm times ``w`` in ``dtype`` (without ``w``: the residual itself).
     ``y [n, width]`` and ``u`` may be rows of a wider matrix and have one type, ``dtype`` or float32. The residual
-    goes to ``out`` (which may be ``x``) or a new tensor. Returns (residual, normed)."""
+    goes to ``out`` (which may be ``x``) or a new tensor. Planes of :func:`few_rows_parts` for ``y``: their sum. Returns
+    (residual, normed)."""
     lib = _require()
     if dtype in _DTYPES:
         both = _host.sum_norm(y, w, dtype == torch.bfloat16, eps, x, u, vec, tokens, mult, out)
         if both is not None:
             return both
+    if y.dim() == 3:
+        raise RuntimeError("sum_norm: planes and terms do not fit")
     width = y.size(1)
     n = y.size(0) if tokens is None else tokens.numel()
     code = _DTYPES[dtype]
@@ -299,6 +309,19 @@ def few_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
         _check(lib.astrai_mix_few_rows_linear(
             x.data_ptr(), k if x.is_contiguous() else x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
             out.data_ptr(), m, n, k, -1 if act is None else ACTIVATIONS[act], int(out_dtype == torch.float32), _stream(x)), lib)
+    return out
+
+
+MAX_PARTS = 4
+
+
+def few_rows_parts(x: torch.Tensor, weight: torch.Tensor, parts: int) -> torch.Tensor:
+    """:func:`few_rows_linear` without a bias as ``[parts, rows, outputs]`` fp32 sums over ranges of K, whose sum the row norms
+    take for the product."""
+    _require()
+    out = _host.few_rows_parts(x, weight, FEW_ROWS, parts)
+    if out is None:
+        raise RuntimeError("few_rows_parts: operands are not covered")
     return out
 
 

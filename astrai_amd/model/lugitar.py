@@ -21,7 +21,7 @@ from torch import Tensor
 from astrai_amd.extension import _mix
 from astrai_amd.model.cache import MixerCache
 from astrai_amd.model.mixers import (Fp32Vector, GatedMLP, LatentAttention, LightningAttention, MixerLM, Rotation,
-                                     assign_checked)
+                                     assign_checked, fed, mixed)
 
 
 @dataclass
@@ -115,10 +115,10 @@ class LugitarLM(MixerLM):
         pre = [layer.norm1.weight for layer in self.layers] + [self.final_norm.weight]
         x, h = _mix.embed_norm(self.embed.weight, input_ids.reshape(-1).contiguous(), pre[0], eps)
         for i, layer in enumerate(self.layers):
-            y = layer.mix(h, ctx)
+            y = mixed(layer.mix, h, ctx)
             if layer.mlp is None:
                 h = _mix.residual_norm(y, x, layer.norm1b.weight, pre[i + 1], mult, eps)
             else:
                 h = _mix.residual_norm(y, x, layer.norm1b.weight, layer.norm2.weight, mult, eps)
-                h = _mix.residual_norm(layer.mlp(h), x, layer.norm2b.weight, pre[i + 1], mult, eps)
+                h = _mix.residual_norm(fed(layer.mlp, h), x, layer.norm2b.weight, pre[i + 1], mult, eps)
         return self.finish(h, x, ctx, logits_at)

@@ -55,6 +55,7 @@ class StepContext:
     batch: int
     seq: int
     run: int = 0
+    parts: bool = False   # the layer's caller adds up what `rows_out` leaves in planes
 
 
 @dataclass(frozen=True)
@@ -161,6 +162,27 @@ def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
     elif few_rows(x, weight, bias):
         return _mix.few_rows_linear(x, weight, bias)
     return F.linear(x, weight, bias)
+
+
+def parts_of(rows: int, n: int, k: int) -> int:
+    """Ranges of K in which a product of few rows is left for the row norm behind it to add up (:func:`_mix.few_rows_parts`): four
+    where the weight has few rows of many values, so that x is most of what a workgroup reads, else one. With the norm (us, one /
+    four): 2048 x 5632 of 1, 8, 32 rows 9.7 / 9.1, 10.6 / 9.5, 14.2 / 10.8; 2048 x 2048 7.2 / 7.2, 7.6 / 7.4, 9.1 / 8.2; 1024 x
+    2816 7.0 / 6.1, 7.4 / 6.3, 9.0 / 7.1; 3072 x 8192 14.0 / 14.4, 14.2 / 14.3, 21.5 / 15.9; 4096 x 11008 of 8, 16 rows 22.7 / 22.4,
+    25.1 / 23.1. Others gain nothing or lose: 2048 x 1024 of 16 rows 6.7 / 6.8, 4096 x 4096 13.8 / 14.0, 6144 x 6144 21.4 / 21.5."""
+    if k < 2048:
+        return 1
+    return _mix.MAX_PARTS if n <= 2048 or (n <= 3072 and rows >= 8) or (n <= 4096 and k >= 2 * n and rows >= 12) else 1
+
+
+def rows_out(module: nn.Module, x: Tensor, parts: bool) -> Tensor:
+    """``module(x)``; with ``parts``, the output of a ``PackedLinear`` as planes that add up to it, where that pays."""
+    if parts and type(module) is PackedLinear and module.bias is None and not observed(module) and x.size(-1):
+        w = module.weight
+        planes = parts_of(x.numel() // x.size(-1), *w.shape)
+        if planes > 1 and few_rows(x, w):
+            return _mix.few_rows_parts(x, w, planes)
+    return module(x)
 
 
 class HeadLinear(Linear):
@@ -420,7 +442,7 @@ class LatentAttention(nn.Module):
             kv = F.linear(c[0] if ctx.batch == 1 else c.reshape(-1, s.rp), self.w_ukv)
             kv = kv.reshape(ctx.batch, -1, kv.size(-1))
             out = _mix.latent_prefill(proj, s, g_off, kv, latent, ctx.start, first)
-        return self.o(out)
+        return rows_out(self.o, out, ctx.parts)
 
 
 class LightningAttention(nn.Module):
@@ -458,7 +480,7 @@ class LightningAttention(nn.Module):
         step = ctx.seq <= LIGHTNING_STEP_MAX or proj.dtype != torch.bfloat16 or not _mix.lightning_chunk_supported(self.dp)
         o = _mix.lightning(proj, off["q"], off["k"], off["v"], self.decay.weight.view(self.heads, -1),
                            ctx.cache.state[self.layer], step)
-        return self.o(_mix.gated_rms_norm(o, proj, off["g"], self.norm.weight, self.count, self.eps))
+        return rows_out(self.o, _mix.gated_rms_norm(o, proj, off["g"], self.norm.weight, self.count, self.eps), ctx.parts)
 
 
 class GroupedAttention(nn.Module):
@@ -509,7 +531,7 @@ class GroupedAttention(nn.Module):
         else:
             out = _mix.gqa_rows(proj, s, off["g"], kv, ctx.positions,
                                 matrix=bf16 and _mix.gqa_rows_supported(s, ctx.cache.max_len))
-        return self.o(out)
+        return rows_out(self.o, out, ctx.parts)
 
 
 class GatedRecurrence(nn.Module):
@@ -568,7 +590,7 @@ class GatedRecurrence(nn.Module):
             u = _mix.conv(proj, off["x"], self.conv.weight, self.conv.bias.weight, ring, ctx.positions, silu=False)
             w = [m.weight if matrix else m.transposed for m in (self.r, self.i)]
             out = _mix.rglru(u, proj, off["y"], *w, *gates, matrix=matrix)
-        return self.o(out)
+        return rows_out(self.o, out, ctx.parts)
 
 
 class ChannelDelta(nn.Module):
@@ -635,7 +657,7 @@ class ChannelDelta(nn.Module):
                 out = _mix.head_gated_rms_norm(o, gate, self.norm.weight, s.vdim, self.eps)
             else:
                 out = _mix.delta_step(proj, *rule, gate, self.norm.weight, state, self.eps, qkv=qkv)
-        return self.o(out)
+        return rows_out(self.o, out, ctx.parts)
 
 
 class GatedMLP(nn.Module):
@@ -651,13 +673,29 @@ class GatedMLP(nn.Module):
             for name, t in assign_checked("feed-forward", lin.expected(), tensors, prefix).items():
                 lin.assign(name, t)
 
-    def forward(self, h: Tensor) -> Tensor:
+    def forward(self, h: Tensor, parts: bool = False) -> Tensor:
         up, rows = self.gate_up, h.numel() // max(h.size(-1), 1)
         if (rows <= _mix.FEW_ROWS or rows >= PROMPT_ROWS) and type(up) is PackedLinear and up.bias is None and not observed(up):
             fused, pays = ((_mix.few_rows_linear, few_rows) if rows <= _mix.FEW_ROWS else (_mix.prompt_linear, prompt_rows))
             if pays(h, up.weight, act=self.act):
-                return self.down(fused(h, up.weight, act=self.act))
-        return self.down(_mix.act_mul(self.gate_up(h), self.act))
+                return rows_out(self.down, fused(h, up.weight, act=self.act), parts)
+        return rows_out(self.down, _mix.act_mul(self.gate_up(h), self.act), parts)
+
+
+MIXERS = (LatentAttention, LightningAttention, GroupedAttention, GatedRecurrence, ChannelDelta)
+
+
+def mixed(mix: nn.Module, h: Tensor, ctx: StepContext) -> Tensor:
+    """``mix(h, ctx)``, possibly as planes that add up to it: where nothing but the row norm sees the result."""
+    ctx.parts = type(mix) in MIXERS and not observed(mix)
+    y = mix(h, ctx)
+    ctx.parts = False
+    return y
+
+
+def fed(mlp: nn.Module, h: Tensor) -> Tensor:
+    """``mlp(h)`` likewise."""
+    return mlp.forward(h, True) if type(mlp) is GatedMLP and not observed(mlp) else mlp(h)
 
 
 class MixerLM(nn.Module):

@@ -23,7 +23,7 @@ from torch import Tensor
 from astrai_amd.extension import _mix
 from astrai_amd.model.cache import MixerCache
 from astrai_amd.model.mixers import (ChannelDelta, Fp32Vector, GatedMLP, GatedRecurrence, GroupedAttention, MixerLM,
-                                     PackedLinear, Rotation, Rows, assign_checked, columns_of, linear_f32)
+                                     PackedLinear, Rotation, Rows, assign_checked, columns_of, fed, linear_f32, mixed)
 
 NO_LOOP = (0, 0, 0)
 
@@ -187,10 +187,10 @@ class SarulixLM(MixerLM):
                 else:
                     y = linear_f32(h, self.loop_in.weight[:b])[:, :w]
                 _, h = _mix.sum_norm(y, layer.norm1.weight, dtype, eps, u=u, vec=self.loop_step[ctx.run].weight, out=x)
-            y = layer.mix(h, ctx)
+            y = mixed(layer.mix, h, ctx)
             if layer.mlp is not None:
                 _, h = _mix.sum_norm(y, layer.norm2.weight, dtype, eps, x=x, out=x)
-                y = layer.mlp(h)
+                y = fed(layer.mlp, h)
             _, h = _mix.sum_norm(y, pre[k + 1], dtype, eps, x=x, out=x)
             if residuals is not None:
                 residuals.append(x.reshape(ctx.batch, ctx.seq, w).clone())

@@ -75,6 +75,18 @@ int astrai_mix_few_rows_linear(const void* x, int64_t ldx, const void* w, const 
                                int64_t n, int64_t k, int act, int out_float, void* stream);
 
 /*
+ * Its fp32 sums over `parts` (at most 4) ranges of K, [parts, m, n] in a plane each, for the row norms below to add up; and those
+ * norms: astrai_mix_sum_norm and astrai_mix_residual_norm (bf16 h) of the sum of y's planes, `plane` floats apart.
+ */
+int astrai_mix_few_rows_parts(const void* x, int64_t ldx, const void* w, float* out, int64_t m, int64_t n, int64_t k, int64_t parts,
+                              void* stream);
+int astrai_mix_sum_norm_parts(const float* y, int64_t ldy, int64_t plane, int64_t parts, float mult, const float* x_in, const float* u,
+                              int64_t ldu, const float* vec, float* x_out, const float* w, void* h, int64_t rows, int64_t width,
+                              float eps, int dtype, void* stream);
+int astrai_mix_residual_norm_parts(const float* y, int64_t plane, int64_t parts, const float* x_in, float* x_out, const float* w_post,
+                                   const float* w_pre, void* h, int64_t rows, int64_t width, float mult, float eps, void* stream);
+
+/*
  * The same of a prompt's rows, on 256 x 256 tiles, bf16 out; k % 64 == 0, n % 8 == 0, x, w and 256 rows of out each under
  * 2 GiB (x and w with 256 rows more). The sums run in one order whatever m is. _takes: whether it takes these sizes.
  */

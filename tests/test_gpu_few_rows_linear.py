@@ -83,3 +83,71 @@ def test_calls_that_are_left_to_the_library():
     assert w.grad is not None
     with pytest.raises(RuntimeError, match="not covered"):
         _mix.few_rows_linear(_mk(1, 65, 256), w)
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 512), (17, 200, 128), (8, 2048, 4224), (33, 3076, 1280), (64, 132, 2048)])
+def test_planes_of_ranges_add_up(parts, m, n, k):
+    """Ranges without items, row ranges of one to three groups, a remainder of rows."""
+    from astrai_amd.extension import _mix
+    x, w = _mk(1, m, k), _mk(2, n, k)
+    planes = _mix.few_rows_parts(x, w, parts)
+    assert planes.shape == (parts, m, n) and planes.dtype == torch.float32
+    exact, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    # fp32 sums: k + parts roundings at most, far fewer in effect
+    assert ((planes.double().sum(0) - exact).abs() <= 2.0 ** -24 * (k + parts) * size).all()
+    assert torch.equal(planes, _mix.few_rows_parts(x, w, parts))
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4])
+@pytest.mark.parametrize("rows,width", [(1, 33), (5, 128), (3, 1000), (9, 2048), (2, 5000), (2, 8200)])
+def test_row_norms_of_planes(parts, rows, width):
+    """Against the norms of the planes' sum, formed in the same order."""
+    from astrai_amd.extension import _mix
+    g = torch.Generator(device=DEV).manual_seed(width + parts)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    planes, x, u, w, v = rand(parts, rows, width), rand(rows, width), rand(rows, width), rand(width), rand(width)
+    total = planes[0].clone()
+    for p in planes[1:]:
+        total += p
+    for more in ({}, {"u": u}, {"vec": v, "mult": 0.5}):
+        got = _mix.sum_norm(planes, w, torch.bfloat16, 1e-5, x=x, **more)
+        want = _mix.sum_norm(total, w, torch.bfloat16, 1e-5, x=x, **more)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    wide = rand(parts, rows, width + 8)
+    got, want = _mix.sum_norm(wide[:, :, :width], w, torch.bfloat16, 1e-5), _mix.sum_norm(wide[:, :, :width].contiguous(), w, torch.bfloat16, 1e-5)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    xs = [x.clone(), x.clone()]
+    got, want = _mix.residual_norm(planes, xs[0], w, v, 0.5, 1e-5), _mix.residual_norm(total, xs[1], w, v, 0.5, 1e-5)
+    assert torch.equal(xs[0], xs[1]) and torch.equal(got, want.bfloat16()) and got.dtype == torch.bfloat16
+    for bad in (planes.bfloat16(), planes[:, :, :-1]):
+        with pytest.raises(RuntimeError):
+            _mix.sum_norm(bad, w, torch.bfloat16, 1e-5)
+
+
+def test_planes_stay_between_a_layer_and_its_norm():
+    """Hooks, wrappers and subclasses see the products; the model's results are those of either way."""
+    from astrai_amd.model import mixers
+    for n, k in ((2048, 5632), (2048, 2048)):
+        assert mixers.parts_of(16, n, k) == 4
+    assert mixers.parts_of(16, 4096, 4096) == mixers.parts_of(16, 2048, 1024) == 1
+    mlp = mixers.GatedMLP(512, 2176)
+    for product in (mlp.gate_up, mlp.down):
+        product.reset_parameters()
+    mlp = mlp.to(DEV).to(torch.bfloat16)
+    h, seen = _mk(3, 16, 512), []
+    with torch.no_grad():
+        assert mixers.fed(mlp, h).shape == (4, 16, 512)
+        want = mlp(h)
+        assert want.shape == (16, 512)
+        assert ((mixers.fed(mlp, h).sum(0) - want.float()).norm() / want.float().norm()) < 2.0 ** -8
+        for module in (mlp, mlp.down):
+            hook = module.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+            assert mixers.fed(mlp, h).shape == (16, 512) and seen.pop() == (16, 512)
+            hook.remove()
+
+        class Other(mixers.GatedMLP):
+            pass
+
+        other = Other(512, 2176).to(DEV).to(torch.bfloat16)
+        assert mixers.fed(other, h).shape == (16, 512)
