@@ -772,4 +772,44 @@ int astrai_mix_delta_chunk(const void* qkv, const void* proj, int64_t ld, int64_
     return check_launch("delta_chunk");
 }
 
+int64_t astrai_mix_delta_blocks_bytes(int64_t batch, int64_t heads, int64_t seq, int64_t dp, int64_t vp) {
+    if (batch < 0 || heads <= 0 || seq < 0 || dp <= 0 || dp % 32 || vp <= 0 || vp % 32 || batch > kMaxInt || heads > kMaxInt || seq > kMaxInt ||
+        vp > kMaxInt || !delta_chunk_supported((int)dp, (int)vp))
+        return -1;
+    return delta_blocks_bytes(batch, heads, seq, (int)dp, (int)vp);
+}
+
+int astrai_mix_delta_blocks(const void* qkv, const void* proj, int64_t ld, int64_t b_off, const float* z,
+                            const float* dt_bias, const float* decay, float* state, void* image, void* out, int64_t batch,
+                            int64_t seq, int64_t heads, int64_t kv_heads, int64_t dp, int64_t vp, float q_scale,
+                            void* stream) {
+    MIX_TRY(check_ptrs("delta_blocks", qkv, proj, (const void*)z, (const void*)dt_bias, (const void*)decay,
+                       (const void*)state, (const void*)image, (const void*)out));
+    MIX_TRY(check_delta("delta_blocks", ld, b_off, batch, seq, heads, kv_heads, dp, vp));
+    if (batch > kMaxGridYZ) return fail(ASTRAI_MIX_BAD_ARG, "delta_blocks: batch %lld", (long long)batch);
+    if (!delta_chunk_supported((int)dp, (int)vp))
+        return fail(ASTRAI_MIX_UNSUPPORTED, "delta_blocks: head size %lld (at most 256)", (long long)dp);
+    DeltaArgs a = {};
+    a.qkv = qkv;
+    a.ldq = 2 * kv_heads * dp + heads * vp;
+    a.proj = proj;
+    a.ld = ld;
+    a.b_off = (int)b_off;
+    a.z = z;
+    a.dt_bias = dt_bias;
+    a.decay = decay;
+    a.state = state;
+    a.image = image;
+    a.out = out;
+    a.batch = (int)batch;
+    a.seq = (int)seq;
+    a.heads = (int)heads;
+    a.kv_heads = (int)kv_heads;
+    a.dp = (int)dp;
+    a.vp = (int)vp;
+    a.q_scale = q_scale;
+    launch_delta_blocks(a, static_cast<hipStream_t>(stream));
+    return check_launch("delta_blocks");
+}
+
 }  // extern "C"

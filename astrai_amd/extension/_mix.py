@@ -72,6 +72,8 @@ PROTOTYPES = {
         [_P, _P] + [_I64] * 3 + [_P, _I64] + [_P] * 6 + [_I64] + [_P] * 3 + [_I64] * 7 + [_F32, _F32, _INT, _P], _INT),
     "astrai_mix_delta_image_bytes": ([_I64], _I64),
     "astrai_mix_delta_chunk": ([_P, _P, _I64, _I64] + [_P] * 6 + [_I64] * 6 + [_F32, _P], _INT),
+    "astrai_mix_delta_blocks_bytes": ([_I64] * 5, _I64),
+    "astrai_mix_delta_blocks": ([_P, _P, _I64, _I64] + [_P] * 6 + [_I64] * 6 + [_F32, _P], _INT),
 }
 
 _lib: Optional[ctypes.CDLL] = None
@@ -885,6 +887,17 @@ def delta_chunk_supported(s: DeltaShape) -> bool:
     return s.dp <= 256
 
 
+def delta_in_blocks(batch: int, seq: int, s: DeltaShape) -> bool:
+    """Whether :func:`delta_chunk` walks blocks of 64 tokens rather than 16: where the walk from block to block is what
+    takes the time, that is few heads, at most one column block to a compute unit, and a prompt long enough for it to be more
+    than the longer preparation. Measured in us, 16 and 64 tokens, heads x size, batch x length: 16 x 128 1 x 4096 212 and 159,
+    1 x 1024 64 and 55, 1 x 640 49 and 45, 1 x 512 41 and 41, 1 x 300 29 and 34, 2 x 2048 143 and 135, 2 x 768 62 and 61,
+    3 x 1024 109 and 110, 4 x 1024 127 and 136, 8 x 1024 220 and 279; 4 x 128 1 x 4096 176 and 108; 32 x 64 1 x 4096 195 and
+    178, 2 x 2048 140 and 157; 32 x 32 1 x 2048 94 and 79; 8 x 256 1 x 2048 170 and 113, 2 x 1024 112 and 90, 8 x 1024 325 and
+    358."""
+    return batch * s.heads <= 32 and batch * s.heads * s.vp <= 4096 and seq >= 640
+
+
 def _delta_checks(what: str, s: DeltaShape, proj, b_off, z, dt_bias, decay, state):
     n = proj.size(0)
     _dense(what, proj.dtype, proj)
@@ -937,17 +950,21 @@ def delta_step(proj: torch.Tensor, s: DeltaShape, b_off: int, z: torch.Tensor, d
 
 
 def delta_chunk(qkv: torch.Tensor, proj: torch.Tensor, s: DeltaShape, b_off: int, z: torch.Tensor,
-                dt_bias: torch.Tensor, decay: torch.Tensor, state: torch.Tensor) -> torch.Tensor:
-    """The same recurrence in chunks on the matrix cores (bf16); returns ``o``, neither normed nor gated."""
+                dt_bias: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, blocks: Optional[bool] = None) -> torch.Tensor:
+    """The same recurrence in chunks on the matrix cores (bf16); returns ``o``, neither normed nor gated. ``blocks``: of 64
+    tokens, else of 16 (None: :func:`delta_in_blocks`)."""
     lib = _require()
     batch, seq = _delta_checks("delta_chunk", s, proj, b_off, z, dt_bias, decay, state)
     _dense("delta_chunk", torch.bfloat16, proj, qkv)
     _shape("delta_chunk", qkv, proj.size(0), s.qkv_cols)
     with _on_device(proj.device):
         out = torch.empty((proj.size(0), s.heads * s.vp), device=proj.device, dtype=proj.dtype)
-        size = lib.astrai_mix_delta_image_bytes(s.dp) * batch * s.heads * -(-seq // DELTA_CHUNK)
+        if blocks is None:
+            blocks = delta_in_blocks(batch, seq, s)
+        size = (lib.astrai_mix_delta_blocks_bytes(batch, s.heads, seq, s.dp, s.vp) if blocks
+                else lib.astrai_mix_delta_image_bytes(s.dp) * batch * s.heads * -(-seq // DELTA_CHUNK))
         image = torch.empty(size, device=proj.device, dtype=torch.uint8)
-        _check(lib.astrai_mix_delta_chunk(
+        _check((lib.astrai_mix_delta_blocks if blocks else lib.astrai_mix_delta_chunk)(
             qkv.data_ptr(), proj.data_ptr(), proj.size(1), b_off, z.data_ptr(), dt_bias.data_ptr(), decay.data_ptr(),
             state.data_ptr(), image.data_ptr(), out.data_ptr(), batch, seq, s.heads, s.kv_heads, s.dp, s.vp, s.q_scale,
             _stream(proj)), lib)

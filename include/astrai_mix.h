@@ -224,7 +224,8 @@ int astrai_mix_rglru_step(const void* proj, int64_t ld, int64_t y_off, int64_t x
  * _step (bf16 or float): out = o / sqrt(mean(o^2) + eps) * norm_w * sigmoid(gate) per head (vdim real columns, gate rows
  * of stride ldg). qkv null (seq <= RING_STEPS): convolves proj's columns from x_off itself and updates the ring.
  * UNSUPPORTED unless vp <= 256 and dp * (vp / 4 rounded up to a power of two, at least 8) <= 16384.
- * _chunk (bf16, dp <= 256): out = o; image: delta_image_bytes * batch * heads * ceil(seq / DELTA_CHUNK) bytes. */
+ * _chunk (bf16, dp <= 256): out = o; image: delta_image_bytes * batch * heads * ceil(seq / DELTA_CHUNK) bytes.
+ * _blocks: the same in blocks of 64 tokens; image: delta_blocks_bytes (-1: sizes not covered). */
 int astrai_mix_delta_step(const void* qkv, const void* proj, int64_t ld, int64_t x_off, int64_t b_off,
                           const float* conv_w, int64_t taps, void* ring, const int64_t* positions, const float* z,
                           const float* dt_bias, const float* decay, const void* gate, int64_t ldg, const float* norm_w,
@@ -235,6 +236,11 @@ int astrai_mix_delta_chunk(const void* qkv, const void* proj, int64_t ld, int64_
                            const float* dt_bias, const float* decay, float* state, void* image, void* out, int64_t batch,
                            int64_t seq, int64_t heads, int64_t kv_heads, int64_t dp, int64_t vp, float q_scale,
                            void* stream);
+int64_t astrai_mix_delta_blocks_bytes(int64_t batch, int64_t heads, int64_t seq, int64_t dp, int64_t vp);
+int astrai_mix_delta_blocks(const void* qkv, const void* proj, int64_t ld, int64_t b_off, const float* z,
+                            const float* dt_bias, const float* decay, float* state, void* image, void* out, int64_t batch,
+                            int64_t seq, int64_t heads, int64_t kv_heads, int64_t dp, int64_t vp, float q_scale,
+                            void* stream);
 
 #ifdef __cplusplus
 }

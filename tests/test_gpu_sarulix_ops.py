@@ -516,6 +516,38 @@ def test_delta_rule_with_equal_keys(dtype):
         c.check(c.run([40, 30], kind), TOL[dtype])
 
 
+@pytest.mark.parametrize("shape", DELTAS + [(9, 3, 32, 64)], ids=str)
+def test_delta_rule_in_blocks(shape, monkeypatch):
+    """Blocks of 64 tokens whatever the size: at their edges, under decays whose products over- and underflow, and with one
+    key over and over. (Seed: one of 2^-9 of a convolved input, where its bf16 rounding falls the other way than the oracle's,
+    is 1.8e-4 of the state under seed 129, in chunks of 16 alike. 80 equal keys: what their writes leave is a difference of
+    rounded inputs, 1.3e-2 of the output after 150 in chunks of 16 alike.)"""
+    monkeypatch.setattr(_mix, "delta_in_blocks", lambda *a: True)
+    for cuts in ([1, 63, 64, 65], [16, 17, 128, 129], [33, 191]):
+        log("delta blocks", shape, cuts)
+        c = Delta(shape, 3, BF16, sum(cuts), batch=2, seed=shape[2] + 2)
+        c.check(c.run(cuts, "chunk"), TOL[BF16])
+    c = Delta(shape, 2, BF16, 144, seed=8, z_std=1.0)
+    c.z[..., ::3] = 60.0
+    c.z[..., 1::3] = -60.0
+    c.z[:, 20:24] = 30.0
+    c.a_log[:] = 0.5
+    c.check(c.run([100, 44], "chunk"), TOL[BF16])
+    c = Delta(shape, 1, BF16, 80, seed=9)
+    c.k[:] = c.k[:, :1]
+    c.b[:], c.z[:] = 6.0, -30.0
+    c.a_log[:] = -6.0
+    c.check(c.run([66, 14], "chunk"), TOL[BF16])
+
+
+def test_delta_rule_in_blocks_where_they_are_taken():
+    shape = (2, 1, 64, 64)
+    for batch, n in ((1, 640), (2, 1030)):
+        assert _mix.delta_in_blocks(batch, n, DeltaShape(2, 1, 64, 64, 64, 0.125))
+        c = Delta(shape, 3, BF16, n, batch=batch, seed=11)
+        c.check(c.run([n], "chunk"), TOL[BF16])
+
+
 def test_a_write_far_back_is_read():
     """One strong write whose key no later key touches, decays all but 1: its value comes back hundreds of tokens
     later, through chunks and steps alike."""
