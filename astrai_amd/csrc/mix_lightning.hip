@@ -2,8 +2,8 @@
 //   S_t = decay S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t,
 // q, k, v being silu of the projections (rounded to the activation type). The state is fp32.
 //
-// Chunk kernel (prompts, bf16). A workgroup takes one head, a slice of 32 or 64 value columns and
-// a segment of the sequence, walking it in chunks of 64 tokens:
+// Chunk kernel (prompts, bf16). A workgroup takes one head, a slice of 32, 64 or 128 value columns
+// and a segment of the sequence, walking it in chunks of 64 tokens:
 //   o_i   = decay^(i+1) S^T q_i + sum_(j <= i) decay^(i-j) (q_i . k_j) v_j
 //   S_new = decay^n S + sum_j decay^(n-1-j) k_j v_j^T
 // on v_mfma_f32_16x16x32_bf16, outputs transposed (value columns as rows, tokens as columns): the
@@ -11,6 +11,15 @@
 // 32-bit factor -- the decayed scores, the state, the decay-weighted values -- enters the matrix
 // cores as two bf16 terms; the state itself stays in fp32 accumulators, wave w owning its rows
 // 16 (w + 4 i) ...
+//
+// What bounds it is the vector arithmetic, most of it silu (an exponential and a reciprocal a value).
+// Slices of 64 columns form silu of a head's q and k once each; where there are workgroups for every
+// compute unit, eight waves take 128 columns and pass q to each other through LDS too, half of the
+// waves to either 64 columns. 16 heads of 128 x 128, slices of 64 and of 128, in us: 32 x 512 tokens
+// 147 and 139, 8 x 2048 204 and 176, 1 x 4096 68 and 63, 4 x 1024 69 and 61; 64 heads, 1 x 8192 375
+// and 331; 32 heads of 96 columns, 16 x 512 134 and 119. With fewer than 256 workgroups the smaller
+// ones are more and faster: 4 x 200 32 and 34, 1 x 300 36 and 39. Converting the next chunk while
+// half of the waves multiply, so that both units work: 140, nothing.
 //
 // With few heads, a long prompt is cut into segments that run side by side: one pass forms every
 // segment's own contribution to the state, a scan turns those into the state each segment starts
@@ -26,15 +35,19 @@ namespace {
 
 constexpr int kC = kLightningChunk;
 
-template <int DP, int VS, bool OUT>
-__global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel(LightningArgs a) {
-    constexpr int kKRow = DP * 2 + 16, kVRow = VS * 2 + 16, kSRow = DP * 2 + 16;   // bytes
+template <int DP, int VS, int W, bool OUT>
+__global__ __launch_bounds__(W * 64, DP <= 128 ? 2 : 1) void lightning_chunk_kernel(LightningArgs a) {
+    constexpr int NT = W * 64, VW = VS * 4 / W;       // value columns of a wave
+    constexpr bool kShareQ = OUT && W == 8;
+    constexpr int kPad = W == 8 ? 32 : 16;            // (32: no bank conflicts in the transposing reads; 16 where two workgroups have to fit)
+    constexpr int kKRow = DP * 2 + kPad, kVRow = VS * 2 + kPad, kSRow = DP * 2 + 16;   // bytes
     constexpr int ND = DP / 32;                       // score steps
     constexpr int NDT = (DP / 16 + 3) / 4;            // state row tiles of a wave
-    constexpr int NVT = VS / 16;
+    constexpr int NVT = VW / 16;
     constexpr int KC8 = DP / 8, VC8 = VS / 8;
-    constexpr int NKL = kC * KC8 / 256, NVL = (kC * VC8 + 255) / 256;
+    constexpr int NKL = kC * KC8 / NT, NVL = (kC * VC8 + NT - 1) / NT, NQ = kShareQ ? NKL : ND;
     __shared__ __attribute__((aligned(16))) uint8_t lk[kC * kKRow];
+    __shared__ __attribute__((aligned(16))) uint8_t lq[kShareQ ? kC * kKRow : 16];
     __shared__ __attribute__((aligned(16))) uint8_t lv[OUT ? kC * kVRow : 16];
     __shared__ __attribute__((aligned(16))) uint8_t lvh[kC * kVRow];
     __shared__ __attribute__((aligned(16))) uint8_t lvl[kC * kVRow];
@@ -43,7 +56,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
     __shared__ float pw[kC + 1];
 
     const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = all & 3, c0 = (all >> 2) * VW;
     const int seg = blockIdx.x, v0 = (int)blockIdx.y * VS;
     const int b = (int)blockIdx.z / a.heads, head = (int)blockIdx.z % a.heads;
     const int chunks = (a.seq + kC - 1) / kC, per_seg = (chunks + a.nseg - 1) / a.nseg;
@@ -54,7 +67,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
     const int64_t state_sz = (int64_t)a.dp * a.vp;
     float* own = a.state + ((int64_t)b * a.heads + head) * state_sz;
     float* segp = a.nseg > 1 ? a.seg_state + (((int64_t)b * a.heads + head) * a.nseg + seg) * state_sz : own;
-    // state: rows d = 16 (wave + 4 i) + 4 g + e, columns v0 + 16 vt + c16
+    // state: rows d = 16 (wave + 4 i) + 4 g + e, columns v0 + c0 + 16 vt + c16
     f32x4 st[NDT][NVT];
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
@@ -62,34 +75,34 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
         for (int vt = 0; vt < NVT; ++vt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int dd = 16 * (wave + 4 * i) + 4 * g + e, v = v0 + 16 * vt + c16;
+                const int dd = 16 * (wave + 4 * i) + 4 * g + e, v = v0 + c0 + 16 * vt + c16;
                 st[i][vt][e] = (OUT && dd < a.dp && v < a.vp) ? segp[(int64_t)dd * a.vp + v] : 0.0f;
             }
 
     const uint16_t* base = static_cast<const uint16_t*>(a.proj) + (int64_t)b * a.seq * a.ld;
     const uint16_t* kp = base + a.k_off + head * a.dp;
     const uint16_t* vp = base + a.v_off + head * a.vp + v0;
-    const uint16_t* qp = base + a.q_off + head * a.dp + 8 * g;
+    const uint16_t* qp = base + a.q_off + head * a.dp;
     const u32x4 zero = {0, 0, 0, 0};
-    u32x4 rk[NKL], rv[NVL], rq[ND];
+    u32x4 rk[NKL], rv[NVL], rq[NQ];
     auto fetch = [&](int t0) {
 #pragma unroll
         for (int i = 0; i < NKL; ++i) {
-            const int c = tid + i * 256, t = t0 + c / KC8, e = (c % KC8) * 8;
+            const int c = tid + i * NT, t = t0 + c / KC8, e = (c % KC8) * 8;
             rk[i] = (t < tok1 && e < a.dp) ? *reinterpret_cast<const u32x4*>(kp + (int64_t)t * a.ld + e) : zero;
         }
 #pragma unroll
         for (int i = 0; i < NVL; ++i) {
-            const int c = tid + i * 256, t = t0 + c / VC8, e = (c % VC8) * 8;
+            const int c = tid + i * NT, t = t0 + c / VC8, e = (c % VC8) * 8;
             rv[i] = (c < kC * VC8 && t < tok1 && v0 + e < a.vp) ? *reinterpret_cast<const u32x4*>(vp + (int64_t)t * a.ld + e)
                                                                  : zero;
         }
         if constexpr (OUT) {
-            const int t = t0 + wave * 16 + c16;
 #pragma unroll
-            for (int i = 0; i < ND; ++i)
-                rq[i] = (t < tok1 && i * 32 + 8 * g < a.dp) ? *reinterpret_cast<const u32x4*>(qp + (int64_t)t * a.ld + i * 32)
-                                                            : zero;
+            for (int i = 0; i < NQ; ++i) {
+                const int c = tid + i * NT, t = t0 + (kShareQ ? c / KC8 : wave * 16 + c16), e = kShareQ ? (c % KC8) * 8 : i * 32 + 8 * g;
+                rq[i] = (t < tok1 && e < a.dp) ? *reinterpret_cast<const u32x4*>(qp + (int64_t)t * a.ld + e) : zero;
+            }
         }
     };
     if (tok0 < tok1) fetch(tok0);
@@ -99,7 +112,12 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
         u32x4 qf[ND];
         if constexpr (OUT) {
 #pragma unroll
-            for (int i = 0; i < ND; ++i) qf[i] = silu8_bf16(rq[i]);
+            for (int i = 0; i < NQ; ++i) {
+                const u32x4 q = silu8_bf16(rq[i]);
+                const int c = tid + i * NT;
+                if constexpr (kShareQ) *reinterpret_cast<u32x4*>(lq + (c / KC8) * kKRow + (c % KC8) * 16) = q;
+                else qf[i] = q;
+            }
             // the state the chunk starts from, [v][d], two terms
 #pragma unroll
             for (int i = 0; i < NDT; ++i)
@@ -110,7 +128,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
                         uint32_t h0, l0, h1, l1;
                         split2(st[i][vt][0], st[i][vt][1], h0, l0);
                         split2(st[i][vt][2], st[i][vt][3], h1, l1);
-                        const int off = (16 * vt + c16) * kSRow + dd * 2;
+                        const int off = (c0 + 16 * vt + c16) * kSRow + dd * 2;
                         *reinterpret_cast<u32x2*>(lsh + off) = u32x2{h0, h1};
                         *reinterpret_cast<u32x2*>(lsl + off) = u32x2{l0, l1};
                     }
@@ -118,12 +136,12 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
         }
 #pragma unroll
         for (int i = 0; i < NKL; ++i) {
-            const int c = tid + i * 256;
+            const int c = tid + i * NT;
             *reinterpret_cast<u32x4*>(lk + (c / KC8) * kKRow + (c % KC8) * 16) = silu8_bf16(rk[i]);
         }
 #pragma unroll
         for (int i = 0; i < NVL; ++i) {
-            const int c = tid + i * 256, j = c / VC8;
+            const int c = tid + i * NT, j = c / VC8;
             if (c < kC * VC8) {
                 const int off = j * kVRow + (c % VC8) * 16;
                 const u32x4 v = silu8_bf16(rv[i]);
@@ -145,6 +163,10 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
         }
         __syncthreads();
         fetch(t0 + kC);
+        if constexpr (kShareQ) {
+#pragma unroll
+            for (int i = 0; i < ND; ++i) qf[i] = *reinterpret_cast<const u32x4*>(lq + (wave * 16 + c16) * kKRow + i * 64 + g * 16);
+        }
 
         // transposed operands: group g supplies contraction rows 4g .. 4g+3 and 16 + 4g .. of a
         // 32-row step, the order in which the score accumulators hold their keys
@@ -157,7 +179,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
                     o[vt] = f32x4{0, 0, 0, 0};
 #pragma unroll
                     for (int i = 0; i < ND; ++i) {
-                        const int off = (16 * vt + c16) * kSRow + i * 64 + g * 16;
+                        const int off = (c0 + 16 * vt + c16) * kSRow + i * 64 + g * 16;
                         o[vt] = mfma16(*reinterpret_cast<const u32x4*>(lsh + off), qf[i], o[vt]);
                         o[vt] = mfma16(*reinterpret_cast<const u32x4*>(lsl + off), qf[i], o[vt]);
                     }
@@ -192,7 +214,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
                             lo[2 * u] = l0;
                             lo[2 * u + 1] = l1;
                         }
-                        const uint8_t* v = lv + (p * 32 + tr_row) * kVRow + tr_col;
+                        const uint8_t* v = lv + (p * 32 + tr_row) * kVRow + c0 * 2 + tr_col;
 #pragma unroll
                         for (int vt = 0; vt < NVT; ++vt) {
                             const u32x4 vf = join(lds_read_tr(v + vt * 32), lds_read_tr(v + vt * 32 + 16 * kVRow));
@@ -203,10 +225,10 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
                 }
                 const int t = t0 + qt;
                 if (t < tok1) {
-                    uint16_t* out = static_cast<uint16_t*>(a.out) + (((int64_t)b * a.seq + t) * a.heads + head) * a.vp + v0;
+                    uint16_t* out = static_cast<uint16_t*>(a.out) + (((int64_t)b * a.seq + t) * a.heads + head) * a.vp + v0 + c0;
 #pragma unroll
                     for (int vt = 0; vt < NVT; ++vt)
-                        if (v0 + vt * 16 < a.vp) Elem<uint16_t>::put4(out + vt * 16 + 4 * g, o[vt]);
+                        if (v0 + c0 + vt * 16 < a.vp) Elem<uint16_t>::put4(out + vt * 16 + 4 * g, o[vt]);
                 }
             }
         }
@@ -230,8 +252,8 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
             }
 #pragma unroll
             for (int vt = 0; vt < NVT; ++vt) {
-                const uint8_t* vh = lvh + row * kVRow + vt * 32 + tr_col;
-                const uint8_t* vl = lvl + row * kVRow + vt * 32 + tr_col;
+                const uint8_t* vh = lvh + row * kVRow + (c0 + vt * 16) * 2 + tr_col;
+                const uint8_t* vl = lvl + row * kVRow + (c0 + vt * 16) * 2 + tr_col;
                 const u32x4 fh = join(lds_read_tr(vh), lds_read_tr(vh + 16 * kVRow));
                 const u32x4 fl = join(lds_read_tr(vl), lds_read_tr(vl + 16 * kVRow));
 #pragma unroll
@@ -250,7 +272,7 @@ __global__ __launch_bounds__(256, DP <= 128 ? 2 : 1) void lightning_chunk_kernel
             for (int vt = 0; vt < NVT; ++vt)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int dd = 16 * (wave + 4 * i) + 4 * g + e, v = v0 + 16 * vt + c16;
+                    const int dd = 16 * (wave + 4 * i) + 4 * g + e, v = v0 + c0 + 16 * vt + c16;
                     if (dd < a.dp && v < a.vp) segp[(int64_t)dd * a.vp + v] = st[i][vt][e];
                 }
     }
@@ -339,21 +361,23 @@ __global__ __launch_bounds__(256) void lightning_step_kernel(LightningArgs a) {
         if (i < nd) *reinterpret_cast<f32x4*>(state + (int64_t)(r + 32 * i) * a.vp) = s[i];
 }
 
-template <int DP, int VS>
+template <int DP, int VS, int W>
 void chunk_t(const LightningArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)a.nseg, (unsigned)((a.vp + VS - 1) / VS), (unsigned)(a.batch * a.heads));
     if (a.nseg > 1) {
-        lightning_chunk_kernel<DP, VS, false><<<grid, 256, 0, stream>>>(a);
+        lightning_chunk_kernel<DP, VS, W, false><<<grid, W * 64, 0, stream>>>(a);
         const int64_t sz = (int64_t)a.dp * a.vp;
         lightning_scan_kernel<<<dim3((unsigned)((sz + 255) / 256), (unsigned)(a.batch * a.heads)), 256, 0, stream>>>(a);
     }
-    lightning_chunk_kernel<DP, VS, true><<<grid, 256, 0, stream>>>(a);
+    lightning_chunk_kernel<DP, VS, W, true><<<grid, W * 64, 0, stream>>>(a);
 }
 
 template <int DP>
 void chunk_d(const LightningArgs& a, hipStream_t stream) {
-    if (a.vp <= 32) chunk_t<DP, 32>(a, stream);
-    else chunk_t<DP, 64>(a, stream);
+    if (a.vp <= 32) return chunk_t<DP, 32, 4>(a, stream);
+    if constexpr (DP == 64 || DP == 128)
+        if (a.vp > 64 && (int64_t)a.batch * a.heads * a.nseg * ((a.vp + 127) / 128) >= 256) return chunk_t<DP, 128, 8>(a, stream);
+    chunk_t<DP, 64, 4>(a, stream);
 }
 
 template <typename T>

@@ -355,6 +355,21 @@ def test_lightning_segments(nseg):
     assert relative_rms(s[:, :, :dim, :vd], state) < 2e-5
 
 
+@pytest.mark.parametrize("dim,vd", [(40, 72), (64, 128), (100, 100), (128, 200)])
+@pytest.mark.parametrize("heads,batch,nseg", [(128, 2, 1), (43, 2, 3)])
+def test_lightning_with_a_workgroup_for_every_compute_unit(heads, batch, nseg, dim, vd):
+    """Slices of 128 value columns, eight waves: at the ends of chunks and of the columns."""
+    decay = [(0.6, 1.0, 0.999, 0.0)[h % 4] for h in range(heads)]
+    for cuts in ([1, 63, 64], [65, 129]) if nseg == 1 else ([129, 193], [200]):   # (a chunk for every segment)
+        q, k, v, dp, vp, proj = lightning_case(heads, dim, vd, sum(cuts), torch.bfloat16, batch, seed=dim)
+        want, state = lightning_want(q, k, v, decay)
+        log("lightning slices of 128", heads, dim, vd, cuts)
+        got, s = lightning_run(proj, cuts, batch, heads, dp, vp, decay, [False] * len(cuts), nseg)
+        assert got[..., vd:].count_nonzero() == 0
+        assert relative_rms(got[..., :vd].flatten(2), want.flatten(2)) < TOL[torch.bfloat16]
+        assert relative_rms(s[:, :, :dim, :vd], state) < 2e-5
+
+
 def test_lightning_remembers_one_far_token():
     """One token writes a large value under its own key; with everything else small, a query for that key thousands
     of tokens later reads decay^distance of it."""
