@@ -56,6 +56,10 @@ __device__ __forceinline__ void split4(f32x4 v, u32x2& hi, u32x2& mid, u32x2& lo
     lo = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
 }
 
+// An operand of 32 tokens, its second tile only where that one is behind the product's own: a NaN there times the zeros of a
+// triangle would reach tokens ahead of it.
+__device__ __forceinline__ u32x4 own_half(u32x4 v, bool both) { return u32x4{v.x, v.y, both ? v.z : 0, both ? v.w : 0}; }
+
 constexpr int kPrepThreads = 512;
 
 // A wave holds eight tokens, a lane two channels (of each 128) of them. LDS: the matrices of one level of pairs, then M, P
@@ -424,7 +428,7 @@ __global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_p
             }
             const float f = beta[16 * w4 + c16];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ts[(16 * i + 4 * g + e) * kLd + 16 * w4 + c16] = x[i][e] * f;
+            for (int e = 0; e < 4; ++e) ts[(16 * i + 4 * g + e) * kLd + 16 * w4 + c16] = i < w4 ? 0.0f : x[i][e] * f;
         }
     }
     __syncthreads();   // M and P are no longer read: their place takes values, then operands on their way out
@@ -448,9 +452,10 @@ __global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_p
                 for (int p = 0; p <= i / 2; ++p) {
                     u32x4 th, tm, tl;
                     fragment(ts, i, p, th, tm, tl);
-                    acc = mfma16(th, vf[p], acc);
-                    acc2 = mfma16(tm, vf[p], acc2);
-                    acc2 = mfma16(tl, vf[p], acc2);
+                    const u32x4 v = own_half(vf[p], 2 * p < i);
+                    acc = mfma16(th, v, acc);
+                    acc2 = mfma16(tm, v, acc2);
+                    acc2 = mfma16(tl, v, acc2);
                 }
                 __builtin_amdgcn_sched_barrier(0);   // (one tile's terms at a time in registers)
                 leave_fragment(Op::kV + (from / 16 + wave) * 4 + i, __builtin_bit_cast(u32x4, acc + acc2));
@@ -482,8 +487,11 @@ __global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_p
 #pragma unroll
                     for (int pp = 0; pp < 2; ++pp) {
                         if (pp > (wave & 1)) break;
-                        const u32x4 gh = *reinterpret_cast<const u32x4*>(src + pp * 3072), gm = *reinterpret_cast<const u32x4*>(src + pp * 3072 + 1024),
-                                    gl = *reinterpret_cast<const u32x4*>(src + pp * 3072 + 2048);
+                        u32x4 gh = *reinterpret_cast<const u32x4*>(src + pp * 3072), gm = *reinterpret_cast<const u32x4*>(src + pp * 3072 + 1024),
+                              gl = *reinterpret_cast<const u32x4*>(src + pp * 3072 + 2048);
+                        gh = own_half(gh, 2 * pp < ii);
+                        gm = own_half(gm, 2 * pp < ii);
+                        gl = own_half(gl, 2 * pp < ii);
                         acc = mfma16(gh, th[x][pp], acc);
                         acc2 = mfma16(gh, tm[x][pp], acc2);
                         acc2 = mfma16(gm, th[x][pp], acc2);
@@ -582,8 +590,9 @@ __global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, i
             u32x4 uh[2], ul[2];
 #pragma unroll
             for (int pp = 0; pp < 2; ++pp) {
-                uh[pp] = u_hi[pp][lane];
-                ul[pp] = u_lo[pp][lane];
+                uh[pp] = own_half(u_hi[pp][lane], 2 * pp < wave);
+                ul[pp] = own_half(u_lo[pp][lane], 2 * pp < wave);
+                if (pp > wave / 2) uh[pp] = ul[pp] = u32x4{0, 0, 0, 0};
             }
 #pragma unroll
             for (int pp = 0; pp < 2; ++pp) {

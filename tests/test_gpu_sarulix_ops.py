@@ -540,6 +540,29 @@ def test_delta_rule_in_blocks(shape, monkeypatch):
     c.check(c.run([66, 14], "chunk"), TOL[BF16])
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")], ids=str)
+@pytest.mark.parametrize("what", ["q", "k", "v", "z", "b"])
+def test_delta_rule_in_blocks_keeps_what_is_not_finite_from_earlier_tokens(what, bad, monkeypatch):
+    """A token's NaN or infinity reaches the same outputs and states as in chunks of 16: none before its 16."""
+    s, n = DeltaShape(3, 3, 64, 64, 64, 0.125), 150
+    for token in (0, 16, 31, 40, 63, 64, 149):
+        g, seen = gen(token), []
+        proj, z = randn(g, n, s.qkv_cols + 8, dtype=BF16), randn(g, n, 3 * 64)
+        if what == "z":
+            z[token, 3] = bad
+        else:
+            proj[token, {"q": 3, "k": 3 * 64 + 3, "v": 6 * 64 + 3, "b": s.qkv_cols}[what]] = bad
+        qkv, proj, z = proj[:, :s.qkv_cols].contiguous().to(DEV), proj.to(DEV), z.to(DEV)
+        for blocks in (False, True):
+            log("delta not finite", what, bad, token, blocks)
+            state = torch.ones(1, 3, 64, 64, device=DEV)
+            monkeypatch.setattr(_mix, "delta_in_blocks", lambda *a: blocks)
+            out = _mix.delta_chunk(qkv, proj, s, s.qkv_cols, z, torch.zeros(3 * 64, device=DEV), torch.ones(3, device=DEV), state)
+            seen.append((out.isfinite(), state.isfinite()))
+        assert all(torch.equal(a, b) for a, b in zip(*seen))
+        assert seen[1][0][:token // 16 * 16].all()
+
+
 def test_delta_rule_in_blocks_where_they_are_taken():
     shape = (2, 1, 64, 64)
     for batch, n in ((1, 640), (2, 1030)):
