@@ -3,8 +3,8 @@
 // column block has nothing else to do. Here a block is one step of the chain. With G_t, L_tj, M and P as there over 64 tokens,
 //   T = (I + M)^-1 diag(beta),   W = T (G K),   V' = T V          (prep, every block of every head at once)
 //   U = V' - W S,   O = (G Q) S + P U,   S <- diag(G_63) S + (L_63 K)^T U       (walk)
-// so that nothing but W S, the difference and L K^T U lies between two states. 16 heads of 128 x 128, 4096 tokens: 212 us there,
-// 159 here (prep 76, walk 83). Pairs (t, j) meet at the middle of their common
+// so that nothing but W S, the difference and L K^T U lies between two states. 16 heads of 128 x 128, 4096 tokens: 211 us there,
+// 162 here (prep 80, walk 82). Pairs (t, j) meet at the middle of their common
 // block of 2, 4 .. 64 tokens, where both factors of L_tj are at most 1. 32-bit factors enter the matrix cores as bf16 terms: two
 // and, where 64 tokens' writes nearly cancel, three (T, G K in T's product, U in the state's) and the product of both low terms;
 // the inverse is formed on fp32 matrix instructions. Against 64 bits the state is 2 to 45% closer than in chunks of 16 over head

@@ -890,7 +890,7 @@ def delta_chunk_supported(s: DeltaShape) -> bool:
 def delta_in_blocks(batch: int, seq: int, s: DeltaShape) -> bool:
     """Whether :func:`delta_chunk` walks blocks of 64 tokens rather than 16: where the walk from block to block is what
     takes the time, that is few heads, at most one column block to a compute unit, and a prompt long enough for it to be more
-    than the longer preparation. Measured in us, 16 and 64 tokens, heads x size, batch x length: 16 x 128 1 x 4096 212 and 159,
+    than the longer preparation. Measured in us, 16 and 64 tokens, heads x size, batch x length: 16 x 128 1 x 4096 211 and 162,
     1 x 1024 64 and 55, 1 x 640 49 and 45, 1 x 512 41 and 41, 1 x 300 29 and 34, 2 x 2048 143 and 135, 2 x 768 62 and 61,
     3 x 1024 109 and 110, 4 x 1024 127 and 136, 8 x 1024 220 and 279; 4 x 128 1 x 4096 176 and 108; 32 x 64 1 x 4096 195 and
     178, 2 x 2048 140 and 157; 32 x 32 1 x 2048 94 and 79; 8 x 256 1 x 2048 170 and 113, 2 x 1024 112 and 90, 8 x 1024 325 and
