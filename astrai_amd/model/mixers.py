@@ -193,12 +193,13 @@ class HeadLinear(Linear):
 
 
 def observed(module: nn.Module) -> bool:
-    """A call of ``module`` runs more than its class's ``forward``: hooks, its own or those of every module, or a
-    ``forward`` set on the instance."""
-    every = nn.modules.module
+    """A call of ``module``, of a class in ``FORWARDS``, runs something else than that class's ``forward``: hooks, its own or
+    those of every module, a compiled call, or a ``forward`` or ``__call__`` put in the place of the one defined here."""
+    every, cls = nn.modules.module, type(module)
     return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
                 or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
-                or every._global_backward_pre_hooks or "forward" in vars(module))
+                or every._global_backward_pre_hooks or module._compiled_call_impl is not None or "forward" in vars(module)
+                or cls.forward is not FORWARDS[cls] or cls.__call__ is not MODULE_CALL)
 
 
 def heads_of(name: str, heads: int, *dims: int) -> Rows:
@@ -683,6 +684,8 @@ class GatedMLP(nn.Module):
 
 
 MIXERS = (LatentAttention, LightningAttention, GroupedAttention, GatedRecurrence, ChannelDelta)
+FORWARDS = {cls: cls.forward for cls in (*MIXERS, GatedMLP, PackedLinear)}   # as defined here
+MODULE_CALL = nn.Module.__call__
 
 
 def mixed(mix: nn.Module, h: Tensor, ctx: StepContext) -> Tensor:

@@ -74,6 +74,48 @@ def test_the_gate_product_is_a_module_call_where_something_watches():
     assert _ways(mlp) == [None, "act_mul", None]
 
 
+def _plane_calls():
+    """(what of a layer is called by the layer's forward, the call, the name under which a compiled call would run)."""
+    from types import SimpleNamespace
+    mlp, x = mixers.GatedMLP(16, 24), torch.randn(4, 16)
+    mix = mixers.LightningAttention(16, 1, 8, 8, [0.5], 1e-5, 0)
+    ctx = SimpleNamespace(parts=False)
+    yield mlp, lambda: mixers.fed(mlp, x)
+    yield mlp.down, lambda: mixers.rows_out(mlp.down, torch.randn(4, 24), True)
+    yield mix, lambda: mixers.mixed(mix, x, ctx)
+    yield mix.o, lambda: mixers.rows_out(mix.o, torch.randn(4, mix.o.weight.size(1)), True)
+    yield mlp.gate_up, lambda: mlp(x)
+
+
+def test_a_call_that_is_not_the_class_s_own_forward_is_made(monkeypatch):
+    """Compiled modules, other forwards and other calls: none is gone around for planes or a fused product."""
+    monkeypatch.setattr(mixers, "parts_of", lambda *a: 4)
+    monkeypatch.setattr(_mix, "act_mul", lambda gu, act: gu[:, :gu.size(1) // 2])
+    for name in ("few_rows_parts", "few_rows_linear"):
+        monkeypatch.setattr(_mix, name, lambda *a, **k: pytest.fail("gone around"))
+    monkeypatch.setattr(mixers, "linear", torch.nn.functional.linear)
+    with torch.no_grad():
+        for module, call in _plane_calls():
+            seen = []
+
+            def instead(*args):
+                """``args``: of the call, or the module in front of them."""
+                args = args[1:] if args[0] is module else args
+                seen.append(len(args) == 1 or not args[1].parts)
+                return torch.ones(4, 48)
+
+            module.compile(backend="eager")
+            module._compiled_call_impl = instead
+            call()
+            module._compiled_call_impl = None
+            for cls, name in ((type(module), "forward"), (torch.nn.Module, "__call__")):
+                with pytest.MonkeyPatch.context() as m:
+                    stock = getattr(cls, name)
+                    m.setattr(cls, name, lambda self, *args: (instead if self is module else stock)(self, *args))
+                    call()
+            assert seen == [True] * 3
+
+
 def test_the_head_is_a_module_call():
     from types import SimpleNamespace
     model = mixers.MixerLM(SimpleNamespace(vocab=8, width=16), [])
