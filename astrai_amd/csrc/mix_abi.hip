@@ -645,6 +645,11 @@ int astrai_mix_conv(const void* proj, int64_t ld, int64_t off, int64_t cols, con
     return check_launch("conv");
 }
 
+int astrai_mix_rglru_held(int64_t batch, int64_t blocks, int64_t bp, int64_t nseg) {
+    return batch > 0 && blocks > 0 && nseg > 0 && bp > 0 && batch <= kMaxInt && blocks <= kMaxInt && nseg <= kMaxInt && bp <= kMaxInt &&
+           batch * blocks <= kMaxInt && rglru_held(batch * blocks * nseg, (int)bp);
+}
+
 int astrai_mix_rglru_chunk(const void* u, const void* proj, int64_t ld, int64_t y_off, const void* w_r, const void* w_i,
                            const float* b_r, const float* b_i, const float* coef, float* state, float* scratch,
                            void* out, int64_t batch, int64_t seq, int64_t blocks, int64_t bp, int64_t nseg,

@@ -264,6 +264,7 @@ struct RglruArgs {
     ConvArgs conv;               // fused step
 };
 bool rglru_chunk_supported(int bp);
+bool rglru_held(int64_t items, int bp);   // items: segments x blocks x sequences
 void launch_rglru_chunk(const RglruArgs& a, hipStream_t stream);
 bool rglru_step_supported(int bp, int seq);
 void launch_rglru_step(const RglruArgs& a, hipStream_t stream);

@@ -562,10 +562,14 @@ void general_t(const RglruArgs& a, hipStream_t stream) {
 bool rglru_chunk_supported(int bp) { return bp <= 1024; }
 
 // Whole groups of four waves of 16 channels whose weights fit the registers of two waves a SIMD are held
-// (1 x 4096 tokens: blocks of 64 44 -> 33 us, of 128 50 -> 37, of 256 63 -> 46); other blocks stream them.
+// (1 x 4096 tokens: blocks of 64 44 -> 33 us, of 128 50 -> 37, of 256 63 -> 46); other blocks stream them. The held
+// kernel's grid is one dimension, of fewer than 2^32 threads.
+bool rglru_held(int64_t items, int bp) {
+    return bp > 0 && bp % 64 == 0 && bp <= 256 && items <= ((int64_t)1 << 32) / (4 * bp) - 8;   // (rounded up to eights)
+}
+
 void launch_rglru_chunk(const RglruArgs& a, hipStream_t stream) {
-    const bool counted = (int64_t)a.nseg * a.blocks * a.batch < 1 << 28;   // (the held kernel's grid is one number)
-    switch (counted ? a.bp : 0) {
+    switch (rglru_held((int64_t)a.nseg * a.blocks * a.batch, a.bp) ? a.bp : 0) {
         case 64: return held_t<2>(a, stream);
         case 128: return held_t<4>(a, stream);
         case 192: return held_t<6>(a, stream);

@@ -70,6 +70,7 @@ PROTOTYPES = {
     "astrai_mix_rglru_step": ([_P] + [_I64] * 3 + [_P, _P, _I64] + [_P] * 9 + [_I64] * 4 + [_P], _INT),
     "astrai_mix_delta_step": (
         [_P, _P] + [_I64] * 3 + [_P, _I64] + [_P] * 6 + [_I64] + [_P] * 3 + [_I64] * 7 + [_F32, _F32, _INT, _P], _INT),
+    "astrai_mix_rglru_held": ([_I64] * 4, _INT),
     "astrai_mix_delta_image_bytes": ([_I64], _I64),
     "astrai_mix_delta_chunk": ([_P, _P, _I64, _I64] + [_P] * 6 + [_I64] * 6 + [_F32, _P], _INT),
     "astrai_mix_delta_blocks_bytes": ([_I64] * 5, _I64),

@@ -201,8 +201,11 @@ int astrai_mix_conv(const void* proj, int64_t ld, int64_t off, int64_t cols, con
  * y columns of proj from y_off, b_r, b_i, coef (<= 0), state [batch, channels] float.
  * _chunk (bf16, bp <= 1024): w [blocks, out, in]; nseg segments of the sequence side by side, scratch
  * [batch, nseg, 2, channels] float when nseg > 1; a segment is a whole number of tiles of 64 tokens.
+ * _held: whether _chunk keeps the weights in registers (bp 64, 128, 192 or 256 and fewer than 2^32 threads in all; a choice of
+ * nseg goes by it), else it streams them.
  * _general (bf16 or float): w [blocks, in, out], scratch [2, batch * seq, channels].
  * _step (bf16, seq <= RING_STEPS): convolves proj's columns from x_off itself and updates the ring (as above). */
+int astrai_mix_rglru_held(int64_t batch, int64_t blocks, int64_t bp, int64_t nseg);
 int astrai_mix_rglru_chunk(const void* u, const void* proj, int64_t ld, int64_t y_off, const void* w_r, const void* w_i,
                            const float* b_r, const float* b_i, const float* coef, float* state, float* scratch,
                            void* out, int64_t batch, int64_t seq, int64_t blocks, int64_t bp, int64_t nseg,

@@ -248,6 +248,12 @@ def test_launch_plans():
     assert _mix.gqa_rows_nsplit(s, 32, 1, 1024) == 4 and _mix.gqa_rows_nsplit(s, 1, 1, 200) == 1
     assert _mix.gqa_rows_nsplit(s, 1, 1, 1 << 20) == _mix.MAX_SPLIT
     assert _mix.rglru_nseg(32, 8, 256, 512) == 1 and _mix.rglru_nseg(1, 1, 64, 100) == 1
+    held = _mix._require().astrai_mix_rglru_held
+    for bp in (64, 128, 192, 256):   # a dimension of a launch holds fewer than 2^32 threads: bp / 64 groups of 256 to an item
+        most = (2 ** 32 - 1) // (bp // 64 * 256) // 8 * 8
+        assert held(1, 1, bp, 1) and held(1, 1, bp, most - 8) and not any(held(1, 1, bp, most + n) for n in range(1, 64))
+        assert not held(65535, 65, bp, 128) and not held(2 ** 31 - 1, 2 ** 31 - 1, bp, 2 ** 31 - 1)
+        assert not held(1, 1, bp + 32, 1) and not held(0, 1, bp, 1)
     assert _mix.rglru_nseg(1, 8, 256, 4096) > 1 and _mix.ring_rows(4) == 3 + _mix.RING_STEPS
 
 
