@@ -333,4 +333,4 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host() { return with_built_for(PyModule_Create(&module), ASTRAI_W8A8_ABI_VERSION); }

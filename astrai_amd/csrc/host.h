@@ -64,6 +64,17 @@ int unlocked(F call) {
     return call();
 }
 
+// What this was built for, which the loader compares: the calls' arguments, the library's header, torch, Python.
+#define ASTRAI_HOST_CALLS_VERSION 1
+PyObject* with_built_for(PyObject* module, int abi_version) {
+    PyObject* const what = module ? Py_BuildValue("(iiss)", ASTRAI_HOST_CALLS_VERSION, abi_version, ASTRAI_TORCH_VERSION,
+                                                  ASTRAI_PYTHON_VERSION) : nullptr;
+    if (what && PyModule_AddObject(module, "BUILT_FOR", what) == 0) return module;
+    Py_XDECREF(what);
+    Py_XDECREF(module);
+    return nullptr;
+}
+
 #define ENTRY(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&name)), METH_FASTCALL, nullptr}
 
 }  // namespace

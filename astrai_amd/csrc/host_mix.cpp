@@ -163,4 +163,4 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_mix", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_mix() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host_mix() { return with_built_for(PyModule_Create(&module), ASTRAI_MIX_ABI_VERSION); }

@@ -12,12 +12,13 @@ anywhere in this module: without the HIP library every call raises.
 from __future__ import annotations
 
 import ctypes
-import importlib
 import weakref
 import os
 from typing import Optional
 
 import torch  # imported before the CDLL so the library binds to torch's HIP runtime
+
+from astrai_amd.extension._native import NoCalls, load_calls
 
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libastrai_w8a8.so")
@@ -105,7 +106,7 @@ PROTOTYPES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
-_host = None   # the native form of the everyday calls (csrc/host.cpp), there whenever _lib is
+_host = NoCalls()   # the native form of the everyday calls (csrc/host.cpp)
 _load_error: Optional[str] = None
 
 
@@ -128,10 +129,10 @@ def load() -> Optional[ctypes.CDLL]:
         got = lib.astrai_w8a8_abi_version()
         if got != ABI_VERSION:
             raise OSError(f"ABI version {got}, expected {ABI_VERSION}")
-        _host = importlib.import_module("astrai_amd.extension._host")
-    except (OSError, AttributeError, ImportError) as e:
+    except (OSError, AttributeError) as e:
         _load_error = f"{type(e).__name__}: {e}"
         return None
+    _host = load_calls("_host", ABI_VERSION)
     _lib = lib
     return _lib
 
@@ -398,10 +399,9 @@ def _plain_bf16(t: torch.Tensor, dev: torch.device) -> bool:
 def linear_fp8_operands(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, inner: int = 1) -> bool:
     """Whether :func:`linear_fp8` takes these: bf16 on one GPU as the kernels read them, ``K % 16 == 0``, nothing empty,
     rows of ``x`` as wide as ``w.size(inner)`` (0: ``x`` is the output's gradient)."""
-    if _host is not None:
-        answer = _host.linear_fp8_operands(x, w, bias, inner)
-        if answer is not None:
-            return answer
+    answer = _host.linear_fp8_operands(x, w, bias, inner)
+    if answer is not None:
+        return answer
     k, dev = x.size(-1), x.device
     return (x.is_cuda and w.dim() == 2 and k == w.size(inner) and k % 16 == 0 and x.numel() > 0 and w.numel() > 0
             and _plain_bf16(x, dev) and _plain_bf16(w, dev)
@@ -1965,7 +1965,7 @@ def attn_prefill_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Op
     mask the block kernel reads the tensors in place (:func:`attn_prefill_strided`); the other cases run the
     ragged paged kernel over the token-major tensors (layout 0 is copied for it), an offset other than
     ``kv_len - q_len`` expressed through the mask."""
-    if mask is None and layout == BLHD and q.dim() == k.dim() == 4 and _host is not None and k.size(2) and attn_prefill_strided_takes(
+    if mask is None and layout == BLHD and q.dim() == k.dim() == 4 and k.size(2) and attn_prefill_strided_takes(
             q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q.size(3)):
         out = _host.attn_prefill(q, k, v, causal_offset, scale if scale and scale > 0.0 else q.size(3) ** -0.5)
         if out is not None:

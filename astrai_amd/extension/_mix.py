@@ -8,7 +8,6 @@ and without the HIP library every call raises (no CPU or PyTorch fallback).
 from __future__ import annotations
 
 import ctypes
-import importlib
 import os
 from dataclasses import dataclass
 from typing import Optional
@@ -16,6 +15,7 @@ from typing import Optional
 import torch  # imported before the CDLL so the library binds to torch's HIP runtime
 
 from astrai_amd.extension._cabi import _LIB_DIR, _on_device, _stream
+from astrai_amd.extension._native import NoCalls, load_calls
 
 LIB_PATH = os.path.join(_LIB_DIR, "libastrai_mix.so")
 
@@ -78,7 +78,7 @@ PROTOTYPES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
-_host = None   # the native form of the commonest calls (csrc/host_mix.cpp), there whenever _lib is
+_host = NoCalls()   # the native form of the commonest calls (csrc/host_mix.cpp)
 _load_error: Optional[str] = None
 
 
@@ -99,10 +99,10 @@ def load() -> Optional[ctypes.CDLL]:
         got = lib.astrai_mix_abi_version()
         if got != ABI_VERSION:
             raise OSError(f"ABI version {got}, expected {ABI_VERSION}")
-        _host = importlib.import_module("astrai_amd.extension._host_mix")
-    except (OSError, AttributeError, ImportError) as e:
+    except (OSError, AttributeError) as e:
         _load_error = f"{type(e).__name__}: {e}"
         return None
+    _host = load_calls("_host_mix", ABI_VERSION)
     _lib = lib
     return _lib
 
@@ -167,17 +167,23 @@ def residual_norm(y: torch.Tensor, x: torch.Tensor, w_post: torch.Tensor, w_pre:
     h = _host.residual_norm(y, x, w_post, w_pre, mult, eps)
     if h is not None:
         return h
-    if y.dim() == 3:
-        raise RuntimeError("residual_norm: planes, residual and weights do not fit")
-    n, width = y.shape
-    code = _dtype(y, "residual_norm")
+    planes = y.dim() == 3
+    if planes and (y.dtype != torch.float32 or not y.size(0)):
+        raise RuntimeError("residual_norm: float32 planes required")
+    n, width = y.shape[-2:]
+    code = 0 if planes else _dtype(y, "residual_norm")
     _dense("residual_norm", y.dtype, y)
     _dense("residual_norm", torch.float32, x, w_post, w_pre)
     _shape("residual_norm", x, n, width)
     _shape("residual_norm", w_post, width)
     _shape("residual_norm", w_pre, width)
     with _on_device(y.device):
-        h = torch.empty_like(y)
+        h = torch.empty((n, width), device=y.device, dtype=torch.bfloat16) if planes else torch.empty_like(y)
+        if planes:
+            _check(lib.astrai_mix_residual_norm_parts(y.data_ptr(), n * width, y.size(0), x.data_ptr(), x.data_ptr(),
+                                                      w_post.data_ptr(), w_pre.data_ptr(), h.data_ptr(), n, width, mult, eps,
+                                                      _stream(y)), lib)
+            return h
         _check(lib.astrai_mix_residual_norm(y.data_ptr(), x.data_ptr(), x.data_ptr(), w_post.data_ptr(),
                                             w_pre.data_ptr(), h.data_ptr(), n, width, mult, eps, code, _stream(y)), lib)
     return h
@@ -216,12 +222,13 @@ def sum_norm(y: torch.Tensor, w: Optional[torch.Tensor], dtype: torch.dtype, eps
         both = _host.sum_norm(y, w, dtype == torch.bfloat16, eps, x, u, vec, tokens, mult, out)
         if both is not None:
             return both
-    if y.dim() == 3:
-        raise RuntimeError("sum_norm: planes and terms do not fit")
-    width = y.size(1)
-    n = y.size(0) if tokens is None else tokens.numel()
+    planes = y.dim() == 3
+    if planes and (y.dtype != torch.float32 or not y.size(0) or tokens is not None):
+        raise RuntimeError("sum_norm: float32 planes without tokens required")
+    width = y.size(-1)
+    n = y.size(-2) if tokens is None else tokens.numel()
     code = _DTYPES[dtype]
-    for t in (y, u):
+    for t in (y[0] if planes else y, u):
         if t is None:
             continue
         if not t.is_cuda or t.dim() != 2 or t.stride(1) != 1 or t.stride(0) < width or t.size(1) != width:
@@ -246,6 +253,11 @@ def sum_norm(y: torch.Tensor, w: Optional[torch.Tensor], dtype: torch.dtype, eps
         if out is None:
             out = torch.empty((n, width), device=y.device, dtype=torch.float32)
         h = torch.empty((n, width), device=y.device, dtype=dtype)
+        if planes:
+            _check(lib.astrai_mix_sum_norm_parts(y.data_ptr(), y.stride(1), y.stride(0), y.size(0), mult, ptr(x), ptr(u),
+                                                 0 if u is None else u.stride(0), ptr(vec), out.data_ptr(), ptr(w),
+                                                 h.data_ptr(), n, width, eps, code, _stream(y)), lib)
+            return out, h
         _check(lib.astrai_mix_sum_norm(y.data_ptr(), y.stride(0), ptr(tokens), y.size(0), mult, ptr(x), ptr(u),
                                        0 if u is None else u.stride(0), ptr(vec), out.data_ptr(), ptr(w), h.data_ptr(),
                                        n, width, eps, int(y.dtype == torch.float32), code, _stream(y)), lib)
@@ -278,7 +290,7 @@ def few_rows_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optio
                               act: Optional[str] = None) -> bool:
     """The calls :func:`few_rows_linear` takes: bf16 on one GPU, up to 64 rows of ``x [.., k]`` at 16-byte
     boundaries, ``k`` a multiple of 128, the outputs of 4, weights under 2 GiB."""
-    if _host is not None and _host.few_rows_linear_takes(x, weight, bias, -1 if act is None else 0, FEW_ROWS):
+    if _host.few_rows_linear_takes(x, weight, bias, -1 if act is None else 0, FEW_ROWS):
         return True
     n, k = weight.size(0) // (1 if act is None else 2), weight.size(1)
     rows = x.numel() // k if k else 0
@@ -321,10 +333,18 @@ MAX_PARTS = 4
 def few_rows_parts(x: torch.Tensor, weight: torch.Tensor, parts: int) -> torch.Tensor:
     """:func:`few_rows_linear` without a bias as ``[parts, rows, outputs]`` fp32 sums over ranges of K, whose sum the row norms
     take for the product."""
-    _require()
+    lib = _require()
     out = _host.few_rows_parts(x, weight, FEW_ROWS, parts)
-    if out is None:
+    if out is not None:
+        return out
+    if not few_rows_linear_supported(x, weight) or parts < 1:
         raise RuntimeError("few_rows_parts: operands are not covered")
+    n, k = weight.shape
+    m = x.numel() // k
+    with _on_device(x.device):
+        out = torch.empty((parts, m, n), device=x.device, dtype=torch.float32)
+        _check(lib.astrai_mix_few_rows_parts(x.data_ptr(), k if x.is_contiguous() else x.stride(0), weight.data_ptr(),
+                                             out.data_ptr(), m, n, k, parts, _stream(x)), lib)
     return out
 
 

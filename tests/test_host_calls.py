@@ -1,5 +1,9 @@
 """The native form of the adapters' everyday calls: what it does not take is left to the adapters (which say what is wrong),
 and what it takes gives the bits that their own path gives."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -32,6 +36,34 @@ def test_what_is_left_to_the_adapters():
     assert mix.few_rows_linear(x, x, None, -1, 64, False) is None and mix.few_rows_linear_takes(sub, x, None, -1, 64) is None
     assert mix.sum_norm(x, None, True, 1e-5, None, None, None, None, 1.0, None) is None
     assert mix.residual_norm(x, x, s, s, 1.0, 1e-5) is None
+
+
+def test_a_native_module_that_was_built_for_others_is_not_used(monkeypatch):
+    from astrai_amd.extension import _native
+    for adapter, name in ((_cabi, "_host"), (_mix, "_host_mix")):
+        assert adapter.load() is not None
+        module = adapter._host
+        assert module.BUILT_FOR[:3] == (_native.CALLS_VERSION, adapter.ABI_VERSION, torch.__version__)
+        older = [module.BUILT_FOR[:i] + ("older",) + module.BUILT_FOR[i + 1:] for i in range(4)]
+        for built_for in (None, *older):
+            with monkeypatch.context() as m:
+                if built_for is None:   # not there at all
+                    m.setitem(sys.modules, "astrai_amd.extension." + name, None)
+                else:
+                    m.setattr(module, "BUILT_FOR", built_for)
+                m.setattr(adapter, "_lib", None)
+                m.setattr(adapter, "_host", module)
+                with pytest.warns(UserWarning, match=name + " is not used"):
+                    assert adapter.load() is not None and adapter.load_error() is None   # the library is there all the same
+                assert adapter._host.few_rows_parts(1) is None and adapter._host is not module
+
+
+def test_the_libraries_need_no_torch():
+    """A machine without it builds the C ABI and leaves the native calls out."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "astrai_amd", "csrc")
+    for target in ("all", "lib", "mix"):
+        plan = subprocess.run(["make", "-n", "-B", "-C", csrc, "PYTHON=false", target], capture_output=True, text=True)
+        assert plan.returncode == 0 and "libastrai_mix.so" in plan.stdout and "_host" not in plan.stdout, plan.stderr
 
 
 def _rand(*shape, dtype=BF16, std=1.0):
@@ -93,6 +125,12 @@ def _calls():
     yield lambda: _mix.sum_norm(wide[:, :512], vec, BF16, 1e-5, res, wide[:, 512:], vec, mult=0.5), True
     yield lambda: _mix.sum_norm(w, vec, BF16, 1e-5, tokens=torch.arange(20, device="cuda"), out=res.clone()), True
     yield lambda: _mix.residual_norm(_rand(20, 512), res.clone(), vec, vec, 0.5, 1e-5), True
+    planes = _rand(3, 20, 512, dtype=torch.float32)
+    yield lambda: _mix.few_rows_parts(wide[:, 256:768], w, 4), True
+    yield lambda: _mix.few_rows_parts(_rand(2, 3, 512), w, 1), True
+    yield lambda: _mix.sum_norm(planes, vec, BF16, 1e-5, res, res, vec, mult=0.5), True
+    yield lambda: _mix.sum_norm(planes.repeat(1, 1, 2)[:, :, 512:], None, BF16, 1e-5), True
+    yield lambda: _mix.residual_norm(planes, res.clone(), vec, vec, 0.5, 1e-5), True
 
 
 @pytest.mark.gpu
