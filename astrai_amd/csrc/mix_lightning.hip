@@ -35,8 +35,10 @@ namespace {
 
 constexpr int kC = kLightningChunk;
 
+// (two waves a SIMD but for the outputs of 256 key channels, which hold 368 registers: those channels' contributions are 21 registers
+// past the half by themselves, 1 x 4096 tokens 135 us in place of 128)
 template <int DP, int VS, int W, bool OUT>
-__global__ __launch_bounds__(W * 64, DP <= 128 ? 2 : 1) void lightning_chunk_kernel(LightningArgs a) {
+__global__ __launch_bounds__(W * 64, DP <= 128 || !OUT ? 2 : 1) void lightning_chunk_kernel(LightningArgs a) {
     constexpr int NT = W * 64, VW = VS * 4 / W;       // value columns of a wave
     constexpr bool kShareQ = OUT && W == 8;
     constexpr int kPad = W == 8 ? 32 : 16;            // (32: no bank conflicts in the transposing reads; 16 where two workgroups have to fit)
