@@ -23,8 +23,8 @@ struct ResidualNormArgs {
     int parts = 1;          // y is the sum of so many planes, fp32
     int64_t plane = 0;
 };
-// y_float: y is float with bf16 h
-void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool y_float, hipStream_t stream);
+// planes: y is planes of float with bf16 h
+void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool planes, hipStream_t stream);
 
 struct SumNormArgs {
     const void* y;          // [rows, ldy], or the embedding table [vocab, ldy] with `tokens`

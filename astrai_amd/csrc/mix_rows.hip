@@ -19,10 +19,10 @@ namespace astrai_mix {
 namespace {
 
 // four columns of y, or of the sum of its planes (requested together, added in order)
-template <typename TY, typename A>
+template <bool PLANES, typename TY, typename A>
 __device__ __forceinline__ f32x4 sum4(const TY* y, const A& a) {
     f32x4 v = Elem<TY>::get4(y);
-    if constexpr (sizeof(TY) == 4) {
+    if constexpr (PLANES) {
         if (a.parts == 4) {
             const f32x4 p = Elem<TY>::get4(y + a.plane), q = Elem<TY>::get4(y + 2 * a.plane), r = Elem<TY>::get4(y + 3 * a.plane);
             v = ((v + p) + q) + r;
@@ -33,10 +33,10 @@ __device__ __forceinline__ f32x4 sum4(const TY* y, const A& a) {
     return v;
 }
 
-template <typename TY, typename A>
+template <bool PLANES, typename TY, typename A>
 __device__ __forceinline__ float sum1(const TY* y, const A& a) {
     float v = Elem<TY>::get(y);
-    if constexpr (sizeof(TY) == 4)
+    if constexpr (PLANES)
         for (int i = 1; i < a.parts; ++i) v += Elem<TY>::get(y + i * a.plane);
     return v;
 }
@@ -44,7 +44,8 @@ __device__ __forceinline__ float sum1(const TY* y, const A& a) {
 // NV > 0: the row sits in NV registers of four per thread (width % 4 == 0, width <= 1024 NV).
 // NV == 0: any width, scalar accesses, x_out is the storage between the passes (a thread reads
 // back only what it wrote).
-template <typename T, typename TY, int NV, bool EMBED>
+// EARLY: the weights are loaded ahead of the reductions, whose barriers no load passes by itself, behind the row's own loads.
+template <typename T, typename TY, int NV, bool EMBED, bool PLANES, bool EARLY>
 __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNormArgs a) {
     __shared__ float slots[kRowThreads / kWave];
     const int64_t row = blockIdx.x;
@@ -63,20 +64,21 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     const float* xi = EMBED ? nullptr : a.x_in + row * w;
 
     if constexpr (NV > 0) {
-        f32x4 v[NV], g_post[NV], g_pre[NV];
+        f32x4 v[NV], g_post[EARLY ? NV : 1], g_pre[EARLY ? NV : 1];
         float s = 0.0f;
-        // (the weights with the row: loads do not move ahead of the reductions' barriers by themselves)
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
-            g_pre[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_pre + c) : f32x4{0, 0, 0, 0};
-            if constexpr (!EMBED) g_post[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_post + c) : f32x4{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = (i * kRowThreads + tid) * 4;
-            v[i] = c < w ? sum4(y + c, a) : f32x4{0, 0, 0, 0};
+            v[i] = c < w ? sum4<PLANES>(y + c, a) : f32x4{0, 0, 0, 0};
             s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        }
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int c = (i * kRowThreads + tid) * 4;
+                g_pre[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_pre + c) : f32x4{0, 0, 0, 0};
+                g_post[i] = c < w ? *reinterpret_cast<const f32x4*>(a.w_post + c) : f32x4{0, 0, 0, 0};
+            }
         }
         if constexpr (!EMBED) {
             f32x4 x[NV];
@@ -102,8 +104,11 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
             for (int i = 0; i < NV; ++i) {
                 const int c = (i * kRowThreads + tid) * 4;
                 if (c < w) {
+                    f32x4 g;
+                    if constexpr (EARLY) g = g_post[i];
+                    else g = *reinterpret_cast<const f32x4*>(a.w_post + c);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[i][e] = x[i][e] + v[i][e] * r * g_post[i][e];
+                    for (int e = 0; e < 4; ++e) v[i][e] = x[i][e] + v[i][e] * r * g[e];
                     s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
                 }
             }
@@ -129,26 +134,28 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
             if (c < w) {
-                f32x4 o;
+                f32x4 o, g;
+                if constexpr (EARLY) g = g_pre[i];
+                else g = *reinterpret_cast<const f32x4*>(a.w_pre + c);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g_pre[i][e];
+                for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[e];
                 Elem<T>::put4(h + c, o);
             }
         }
     } else {
         float mean = 0.0f, r = 0.0f, s = 0.0f, q = 0.0f;
         if constexpr (!EMBED) {
-            for (int c = tid; c < w; c += kRowThreads) s += sum1(y + c, a);
+            for (int c = tid; c < w; c += kRowThreads) s += sum1<PLANES>(y + c, a);
             mean = block_sum(s, slots) * inv_w;
             for (int c = tid; c < w; c += kRowThreads) {
-                const float d = sum1(y + c, a) - mean;
+                const float d = sum1<PLANES>(y + c, a) - mean;
                 q += d * d;
             }
             r = a.mult / sqrtf(block_sum(q, slots) * inv_w + a.eps);
         }
         s = q = 0.0f;
         for (int c = tid; c < w; c += kRowThreads) {
-            float v = sum1(y + c, a);
+            float v = sum1<PLANES>(y + c, a);
             if constexpr (!EMBED) v = xi[c] + (v - mean) * r * a.w_post[c];
             xo[c] = v;
             s += v;
@@ -163,20 +170,27 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(ResidualNorm
     }
 }
 
-template <typename T, typename TY, bool EMBED>
+// Early weights shorten the chain of four reductions (us, late and early: 32 rows of 2048 3.7 and 3.4, of 8192 6.7 and 5.6; 4096
+// rows of 8192 69 and 67, fp32 107 and 98), but rows past 4096 values then hold 150 registers, three workgroups a compute unit in
+// place of five: where the rows go round once with those and twice with these they are late (1000 rows of 5000 10.8, 12.8). An
+// embedding's norm has one chain of two, and late weights leave it more waves (4096 rows of 8192 56, 62).
+template <typename T, typename TY, bool EMBED, bool PLANES>
 void residual_norm_t(const ResidualNormArgs& a, hipStream_t stream) {
+    constexpr bool EARLY = !EMBED;
     const dim3 grid((unsigned)a.rows), block(kRowThreads);
     const int w = a.width;
-    if (w % 4 != 0 || a.plane % 4 != 0 || w > 8192) residual_norm_kernel<T, TY, 0, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 1024) residual_norm_kernel<T, TY, 1, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 2048) residual_norm_kernel<T, TY, 2, EMBED><<<grid, block, 0, stream>>>(a);
-    else if (w <= 4096) residual_norm_kernel<T, TY, 4, EMBED><<<grid, block, 0, stream>>>(a);
-    else residual_norm_kernel<T, TY, 8, EMBED><<<grid, block, 0, stream>>>(a);
+    if (w % 4 != 0 || a.plane % 4 != 0 || w > 8192) residual_norm_kernel<T, TY, 0, EMBED, PLANES, false><<<grid, block, 0, stream>>>(a);
+    else if (w <= 1024) residual_norm_kernel<T, TY, 1, EMBED, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else if (w <= 2048) residual_norm_kernel<T, TY, 2, EMBED, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else if (w <= 4096) residual_norm_kernel<T, TY, 4, EMBED, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else if (EMBED || (a.rows > 3 * 256 && a.rows <= 5 * 256))
+        residual_norm_kernel<T, TY, 8, EMBED, PLANES, false><<<grid, block, 0, stream>>>(a);
+    else residual_norm_kernel<T, TY, 8, EMBED, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
 }
 
 // x <- mult * (table[token] or y) + x_in + u + vec, each but the first optional; h = x / sqrt(mean(x^2) + eps) * w,
-// or x itself without w. TY: type of y and u. NV as above.
-template <typename T, typename TY, int NV>
+// or x itself without w. TY: type of y and u. NV and EARLY as above.
+template <typename T, typename TY, int NV, bool PLANES, bool EARLY>
 __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     __shared__ float slots[kRowThreads / kWave];
     const int64_t row = blockIdx.x;
@@ -192,20 +206,14 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     float* xo = a.x_out + row * w;
     T* h = static_cast<T*>(a.h) + row * w;
     if constexpr (NV > 0) {
-        f32x4 v[NV], g[NV];
+        f32x4 v[NV], g_early[EARLY ? NV : 1];
         float s = 0.0f;
-        // (the weights with the row: a load does not move ahead of the reduction's barrier by itself)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = (i * kRowThreads + tid) * 4;
-            g[i] = a.w && c < w ? *reinterpret_cast<const f32x4*>(a.w + c) : f32x4{0, 0, 0, 0};
-        }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = (i * kRowThreads + tid) * 4;
             v[i] = f32x4{0, 0, 0, 0};
             if (c < w) {
-                v[i] = sum4(y + c, a);
+                v[i] = sum4<PLANES>(y + c, a);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[i][e] *= a.mult;
                 if (xi) v[i] += *reinterpret_cast<const f32x4*>(xi + c);
@@ -215,6 +223,13 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
             }
             s += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
         }
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int c = (i * kRowThreads + tid) * 4;
+                g_early[i] = a.w && c < w ? *reinterpret_cast<const f32x4*>(a.w + c) : f32x4{0, 0, 0, 0};
+            }
+        }
         float r = 1.0f;
         if (a.w) r = 1.0f / sqrtf(block_sum(s, slots) / (float)w + a.eps);
 #pragma unroll
@@ -223,8 +238,11 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
             if (c < w) {
                 f32x4 o = v[i];
                 if (a.w) {
+                    f32x4 g;
+                    if constexpr (EARLY) g = g_early[i];
+                    else g = *reinterpret_cast<const f32x4*>(a.w + c);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[i][e];
+                    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * r * g[e];
                 }
                 Elem<T>::put4(h + c, o);
             }
@@ -232,7 +250,7 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     } else {
         float s = 0.0f, r = 1.0f;
         for (int c = tid; c < w; c += kRowThreads) {
-            float v = sum1(y + c, a) * a.mult;
+            float v = sum1<PLANES>(y + c, a) * a.mult;
             if (xi) v += xi[c];
             if (u) v += Elem<TY>::get(u + c);
             if (a.vec) v += a.vec[c];
@@ -244,15 +262,28 @@ __global__ __launch_bounds__(kRowThreads) void sum_norm_kernel(SumNormArgs a) {
     }
 }
 
-template <typename T, typename TY>
-void sum_norm_t(const SumNormArgs& a, hipStream_t stream) {
+template <typename T, typename TY, bool PLANES, bool EARLY>
+void sum_norm_e(const SumNormArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)a.rows), block(kRowThreads);
     const int w = a.width;
-    if (w % 4 != 0 || a.ldy % 4 != 0 || a.plane % 4 != 0 || a.ldu % 4 != 0 || w > 8192) sum_norm_kernel<T, TY, 0><<<grid, block, 0, stream>>>(a);
-    else if (w <= 1024) sum_norm_kernel<T, TY, 1><<<grid, block, 0, stream>>>(a);
-    else if (w <= 2048) sum_norm_kernel<T, TY, 2><<<grid, block, 0, stream>>>(a);
-    else if (w <= 4096) sum_norm_kernel<T, TY, 4><<<grid, block, 0, stream>>>(a);
-    else sum_norm_kernel<T, TY, 8><<<grid, block, 0, stream>>>(a);
+    if (w <= 1024) sum_norm_kernel<T, TY, 1, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else if (w <= 2048) sum_norm_kernel<T, TY, 2, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else if (w <= 4096) sum_norm_kernel<T, TY, 4, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+    else sum_norm_kernel<T, TY, 8, PLANES, EARLY><<<grid, block, 0, stream>>>(a);
+}
+
+// Early weights shorten a chain of launches (us, late and early: 32 rows of 2048 3.30 and 3.26, of 8192 7.0 and 6.9, fp32 7.1 and
+// 6.9); where rows go round the compute units several times, their registers cost waves in flight (4096 rows of 8192 96 and 98,
+// of 5000 50 and 54, fp32 of 4096 65 and 67).
+constexpr int64_t kEarlyRows = 1024;
+
+template <typename T, typename TY, bool PLANES>
+void sum_norm_t(const SumNormArgs& a, hipStream_t stream) {
+    const int w = a.width;
+    if (w % 4 != 0 || a.ldy % 4 != 0 || a.plane % 4 != 0 || a.ldu % 4 != 0 || w > 8192)
+        sum_norm_kernel<T, TY, 0, PLANES, false><<<dim3((unsigned)a.rows), dim3(kRowThreads), 0, stream>>>(a);
+    else if (a.rows <= kEarlyRows) sum_norm_e<T, TY, PLANES, true>(a, stream);
+    else sum_norm_e<T, TY, PLANES, false>(a, stream);
 }
 
 // gu [rows, 2 ff] (gate, then up), h [rows, ff]; ff % 8 == 0
@@ -340,21 +371,26 @@ __global__ __launch_bounds__(256) void head_gated_rms_norm_kernel(HeadNormArgs a
 
 }  // namespace
 
-void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool y_float, hipStream_t stream) {
+void launch_residual_norm(const ResidualNormArgs& a, int dtype, bool planes, hipStream_t stream) {
     if (dtype) {
-        if (a.tokens) residual_norm_t<float, float, true>(a, stream);
-        else residual_norm_t<float, float, false>(a, stream);
+        if (a.tokens) residual_norm_t<float, float, true, false>(a, stream);
+        else residual_norm_t<float, float, false, false>(a, stream);
     } else {
-        if (a.tokens) residual_norm_t<uint16_t, uint16_t, true>(a, stream);
-        else if (y_float) residual_norm_t<uint16_t, float, false>(a, stream);
-        else residual_norm_t<uint16_t, uint16_t, false>(a, stream);
+        if (a.tokens) residual_norm_t<uint16_t, uint16_t, true, false>(a, stream);
+        else if (planes) residual_norm_t<uint16_t, float, false, true>(a, stream);
+        else residual_norm_t<uint16_t, uint16_t, false, false>(a, stream);
     }
 }
 
 void launch_sum_norm(const SumNormArgs& a, int dtype, bool y_float, hipStream_t stream) {
-    if (dtype) sum_norm_t<float, float>(a, stream);
-    else if (y_float) sum_norm_t<uint16_t, float>(a, stream);
-    else sum_norm_t<uint16_t, uint16_t>(a, stream);
+    if (a.parts > 1) {
+        if (dtype) sum_norm_t<float, float, true>(a, stream);
+        else sum_norm_t<uint16_t, float, true>(a, stream);
+    } else {
+        if (dtype) sum_norm_t<float, float, false>(a, stream);
+        else if (y_float) sum_norm_t<uint16_t, float, false>(a, stream);
+        else sum_norm_t<uint16_t, uint16_t, false>(a, stream);
+    }
 }
 
 void launch_act_mul(const void* gu, void* h, int64_t rows, int ff, int act, int dtype, hipStream_t stream) {

@@ -65,6 +65,25 @@ def test_sum_norm(width, dtype):
     assert relative_rms(out, want) < 1e-6 and relative_rms(h, want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", [BF16, torch.float32], ids=str)
+@pytest.mark.parametrize("width", [100, 2048, 4096, 5000])
+def test_a_row_s_norm_does_not_depend_on_how_many_there_are(width, dtype):
+    """Weights loaded ahead of the reductions and behind them, at the lines between: the same bits."""
+    g, rows = gen(width), 1281
+    y, u = (randn(g, rows, width, dtype=dtype).to(DEV) for _ in range(2))
+    x, w, v = randn(g, rows, width).to(DEV), randn(g, width).to(DEV), randn(g, width).to(DEV)
+
+    def norms(n):
+        planes, a, b = torch.stack([y[:n].float(), u[:n].float()]), x[:n].clone(), x[:n].clone()
+        return (*_mix.sum_norm(y[:n], w, dtype, 1e-5, x=x[:n], u=u[:n], vec=v), _mix.residual_norm(y[:n], a, w, v, 0.5, 1e-5), a,
+                *_mix.sum_norm(planes, w, dtype, 1e-5, x=x[:n]), _mix.residual_norm(planes, b, w, v, 0.5, 1e-5), b)
+
+    few = norms(70)
+    for n in (768, 769, 1024, 1025, 1280, 1281):
+        log("rows", width, dtype, n)
+        assert all(torch.equal(a, b[:70]) for a, b in zip(few, norms(n), strict=True))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gelu_product(dtype):
     g = gen(5)
@@ -565,7 +584,7 @@ def test_delta_rule_in_blocks_keeps_what_is_not_finite_from_earlier_tokens(what,
 
 def test_delta_rule_in_blocks_where_they_are_taken():
     shape = (2, 1, 64, 64)
-    for batch, n in ((1, 640), (2, 1030)):
+    for batch, n in ((1, 768), (2, 1030)):
         assert _mix.delta_in_blocks(batch, n, DeltaShape(2, 1, 64, 64, 64, 0.125))
         c = Delta(shape, 3, BF16, n, batch=batch, seed=11)
         c.check(c.run([n], "chunk"), TOL[BF16])
