@@ -912,11 +912,14 @@ def delta_in_blocks(batch: int, seq: int, s: DeltaShape) -> bool:
     """Whether :func:`delta_chunk` walks blocks of 64 tokens rather than 16: where the walk from block to block is what
     takes the time, that is few heads, at most one column block to a compute unit, and a prompt long enough for it to be more
     than the longer preparation. Measured in us, 16 and 64 tokens, heads x size, batch x length: 16 x 128 1 x 4096 211 and 162,
-    1 x 1024 64 and 55, 1 x 640 49 and 45, 1 x 512 41 and 41, 1 x 300 29 and 34, 2 x 2048 143 and 135, 2 x 768 62 and 61,
+    1 x 1024 64 and 55, 1 x 640 49 and 45, 1 x 512 41 and 41, 1 x 300 29 and 34, 2 x 2048 143 and 135,
     3 x 1024 109 and 110, 4 x 1024 127 and 136, 8 x 1024 220 and 279; 4 x 128 1 x 4096 176 and 108; 32 x 64 1 x 4096 195 and
     178, 2 x 2048 140 and 157; 32 x 32 1 x 2048 94 and 79; 8 x 256 1 x 2048 170 and 113, 2 x 1024 112 and 90, 8 x 1024 325 and
-    358."""
-    return batch * s.heads <= 32 and batch * s.heads * s.vp <= 4096 and seq >= 640
+    358. The line in the length: 640 tokens 1 x 128 37.7 and 38.7, 4 x 64 30.9 and 31.8, 700 1 x 64 31.4 and 32.1, from 768 on
+    blocks are ahead (2 x 768 of 8 x 256 86 and 74); with more than 16 heads on more than half of the units later: 32 x 128 700
+    tokens 55.8 and 59.3, 2 x 768 of 16 x 128 60.4 and 61.8, 900 ahead by 2%."""
+    heads, columns = batch * s.heads, batch * s.heads * s.vp
+    return heads <= 32 and columns <= 4096 and seq >= (896 if heads > 16 and columns > 2048 else 768)
 
 
 def _delta_checks(what: str, s: DeltaShape, proj, b_off, z, dt_bias, decay, state):

@@ -248,6 +248,12 @@ def test_launch_plans():
     assert _mix.gqa_rows_nsplit(s, 32, 1, 1024) == 4 and _mix.gqa_rows_nsplit(s, 1, 1, 200) == 1
     assert _mix.gqa_rows_nsplit(s, 1, 1, 1 << 20) == _mix.MAX_SPLIT
     assert _mix.rglru_nseg(32, 8, 256, 512) == 1 and _mix.rglru_nseg(1, 1, 64, 100) == 1
+    # blocks of 64 tokens where they are the faster ones: not for 640 and 700 tokens (1 x 128: 37.7 us in chunks, 38.7)
+    blocks = lambda heads, size, batch, seq: _mix.delta_in_blocks(batch, seq, _mix.DeltaShape(heads, heads, size, size, size, 0.1))
+    for heads, size, batch, seq in ((1, 128, 1, 640), (4, 64, 8, 640), (32, 128, 1, 700), (1, 64, 1, 700), (16, 128, 2, 768), (64, 32, 1, 4096)):
+        assert not blocks(heads, size, batch, seq)
+    for heads, size, batch, seq in ((1, 128, 1, 768), (16, 64, 2, 768), (8, 256, 2, 768), (32, 128, 1, 900), (16, 128, 1, 4096)):
+        assert blocks(heads, size, batch, seq)
     held = _mix._require().astrai_mix_rglru_held
     for bp in (64, 128, 192, 256):   # a dimension of a launch holds fewer than 2^32 threads: bp / 64 groups of 256 to an item
         most = (2 ** 32 - 1) // (bp // 64 * 256) // 8 * 8
