@@ -130,7 +130,12 @@ __device__ __forceinline__ void tile_step(const u32x4 (&kf)[D / 32], const u32x4
         sc[i] = ok ? sc[i] * scale : kNegBig;
         tm = fmaxf(tm, sc[i]);
     }
-    tm = column_max(tm);
+    if constexpr (D == 32) {   // (through LDS, whose pipe has room here: a step of 32 x 3000 keys 23.5 us, in registers 24.0)
+        tm = fmaxf(tm, __shfl_xor(tm, 16, kWave));
+        tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
+    } else {
+        tm = column_max(tm);
+    }
     const float m_new = fmaxf(m, tm);
     const float alpha = __expf(m - m_new);
     float p[4], ps = 0.0f;
@@ -163,8 +168,11 @@ __device__ __forceinline__ float query_sum(float l) {
 }
 
 // workspace per (row block, kv head, split): kNQ rows of [D values | max | sum]
+// Heads of 32 could have eight waves a SIMD: all 2048 workgroups of a causal prompt would then start together, long and short
+// ones where they fall; with seven the last 256 go where there is room (16 / 4 heads, 4 x 1000 tokens 64 us, with eight 69; 8 x
+// 700 keys, 200 tokens 37 and 40).
 template <int D, bool MASK>
-__global__ __launch_bounds__(256) void attn_rows_partial_kernel(AttnRowsArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 32 ? 7 : 8))) void attn_rows_partial_kernel(AttnRowsArgs a) {
     constexpr int STEPS = D / 32;           // score MFMAs per key tile
     constexpr int CHUNKS = D / 16;          // 16-dim output chunks
     constexpr int DV = D / 16;              // value dims a lane fetches per key
