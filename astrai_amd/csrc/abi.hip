@@ -848,8 +848,9 @@ int astrai_w8a8_linear_fp8_bf16(const void* x, void* x8, float* x_step, float* x
         if (w) w8a8::launch_amax_bf16(w, nullptr, w_maxima, n * k, s);
         if (w) w8a8::launch_quantize_fp8_measured(w, w8, {w_maxima, fmax, pow2_margin}, w_step, n * k, fmt, s);
     } else {
-        pushed = !w && w8a8::launch_quantize_fp8_pushed(x, x8, {x_hist, x_len, x_idx, x_step, fmax, pow2_margin}, x_maxima, m * k,
-                                                        fmt, s);
+        // (a step that is x's and the codes' at once is refreshed behind the product that reads it)
+        pushed = !w && w_step != x_step &&
+                 w8a8::launch_quantize_fp8_pushed(x, x8, {x_hist, x_len, x_idx, x_step, fmax, pow2_margin}, x_maxima, m * k, fmt, s);
         if (pushed) product_step = x_maxima;
         else w8a8::launch_quantize_fp8(x, x8, x_step, nullptr, x_maxima, m * k, fmt, s);
         if (w) w8a8::launch_quantize_fp8(w, w8, w_step, nullptr, w_maxima, n * k, fmt, s);

@@ -73,6 +73,19 @@ def test_few_values(monkeypatch, recipe, rows):
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("rows", [1, 100])   # pushed in the quantizer's launch, behind the product
+def test_a_step_that_two_operands_share(rows):
+    """One tensor as the step of x and of the weight's codes: the product reads it before it is refreshed."""
+    from astrai_amd.extension import _cabi
+    x, w, got = _mk(1, rows, 512, std=3.0), _mk(2, 64, 512), []
+    codes = (w.float() / 0.01).clamp(-448, 448).to(torch.float8_e4m3fn)
+    for shared in (False, True):
+        sx, hist = torch.full((1,), 0.01, device=DEV), torch.ones(4, device=DEV)
+        out = _cabi.linear_fp8(x, w, None, codes, (sx, sx if shared else sx.clone()), ((hist, 1), None), 0, 448.0, 1.0)
+        got.append((out, sx, hist))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and got[1][1] != 0.01
+
+
 @pytest.mark.parametrize("recipe", [lambda: fp8.DelayedScaling(history_len=3, margin=1), fp8.DynamicScaling])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 512), (48, 512, 256), (100, 272, 1024), (130, 1040, 272), (1037, 256, 512)])
 @pytest.mark.parametrize("bias,fmt", [(False, "hybrid"), (True, "hybrid"), (True, "e4m3")])
