@@ -1106,7 +1106,8 @@ def attn_paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     ``ml_part_buf`` is not needed. ``mask``: bool ``[batch, width]``, True = attend
     that position (entry_utils.cuh:226-237); positions past ``width`` are not attended."""
     lib = _require()
-    if mask is new_k is new_v is out_buf is o_part_buf is None and q.dim() == k_cache.dim() == 3 and req_to_token.dim() == 2:
+    if (mask is new_k is new_v is out_buf is o_part_buf is None and q.dim() == k_cache.dim() == 3 and req_to_token.dim() == 2
+            and q.is_contiguous()):
         (b, h, d), hkv = q.shape, k_cache.size(1)
         general = hkv == 0 or _decode_is_general(h, hkv, d)
         splits = nsplit if nsplit > 0 else (_rows_decode_nsplit if general else paged_nsplit)(b * hkv, req_to_token.size(1))
