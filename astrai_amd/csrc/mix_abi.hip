@@ -779,7 +779,7 @@ int astrai_mix_delta_chunk(const void* qkv, const void* proj, int64_t ld, int64_
 
 int64_t astrai_mix_delta_blocks_bytes(int64_t batch, int64_t heads, int64_t seq, int64_t dp, int64_t vp) {
     if (batch < 0 || heads <= 0 || seq < 0 || dp <= 0 || dp % 32 || vp <= 0 || vp % 32 || batch > kMaxInt || heads > kMaxInt || seq > kMaxInt ||
-        vp > kMaxInt || !delta_chunk_supported((int)dp, (int)vp))
+        vp > kMaxInt || batch * heads > kMaxInt || !delta_blocks_supported(batch, heads, seq, (int)dp, (int)vp))
         return -1;
     return delta_blocks_bytes(batch, heads, seq, (int)dp, (int)vp);
 }
@@ -792,8 +792,9 @@ int astrai_mix_delta_blocks(const void* qkv, const void* proj, int64_t ld, int64
                        (const void*)state, (const void*)image, (const void*)out));
     MIX_TRY(check_delta("delta_blocks", ld, b_off, batch, seq, heads, kv_heads, dp, vp));
     if (batch > kMaxGridYZ) return fail(ASTRAI_MIX_BAD_ARG, "delta_blocks: batch %lld", (long long)batch);
-    if (!delta_chunk_supported((int)dp, (int)vp))
-        return fail(ASTRAI_MIX_UNSUPPORTED, "delta_blocks: head size %lld (at most 256)", (long long)dp);
+    if (!delta_blocks_supported(batch, heads, seq, (int)dp, (int)vp))
+        return fail(ASTRAI_MIX_UNSUPPORTED, "delta_blocks: %lld x %lld heads of %lld, %lld (keys at most 256) or %lld tokens",
+                    (long long)batch, (long long)heads, (long long)dp, (long long)vp, (long long)seq);
     DeltaArgs a = {};
     a.qkv = qkv;
     a.ldq = 2 * kv_heads * dp + heads * vp;

@@ -10,6 +10,8 @@
 // the inverse is formed on fp32 matrix instructions. Against 64 bits the state is 2 to 45% closer than in chunks of 16 over head
 // sizes 32 to 256, random, slow and strong decays, and up to 35 times with one key over and over; two terms throughout were 5 to
 // 40% further off, 4 times with equal keys.
+#include <algorithm>
+
 #include "mix_common.cuh"
 #include "mix_launchers.h"
 
@@ -69,7 +71,7 @@ constexpr int kPrepThreads = 512;
 // scratch memory). A third of what is left is the wait for the first loads, which two workgroups a compute unit begin together:
 // 225 MB at 2.9 TB/s in all. The heads of a token run side by side (8 heads of 256, 2048 tokens: 106 us in place of 112).
 template <int DP>
-__global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_prep_kernel(DeltaArgs a, int blocks) {
+__global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_prep_kernel(DeltaArgs a, int blocks, int first) {
     using Op = Operands<DP>;
     constexpr int NS = Op::NS, NB = (DP + 127) / 128, CH = DP < 128 ? DP : 128;   // channels at a time
     constexpr int kRow = CH * 2 + 16, kMat = kBlock * kRow, kLd = kBlock + 4;      // bytes; floats
@@ -87,7 +89,7 @@ __global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_p
     const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int block = (int)blockIdx.x / a.heads, h = (int)blockIdx.x % a.heads, b = blockIdx.y, grp = h / (a.heads / a.kv_heads);
-    const int t0 = block * kBlock, n = min(kBlock, a.seq - t0);
+    const int t0 = (first + block) * kBlock, n = min(kBlock, a.seq - t0);
     const int64_t row0 = (int64_t)b * a.seq + t0;
     const uint16_t* q = static_cast<const uint16_t*>(a.qkv) + row0 * a.ldq + grp * a.dp;
     const uint16_t* k = q + a.kv_heads * a.dp;
@@ -518,7 +520,7 @@ __global__ __launch_bounds__(kPrepThreads, DP <= 128 ? 4 : 2) void delta_block_p
 // paths meet, every load would be waited for. The column blocks of a head run on one XCD and find its operands in that L2, into
 // which each touches its share of a block three ahead (84 us without).
 template <int DP>
-__global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, int blocks) {
+__global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, int blocks, int first) {
     using Op = Operands<DP>;
     constexpr int NS = Op::NS, NO = (NS + 3) / 4;    // steps of channels; of them a wave's own
     __shared__ u32x4 s_hi[NS][64], s_lo[NS][64], u_hi[2][64], u_lo[2][64], u_end[2][64];
@@ -548,7 +550,7 @@ __global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, i
             for (int hl = 0; hl < 2; ++hl) p[pp][hl] = w8a8::buf_load16(r, pp <= wave / 2 ? lane * 16 : kOutOfRange, (at + 2 * pp + hl) * 1024);
         };
         const int ldo = a.heads * a.vp;
-        uint16_t* out = static_cast<uint16_t*>(a.out) + (int64_t)b * a.seq * ldo;
+        uint16_t* out = static_cast<uint16_t*>(a.out) + ((int64_t)b * a.seq + (int64_t)first * kBlock) * ldo;
         const uint32_t out_lane = (uint32_t)((16 * wave + 4 * g) * ldo + h * a.vp + v) * 2;
 #pragma unroll
         for (int s = 0; s < NS; ++s) load_q(s);
@@ -602,7 +604,7 @@ __global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, i
                 load_p(pp);
             }
             const f32x4 o = o0 + (o1 + o2);
-            const __amdgpu_buffer_rsrc_t ro = w8a8::make_rsrc(out, (uint32_t)(min(kBlock, a.seq - c * kBlock) * ldo) * 2);   // (ends at the last token)
+            const __amdgpu_buffer_rsrc_t ro = w8a8::make_rsrc(out, (uint32_t)(min(kBlock, a.seq - (first + c) * kBlock) * ldo) * 2);   // (ends at the last token)
 #pragma unroll
             for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b16(w8a8::f32_to_bf16(o[e]), ro, out_lane + (uint32_t)(e * ldo) * 2, 0, 0);
             out += kBlock * ldo;
@@ -734,6 +736,20 @@ __global__ __launch_bounds__(512, 1) void delta_block_walk_kernel(DeltaArgs a, i
             }
 }
 
+int64_t pieces_of(int dp, int vp) {
+    return dp <= 32 ? Operands<32>::pieces(vp) : dp <= 64 ? Operands<64>::pieces(vp) : dp <= 128 ? Operands<128>::pieces(vp) : Operands<256>::pieces(vp);
+}
+
+// Blocks that are prepared and walked at a time. Operands take 141 KiB a block and head of 128 where chunks of 16 take 108 for as
+// many tokens; prompts whose operands are more than this go in equal parts, from whose states each next one starts, so that they
+// need less than they would in chunks (16 heads of 128, 1 x 32768 tokens: 376 MiB, 864 in chunks), others 120 MiB more at most.
+constexpr int64_t kImageMost = (int64_t)512 << 20;
+int64_t blocks_at_a_time(int64_t heads, int64_t seq, int dp, int vp) {
+    const int64_t blocks = (seq + kBlock - 1) / kBlock, bytes = heads * blocks * pieces_of(dp, vp) * 1024;
+    const int64_t parts = std::min((bytes + kImageMost - 1) / kImageMost, blocks);
+    return parts > 1 ? (blocks + parts - 1) / parts : blocks;
+}
+
 template <int DP>
 void blocks_t(const DeltaArgs& a, hipStream_t stream) {
     constexpr int CH = DP < 128 ? DP : 128, mat = 4 * kBlock * (CH * 2 + 16), fp32 = 3 * kBlock * (kBlock + 4) * 4 + 4 * 1088;
@@ -741,16 +757,26 @@ void blocks_t(const DeltaArgs& a, hipStream_t stream) {
     static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_block_prep_kernel<DP>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, shared);
     (void)once;
-    const int blocks = (a.seq + kBlock - 1) / kBlock, groups = (a.batch * a.heads + 7) / 8;
-    delta_block_prep_kernel<DP><<<dim3((unsigned)blocks * (unsigned)a.heads, (unsigned)a.batch), kPrepThreads, shared, stream>>>(a, blocks);
-    delta_block_walk_kernel<DP><<<(unsigned)(groups * 8 * (a.vp / 16)), 512, 0, stream>>>(a, blocks);
+    const int all = (a.seq + kBlock - 1) / kBlock, groups = (a.batch * a.heads + 7) / 8;
+    const int most = (int)blocks_at_a_time((int64_t)a.batch * a.heads, a.seq, a.dp, a.vp);
+    for (int first = 0; first < all; first += most) {
+        const int blocks = std::min(most, all - first);
+        delta_block_prep_kernel<DP><<<dim3((unsigned)blocks * (unsigned)a.heads, (unsigned)a.batch), kPrepThreads, shared, stream>>>(a, blocks, first);
+        delta_block_walk_kernel<DP><<<(unsigned)(groups * 8 * (a.vp / 16)), 512, 0, stream>>>(a, blocks, first);
+    }
 }
 
 }  // namespace
 
 int64_t delta_blocks_bytes(int64_t batch, int64_t heads, int64_t seq, int dp, int vp) {
-    const int p = dp <= 32 ? Operands<32>::pieces(vp) : dp <= 64 ? Operands<64>::pieces(vp) : dp <= 128 ? Operands<128>::pieces(vp) : Operands<256>::pieces(vp);
-    return batch * heads * ((seq + kBlock - 1) / kBlock) * p * 1024;
+    return batch * heads * blocks_at_a_time(batch * heads, seq, dp, vp) * pieces_of(dp, vp) * 1024;
+}
+
+// (a dimension of a launch holds fewer than 2^32 threads, a descriptor 2^32 bytes: 64 rows of out, a block's operands)
+bool delta_blocks_supported(int64_t batch, int64_t heads, int64_t seq, int dp, int vp) {
+    constexpr int64_t most = ((int64_t)1 << 32) - 1;
+    return delta_chunk_supported(dp, vp) && heads * vp * kBlock * 2 <= most && pieces_of(dp, vp) * 1024 <= most &&
+           (batch * heads + 7) / 8 * 8 * (vp / 16) * 512 <= most && blocks_at_a_time(batch * heads, seq, dp, vp) * heads * kPrepThreads <= most;
 }
 
 void launch_delta_blocks(const DeltaArgs& a, hipStream_t stream) {

@@ -302,6 +302,7 @@ int64_t delta_image_bytes(int dp);
 // chunked form on the matrix cores, bf16; out is neither normed nor gated
 void launch_delta_chunk(const DeltaArgs& a, hipStream_t stream);
 // the same in blocks of 64 tokens; image: delta_blocks_bytes
+bool delta_blocks_supported(int64_t batch, int64_t heads, int64_t seq, int dp, int vp);
 int64_t delta_blocks_bytes(int64_t batch, int64_t heads, int64_t seq, int dp, int vp);
 void launch_delta_blocks(const DeltaArgs& a, hipStream_t stream);
 

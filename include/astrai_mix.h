@@ -228,7 +228,9 @@ int astrai_mix_rglru_step(const void* proj, int64_t ld, int64_t y_off, int64_t x
  * of stride ldg). qkv null (seq <= RING_STEPS): convolves proj's columns from x_off itself and updates the ring.
  * UNSUPPORTED unless vp <= 256 and dp * (vp / 4 rounded up to a power of two, at least 8) <= 16384.
  * _chunk (bf16, dp <= 256): out = o; image: delta_image_bytes * batch * heads * ceil(seq / DELTA_CHUNK) bytes.
- * _blocks: the same in blocks of 64 tokens; image: delta_blocks_bytes (-1: sizes not covered). */
+ * _blocks: the same in blocks of 64 tokens; image: delta_blocks_bytes (-1: sizes not covered), which depends on vp too and is at
+ * most 512 MiB or one block of every head: longer prompts go in equal parts. It is the faster one for few heads and long prompts:
+ * batch * heads <= 32, batch * heads * vp <= 4096 and seq >= 768 (896 with more than 16 heads and batch * heads * vp > 2048). */
 int astrai_mix_delta_step(const void* qkv, const void* proj, int64_t ld, int64_t x_off, int64_t b_off,
                           const float* conv_w, int64_t taps, void* ring, const int64_t* positions, const float* z,
                           const float* dt_bias, const float* decay, const void* gate, int64_t ldg, const float* norm_w,

@@ -582,6 +582,26 @@ def test_delta_rule_in_blocks_keeps_what_is_not_finite_from_earlier_tokens(what,
         assert seen[1][0][:token // 16 * 16].all()
 
 
+@pytest.mark.parametrize("batch,seq,cut", [(1, 16400, 129 * 64), (2, 8300, 65 * 64)])
+def test_delta_rule_in_blocks_of_a_prompt_in_parts(batch, seq, cut):
+    """Operands of more than 512 MiB are formed and walked in two parts: the bits of a call for each, at a block's edge."""
+    s = DeltaShape(16, 16, 128, 128, 128, 0.09)
+    size = _mix._require().astrai_mix_delta_blocks_bytes
+    assert size(batch, 16, seq, 128, 128) == size(batch, 16, cut, 128, 128) < size(batch, 16, cut + 64, 128, 128)
+    torch.manual_seed(seq)
+    mk = lambda cols, dtype=BF16: torch.randn(batch, seq, cols, device=DEV).to(dtype)
+    qkv, proj, z, dt, decay = mk(s.qkv_cols), mk(s.qkv_cols + 16), mk(16 * 128, torch.float32), torch.zeros(16 * 128, device=DEV), torch.ones(16, device=DEV)
+    got = []
+    for cuts in ([(0, seq)], [(0, cut), (cut, seq)]):
+        state, outs = torch.ones(batch, 16, 128, 128, device=DEV), []
+        for a, b in cuts:
+            log("delta parts", batch, a, b)
+            part = [t[:, a:b].reshape(batch * (b - a), -1).contiguous() for t in (qkv, proj, z)]
+            outs.append(_mix.delta_chunk(part[0], part[1], s, s.qkv_cols, part[2], dt, decay, state, blocks=True).view(batch, b - a, -1))
+        got.append((torch.cat(outs, 1), state))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and got[0][0].isfinite().all()
+
+
 def test_delta_rule_in_blocks_where_they_are_taken():
     shape = (2, 1, 64, 64)
     for batch, n in ((1, 768), (2, 1030)):

@@ -254,7 +254,16 @@ def test_launch_plans():
         assert not blocks(heads, size, batch, seq)
     for heads, size, batch, seq in ((1, 128, 1, 768), (16, 64, 2, 768), (8, 256, 2, 768), (32, 128, 1, 900), (16, 128, 1, 4096)):
         assert blocks(heads, size, batch, seq)
-    held = _mix._require().astrai_mix_rglru_held
+    # their workspace: 30% more than that of chunks up to 512 MiB, less than it past them
+    lib = _mix._require()
+    for heads, size in ((16, 128), (32, 32), (2, 256), (32, 64)):
+        image = lib.astrai_mix_delta_image_bytes(size) * heads
+        for seq in (100, 4096, 30000, 70001, 1 << 20):
+            need = lib.astrai_mix_delta_blocks_bytes(1, heads, seq, size, size)
+            assert 0 < need <= max(image * -(-seq // 16), 512 << 20) and need <= image * -(-seq // 64) * 4 * 4 / 3
+    for bad in ((1, 1 << 20, 64, 128, 128), (1, 1, 64, 128, 1 << 24), (1 << 20, 64, 64, 128, 128), (1, 1, 64, 288, 32), (1, 1, 64, 100, 32)):
+        assert lib.astrai_mix_delta_blocks_bytes(*bad) == -1   # past a launch's or a descriptor's reach, or not a multiple of 32
+    held = lib.astrai_mix_rglru_held
     for bp in (64, 128, 192, 256):   # a dimension of a launch holds fewer than 2^32 threads: bp / 64 groups of 256 to an item
         most = (2 ** 32 - 1) // (bp // 64 * 256) // 8 * 8
         assert held(1, 1, bp, 1) and held(1, 1, bp, most - 8) and not any(held(1, 1, bp, most + n) for n in range(1, 64))
