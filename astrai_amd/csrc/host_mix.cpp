@@ -32,7 +32,7 @@ struct FewRows {
         n = w->size(0) / (act < 0 ? 1 : 2), k = w->size(1), m = k ? x->numel() / k : 0;
         if (x->size(-1) != k || m <= 0 || m > most || k % 128 || n % 4 || w->numel() * 2 >= (int64_t)1 << 31 ||
             x->scalar_type() != at::kBFloat16 || !plain16(*w, at::kBFloat16, dev) || !near16(*x) ||
-            (bias && (act >= 0 || !plain(*bias, at::kBFloat16, dev) || !near16(*bias, 8))))
+            (bias && (act >= 0 || bias->numel() != n || !plain(*bias, at::kBFloat16, dev) || !near16(*bias, 8))))
             return false;
         ldx = k;
         if (x->is_contiguous()) return true;

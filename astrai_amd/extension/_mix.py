@@ -300,7 +300,7 @@ def few_rows_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optio
         return False
     if not weight.is_contiguous() or weight.data_ptr() % 16 or x.data_ptr() % 16:
         return False
-    if bias is not None and not (act is None and bias.dtype == torch.bfloat16 and bias.device == x.device
+    if bias is not None and not (act is None and bias.numel() == n and bias.dtype == torch.bfloat16 and bias.device == x.device
                                  and bias.is_contiguous() and bias.data_ptr() % 8 == 0):
         return False
     return x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and k <= x.stride(0) < 2 ** 23)
@@ -360,7 +360,7 @@ def prompt_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optiona
         return False
     if not weight.is_contiguous() or weight.data_ptr() % 16 or x.data_ptr() % 16:
         return False
-    if bias is not None and not (act is None and bias.dtype == torch.bfloat16 and bias.device == x.device
+    if bias is not None and not (act is None and bias.numel() == n and bias.dtype == torch.bfloat16 and bias.device == x.device
                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0):
         return False
     if not (x.is_contiguous() or (x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k)):

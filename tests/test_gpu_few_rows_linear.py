@@ -85,6 +85,24 @@ def test_calls_that_are_left_to_the_library():
         _mix.few_rows_linear(_mk(1, 65, 256), w)
 
 
+def test_a_bias_of_another_size_is_left_to_the_library():
+    """The kernels would read as many values as there are outputs."""
+    from astrai_amd.extension import _mix
+    from astrai_amd.model import mixers
+    w = _mk(2, 264, 256)
+    for x in (_mk(1, 8, 256), _mk(3, 4096, 256)):
+        for bias in (_mk(4, 1), _mk(5, 263), _mk(6, 1, 264)):
+            takes = bias.numel() == 264
+            assert _mix.few_rows_linear_supported(x[:8], w, bias) == takes and _mix.prompt_linear_supported(x, w, bias) == takes
+            if not takes:
+                with pytest.raises(RuntimeError, match="not covered"):
+                    _mix.few_rows_linear(x[:8], w, bias)
+        with torch.no_grad():
+            assert torch.equal(mixers.linear(x, w, _mk(4, 1)), F.linear(x, w, _mk(4, 1)))
+            with pytest.raises(RuntimeError):
+                mixers.linear(x, w, _mk(5, 263))
+
+
 @pytest.mark.parametrize("parts", [1, 2, 3, 4])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 512), (17, 200, 128), (8, 2048, 4224), (33, 3076, 1280), (64, 132, 2048)])
 def test_planes_of_ranges_add_up(parts, m, n, k):
