@@ -192,13 +192,16 @@ class HeadLinear(Linear):
         return linear(x, self.weight, self.bias)
 
 
+every = nn.modules.module   # (its hooks are every module's)
+
+
 def observed(module: nn.Module) -> bool:
     """A call of ``module``, of a class in ``FORWARDS``, runs something else than that class's ``forward``: hooks, its own or
     those of every module, a compiled call, or a ``forward`` or ``__call__`` put in the place of the one defined here."""
-    every, cls = nn.modules.module, type(module)
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+    own, cls = module.__dict__, type(module)   # (five times a layer: no attribute lookups through the module)
+    return bool(own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
                 or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
-                or every._global_backward_pre_hooks or module._compiled_call_impl is not None or "forward" in vars(module)
+                or every._global_backward_pre_hooks or own.get("_compiled_call_impl") or "forward" in own
                 or cls.forward is not FORWARDS[cls] or cls.__call__ is not MODULE_CALL)
 
 
