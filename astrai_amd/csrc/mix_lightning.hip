@@ -17,9 +17,12 @@
 // compute unit, eight waves take 128 columns and pass q to each other through LDS too, half of the
 // waves to either 64 columns. 16 heads of 128 x 128, slices of 64 and of 128, in us: 32 x 512 tokens
 // 147 and 139, 8 x 2048 204 and 176, 1 x 4096 68 and 63, 4 x 1024 69 and 61; 64 heads, 1 x 8192 375
-// and 331; 32 heads of 96 columns, 16 x 512 134 and 119. With fewer than 256 workgroups the smaller
-// ones are more and faster: 4 x 200 32 and 34, 1 x 300 36 and 39. Converting the next chunk while
-// half of the waves multiply, so that both units work: 140, nothing.
+// and 331; 32 heads of 96 columns, 16 x 512 134 and 119; 16 heads of 64 x 128: 32 x 512 81 and 75,
+// 8 x 2048 121 and 110, 1 x 4096 47 and 44. With fewer than 256 workgroups the smaller ones are more
+// and faster: 4 x 200 32 and 34, 1 x 300 36 and 39; and so they are where many workgroups of 64 key
+// channels have a chunk or two each, most of it their state's way in and out (16 heads of 64 x 128,
+// 128 x 64 67 and 72, 64 heads, 32 x 64 66 and 70; on less than 1024 32 x 64 22.1 and 20.5).
+// Converting the next chunk while half of the waves multiply, so that both units work: 140, nothing.
 //
 // With few heads, a long prompt is cut into segments that run side by side: one pass forms every
 // segment's own contribution to the state, a scan turns those into the state each segment starts
@@ -377,8 +380,11 @@ void chunk_t(const LightningArgs& a, hipStream_t stream) {
 template <int DP>
 void chunk_d(const LightningArgs& a, hipStream_t stream) {
     if (a.vp <= 32) return chunk_t<DP, 32, 4>(a, stream);
-    if constexpr (DP == 64 || DP == 128)
-        if (a.vp > 64 && (int64_t)a.batch * a.heads * a.nseg * ((a.vp + 127) / 128) >= 256) return chunk_t<DP, 128, 8>(a, stream);
+    if constexpr (DP == 64 || DP == 128) {
+        const int64_t groups = (int64_t)a.batch * a.heads * a.nseg * ((a.vp + 127) / 128), chunks = (a.seq + kC - 1) / kC;
+        const bool starts = DP == 64 && a.vp % 128 == 0 && groups >= 1024 && chunks <= 2 * a.nseg;
+        if (a.vp > 64 && groups >= 256 && !starts) return chunk_t<DP, 128, 8>(a, stream);
+    }
     chunk_t<DP, 64, 4>(a, stream);
 }
 

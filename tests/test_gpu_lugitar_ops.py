@@ -356,7 +356,7 @@ def test_lightning_segments(nseg):
 
 
 @pytest.mark.parametrize("dim,vd", [(40, 72), (64, 128), (100, 100), (128, 200)])
-@pytest.mark.parametrize("heads,batch,nseg", [(128, 2, 1), (43, 2, 3)])
+@pytest.mark.parametrize("heads,batch,nseg", [(128, 2, 1), (43, 2, 3), (300, 4, 1)])
 def test_lightning_with_a_workgroup_for_every_compute_unit(heads, batch, nseg, dim, vd):
     """Slices of 128 value columns, eight waves: at the ends of chunks and of the columns."""
     decay = [(0.6, 1.0, 0.999, 0.0)[h % 4] for h in range(heads)]
