@@ -67,7 +67,7 @@ constexpr int kPrepThreads = 512;
 // A wave holds eight tokens, a lane two channels (of each 128) of them. LDS: the matrices of one level of pairs, then M, P
 // and T in fp32 in their place, then values and operands on their way out. All loads come before the first store (those of
 // the values, behind the stores at first, took a quarter of the time: 91 us in place of 80), and the operands that need no T
-// leave before it, so that their factors' registers are free for its terms (159 us for the whole rule, 213 with 87 registers in
+// leave before it, so that their factors' registers are free for its terms (162 us for the whole rule, 213 with 87 registers in
 // scratch memory). A third of what is left is the wait for the first loads, which two workgroups a compute unit begin together:
 // 225 MB at 2.9 TB/s in all. The heads of a token run side by side (8 heads of 256, 2048 tokens: 106 us in place of 112).
 template <int DP>

@@ -14,8 +14,8 @@
 //
 // Several ranges of K by workgroups of their own (splits) make the row ranges longer and the part of x that a workgroup reads
 // shorter: x is most of the bytes that a workgroup pulls out of L2 where the weights have few rows. The fp32 sums of the
-// ranges lie in planes that the row norm behind the product adds up. With that norm (us, one range / four): 32 rows of 5632 ->
-// 2048 14.2 / 10.8, 2048 -> 2048 9.1 / 8.2; 16 rows 12.6 / 9.9, 8.2 / 7.5; 1 row 9.7 / 9.1, 7.2 / 7.2.
+// ranges lie in planes that the row norm behind the product adds up. With that norm (us, one range / four): 64 rows of 5632 ->
+// 2048 18.7 / 12.4, 2048 -> 2048 10.9 / 9.0; 32 rows 13.8 / 11.0, 8.7 / 7.9; 16 rows 11.7 / 9.9, 8.1 / 7.2; 1 row 9.9 / 9.6, 7.3 / 6.8.
 //
 // What bounds it (graph replays over weights that no cache holds): the stream from 20 MB on (2048 -> 32000, 131 MB, 22.5 us at 1
 // token, 5.8 TB/s), below it launch and the load path's 16 cycles for every 1 KiB instruction, of x as much as of the

@@ -1046,6 +1046,8 @@ void launch_quantize_fp8_measured(const void* x, void* x8, const MeasuredStep& m
 // 8.6, 64 (131072 values, the limit) 12.1 -> 11.4; 4096 x 4096, 8 tokens 12.4 -> 9.4, 32 12.9 -> 12.1; at 180000 values the
 // workgroups' reads cost more than the launch (13.6, 14.3). Delayed, weight codes kept: 1 token 7.6 -> 5.9, 8 x 4096
 // values 12.0 -> 11.5: one compute unit's fourteen instructions a value catch up with the launch. Eager calls 2.6 us each less.
+// A thread's loads and vectors are as many as the size needs; one instance of the most for all sizes: dynamic 1, 8, 16 tokens of 1024
+// values 5.2 -> 5.6, 5.9 -> 7.0, 6.4 -> 7.2, delayed 5.3 -> 6.0, 6.0 -> 6.5, 6.8 -> 7.2.
 bool launch_quantize_fp8_small(const void* x, void* x8, const MeasuredStep& measured, float* scale, int64_t total, int fmt,
                                hipStream_t stream) {
     if (total % 8 || total > kSmallMeasured) return false;

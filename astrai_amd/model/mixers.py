@@ -167,9 +167,11 @@ def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None) -> Tensor:
 def parts_of(rows: int, n: int, k: int) -> int:
     """Ranges of K in which a product of few rows is left for the row norm behind it to add up (:func:`_mix.few_rows_parts`): four
     where the weight has few rows of many values, so that x is most of what a workgroup reads, else one. With the norm (us, one /
-    four): 2048 x 5632 of 1, 8, 32 rows 9.7 / 9.1, 10.6 / 9.5, 14.2 / 10.8; 2048 x 2048 7.2 / 7.2, 7.6 / 7.4, 9.1 / 8.2; 1024 x
-    2816 7.0 / 6.1, 7.4 / 6.3, 9.0 / 7.1; 3072 x 8192 14.0 / 14.4, 14.2 / 14.3, 21.5 / 15.9; 4096 x 11008 of 8, 16 rows 22.7 / 22.4,
-    25.1 / 23.1. Others gain nothing or lose: 2048 x 1024 of 16 rows 6.7 / 6.8, 4096 x 4096 13.8 / 14.0, 6144 x 6144 21.4 / 21.5."""
+    four): 2048 x 5632 of 1, 8, 32, 64 rows 9.9 / 9.6, 10.3 / 9.5, 13.8 / 11.0, 18.7 / 12.4; 2048 x 2048 7.3 / 6.8, 7.4 / 7.2, 8.7 /
+    7.9, 10.9 / 9.0; 1024 x 2816 7.2 / 5.9, 7.4 / 6.4, 9.1 / 6.9, 11.2 / 8.2; 3072 x 8192 14.7 / 14.8, 15.7 / 15.1, 19.8 / 16.4, 25.4 /
+    18.8; 4096 x 11008 of 8, 16, 64 rows 23.5 / 23.5, 25.9 / 24.3, 35.9 / 30.5; of 30 sizes and 9 row counts to 64 that this takes,
+    one is 1% slower with four. Others gain nothing or lose: 2048 x 1024 of 16 rows 6.7 / 6.8, 4096 x 4096 13.6 / 14.0, 4096 x 2048 of
+    64 13.2 / 14.1, 6144 x 6144 of 16 21.4 / 21.5."""
     if k < 2048:
         return 1
     return _mix.MAX_PARTS if n <= 2048 or (n <= 3072 and rows >= 8) or (n <= 4096 and k >= 2 * n and rows >= 12) else 1
