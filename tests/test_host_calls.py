@@ -187,3 +187,40 @@ def test_errors_are_the_adapters():
         _cabi.attn_paged_decode(q, pool, pool, *ints)
     with pytest.raises(RuntimeError, match="not covered"):
         _mix.few_rows_linear(_rand(65, 256), w)
+
+
+@pytest.mark.gpu
+def test_both_forms_take_the_same_operands(monkeypatch):
+    """The conditions stand in the native module and in the adapters: the same answers over every form of every operand."""
+    def forms(rows, cols, dtype=BF16):
+        t = _rand(rows * 2 + 1, cols * 2 + 16).to(dtype)
+        yield t[:rows, :cols].contiguous()
+        yield t[:rows, :cols]                                      # rows of a wider matrix
+        yield t.flatten()[1:1 + rows * cols].view(rows, cols)      # at an odd address
+        yield t.flatten()[4:4 + rows * cols].view(rows, cols)      # at 8 bytes
+        yield t[:cols, :rows].t() if cols <= t.size(0) else t[:rows, 0:2 * cols:2]
+        yield t[:rows, :cols].float()
+        yield t[:rows, :cols].contiguous().cpu()
+        yield t[:rows, :cols - 16].contiguous()
+        yield t[:0, :cols]
+        yield t[:rows, :cols].reshape(rows, 1, cols)
+
+    def vectors(n):
+        return [None, *(f.reshape(f.size(0), -1)[:, 0] if i == 4 else f.flatten() for i, f in enumerate(forms(1, n)) if i != 1)]
+
+    asks = 0
+    for x in (*forms(8, 256), *forms(65, 256), _rand(256)):
+        for w in forms(64, 256):
+            if w.dim() != 2:
+                continue
+            for bias in vectors(64):
+                calls = [lambda: _cabi.linear_fp8_operands(x, w, bias), lambda: _cabi.linear_fp8_operands(x, w, bias, 0)]
+                calls += [lambda act=act: _mix.few_rows_linear_supported(x, w, bias, act) for act in (None, "silu")]
+                for call in calls:
+                    with monkeypatch.context() as m:
+                        m.setattr(_cabi, "_host", Refuses())
+                        m.setattr(_mix, "_host", Refuses())
+                        want = call()
+                    assert call() == want, (x.shape, x.stride(), x.dtype, w.shape, w.stride(), w.dtype, bias is None or bias.shape)
+                    asks += 1
+    assert asks > 5000
