@@ -3,6 +3,7 @@
 
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
@@ -12,8 +13,11 @@ namespace {
 
 using at::Tensor;
 
-// the argument's tensor, or null (None, another type, a subclass)
-const Tensor* tensor_of(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// The argument's tensor, or null (None, another type, a subclass). None is one under torch.jit.trace, which would record the
+// outputs' allocation and not what is written into them.
+const Tensor* tensor_of(PyObject* o) {
+    return THPVariable_CheckExact(o) && !torch::jit::tracer::isTracing() ? &THPVariable_Unpack(o) : nullptr;
+}
 
 // an optional tensor: false if the argument is something else
 bool optional(PyObject* o, const Tensor*& t) {

@@ -58,6 +58,16 @@ def test_a_native_module_that_was_built_for_others_is_not_used(monkeypatch):
                 assert adapter._host.few_rows_parts(1) is None and adapter._host is not module
 
 
+def test_nothing_is_taken_while_torch_traces():
+    assert _cabi.load() is not None
+    x, seen = torch.zeros(2, 128, dtype=BF16), []
+    ask = lambda: seen.append(_cabi._host.linear_fp8_operands(x, x, None, 1))
+    ask()
+    torch.jit.trace(lambda t: (ask(), t + 1)[1], (x,), check_trace=False)
+    ask()
+    assert seen == [False, None, False]
+
+
 def test_the_libraries_need_no_torch():
     """A machine without it builds the C ABI and leaves the native calls out."""
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "astrai_amd", "csrc")
