@@ -12,6 +12,8 @@
 // kernels (gemm_pingpong.cuh): 128 activation rows then 128 weight rows of 128 bytes, chunk
 // c of row r at position c ^ (r & 7) ^ ((r >> 3) & 1); weight rows are the first MFMA operand.
 #pragma once
+#include <type_traits>
+
 #include "gemm_pingpong.cuh"
 
 namespace w8a8 {
@@ -31,6 +33,9 @@ struct Mid128Cfg {
 // read into a second register set beside the MFMAs of slab k; 1050 cycles a slab, bound by LDS (96 KiB of fragments, 32 KiB of
 // loads). int8 / fp8, us: 256 x 11264 x 2048 14.7 / 14.2 -> 13.1 / 12.6, 640 x 4096 x 4096 22.8 / 22.5 -> 20.5 / 18.7, 130 x 11008
 // x 4096 22.4 / 23.7 -> 18.7 / 18.4, 600 x 4096 x 11008 49.2 / 49.4 -> 43.9 / 39.9; 2048^3 (256 tiles) 16.0 / 15.1 either way.
+// 128-block scales (steps four slabs at a time, scaled additions behind the other half's MFMAs): 1454 x 2048 x 7168 57.2 -> 35.6, 600 x
+// 4096 x 4096 34.5 -> 21.5, 450 x 7168 x 2048 17.6 -> 14.0, 2600 x 1536 x 7168 59.6 -> 39.2, 600 x 4096 x 640 8.5 -> 8.0; with a step a
+// slab and row in this ring 51.5 and 31.3 of the first two: 16 scattered loads a slab held up the load path that the slabs take.
 // Up to four slabs the ring is filled once, and its larger prologue is a loss (600 x 4096 x 256 6.9 / 6.4 -> 7.3 / 7.0, x 512
 // 7.9 / 7.5 -> 8.1 / 7.75; x 640 the first where it is none): two stages.
 template <class Op, int ScaleKind, bool RoundFirst, int S>
@@ -137,10 +142,10 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid12
 
     // ---- 128-block scales: a slab is exactly one K-block. The slab's product is formed in a
     // temporary and joins the accumulator scaled by the activation rows' and the weight block's
-    // steps (the tile's 128 columns lie in one weight block); the steps of slab k + 1 are requested
+    // steps (the tile's 128 columns lie in one weight block). With two stages the steps of slab k + 1 are requested
     // while slab k is computed.
-    [[maybe_unused]] float blk_sa[MI], blk_sa_next[MI];
-    [[maybe_unused]] float blk_sb = 0.0f, blk_sb_next = 0.0f;
+    [[maybe_unused]] float blk_step[MI], blk_sa_next[MI];
+    [[maybe_unused]] float blk_sb_next = 0.0f;
     [[maybe_unused]] const int kblocks = K >> 7;
     auto request_steps = [&](int kb) {
         if constexpr (ScaleKind == SCALE_BLOCK128) {
@@ -177,7 +182,7 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid12
                     for (int j = 0; j < 16; ++j) part[j] = 0;
 #pragma unroll
                     for (int q = 0; q < Op::STEPS; ++q) part = Op::mma_step(q, wf[ni], xf[mi], part);
-                    const float sc = blk_sa[mi] * blk_sb;
+                    const float sc = blk_step[mi];
 #pragma unroll
                     for (int j = 0; j < 16; ++j) acc[ni][mi][j] += part[j] * sc;
                 }
@@ -199,8 +204,7 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid12
         for (int k = 0; k < ksteps; ++k) {
             if constexpr (ScaleKind == SCALE_BLOCK128) {
     #pragma unroll
-                for (int mi = 0; mi < MI; ++mi) blk_sa[mi] = blk_sa_next[mi];
-                blk_sb = blk_sb_next;
+                for (int mi = 0; mi < MI; ++mi) blk_step[mi] = blk_sa_next[mi] * blk_sb_next;
             }
             if (k + 1 < ksteps) {
                 issue((k + 1) & 1, k + 1);
@@ -219,31 +223,107 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid12
             phase_barrier();
         }
     } else {
-        static_assert(ScaleKind != SCALE_BLOCK128, "the wait counts leave no room for the steps' loads");
         u32x4 xa[MI][4], wa[NI][4], xb[MI][4], wb[NI][4];
+        // 128-block scales: a row's steps of four slabs are one load (16 lines for each row and slab otherwise, and the load path
+        // that the slabs come through takes a line a cycle), requested in the first slab of the four before, ahead of its slab
+        // loads; past the last slab and past M they are never used. MI + 1 vector loads whatever the compiler makes of the
+        // addresses: the waits count them.
+        constexpr int STEPS = ScaleKind == SCALE_BLOCK128 ? MI + 1 : 0;
+        [[maybe_unused]] u32x4 steps[MI + 1], steps_next[MI + 1];
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsa = make_rsrc(g.sa, STEPS ? (uint32_t)g.m * (uint32_t)kblocks * 4u : 0u);
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsb = make_rsrc(g.sb, STEPS ? (uint32_t)tiles_n * (uint32_t)kblocks * 4u : 0u);
+        auto request = [&](int kb, u32x4 (&d)[MI + 1]) __attribute__((always_inline)) {
+            if constexpr (STEPS > 0) {
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+                    d[mi] = buf_load16(rsa, (uint32_t)(mw + mi * 32 + lrow) * (uint32_t)kblocks * 4u, (uint32_t)kb * 4u);
+                d[MI] = buf_load16(rsb, (uint32_t)(n0 >> 7) * (uint32_t)kblocks * 4u, (uint32_t)kb * 4u);
+            }
+        };
+        // Two waves of a SIMD meet at the barrier of every slab, so that a slab's scaled additions, left to its end, run with the matrix
+        // cores idle: each half goes behind the other half's MFMAs instead, the second half's into the next slab.
+        [[maybe_unused]] Acc part[MI];
+        [[maybe_unused]] float behind = 0.0f;
+        if constexpr (STEPS > 0) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) part[MI - 1][j] = 0;
+        }
+        auto multiply_scaled = [&](u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4]) __attribute__((always_inline)) {
+            static_assert(MI == 2 && NI == 1, "halves");
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) {
+                const float sc = mi == 0 ? behind : blk_step[0];
+#pragma unroll
+                for (int q = 0; q < Op::STEPS; ++q) {
+                    if (q == 0) part[mi] = Op::mma_step(q, wf[0], xf[mi], Acc{});
+                    else part[mi] = Op::mma_step(q, wf[0], xf[mi], part[mi]);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 16 / Op::STEPS * q; j < 16 / Op::STEPS * (q + 1); ++j) acc[0][1 - mi][j] += part[1 - mi][j] * sc;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            behind = blk_step[1];
+        };
+        request(0, steps);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < S; ++t) issue(t, t);
         wait_vmcnt<4 * (S - 1)>();
         phase_barrier();
         read(0, xa, wa);
-        // in: this slab's fragments, its reads under way
-        auto slab = [&](int k, u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4], u32x4 (&xn)[MI][4], u32x4 (&wn)[NI][4])
+        // in: this slab's fragments, its reads under way. AT: which of its four slabs; MORE: four more follow them, whose steps
+        // the first requests (both with 128-block scales)
+        auto slab = [&](auto at, auto more, int k, u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4], u32x4 (&xn)[MI][4], u32x4 (&wn)[NI][4])
                         __attribute__((always_inline)) {
+            constexpr int AT = decltype(at)::value;
+            constexpr bool MORE = decltype(more)::value;
             wait_lgkmcnt0();
-            wait_vmcnt<4 * (S - 2)>();   // slab k + 1 has landed
+            wait_vmcnt<4 * (S - 2) + (MORE && (AT == 1 || AT == 2) ? STEPS : 0)>();   // slab k + 1 has landed
             phase_barrier();             // for every wave, and every wave has read slab k: its stage is free
+            if constexpr (STEPS > 0) {
+                if constexpr (MORE && AT == 0) {
+                    request(k + 4, steps_next);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi) blk_step[mi] = __uint_as_float(steps[mi][AT]) * __uint_as_float(steps[MI][AT]);
+            }
             issue(k & (S - 1), k + S);
             read((k + 1) & (S - 1), xn, wn);   // (past the last slab: zeros)
             __builtin_amdgcn_sched_barrier(0);
-            multiply(xf, wf);
+            if constexpr (STEPS > 0) multiply_scaled(xf, wf);
+            else multiply(xf, wf);
         };
+        constexpr std::integral_constant<int, 0> at0{};
         int k = 0;
-        for (; k + 1 < ksteps; k += 2) {
-            slab(k, xa, wa, xb, wb);
-            slab(k + 1, xb, wb, xa, wa);
+        if constexpr (STEPS > 0) {
+            constexpr std::integral_constant<int, 1> at1{};
+            constexpr std::integral_constant<int, 2> at2{};
+            constexpr std::integral_constant<int, 3> at3{};
+            for (; k + 3 < ksteps; k += 4) {
+                slab(at0, std::true_type{}, k, xa, wa, xb, wb);
+                slab(at1, std::true_type{}, k + 1, xb, wb, xa, wa);
+                slab(at2, std::true_type{}, k + 2, xa, wa, xb, wb);
+                slab(at3, std::true_type{}, k + 3, xb, wb, xa, wa);
+#pragma unroll
+                for (int i = 0; i <= MI; ++i) steps[i] = steps_next[i];
+            }
+            if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wb);
+            if (k + 1 < ksteps) slab(at1, std::false_type{}, k + 1, xb, wb, xa, wa);
+            if (k + 2 < ksteps) slab(at2, std::false_type{}, k + 2, xa, wa, xb, wb);
+        } else {
+            for (; k + 1 < ksteps; k += 2) {
+                slab(at0, std::false_type{}, k, xa, wa, xb, wb);
+                slab(at0, std::false_type{}, k + 1, xb, wb, xa, wa);
+            }
+            if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wb);
         }
-        if (k < ksteps) slab(k, xa, wa, xb, wb);
         wait_vmcnt<0>();
+        if constexpr (STEPS > 0) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[0][1][j] += part[1][j] * behind;
+        }
     }
 
     // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad): 8-byte stores
@@ -308,7 +388,7 @@ inline void launch_mid128(const GemmArgs& g, hipStream_t stream) {
     if constexpr (!RoundFirst && ScaleKind == SCALE_TENSOR)
         if (g.round_first) return launch_mid128<Op, ScaleKind, true>(g, stream);
     const int tiles = ((g.m + Cfg::BM - 1) / Cfg::BM) * ((g.n + Cfg::BN - 1) / Cfg::BN);
-    if constexpr (S == 2 && ScaleKind != SCALE_BLOCK128)
+    if constexpr (S == 2)
         if (tiles <= 256 && g.k > 512) return launch_mid128<Op, ScaleKind, RoundFirst, 4>(g, stream);
     constexpr int lds_bytes = S * Cfg::STAGE_BYTES;
     auto kern = gemm_mid128_kernel<Op, ScaleKind, RoundFirst, S>;

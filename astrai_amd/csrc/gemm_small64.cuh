@@ -16,6 +16,8 @@
 // LDS layout of a slab, load plan per wave (rows 16 w .. 16 w + 15 of both operands), fragment
 // reads, accumulator layout and epilogue are those of gemm_mid128_kernel.
 #pragma once
+#include <type_traits>
+
 #include "gemm_pingpong.cuh"
 
 namespace w8a8 {
@@ -34,7 +36,7 @@ struct Small64Cfg {
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it (see gemm_mid128.cuh; 200 x 2048
 // x 2048 6.2 us, with the choice in the epilogue 6.3)
 template <class Op, int ScaleKind, int S, bool RoundFirst>
-__global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm_small64_kernel(GemmArgs g) {
     using Cfg = Small64Cfg<S>;
     using Acc = typename Op::Acc;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -130,23 +132,32 @@ __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
 
     // ---- 128-block scales: a slab is exactly one K-block and the tile's 64 columns lie in one
     // weight block. The slab's product is formed in a temporary and joins the accumulator scaled by
-    // the row's and the block's steps, requested one slab ahead -- two loads an iteration, issued
-    // BEFORE the iteration's four slab loads, so that "all but the four youngest" below still means
-    // slab k + 1 has landed, and the steps with it.
-    [[maybe_unused]] float blk_sa_next = 0.0f, blk_sb_next = 0.0f;
-    [[maybe_unused]] const int kblocks = ksteps;
-    auto request_steps = [&](int kb) __attribute__((always_inline)) {
-        if constexpr (ScaleKind == SCALE_BLOCK128) {
-            static_assert(S == 4, "the wait counts of the block-scaled loop are written for four stages");
-            const int mrow = mw + lrow;
-            const int kc = min(kb, kblocks - 1);   // past the end: a harmless re-read
-            blk_sa_next = (mrow < g.m) ? g.sa[(size_t)mrow * kblocks + kc] : 0.0f;
-            blk_sb_next = g.sb[(size_t)(n0 >> 7) * kblocks + kc];
+    // the row's and the block's steps, behind the MFMAs of the next slab. The steps of four slabs are one load of the row's and
+    // one of the block's (a load a slab touched a line a row, on the load path that the slabs come through), requested in the
+    // first slab of the four before, ahead of its slab loads; past the last slab and past M they are never used. Buffer loads
+    // whatever the compiler makes of the addresses: the waits count them. 145 x 4096 x 4096 12.9 -> 9.4 us (9.0 with one scale),
+    // 300 x 4096 x 4096 19.6 -> 15.5, 600 x 1536 x 7168 22.4 -> 18.1, 70 x 7168 x 2048 8.1 -> 6.5; the products behind the next slab's
+    // MFMAs alone 11.3, 20.4, 19.9, 7.35.
+    constexpr int STEPS = ScaleKind == SCALE_BLOCK128 ? 2 : 0;
+    [[maybe_unused]] u32x4 steps[2], steps_next[2];
+    [[maybe_unused]] float behind = 0.0f;
+    [[maybe_unused]] Acc pa, pb;
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsa = make_rsrc(g.sa, STEPS ? (uint32_t)g.m * (uint32_t)ksteps * 4u : 0u);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsb = make_rsrc(g.sb, STEPS ? (uint32_t)((g.n + 127) >> 7) * (uint32_t)ksteps * 4u : 0u);
+    auto request_steps = [&](int kb, u32x4 (&d)[2]) __attribute__((always_inline)) {
+        if constexpr (STEPS > 0) {
+            d[0] = buf_load16(rsa, (uint32_t)(mw + lrow) * (uint32_t)ksteps * 4u, (uint32_t)kb * 4u);
+            d[1] = buf_load16(rsb, (uint32_t)(n0 >> 7) * (uint32_t)ksteps * 4u, (uint32_t)kb * 4u);
         }
     };
+    if constexpr (STEPS > 0) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) pb[j] = 0;
+    }
 
     // ---- prologue: slabs 0 .. S-2 in flight; slab 0 visible and in the first register set
-    request_steps(0);
+    request_steps(0, steps);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < S - 1; ++s) issue(s, s);
     wait_vmcnt<4 * (S - 2)>();
@@ -156,22 +167,34 @@ __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
     int rd_stage = 1;        // stage of slab k + 1
     int wr_stage = S - 1;    // stage of slab k + S - 1
     // one slab: MFMAs on (xc, wc) = slab k; slab k + 1 published and read into (xn, wn); slab k + S - 1 requested
-    auto step = [&](int k, const u32x4 (&xc)[4], const u32x4 (&wc)[4], u32x4 (&xn)[4], u32x4 (&wn)[4]) __attribute__((always_inline)) {
-        wait_vmcnt<4 * (S - 3)>();   // own loads of slab k + 1 (younger: slabs k + 2 .. k + S - 2)
+    // (128-block scales: AT: which of its four slabs; MORE: four more follow them, whose steps the first requests; part, before:
+    // this slab's product and the last one's)
+    auto step = [&](auto at, auto more, int k, const u32x4 (&xc)[4], const u32x4 (&wc)[4], u32x4 (&xn)[4], u32x4 (&wn)[4],
+                    [[maybe_unused]] Acc& part, [[maybe_unused]] const Acc& before) __attribute__((always_inline)) {
+        constexpr int AT = decltype(at)::value;
+        constexpr bool MORE = decltype(more)::value;
+        wait_vmcnt<4 * (S - 3) + (MORE && AT == 1 ? STEPS : 0)>();   // own loads of slab k + 1 (younger: slabs k + 2 .. k + S - 2)
         wait_lgkmcnt0();             // own reads of slab k
         phase_barrier();
-        [[maybe_unused]] const float sc = blk_sa_next * blk_sb_next;   // slab k's steps
-        request_steps(k + 1);
+        if constexpr (STEPS > 0 && MORE && AT == 0) {
+            static_assert(S == 4, "the waits of the block-scaled loop are written for four stages");
+            request_steps(k + 4, steps_next);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         issue(wr_stage, k + S - 1);
         read(rd_stage, xn, wn);
         if constexpr (ScaleKind == SCALE_BLOCK128) {
-            Acc part;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 16; ++j) part[j] = 0;
+            for (int q = 0; q < Op::STEPS; ++q) {
+                if (q == 0) part = Op::mma_step(q, wc, xc, Acc{});
+                else part = Op::mma_step(q, wc, xc, part);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = 0; q < Op::STEPS; ++q) part = Op::mma_step(q, wc, xc, part);
-#pragma unroll
-            for (int j = 0; j < 16; ++j) acc[j] += part[j] * sc;
+                for (int j = 16 / Op::STEPS * q; j < 16 / Op::STEPS * (q + 1); ++j) acc[j] += before[j] * behind;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            behind = __uint_as_float(steps[0][AT]) * __uint_as_float(steps[1][AT]);
         } else {
 #pragma unroll
             for (int q = 0; q < Op::STEPS; ++q) acc = Op::mma_step(q, wc, xc, acc);
@@ -179,9 +202,33 @@ __global__ __launch_bounds__(256) void gemm_small64_kernel(GemmArgs g) {
         rd_stage = (rd_stage == S - 1) ? 0 : rd_stage + 1;
         wr_stage = (wr_stage == S - 1) ? 0 : wr_stage + 1;
     };
-    for (int k = 0; k < ksteps; k += 2) {
-        step(k, xa, wa, xb, wb);
-        if (k + 1 < ksteps) step(k + 1, xb, wb, xa, wa);
+    constexpr std::integral_constant<int, 0> at0{};
+    if constexpr (STEPS > 0) {
+        constexpr std::integral_constant<int, 1> at1{};
+        constexpr std::integral_constant<int, 2> at2{};
+        constexpr std::integral_constant<int, 3> at3{};
+        int k = 0;
+        for (; k + 3 < ksteps; k += 4) {
+            step(at0, std::true_type{}, k, xa, wa, xb, wb, pa, pb);
+            step(at1, std::true_type{}, k + 1, xb, wb, xa, wa, pb, pa);
+            step(at2, std::true_type{}, k + 2, xa, wa, xb, wb, pa, pb);
+            step(at3, std::true_type{}, k + 3, xb, wb, xa, wa, pb, pa);
+            steps[0] = steps_next[0];
+            steps[1] = steps_next[1];
+        }
+        if (k < ksteps) step(at0, std::false_type{}, k, xa, wa, xb, wb, pa, pb);
+        if (k + 1 < ksteps) step(at1, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
+        if (k + 2 < ksteps) step(at2, std::false_type{}, k + 2, xa, wa, xb, wb, pa, pb);
+    } else {
+        for (int k = 0; k < ksteps; k += 2) {
+            step(at0, std::false_type{}, k, xa, wa, xb, wb, pa, pb);
+            if (k + 1 < ksteps) step(at0, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
+        }
+    }
+    if constexpr (STEPS > 0) {
+        const Acc& last = (ksteps & 1) ? pa : pb;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] += last[j] * behind;
     }
     // no load outlives the kernel's use of LDS: the remaining ones ran on empty descriptors or are waited for here
     wait_vmcnt<0>();
