@@ -323,7 +323,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
     // shadow of one 32x32x64 MFMA. While the eight MFMAs of sub-tile 0 issue,
     // sub-tile 1 (not yet touched in this slab) is brought to this slab's scale;
     // while those of sub-tile 1 issue, sub-tile 0 (finished for this slab) is
-    // brought to the next slab's. The scales are therefore requested two slabs
+    // brought to the next slab's. The scales are therefore requested at least two slabs
     // ahead, after the phase's slab loads (a wait in front of a slab load would
     // delay it), and turned into factors in the next operand-read
     // phase, when every load older than them has landed long ago: a scale load
@@ -342,16 +342,18 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
         make_rsrc(g.sa, kBlk ? (uint32_t)g.m * (uint32_t)kblocks * 4u : 0u);
     [[maybe_unused]] const uint32_t sa_off =
         (uint32_t)(m0 + wave_m * Cfg::WAVE_M + lane) * (uint32_t)kblocks * 4u;
-    // (a wave whose columns all lie past N clamps to the last block: its outputs are dropped)
-    [[maybe_unused]] const float* const sb_row =
-        kBlk ? g.sb + (size_t)min((n0 + wave_n * Cfg::WAVE_N) >> 7, ((g.n + 127) >> 7) - 1) * kblocks : nullptr;
-    [[maybe_unused]] float blk_sa_ld = 1.0f, blk_sb_ld = 1.0f;  // scales in flight
-    [[maybe_unused]] auto load_block_scales = [&](int kb) {
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsb =
+        make_rsrc(g.sb, kBlk ? (uint32_t)((g.n + 127) >> 7) * (uint32_t)kblocks * 4u : 0u);
+    // (a wave whose columns all lie past N: zeros, its outputs are dropped)
+    [[maybe_unused]] const uint32_t sb_off = (uint32_t)((n0 + wave_n * Cfg::WAVE_N) >> 7) * (uint32_t)kblocks * 4u;
+    // Scales in flight: a row's (and the weight block's) of four slabs in one load, requested where the last four are used up.
+    // (A load a slab touches a line for each of the 64 rows, 512 of the 1536 cycles a slab that the load path was busy for: 8192 x 2048 x
+    // 7168 113 -> 110.8 us, 4096^3 66.4 -> 64.8, 2600 x 4096 x 4096 53.0 -> 51.9, 1454 x 7168 x 2048 29.5 -> 29.0.)
+    [[maybe_unused]] u32x4 blk_sa_ld, blk_sb_ld;
+    [[maybe_unused]] auto load_block_scales = [&](int kb) {   // kb: a multiple of four; past the end they are never used
         if constexpr (kBlk) {
-            kb = min(kb, kblocks - 1);  // past the end: a harmless re-read
-            blk_sb_ld = sb_row[kb];
-            blk_sa_ld = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(rsa, sa_off, (uint32_t)kb * 4u, 0));
+            blk_sb_ld = buf_load16(rsb, sb_off, (uint32_t)kb * 4u);
+            blk_sa_ld = buf_load16(rsa, sa_off, (uint32_t)kb * 4u);
         }
     };
     [[maybe_unused]] auto at_least = [](float step) {
@@ -360,11 +362,15 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
         asm("v_maximum3_f32 %0, |%1|, %2, %2" : "=v"(m) : "v"(step), "s"(kLeastStep));
         return copysignf(m, step);
     };
-    // the scales in flight, per sub-tile
-    [[maybe_unused]] auto landed_scales = [&](float (&next)[2]) {
+    // slab kb's, per sub-tile
+    [[maybe_unused]] auto landed_scales = [&](int kb, float (&next)[2]) {
+        auto of_slab = [&](const u32x4& four) {
+            const uint32_t even = (kb & 2) ? four.z : four.x, odd = (kb & 2) ? four.w : four.y;
+            return __uint_as_float((kb & 1) ? odd : even);
+        };
         // v_permlane32_swap of a register with itself: first result = the low
         // half's values in both halves (rows 0..31), second = the high half's
-        const float sa = at_least(blk_sa_ld), sb = at_least(blk_sb_ld);
+        const float sa = at_least(of_slab(blk_sa_ld)), sb = at_least(of_slab(blk_sb_ld));
         const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(sa), __float_as_uint(sa), false, false);
         next[0] = __uint_as_float(both[0]) * sb;
         next[1] = __uint_as_float(both[1]) * sb;
@@ -373,9 +379,9 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
     // slab loads the compiler would wait for those too), behind its slab loads they become factors: while the operand
     // reads are under way, not after them in front of the barrier (3001 x 2048 x 7168 75.9 -> 70.6 us, 8192 103 -> 101)
     [[maybe_unused]] float blk_next[2];
-    [[maybe_unused]] auto take_scales = [&] {
+    [[maybe_unused]] auto take_scales = [&](int k) {
         if constexpr (kBlk) {
-            landed_scales(blk_next);
+            landed_scales(k + 1, blk_next);
             asm volatile("" : "+v"(blk_next[0]), "+v"(blk_next[1]));
         }
     };
@@ -422,8 +428,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
     load_block_scales(0);
     __builtin_amdgcn_s_waitcnt(0);  // vmcnt(0) lgkmcnt(0) expcnt(0)
     if constexpr (kBlk) {
-        landed_scales(blk_s);  // the accumulators start out at slab 0's scale
-        load_block_scales(1);
+        landed_scales(0, blk_s);  // the accumulators start out at slab 0's scale
     }
     __syncthreads();
     PP_STAMP();
@@ -445,10 +450,10 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
         int xs = 0;  // k % 3
         for (int k = 0; k < ksteps; ++k) {
             read_frags(xs, k & 1);
-            take_scales();
+            take_scales(k);
             if (k >= 1 && k + 1 < ksteps) issue_loads(k + 1, (k + 1) & 1);
             next_factors(k);
-            load_block_scales(k + 2);
+            if (kBlk && (k & 3) == 2) load_block_scales(k + 2);
             // always one touch, so that "all but the last one" below means the slab
             // loads; past the end it re-touches the last slab (an L2 hit)
             prefetch(min(k + kPrefetch, ksteps - 1));
@@ -470,18 +475,20 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_pingpong_kernel(GemmArgs g)
         // memory phase of slab k and the barrier that ends it
         auto memory_phase = [&](int k, int xs) {
             read_frags(xs, k & 1);
-            take_scales();
+            take_scales(k);
             const int xs2 = (xs == 0) ? 2 : xs - 1;  // (k + 2) % 3
             const bool more = k + 2 < ksteps;
             if (more) issue_loads(k + 2, xs2);
             next_factors(k);
-            load_block_scales(k + 2);
+            const bool scales = kBlk && (k & 3) == 2;
+            if (scales) load_block_scales(k + 2);
             prefetch(min(k + 2 + kPrefetch, ksteps - 1));
             wait_lgkmcnt0();
             // slab k+1 (issued one slab ago) must have landed; this slab's eight
             // loads and the two latest touches may stay in flight
-            // (block scales: and this phase's two scale loads)
-            if (more) wait_vmcnt<8 + 2 * kTouch + (kBlk ? 2 : 0)>();
+            // (block scales: and this phase's two scale loads, if any)
+            if (more && scales) wait_vmcnt<8 + 2 * kTouch + 2>();
+            else if (more) wait_vmcnt<8 + 2 * kTouch>();
             else wait_vmcnt<kTouch>();
             phase_barrier();  // B_{k+1}
         };
