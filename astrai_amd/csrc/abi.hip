@@ -925,6 +925,26 @@ int astrai_w8a8_linear_fp8_backward_bf16(const void* g, const void* x, const voi
     return check_launch(what);
 }
 
+int64_t astrai_w8a8_linear_backward_scratch_bytes(int64_t m, int64_t n, int64_t k) {
+    return w8a8::linear_grad_bf16_supported(m, n, k) ? w8a8::linear_grad_bf16_scratch_bytes(m, n, k) : -1;
+}
+
+int astrai_w8a8_linear_backward_bf16(const void* g, const void* x, const void* w, void* scratch, void* grad_x, void* grad_w,
+                                     void* grad_bias, int64_t m, int64_t n, int64_t k, void* stream) {
+    const char* what = "linear_backward_bf16";
+    if (!g || (!grad_x && !grad_w) || (grad_x && !w) || (grad_w && !x) || (grad_bias && !grad_w))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
+    if (!aligned16(g) || !aligned16(x) || !aligned16(w) || !aligned16(scratch) || !aligned16(grad_x) || !aligned16(grad_w) ||
+        !aligned16(grad_bias))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
+    if (!w8a8::linear_grad_bf16_supported(m, n, k))
+        return fail(ASTRAI_W8A8_UNSUPPORTED, "%s: needs N %% 64 == 0, K %% 8 == 0 and operands of up to 2 GiB", what);
+    if (!scratch && w8a8::linear_grad_bf16_scratch_bytes(m, n, k))
+        return fail(ASTRAI_W8A8_BAD_ARG, "%s: null scratch", what);
+    w8a8::launch_linear_grad_bf16(g, x, w, scratch, grad_x, grad_w, grad_bias, m, n, k, static_cast<hipStream_t>(stream));
+    return check_launch(what);
+}
+
 int astrai_w8a8_gemm_fp8_ptpc(const void* a8, const void* b8, const float* sa, const float* sb,
                               const void* bias, void* out, int64_t m, int64_t n, int64_t k,
                               int fmt, void* stream) {

@@ -129,12 +129,12 @@ struct TileCoord {
 // tile-rows so that the ~32 tiles resident on one XCD share A rows and B rows. (Also where the tiles are no multiple
 // of 8, which dealt them out in launch order before: int8 3001 x 4096 x 11008 165 -> 158 us, fp8 175 -> 168 at 3700
 // tokens, bf16 tiles of twice the bytes 2500 x 4096 x 22016 466 -> 332.)
+template <int GROUP = 4>
 __device__ __forceinline__ TileCoord map_tile(int tiles_m, int tiles_n) {
     const int nwg = tiles_m * tiles_n;
     int pid = blockIdx.x;
     const int per = nwg >> 3, rest = nwg & 7, xcd = pid & 7;   // the first `rest` of them take one tile more
     pid = xcd * per + min(xcd, rest) + (pid >> 3);
-    constexpr int GROUP = 4;
     const int width = GROUP * tiles_n;
     const int group = pid / width;
     const int first_m = group * GROUP;

@@ -293,6 +293,21 @@ bool launch_gemm_int8_rope_cache(const GemmArgs& g, const RopeCacheArgs& rc, hip
 // at least 192 output tiles of 256 x 256, K % 128 == 0; false when the shape does not fit
 bool launch_gemm_int8_rope_cache_large(const GemmArgs& g, const RopeCacheArgs& rc, hipStream_t stream);
 
+// grad_gemm.hip: the products of a Linear's backward on bf16 tensors as they are: gx [m, k] = g w, gw [n, k] = g^T x (either may
+// be null) and, with gw, gb [n], the column sums of g (or null). m, n, k > 0, n % 64 == 0, k % 8 == 0 and operands of up to 2
+// GiB; scratch of linear_grad_bf16_scratch_bytes, 16-byte aligned.
+struct GradGemmArgs {      // out [p, q] = sum over t of A(p, t) B(t, q); B [t, q], A [p, t] or [t, p]
+    const void *a, *b;
+    void *out, *sums;      // sums: A's over t, bf16 [p], or null
+    float* partial;        // several ranges of t: a plane of fp32 results (and sums) each
+    int64_t plane;         // floats of one
+    int p, q, t, splits, slabs_per_split;
+};
+bool linear_grad_bf16_supported(int64_t m, int64_t n, int64_t k);
+int64_t linear_grad_bf16_scratch_bytes(int64_t m, int64_t n, int64_t k);
+void launch_linear_grad_bf16(const void* g, const void* x, const void* w, void* scratch, void* gx, void* gw, void* gb, int64_t m,
+                             int64_t n, int64_t k, hipStream_t stream);
+
 // mfma_probe.hip: one instruction of MFMA shape `kind` on a zero accumulator, one wave;
 // d_raw[lane][reg] are the accumulator registers as they are (4 or 16 per lane)
 bool launch_mfma_probe(int kind, const void* a, const void* b, void* d_raw, hipStream_t stream);

@@ -34,4 +34,16 @@ __device__ __forceinline__ void lds_dma16(u32x4 desc, uint32_t lds_addr, uint32_
         : "memory");
 }
 
+// The same at lds_addr + AT, soff (a scalar register) further on in memory: range-checked as part of the offset
+template <int AT>
+__device__ __forceinline__ void lds_dma16_at(u32x4 desc, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
+    __asm__ volatile(
+        "s_add_u32 m0, %0, %4\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "s"(lds_addr), "v"(voff), "s"(desc), "s"(soff), "n"(AT)
+        : "memory", "scc");
+}
+
 }  // namespace w8a8

@@ -99,6 +99,8 @@ PROTOTYPES = {
     "astrai_w8a8_linear_fp8_backward_scratch_bytes": ([_I64] * 3, _I64),
     "astrai_w8a8_linear_fp8_backward_bf16": (
         [_P] * 10 + [_I64] * 3 + [_INT, _P, _INT, _INT, _F32, _F32, _P], _INT),
+    "astrai_w8a8_linear_backward_scratch_bytes": ([_I64] * 3, _I64),
+    "astrai_w8a8_linear_backward_bf16": ([_P] * 7 + [_I64] * 3 + [_P], _INT),
     "astrai_w8a8_gemv_int8_ptpc": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_tiled": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P], _INT),
     "astrai_w8a8_gemm_int8_ptpc_rope_cache": (
@@ -481,6 +483,39 @@ def linear_fp8_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, want_
             g.data_ptr(), x.data_ptr(), w.data_ptr(), *(_ptr(t) for t in steps), scratch.data_ptr(), gx.data_ptr(),
             gw.data_ptr(), gb.data_ptr() if want_bias else None, m, n, k, fmt, *_ring(ring, g), fmax, pow2_margin, _stream(g)),
             lib)
+    return gx, gw, gb
+
+
+def linear_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, masks):
+    """Input, weight and bias gradient of a bf16 Linear (empty tensors where ``masks`` ask for none), ``g [m, n]``, ``x [m,
+    k]``, ``w [n, k]``; ``None`` for what the kernels do not take as it is.
+
+    The input gradient is the library's product where its 128 x 128 tiles take more than one round of the compute units: these
+    kernels are 0.83 to 1.14 times as fast there (4096 x 4096 x 4096 130 us, the library 108; 1700 x 4096 x 4096 58 and 63), and 1.0
+    to 3 times up to there (552 x 11264 x 2048 40 and 91, 1700 x 2048 x 2048 18 and 26; 256 x 2048 x 2048 14.4 and 13.5). So is the weight
+    gradient of the largest whole blocks without a bias (operands from memory: 4096 x 4096 x 4096 141 us, the library 136, and 20 more
+    for the sums; 8192 x 8192 x 2048 268 and 243; 2500 x 11264 x 2048 122 and 155, 1024 x 4096 x 11008 125 and 121)."""
+    lib = _require()
+    if not (g.is_cuda and all(_plain_bf16(t, g.device) for t in (g, x, w)) and (masks[0] or masks[1])
+            and (masks[1] or not masks[2])):
+        return None
+    (n, k), m, dev = w.shape, g.size(0), g.device
+    if x.shape != (m, k) or g.size(1) != n:
+        return None
+    scratch_bytes = lib.astrai_w8a8_linear_backward_scratch_bytes(m, n, k)
+    if scratch_bytes < 0:
+        return None
+    own_x = masks[0] and -(-m // 128) * -(-k // 128) <= 256
+    own_w = masks[1] and (masks[2] or m % 64 != 0 or m * n * k < 6e10)
+    with _on_device(dev):
+        gx = torch.mm(g, w) if masks[0] and not own_x else torch.empty(x.shape if own_x else 0, device=dev, dtype=x.dtype)
+        gw = torch.mm(g.t(), x) if masks[1] and not own_w else torch.empty(w.shape if own_w else 0, device=dev, dtype=w.dtype)
+        gb = torch.empty(n if masks[2] else 0, device=dev, dtype=w.dtype)
+        if own_x or own_w:
+            scratch = torch.empty(scratch_bytes, device=dev, dtype=torch.uint8) if scratch_bytes else None
+            _check(lib.astrai_w8a8_linear_backward_bf16(
+                g.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(scratch), gx.data_ptr() if own_x else None,
+                gw.data_ptr() if own_w else None, gb.data_ptr() if masks[2] else None, m, n, k, _stream(g)), lib)
     return gx, gw, gb
 
 

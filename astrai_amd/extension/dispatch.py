@@ -13,6 +13,8 @@ from typing import Callable, List, Optional
 import torch
 from torch.library import Library
 
+from astrai_amd.extension import _cabi
+
 Handler = Callable[[torch.Tensor, torch.Tensor, Optional[torch.Tensor]], Optional[torch.Tensor]]
 
 _handlers: List[Handler] = []
@@ -38,7 +40,7 @@ def _linear_backward_cuda_impl(input_tensor, grad_output, weight, output_mask):
     """Overriding ``linear`` on the CUDA key makes autograd call
     ``aten::linear_backward``, which has no stock CUDA kernel; policies may take
     it (fp8 backward), otherwise this is the plain matmul form the reference
-    falls back to (fp8.py:382-401)."""
+    falls back to (fp8.py:382-401), in bf16 on the backward's own kernels."""
     for h in _backward_handlers:
         out = h(input_tensor, grad_output, weight, output_mask)
         if out is not None:
@@ -47,6 +49,11 @@ def _linear_backward_cuda_impl(input_tensor, grad_output, weight, output_mask):
     grad = grad_output.to(dt)
     g2 = grad.reshape(-1, weight.size(0))
     x2 = input_tensor.reshape(-1, input_tensor.size(-1)).to(dt)
+
+    if dt == torch.bfloat16 and g2.is_cuda and input_tensor.dtype == dt and _cabi.load() is not None:
+        grads = _cabi.linear_backward(g2, x2, weight, output_mask)
+        if grads is not None:
+            return (grads[0].reshape_as(input_tensor) if output_mask[0] else grads[0]), grads[1], grads[2]
 
     def none():
         return torch.empty(0, device=input_tensor.device, dtype=input_tensor.dtype)

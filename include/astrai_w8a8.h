@@ -620,6 +620,17 @@ int astrai_w8a8_linear_fp8_backward_bf16(const void* g_bf16, const void* x_bf16,
                                          float* g_hist, int g_len, int g_idx, float fmax, float pow2_margin, void* stream);
 
 /*
+ * A Linear's backward in bf16 (fp32 sums, each result rounded once): grad_x [m, k] = g w, grad_w [n, k] = g^T x, grad_bias [n]
+ * the column sums of g, from the tensors as they are (g [m, n], x [m, k], w [n, k]). grad_x or grad_w may be NULL, grad_bias
+ * too and is formed with grad_w. n % 64 == 0, k % 8 == 0 and operands of up to 2 GiB, else ASTRAI_W8A8_UNSUPPORTED (and -1
+ * bytes of scratch); all pointers 16-byte aligned. scratch: astrai_w8a8_linear_backward_scratch_bytes(m, n, k) bytes.
+ */
+int64_t astrai_w8a8_linear_backward_scratch_bytes(int64_t m, int64_t n, int64_t k);
+int astrai_w8a8_linear_backward_bf16(const void* g_bf16, const void* x_bf16, const void* w_bf16, void* scratch,
+                                     void* grad_x_bf16, void* grad_w_bf16, void* grad_bias_bf16, int64_t m, int64_t n, int64_t k,
+                                     void* stream);
+
+/*
  * The decode int8 kernels on their own: same contract as
  * astrai_w8a8_gemm_int8_ptpc but requires M <= 128 and K % 256 == 0, and
  * returns ASTRAI_W8A8_UNSUPPORTED otherwise.
