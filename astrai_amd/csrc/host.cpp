@@ -3,10 +3,14 @@
 // attribute reads, allocations and ctypes in Python / here / its kernels alone (us): int8, 16 tokens through 4096 x 11008
 // weights 15.3 / 11.9 / 11.6; fp8 21.5 / 16 / 15.4; 128-block fp8, 4 tokens, 7168 x 2048 21.8 / 14.7 / 8.3; paged decode, 4 x
 // 500 keys 13.6 / 9.8 / 9.4; attention of 100 dense tokens 12.4 / 7.0 / 6.5; an fp8 training step of 256 tokens, 2048 x 2048
-// 152 / 122. A function returns None where a call is not the plain case that it checks for; the adapter then takes its own
+// 152 / 122; of 300 tokens, 2048 x 3072, whose bf16 backward is one call too, 81 / 61. A function returns None where a call is not the plain case that it checks for; the adapter then takes its own
 // path, which says what is wrong or makes it right. Only exact torch.Tensor / Parameter objects are plain: subclasses see
 // the operations that they would see without this module.
 #include "host.h"
+
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 
 #include "../../include/astrai_w8a8.h"
 
@@ -151,6 +155,36 @@ PyObject* linear_fp8_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) 
     END_HANDLE_TH_ERRORS
 }
 
+// linear_backward(g, x, w, want_x, want_w, want_bias): the kernels' own products, those that want_* ask for
+PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    const Tensor *g, *x, *w;
+    if (n_args != 6 || !(g = tensor_of(a[0])) || !(x = tensor_of(a[1])) || !(w = tensor_of(a[2])) || !PyBool_Check(a[3]) ||
+        !PyBool_Check(a[4]) || !PyBool_Check(a[5]) || !g->is_cuda() || g->dim() != 2 || x->dim() != 2 || w->dim() != 2)
+        Py_RETURN_NONE;
+    const auto dev = g->device();
+    const int64_t m = g->size(0), n = w->size(0), k = w->size(1);
+    const bool want_x = a[3] == Py_True, want_w = a[4] == Py_True, want_bias = a[5] == Py_True;
+    if (g->size(1) != n || x->size(0) != m || x->size(1) != k || !plain16(*g, at::kBFloat16, dev) || !plain16(*x, at::kBFloat16, dev) ||
+        !plain16(*w, at::kBFloat16, dev) || !(want_x || want_w) || (want_bias && !want_w))
+        Py_RETURN_NONE;
+    const int64_t need = astrai_w8a8_linear_backward_scratch_bytes(m, n, k);
+    if (need < 0) Py_RETURN_NONE;
+    const c10::DeviceGuard guard(dev);
+    const Tensor scratch = need ? bytes(need, dev) : Tensor();
+    const auto bf16 = at::TensorOptions().device(dev).dtype(at::kBFloat16);
+    auto matrix = [&](bool want, int64_t rows) { return want ? at::empty({rows, k}, bf16) : at::empty({0}, bf16); };
+    Tensor gx = matrix(want_x, m), gw = matrix(want_w, n), gb = at::empty({want_bias ? n : 0}, bf16);
+    const int rc = unlocked([&] {
+        return astrai_w8a8_linear_backward_bf16(g->data_ptr(), x->data_ptr(), w->data_ptr(), need ? scratch.data_ptr() : nullptr,
+                                                want_x ? gx.data_ptr() : nullptr, want_w ? gw.data_ptr() : nullptr,
+                                                want_bias ? gb.data_ptr() : nullptr, m, n, k, stream_of(dev));
+    });
+    if (rc) return failed(rc);
+    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(gx)), THPVariable_Wrap(std::move(gw)), THPVariable_Wrap(std::move(gb)));
+    END_HANDLE_TH_ERRORS
+}
+
 // quantize_block128_act(x)
 PyObject* quantize_block128_act(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
@@ -192,6 +226,35 @@ PyObject* mm_block128(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
                                              out.data_ptr(), m, n, k, stream_of(dev));
     });
     return rc ? failed(rc) : THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// Whether a dispatcher op on these would do nothing but call its device kernel: plain tensors of one GPU that need no
+// gradient and carry no tangent, no dispatch or function mode, transform, trace or functionalization about.
+bool nothing_above(std::initializer_list<const Tensor*> tensors) {
+    using K = c10::DispatchKey;
+    static const c10::DispatchKeySet above({K::Python, K::PythonTLSSnapshot, K::PythonDispatcher, K::PreDispatch, K::Functionalize,
+                                            K::FuncTorchDynamicLayerFrontMode, K::FuncTorchDynamicLayerBackMode, K::FuncTorchBatched,
+                                            K::FuncTorchVmapMode, K::FuncTorchGradWrapper, K::FuncTorchBatchedDecomposition,
+                                            K::BatchedNestedTensor, K::NestedTensor, K::Tracer, K::Fake, K::Negative, K::Conjugate,
+                                            K::DeferredInit});
+    const auto on = c10::impl::tls_local_dispatch_key_set();
+    if (!(on.included_ & above).empty() || at::impl::torch_function_mode_enabled()) return false;
+    const bool grads = c10::GradMode::is_enabled();
+    for (const Tensor* t : tensors)
+        if (t && (!(t->key_set() & above).empty() || (grads && t->requires_grad()) || t->_fw_grad(0).defined())) return false;
+    return true;
+}
+
+// mm_block128_eager(a, b, sa, sb, bias): the op fp8_gemm_blockscaled where nothing is above its device kernel
+PyObject* mm_block128_eager(PyObject* self, PyObject* const* args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    const Tensor* t[5] = {};
+    if (n_args != 5 || !optional(args[4], t[4])) Py_RETURN_NONE;
+    for (int i = 0; i < 4; ++i)
+        if (!(t[i] = tensor_of(args[i]))) Py_RETURN_NONE;
+    if (!nothing_above({t[0], t[1], t[2], t[3], t[4]})) Py_RETURN_NONE;
+    return mm_block128(self, args, n_args);
     END_HANDLE_TH_ERRORS
 }
 
@@ -326,8 +389,8 @@ PyObject* attn_prefill(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {ENTRY(linear_int8), ENTRY(linear_fp8_operands), ENTRY(linear_fp8), ENTRY(linear_fp8_backward),
-                         ENTRY(quantize_block128_act), ENTRY(mm_block128), ENTRY(attn_paged_decode), ENTRY(attn_paged_prefill),
+PyMethodDef methods[] = {ENTRY(linear_int8), ENTRY(linear_fp8_operands), ENTRY(linear_fp8), ENTRY(linear_fp8_backward), ENTRY(linear_backward),
+                         ENTRY(quantize_block128_act), ENTRY(mm_block128), ENTRY(mm_block128_eager), ENTRY(attn_paged_decode), ENTRY(attn_paged_prefill),
                          ENTRY(attn_prefill), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods};
 

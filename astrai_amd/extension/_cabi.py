@@ -496,17 +496,21 @@ def linear_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, masks):
     gradient of the largest whole blocks without a bias (operands from memory: 4096 x 4096 x 4096 141 us, the library 136, and 20 more
     for the sums; 8192 x 8192 x 2048 268 and 243; 2500 x 11264 x 2048 122 and 155, 1024 x 4096 x 11008 125 and 121)."""
     lib = _require()
-    if not (g.is_cuda and all(_plain_bf16(t, g.device) for t in (g, x, w)) and (masks[0] or masks[1])
+    (n, k), m, dev = w.shape, g.size(0), g.device
+    own_x = masks[0] and -(-m // 128) * -(-k // 128) <= 256
+    own_w = masks[1] and (masks[2] or m % 64 != 0 or m * n * k < 6e10)
+    if own_x == masks[0] and own_w == masks[1]:
+        grads = _host.linear_backward(g, x, w, *masks)
+        if grads is not None:
+            return grads
+    if not (g.is_cuda and all(_plain_bf16(t, dev) for t in (g, x, w)) and (masks[0] or masks[1])
             and (masks[1] or not masks[2])):
         return None
-    (n, k), m, dev = w.shape, g.size(0), g.device
     if x.shape != (m, k) or g.size(1) != n:
         return None
     scratch_bytes = lib.astrai_w8a8_linear_backward_scratch_bytes(m, n, k)
     if scratch_bytes < 0:
         return None
-    own_x = masks[0] and -(-m // 128) * -(-k // 128) <= 256
-    own_w = masks[1] and (masks[2] or m % 64 != 0 or m * n * k < 6e10)
     with _on_device(dev):
         gx = torch.mm(g, w) if masks[0] and not own_x else torch.empty(x.shape if own_x else 0, device=dev, dtype=x.dtype)
         gw = torch.mm(g.t(), x) if masks[1] and not own_w else torch.empty(w.shape if own_w else 0, device=dev, dtype=w.dtype)
@@ -1755,6 +1759,13 @@ def mm_fp8_block128(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torc
                 a_c.data_ptr(), b_c.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias),
                 out.data_ptr(), m, n, k, _stream(a)), lib)
     return out
+
+
+def mm_fp8_block128_eager(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
+                          bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """:func:`mm_fp8_block128` where a dispatcher op would do nothing but call it: plain operands as the kernels read them, no
+    gradients, modes, transforms or traces about. ``None`` elsewhere."""
+    return _host.mm_block128_eager(a, b, sa, sb, bias)
 
 
 # ---------------------------------------------------------------------------

@@ -62,6 +62,7 @@ def _fp8_block_mm_module() -> SimpleNamespace:
         quantize_fp8_block128_act=_cabi.quantize_fp8_block128_act,
         quantize_fp8_block128_weight=_cabi.quantize_fp8_block128_weight,
         mm_fp8_block128=_cabi.mm_fp8_block128,
+        mm_fp8_block128_eager=_cabi.mm_fp8_block128_eager,
     )
 
 

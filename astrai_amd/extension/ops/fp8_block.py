@@ -70,4 +70,9 @@ def quantize_weight_block128(w: torch.Tensor):
 
 
 def mm_fp8_blockscaled(a8, b8, sa, sb, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The op, or, where nothing is above its device kernel, the kernel: the op's layers are 6 of the 9 us of a small call."""
+    if not torch.compiler.is_compiling() and is_available("fp8_block_mm"):
+        out = _mod().mm_fp8_block128_eager(a8, b8, sa, sb, bias)
+        if out is not None:
+            return out
     return fp8_gemm_blockscaled(a8, b8, sa, sb, bias)
