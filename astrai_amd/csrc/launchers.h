@@ -102,6 +102,22 @@ constexpr int64_t kFusedRowMax = 8192;
 void launch_add_rmsnorm_quantize_int8_rows(const void* x, const void* res, const void* w, float eps,
                                            void* sum_out, void* y_out, void* xq, float* s,
                                            int64_t rows, int64_t k, hipStream_t stream);
+// The same at the start of a forward: x[r] = table[tokens[r]] is looked up and written out, and rotary[i] = freqs[positions[i]] as
+// fp32 in the same launch. A token or position outside its table reads as NaN.
+struct StartArgs {
+    const void* table;           // bf16 [vocab, k]
+    const int64_t* tokens;       // [rows]
+    int64_t vocab;
+    const void* freqs;           // bf16 or fp32 [max_pos, cols]
+    const int64_t* positions;    // [n_pos]
+    int64_t max_pos, n_pos, cols;
+    int freqs_float;
+    float* rotary;               // [n_pos, cols]
+    void* x_out;                 // bf16 [rows, k]
+    unsigned row_blocks;         // filled in by the launcher: workgroups of rows, ahead of those of rotary
+};
+void launch_embed_rmsnorm_quantize_int8_rows(const StartArgs& e, const void* w, float eps, void* xq, float* s, int64_t rows,
+                                             int64_t k, hipStream_t stream);
 // block > 0: gate and up columns come in pieces of `block` columns, 2 * block apart
 void launch_silu_mul_quantize_int8_rows(const void* gate, const void* up, int64_t ld, int64_t block,
                                         void* h_out, void* hq, float* s, int64_t rows, int64_t width,

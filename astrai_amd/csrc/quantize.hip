@@ -622,12 +622,39 @@ __global__ __launch_bounds__(kThreads) void add_bias_bf16_kernel(uint16_t* out, 
 // with rstd = rsqrt(mean(s^2) + eps) in fp32 -- one rounding, the arithmetic of
 // F.rms_norm on a bf16 tensor (model/components/norm.py:7-15) -- then the per-row
 // int8 quantizer on y.
+// START: x is the embedding table (StartArgs), and the launch's last workgroups look up the rotary rows: a decode step is three
+// launches of about 2 us each in the chain shorter (dense decoder, 2 layers: 32 sequences 127.8 -> 122.2 us, 5 sequences 98.5 ->
+// 91.9), and a prompt reads its tokens' rows once (32 x 512: 1724 -> 1716).
+__device__ __forceinline__ void rotary_rows(const StartArgs& e) {
+    const int64_t at = (int64_t)(blockIdx.x - e.row_blocks) * kThreads + threadIdx.x;
+    if (at >= e.n_pos * e.cols) return;
+    const int64_t i = at / e.cols, pos = e.positions[i], from = pos * e.cols + (at - i * e.cols);
+    float v = __uint_as_float(0x7fc00000u);
+    if (pos >= 0 && pos < e.max_pos)
+        v = e.freqs_float ? static_cast<const float*>(e.freqs)[from] : bf16_to_f32(static_cast<const uint16_t*>(e.freqs)[from]);
+    e.rotary[at] = v;
+}
+
+// a row's place in the table, -1 outside it
+__device__ __forceinline__ int64_t table_row(const StartArgs& e, int64_t row) {
+    const int64_t tok = e.tokens[row];
+    return tok >= 0 && tok < e.vocab ? tok : -1;
+}
+
+__device__ __forceinline__ u32x4 table_piece(const uint16_t* table, int64_t at, int64_t k, int64_t i) {
+    return at >= 0 ? *reinterpret_cast<const u32x4*>(table + at * k + i * 8) : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
+}
+
+template <bool START>
 __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
     const uint16_t* __restrict__ w, float eps, uint16_t* __restrict__ sum_out,
-    uint16_t* __restrict__ y_out, int8_t* __restrict__ xq, float* __restrict__ s, int64_t k) {
+    uint16_t* __restrict__ y_out, int8_t* __restrict__ xq, float* __restrict__ s, int64_t k, StartArgs e) {
     __shared__ float slots[kThreads / kWave];
+    if (START && blockIdx.x >= e.row_blocks) return rotary_rows(e);
     const int64_t row = blockIdx.x;
+    [[maybe_unused]] int64_t from = 0;
+    if constexpr (START) from = table_row(e, row);
     const int64_t nvec = k >> 3;
     float v[kCache][8];
     // the norm weights are requested with the row, not after the reduction's barrier (a load does
@@ -643,8 +670,14 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kerne
     for (int c = 0; c < kCache; ++c) {
         const int64_t i = threadIdx.x + (int64_t)c * kThreads;
         if (i < nvec) {
-            unpack8(*reinterpret_cast<const u32x4*>(x + row * k + i * 8), v[c]);
-            if (res) {
+            if constexpr (START) {
+                const u32x4 piece = table_piece(static_cast<const uint16_t*>(e.table), from, k, i);
+                *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(e.x_out) + row * k + i * 8) = piece;
+                unpack8(piece, v[c]);
+            } else {
+                unpack8(*reinterpret_cast<const u32x4*>(x + row * k + i * 8), v[c]);
+            }
+            if (!START && res) {
                 float r[8];
                 unpack8(*reinterpret_cast<const u32x4*>(res + row * k + i * 8), r);
 #pragma unroll
@@ -667,7 +700,7 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kerne
             for (int j = 0; j < 8; ++j) v[c][j] = g[j] * (rstd * v[c][j]);
             const u32x4 packed = round8_bf16(v[c]);
             local = fmaxf(local, amax8(v[c]));
-            if (y_out) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
+            if (!START && y_out) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
         }
     }
     const float step = fmaxf(block_max(local, slots), 1e-12f) / 127.0f;
@@ -688,15 +721,22 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kerne
 // NORM: y = bf16(w * (rstd * x)), rstd = rsqrt(mean(x^2) + eps), then the per-row int8
 // quantizer on y; otherwise the quantizer on x itself. The sum of squares is taken in the
 // order of the one-workgroup-per-row kernel, so both kernels give a row the same bits.
-template <int KC, bool NORM>
+// START as above; the token of the row after the next is requested with the next row's pieces.
+template <int KC, bool NORM, bool START>
 __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, float eps,
-    uint16_t* __restrict__ y_out, int8_t* __restrict__ xq, float* __restrict__ s, int64_t rows, int64_t k) {
+    uint16_t* __restrict__ y_out, int8_t* __restrict__ xq, float* __restrict__ s, int64_t rows, int64_t k, StartArgs e) {
+    if (START && blockIdx.x >= e.row_blocks) return rotary_rows(e);
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t nvec = k >> 3;
-    const int64_t stride = (int64_t)gridDim.x * (kThreads / kWave);
+    const int64_t stride = (int64_t)(START ? e.row_blocks : gridDim.x) * (kThreads / kWave);
     int64_t row = (int64_t)blockIdx.x * (kThreads / kWave) + (threadIdx.x >> 6);
     if (row >= rows) return;
+    [[maybe_unused]] int64_t from = -1, from_next = -1;
+    if constexpr (START) {
+        from = table_row(e, row);
+        if (row + stride < rows) from_next = table_row(e, row + stride);
+    }
     const u32x4 zero = {0u, 0u, 0u, 0u};
     [[maybe_unused]] u32x4 wr[KC];
     if constexpr (NORM) {
@@ -710,15 +750,23 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
         const int64_t i = lane + (int64_t)c * kWave;
-        cur[c] = i < nvec ? *reinterpret_cast<const u32x4*>(x + row * k + i * 8) : zero;
+        if constexpr (START) cur[c] = i < nvec ? table_piece(x, from, k, i) : zero;
+        else cur[c] = i < nvec ? *reinterpret_cast<const u32x4*>(x + row * k + i * 8) : zero;
     }
     for (; row < rows; row += stride) {
         const int64_t nr = row + stride;
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             const int64_t i = lane + (int64_t)c * kWave;
-            nxt[c] = (nr < rows && i < nvec) ? *reinterpret_cast<const u32x4*>(x + nr * k + i * 8) : zero;
+            if constexpr (START) {
+                nxt[c] = (nr < rows && i < nvec) ? table_piece(x, from_next, k, i) : zero;
+                if (i < nvec) __builtin_nontemporal_store(cur[c], reinterpret_cast<u32x4*>(static_cast<uint16_t*>(e.x_out) + row * k + i * 8));
+            } else {
+                nxt[c] = (nr < rows && i < nvec) ? *reinterpret_cast<const u32x4*>(x + nr * k + i * 8) : zero;
+            }
         }
+        if constexpr (START)
+            if (nr + stride < rows) from_next = table_row(e, nr + stride);
         float v[KC][8];
         float local = 0.0f;
         if constexpr (NORM) {
@@ -750,7 +798,7 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
                 const u32x4 packed = round8_bf16(v[c]);
                 local = fmaxf(local, amax8(v[c]));
                 const int64_t i = lane + (int64_t)c * kWave;
-                if (y_out && i < nvec) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
+                if (!START && y_out && i < nvec) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
             }
         } else {
 #pragma unroll
@@ -780,20 +828,23 @@ inline bool wave_rows_fit(int64_t rows, int64_t k) {
     return rows >= kWaveRowsMin && k <= kWaveRowsMaxK && (k & 7) == 0;
 }
 
-template <bool NORM>
+inline unsigned rotary_blocks(const StartArgs& e) { return (unsigned)((e.n_pos * e.cols + kThreads - 1) / kThreads); }
+
+template <bool NORM, bool START = false>
 void launch_wave_rows(const uint16_t* x, const uint16_t* w, float eps, uint16_t* y_out, int8_t* xq,
-                      float* s, int64_t rows, int64_t k, hipStream_t stream) {
+                      float* s, int64_t rows, int64_t k, hipStream_t stream, StartArgs e = {}) {
     // The norm kernel keeps the norm weights in registers: four workgroups of four waves per compute
     // unit, each wave walking over its share of rows. The plain quantizer has nothing to keep and is
     // fastest with a wave per row (16,384 x 2048: 22.0 us against 25.1 us; the norm 22.7 against 25.0).
     const int64_t want = (rows + 3) / 4;
     const int64_t cap = NORM ? 1024 : 4096;
-    const dim3 grid((unsigned)(want < cap ? want : cap)), block(kThreads);
+    e.row_blocks = (unsigned)(want < cap ? want : cap);
+    const dim3 grid(e.row_blocks + rotary_blocks(e)), block(kThreads);
     const int64_t pieces = (k / 8 + kWave - 1) / kWave;
-    if (pieces <= 1) wave_rows_int8_kernel<1, NORM><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k);
-    else if (pieces <= 2) wave_rows_int8_kernel<2, NORM><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k);
-    else if (pieces <= 4) wave_rows_int8_kernel<4, NORM><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k);
-    else wave_rows_int8_kernel<8, NORM><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k);
+    if (pieces <= 1) wave_rows_int8_kernel<1, NORM, START><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k, e);
+    else if (pieces <= 2) wave_rows_int8_kernel<2, NORM, START><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k, e);
+    else if (pieces <= 4) wave_rows_int8_kernel<4, NORM, START><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k, e);
+    else wave_rows_int8_kernel<8, NORM, START><<<grid, block, 0, stream>>>(x, w, eps, y_out, xq, s, rows, k, e);
 }
 
 // silu(g) = g / (1 + exp(-g)) on the hardware's exp2 and reciprocal (each within one ulp
@@ -1183,10 +1234,22 @@ void launch_add_rmsnorm_quantize_int8_rows(const void* x, const void* res, const
                                static_cast<uint16_t*>(y_out), static_cast<int8_t*>(xq), s, rows, k, stream);
         return;
     }
-    add_rmsnorm_quantize_int8_rows_kernel<<<dim3((unsigned)rows), dim3(kThreads), 0, stream>>>(
+    add_rmsnorm_quantize_int8_rows_kernel<false><<<dim3((unsigned)rows), dim3(kThreads), 0, stream>>>(
         static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(res),
         static_cast<const uint16_t*>(w), eps, static_cast<uint16_t*>(sum_out),
-        static_cast<uint16_t*>(y_out), static_cast<int8_t*>(xq), s, k);
+        static_cast<uint16_t*>(y_out), static_cast<int8_t*>(xq), s, k, StartArgs{});
+}
+
+void launch_embed_rmsnorm_quantize_int8_rows(const StartArgs& e, const void* w, float eps, void* xq, float* s, int64_t rows,
+                                             int64_t k, hipStream_t stream) {
+    if (rows <= 0 || k <= 0) return;
+    if (wave_rows_fit(rows, k))
+        return launch_wave_rows<true, true>(static_cast<const uint16_t*>(e.table), static_cast<const uint16_t*>(w), eps, nullptr,
+                                            static_cast<int8_t*>(xq), s, rows, k, stream, e);
+    StartArgs a = e;
+    a.row_blocks = (unsigned)rows;
+    add_rmsnorm_quantize_int8_rows_kernel<true><<<dim3(a.row_blocks + rotary_blocks(a)), dim3(kThreads), 0, stream>>>(
+        nullptr, nullptr, static_cast<const uint16_t*>(w), eps, nullptr, nullptr, static_cast<int8_t*>(xq), s, k, a);
 }
 
 void launch_silu_mul_quantize_int8_rows(const void* gate, const void* up, int64_t ld, int64_t block,

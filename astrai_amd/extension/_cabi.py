@@ -46,6 +46,8 @@ PROTOTYPES = {
     "astrai_w8a8_quantize_transpose_padded_bf16_fp8": ([_P] * 6 + [_I64] * 3 + [_INT, _P], _INT),
     "astrai_w8a8_gradient_stats": ([_P] * 4 + [_I64] * 2 + [_P], _INT),
     "astrai_w8a8_quantize_bf16_int8_rows": ([_P, _P, _P, _I64, _I64, _P], _INT),
+    "astrai_w8a8_embed_rmsnorm_quantize_int8_rows": (
+        [_P, _I64, _P, _P, _F32, _P, _P, _P, _I64, _I64, _P, _INT, _I64, _I64, _P, _I64, _P, _P], _INT),
     "astrai_w8a8_add_rmsnorm_quantize_int8_rows": (
         [_P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _I64, _I64, _P], _INT),
     "astrai_w8a8_silu_mul_quantize_int8_rows": ([_P, _P, _I64, _P, _P, _P, _I64, _I64, _P], _INT),
@@ -820,6 +822,32 @@ def add_rmsnorm_quantize_int8(x: torch.Tensor, weight: torch.Tensor, eps: float,
             x2.data_ptr(), _ptr(r2), weight.contiguous().data_ptr(), float(eps), _ptr(t), _ptr(y),
             xq.data_ptr(), s.data_ptr(), rows, k, _stream(x)), lib)
     return (xq, s, None if t is None else t.reshape(x.shape), None if y is None else y.reshape(x.shape))
+
+
+def embed_rmsnorm_quantize_int8(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, eps: float, freqs: torch.Tensor,
+                                positions: torch.Tensor):
+    """The start of a forward in one kernel: ``x = table[ids]``, ``y = rms_norm(x) * weight``, per-row int8 of ``y``, and ``freqs``
+    (``[places, pairs, 2]``) at ``positions`` in fp32. Ids and positions outside their tables give NaN. Returns ``(x [*ids.shape, K],
+    xq [R,K], s [R,1], rotary [1, *positions.shape, pairs, 2])``, or ``None`` for operands the kernel does not take as they are."""
+    lib = _require()
+    dev, k = table.device, table.size(-1)
+    if not (table.is_cuda and _plain_bf16(table, dev) and table.dim() == 2 and _plain_bf16(weight, dev) and weight.shape == (k,)
+            and fused_rows_supported(k) and ids.numel() and positions.numel() and positions.dim() == 1
+            and all(t.dtype == torch.int64 and t.device == dev and t.is_contiguous() for t in (ids, positions))
+            and freqs.dim() == 3 and freqs.numel() and freqs.device == dev and freqs.is_contiguous()
+            and freqs.dtype in (torch.bfloat16, torch.float32)):
+        return None
+    rows, n_pos = ids.numel(), positions.numel()
+    with _on_device(dev):
+        x = torch.empty((*ids.shape, k), device=dev, dtype=torch.bfloat16)
+        xq = torch.empty((rows, k), device=dev, dtype=torch.int8)
+        s = torch.empty((rows, 1), device=dev, dtype=torch.float32)
+        rotary = torch.empty((1, n_pos, *freqs.shape[1:]), device=dev, dtype=torch.float32)
+        _check(lib.astrai_w8a8_embed_rmsnorm_quantize_int8_rows(
+            table.data_ptr(), table.size(0), ids.data_ptr(), weight.data_ptr(), float(eps), x.data_ptr(), xq.data_ptr(), s.data_ptr(),
+            rows, k, freqs.data_ptr(), freqs.dtype == torch.float32, freqs.size(0), freqs[0].numel(), positions.data_ptr(), n_pos,
+            rotary.data_ptr(), _stream(table)), lib)
+    return x, xq, s, rotary
 
 
 def silu_mul_quantize_int8(gate: torch.Tensor, up: torch.Tensor, want_h: bool = False):

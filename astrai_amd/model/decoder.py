@@ -306,16 +306,17 @@ class DecoderBlock(nn.Module):
         x = self.attention(self.input_norm(x), rotary_emb, kv_cache, positions, key_mask) + x
         return self.mlp(self.post_attention_norm(x)) + x
 
-    def _forward_fused_int8(self, x, rotary_emb, kv_cache, positions, key_mask):
+    def _forward_fused_int8(self, x, rotary_emb, kv_cache, positions, key_mask, normed=None):
         """The block on int8 projections with fused producers and epilogues: each norm is one
         kernel with the per-token quantizer, and the output and down projections add the
-        residual stream in their epilogues (``attn_output + x``, ``mlp_output + x``)."""
+        residual stream in their epilogues (``attn_output + x``, ``mlp_output + x``). ``normed``: the normed and quantized
+        ``x``, if it is there already."""
         # (the C-ABI wrappers directly: a dispatcher round trip per call is what an eager decode step,
         # ~220 launches of a few microseconds each, would otherwise spend most of its time in)
         from astrai_amd.extension import _cabi
         f, att = self.fused_int8, self.attention
         b, s, d = x.shape
-        xq, sx, _, _ = _cabi.add_rmsnorm_quantize_int8(x, self.input_norm.weight, self.input_norm.norm_eps)
+        xq, sx = normed or _cabi.add_rmsnorm_quantize_int8(x, self.input_norm.weight, self.input_norm.norm_eps)[:2]
         if kv_cache is None:
             qkv = _cabi.mm_int8(xq, f.wqkv, sx, f.sqkv).reshape(b, s, -1)
             nq, nkv = att.n_heads * att.head_dim, att.n_kv_heads * att.head_dim
@@ -374,6 +375,20 @@ class AutoRegressiveLM(nn.Module):
             raise ValueError(f"checkpoint does not match the model: missing {missing}, unexpected {unexpected}")
         return self
 
+    def _start_fused_int8(self, ids: Tensor, positions: Tensor):
+        """Embedding rows, the rotary table's rows and the first block's normed and quantized input out of one kernel:
+        ``(x, rotary, (xq, sx))``. ``None`` where the embedding or the block is not this file's own, unobserved, or the kernel
+        does not take the operands."""
+        emb, w = self.embed_tokens, self.embed_tokens.weight
+        if (self.fused_int8 is None or not _fused_int8_active(w) or not len(self.layers) or _observed(emb, Embedding)
+                or type(self.layers[0]) is not DecoderBlock or "_forward_fused_int8" in self.layers[0].__dict__
+                or any(type(t) not in (Tensor, nn.Parameter) for t in (ids, w, positions))):
+            return None
+        from astrai_amd.extension import _cabi
+        norm = self.layers[0].input_norm
+        out = _cabi.embed_rmsnorm_quantize_int8(ids, w.detach(), norm.weight.detach(), norm.norm_eps, self.freqs_cis, positions)
+        return None if out is None else (out[0], out[3], out[1:3])
+
     def new_cache(self, batch: int, max_len: int) -> DenseKVCache:
         w = self.embed_tokens.weight
         return DenseKVCache(self.config, batch, max_len, w.device, w.dtype)
@@ -388,11 +403,15 @@ class AutoRegressiveLM(nn.Module):
         if input_ids.ndim != 2:
             raise ValueError("input_ids must be [batch, seq_len]")
         b, s = input_ids.shape
-        x = self.embed_tokens(input_ids)
         if positions is None:
             positions = (torch.arange(s, device=input_ids.device) if kv_cache is None
                          else kv_cache.next_positions(s))
-        rotary = self.freqs_cis.index_select(0, positions).unsqueeze(0).float()
+        start = self._start_fused_int8(input_ids, positions)
+        if start is not None:
+            x, rotary, normed = start
+        else:
+            x, normed = self.embed_tokens(input_ids), None
+            rotary = self.freqs_cis.index_select(0, positions).unsqueeze(0).float()
         key_mask = None
         if kv_cache is not None:
             key_mask = _KeyMask(positions, kv_cache.max_len,
@@ -400,7 +419,10 @@ class AutoRegressiveLM(nn.Module):
         if self.fused_int8 is not None and _fused_int8_active(x):
             from astrai_amd.extension import _cabi
             for layer in self.layers:
-                x = layer._forward_fused_int8(x, rotary, kv_cache, positions, key_mask)
+                if normed is not None:
+                    x, normed = layer._forward_fused_int8(x, rotary, kv_cache, positions, key_mask, normed), None
+                else:
+                    x = layer._forward_fused_int8(x, rotary, kv_cache, positions, key_mask)
             if logits_at is not None:
                 s, x = logits_at.numel(), x.index_select(1, logits_at)
             hq, sh, _, hidden = _cabi.add_rmsnorm_quantize_int8(x, self.norm.weight, self.norm.norm_eps,
@@ -413,6 +435,19 @@ class AutoRegressiveLM(nn.Module):
             x = x.index_select(1, logits_at)
         hidden = self.norm(x)
         return {"logits": self.lm_head(hidden), "hidden_states": hidden}
+
+
+_EMBED, _CALL, _every = Embedding.forward, nn.Module.__call__, nn.modules.module   # as defined here; every module's hooks
+
+
+def _observed(module: nn.Module, cls: type) -> bool:
+    """A call of ``module`` runs something else than ``Embedding.forward`` as defined here: another class, hooks, a compiled
+    call, a replaced ``forward``."""
+    own = module.__dict__
+    return bool(type(module) is not cls or cls.forward is not _EMBED or cls.__call__ is not _CALL or "forward" in own
+                or own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or own.get("_compiled_call_impl") or _every._global_forward_hooks or _every._global_forward_pre_hooks
+                or _every._global_backward_hooks or _every._global_backward_pre_hooks)
 
 
 def _fused_int8_active(x: Tensor) -> bool:

@@ -167,6 +167,15 @@ int astrai_w8a8_add_rmsnorm_quantize_int8_rows(const void* x_bf16, const void* r
                                                const void* weight_bf16, float eps,
                                                void* sum_out_bf16, void* y_out_bf16, void* xq,
                                                float* s, int64_t rows, int64_t k, void* stream);
+/*
+ * The start of a forward in one launch: x_out[r,:] = table[tokens[r],:] (bf16 [vocab, k]), its norm and codes as above, and
+ * rotary[i,:] = freqs[positions[i],:] (bf16 or, with freqs_float, fp32 [max_pos, cols]) as fp32. A token or position outside
+ * its table reads as NaN. K % 8 == 0, K <= 8192.
+ */
+int astrai_w8a8_embed_rmsnorm_quantize_int8_rows(const void* table_bf16, int64_t vocab, const int64_t* tokens,
+                                                 const void* weight_bf16, float eps, void* x_out_bf16, void* xq, float* s,
+                                                 int64_t rows, int64_t k, const void* freqs, int freqs_float, int64_t max_pos,
+                                                 int64_t cols, const int64_t* positions, int64_t n_pos, float* rotary, void* stream);
 int astrai_w8a8_silu_mul_quantize_int8_rows(const void* gate_bf16, const void* up_bf16, int64_t ld,
                                             void* h_out_bf16, void* hq, float* s, int64_t rows,
                                             int64_t width, void* stream);
