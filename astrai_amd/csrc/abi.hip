@@ -653,13 +653,13 @@ int astrai_w8a8_attn_paged_prefill_masked_bf16(
     return check_launch("attn_paged_prefill_bf16");
 }
 
-// The prompt shapes that both kernels take (attn_prefill_split_supported) run the block kernel from this many
-// (64-row tile, query head) pairs, and attn_rows.hip with its context split below: the block kernel does not
-// split a context, so a few tiles over a long one leave the chip idle. Measured, split rows kernel -> block
-// kernel: 256 pairs 47 -> 18 us (32 / 8 heads x 64, 4 x 200 tokens behind 500), 31 -> 22 us (16 / 16 x 64, same),
-// 41 -> 38 us (16 / 2 x 64, 2 x 256 behind 1000); 128 pairs 31 -> 35 us (16 / 16 x 64, 2 x 256 behind 1000),
-// 75 -> 81 us (32 / 8 x 64, 256 behind 4000).
-constexpr int64_t kPrefillMinRowBlocks = 256;
+// The prompt shapes that both kernels take run the block kernel, its keys in parts where the schedule is short. Up to this
+// many (64-row tile, query head) pairs attn_rows.hip keeps what may lie behind many keys, where its waves of 16 rows and 16
+// splits fill more of the chip: us there / in the block kernel, 1 x 33 tokens behind 400: 10.1 / 12.2 (16/16 heads x 64),
+// 11.7 / 16.1 (32/4 x 64), 12.7 / 14.5 (16/16 x 128); 1 x 64 behind 500 11.7 / 12.2, 15.7 / 14.8 (16/16 x 128). With 128
+// keys at most: 1 x 33 8.9 / 6.5, 1 x 128 13.0 / 8.2 (16/16 x 64); and from 48 pairs on the block kernel's parts are the
+// faster also behind many (3 x 64 behind 500, 16/16 x 64: 15.1 / 13.9).
+constexpr int64_t kRowsMaxPairs = 32;
 
 int64_t astrai_w8a8_attn_paged_rows_workspace_floats(int64_t batch_or_tiles, int64_t n_heads,
                                                      int64_t n_kv_heads, int64_t head_dim,
@@ -706,7 +706,7 @@ int astrai_w8a8_attn_paged_rows_bf16(
                     (long long)need);
     if (prefill && !mask && w8a8::attn_prefill_split_supported((int)n_heads, (int)n_kv_heads, (int)head_dim) &&
         w8a8::attn_prefill_pool_ok(num_slots, (int)n_kv_heads, (int)head_dim) &&
-        (nsplit == 1 || batch_or_tiles * n_heads >= kPrefillMinRowBlocks)) {
+        (nsplit == 1 || batch_or_tiles * n_heads > kRowsMaxPairs || max_context_len <= 128)) {
         w8a8::AttnPrefillArgs p{};
         p.q = q; p.k_cache = k_pool; p.v_cache = v_pool; p.out = out;
         p.n_heads = (int)n_heads; p.n_kv_heads = (int)n_kv_heads; p.head_dim = (int)head_dim; p.scale = scale;
@@ -715,6 +715,7 @@ int astrai_w8a8_attn_paged_rows_bf16(
         p.q_tile_to_batch = q_tile_to_batch; p.q_tile_to_index = q_tile_to_index;
         p.num_q_tiles = (int)batch_or_tiles; p.causal = causal ? 1 : 0;
         p.rtt_stride = max_context_len; p.num_slots = num_slots; p.num_requests = num_requests;
+        p.ws = workspace; p.nsplit = w8a8::attn_prefill_parts(batch_or_tiles, (int)n_heads, max_context_len, (int)nsplit);
         if (!w8a8::launch_attn_prefill(p, static_cast<hipStream_t>(stream)))
             return fail(ASTRAI_W8A8_UNSUPPORTED, "attn_paged_rows_bf16: shape not supported");
         return check_launch("attn_paged_rows_bf16");

@@ -76,6 +76,39 @@ constexpr uint32_t kMissing = 0xffffff00u;
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
+constexpr int kMaxParts = 16;
+typedef float f32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));  // (a caller's workspace is aligned to floats only)
+typedef float f32x2_at4 __attribute__((ext_vector_type(2), aligned(4)));
+
+// What a wave leaves of a part: the accumulators as its lanes hold them, four dims of a row after four, then maximum
+// (log2 units) and sum of its 32 rows. Waves in the order of the workgroups that a schedule without parts has.
+__host__ __device__ constexpr int part_floats(int d) { return 32 * (d + 2); }
+
+// Parts of the keys, for schedules with few (64-row tile, query head) pairs: n of them leave blocks / n of the 64-key
+// blocks in the chain, 1 to 1.5 us each, and cost a write and a read of fp32 accumulators, 1 us for 48 to 64 pairs and part;
+// the sum is least at about n = sqrt(96 blocks / pairs). A block of queries counts its own keys. The launch, which knows
+// only how many there can be, has no parts where they would not save what they and the second launch cost.
+// Measured (graph replays, us), attn_rows.hip with its split, which these schedules ran before, -> here; one part in brackets:
+//   16/16 heads x 64:  1 x 33 tokens 8.9 -> 6.5, 1 x 256 15.8 -> 11.1, 3 x 64 behind 2000 24.0 -> 21.0 (41.5), 1 x 300
+//   behind 1500 31.6 -> 23.6 (37.6);  32/8 x 64: 1 x 33 10.3 -> 5.8, 1 x 256 30.1 -> 9.5, 3 x 64 behind 2000 32.8 -> 19.4
+//   (35.9), 1 x 300 behind 1500 53.6 -> 27.2 (32.8);  16/16 x 128: 10.6 -> 7.8, 21.0 -> 14.5, 35.5 -> 24.0 (58.3),
+//   48.3 -> 29.8 (52.3).
+// From 256 pairs on there are none: those schedules ran here before, in one launch, and with a wide table over short
+// contexts the second would be paid for nothing (4 x 256 behind 1000, 16/16 x 64: 26 us with one part and two).
+constexpr int kMaxPartPairs = 256, kPairsPerBlock = 96, kMergeBlocks = 1;
+
+__host__ __device__ inline int part_count(int blocks, int64_t pairs, int nsplit) {
+    int n = 1;
+    while (n < nsplit && n < blocks && (int64_t)(n + 1) * (n + 1) * pairs <= (int64_t)blocks * kPairsPerBlock) ++n;
+    return n;
+}
+
+// 64-key blocks of a part of `blocks` of them
+__device__ __forceinline__ int part_blocks(const AttnPrefillArgs& a, int blocks) {
+    const int n = part_count(blocks, (int64_t)a.num_q_tiles * a.n_heads, a.nsplit);
+    return (blocks + n - 1) / n;
+}
+
 // PAGED: the queries are packed [total_q, heads, D] with per-request row ranges
 // (qo_indptr), the caches are token-granular pools [slots, kv_heads, D] reached through
 // req_to_token, and a 64-row query tile t of the caller's schedule belongs to request
@@ -88,7 +121,9 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 // MASK (paged only): a bool tensor says, per sequence, (head,) (query row,) and position,
 // what may be attended on top of the causal range (csrc/kernels/attention/mma_utils.cuh:190-199);
 // every tile then takes the masking path.
-template <int D, int NREP, int QSUB, bool PAGED, bool MASK, bool SPLIT>
+// PARTS (paged, no mask): part `split` of a.nsplit takes the 64-key blocks part_blocks() gives it, of which nothing but
+// the table and the limits know; a block of queries with more than one part leaves them to merge_parts_kernel.
+template <int D, int NREP, int QSUB, bool PAGED, bool MASK, bool SPLIT, bool PARTS = false>
 __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && NREP * QSUB == 4 ? 3 : 2) void attn_prefill_kernel(AttnPrefillArgs a) {
     constexpr int WAVES = NREP * QSUB;
     constexpr int QB = 32 * QSUB;                 // query tokens per workgroup
@@ -118,6 +153,9 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
     const uint16_t* qbase;      // row 0 of the sequence, this wave's head
     int64_t q_row_stride;       // elements between consecutive query rows
     int pq, kmax;               // this lane's newest visible key; the block's newest
+    [[maybe_unused]] int part = 0;
+    [[maybe_unused]] bool whole = true;         // this part is all there is
+    [[maybe_unused]] float* part_ws = nullptr;  // where it goes otherwise
     [[maybe_unused]] const int* table = nullptr;
     [[maybe_unused]] int b_dense = 0, seq_index = 0;
     [[maybe_unused]] int64_t block_pos = -1;  // dense, with positions: that of the block's row `lane`
@@ -125,7 +163,12 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
         constexpr int SUBS = 64 / QB;  // workgroups that share a tile
         const int idx = (int)(gridDim.x - 1 - blockIdx.x);
         hk = idx % a.n_kv_heads;
-        const int sub = (idx / a.n_kv_heads) % SUBS, tile = idx / (SUBS * a.n_kv_heads);
+        int item = idx / a.n_kv_heads;
+        if constexpr (PARTS) {
+            part = item % a.nsplit;
+            item /= a.nsplit;
+        }
+        const int sub = item % SUBS, tile = item / SUBS;
         const int req_i = a.q_tile_to_batch[tile];
         seq_index = req_i;
         const int q_start = a.qo_indptr[req_i];
@@ -143,6 +186,16 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
         const int shift = a.causal ? kv_len - rows_total : INT_MIN;
         pq = a.causal ? min(shift + row0 + qsub * 32 + qi, kv_len - 1) : kv_len - 1;
         kmax = a.causal ? min(shift + last, kv_len - 1) : kv_len - 1;
+        if constexpr (PARTS) {
+            const int blocks = max(kmax, 0) / kKB + 1, per = part_blocks(a, blocks);
+            if (part * per >= blocks) return;
+            const int key0 = part * per * kKB;
+            whole = per >= blocks;
+            table += key0;
+            pq = min(pq - key0, per * kKB - 1);
+            kmax = min(kmax - key0, per * kKB - 1);
+part_ws = a.ws + ((((int64_t)item * a.n_kv_heads + hk) * WAVES + wave) * a.nsplit + part) * part_floats(D);
+        }
     } else {
         const int nqb = (a.seq + QB - 1) / QB;
         const int groups = a.batch * a.n_kv_heads;
@@ -681,6 +734,16 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
     }
+    if constexpr (PARTS)
+        if (!whole) {
+#pragma unroll
+            for (int g = 0; g < D / 8; ++g) {
+                const f32x16& v = o[g / 4];
+                *reinterpret_cast<f32x4_at4*>(part_ws + g * 256 + lane * 4) = f32x4_at4{v[g % 4 * 4], v[g % 4 * 4 + 1], v[g % 4 * 4 + 2], v[g % 4 * 4 + 3]};
+            }
+            if (h == 0) *reinterpret_cast<f32x2_at4*>(part_ws + 32 * D + 2 * qi) = f32x2_at4{has_value ? m_run : kNegBig, l_run};
+            return;
+        }
     {
         uint8_t* const mine = lds + wave * TILE;
 #pragma unroll
@@ -706,6 +769,61 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
     }
 }
 
+// A wave merges eight dims of the 32 rows that a wave above had. Everything the workspace could hold is requested
+// before the schedule is, which says how much of it there is: two memory round trips, not four.
+template <int D, int NREP, int QSUB>
+__global__ __launch_bounds__(256) void merge_parts_kernel(AttnPrefillArgs a, int64_t waves) {
+    constexpr int WAVES = NREP * QSUB, QB = 32 * QSUB, SUBS = 64 / QB;
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int64_t idx = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t src = idx / (D / 8);
+    const int g = (int)(idx % (D / 8));
+    if (src >= waves) return;
+    const float* const ws = a.ws + src * a.nsplit * part_floats(D);
+    f32x4 x[kMaxParts];
+    float pm[kMaxParts], pl[kMaxParts];
+#pragma unroll
+    for (int j = 0; j < kMaxParts; ++j) {
+        pm[j] = kNegBig;
+        if (j < a.nsplit) {
+            const float* const p = ws + j * part_floats(D);
+            x[j] = *reinterpret_cast<const f32x4_at4*>(p + g * 256 + lane * 4);
+            const f32x2_at4 ml = *reinterpret_cast<const f32x2_at4*>(p + 32 * D + 2 * (lane & 31));
+            pm[j] = ml.x;
+            pl[j] = ml.y;
+        }
+    }
+    const int wave = (int)(src % WAVES), hk = (int)(src / WAVES % a.n_kv_heads);
+    const int64_t item = src / WAVES / a.n_kv_heads, tile = item / SUBS;
+    const int req_i = a.q_tile_to_batch[tile], q_start = a.qo_indptr[req_i];
+    const int rows_total = a.qo_indptr[req_i + 1] - q_start;
+    const int row0 = a.q_tile_to_index[tile] * 64 + (int)(item % SUBS) * QB, row = row0 + wave / NREP * 32 + (lane & 31);
+    const int64_t req = a.req_pool_indices[req_i];
+    const int kv_len = req >= 0 && req < a.num_requests ? (int)min((int64_t)(a.kv_indptr[req_i + 1] - a.kv_indptr[req_i]), a.rtt_stride) : 0;
+    const int last = min(row0 + QB, rows_total) - 1;
+    const int kmax = a.causal ? min(kv_len - rows_total + last, kv_len - 1) : kv_len - 1;
+    const int blocks = max(kmax, 0) / kKB + 1, per = part_blocks(a, blocks), parts = (blocks + per - 1) / per;
+    if (row >= rows_total || parts == 1) return;  // (the one part wrote the output)
+    float m = kNegBig;
+#pragma unroll
+    for (int j = 0; j < kMaxParts; ++j)
+        if (j < parts) m = fmaxf(m, pm[j]);
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    float l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kMaxParts; ++j)
+        if (j < parts) {
+            const float f = __builtin_amdgcn_exp2f(pm[j] - m);
+            l += pl[j] * f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += x[j][i] * f;
+        }
+    const float inv = l != 0.0f ? 1.0f / l : 0.0f;  // a row with no visible key yields zeros
+    const int dim = 8 * g + 4 * h;
+    uint16_t* const out = static_cast<uint16_t*>(a.out) + ((int64_t)(q_start + row) * a.n_heads + hk * NREP + wave % NREP) * D + dim;
+    *reinterpret_cast<u32x2*>(out) = u32x2{pack_bf16x2(v[0] * inv, v[1] * inv), pack_bf16x2(v[2] * inv, v[3] * inv)};
+}
+
 template <int D, int NREP, int QSUB, bool SPLIT>
 bool launch_shape(const AttnPrefillArgs& a, hipStream_t stream) {
     // tokens per workgroup: a schedule tile has 64 rows, and the kernel reads the positions of 64
@@ -714,13 +832,18 @@ bool launch_shape(const AttnPrefillArgs& a, hipStream_t stream) {
     const int rows = 32 * (narrow ? QP : QSUB);
     const int64_t wgs = paged ? (int64_t)a.num_q_tiles * (64 / rows) * a.n_kv_heads
                               : (int64_t)((a.seq + rows - 1) / rows) * a.batch * a.n_kv_heads;
-    if (wgs > INT_MAX) return false;
+    if (wgs * std::max(a.nsplit, 1) > INT_MAX) return false;
     const dim3 grid((unsigned)wgs), block(64 * NREP * (narrow ? QP : QSUB));
     if (paged && a.mask) {
         if constexpr (!SPLIT)
             attn_prefill_kernel<D, NREP, QP, true, true, SPLIT><<<grid, block, 0, stream>>>(a);
         else
             return false;
+    } else if (paged && a.nsplit > 1) {
+        const int64_t waves = wgs * NREP * QP, merges = (waves * (D / 8) + 3) / 4;
+        if (merges > INT_MAX) return false;
+        attn_prefill_kernel<D, NREP, QP, true, false, SPLIT, true><<<dim3((unsigned)(wgs * a.nsplit)), block, 0, stream>>>(a);
+        merge_parts_kernel<D, NREP, QP><<<dim3((unsigned)merges), dim3(256), 0, stream>>>(a, waves);
     } else if (paged) {
         attn_prefill_kernel<D, NREP, QP, true, false, SPLIT><<<grid, block, 0, stream>>>(a);
     } else if (narrow) {
@@ -749,7 +872,16 @@ bool attn_prefill_pool_ok(int64_t num_slots, int n_kv_heads, int head_dim) {
     return num_slots <= (int64_t)kMissing / (2 * (int64_t)n_kv_heads * head_dim);
 }
 
+int attn_prefill_parts(int64_t tiles, int n_heads, int64_t max_keys, int nsplit) {
+    const int64_t pairs = tiles * n_heads;
+    if (nsplit <= 1 || pairs >= kMaxPartPairs) return 1;
+    const int blocks = (int)((max_keys + kKB - 1) / kKB), n = part_count(blocks, pairs, std::min(nsplit, kMaxParts));
+    const int64_t cost = 2 * n * pairs / kPairsPerBlock + kMergeBlocks;
+    return blocks - (blocks + n - 1) / n >= cost ? n : 1;
+}
+
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream) {
+    if (a.nsplit > 1 && (a.nsplit > kMaxParts || !a.ws || a.mask || !a.req_to_token)) return false;
     const bool split = attn_prefill_split_supported(a.n_heads, a.n_kv_heads, a.head_dim);
     if (!split && !attn_prefill_supported(a.n_heads, a.n_kv_heads, a.head_dim)) return false;
     const bool paged = a.req_to_token != nullptr;

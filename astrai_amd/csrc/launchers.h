@@ -225,12 +225,18 @@ struct AttnPrefillArgs {
     const uint8_t* mask;
     int64_t mask_b_stride, mask_h_stride, mask_l_stride;
     int mask_rows, mask_width;
+    // paged mode without a mask, optional: the keys of a block of queries in up to nsplit parts, each of them a
+    // workgroup's; ws: as many floats as attn_rows_workspace_floats(...) asks for
+    float* ws;
+    int nsplit;
 };
 bool attn_prefill_supported(int n_heads, int n_kv_heads, int head_dim);
 // the shapes it takes in place of attn_rows.hip (probabilities as two bf16 terms, no mask tensor)
 bool attn_prefill_split_supported(int n_heads, int n_kv_heads, int head_dim);
 // pools whose rows its 32-bit offsets reach (under 4 GiB)
 bool attn_prefill_pool_ok(int64_t num_slots, int n_kv_heads, int head_dim);
+// paged: how many parts to launch for contexts of up to max_keys keys, at most nsplit (1: none)
+int attn_prefill_parts(int64_t tiles, int n_heads, int64_t max_keys, int nsplit);
 bool launch_attn_prefill(const AttnPrefillArgs& a, hipStream_t stream);
 
 // attn_rows.hip: paged attention for every head_dim in {32, 64, 128, 256} and every

@@ -1285,7 +1285,7 @@ def _paged_rows(lib, q, k_pool, v_pool, rtt, rpi, kv_indptr, schedule, m_args, o
 
 
 def _rows_nsplit(tiles: int, n_kv_heads: int) -> int:
-    """Context splits of the general paged kernel over a schedule of ``tiles``."""
+    """Context splits of a schedule of ``tiles``, at most: the block kernel makes as many parts as a context is worth."""
     return max(1, min(16, 2048 // max(1, tiles * 4 * n_kv_heads)))   # at least: one wave per row block, 4+ blocks per tile
 
 
@@ -1306,8 +1306,8 @@ def attn_paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
     bool, True = attend, ``[batch, kv]`` or ``[batch, 1 | H, rows, kv]`` with ``rows`` counted
     inside each sequence (entry_utils.cuh:326-346); rows and positions the mask does not hold
     are not attended. Returns ``[total_q, H, head_dim]`` bf16. head_dim 128 with a grouping of
-    2, 4 or 8 runs the MFMA block kernel; other shapes the general kernel, whose context split
-    ``nsplit`` (0: chosen here) only matters for short schedules."""
+    2, 4 or 8 runs the MFMA block kernel; other shapes that kernel or the general one, whose context split
+    ``nsplit`` (0: chosen here; the block kernel makes fewer parts of short keys) only matters for short schedules."""
     lib = _require()
     if mask is None and q.dim() == k_cache.dim() == 3 and k_cache.size(1):
         h, hkv, d = q.size(1), k_cache.size(1), q.size(2)
@@ -1882,8 +1882,8 @@ def _strided_view(t, layout):
     return t, (s[0], s[1], s[2]) if layout == BHLD else (s[0], s[2], s[1])
 
 
-# (tile of 64 query rows, query head) pairs from which the block kernel serves the shapes that the general
-# kernel with its context split serves otherwise (kPrefillMinRowBlocks in csrc/abi.hip, with the figures)
+# (tile of 64 query rows, query head) pairs from which the block kernel fills the chip without a context split
+# (kMaxPartPairs in csrc/attn_prefill.hip, with the figures)
 PREFILL_MIN_ROW_BLOCKS = 256
 
 

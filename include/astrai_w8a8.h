@@ -491,7 +491,7 @@ int astrai_w8a8_attn_paged_prefill_masked_bf16(
  * split): bf16 MFMAs for the scores and for P.V (P as a bf16 head plus a bf16 remainder), fp32
  * softmax statistics and accumulation, one rounding of the output. Correct for every shape;
  * prefill without a mask at head_dim 64, or 128 with n_heads == n_kv_heads, runs the block kernel
- * of attn_prefill_bf16 with P in two terms where there are enough tiles for it.
+ * of attn_prefill_bf16 with P in two terms, short schedules with the keys in up to nsplit parts.
  *   nsplit     in [1, 64]: 1 = every wave owns a whole context and writes the output itself,
  *              no workspace (NULL allowed); > 1 = partial results in the workspace and a
  *              merge kernel
