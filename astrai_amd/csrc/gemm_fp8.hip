@@ -2,11 +2,12 @@
 // e4m3 / fp32 output) or one scale per activation row and per weight row (bf16 output).
 // Large shapes run 256x256 tiles: the four-wave 128x128-register-tile kernel for bf16
 // output (v_mfma_f32_16x16x128_f8f6f4), the eight-wave ping-pong kernel (32x32x64) for the other outputs; bf16 shapes with too few of
-// those tiles for the chip run 128x128 tiles of that instruction; the generic
+// those tiles for the chip run 128x256, 128x128 or 64x64 tiles of that instruction; the generic
 // tiled kernel takes everything else.
 #include "gemm_wave128_q16.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
+#include "gemm_wide256.cuh"
 #include "gemm_tile.cuh"
 
 namespace w8a8 {
@@ -24,6 +25,7 @@ void launch_big(const GemmArgs& g, hipStream_t stream) {
 }
 template <int Fmt, int ScaleKind>
 void launch_for(const GemmArgs& g, hipStream_t stream) {
+    if (wide256_shape_ok(g)) return launch_wide256<Op32F8<Fmt>, ScaleKind>(g, stream);
 #ifndef W8A8_NO_WAVE128
     if (wave128_takes(g)) {
         GemmArgs head, tail;
@@ -34,7 +36,8 @@ void launch_for(const GemmArgs& g, hipStream_t stream) {
         }
         if (const int r = tile_tail_rows(g)) {
             split_rows(g, r, ScaleKind == SCALE_ROWCOL, head, tail);
-            if (mid128_shape_ok(tail)) launch_mid128<Op32F8<Fmt>, ScaleKind>(tail, stream);
+            if (wide256_shape_ok(tail)) launch_wide256<Op32F8<Fmt>, ScaleKind>(tail, stream);
+            else if (mid128_shape_ok(tail)) launch_mid128<Op32F8<Fmt>, ScaleKind>(tail, stream);
             else launch_small64<Op32F8<Fmt>, ScaleKind>(tail, stream);
             return launch_big<Fmt, ScaleKind>(head, stream);
         }

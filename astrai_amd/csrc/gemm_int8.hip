@@ -1,17 +1,22 @@
 // int8 x int8 -> int32 MFMA GEMMs, per-token x per-channel dequant epilogue.
 // Large shapes run on 256x256 tiles: the four-wave
 // 128x128-register-tile kernel (v_mfma_i32_16x16x64_i8) for bf16 output, the eight-wave ping-pong kernel (32x32x32)
-// for int32 output; shapes with too few of those tiles for the chip run 128x128
+// for int32 output; shapes with too few of those tiles for the chip run 128x256, 128x128 or 64x64
 // tiles of the latter instruction; the generic tiled kernel takes everything else.
 #include "gemm_wave128_i8.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
+#include "gemm_wide256.cuh"
 #include "gemm_tile.cuh"
 
 namespace w8a8 {
 
 bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_decode_kernel) {
     if (!tiled_shape_ok(g)) return false;
+    if (wide256_shape_ok(g)) {
+        launch_wide256<Op32I8, SCALE_ROWCOL>(g, stream);
+        return true;
+    }
 #ifndef W8A8_NO_WAVE128
     if (wave128_takes(g)) {
         GemmArgs head, tail;
@@ -24,7 +29,8 @@ bool launch_gemm_int8_tiled(const GemmArgs& g, hipStream_t stream, bool tail_on_
         }
         if (const int r = tile_tail_rows(g)) {
             split_rows(g, r, true, head, tail);
-            if (mid128_shape_ok(tail)) launch_mid128<Op32I8, SCALE_ROWCOL>(tail, stream);
+            if (wide256_shape_ok(tail)) launch_wide256<Op32I8, SCALE_ROWCOL>(tail, stream);
+            else if (mid128_shape_ok(tail)) launch_mid128<Op32I8, SCALE_ROWCOL>(tail, stream);
             else launch_small64<Op32I8, SCALE_ROWCOL>(tail, stream);
             launch_wave128_i8<>(head, stream);
             return true;

@@ -24,6 +24,7 @@ struct Mid128Cfg {
     static constexpr int MI = 2, NI = 1;                 // 32-row sub-tiles per wave: 64 m x 32 n
     static constexpr int OPERAND_BYTES = 128 * BK;       // one operand's slab: 16 KiB
     static constexpr int STAGE_BYTES = 2 * OPERAND_BYTES;
+    static_assert(TileOut<BM, BN, THREADS>::BYTES <= 2 * STAGE_BYTES, "outputs fit the stages");
 };
 
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it. An instance of its own: chosen
@@ -326,47 +327,33 @@ __global__ __launch_bounds__(Mid128Cfg::THREADS, S == 2 ? 4 : 2) void gemm_mid12
         }
     }
 
-    // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad): 8-byte stores
+    // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad)
     if (g.out_kind != OUT_BF16) return;   // (the launcher sends other outputs elsewhere)
-    uint16_t* const out = static_cast<uint16_t*>(g.out);
-    const bool vec_ok = (g.n & 3) == 0;
+    TileOut<Cfg::BM, Cfg::BN, Cfg::THREADS>::store(g, lds, m0, n0, [&](auto put) __attribute__((always_inline)) {
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
-        const int m = mw + mi * 32 + lrow;
-        if (m >= g.m) continue;
+        for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
+            for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = nw + ni * 32 + q * 8 + lgrp * 4;
-                if (n >= g.n) continue;
-                float v[4];
+                for (int q = 0; q < 4; ++q) {
+                    const int c = wave_n * 32 + ni * 32 + q * 8 + lgrp * 4;
+                    float v[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float f = (float)acc[ni][mi][4 * q + j];
-                    if constexpr (ScaleKind == SCALE_BLOCK128) {
-                        v[j] = f + ((bias && n + j < g.n) ? bf16_to_f32(bias[n + j]) : 0.0f);
-                    } else if constexpr (ScaleKind == SCALE_TENSOR) {
-                        v[j] = RoundFirst ? add_bias(f * s_tensor, b4[ni][q][j], true) : f * s_tensor + b4[ni][q][j];
-                    } else {
+                    for (int j = 0; j < 4; ++j) {
+                        const float f = (float)acc[ni][mi][4 * q + j];
+                        if constexpr (ScaleKind == SCALE_BLOCK128) {
+                            v[j] = f + ((bias && n0 + c + j < g.n) ? bf16_to_f32(bias[n0 + c + j]) : 0.0f);
+                        } else if constexpr (ScaleKind == SCALE_TENSOR) {
+                            v[j] = RoundFirst ? add_bias(f * s_tensor, b4[ni][q][j], true) : f * s_tensor + b4[ni][q][j];
+                        } else {
 #pragma clang fp contract(off)
-                        const float scaled = f * sx[mi] * sw4[ni][q][j];
-                        v[j] = scaled + b4[ni][q][j];
+                            const float scaled = f * sx[mi] * sw4[ni][q][j];
+                            v[j] = scaled + b4[ni][q][j];
+                        }
                     }
+                    put(wave_m * 64 + mi * 32 + lrow, c, v);
                 }
-                const size_t o = (size_t)m * g.n + n;
-                if (vec_ok) {
-                    u32x2 pk;
-                    pk.x = pack_bf16x2(v[0], v[1]);
-                    pk.y = pack_bf16x2(v[2], v[3]);
-                    *reinterpret_cast<u32x2*>(out + o) = pk;
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (n + j < g.n) out[o + j] = f32_to_bf16(v[j]);
-                }
-            }
-    }
+    });
 }
 
 // bf16 output, K in whole slabs, and a shape this tile size suits: at least 140 tiles of 128 x 128
