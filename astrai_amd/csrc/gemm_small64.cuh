@@ -35,14 +35,22 @@ struct Small64Cfg {
 
 // RoundFirst (per-tensor scales): the product is rounded to bf16 before the bias joins it (see gemm_mid128.cuh; 200 x 2048
 // x 2048 6.2 us, with the choice in the epilogue 6.3)
-template <class Op, int ScaleKind, int S, bool RoundFirst>
-__global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm_small64_kernel(GemmArgs g) {
+// G: groups of four waves. 2: where each tile has a compute unit to itself, two groups form the tile over half of K each, with
+// rings of their own, and add their sums at the end; the one covers the other's waits, and a barrier publishes two slabs. us, one
+// group -> two, int8 / fp8: 200 x 4096 x 11008 27.3 / 26.6 -> 23.6 / 22.6, 193 x 2048 x 5632 13.9 / 12.9 -> 11.9 / 11.2, 256 x 4096 x
+// 4096 12.6 / 11.5 -> 11.2 / 10.7, 300 x 2048 x 2048 8.4 / 7.8 -> 7.6 / 7.3, 200 x 2048 x 256 5.7 / 5.2 -> 5.5 / 5.15. 128-block scales
+// gain from 40 slabs on, where their longer prologue is made up for: 374 x 1536 x 7168 17.4 -> 15.5, 70 x 2048 x 7168 14.5 -> 13.2, 145 x
+// 4096 x 4096 10.3 -> 10.0, 250 x 4096 x 4096 10.7 -> 10.8, 100 x 7168 x 2048 7.1 -> 7.3. (Four waves of the whole tile over a
+// quarter of K each, with no barrier and every slab read once: the same with long K, 0.6 to 1.4 us slower with up to 16 slabs.)
+template <class Op, int ScaleKind, int S, bool RoundFirst, int G>
+__global__ __launch_bounds__(256 * G, G == 2 || ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm_small64_kernel(GemmArgs g) {
     using Cfg = Small64Cfg<S>;
     using Acc = typename Op::Acc;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int wave_m = wave & 1, wave_n = wave >> 1;   // 2 x 2 waves
     const int lrow = lane & 31, lgrp = lane >> 5;
 
@@ -52,6 +60,10 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
     const int m0 = tc.tm * Cfg::BM, n0 = tc.tn * Cfg::BN;
     const int K = g.k;
     const int ksteps = K >> 7;
+    // the group's slabs: `count` of them from `first` on, those from `end` on zeros
+    const int count = (ksteps + G - 1) / G, first = group * count, end = min(first + count, ksteps);
+    constexpr int QUADS = 4 / G;              // of a wave's accumulators, that it finishes: from quad0 on
+    const int quad0 = group * QUADS;
 
     // epilogue operands, requested now
     const EpilogueScalars es = load_epilogue_scalars<ScaleKind>(g);
@@ -62,13 +74,13 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
         const int m = mw + lrow;
         sx = (m < g.m) ? g.sa[m] : 0.0f;
     }
-    f32x4 sw4[4], b4[4];
+    f32x4 sw4[QUADS], b4[QUADS];
     const uint16_t* bias = static_cast<const uint16_t*>(g.bias);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < QUADS; ++q)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int n = nw + q * 8 + lgrp * 4 + j;
+            const int n = nw + (quad0 + q) * 8 + lgrp * 4 + j;
             sw4[q][j] = 1.0f;
             b4[q][j] = 0.0f;
             if (n < g.n) {
@@ -94,9 +106,10 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
         w_off[1] = wr + (uint32_t)(c0 ^ 1) * 16;
     }
     const uint32_t row8 = 8u * (uint32_t)K;
-    uint8_t* const dma_base = lds + wave * (16 * 128);
+    uint8_t* const ring = lds + group * Cfg::LDS_BYTES;
+    uint8_t* const dma_base = ring + wave * (16 * 128);
     auto issue = [&](int stage, int slab) __attribute__((always_inline)) {
-        const bool live = slab < ksteps;
+        const bool live = slab < end;
         const __amdgpu_buffer_rsrc_t rx = make_rsrc(g.a, live ? x_bytes : 0u);
         const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.b, live ? w_bytes : 0u);
         const uint32_t k0 = (uint32_t)slab << 7;
@@ -118,7 +131,7 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
     const int x_rd = (wave_m * 32) * 128;
     const int w_rd = Cfg::OPERAND_BYTES + (wave_n * 32) * 128;
     auto read = [&](int stage, u32x4 (&xf)[4], u32x4 (&wf)[4]) __attribute__((always_inline)) {
-        const uint8_t* const base = lds + stage * Cfg::STAGE_BYTES;
+        const uint8_t* const base = ring + stage * Cfg::STAGE_BYTES;
 #pragma unroll
         for (int j = 0; j < 4; ++j) wf[j] = *reinterpret_cast<const u32x4*>(base + w_rd + frag_off[j]);
 #pragma unroll
@@ -156,10 +169,10 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
     }
 
     // ---- prologue: slabs 0 .. S-2 in flight; slab 0 visible and in the first register set
-    request_steps(0, steps);
+    request_steps(first, steps);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int s = 0; s < S - 1; ++s) issue(s, s);
+    for (int s = 0; s < S - 1; ++s) issue(s, first + s);
     wait_vmcnt<4 * (S - 2)>();
     phase_barrier();
     read(0, xa, wa);
@@ -194,7 +207,7 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
                 for (int j = 16 / Op::STEPS * q; j < 16 / Op::STEPS * (q + 1); ++j) acc[j] += before[j] * behind;
                 __builtin_amdgcn_sched_barrier(0);
             }
-            behind = __uint_as_float(steps[0][AT]) * __uint_as_float(steps[1][AT]);
+            behind = G == 1 || k < end ? __uint_as_float(steps[0][AT]) * __uint_as_float(steps[1][AT]) : 0.0f;
         } else {
 #pragma unroll
             for (int q = 0; q < Op::STEPS; ++q) acc = Op::mma_step(q, wc, xc, acc);
@@ -203,12 +216,12 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
         wr_stage = (wr_stage == S - 1) ? 0 : wr_stage + 1;
     };
     constexpr std::integral_constant<int, 0> at0{};
+    int k = first;
     if constexpr (STEPS > 0) {
         constexpr std::integral_constant<int, 1> at1{};
         constexpr std::integral_constant<int, 2> at2{};
         constexpr std::integral_constant<int, 3> at3{};
-        int k = 0;
-        for (; k + 3 < ksteps; k += 4) {
+        for (; k + 3 < first + count; k += 4) {
             step(at0, std::true_type{}, k, xa, wa, xb, wb, pa, pb);
             step(at1, std::true_type{}, k + 1, xb, wb, xa, wa, pb, pa);
             step(at2, std::true_type{}, k + 2, xa, wa, xb, wb, pa, pb);
@@ -216,22 +229,48 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
             steps[0] = steps_next[0];
             steps[1] = steps_next[1];
         }
-        if (k < ksteps) step(at0, std::false_type{}, k, xa, wa, xb, wb, pa, pb);
-        if (k + 1 < ksteps) step(at1, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
-        if (k + 2 < ksteps) step(at2, std::false_type{}, k + 2, xa, wa, xb, wb, pa, pb);
+        if (k < first + count) step(at0, std::false_type{}, k, xa, wa, xb, wb, pa, pb);
+        if (k + 1 < first + count) step(at1, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
+        if (k + 2 < first + count) step(at2, std::false_type{}, k + 2, xa, wa, xb, wb, pa, pb);
     } else {
-        for (int k = 0; k < ksteps; k += 2) {
+        for (; k < first + count; k += 2) {
             step(at0, std::false_type{}, k, xa, wa, xb, wb, pa, pb);
-            if (k + 1 < ksteps) step(at0, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
+            if (k + 1 < first + count) step(at0, std::false_type{}, k + 1, xb, wb, xa, wa, pb, pa);
         }
     }
     if constexpr (STEPS > 0) {
-        const Acc& last = (ksteps & 1) ? pa : pb;
+        const Acc& last = (count & 1) ? pa : pb;
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[j] += last[j] * behind;
     }
     // no load outlives the kernel's use of LDS: the remaining ones ran on empty descriptors or are waited for here
     wait_vmcnt<0>();
+
+    // ---- two groups: each finishes half of the quads, with the other's sums of them
+    [[maybe_unused]] typename Op::AccScalar half[8];
+    if constexpr (G == 2) {
+        typedef typename Op::AccScalar Four __attribute__((ext_vector_type(4)));
+        wait_lgkmcnt0();
+        phase_barrier();   // the rings are free: every wave's reads of them, and loads into them, are behind it
+        uint8_t* const there = lds + wave * 2048 + lane * 16;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            Four give;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                give[j] = group ? acc[4 * i + j] : acc[8 + 4 * i + j];
+                half[4 * i + j] = group ? acc[8 + 4 * i + j] : acc[4 * i + j];
+            }
+            *reinterpret_cast<Four*>(there + (1 - group) * 8192 + i * 1024) = give;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const Four got = *reinterpret_cast<const Four*>(there + group * 8192 + i * 1024);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) half[4 * i + j] += got[j];
+        }
+    }
 
     // ---- epilogue: a lane holds four consecutive n of one m per quad: 8-byte stores
     uint16_t* const out = static_cast<uint16_t*>(g.out);
@@ -239,13 +278,13 @@ __global__ __launch_bounds__(256, ScaleKind == SCALE_BLOCK128 ? 2 : 1) void gemm
     const int m = mw + lrow;
     if (m >= g.m) return;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int n = nw + q * 8 + lgrp * 4;
+    for (int q = 0; q < QUADS; ++q) {
+        const int n = nw + (quad0 + q) * 8 + lgrp * 4;
         if (n >= g.n) continue;
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float f = (float)acc[4 * q + j];
+            const float f = G == 2 ? (float)half[4 * q + j] : (float)acc[4 * q + j];
             if constexpr (ScaleKind == SCALE_BLOCK128) {
                 v[j] = f + ((bias && n + j < g.n) ? bf16_to_f32(bias[n + j]) : 0.0f);
             } else if constexpr (ScaleKind == SCALE_TENSOR) {
@@ -281,17 +320,20 @@ inline bool small64_shape_ok(const GemmArgs& g) {
 // kernel is the 16 KiB a 64 x 64 tile pulls out of L2 per slab, not latency.
 constexpr int kSmall64Stages = 4;
 
-template <class Op, int ScaleKind, bool RoundFirst = false>
+template <class Op, int ScaleKind, bool RoundFirst = false, int G = 1>
 inline void launch_small64(const GemmArgs& g, hipStream_t stream) {
     using Cfg = Small64Cfg<kSmall64Stages>;
     if constexpr (!RoundFirst && ScaleKind == SCALE_TENSOR)
         if (g.round_first) return launch_small64<Op, ScaleKind, true>(g, stream);
     const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64);
-    auto kern = gemm_small64_kernel<Op, ScaleKind, kSmall64Stages, RoundFirst>;
+    if constexpr (G == 1)
+        if (tiles <= 256 && (ScaleKind != SCALE_BLOCK128 || g.k >= 40 * 128))
+            return launch_small64<Op, ScaleKind, RoundFirst, 2>(g, stream);
+    auto kern = gemm_small64_kernel<Op, ScaleKind, kSmall64Stages, RoundFirst, G>;
     static std::atomic<uint64_t> lds_allowed{0};
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), G * Cfg::LDS_BYTES, lds_allowed);
     note_kernel("small64");
-    kern<<<dim3((unsigned)tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(g);
+    kern<<<dim3((unsigned)tiles), dim3(G * Cfg::THREADS), G * Cfg::LDS_BYTES, stream>>>(g);
 }
 
 }  // namespace w8a8

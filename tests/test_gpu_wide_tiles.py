@@ -1,4 +1,4 @@
-"""8-bit products on tiles of 128 x 256 and of 128 x 128: every remainder of rows, columns and slabs, and columns whose rows of
+"""8-bit products on tiles of 128 x 256, of 128 x 128 and, one to a compute unit, of 64 x 64: every remainder of rows, columns and slabs, and columns whose rows of
 outputs are whole 16-byte pieces, whole 8-byte pieces or neither."""
 
 import pytest
@@ -12,7 +12,9 @@ DEV = "cuda"
 # rows, columns, K, kernel: 1 to 7 slabs (three stages, two slabs a turn); one row or column past a tile, one short of it
 CASES = [(2049, 2049, 128, "mid128x256"), (2047, 2302, 256, "mid128x256"), (2100, 2060, 384, "mid128x256"), (1281, 3080, 512, "mid128x256"),
          (4090, 1100, 640, "mid128x256"), (300, 11264, 768, "mid128x256"), (129, 16640, 896, "mid128x256"), (16512, 256, 640, "mid128x256"),
-         (1500, 1501, 128, "mid128"), (1530, 1500, 640, "mid128"), (1409, 1544, 768, "mid128"), (1537, 1410, 384, "mid128")]
+         (1500, 1501, 128, "mid128"), (1530, 1500, 640, "mid128"), (1409, 1544, 768, "mid128"), (1537, 1410, 384, "mid128")] + [
+    # halves of K: odd and even counts of slabs, one, and fewer than the ring's stages
+    (130 + 9 * i, 1021 + i, 128 * i, "small64") for i in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17)]
 
 
 @pytest.mark.parametrize("m,n,k,kernel", CASES)
@@ -49,3 +51,25 @@ def test_fp8(m, n, k, kernel, fmt):
     out = _cabi.mm_fp8(a, b, sa, sb, 0, None, bias)
     exact = acc * sa[:, None].double() * sb.double() + bias.double()
     assert_bf16_close(out, exact.to(torch.bfloat16), what="a step per row and column")
+
+
+@pytest.mark.parametrize("slabs", [40, 41, 42, 43, 45, 46])
+def test_block128_in_two_halves(slabs):
+    """Steps spread over seven octaves; a row's step that is not a number stays in its row, also where the second half of the row
+    ahead of it is a slab short."""
+    from astrai_amd.extension import _cabi
+    from oracle import w8a8_oracle as O
+    m, n, k = 70 + slabs, 200, 128 * slabs
+    print(f"case m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(slabs)
+    a, b = (torch.randn(i, k, generator=g).to(torch.float8_e4m3fn) for i in (m, n))
+    sa = 2.0 ** (torch.rand(m, slabs, generator=g) * 7 - 5)
+    sb = 2.0 ** (torch.rand((n + 127) // 128, slabs, generator=g) * 7 - 5)
+    want = O.fp8_gemm_blockscaled(a, b, sa, sb)
+    out = _cabi.mm_fp8_block128(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV))
+    assert _cabi.last_kernel() == "small64"
+    assert_bf16_close(out, want, what=f"{slabs} slabs")
+    sa[5, 0], sb[1, 0] = float("nan"), float("inf")
+    out = _cabi.mm_fp8_block128(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV)).cpu()
+    assert out[5].isnan().all() and torch.isfinite(out[torch.arange(m) != 5, :128]).all()
+    assert not torch.isfinite(out[:, 128:]).any()
