@@ -163,12 +163,14 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
         constexpr int SUBS = 64 / QB;  // workgroups that share a tile
         const int idx = (int)(gridDim.x - 1 - blockIdx.x);
         hk = idx % a.n_kv_heads;
-        int item = idx / a.n_kv_heads;
+        int sub = (idx / a.n_kv_heads) % SUBS, tile = idx / (SUBS * a.n_kv_heads);
+        [[maybe_unused]] int item = 0;
         if constexpr (PARTS) {
+            item = idx / a.n_kv_heads;
             part = item % a.nsplit;
             item /= a.nsplit;
+            sub = item % SUBS, tile = item / SUBS;
         }
-        const int sub = item % SUBS, tile = item / SUBS;
         const int req_i = a.q_tile_to_batch[tile];
         seq_index = req_i;
         const int q_start = a.qo_indptr[req_i];
@@ -194,7 +196,7 @@ __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && 
             table += key0;
             pq = min(pq - key0, per * kKB - 1);
             kmax = min(kmax - key0, per * kKB - 1);
-part_ws = a.ws + ((((int64_t)item * a.n_kv_heads + hk) * WAVES + wave) * a.nsplit + part) * part_floats(D);
+            part_ws = a.ws + ((((int64_t)item * a.n_kv_heads + hk) * WAVES + wave) * a.nsplit + part) * part_floats(D);
         }
     } else {
         const int nqb = (a.seq + QB - 1) / QB;
