@@ -187,10 +187,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 32 
     const int nq = n_rep * rows;  // <= kNQ
     int64_t item = (int64_t)blockIdx.x * 4 + wave;
     if (item >= a.num_items) return;
-    const int split = (int)(item % a.nsplit);
-    item /= a.nsplit;
-    const int hk = (int)(item % a.n_kv_heads);
-    const int block = (int)(item / a.n_kv_heads);
+    // Which wave has what, for steps whose splits can be 120 keys and more: neighbours have the KV heads of one range of keys, and
+    // so fetch neighbouring pieces of the same pool rows (128 bytes a head of 64) at about the same time; with a head's splits side
+    // by side the pieces of a row came up all over the launch (16/16 heads x 64, 40 x 3000 keys 115 us, 2.9 TB/s, and 90, 3.7; 16/4
+    // x 32, 32 x 3000 20.8 and 19.0; 32/8 x 64, 20 x 6000 50.7 and 49.8). Shorter ranges gain nothing (7 x 3000 in 46 splits 16.5, 16.8).
+    const bool heads_first = !a.qo_indptr && a.rtt_stride >= 120 * (int64_t)a.nsplit;
+    const int inner = heads_first ? a.n_kv_heads : a.nsplit, outer = heads_first ? a.nsplit : a.n_kv_heads;
+    int of_inner, of_outer, block;
+    if (a.num_items <= UINT32_MAX) {
+        const uint32_t i = (uint32_t)item, rest = i / (uint32_t)inner;
+        of_inner = (int)(i - rest * (uint32_t)inner), block = (int)(rest / (uint32_t)outer), of_outer = (int)(rest - (uint32_t)block * (uint32_t)outer);
+    } else {
+        of_inner = (int)(item % inner);
+        item /= inner;
+        of_outer = (int)(item % outer), block = (int)(item / outer);
+    }
+    const int hk = heads_first ? of_inner : of_outer, split = heads_first ? of_outer : of_inner;
     const RowBlock rb = row_block(a, block);
     if (rb.r0 >= rb.q_len) return;  // the schedule's tile reaches past the sequence: nothing reads this block
 

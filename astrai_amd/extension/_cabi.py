@@ -1070,8 +1070,12 @@ def _decode_is_general(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
 def _rows_decode_nsplit(pairs: int, max_keys: int) -> int:
     """Context splits of the general kernel's step, one wave per (sequence, kv head, split): three to a SIMD (two, three, 32 /
     8 heads x 64: 32 x 3000 keys 35.0 us, 31.2; 128 x 1000 43.5, 38.0; 16 / 16 heads x 64, 64 x 1500: 62, 54.7; fewer
-    pairs the same)."""
-    return max(1, min(64, 3072 // max(1, pairs), max_keys // 64))
+    pairs the same). Where that is one split, two from 480 keys on: of a ragged batch's waves the longest are left alone (16 / 16
+    heads x 64, one split and two: 100 x 600 58.5, 46.7; 100 x 1300 121, 89; 128 x 500 50.7, 50.0; 128 x 300 32.1, 33.1)."""
+    splits = 3072 // max(1, pairs)
+    if splits == 1 and max_keys >= 480:
+        splits = 2
+    return max(1, min(64, splits, max_keys // 64))
 
 
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,

@@ -1,0 +1,36 @@
+"""Paged steps of the general kernel, whose waves take KV heads side by side where a split's share of the slot table is 120
+positions or more and splits side by side otherwise: both sides of that line, KV heads that fill no whole workgroup."""
+
+import pytest
+import torch
+
+from oracle import decoder_oracle as D
+from tests.helpers import assert_bf16_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("h,hkv,d", [(6, 3, 64), (5, 5, 32), (16, 16, 64), (7, 1, 256)])
+@pytest.mark.parametrize("width,nsplit", [(119, 1), (120, 1), (720, 2), (720, 5), (720, 6), (719, 6), (720, 7), (7680, 64), (7679, 64)])
+def test_either_order(h, hkv, d, width, nsplit):
+    from astrai_amd.extension import _cabi
+    print(f"case h={h} hkv={hkv} d={d} width={width} nsplit={nsplit}", flush=True)
+    g = torch.Generator().manual_seed(width + nsplit + h)
+    lens = [min(width, n) for n in (width, 1, 117, 0, 720)]
+    pool = sum(lens) + 3
+    q, k, v = (torch.randn(n, heads, d, generator=g).to(torch.bfloat16) for n, heads in ((len(lens), h), (pool, hkv), (pool, hkv)))
+    slots, table, at = torch.randperm(pool, generator=g).int(), torch.full((len(lens), width), -1, dtype=torch.int32), 0
+    for i, n in enumerate(lens):
+        table[i, :n] = slots[at:at + n]
+        at += n
+    rows = torch.arange(len(lens), dtype=torch.int32)
+    indptr = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    args = (q, k, v, table, rows, indptr)
+    got = _cabi.attn_paged_decode(*(t.to(DEV) for t in args), nsplit=nsplit)
+    assert_bf16_close(got, D.attn_paged_decode(*args), what=f"{nsplit} splits of {width}")
+
+
+def test_two_splits_of_many_pairs():
+    from astrai_amd.extension import _cabi
+    assert [_cabi._rows_decode_nsplit(p, w) for p, w in ((1536, 479), (1537, 479), (1537, 480), (3072, 8192), (3073, 8192))] == [2, 1, 2, 2, 1]
