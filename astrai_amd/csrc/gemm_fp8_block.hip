@@ -7,6 +7,7 @@
 #include "gemm_wave128.cuh"
 #include "gemm_mid128.cuh"
 #include "gemm_small64.cuh"
+#include "gemm_wide256.cuh"
 #include "gemm_tile.cuh"
 
 namespace w8a8 {
@@ -22,6 +23,12 @@ bool large_tiles_take(const GemmArgs& g) {
     return pingpong_shape_ok(g) || (g.k >= 256 && (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 256);
 }
 
+// Tiles of 128 x 256 where those are one round of the chip and 128 x 128 tiles more than one, ahead of the large tiles, which leave
+// half of the chip idle there (us, 256 x 256 / 128 x 256: 2100 x 2048 x 7168 73 / 59, 4000 x 2048 x 7168 77 / 72, 1100 x 4096 x 4096 46 /
+// 37.5, 2000 x 4096 x 4096 49 / 46, 700 x 7168 x 2048 25.6 / 23.4, 2100 x 2048 x 1024 16.5 / 15.7; with fewer slabs their start and
+// end are the longer ones: 2000 x 4096 x 640 14.2 / 15.3, 1100 x 4096 x 512 12.0 / 12.1).
+bool wide_tiles_take(const GemmArgs& g) { return g.k >= 1024 && wide256_shape_ok(g); }
+
 // Tails on smaller tiles as in tile_tail_rows (one launch / two; tiles of the tail): 4300 x 4096 x 4096 102 / 79 us (64), x 256
 // 19.8 / 17.5; 4500 x 4096 x 4096 101 / 86 (128); 4700 101 / 98 (192), x 256 19.6 / 19.9; 5000 x 4096 x 256 (256) 19.9 / 21.8, x
 // 1024 36.3 / 37.1, x 1536 46.1 / 46.1, x 4096 101 / 100, x 11008 249 / 233: more than 192 only with K from 1536 on.
@@ -31,6 +38,10 @@ int64_t block_tail_tiles(const GemmArgs& g) { return g.k >= 1536 ? 256 : 192; }
 
 bool launch_gemm_fp8_block128_tiled(const GemmArgs& g, hipStream_t stream) {
     if (!tiled_shape_ok(g) || (g.k & 127) != 0) return false;
+    if (wide_tiles_take(g)) {
+        launch_wide256<Op32F8<0>, SCALE_BLOCK128>(g, stream);
+        return true;
+    }
     if (large_tiles_take(g)) {
         if (const int r = tile_tail_rows(g, block_tail_tiles(g))) {
             GemmArgs head, tail;

@@ -10,6 +10,8 @@
 // slab the loads and reads go changes nothing as long as they are spread (all loads behind the first three MFMAs: 4 to 8% slower).
 // LDS layout of a slab, load plan, fragment reads and accumulator layout are those of gemm_mid128_kernel.
 #pragma once
+#include <type_traits>
+
 #include "gemm_pingpong.cuh"
 
 namespace w8a8 {
@@ -116,6 +118,29 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[ni][mi][j] = 0;
 
+    // ---- 128-block scales: a slab is one K-block, a wave's 128 columns one weight block. A sub-tile's product of a slab is formed apart
+    // and joins the accumulator scaled by the row's and the block's steps, behind the next sub-tile's MFMAs. A row's steps of four slabs
+    // are one load, requested in the first slab of the four before, ahead of its slab loads; past the last slab and past M they
+    // are never used.
+    constexpr int STEPS = ScaleKind == SCALE_BLOCK128 ? MI + 1 : 0;
+    [[maybe_unused]] u32x4 steps[MI + 1], steps_next[MI + 1];
+    [[maybe_unused]] Acc part[2];
+    [[maybe_unused]] float behind = 0.0f;
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsa = make_rsrc(g.sa, STEPS ? (uint32_t)g.m * (uint32_t)ksteps * 4u : 0u);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsb = make_rsrc(g.sb, STEPS ? (uint32_t)((g.n + 127) >> 7) * (uint32_t)ksteps * 4u : 0u);
+    auto request = [&](int kb, u32x4 (&d)[MI + 1]) __attribute__((always_inline)) {
+        if constexpr (STEPS > 0) {
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) d[mi] = buf_load16(rsa, (uint32_t)(mw + mi * 32 + lrow) * (uint32_t)ksteps * 4u, (uint32_t)kb * 4u);
+            d[MI] = buf_load16(rsb, (uint32_t)((n0 + nw) >> 7) * (uint32_t)ksteps * 4u, (uint32_t)kb * 4u);
+        }
+    };
+    if constexpr (STEPS > 0) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) part[(MI * NI - 1) & 1][j] = 0;
+        request(0, steps);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
@@ -134,16 +159,38 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     uint8_t* next = lds + Cfg::STAGE_BYTES;          // of slab k + 1
     uint8_t* const last = lds + (S - 1) * Cfg::STAGE_BYTES;
     // in: this slab's fragments, their reads under way
-    auto slab = [&](int k, const u32x4 (&xf)[MI][4], const u32x4 (&wf)[NI][4], u32x4 (&xn)[MI][4], u32x4 (&wn)[NI][4])
+    auto slab = [&](auto at, auto more, int k, u32x4 (&xf)[MI][4], u32x4 (&wf)[NI][4], u32x4 (&xn)[MI][4], u32x4 (&wn)[NI][4])
                     __attribute__((always_inline)) {
+        constexpr int AT = decltype(at)::value;
+        constexpr bool MORE = decltype(more)::value;
         wait_lgkmcnt0();
-        wait_vmcnt<Cfg::LOADS*(S - 2)>();   // slab k + 1 has landed
+        wait_vmcnt<Cfg::LOADS*(S - 2) + (MORE && AT == 1 ? STEPS : 0)>();   // slab k + 1 has landed
         phase_barrier();                    // for every wave, and every wave has read slab k: its stage is free
+        [[maybe_unused]] float step[MI];
+        if constexpr (STEPS > 0) {
+            if constexpr (MORE && AT == 0) {
+                request(k + 4, steps_next);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) step[mi] = __uint_as_float(steps[mi][AT]) * __uint_as_float(steps[MI][AT]);
+        }
         constexpr int MFMAS = Op::STEPS * NI * MI, BUSY = MFMAS * 3 / 4;   // reads and loads behind the first three quarters
 #pragma unroll
         for (int i = 0; i < MFMAS; ++i) {
-            const int q = i / (NI * MI), ni = i / MI % NI, mi = i % MI;
-            acc[ni][mi] = Op::mma_step(q, wf[ni], xf[mi], acc[ni][mi]);
+            if constexpr (STEPS > 0) {
+                const int t = i / Op::STEPS, q = i % Op::STEPS, before = (t + NI * MI - 1) % (NI * MI);
+                const float by = t == 0 ? behind : step[before % MI];
+                if (q == 0) part[t & 1] = Op::mma_step(q, wf[t / MI], xf[t % MI], Acc{});
+                else part[t & 1] = Op::mma_step(q, wf[t / MI], xf[t % MI], part[t & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 16 / Op::STEPS * q; j < 16 / Op::STEPS * (q + 1); ++j)
+                    acc[before / MI][before % MI][j] += part[before & 1][j] * by;
+            } else {
+                const int q = i / (NI * MI), ni = i / MI % NI, mi = i % MI;
+                acc[ni][mi] = Op::mma_step(q, wf[ni], xf[mi], acc[ni][mi]);
+            }
             __builtin_amdgcn_sched_barrier(0);
             if (i < BUSY) {
 #pragma unroll
@@ -153,16 +200,39 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (STEPS > 0) behind = step[MI - 1];
         here = next;
         next = next == last ? lds : next + Cfg::STAGE_BYTES;
     };
+    constexpr std::integral_constant<int, 0> at0{};
     int k = 0;
-    for (; k + 1 < ksteps; k += 2) {
-        slab(k, xa, wa, xb, wb);
-        slab(k + 1, xb, wb, xa, wa);
+    if constexpr (STEPS > 0) {
+        constexpr std::integral_constant<int, 1> at1{};
+        constexpr std::integral_constant<int, 2> at2{};
+        constexpr std::integral_constant<int, 3> at3{};
+        for (; k + 3 < ksteps; k += 4) {
+            slab(at0, std::true_type{}, k, xa, wa, xb, wb);
+            slab(at1, std::true_type{}, k + 1, xb, wb, xa, wa);
+            slab(at2, std::true_type{}, k + 2, xa, wa, xb, wb);
+            slab(at3, std::true_type{}, k + 3, xb, wb, xa, wa);
+#pragma unroll
+            for (int i = 0; i <= MI; ++i) steps[i] = steps_next[i];
+        }
+        if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wb);
+        if (k + 1 < ksteps) slab(at1, std::false_type{}, k + 1, xb, wb, xa, wa);
+        if (k + 2 < ksteps) slab(at2, std::false_type{}, k + 2, xa, wa, xb, wb);
+    } else {
+        for (; k + 1 < ksteps; k += 2) {
+            slab(at0, std::false_type{}, k, xa, wa, xb, wb);
+            slab(at0, std::false_type{}, k + 1, xb, wb, xa, wa);
+        }
+        if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wb);
     }
-    if (k < ksteps) slab(k, xa, wa, xb, wb);
     wait_vmcnt<0>();   // (the loads of slabs past the end)
+    if constexpr (STEPS > 0) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[NI - 1][MI - 1][j] += part[(MI * NI - 1) & 1][j] * behind;
+    }
 
     // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad)
     TileOut<Cfg::BM, Cfg::BN, Cfg::THREADS>::store(g, lds, m0, n0, [&](auto put) __attribute__((always_inline)) {
@@ -216,7 +286,7 @@ inline void launch_wide256(const GemmArgs& g, hipStream_t stream) {
     auto kern = gemm_wide256_kernel<Op, ScaleKind, RoundFirst>;
     static std::atomic<uint64_t> lds_allowed{0};
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::LDS_BYTES, lds_allowed);
-    note_kernel("mid128x256");
+    note_kernel(ScaleKind == SCALE_BLOCK128 ? "mid128x256_block128" : "mid128x256");
     kern<<<dim3((unsigned)tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(g);
 }
 

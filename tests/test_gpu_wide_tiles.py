@@ -73,3 +73,26 @@ def test_block128_in_two_halves(slabs):
     out = _cabi.mm_fp8_block128(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV)).cpu()
     assert out[5].isnan().all() and torch.isfinite(out[torch.arange(m) != 5, :128]).all()
     assert not torch.isfinite(out[:, 128:]).any()
+
+
+@pytest.mark.parametrize("slabs,n", [(8, 3716), (9, 3715), (10, 3712), (11, 3716), (12, 3720), (13, 3713), (14, 3584)])
+def test_block128_wide(slabs, n):
+    """Every count of slabs modulo four (steps come four at a time) and three (stages); steps spread over seven octaves, one of them
+    not a number."""
+    from astrai_amd.extension import _cabi
+    from oracle import w8a8_oracle as O
+    m, k = 1163, 128 * slabs
+    print(f"case m={m} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(slabs)
+    a, b = (torch.randn(i, k, generator=g).to(torch.float8_e4m3fn) for i in (m, n))
+    sa = 2.0 ** (torch.rand(m, slabs, generator=g) * 7 - 5)
+    sb = 2.0 ** (torch.rand((n + 127) // 128, slabs, generator=g) * 7 - 5)
+    want = O.fp8_gemm_blockscaled(a, b, sa, sb)
+    run = lambda: _cabi.mm_fp8_block128(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV))   # noqa: E731
+    out = run()
+    assert _cabi.last_kernel() == "mid128x256_block128"
+    assert_bf16_close(out, want, what=f"{slabs} slabs")
+    sa[5, slabs // 2], sb[3, slabs - 1] = float("nan"), float("inf")
+    out, hit = run().cpu(), torch.zeros(m, n, dtype=torch.bool)
+    hit[5], hit[:, 384:512] = True, True
+    assert torch.equal(~torch.isfinite(out), hit)
