@@ -639,9 +639,10 @@ int astrai_mix_conv(const void* proj, int64_t ld, int64_t off, int64_t cols, con
     MIX_TRY(check_block("conv", batch, seq, seq, ld, 8));
     MIX_TRY(check_conv("conv", ld, off, cols, w, bias, taps, ring, positions));
     if (batch * seq * (cols / 4) > (int64_t)kMaxInt * 64) return fail(ASTRAI_MIX_BAD_ARG, "conv: too many elements");
-    const ConvArgs a = conv_args(proj, ld, off, cols, w, bias, taps, ring, positions, out, batch, seq, silu);
+    ConvArgs a = conv_args(proj, ld, off, cols, w, bias, taps, ring, positions, out, batch, seq, silu);
+    a.tail = tail;
     if (out) launch_conv(a, dtype, static_cast<hipStream_t>(stream));
-    if (tail) launch_conv_tail(a, dtype, static_cast<hipStream_t>(stream));
+    else if (tail) launch_conv_tail(a, dtype, static_cast<hipStream_t>(stream));
     return check_launch("conv");
 }
 

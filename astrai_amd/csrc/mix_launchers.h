@@ -240,6 +240,7 @@ struct ConvArgs {
     void* out;                 // [batch * seq, cols]
     int batch, seq, taps, ring_rows;
     int silu;
+    int tail = 0;              // launch_conv: the block's last inputs go into the ring as well
 };
 void launch_conv(const ConvArgs& a, int dtype, hipStream_t stream);        // reads the ring
 void launch_conv_tail(const ConvArgs& a, int dtype, hipStream_t stream);   // writes the last inputs into it

@@ -72,8 +72,8 @@ class MixerCache(StepCache):
 
     def reset(self) -> None:
         super().reset()
-        for s in self.state.values():
-            s.zero_()
+        if self.state:
+            torch._foreach_zero_(list(self.state.values()))   # one launch
 
 
 class RequestCaches:
