@@ -24,10 +24,12 @@ bool large_tiles_take(const GemmArgs& g) {
 }
 
 // Tiles of 128 x 256 where those are one round of the chip and 128 x 128 tiles more than one, ahead of the large tiles, which leave
-// half of the chip idle there (us, 256 x 256 / 128 x 256: 2100 x 2048 x 7168 73 / 59, 4000 x 2048 x 7168 77 / 72, 1100 x 4096 x 4096 46 /
-// 37.5, 2000 x 4096 x 4096 49 / 46, 700 x 7168 x 2048 25.6 / 23.4, 2100 x 2048 x 1024 16.5 / 15.7; with fewer slabs their start and
-// end are the longer ones: 2000 x 4096 x 640 14.2 / 15.3, 1100 x 4096 x 512 12.0 / 12.1).
-bool wide_tiles_take(const GemmArgs& g) { return g.k >= 1024 && wide256_shape_ok(g); }
+// half of the chip idle there (us, 256 x 256 / 128 x 256: 2100 x 2048 x 7168 73 / 52, 4000 x 2048 x 7168 77 / 66, 1100 x 4096 x 4096 46 /
+// 32, 2000 x 4096 x 4096 49 / 40, 700 x 7168 x 2048 25.6 / 19.9, 2100 x 2048 x 1024 16.5 / 12.8, 1100 x 4096 x 256 9.5 / 8.6, 1700 10.4 / 9.8; not the fullest with the fewest slabs, 2048 10.2 / 10.4).
+bool wide_tiles_take(const GemmArgs& g) {
+    const int64_t small = (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128);
+    return g.k >= (small > 448 ? 384 : 256) && wide256_shape_ok(g);
+}
 
 // Tails on smaller tiles as in tile_tail_rows (one launch / two; tiles of the tail): 4300 x 4096 x 4096 102 / 79 us (64), x 256
 // 19.8 / 17.5; 4500 x 4096 x 4096 101 / 86 (128); 4700 101 / 98 (192), x 256 19.6 / 19.9; 5000 x 4096 x 256 (256) 19.9 / 21.8, x

@@ -64,7 +64,7 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
 }
 
 // Plain bf16 products that the large tiles take, behind wide256_shape_ok: where they fill most of the chip, or from 449 tiles of 128 x
-// 128 on (with K up to 512, or past what tiles of 128 x 256 do in one round). Two
+// 128 on (those past what tiles of 128 x 256 do in one round). Two
 // workgroups of those share a compute unit and take longer the more units have two, where a round of large tiles costs
 // the same however empty (us, 128 x 128 / large, fp8 and int8: 2048 x 4096 x 512 14.5 / 12.0 and 15.1 / 13.5, x 4096 37.8 / 37.5
 // and 41.2 / 40.1, x 11008 87 / 86 and 96 / 90; 640 x 11776 x 4096, 460 tiles, 43 / 37 and 44 / 40). What it costs: up to 480

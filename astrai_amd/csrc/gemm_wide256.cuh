@@ -1,13 +1,13 @@
 // 8-bit NT GEMM on tiles of 128 (m) x 256 (n): products whose tiles of 128 x 128 are one to two rounds of the chip, so
 // that a compute unit takes two of those or one of these.
 //
-// Four waves of 64 x 128 (two by four MFMA 32x32 sub-tiles, 128 accumulator registers), one workgroup per compute unit. What
-// bounds tiles of 128 x 128 is LDS: 96 KiB of fragments and 32 KiB of loads for 512 cycles of MFMAs. Here it is 96 + 48 KiB for 1024.
-// K in 128-byte slabs through three LDS stages of 48 KiB, filled three slabs ahead by direct-to-LDS loads. One wave a SIMD has
-// nobody to cover its reads, so they go between its own MFMAs: slab k + 1 is read into a second register set, and slab k + 3
-// requested into the stage of slab k (which every wave has read before the one barrier of a slab), behind slab k's MFMAs. A slab
-// takes 0.69 us (fp8, K = 11008, 144 tiles): without the loads 0.56, without the MFMAs 0.62, without the reads 0.65; where in the
-// slab the loads and reads go changes nothing as long as they are spread (all loads behind the first three MFMAs: 4 to 8% slower).
+// Eight waves of 64 x 64 (two by two MFMA 32x32 sub-tiles, 64 accumulator registers), one workgroup per compute unit. What
+// bounds tiles of 128 x 128 is LDS: 96 KiB of fragments and 32 KiB of loads for 512 cycles of MFMAs. Here it is 128 + 48 KiB for 1024.
+// K in 128-byte slabs through three LDS stages of 48 KiB, filled three slabs ahead by direct-to-LDS loads: slab k + 1 is read into a
+// second register set, and slab k + 3 requested into the stage of slab k (which every wave has read before the one barrier of a slab),
+// behind slab k's MFMAs. Four waves of 64 x 128 (96 + 48 KiB, one wave a SIMD) took 0.69 us a slab (fp8, K = 11008, 144 tiles; without the
+// loads 0.56, without the MFMAs 0.62, without the reads 0.65) and were 1 to 10% slower, most with few slabs; with all loads of a slab
+// behind its first three MFMAs 4 to 8% slower still.
 // LDS layout of a slab, load plan, fragment reads and accumulator layout are those of gemm_mid128_kernel.
 #pragma once
 #include <type_traits>
@@ -18,19 +18,19 @@ namespace w8a8 {
 
 struct Wide256Cfg {
     static constexpr int BM = 128, BN = 256, BK = 128;
-    static constexpr int THREADS = 256;
-    static constexpr int MI = 2, NI = 4;                    // 32-row sub-tiles per wave: 64 m x 128 n
+    static constexpr int THREADS = 512, WAVES = 8;
+    static constexpr int MI = 2, NI = 2;                    // 32-row sub-tiles per wave: 64 m x 64 n
     static constexpr int STAGES = 3;
     static constexpr int X_BYTES = BM * BK;                 // 16 KiB, then 32 KiB of weights
     static constexpr int STAGE_BYTES = (BM + BN) * BK;
     static constexpr int COLUMNS = STAGES * STAGE_BYTES;    // the columns' steps and biases behind the stages
     static constexpr int LDS_BYTES = COLUMNS + 2 * BN * 4;
     static_assert(TileOut<BM, BN, THREADS>::BYTES <= COLUMNS, "outputs fit ahead of the columns");
-    static constexpr int LOADS = (BM + BN) / 8 / 4;         // of a wave and slab: eight rows each
+    static constexpr int X_LOADS = BM / 8 / WAVES, LOADS = (BM + BN) / 8 / WAVES;   // of a wave and slab: eight rows each
 };
 
 template <class Op, int ScaleKind, bool RoundFirst>
-__global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(GemmArgs g) {
+__global__ __launch_bounds__(Wide256Cfg::THREADS, 2) void gemm_wide256_kernel(GemmArgs g) {
     using Cfg = Wide256Cfg;
     using Acc = typename Op::Acc;
     constexpr int MI = Cfg::MI, NI = Cfg::NI, S = Cfg::STAGES;
@@ -38,7 +38,7 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wave_m = wave & 1, wave_n = wave >> 1;   // 2 x 2 waves
+    const int wave_m = wave & 1, wave_n = wave >> 1;   // 2 x 4 waves
     const int lrow = lane & 31, lgrp = lane >> 5;
 
     const TileCoord tc = map_tile((g.m + Cfg::BM - 1) / Cfg::BM, (g.n + Cfg::BN - 1) / Cfg::BN);
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     // epilogue operands, requested now: a row's step in a register, a column's step and bias for LDS
     const EpilogueScalars es = load_epilogue_scalars<ScaleKind>(g);
     [[maybe_unused]] const float s_tensor = es.sa * es.sb;
-    const int mw = m0 + wave_m * 64, nw = wave_n * 128;   // (nw: inside the tile)
+    const int mw = m0 + wave_m * 64, nw = wave_n * 32 * NI;   // (nw: inside the tile)
     float sx[MI];
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
@@ -61,20 +61,20 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     }
     const uint16_t* bias = static_cast<const uint16_t*>(g.bias);
     float col_step = 1.0f, col_bias = 0.0f;
-    if (n0 + (int)threadIdx.x < g.n) {
+    if ((int)threadIdx.x < Cfg::BN && n0 + (int)threadIdx.x < g.n) {
         if constexpr (ScaleKind == SCALE_ROWCOL) col_step = g.sb[n0 + threadIdx.x];
         if (bias) col_bias = bf16_to_f32(bias[n0 + threadIdx.x]);
     }
 
-    // ---- direct-to-LDS load plan: wave w fills rows 32w .. 32w+31 of the activations and 64w .. 64w+63 of the weights, 8
+    // ---- direct-to-LDS load plan: wave w fills rows 16w .. 16w+15 of the activations and 32w .. 32w+31 of the weights, 8
     // rows per instruction. Lane l lands at row l>>3, position l&7 of its 1 KiB block and fetches logical chunk (l&7) ^ f(row): c0
     // for even instructions, c0 ^ 1 for odd ones. Rows past M / N are past the buffer's num_records and read as zero.
     const uint32_t x_bytes = (uint32_t)g.m * (uint32_t)K, w_bytes = (uint32_t)g.n * (uint32_t)K;
     uint32_t x_off[2], w_off[2];
     {
         const int c0 = (lane & 7) ^ (lane >> 3);
-        const uint32_t xr = (uint32_t)(m0 + wave * 32 + (lane >> 3)) * (uint32_t)K;
-        const uint32_t wr = (uint32_t)(n0 + wave * 64 + (lane >> 3)) * (uint32_t)K;
+        const uint32_t xr = (uint32_t)(m0 + wave * 8 * Cfg::X_LOADS + (lane >> 3)) * (uint32_t)K;
+        const uint32_t wr = (uint32_t)(n0 + wave * 16 * Cfg::X_LOADS + (lane >> 3)) * (uint32_t)K;
         x_off[0] = xr + (uint32_t)c0 * 16;
         x_off[1] = xr + (uint32_t)(c0 ^ 1) * 16;
         w_off[0] = wr + (uint32_t)c0 * 16;
@@ -85,11 +85,11 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     auto load = [&](int r, uint8_t* stage, int slab) __attribute__((always_inline)) {
         const uint32_t k0 = (uint32_t)slab << 7;
         const bool live = slab < ksteps;
-        if (r < 4) {
-            lds_dma16(make_rsrc(g.a, live ? x_bytes : 0u), stage + wave * 4096 + r * 1024, x_off[r & 1] + (uint32_t)r * row8, k0);
+        if (r < Cfg::X_LOADS) {
+            lds_dma16(make_rsrc(g.a, live ? x_bytes : 0u), stage + (wave * Cfg::X_LOADS + r) * 1024, x_off[r & 1] + (uint32_t)r * row8, k0);
         } else {
-            const int i = r - 4;
-            lds_dma16(make_rsrc(g.b, live ? w_bytes : 0u), stage + Cfg::X_BYTES + wave * 8192 + i * 1024,
+            const int i = r - Cfg::X_LOADS;
+            lds_dma16(make_rsrc(g.b, live ? w_bytes : 0u), stage + Cfg::X_BYTES + (wave * 2 * Cfg::X_LOADS + i) * 1024,
                       w_off[i & 1] + (uint32_t)i * row8, k0);
         }
     };
@@ -118,13 +118,13 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[ni][mi][j] = 0;
 
-    // ---- 128-block scales: a slab is one K-block, a wave's 128 columns one weight block. A sub-tile's product of a slab is formed apart
-    // and joins the accumulator scaled by the row's and the block's steps, behind the next sub-tile's MFMAs. A row's steps of four slabs
-    // are one load, requested in the first slab of the four before, ahead of its slab loads; past the last slab and past M they
-    // are never used.
+    // ---- 128-block scales: a slab is one K-block, a wave's columns lie in one weight block. A sub-tile's product of a slab is formed
+    // apart and joins the accumulator scaled by the row's and the block's steps ahead of the next sub-tile's MFMAs, with the
+    // other wave's of the SIMD beside it. A row's steps of four slabs are one load, requested in the last slab before them, ahead of its
+    // slab loads; past the last slab and past M they are never used.
     constexpr int STEPS = ScaleKind == SCALE_BLOCK128 ? MI + 1 : 0;
-    [[maybe_unused]] u32x4 steps[MI + 1], steps_next[MI + 1];
-    [[maybe_unused]] Acc part[2];
+    [[maybe_unused]] u32x4 steps[MI + 1];
+    [[maybe_unused]] Acc part;
     [[maybe_unused]] float behind = 0.0f;
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsa = make_rsrc(g.sa, STEPS ? (uint32_t)g.m * (uint32_t)ksteps * 4u : 0u);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsb = make_rsrc(g.sb, STEPS ? (uint32_t)((g.n + 127) >> 7) * (uint32_t)ksteps * 4u : 0u);
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     };
     if constexpr (STEPS > 0) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) part[(MI * NI - 1) & 1][j] = 0;
+        for (int j = 0; j < 16; ++j) part[j] = 0;
         request(0, steps);
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -146,8 +146,10 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
 #pragma unroll
         for (int r = 0; r < Cfg::LOADS; ++r) load(r, lds + s * Cfg::STAGE_BYTES, s);
     float* const columns = reinterpret_cast<float*>(lds + Cfg::COLUMNS);
-    columns[threadIdx.x] = col_step;
-    columns[Cfg::BN + threadIdx.x] = col_bias;
+    if ((int)threadIdx.x < Cfg::BN) {
+        columns[threadIdx.x] = col_step;
+        columns[Cfg::BN + threadIdx.x] = col_bias;
+    }
     wait_vmcnt<Cfg::LOADS*(S - 1)>();
     wait_lgkmcnt0();
     phase_barrier();
@@ -163,41 +165,64 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
                     __attribute__((always_inline)) {
         constexpr int AT = decltype(at)::value;
         constexpr bool MORE = decltype(more)::value;
-        wait_lgkmcnt0();
-        wait_vmcnt<Cfg::LOADS*(S - 2) + (MORE && AT == 1 ? STEPS : 0)>();   // slab k + 1 has landed
-        phase_barrier();                    // for every wave, and every wave has read slab k: its stage is free
         [[maybe_unused]] float step[MI];
+        auto arrive = [&]() __attribute__((always_inline)) {
+            wait_lgkmcnt0();
+            wait_vmcnt<Cfg::LOADS*(S - 2)>();   // slab k + 1 has landed
+            phase_barrier();                    // for every wave, and every wave has read slab k: its stage is free
+        };
         if constexpr (STEPS > 0) {
-            if constexpr (MORE && AT == 0) {
-                request(k + 4, steps_next);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            // MFMA i of 8; the columns' fragments are overwritten by the next slab's where they have been used last
+            static_assert(Op::STEPS == 2 && MI == 2 && NI == 2 && Cfg::LOADS == 6, "places of the reads and loads");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xc07f | 4 << 8);   // all but the last four reads: those of the second columns
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi) step[mi] = __uint_as_float(steps[mi][AT]) * __uint_as_float(steps[MI][AT]);
-        }
-        constexpr int MFMAS = Op::STEPS * NI * MI, BUSY = MFMAS * 3 / 4;   // reads and loads behind the first three quarters
 #pragma unroll
-        for (int i = 0; i < MFMAS; ++i) {
-            if constexpr (STEPS > 0) {
-                const int t = i / Op::STEPS, q = i % Op::STEPS, before = (t + NI * MI - 1) % (NI * MI);
-                const float by = t == 0 ? behind : step[before % MI];
-                if (q == 0) part[t & 1] = Op::mma_step(q, wf[t / MI], xf[t % MI], Acc{});
-                else part[t & 1] = Op::mma_step(q, wf[t / MI], xf[t % MI], part[t & 1]);
+            for (int i = 0; i < 8; ++i) {
+                const int t = i / 2, q = i % 2;
+                if (q == 0) {   // the last sub-tile's product joins its sums, then this one's takes its place
+                    const int before = (t + 3) % 4;
+                    const float by = t == 0 ? behind : step[before % MI];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) acc[before / MI][before % MI][j] += part[j] * by;
+                    __builtin_amdgcn_sched_barrier(0);
+                    part = Op::mma_step(q, wf[t / MI], xf[t % MI], Acc{});
+                } else {
+                    part = Op::mma_step(q, wf[t / MI], xf[t % MI], part);
+                }
                 __builtin_amdgcn_sched_barrier(0);
+                if (i == 1) {
+                    arrive();
+                    if constexpr (MORE && AT == 3) {
+                        request(k + 1, steps);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                if (i >= 1 && i < 7) load(i - 1, here, k + S);
+                if (i >= 1 && i < 5) read(2 * i - 2, next, xn, wf), read(2 * i - 1, next, xn, wf);
+                if (i >= 5 && i < 7) read(2 * i - 2, next, xn, wf), read(2 * i - 1, next, xn, wf);
+                if (i == 7)
 #pragma unroll
-                for (int j = 16 / Op::STEPS * q; j < 16 / Op::STEPS * (q + 1); ++j)
-                    acc[before / MI][before % MI][j] += part[before & 1][j] * by;
-            } else {
+                    for (int r = 12; r < 16; ++r) read(r, next, xn, wf);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            arrive();
+            constexpr int MFMAS = Op::STEPS * NI * MI, BUSY = MFMAS * 3 / 4;   // reads and loads behind the first three quarters
+#pragma unroll
+            for (int i = 0; i < MFMAS; ++i) {
                 const int q = i / (NI * MI), ni = i / MI % NI, mi = i % MI;
                 acc[ni][mi] = Op::mma_step(q, wf[ni], xf[mi], acc[ni][mi]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (i < BUSY) {
-#pragma unroll
-                for (int r = READS * i / BUSY; r < READS * (i + 1) / BUSY; ++r) read(r, next, xn, wn);
-#pragma unroll
-                for (int r = Cfg::LOADS * i / BUSY; r < Cfg::LOADS * (i + 1) / BUSY; ++r) load(r, here, k + S);
                 __builtin_amdgcn_sched_barrier(0);
+                if (i < BUSY) {
+#pragma unroll
+                    for (int r = READS * i / BUSY; r < READS * (i + 1) / BUSY; ++r) read(r, next, xn, wn);
+#pragma unroll
+                    for (int r = Cfg::LOADS * i / BUSY; r < Cfg::LOADS * (i + 1) / BUSY; ++r) load(r, here, k + S);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         if constexpr (STEPS > 0) behind = step[MI - 1];
@@ -211,16 +236,14 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
         constexpr std::integral_constant<int, 2> at2{};
         constexpr std::integral_constant<int, 3> at3{};
         for (; k + 3 < ksteps; k += 4) {
-            slab(at0, std::true_type{}, k, xa, wa, xb, wb);
-            slab(at1, std::true_type{}, k + 1, xb, wb, xa, wa);
-            slab(at2, std::true_type{}, k + 2, xa, wa, xb, wb);
-            slab(at3, std::true_type{}, k + 3, xb, wb, xa, wa);
-#pragma unroll
-            for (int i = 0; i <= MI; ++i) steps[i] = steps_next[i];
+            slab(at0, std::true_type{}, k, xa, wa, xb, wa);
+            slab(at1, std::true_type{}, k + 1, xb, wa, xa, wa);
+            slab(at2, std::true_type{}, k + 2, xa, wa, xb, wa);
+            slab(at3, std::true_type{}, k + 3, xb, wa, xa, wa);
         }
-        if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wb);
-        if (k + 1 < ksteps) slab(at1, std::false_type{}, k + 1, xb, wb, xa, wa);
-        if (k + 2 < ksteps) slab(at2, std::false_type{}, k + 2, xa, wa, xb, wb);
+        if (k < ksteps) slab(at0, std::false_type{}, k, xa, wa, xb, wa);
+        if (k + 1 < ksteps) slab(at1, std::false_type{}, k + 1, xb, wa, xa, wa);
+        if (k + 2 < ksteps) slab(at2, std::false_type{}, k + 2, xa, wa, xb, wa);
     } else {
         for (; k + 1 < ksteps; k += 2) {
             slab(at0, std::false_type{}, k, xa, wa, xb, wb);
@@ -231,7 +254,7 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
     wait_vmcnt<0>();   // (the loads of slabs past the end)
     if constexpr (STEPS > 0) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) acc[NI - 1][MI - 1][j] += part[(MI * NI - 1) & 1][j] * behind;
+        for (int j = 0; j < 16; ++j) acc[NI - 1][MI - 1][j] += part[j] * behind;
     }
 
     // ---- epilogue: a lane holds four consecutive n of one m per (sub-tile, quad)
@@ -266,15 +289,14 @@ __global__ __launch_bounds__(Wide256Cfg::THREADS, 1) void gemm_wide256_kernel(Ge
 }
 
 // bf16 output, K in whole slabs, more tiles of 128 x 128 than compute units and no more of these than that. us, int8 / fp8, on tiles
-// of 128 x 128 (to 448 of them, else 256 x 256) -> here: 1111 x 4096 x 11008 86 / 84 -> 67 / 62, 2048 x 4096 x 4096 43.9 / 41.7 ->
-// 36.5 / 33, 1100 x 4096 x 4096 36.2 / 35.0 -> 29.5 / 26.8, 1954 x 3072 x 2048 25.0 / 23.3 -> 20.6 / 19.1, 4000 x 2048 x 2048 27.4 /
-// 25.9 -> 24.2 / 22.0, 500 x 11264 x 2048 24.6 / 22.5 -> 19.9 / 18.6, 1200 x 4096 x 256 12.2 / 11.4 -> 10.1 / 9.4; a few slabs are
-// one round of 256 x 256 tiles as well, 2000 x 4096 x 384 13.0 / 11.4 and 12.3 / 11.5, x 640 15.3 / 13.5 and 14.0 / 13.0. With half as
+// of 128 x 128 (to 448 of them, else 256 x 256) -> here: 1111 x 4096 x 11008 86 / 84 -> 66 / 61, 2048 x 4096 x 4096 43.9 / 41.7 ->
+// 35.8 / 33, 1100 x 4096 x 4096 36.2 / 35.0 -> 27.8 / 25.4, 1954 x 3072 x 2048 25.0 / 23.3 -> 18.6 / 17.5, 4000 x 2048 x 2048 27.4 /
+// 25.9 -> 21.9 / 20.3, 500 x 11264 x 2048 24.6 / 22.5 -> 17.8 / 17.0, 1200 x 4096 x 256 12.2 / 11.4 -> 8.8 / 8.4. With half as
 // many tiles those of 128 x 128 are one round too, and the faster one (900 x 4096 x 4096, 256 of them, 23.5 of fp8).
 inline bool wide256_shape_ok(const GemmArgs& g) {
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 128 || g.out_kind != OUT_BF16) return false;
     const int64_t tm = (g.m + 127) / 128, small = tm * ((g.n + 127) / 128);
-    return small > 256 && tm * ((g.n + 255) / 256) <= 256 && (small <= 448 || g.k > 512);
+    return small > 256 && tm * ((g.n + 255) / 256) <= 256;
 }
 
 template <class Op, int ScaleKind, bool RoundFirst = false>
