@@ -38,6 +38,15 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
         for (int j = 0; j < TAPS; ++j) w[j] = *reinterpret_cast<const f32x4*>(a.taps_w + (int64_t)j * a.cols + c);
 #pragma unroll
         for (int j = 1; j < TAPS; ++j) x[j] = conv_input4<T>(a, b, start, t0 - TAPS + j, c);
+        static_assert(TAPS - 1 <= kStrip, "no other strip reads the ring");
+        const bool ringed = a.tail && t0 == 0;
+        const int n = min(TAPS - 1, a.seq);
+        f32x4 keep[TAPS - 1];   // (asked for with the rest: one after the other at the end they cost what the launch did)
+        if (ringed) {
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS; ++j)
+                if (j < n) keep[j] = conv_input4<T>(a, b, start, a.seq - n + j, c);
+        }
 #pragma unroll
         for (int i = 0; i < kStrip; ++i) {
             const int t = t0 + i;
@@ -53,10 +62,11 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
                 finish(t, s);
             }
         }
-        static_assert(TAPS - 1 <= kStrip, "no other strip reads the ring");
-        if (a.tail && t0 == 0) {
-            const int n = min(TAPS - 1, a.seq);
-            for (int j = 0; j < n; ++j) ring_put4<T>(a, b, start, a.seq - n + j, c);
+        if (ringed) {
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS; ++j)
+                if (const int64_t p = start + a.seq - n + j; j < n && p >= 0)
+                    Elem<T>::put4(static_cast<T*>(a.ring) + ring_row(a, b, p) * a.cols + c, keep[j]);
         }
     } else {
         for (int t = t0; t < t1; ++t) finish(t, conv_at4<T>(a, b, start, t, c));
