@@ -260,19 +260,19 @@ int astrai_w8a8_add_rmsnorm_quantize_int8_rows(const void* x, const void* res, c
 int astrai_w8a8_embed_rmsnorm_quantize_int8_rows(const void* table, int64_t vocab, const int64_t* tokens, const void* weight, float eps,
                                                  void* x_out, void* xq, float* s, int64_t rows, int64_t k, const void* freqs,
                                                  int freqs_float, int64_t max_pos, int64_t cols, const int64_t* positions,
-                                                 int64_t n_pos, float* rotary, void* stream) {
+                                                 int64_t n_pos, int64_t seq, float* rotary, void* stream) {
     const char* what = "embed_rmsnorm_quantize_int8_rows";
     if (!table || !tokens || !weight || !x_out || !xq || !s || !freqs || !positions || !rotary)
         return fail(ASTRAI_W8A8_BAD_ARG, "%s: null pointer", what);
     if (vocab <= 0 || rows <= 0 || k <= 0 || max_pos <= 0 || cols <= 0 || n_pos <= 0 || rows > 0x3fffffff || cols > kMaxDim ||
-        n_pos > kMaxDim || n_pos * cols > kMaxDim)
+        n_pos > kMaxDim || n_pos * cols > kMaxDim || seq < 0 || seq > n_pos)
         return fail(ASTRAI_W8A8_BAD_ARG, "%s: bad dims", what);
     if (!(eps >= 0.0f)) return fail(ASTRAI_W8A8_BAD_ARG, "%s: eps must be >= 0", what);
     if ((k & 7) != 0 || k > w8a8::kFusedRowMax)
         return fail(ASTRAI_W8A8_UNSUPPORTED, "%s: K must be a multiple of 8 and at most 8192", what);
     if (!aligned16(table) || !aligned16(weight) || !aligned16(x_out) || !aligned16(xq))
         return fail(ASTRAI_W8A8_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
-    const w8a8::StartArgs e{table, tokens, vocab, freqs, positions, max_pos, n_pos, cols, freqs_float, rotary, x_out, 0u};
+    const w8a8::StartArgs e{table, tokens, vocab, freqs, positions, max_pos, n_pos, cols, seq, freqs_float, rotary, x_out, 0u};
     w8a8::launch_embed_rmsnorm_quantize_int8_rows(e, weight, eps, xq, s, rows, k, static_cast<hipStream_t>(stream));
     return check_launch(what);
 }

@@ -103,7 +103,8 @@ void launch_add_rmsnorm_quantize_int8_rows(const void* x, const void* res, const
                                            void* sum_out, void* y_out, void* xq, float* s,
                                            int64_t rows, int64_t k, hipStream_t stream);
 // The same at the start of a forward: x[r] = table[tokens[r]] is looked up and written out, and rotary[i] = freqs[positions[i]] as
-// fp32 in the same launch. A token or position outside its table reads as NaN.
+// fp32 in the same launch. A token or position outside its table reads as NaN in x and rotary, x of a row whose positions[r % seq] is
+// outside too; codes and steps of such rows are finite.
 struct StartArgs {
     const void* table;           // bf16 [vocab, k]
     const int64_t* tokens;       // [rows]
@@ -111,6 +112,7 @@ struct StartArgs {
     const void* freqs;           // bf16 or fp32 [max_pos, cols]
     const int64_t* positions;    // [n_pos]
     int64_t max_pos, n_pos, cols;
+    int64_t seq;                 // row r stands at positions[r % seq]; 0: rows and positions have nothing in common
     int freqs_float;
     float* rotary;               // [n_pos, cols]
     void* x_out;                 // bf16 [rows, k]

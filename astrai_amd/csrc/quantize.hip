@@ -618,13 +618,9 @@ __global__ __launch_bounds__(kThreads) void add_bias_bf16_kernel(uint16_t* out, 
     }
 }
 
-// s = bf16(x + res) (when res is given; written to sum_out), y = bf16(w * (rstd * s))
-// with rstd = rsqrt(mean(s^2) + eps) in fp32 -- one rounding, the arithmetic of
-// F.rms_norm on a bf16 tensor (model/components/norm.py:7-15) -- then the per-row
-// int8 quantizer on y.
-// START: x is the embedding table (StartArgs), and the launch's last workgroups look up the rotary rows: a decode step is three
-// launches of about 2 us each in the chain shorter (dense decoder, 2 layers: 32 sequences 127.8 -> 122.2 us, 5 sequences 98.5 ->
-// 91.9), and a prompt reads its tokens' rows once (32 x 512: 1724 -> 1716).
+// The START instances below: x is the embedding table (StartArgs), and the launch's last workgroups look up the rotary rows: a decode
+// step is three launches of about 2 us each in the chain shorter (dense decoder, 2 layers: 32 sequences 127.8 -> 122.2 us, 5 sequences
+// 98.5 -> 91.9), and a prompt reads its tokens' rows once (32 x 512: 1724 -> 1716).
 __device__ __forceinline__ void rotary_rows(const StartArgs& e) {
     const int64_t at = (int64_t)(blockIdx.x - e.row_blocks) * kThreads + threadIdx.x;
     if (at >= e.n_pos * e.cols) return;
@@ -635,16 +631,27 @@ __device__ __forceinline__ void rotary_rows(const StartArgs& e) {
     e.rotary[at] = v;
 }
 
-// a row's place in the table, -1 outside it
+// a row's place in the table, -1 where its token is outside it, or its position outside the other
 __device__ __forceinline__ int64_t table_row(const StartArgs& e, int64_t row) {
-    const int64_t tok = e.tokens[row];
-    return tok >= 0 && tok < e.vocab ? tok : -1;
+    const int64_t tok = e.tokens[row], pos = e.seq ? e.positions[(uint32_t)row % (uint32_t)e.seq] : 0;
+    return tok >= 0 && tok < e.vocab && pos >= 0 && pos < e.max_pos ? tok : -1;
 }
 
 __device__ __forceinline__ u32x4 table_piece(const uint16_t* table, int64_t at, int64_t k, int64_t i) {
     return at >= 0 ? *reinterpret_cast<const u32x4*>(table + at * k + i * 8) : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
 }
 
+// A row's step from its largest magnitude, which ignores what is not a number, as the quantizers' does: keys and values of such a row
+// stay finite. Where y goes out too, a row of y that is no number by its norm has such a step, and what is formed of its codes says
+// so as y does: a token or position outside its table ends in logits of NaN.
+__device__ __forceinline__ float row_step(float largest, float rstd, bool y_out) {
+    return y_out && rstd != rstd ? rstd : fmaxf(largest, 1e-12f) / 127.0f;
+}
+
+// s = bf16(x + res) (when res is given; written to sum_out), y = bf16(w * (rstd * s))
+// with rstd = rsqrt(mean(s^2) + eps) in fp32 -- one rounding, the arithmetic of
+// F.rms_norm on a bf16 tensor (model/components/norm.py:7-15) -- then the per-row
+// int8 quantizer on y.
 template <bool START>
 __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
@@ -703,7 +710,7 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kerne
             if (!START && y_out) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
         }
     }
-    const float step = fmaxf(block_max(local, slots), 1e-12f) / 127.0f;
+    const float step = row_step(block_max(local, slots), rstd, !START && y_out);
     if (threadIdx.x == 0) s[row] = step;
 #pragma unroll
     for (int c = 0; c < kCache; ++c) {
@@ -769,6 +776,7 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
             if (nr + stride < rows) from_next = table_row(e, nr + stride);
         float v[KC][8];
         float local = 0.0f;
+        [[maybe_unused]] float rstd = 1.0f;
         if constexpr (NORM) {
             // The sum of squares in the order of the one-workgroup-per-row kernel, so that a row's
             // rstd -- and with it y and every code -- does not depend on how many rows a launch
@@ -788,7 +796,7 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
             float ss = ssw[0];
 #pragma unroll
             for (int wv = 1; wv < 4; ++wv) ss += ssw[wv];
-            const float rstd = rsqrtf(ss / (float)k + eps);
+            rstd = rsqrtf(ss / (float)k + eps);
 #pragma unroll
             for (int c = 0; c < KC; ++c) {
                 float g[8];
@@ -807,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
                 local = fmaxf(local, amax8(v[c]));
             }
         }
-        const float step = fmaxf(wave_max(local), 1e-12f) / 127.0f;
+        const float step = row_step(wave_max(local), rstd, NORM && !START && y_out);
         if (lane == 0) s[row] = step;
 #pragma unroll
         for (int c = 0; c < KC; ++c) {

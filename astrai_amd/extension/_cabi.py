@@ -47,7 +47,7 @@ PROTOTYPES = {
     "astrai_w8a8_gradient_stats": ([_P] * 4 + [_I64] * 2 + [_P], _INT),
     "astrai_w8a8_quantize_bf16_int8_rows": ([_P, _P, _P, _I64, _I64, _P], _INT),
     "astrai_w8a8_embed_rmsnorm_quantize_int8_rows": (
-        [_P, _I64, _P, _P, _F32, _P, _P, _P, _I64, _I64, _P, _INT, _I64, _I64, _P, _I64, _P, _P], _INT),
+        [_P, _I64, _P, _P, _F32, _P, _P, _P, _I64, _I64, _P, _INT, _I64, _I64, _P, _I64, _I64, _P, _P], _INT),
     "astrai_w8a8_add_rmsnorm_quantize_int8_rows": (
         [_P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _I64, _I64, _P], _INT),
     "astrai_w8a8_silu_mul_quantize_int8_rows": ([_P, _P, _I64, _P, _P, _P, _I64, _I64, _P], _INT),
@@ -798,7 +798,8 @@ def quantize_int8_rows(x: torch.Tensor):
 def add_rmsnorm_quantize_int8(x: torch.Tensor, weight: torch.Tensor, eps: float,
                               res: Optional[torch.Tensor] = None, want_y: bool = False):
     """``t = x + res`` (bf16, when ``res`` is given), ``y = rms_norm(t) * weight``, per-row
-    int8 of ``y`` in one kernel. Returns ``(xq [R,K], s [R,1], t or None, y or None)``."""
+    int8 of ``y`` in one kernel. Returns ``(xq [R,K], s [R,1], t or None, y or None)``. The quantizer's maximum ignores NaN; with ``y``,
+    a row that is NaN by its norm has a step of NaN."""
     lib = _require()
     _gpu(x, "add_rmsnorm_quantize_int8")
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
@@ -827,8 +828,9 @@ def add_rmsnorm_quantize_int8(x: torch.Tensor, weight: torch.Tensor, eps: float,
 def embed_rmsnorm_quantize_int8(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, eps: float, freqs: torch.Tensor,
                                 positions: torch.Tensor):
     """The start of a forward in one kernel: ``x = table[ids]``, ``y = rms_norm(x) * weight``, per-row int8 of ``y``, and ``freqs``
-    (``[places, pairs, 2]``) at ``positions`` in fp32. Ids and positions outside their tables give NaN. Returns ``(x [*ids.shape, K],
-    xq [R,K], s [R,1], rotary [1, *positions.shape, pairs, 2])``, or ``None`` for operands the kernel does not take as they are."""
+    (``[places, pairs, 2]``) at ``positions`` in fp32. The last dimension of ``ids`` is at ``positions`` where it is as long. Ids and
+    positions outside their tables give NaN in ``x`` and ``rotary``, and finite codes and steps. Returns ``(x [*ids.shape, K], xq [R,K], s
+    [R,1], rotary [1, *positions.shape, pairs, 2])``, or ``None`` for operands the kernel does not take as they are."""
     lib = _require()
     dev, k = table.device, table.size(-1)
     if not (table.is_cuda and _plain_bf16(table, dev) and table.dim() == 2 and _plain_bf16(weight, dev) and weight.shape == (k,)
@@ -846,7 +848,7 @@ def embed_rmsnorm_quantize_int8(ids: torch.Tensor, table: torch.Tensor, weight: 
         _check(lib.astrai_w8a8_embed_rmsnorm_quantize_int8_rows(
             table.data_ptr(), table.size(0), ids.data_ptr(), weight.data_ptr(), float(eps), x.data_ptr(), xq.data_ptr(), s.data_ptr(),
             rows, k, freqs.data_ptr(), freqs.dtype == torch.float32, freqs.size(0), freqs[0].numel(), positions.data_ptr(), n_pos,
-            rotary.data_ptr(), _stream(table)), lib)
+            n_pos if ids.dim() and ids.size(-1) == n_pos else 0, rotary.data_ptr(), _stream(table)), lib)
     return x, xq, s, rotary
 
 

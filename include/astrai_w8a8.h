@@ -153,7 +153,8 @@ int astrai_w8a8_quantize_bf16_int8_rows(const void* x_bf16, void* xq, float* s,
  *   t[r,:]  = res ? bf16(x[r,:] + res[r,:]) : x[r,:]          (written to sum_out when res and sum_out are given)
  *   y[r,k]  = bf16(weight[k] * (t[r,k] * rsqrt(mean_k t[r,k]^2 + eps)))   fp32 arithmetic, one rounding
  *   s[r], xq[r,:] = the per-row int8 quantizer applied to y[r,:]
- * res, sum_out, y_out may be NULL (y_out receives y when given). K % 8 == 0, K <= 8192.
+ * res, sum_out, y_out may be NULL (y_out receives y when given). K % 8 == 0, K <= 8192. The quantizer's maximum ignores NaN; with
+ * y_out, s[r] is NaN where mean_k t[r,k]^2 is.
  *
  * silu_mul: replaces ``up(x) * F.silu(gate(x))`` of MLP.forward
  * (astrai/model/components/mlp.py:41) and the quantizer in front of ``down``.
@@ -169,13 +170,15 @@ int astrai_w8a8_add_rmsnorm_quantize_int8_rows(const void* x_bf16, const void* r
                                                float* s, int64_t rows, int64_t k, void* stream);
 /*
  * The start of a forward in one launch: x_out[r,:] = table[tokens[r],:] (bf16 [vocab, k]), its norm and codes as above, and
- * rotary[i,:] = freqs[positions[i],:] (bf16 or, with freqs_float, fp32 [max_pos, cols]) as fp32. A token or position outside
- * its table reads as NaN. K % 8 == 0, K <= 8192.
+ * rotary[i,:] = freqs[positions[i],:] (bf16 or, with freqs_float, fp32 [max_pos, cols]) as fp32. Row r stands at positions[r % seq]
+ * (seq <= n_pos; 0: at none of them). Outside the tables x_out (for a token, or the row's position) and rotary are NaN; codes and
+ * step of such a row are finite. K % 8 == 0, K <= 8192.
  */
 int astrai_w8a8_embed_rmsnorm_quantize_int8_rows(const void* table_bf16, int64_t vocab, const int64_t* tokens,
                                                  const void* weight_bf16, float eps, void* x_out_bf16, void* xq, float* s,
                                                  int64_t rows, int64_t k, const void* freqs, int freqs_float, int64_t max_pos,
-                                                 int64_t cols, const int64_t* positions, int64_t n_pos, float* rotary, void* stream);
+                                                 int64_t cols, const int64_t* positions, int64_t n_pos, int64_t seq, float* rotary,
+                                                 void* stream);
 int astrai_w8a8_silu_mul_quantize_int8_rows(const void* gate_bf16, const void* up_bf16, int64_t ld,
                                             void* h_out_bf16, void* hq, float* s, int64_t rows,
                                             int64_t width, void* stream);

@@ -69,3 +69,45 @@ def test_model_takes_it_and_leaves_observed_embeddings_alone():
         del model.embed_tokens.forward
         assert torch.equal(model(ids.int(), model.new_cache(2, 16))["logits"], got)   # (another type of ids: the plain way)
     assert model._start_fused_int8(ids, torch.arange(9, device=DEV)) is None   # the policy is off
+
+
+@pytest.mark.parametrize("rows,width", [(4, 256), (4, 8192), (700, 256), (700, 4096)])
+def test_a_row_of_nan_has_such_a_step_where_the_norm_goes_out(rows, width):
+    from astrai_amd.extension import _cabi
+    r = torch.Generator().manual_seed(rows)
+    x, weight = (torch.randn(*s, generator=r).bfloat16().to(DEV) for s in ((rows, width), (width,)))
+    wq, ws, _, wy = _cabi.add_rmsnorm_quantize_int8(x, weight, 1e-5, None, True)
+    x[1, 5] = float("nan")
+    good = torch.arange(rows, device=DEV) != 1
+    xq, s, _, y = _cabi.add_rmsnorm_quantize_int8(x, weight, 1e-5, None, True)
+    assert s[1].isnan().all() and y[1].isnan().all()
+    assert torch.equal(s[good], ws[good]) and torch.equal(xq[good], wq[good]) and torch.equal(y[good], wy[good])
+    s = _cabi.add_rmsnorm_quantize_int8(x, weight, 1e-5)[1]
+    assert torch.isfinite(s).all() and torch.equal(s[good], ws[good])
+
+
+@pytest.mark.parametrize("batch,seq,cached", [(2, 9, True), (2, 9, False), (1, 600, True), (5, 1, True)])
+def test_logits_of_what_is_outside_the_tables(batch, seq, cached):
+    """NaN for such a token and for one at such a place; what does not attend to it as ever."""
+    from astrai_amd.extension import w8a8
+    from astrai_amd.model import AutoRegressiveLM, AutoRegressiveLMConfig, fuse_int8_weights
+    torch.manual_seed(0)
+    places = 640
+    model = AutoRegressiveLM(AutoRegressiveLMConfig(hidden_size=512, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                                                    intermediate_size=1024, vocab_size=128, max_position_embeddings=places)).to(DEV).bfloat16()
+    fuse_int8_weights(model)
+    ids = torch.randint(0, 128, (batch, seq), device=DEV)
+    run = lambda t, at=None: model(t, model.new_cache(batch, 1300) if cached else None, at)["logits"]  # noqa: E731
+    with torch.no_grad(), w8a8.int8_autocast(True):
+        want = run(ids)
+        assert torch.isfinite(want).all()
+        for bad in (128, -1, 1 << 40):
+            wrong = ids.clone()
+            wrong[batch - 1, seq // 2] = bad
+            assert model._start_fused_int8(wrong, torch.arange(seq, device=DEV)) is not None
+            got = run(wrong)
+            assert got[batch - 1, seq // 2].isnan().all()
+            assert torch.equal(got[:batch - 1], want[:batch - 1]) and torch.equal(got[batch - 1, :seq // 2], want[batch - 1, :seq // 2])
+        at = torch.arange(places - seq // 2, places - seq // 2 + seq, device=DEV)
+        got = run(ids, at)
+        assert torch.isfinite(got[:, :seq // 2]).all() and got[:, seq // 2:].isnan().all()
