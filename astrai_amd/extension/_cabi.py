@@ -23,7 +23,7 @@ from astrai_amd.extension._native import NoCalls, load_calls
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libastrai_w8a8.so")
 
-ABI_VERSION = 1
+ABI_VERSION = 2
 OUT_BF16, OUT_E4M3, OUT_ACC = 0, 1, 2
 
 _P = ctypes.c_void_p

@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define ASTRAI_W8A8_ABI_VERSION 1
+#define ASTRAI_W8A8_ABI_VERSION 2
 
 /* status codes */
 #define ASTRAI_W8A8_OK 0
