@@ -1057,22 +1057,11 @@ def paged_nsplit(pairs: int, max_keys: int) -> int:
     CU, none that could not hold 160 keys, against two (16 / 4 heads, 32 x 3000 keys 33.2 us, 31.1; 32 / 4 heads 40.8,
     36.2; 64 x 1500 32.4, 28.7). The context's length decides and only the table's width is known here: up to some 500
     keys behind a wide table two are as good or better (64 x 100 9.5, 10.5; 64 x 300 13.5, 13.3; 32 x 530 12.3, 13.0), past
-    1000 three. Where that is two or one, three all
-    the same from 800 keys on, if the pairs are no whole rounds of the CUs (ragged batches, then batches of one length: 71 x
-    1499, 32 / 8 heads, 76 us, 66; 108, 95; 40 x 3000, 16 / 16 heads, 183, 141; 215, 196; 100 x 1300, 16 / 16, 151, 142; 220, 210;
-    40 x 1200, 32 / 8, 46, 41; 52, 48; even, 128 x 1000, 16 / 4, 45.3, 44.7; 55, 62)."""
+    1000 three."""
     pairs = max(1, pairs)
     if pairs >= 64:
-        splits = 768 // pairs
-        if splits <= 2 and max_keys >= 800 and _uneven(pairs):
-            splits = 3
-        return max(1, min(splits, max_keys // 160))
+        return max(1, min(768 // pairs, max_keys // 160))
     return max(1, min(64, 512 // pairs, max_keys // 64))
-
-
-def _uneven(pairs: int) -> bool:
-    """Workgroups of a pair each, up to eight to a CU, that leave some CUs one short: a twentieth of all or more."""
-    return 256 < pairs <= 2048 and -pairs % 256 * 20 >= pairs
 
 
 def _decode_is_general(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
@@ -1083,13 +1072,8 @@ def _decode_is_general(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
 def _rows_decode_nsplit(pairs: int, max_keys: int) -> int:
     """Context splits of the general kernel's step, one wave per (sequence, kv head, split): three to a SIMD (two, three, 32 /
     8 heads x 64: 32 x 3000 keys 35.0 us, 31.2; 128 x 1000 43.5, 38.0; 16 / 16 heads x 64, 64 x 1500: 62, 54.7; fewer
-    pairs the same). Where that is one split, two from 480 keys on, if the pairs are no whole rounds of the CUs (16 / 16 heads x
-    64, one split and two, ragged batches, then batches of one length: 100 x 600 58.5, 46.7; 67, 66; 100 x 1300 121, 89; 135, 129;
-    even, 128 x 500, 50.7, 50.0; 58.5, 62)."""
-    splits = 3072 // max(1, pairs)
-    if splits == 1 and max_keys >= 480 and _uneven(pairs):
-        splits = 2
-    return max(1, min(64, splits, max_keys // 64))
+    pairs the same)."""
+    return max(1, min(64, 3072 // max(1, pairs), max_keys // 64))
 
 
 def attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
