@@ -38,8 +38,10 @@ struct Small64Cfg {
 // G: groups of four waves. 2: where each tile has a compute unit to itself, two groups form the tile over half of K each, with
 // rings of their own, and add their sums at the end; the one covers the other's waits, and a barrier publishes two slabs. us, one
 // group -> two, int8 / fp8: 200 x 4096 x 11008 27.3 / 26.6 -> 23.6 / 22.6, 193 x 2048 x 5632 13.9 / 12.9 -> 11.9 / 11.2, 256 x 4096 x
-// 4096 12.6 / 11.5 -> 11.2 / 10.7, 300 x 2048 x 2048 8.4 / 7.8 -> 7.6 / 7.3, 200 x 2048 x 256 5.7 / 5.2 -> 5.5 / 5.15. 128-block scales
-// gain from 40 slabs on, where their longer prologue is made up for: 374 x 1536 x 7168 17.4 -> 15.5, 70 x 2048 x 7168 14.5 -> 13.2, 145 x
+// 4096 12.6 / 11.5 -> 11.2 / 10.7, 300 x 2048 x 2048 8.4 / 7.8 -> 7.6 / 7.3. With few slabs the exchange of the sums costs more than
+// the half chain saves, an odd slab more still (500 x 2048 x 128 4.2 / 3.9 -> 4.5 / 4.3, x 640 4.9 / 4.6 -> 5.2 / 5.0; one
+// group's time over two's with 8 slabs 1.02 / 0.98, 10 1.04 / 1.00, 11 1.01 / 0.98, 12 1.05 / 1.02): from 10 slabs with a step a row and column, from
+// 12 with one step. 128-block scales gain from 40 slabs on, where their longer prologue is made up for: 374 x 1536 x 7168 17.4 -> 15.5, 70 x 2048 x 7168 14.5 -> 13.2, 145 x
 // 4096 x 4096 10.3 -> 10.0, 250 x 4096 x 4096 10.7 -> 10.8, 100 x 7168 x 2048 7.1 -> 7.3. (Four waves of the whole tile over a
 // quarter of K each, with no barrier and every slab read once: the same with long K, 0.6 to 1.4 us slower with up to 16 slabs.)
 template <class Op, int ScaleKind, int S, bool RoundFirst, int G>
@@ -326,8 +328,9 @@ inline void launch_small64(const GemmArgs& g, hipStream_t stream) {
     if constexpr (!RoundFirst && ScaleKind == SCALE_TENSOR)
         if (g.round_first) return launch_small64<Op, ScaleKind, true>(g, stream);
     const int64_t tiles = (int64_t)((g.m + 63) / 64) * ((g.n + 63) / 64);
+    constexpr int kTwoGroups = ScaleKind == SCALE_BLOCK128 ? 40 : ScaleKind == SCALE_TENSOR ? 12 : 10;   // slabs from which they gain
     if constexpr (G == 1)
-        if (tiles <= 256 && (ScaleKind != SCALE_BLOCK128 || g.k >= 40 * 128))
+        if (tiles <= 256 && g.k >= kTwoGroups * 128)
             return launch_small64<Op, ScaleKind, RoundFirst, 2>(g, stream);
     auto kern = gemm_small64_kernel<Op, ScaleKind, kSmall64Stages, RoundFirst, G>;
     static std::atomic<uint64_t> lds_allowed{0};

@@ -13,8 +13,8 @@ DEV = "cuda"
 CASES = [(2049, 2049, 128, "mid128x256"), (2047, 2302, 256, "mid128x256"), (2100, 2060, 384, "mid128x256"), (1281, 3080, 512, "mid128x256"),
          (4090, 1100, 640, "mid128x256"), (300, 11264, 768, "mid128x256"), (129, 16640, 896, "mid128x256"), (16512, 256, 640, "mid128x256"),
          (1500, 1501, 128, "mid128"), (1530, 1500, 640, "mid128"), (1409, 1544, 768, "mid128"), (1537, 1410, 384, "mid128")] + [
-    # halves of K: odd and even counts of slabs, one, and fewer than the ring's stages
-    (130 + 9 * i, 1021 + i, 128 * i, "small64") for i in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17)]
+    # one group of waves up to nine slabs (eleven with one step), then halves of K: odd and even counts of slabs
+    (130 + 9 * i, 1021 + i, 128 * i, "small64") for i in (1, 2, 3, 4, 5, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17)]
 
 
 @pytest.mark.parametrize("m,n,k,kernel", CASES)
