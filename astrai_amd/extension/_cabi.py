@@ -493,10 +493,14 @@ def linear_backward(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, masks):
     k]``, ``w [n, k]``; ``None`` for what the kernels do not take as it is.
 
     The input gradient is the library's product where its 128 x 128 tiles take more than one round of the compute units: these
-    kernels are 0.83 to 1.14 times as fast there (4096 x 4096 x 4096 130 us, the library 108; 1700 x 4096 x 4096 58 and 63), and 1.0
-    to 3 times up to there (552 x 11264 x 2048 40 and 91, 1700 x 2048 x 2048 18 and 26; 256 x 2048 x 2048 14.4 and 13.5). So is the weight
-    gradient of the largest whole blocks without a bias (operands from memory: 4096 x 4096 x 4096 141 us, the library 136, and 20 more
-    for the sums; 8192 x 8192 x 2048 268 and 243; 2500 x 11264 x 2048 122 and 155, 1024 x 4096 x 11008 125 and 121)."""
+    kernels are 0.83 to 1.14 times as fast there (4096 x 4096 x 4096 130 us, the library 108; 1700 x 4096 x 4096 58 and 63), and up to
+    there mostly 1.0 to 3 times (552 x 11264 x 2048 40 and 91, 1700 x 2048 x 2048 18 and 26). Small products are up to 3 us longer on
+    the card (256 x 2048 x 2048 14.2 and 12.1, 16 x 1024 x 1024 7.7 and 4.9), which an eager call does not see: the library's takes the
+    host 15 us more (16 and 27, 12 and 27 a call).
+    So is the weight gradient of the largest whole blocks without a bias (operands from memory: 4096 x 8192 x 8192 537 us, the library
+    478; 4096 x 11264 x 2048 177 and 171). Below, the two lie within some 10% of each other from about 2e10 products on and change
+    places with where the operands were last (2048 x 4096 x 4096 0.87 to 1.04 times as fast, 2048 x 2048 x 5632 0.97 to 1.16, 1024 x 4096 x
+    11008 1.03, but behind the library's input gradient 0.9 for both); smaller ones are up to 4 times as fast here."""
     lib = _require()
     (n, k), m, dev = w.shape, g.size(0), g.device
     own_x = masks[0] and -(-m // 128) * -(-k // 128) <= 256
