@@ -9,6 +9,7 @@
 #include "host.h"
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 
@@ -230,7 +231,7 @@ PyObject* mm_block128(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 }
 
 // Whether a dispatcher op on these would do nothing but call its device kernel: plain tensors of one GPU that need no
-// gradient and carry no tangent, no dispatch or function mode, transform, trace or functionalization about.
+// gradient and carry no tangent, no dispatch or function mode, transform, trace, functionalization or profiler about.
 bool nothing_above(std::initializer_list<const Tensor*> tensors) {
     using K = c10::DispatchKey;
     static const c10::DispatchKeySet above({K::Python, K::PythonTLSSnapshot, K::PythonDispatcher, K::PreDispatch, K::Functionalize,
@@ -239,7 +240,7 @@ bool nothing_above(std::initializer_list<const Tensor*> tensors) {
                                             K::BatchedNestedTensor, K::NestedTensor, K::Tracer, K::Fake, K::Negative, K::Conjugate,
                                             K::DeferredInit});
     const auto on = c10::impl::tls_local_dispatch_key_set();
-    if (!(on.included_ & above).empty() || at::impl::torch_function_mode_enabled()) return false;
+    if (!(on.included_ & above).empty() || at::impl::torch_function_mode_enabled() || at::hasCallbacks()) return false;
     const bool grads = c10::GradMode::is_enabled();
     for (const Tensor* t : tensors)
         if (t && (!(t->key_set() & above).empty() || (grads && t->requires_grad()) || t->_fw_grad(0).defined())) return false;

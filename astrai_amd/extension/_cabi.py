@@ -1798,7 +1798,7 @@ def mm_fp8_block128(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torc
 def mm_fp8_block128_eager(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
                           bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """:func:`mm_fp8_block128` where a dispatcher op would do nothing but call it: plain operands as the kernels read them, no
-    gradients, modes, transforms or traces about. ``None`` elsewhere."""
+    gradients, modes, transforms, traces or profilers about. ``None`` elsewhere."""
     return _host.mm_block128_eager(a, b, sa, sb, bias)
 
 

@@ -81,6 +81,20 @@ def test_what_stands_above_sees_the_op():
 
 
 @pytest.mark.gpu
+def test_a_profile_has_the_op():
+    from torch.profiler import ProfilerActivity, profile
+    from astrai_amd.extension import _cabi
+    from astrai_amd.extension.ops import fp8_block as blk
+    args = _operands()
+    want = blk.mm_fp8_blockscaled(*args)
+    with profile(activities=[ProfilerActivity.CPU]) as p:
+        assert _cabi.mm_fp8_block128_eager(*args) is None
+        got = blk.mm_fp8_blockscaled(*args)
+    assert torch.equal(got, want) and any("fp8_gemm_blockscaled" in e.key for e in p.key_averages())
+    assert _cabi.mm_fp8_block128_eager(*args) is not None
+
+
+@pytest.mark.gpu
 def test_bf16_backward_native_and_adapter(monkeypatch):
     """The native form of the bf16 backward and the adapter's own path: the same bits, the same refusals."""
     from astrai_amd.extension import _cabi
