@@ -13,7 +13,7 @@ DEV = "cuda"
 
 # (5 slabs are the fewest of the 128 x 128 tiles' ring of four stages, one and four those of its two stages)
 @pytest.mark.parametrize("m,n,slabs,kernel", [(65 + 7 * s, 200 if s % 2 else 333, s, "small64") for s in range(1, 10)] +
-                         [(1100, 2048, s, "mid128_block128") for s in (1, 4, 5, 6, 7, 8, 9)] + [(1301, 1804, 11, "mid128_block128")] +
+                         [(1100, 2048, s, "mid128_block128") for s in (1, 4, 5, 6, 7, 8, 9)] + [(1301, 1804, 11, "mid128_block128"), (1100, 2045, 6, "mid128_block128"), (1029, 2047, 4, "mid128_block128")] +
                          [(2500, 4096, s, "pingpong_block128") for s in (2, 3, 4, 5, 6, 9)])
 def test_steps_of_every_slab(m, n, slabs, kernel):
     """Steps spread over seven octaves from row to row and from block to block: one of another row, column block or slab
