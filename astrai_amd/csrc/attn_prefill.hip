@@ -121,7 +121,7 @@ __device__ __forceinline__ int part_blocks(const AttnPrefillArgs& a, int blocks)
 // MASK (paged only): a bool tensor says, per sequence, (head,) (query row,) and position,
 // what may be attended on top of the causal range (csrc/kernels/attention/mma_utils.cuh:190-199);
 // every tile then takes the masking path.
-// PARTS (paged, no mask): part `split` of a.nsplit takes the 64-key blocks part_blocks() gives it, of which nothing but
+// PARTS (paged, no mask, SPLIT): part `split` of a.nsplit takes the 64-key blocks part_blocks() gives it, of which nothing but
 // the table and the limits know; a block of queries with more than one part leaves them to merge_parts_kernel.
 template <int D, int NREP, int QSUB, bool PAGED, bool MASK, bool SPLIT, bool PARTS = false>
 __global__ __launch_bounds__(64 * NREP * QSUB, NREP * QSUB < 4 ? 1 : D == 64 && NREP * QSUB == 4 ? 3 : 2) void attn_prefill_kernel(AttnPrefillArgs a) {
@@ -842,10 +842,14 @@ bool launch_shape(const AttnPrefillArgs& a, hipStream_t stream) {
         else
             return false;
     } else if (paged && a.nsplit > 1) {
-        const int64_t waves = wgs * NREP * QP, merges = (waves * (D / 8) + 3) / 4;
-        if (merges > INT_MAX) return false;
-        attn_prefill_kernel<D, NREP, QP, true, false, SPLIT, true><<<dim3((unsigned)(wgs * a.nsplit)), block, 0, stream>>>(a);
-        merge_parts_kernel<D, NREP, QP><<<dim3((unsigned)merges), dim3(256), 0, stream>>>(a, waves);
+        if constexpr (SPLIT) {
+            const int64_t waves = wgs * NREP * QP, merges = (waves * (D / 8) + 3) / 4;
+            if (merges > INT_MAX) return false;
+            attn_prefill_kernel<D, NREP, QP, true, false, SPLIT, true><<<dim3((unsigned)(wgs * a.nsplit)), block, 0, stream>>>(a);
+            merge_parts_kernel<D, NREP, QP><<<dim3((unsigned)merges), dim3(256), 0, stream>>>(a, waves);
+        } else {
+            return false;
+        }
     } else if (paged) {
         attn_prefill_kernel<D, NREP, QP, true, false, SPLIT><<<grid, block, 0, stream>>>(a);
     } else if (narrow) {
