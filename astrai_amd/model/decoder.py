@@ -97,6 +97,21 @@ class Embedding(nn.Module):
         return F.embedding(x, self.weight)
 
 
+MODULE_CALL = nn.Module.__call__
+FORWARDS = {Embedding: Embedding.forward}   # of classes whose calls may be passed by, as defined
+every = nn.modules.module   # (its hooks are every module's)
+
+
+def observed(module: nn.Module) -> bool:
+    """A call of ``module``, of a class in ``FORWARDS``, runs something else than that class's ``forward``: hooks, its own or
+    those of every module, a compiled call, or a ``forward`` or ``__call__`` put in the place of the one defined here."""
+    own, cls = module.__dict__, type(module)   # (five times a layer: no attribute lookups through the module)
+    return bool(own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
+                or every._global_backward_pre_hooks or own.get("_compiled_call_impl") or "forward" in own
+                or cls.forward is not FORWARDS[cls] or cls.__call__ is not MODULE_CALL)
+
+
 def get_rotary_emb(dim: int, max_len: int, base: float = 10000.0) -> Tensor:
     """``[max_len, dim/2, 2]`` fp32 table of (cos, sin), angles computed in fp64."""
     theta = base ** (-torch.arange(0, dim, 2, dtype=torch.float64) / dim)
@@ -380,7 +395,7 @@ class AutoRegressiveLM(nn.Module):
         ``(x, rotary, (xq, sx))``. ``None`` where the embedding or the block is not this file's own, unobserved, or the kernel
         does not take the operands."""
         emb, w = self.embed_tokens, self.embed_tokens.weight
-        if (self.fused_int8 is None or not _fused_int8_active(w) or not len(self.layers) or _observed(emb, Embedding)
+        if (self.fused_int8 is None or not _fused_int8_active(w) or not len(self.layers) or type(emb) is not Embedding or observed(emb)
                 or type(self.layers[0]) is not DecoderBlock or "_forward_fused_int8" in self.layers[0].__dict__
                 or any(type(t) not in (Tensor, nn.Parameter) for t in (ids, w, positions))):
             return None
@@ -435,19 +450,6 @@ class AutoRegressiveLM(nn.Module):
             x = x.index_select(1, logits_at)
         hidden = self.norm(x)
         return {"logits": self.lm_head(hidden), "hidden_states": hidden}
-
-
-_EMBED, _CALL, _every = Embedding.forward, nn.Module.__call__, nn.modules.module   # as defined here; every module's hooks
-
-
-def _observed(module: nn.Module, cls: type) -> bool:
-    """A call of ``module`` runs something else than ``Embedding.forward`` as defined here: another class, hooks, a compiled
-    call, a replaced ``forward``."""
-    own = module.__dict__
-    return bool(type(module) is not cls or cls.forward is not _EMBED or cls.__call__ is not _CALL or "forward" in own
-                or own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
-                or own.get("_compiled_call_impl") or _every._global_forward_hooks or _every._global_forward_pre_hooks
-                or _every._global_backward_hooks or _every._global_backward_pre_hooks)
 
 
 def _fused_int8_active(x: Tensor) -> bool:

@@ -32,7 +32,7 @@ from torch.autograd import forward_ad
 from astrai_amd.extension import _mix, dispatch
 from astrai_amd.extension._mix import RING_STEPS, DeltaShape, GqaShape, LatentShape, pad_to
 from astrai_amd.model.cache import MixerCache
-from astrai_amd.model.decoder import Embedding, Linear, rotary_table, yarn_frequencies
+from astrai_amd.model.decoder import FORWARDS, Embedding, Linear, observed, rotary_table, yarn_frequencies
 
 # a block of at most this many tokens attends in the latent space, longer ones form keys and values
 LATENT_ROWS_MAX = 16
@@ -192,19 +192,6 @@ class HeadLinear(Linear):
 
     def forward(self, x: Tensor) -> Tensor:
         return linear(x, self.weight, self.bias)
-
-
-every = nn.modules.module   # (its hooks are every module's)
-
-
-def observed(module: nn.Module) -> bool:
-    """A call of ``module``, of a class in ``FORWARDS``, runs something else than that class's ``forward``: hooks, its own or
-    those of every module, a compiled call, or a ``forward`` or ``__call__`` put in the place of the one defined here."""
-    own, cls = module.__dict__, type(module)   # (five times a layer: no attribute lookups through the module)
-    return bool(own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
-                or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
-                or every._global_backward_pre_hooks or own.get("_compiled_call_impl") or "forward" in own
-                or cls.forward is not FORWARDS[cls] or cls.__call__ is not MODULE_CALL)
 
 
 def heads_of(name: str, heads: int, *dims: int) -> Rows:
@@ -689,8 +676,7 @@ class GatedMLP(nn.Module):
 
 
 MIXERS = (LatentAttention, LightningAttention, GroupedAttention, GatedRecurrence, ChannelDelta)
-FORWARDS = {cls: cls.forward for cls in (*MIXERS, GatedMLP, PackedLinear)}   # as defined here
-MODULE_CALL = nn.Module.__call__
+FORWARDS.update({cls: cls.forward for cls in (*MIXERS, GatedMLP, PackedLinear)})   # as defined here
 
 
 def mixed(mix: nn.Module, h: Tensor, ctx: StepContext) -> Tensor:
