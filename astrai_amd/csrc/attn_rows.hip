@@ -187,13 +187,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 32 
     const int nq = n_rep * rows;  // <= kNQ
     int64_t item = (int64_t)blockIdx.x * 4 + wave;
     if (item >= a.num_items) return;
-    // Which wave has what, for steps whose splits can be 120 keys and more: neighbours have the KV heads of one range of keys, and
+    // Which wave has what, for steps of 480 keys and more whose splits can be 120 and more: neighbours have the KV heads of one range of keys, and
     // so fetch neighbouring pieces of the same pool rows (128 bytes a head of 64) at about the same time; with a head's splits side
     // by side the pieces of a row came up all over the launch (16/16 heads x 64, 40 x 3000 keys 115 us, 2.9 TB/s, and 90, 3.7; 16/4
-    // x 32, 32 x 3000 20.8 and 19.0; 32/8 x 64, 20 x 6000 50.7 and 49.8). Shorter ranges gain nothing (7 x 3000 in 46 splits 16.5, 16.8). The
-    // table's width decides: behind one of 4096, contexts of 240 to 700 keys are 1 to 4% faster all the same, of 100 1% slower (40 x 100,
-    // 16/16 x 64, 10.9 and 12.1). By each context's own length, known only from memory, every call's chain is 1% longer.
-    const bool heads_first = !a.qo_indptr && a.rtt_stride >= 120 * (int64_t)a.nsplit;
+    // x 32, 32 x 3000 20.8 and 19.0; 32/8 x 64, 20 x 6000 50.7 and 49.8). Shorter ranges gain nothing (7 x 3000 in 46 splits 16.5,
+    // 16.8), and few keys lose up to 3% (16/16 x 64, 71 x 386 in two splits 26.6, 27.1). The table's width decides: behind one of 4096,
+    // contexts of 240 to 700 keys are 1 to 4% faster all the same, of 100 1% slower (40 x 100, 16/16 x 64, 10.9 and 12.1). By each
+    // context's own length, known only from memory, every call's chain is 1% longer.
+    const bool heads_first = !a.qo_indptr && a.rtt_stride >= max((int64_t)480, 120 * (int64_t)a.nsplit);
     const int inner = heads_first ? a.n_kv_heads : a.nsplit, outer = heads_first ? a.nsplit : a.n_kv_heads;
     int of_inner, of_outer, block;
     if (a.num_items <= UINT32_MAX) {

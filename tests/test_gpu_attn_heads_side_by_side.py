@@ -1,5 +1,6 @@
-"""Paged steps of the general kernel, whose waves take KV heads side by side where a split's share of the slot table is 120
-positions or more and splits side by side otherwise: both sides of that line, KV heads that fill no whole workgroup."""
+"""Paged steps of the general kernel, whose waves take KV heads side by side where the slot table has 480 positions or
+more and a split's share of them is 120, and splits side by side otherwise: both sides of those lines, KV heads that fill no whole
+workgroup."""
 
 import pytest
 import torch
@@ -12,7 +13,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("h,hkv,d", [(6, 3, 64), (5, 5, 32), (16, 16, 64), (7, 1, 256)])
-@pytest.mark.parametrize("width,nsplit", [(119, 1), (120, 1), (720, 2), (720, 5), (720, 6), (719, 6), (720, 7), (7680, 64), (7679, 64)])
+@pytest.mark.parametrize("width,nsplit", [(119, 1), (120, 1), (479, 2), (480, 2), (480, 4), (480, 5), (720, 2), (720, 5), (720, 6), (719, 6), (720, 7), (7680, 64), (7679, 64)])
 def test_either_order(h, hkv, d, width, nsplit):
     from astrai_amd.extension import _cabi
     print(f"case h={h} hkv={hkv} d={d} width={width} nsplit={nsplit}", flush=True)
