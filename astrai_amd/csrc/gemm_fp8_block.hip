@@ -14,10 +14,10 @@ namespace w8a8 {
 
 namespace {
 
-// Tiles of 256 x 256 where they fill most of the chip, or where 128 x 128 tiles would put a second workgroup on compute
-// units (from 257 of them), which takes nearly twice as long as one, where a round of large tiles costs little more than the
-// first (us, 128 x 128 / large: 1100 x 4096 x 4096, 288 tiles, 56 / 43, x 512 12.7 / 11.4; 2300 x 2048 x 7168 97 / 71; 900 x
-// 7168 x 2048, 448 tiles, 32 / 26. Only 264 tiles whose last rows are nearly empty end sooner: 257 x 11264 x 2048 22 / 25).
+// Tiles of 256 x 256, behind those of 128 x 256, where they fill most of the chip, or where 128 x 128 tiles would put a second workgroup
+// on compute units (from 257 of them), which takes nearly twice as long as one, where a round of large tiles costs little more
+// than the first (us, 128 x 128 / large: 14000 x 640 x 2048, 550 tiles, 42 / 25.5, x 512 14.5 / 11.5; 17000 x 384 x 2048, 399 tiles, 28.5 /
+// 24.5, x 11008 152 / 117. Up to 512 tiles with few slabs end sooner: 17000 x 384 x 512 9.9 / 10.7, 12000 x 640 x 256 8.3 / 8.8).
 bool large_tiles_take(const GemmArgs& g) {
     if ((g.n & 7) != 0 || g.out_kind != OUT_BF16) return false;
     return pingpong_shape_ok(g) || (g.k >= 256 && (int64_t)((g.m + 127) / 128) * ((g.n + 127) / 128) > 256);

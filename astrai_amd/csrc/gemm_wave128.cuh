@@ -64,11 +64,11 @@ inline void split_rows(const GemmArgs& g, int r, bool rowcol, GemmArgs& head, Ge
 }
 
 // Plain bf16 products that the large tiles take, behind wide256_shape_ok: where they fill most of the chip, or from 449 tiles of 128 x
-// 128 on (those past what tiles of 128 x 256 do in one round). Two
+// 128 on (those past what tiles of 128 x 256 do in one round: few columns). Two
 // workgroups of those share a compute unit and take longer the more units have two, where a round of large tiles costs
-// the same however empty (us, 128 x 128 / large, fp8 and int8: 2048 x 4096 x 512 14.5 / 12.0 and 15.1 / 13.5, x 4096 37.8 / 37.5
-// and 41.2 / 40.1, x 11008 87 / 86 and 96 / 90; 640 x 11776 x 4096, 460 tiles, 43 / 37 and 44 / 40). What it costs: up to 480
-// tiles with K of 2048 to 5632 1 to 5% (1800 x 4096 x 4096 36.5 / 37.9 and 39.5 / 40.2).
+// the same however empty (us, 128 x 128 / large, fp8 and int8: 14000 x 640 x 512, 550 tiles, 12.1 / 11.0 and 13.2 / 12.6, x 4096 48 / 36
+// and 53 / 39; 12000 x 640 x 11008, 470 tiles, 103 / 89 and 106 / 91). What it costs: up to 512 tiles with K to 4096 (12000 x 640 x 512
+// 9.6 / 10.8 and 10.4 / 12.4, x 2048 19.9 / 22.0 and 21.7 / 23.9, x 4096 34.0 / 36.2 and 37.0 / 38.7).
 inline bool wave128_takes(const GemmArgs& g) {
     if (wave128_shape_ok(g)) return true;
     if (!tiled_shape_ok(g) || (g.k & 127) != 0 || g.k < 256 || g.out_kind != OUT_BF16 || (g.n & 7) != 0 || g.n > (1 << 22))
