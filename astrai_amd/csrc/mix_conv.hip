@@ -41,11 +41,12 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
         static_assert(TAPS - 1 <= kStrip, "no other strip reads the ring");
         const bool ringed = a.tail && t0 == 0;
         const int n = min(TAPS - 1, a.seq);
-        f32x4 keep[TAPS - 1];   // (asked for with the rest: one after the other at the end they cost what the launch did)
+        typedef uint32_t Quad __attribute__((ext_vector_type(sizeof(T))));   // four inputs as they are stored
+        Quad keep[TAPS - 1];   // (asked for with the rest: one after the other at the end they cost what the launch did)
         if (ringed) {
 #pragma unroll
             for (int j = 0; j + 1 < TAPS; ++j)
-                if (j < n) keep[j] = conv_input4<T>(a, b, start, a.seq - n + j, c);
+                if (j < n) keep[j] = *reinterpret_cast<const Quad*>(static_cast<const T*>(a.proj) + ((int64_t)b * a.seq + a.seq - n + j) * a.ld + a.off + c);
         }
 #pragma unroll
         for (int i = 0; i < kStrip; ++i) {
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a) {
 #pragma unroll
             for (int j = 0; j + 1 < TAPS; ++j)
                 if (const int64_t p = start + a.seq - n + j; j < n && p >= 0)
-                    Elem<T>::put4(static_cast<T*>(a.ring) + ring_row(a, b, p) * a.cols + c, keep[j]);
+                    *reinterpret_cast<Quad*>(static_cast<T*>(a.ring) + ring_row(a, b, p) * a.cols + c) = keep[j];
         }
     } else {
         for (int t = t0; t < t1; ++t) finish(t, conv_at4<T>(a, b, start, t, c));
