@@ -641,12 +641,10 @@ __device__ __forceinline__ u32x4 table_piece(const uint16_t* table, int64_t at, 
     return at >= 0 ? *reinterpret_cast<const u32x4*>(table + at * k + i * 8) : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
 }
 
-// A row's step from its largest magnitude, which ignores what is not a number, as the quantizers' does: keys and values of such a row
-// stay finite. Where y goes out too, a row of y that is no number by its norm has such a step, and what is formed of its codes says
-// so as y does: a token or position outside its table ends in logits of NaN.
-__device__ __forceinline__ float row_step(float largest, float rstd, bool y_out) {
-    return y_out && rstd != rstd ? rstd : fmaxf(largest, 1e-12f) / 127.0f;
-}
+// The step that goes out with a row's codes. It comes from the largest magnitude, which ignores what is not a number, as the quantizers'
+// does: keys and values of such a row stay finite. Where y goes out too, a row of y that is no number by its norm has such a step, and
+// what is formed of its codes says so as y does: a token or position outside its table ends in logits of NaN.
+__device__ __forceinline__ float step_out(float step, float rstd, bool y_out) { return y_out && rstd != rstd ? rstd : step; }
 
 // s = bf16(x + res) (when res is given; written to sum_out), y = bf16(w * (rstd * s))
 // with rstd = rsqrt(mean(s^2) + eps) in fp32 -- one rounding, the arithmetic of
@@ -710,8 +708,8 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_quantize_int8_rows_kerne
             if (!START && y_out) *reinterpret_cast<u32x4*>(y_out + row * k + i * 8) = packed;
         }
     }
-    const float step = row_step(block_max(local, slots), rstd, !START && y_out);
-    if (threadIdx.x == 0) s[row] = step;
+    const float step = fmaxf(block_max(local, slots), 1e-12f) / 127.0f;
+    if (threadIdx.x == 0) s[row] = step_out(step, rstd, !START && y_out);
 #pragma unroll
     for (int c = 0; c < kCache; ++c) {
         const int64_t i = threadIdx.x + (int64_t)c * kThreads;
@@ -815,8 +813,8 @@ __global__ __launch_bounds__(kThreads) void wave_rows_int8_kernel(
                 local = fmaxf(local, amax8(v[c]));
             }
         }
-        const float step = row_step(wave_max(local), rstd, NORM && !START && y_out);
-        if (lane == 0) s[row] = step;
+        const float step = fmaxf(wave_max(local), 1e-12f) / 127.0f;
+        if (lane == 0) s[row] = step_out(step, rstd, NORM && !START && y_out);
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             const int64_t i = lane + (int64_t)c * kWave;
